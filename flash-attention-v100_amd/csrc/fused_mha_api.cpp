@@ -19,6 +19,8 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -31,10 +33,14 @@
 namespace {
 
 void check_arch(int device) {
+  // The property query copies a structure of more than a kilobyte; the answer never changes.
+  static std::atomic<bool> known_gfx950[64];
+  if (device >= 0 && device < 64 && known_gfx950[device].load(std::memory_order_relaxed)) return;
   hipDeviceProp_t prop;
   TORCH_CHECK(hipGetDeviceProperties(&prop, device) == hipSuccess, "hipGetDeviceProperties failed");
   TORCH_CHECK(std::strncmp(prop.gcnArchName, "gfx950", 6) == 0, "This repo only supports gfx950 (MI355X) GPUs, got ",
               prop.gcnArchName);
+  if (device >= 0 && device < 64) known_gfx950[device].store(true, std::memory_order_relaxed);
 }
 
 void check_rc(int rc, const char* what) {
@@ -64,7 +70,7 @@ Operand operand(const at::Tensor& x) {
 
 }  // namespace
 
-std::vector<at::Tensor> mha_fwd(at::Tensor& q,        // batch x seqlen x heads x head_size
+std::vector<at::Tensor> mha_fwd(const at::Tensor& q,  // batch x seqlen x heads x head_size
                                 const at::Tensor& k,  // batch x seqlen x heads x head_size
                                 const at::Tensor& v,  // batch x seqlen x heads x head_size
                                 c10::optional<at::Tensor>& out_, const float softmax_scale, bool is_causal) {
@@ -184,8 +190,53 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
   return {dq, dk, dv};
 }
 
+namespace {
+
+at::Tensor last_dim_contiguous(const at::Tensor& x) { return x.stride(-1) == 1 ? x : x.contiguous(); }
+
+// The autograd node of flash_attn_func.  Native on purpose: a torch.autograd.Function written in Python
+// costs about 60 us per forward and backward, most of it in handing the interpreter lock to the engine's
+// device thread and back, which is more than the kernels of a small problem take.
+class AttentionNode : public torch::autograd::Function<AttentionNode> {
+ public:
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q_in, const at::Tensor& k_in,
+                            const at::Tensor& v_in, double softmax_scale, bool is_causal) {
+    const at::Tensor q = last_dim_contiguous(q_in), k = last_dim_contiguous(k_in), v = last_dim_contiguous(v_in);
+    c10::optional<at::Tensor> none;
+    auto out_lse = mha_fwd(q, k, v, none, (float)softmax_scale, is_causal);
+    ctx->save_for_backward(torch::autograd::variable_list{q, k, v, out_lse[0], out_lse[1]});
+    ctx->saved_data["softmax_scale"] = softmax_scale;
+    ctx->saved_data["causal"] = is_causal;
+    return out_lse[0];
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grad_out) {
+    const auto saved = ctx->get_saved_variables();
+    c10::optional<at::Tensor> none_q, none_k, none_v;
+    auto grads = mha_bwd(last_dim_contiguous(grad_out[0]), saved[0], saved[1], saved[2], saved[3], saved[4], none_q,
+                         none_k, none_v, (float)ctx->saved_data["softmax_scale"].toDouble(),
+                         ctx->saved_data["causal"].toBool());
+    return {grads[0], grads[1], grads[2], at::Tensor(), at::Tensor()};
+  }
+};
+
+}  // namespace
+
+// flash_attn_func: attention with its gradient.  softmax_scale defaults to head_size ** -0.5.
+at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                     c10::optional<double> softmax_scale, bool is_causal) {
+  const double scale = softmax_scale.has_value() ? *softmax_scale : std::pow((double)q.size(-1), -0.5);
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+    return AttentionNode::apply(q, k, v, scale, is_causal);
+  c10::optional<at::Tensor> none;
+  return mha_fwd(last_dim_contiguous(q), last_dim_contiguous(k), last_dim_contiguous(v), none, (float)scale,
+                 is_causal)[0];
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "FlashAttention forward/backward for gfx950";
+  m.def("attention", &attention, "Attention, differentiable in q, k and v");
   m.def("fwd", &mha_fwd, "Forward pass");
   m.def("bwd", &mha_bwd, "Backward pass");
 }
