@@ -359,13 +359,19 @@ struct Strides {
 };
 
 // ---------------------------------------------------------------------------
-// Forward.  Block = 8 waves = 256 queries, wave = 32 queries; K/V tiles of 64
-// keys stream through a 3-slot LDS ring, copied asynchronously two tiles ahead.
+// Forward for D = 128 where blocks of 256 queries share out evenly over the CUs
+// (rule: launch_forward).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
+// tiles of 64 keys stream through a 3-slot LDS ring, copied asynchronously two
+// tiles ahead.
 //
-// Online softmax as in reference kernel/fused_mha_kernel.cu:159-181, except
-// that the running max is only raised (and O, l rescaled) when it grew by more
-// than kRescaleLog2 in the exp2 domain, which is rare after the first tiles;
-// probabilities then stay below 2^kRescaleLog2 and the final O/l is unchanged.
+// Online softmax as in reference kernel/fused_mha_kernel.cu:159-181, except that
+// no tile's maximum is looked for as long as the running one serves: the
+// probabilities of a tile are formed relative to the running maximum first, and
+// only if a lane's sum over its 32 keys of the tile exceeds kRescaleSum (so every
+// single one stays far below the fp16 range) or is no number (no maximum yet) the
+// maximum is raised, O and l are rescaled, and they are formed again.  That takes
+// the 16 max instructions and the exchange between the half waves out of nearly
+// every tile (B2 H16 N4096 D128 without mask: 254 -> 243 us).
 //
 // The two waves that share a SIMD (w and w+4) run the same three steps per
 // tile, scores (MFMA), softmax (VALU), accumulate (MFMA), in rotated order:
@@ -374,12 +380,11 @@ struct Strides {
 // and V(j-1) in iteration j, so one barrier per iteration is enough, and one
 // wave's MFMA stretch coincides with the other's VALU stretch.
 // ---------------------------------------------------------------------------
-constexpr float kRescaleLog2 = 8.f;
+constexpr float kRescaleSum = 4096.f;
 constexpr int kFwdWaves = 8;
 constexpr int kFwdThreads = kFwdWaves * 64;
 constexpr int kFwdBlockQ = kFwdWaves * kResident;
 constexpr int kRing = 3;
-constexpr int kFwdBlockKernelMaxN = 1024;  // D = 64, causal: longest sequence the one-block kernel takes
 
 // The kernel is persistent: the launch has one work group per CU (fewer for small
 // problems) and each walks its own list of blocks (PersistentBlocks).  While a block's
@@ -502,36 +507,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto softmax = [&](int t) __attribute__((always_inline)) {
-    if (t < 0 || t >= ntw) return;
-    const int key0 = t * kTile;
-    if ((CAUSAL && key0 + kTile - 1 > q0w) || (key0 + kTile > N)) {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          int key = key0 + acc_row(rb, r, hh);
-          if ((CAUSAL && key > qi) || key >= N) s[rb][r] = -INFINITY;
-        }
-    }
-    float mx = s[0][0];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
-    mx = fmaxf(mx, other_half(mx));
-    const float m_new = fmaxf(m_run, mx);
-    if (__builtin_amdgcn_ballot_w64((m_new - m_run) * c > kRescaleLog2) != 0) {
-      const float alpha = fast_exp2((m_run - m_new) * c);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int db = 0; db < G::kDBlocks; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-    }
-    // Row sums with plain fp32 adds: the dot-product instructions share the
-    // matrix pipeline and stall behind the other wave's MFMAs.
+  auto exponentials = [&]() __attribute__((always_inline)) {
     const float mc = m_run * c;
     float l0 = 0.f, l1 = 0.f;
 #pragma unroll
@@ -546,7 +522,41 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
         l1 += p1;
       }
     }
-    l_run += l0 + l1;
+    return l0 + l1;
+  };
+  auto softmax = [&](int t) __attribute__((always_inline)) {
+    if (t < 0 || t >= ntw) return;
+    const int key0 = t * kTile;
+    if ((CAUSAL && key0 + kTile - 1 > q0w) || (key0 + kTile > N)) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          int key = key0 + acc_row(rb, r, hh);
+          if ((CAUSAL && key > qi) || key >= N) s[rb][r] = -INFINITY;
+        }
+    }
+    // Optimistic: probabilities relative to the running maximum as it stands.  If any lane's sum over its 32 keys is
+    // past kRescaleSum (or not a number: no maximum yet), the maximum is brought up to date and they are formed again.
+    float lt = exponentials();
+    if (__builtin_amdgcn_ballot_w64(!(lt <= kRescaleSum)) != 0) {
+      float mx = s[0][0];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
+      mx = fmaxf(mx, other_half(mx));
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = fast_exp2((m_run - m_new) * c);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < G::kDBlocks; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+      lt = exponentials();
+    }
+    l_run += lt;
   };
   auto accumulate = [&](const char* Vl, int t) __attribute__((always_inline)) {
     if (t < 0 || t >= ntw) return;
@@ -713,155 +723,184 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
   else run(IntTag<1>{});
 }
 
-// The forward with one block per work group (no persistence, output staged in the rings once the
-// block is done, fragment reads scheduled by hints): with D = 64 it needs few enough registers
-// and little enough LDS (48 KiB) for two work groups per CU, which the persistent kernel does not.
-// The launcher uses it for D = 64 when that matters more than the persistent kernel's balancing
-// and prefetching: without causal masking (all blocks weigh the same) and for short sequences.
+// ---------------------------------------------------------------------------
+// Forward for D = 64, and for D = 128 where blocks of 256 queries would leave CUs idle (rule: launch_forward).  Block = 4
+// waves, one per SIMD, of 32 queries each; two blocks share a CU.
+//
+// What bounds it: a wave issues one instruction every 4-5 cycles, so one that runs scores, softmax and accumulation one
+// after the other needs 1,800 cycles per 32 x 64 tile at D = 64 (MFMA 512, vector instructions 700) and a SIMD needs
+// several such waves before either unit is busy, which small problems do not have.  Here the three are interleaved
+// inside the wave: step j runs softmax(j) and spreads the MFMAs of accumulate(j - 1) and scores(j + 1) between its vector
+// instructions, in an order that is written out and pinned.  A wave alone on its SIMD then needs 1,450 cycles (B1 H4
+// N8192 D64: 168 -> 83 us against the 8-wave kernel; D128: 184 -> 134 us); with two waves per SIMD and all CUs busy
+// the chip runs at its power limit (B1 H12 N8192 D64: 263 -> 220 us).
+// Small blocks cost twice the K/V copies per query of 256-query blocks and are worth it for balance: B1 H32 N1500 D128
+// causal 41 -> 31 us, B4 H16 N1024 D64 causal 24 -> 17 us, B16 H12 N512 D64 24 -> 20 us, B3 H20 N1031 D128 67 -> 50 us.
+// Three blocks per CU at D = 64 (168 registers) gain 2 % on the long shape and lose 2-5 % on the short ones: not taken.
+//
+// The maximum is handled as in fmha_fwd_kernel.  Bringing it up to date happens outside the main loop, so that the loop
+// itself holds nothing twice.  K and V have two slots each; a tile is copied one tile ahead of its use.
+// ---------------------------------------------------------------------------
+constexpr int kPipeWaves = 4;
+constexpr int kPipeThreads = kPipeWaves * 64;
+constexpr int kPipeBlockQ = kPipeWaves * kResident;
+// kCount copies of 1 KiB to consecutive blocks of LDS: lane l's 16 bytes of block u land at lds + 1024 * u + 16 * l.
+// The instruction's offset counts for both addresses, so they come from base + voff + 64 * u with voff lowered by
+// 960 * u.
+template <int kCount>
+__device__ __forceinline__ void copy16_blocks(const half_t* base, int voff, unsigned lds) {
+  static_assert(kCount == 2 || kCount == 4, "");
+  unsigned saved_m0;
+  if constexpr (kCount == 2) {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %3, %1\n\t"
+        "global_load_lds_dwordx4 %4, %1 offset:1024\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved_m0)
+        : "s"(base), "s"(lds), "v"(voff), "v"(voff - 960)
+        : "memory");
+  } else {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %3, %1\n\t"
+        "global_load_lds_dwordx4 %4, %1 offset:1024\n\t"
+        "global_load_lds_dwordx4 %5, %1 offset:2048\n\t"
+        "global_load_lds_dwordx4 %6, %1 offset:3072\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved_m0)
+        : "s"(base), "s"(lds), "v"(voff), "v"(voff - 960), "v"(voff - 1920), "v"(voff - 2880)
+        : "memory");
+  }
+}
+// Two fp32 values as a pair of fp16 values, at this place in the program: seen through, the optimiser moves the
+// conversions of a tile past the next branch, and keeps the fp32 values in registers until then.
+__device__ __forceinline__ unsigned pack_f16(float lo, float hi) {
+  unsigned r = __builtin_bit_cast(unsigned, h2{(half_t)lo, (half_t)hi});
+  asm volatile("" : "+v"(r));
+  return r;
+}
+
 template <int D, bool CAUSAL>
-__global__ void __launch_bounds__(kFwdThreads, 1)
-fmha_fwd_block_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
-                int nmb, float c, int negate_q) {
+__global__ void __launch_bounds__(kPipeThreads, 2)
+fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                     Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
+                     int nmb, float c, int negate_q) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
-  constexpr int kIPW = T::kInstrs / kFwdWaves;  // copy instructions per wave per tile
-  // K ring then V ring, kRing slots each.  The copies into the ring are inline
-  // asm (see copy16), so slots can be addressed at run time.
-  __shared__ __attribute__((aligned(1024))) char smem[2 * kRing * T::kBytes];
-  char* const k_ring = smem;
-  char* const v_ring = smem + kRing * T::kBytes;
+  constexpr int kDB = G::kDBlocks;
+  constexpr int kIPW = T::kInstrs / kPipeWaves;
+  static_assert(kIPW == T::kNC, "a wave copies the 16 rows of one block row of a tile");
+  // two K tiles, then two V tiles; tile t of either sits in slot t & 1
+  __shared__ __attribute__((aligned(1024))) char smem[4 * T::kBytes];
+  constexpr int kVOff = 2 * T::kBytes;
 
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i = lane & 31, hh = lane >> 5;
+  // what depends on the lane is worked out again where it is needed, not kept in registers across the main loop
+  auto lane_now = []() __attribute__((always_inline)) {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t & 63;
+  };
   int bh, mb;
-  slice_and_block(nmb, bh, mb);
+  fmha_scheduled_block(blockIdx.x, gridDim.x / nmb, nmb, CAUSAL, N % kPipeBlockQ != 0, bh, mb);
   const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O is dense
   const long head_off = ((long)b * N * H + h) * D;
-  const half_t* Qb = Q + b * qs.b + (long)h * qs.h;
-  const half_t* Kb = K + b * ks.b + (long)h * ks.h;
-  const half_t* Vb = V + b * vs.b + (long)h * vs.h;
-
-  const int m0 = mblk * kFwdBlockQ;
+  const int m0 = mblk * kPipeBlockQ;
   const int q0w = m0 + wave * kResident;
-  const int qi = q0w + i;
 
-  // nt: tiles the block streams; ntw: tiles this wave has unmasked keys in.
-  int nt = (N + kTile - 1) / kTile;
-  int ntw = nt;
+  const int nt_all = (N + kTile - 1) / kTile;
+  int nt = nt_all, ntw = q0w < N ? nt_all : 0;  // tiles the block streams; tiles this wave works on
   if (CAUSAL) {
-    nt = min(nt, (min(m0 + kFwdBlockQ, N) - 1) / kTile + 1);
-    ntw = min(nt, (min(q0w + kResident, N) - 1) / kTile + 1);
-    if (q0w >= N) ntw = 0;
+    nt = min(nt, (min(m0 + kPipeBlockQ, N) - 1) / kTile + 1);
+    ntw = q0w < N ? min(nt, (min(q0w + kResident, N) - 1) / kTile + 1) : 0;
   }
 
-  // this wave's share of every tile copy
-  int c_row[kIPW], c_kgoff[kIPW], c_vgoff[kIPW], c_blk[kIPW];
-#pragma unroll
-  for (int u = 0; u < kIPW; ++u) {
-    const int t = wave * kIPW + u;
-    copy_src<D>(t, lane, ks.n, c_row[u], c_kgoff[u]);
-    copy_src<D>(t, lane, vs.n, c_row[u], c_vgoff[u]);
-    c_blk[u] = t * 1024;
+  // Wave w copies rows 16 w .. 16 w + 15 of every tile, 64 bytes of each per instruction; in the last tile rows past
+  // the end re-read row N-1.  Offsets are relative to kBack bytes before the tile (see copy16_blocks).
+  constexpr int kBack = 960 * (kIPW - 1);
+  int k_goff, v_goff, c_past;  // c_past: how many rows past the end this lane's row of the last tile is
+  {
+    const int lane = lane_now(), row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ (lane >> 4)) * 16;
+    k_goff = row * ks.n * 2 + col + kBack;
+    v_goff = row * vs.n * 2 + col + kBack;
+    asm volatile("" : "+v"(k_goff), "+v"(v_goff));
+    c_past = max((nt_all - 1) * kTile + row - (N - 1), 0) * 2;
   }
-  auto copy_tile = [&](const half_t* src, int src_rs, const int (&goff)[kIPW], char* dst, int tile_idx)
-                       __attribute__((always_inline)) {
-    const int row0 = tile_idx * kTile;
-    const half_t* tp = src + (long)row0 * src_rs;  // wave-uniform
-    if (row0 + kTile <= N) {
-#pragma unroll
-      for (int u = 0; u < kIPW; ++u) copy16(tp, goff[u], dst + c_blk[u]);
-    } else {
-#pragma unroll
-      for (int u = 0; u < kIPW; ++u) {  // rows past the end re-read row N-1
-        const int back = max(row0 + c_row[u] - (N - 1), 0);
-        copy16(tp, goff[u] - back * src_rs * 2, dst + c_blk[u]);
-      }
-    }
+  const half_t* kp = K + b * ks.b + (long)h * ks.h - kBack / 2;  // the next tile to copy
+  const half_t* vp = V + b * vs.b + (long)h * vs.h - kBack / 2;
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const unsigned lds_w = lds0 + wave * (kIPW * 1024);
+  auto copy_k = [&](int tile, int slot) __attribute__((always_inline)) {
+    if (tile == nt_all - 1) k_goff -= c_past * ks.n;
+    copy16_blocks<kIPW>(kp, k_goff, lds_w + slot * T::kBytes);
+    kp += (long)kTile * ks.n;
   };
-
-  copy_tile(Kb, ks.n, c_kgoff, k_ring, 0);
-  if (nt > 1) copy_tile(Kb, ks.n, c_kgoff, k_ring + T::kBytes, 1);
-  copy_tile(Vb, vs.n, c_vgoff, v_ring, 0);
+  auto copy_v = [&](int tile, int slot) __attribute__((always_inline)) {
+    if (tile == nt_all - 1) v_goff -= c_past * vs.n;
+    copy16_blocks<kIPW>(vp, v_goff, lds_w + kVOff + slot * T::kBytes);
+    vp += (long)kTile * vs.n;
+  };
+  copy_k(0, 0);
+  if (nt > 1) copy_k(1, 1);
 
   h8 qf[G::kKSteps];
   {
-    const half_t* qp = Qb + (long)min(qi, N - 1) * qs.n + hh * 8;
+    const half_t* qp = Q + b * qs.b + (long)h * qs.h + (long)min(q0w + (lane_now() & 31), N - 1) * qs.n +
+                       (lane_now() >> 5) * 8;
 #pragma unroll
     for (int kk = 0; kk < G::kKSteps; ++kk) {
       qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
       if (negate_q) qf[kk] = -qf[kk];
     }
   }
-
   int k_off[2], v_off[2];
-  swz_rows_off<D>(lane, k_off);
-  swz_cols_off<D>(lane, v_off);
+  swz_rows_off<D>(lane_now(), k_off);
+  swz_cols_off<D>(lane_now(), v_off);
+  const unsigned ka0 = opaque_lds_address(smem + k_off[0]), ka1 = opaque_lds_address(smem + k_off[1]);
+  const unsigned va0 = opaque_lds_address(smem + v_off[0]), va1 = opaque_lds_address(smem + v_off[1]);
+  auto k_frag = [&](unsigned at, int n) __attribute__((always_inline)) {  // at: byte offset of the tile's slot
+    return swz_rows_at<D>(ka0 + at, ka1 + at, n & 1, n >> 1);
+  };
+  auto v_frag = [&](unsigned at, int n) __attribute__((always_inline)) {
+    return swz_cols_at<D>(va0 + kVOff + at, va1 + kVOff + at, n / kDB, n % kDB);
+  };
 
-  f16v o[G::kDBlocks];
+  f16v o[kDB];
 #pragma unroll
-  for (int db = 0; db < G::kDBlocks; ++db)
+  for (int db = 0; db < kDB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
-  f16v s[2];   // scores of the tile in flight
-  h8 pf[4];    // its probabilities, fp16, B-operand order
+  float mc = -INFINITY, l_run = 0.f;
+  f16v sA[2], sB[2];
+  u4v pf[4];  // probabilities of a tile, fp16 pairs in B-operand order
+  f16v zero;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero[r] = 0.f;
 
-  auto scores = [&](const char* Kl, int t) __attribute__((always_inline)) {
-    if (t >= ntw) return;
+  constexpr int kLead = 3;  // LDS fragments are read this many MFMAs ahead (2 to 5 make no difference)
+  constexpr int kNS = 2 * G::kKSteps, kNP = 4 * kDB;  // MFMAs of a tile: scores, accumulation
+  static_assert(kNS == kNP, "");
+  auto scores = [&](unsigned at, f16v (&s)[2]) __attribute__((always_inline)) {
+    h8 frag[kLead];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int n = 0; n < kLead; ++n) frag[n] = k_frag(at, n);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[rb][r] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < G::kKSteps; ++kk) {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb) s[rb] = mfma(swz_rows<D>(Kl, rb, kk, k_off), qf[kk], s[rb]);
+    for (int n = 0; n < kNS; ++n) {
+      const int rb = n & 1, kk = n >> 1;
+      s[rb] = mfma(frag[n % kLead], qf[kk], kk == 0 ? zero : s[rb]);
+      if (n + kLead < kNS) frag[n % kLead] = k_frag(at, n + kLead);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // LDS reads run kLead MFMAs ahead of their use.
-    constexpr int kN = 2 * G::kKSteps, kLead = 4;
-    __builtin_amdgcn_sched_group_barrier(0x100, kLead, 0);
-#pragma unroll
-    for (int n = 0; n < kN - kLead; ++n) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, kLead, 0);
   };
-  auto softmax = [&](int t) __attribute__((always_inline)) {
-    if (t < 0 || t >= ntw) return;
-    const int key0 = t * kTile;
-    if ((CAUSAL && key0 + kTile - 1 > q0w) || (key0 + kTile > N)) {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          int key = key0 + acc_row(rb, r, hh);
-          if ((CAUSAL && key > qi) || key >= N) s[rb][r] = -INFINITY;
-        }
-    }
-    float mx = s[0][0];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
-    mx = fmaxf(mx, other_half(mx));
-    const float m_new = fmaxf(m_run, mx);
-    if (__builtin_amdgcn_ballot_w64((m_new - m_run) * c > kRescaleLog2) != 0) {
-      const float alpha = fast_exp2((m_run - m_new) * c);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int db = 0; db < G::kDBlocks; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-    }
-    // Row sums with plain fp32 adds: the dot-product instructions share the
-    // matrix pipeline and stall behind the other wave's MFMAs.
-    const float mc = m_run * c;
+  auto exponentials = [&](const f16v (&s)[2]) __attribute__((always_inline)) {
     float l0 = 0.f, l1 = 0.f;
 #pragma unroll
     for (int c16 = 0; c16 < 4; ++c16) {
@@ -869,75 +908,187 @@ fmha_fwd_block_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
       for (int e = 0; e < 8; e += 2) {
         const float p0 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e], c, -mc));
         const float p1 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e + 1], c, -mc));
-        pf[c16][e] = (half_t)p0;
-        pf[c16][e + 1] = (half_t)p1;
+        pf[c16][e >> 1] = pack_f16(p0, p1);
         l0 += p0;
         l1 += p1;
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    l_run += l0 + l1;
+    return l0 + l1;
   };
-  auto accumulate = [&](const char* Vl, int t) __attribute__((always_inline)) {
-    if (t < 0 || t >= ntw) return;
+  auto mask = [&](f16v (&s)[2], int t) __attribute__((always_inline)) {
+    const int key0 = t * kTile;
+    if ((CAUSAL && key0 + kTile - 1 > q0w) || (key0 + kTile > N)) {
+      const int lane = lane_now();
+      const int last = (CAUSAL ? min(q0w + (lane & 31), N - 1) : N - 1) - key0 - 4 * (lane >> 5);  // last key that counts
 #pragma unroll
-    for (int c16 = 0; c16 < 4; ++c16) {
+      for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-      for (int db = 0; db < G::kDBlocks; ++db) o[db] = mfma(swz_cols<D>(Vl, c16, db, v_off), pf[c16], o[db]);
+        for (int r = 0; r < 16; ++r)
+          if (acc_row(rb, r, 0) > last) s[rb][r] = -INFINITY;
     }
-    // LDS reads (two per MFMA) run kLead MFMAs ahead of their use.
-    constexpr int kN = 4 * G::kDBlocks, kLead = 4;
-    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kLead, 0);
-#pragma unroll
-    for (int n = 0; n < kN - kLead; ++n) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, kLead, 0);
   };
-
-  const bool first_group = wave < kFwdWaves / 2;
-  // Everything issued so far (Q rows, first copies) is waited for here, once,
-  // so that no wait for a register load is left to be placed inside the loop,
-  // where it would also wait for the copies in flight.
-  wait_vm<0>();
-  // Iteration j: K(j) sits in K slot j % 3, V(j-1) in V slot (j-1) % 3; K(j+2)
-  // is copied into K slot (j+2) % 3 and V(j+1) into V slot (j+1) % 3.
-  auto run = [&](auto group_tag) __attribute__((always_inline)) {
-    constexpr bool kFirst = decltype(group_tag)::value == 0;
-    int s0 = 0, s1 = 1, s2 = 2;  // j % 3, (j+1) % 3, (j+2) % 3
-    for (int j = 0; j <= nt; ++j) {
-      // K(j) and V(j-1) were issued two iterations ago; what the previous
-      // iteration issued (K(j+1), V(j)) may still be in flight.
-      if (j + 1 < nt) wait_vm<2 * kIPW>();
-      else if (j < nt) wait_vm<kIPW>();
-      else wait_vm<0>();
-      block_barrier();
-      if (j + 2 < nt) copy_tile(Kb, ks.n, c_kgoff, k_ring + s2 * T::kBytes, j + 2);
-      if (j + 1 < nt) copy_tile(Vb, vs.n, c_vgoff, v_ring + s1 * T::kBytes, j + 1);
-      const char* Kl = k_ring + s0 * T::kBytes;
-      const char* Vl = v_ring + s2 * T::kBytes;
-      if (kFirst) {
-        accumulate(Vl, j - 1);
-        if (j < nt) { scores(Kl, j); softmax(j); }
-      } else {
-        softmax(j - 1);
-        accumulate(Vl, j - 1);
-        if (j < nt) scores(Kl, j);
+  auto too_large = [&](float lt) __attribute__((always_inline)) {
+    return __builtin_amdgcn_ballot_w64(!(lt <= kRescaleSum)) != 0;
+  };
+  // probabilities of a tile with the running maximum brought up to date
+  auto raise_max = [&](const f16v (&s)[2]) __attribute__((always_inline)) {
+    float mx = s[0][0];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
+    mx = fmaxf(mx, other_half(mx));
+    const float mc_new = fmaxf(mc, mx * c);
+    const float alpha = fast_exp2(mc - mc_new);
+    mc = mc_new;
+    l_run *= alpha;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+    l_run += exponentials(s);
+  };
+  auto accumulate = [&](unsigned at) __attribute__((always_inline)) {
+    h8 frag[kLead];
+#pragma unroll
+    for (int n = 0; n < kLead; ++n) frag[n] = v_frag(at, n);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < kNP; ++n) {
+      o[n % kDB] = mfma(frag[n % kLead], __builtin_bit_cast(h8, pf[n / kDB]), o[n % kDB]);
+      if (n + kLead < kNP) frag[n % kLead] = v_frag(at, n + kLead);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // Iteration j uses K(j+1) and V(j-1), both in slot (j+1) & 1; K(j+2) and V(j) are copied into the other one.
+  auto top_wait = [&]() __attribute__((always_inline)) {
+    wait_vm<0>();
+    block_barrier();
+  };
+  auto top_copy = [&](int j, int slot) __attribute__((always_inline)) {
+    if (j + 2 < nt) copy_k(j + 2, slot);
+    if (j < nt) copy_v(j, slot);
+  };
+  // The pipelined step of tile j: softmax(j) with the MFMAs of accumulate(j-1) and scores(j+1) spread between its
+  // vector instructions.  Per 16 keys: kDB MFMAs of the accumulation, then as many of the scores.
+  auto step = [&](int j, auto slot_tag, const f16v (&s)[2], f16v (&sn)[2]) __attribute__((always_inline)) {
+    constexpr int kSlot = decltype(slot_tag)::value;  // (j + 1) & 1
+    constexpr unsigned at = kSlot * T::kBytes;
+    constexpr int kM = kNS + kNP;
+    h8 frag[kLead];
+    float l0 = 0.f, l1 = 0.f, p0 = 0.f, p1 = 0.f;
+    auto read = [&](int m) __attribute__((always_inline)) {
+      const int ch = m / (2 * kDB), in = m % (2 * kDB);
+      return in < kDB ? v_frag(at, ch * kDB + in) : k_frag(at, ch * kDB + in - kDB);
+    };
+    auto start = [&](int x) __attribute__((always_inline)) {
+      const int c16 = x >> 2, e = (x & 3) * 2;
+      p0 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e], c, -mc));
+      p1 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e + 1], c, -mc));
+    };
+    auto finish = [&](int x) __attribute__((always_inline)) {
+      const int c16 = x >> 2, e = (x & 3) * 2;
+      l0 += p0;
+      l1 += p1;
+      asm volatile("" : "+v"(l0), "+v"(l1));  // sums now, not all at the end
+      pf[c16][e >> 1] = pack_f16(p0, p1);
+    };
+    top_wait();
+#pragma unroll
+    for (int m = 0; m < kLead; ++m) frag[m] = read(m);
+    top_copy(j, 1 - kSlot);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < kM + 2; ++m) {
+      if (m < kM) {
+        const int ch = m / (2 * kDB), in = m % (2 * kDB);
+        if (in < kDB) {
+          o[in] = mfma(frag[m % kLead], __builtin_bit_cast(h8, pf[ch]), o[in]);
+        } else {
+          const int n = ch * kDB + in - kDB, rb = n & 1, kk = n >> 1;
+          sn[rb] = mfma(frag[m % kLead], qf[kk], kk == 0 ? zero : sn[rb]);
+        }
+        if (m + kLead < kM) frag[m % kLead] = read(m + kLead);
       }
-      const int t = s0; s0 = s1; s1 = s2; s2 = t;
+      if (D == 64) {
+        if (m >= 1 && m - 1 < 16) finish(m - 1);
+        if (m < 16) start(m);
+      } else {
+        if (m & 1) {
+          if (m >= 3 && m < 35) finish((m - 3) / 2);
+        } else if (m >= 2 && m < 34) {
+          start((m - 2) / 2);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    return l0 + l1;
   };
-  // Each group runs its own copy of the loop: no joins between the two
-  // orders inside the loop, so no register shuffling at branch merges.
-  if (first_group) run(IntTag<0>{});
-  else run(IntTag<1>{});
 
+  wait_vm<0>();  // Q rows and the first tiles: no wait for a register load is left to be placed in the loop
+  block_barrier();
+  if (ntw > 0) scores(0, sA);
+  int j = 0;
+  if (ntw > 1) {
+    top_wait();
+    top_copy(0, 0);
+    scores(T::kBytes, sB);
+    raise_max(sA);
+    ++j;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) sA[rb] = sB[rb];
+    // Main loop, two tiles per round, the scores alternating between two sets of registers: those of odd tiles in
+    // sA, of even ones in sB.  It is left where a tile's probabilities came out too large, so that what has to be
+    // done then costs it no registers.
+    bool odd_done = false;
+    for (;;) {
+      int why;
+      for (;;) {
+        if (!odd_done) {
+          if (j + 2 > ntw) { why = 0; break; }
+          const float lt = step(j, IntTag<0>{}, sA, sB);
+          if (too_large(lt)) { why = 1; break; }
+          l_run += lt;
+          ++j;
+        }
+        odd_done = false;
+        if (j + 2 > ntw) { why = 2; break; }
+        const float lt = step(j, IntTag<1>{}, sB, sA);
+        if (too_large(lt)) { why = 3; break; }
+        l_run += lt;
+        ++j;
+      }
+      if (why == 0) break;
+      if (why == 2) {
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) sA[rb] = sB[rb];
+        break;
+      }
+      if (why == 1) raise_max(sA);
+      else raise_max(sB);
+      ++j;
+      odd_done = why == 1;
+    }
+  }
+  // the wave's last tile (the one with a mask, if any) and the accumulation after it
+  for (; j <= nt; ++j) {
+    const unsigned at = ((j + 1) & 1) * T::kBytes;
+    top_wait();
+    top_copy(j, j & 1);
+    if (j > 0 && j <= ntw) accumulate(at);
+    if (j < ntw) {
+      mask(sA, j);
+      raise_max(sA);
+    }
+  }
+
+  block_barrier();  // every wave is done with the rings: they become the staging tiles
+  const int lane = lane_now(), qi = q0w + (lane & 31);
   const float l_tot = l_run + other_half(l_run);
   const float inv = 1.f / l_tot;
-  static_assert(kFwdWaves * StageGeom<D>::kBytes <= 2 * kRing * T::kBytes, "the output staging tiles fit the rings");
-  block_barrier();  // every wave is done with the rings: they become the staging tiles
   store_resident<D>(O + head_off, rs, q0w, N, o, inv, lane, smem + wave * StageGeom<D>::kBytes);
-  if (hh == 0 && qi < N) LSE[((long)b * H + h) * N + qi] = (m_run * c + __builtin_amdgcn_logf(l_tot)) * kLn2;
+  if (lane < 32 && qi < N) LSE[((long)b * H + h) * N + qi] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
 }
 
 // ---------------------------------------------------------------------------
@@ -1889,26 +2040,39 @@ bool bad_strides(const fused_mha_strides* st) {
   return st->seq >= (1 << 24) || st->head >= (1LL << 31);
 }
 
+// Whether the persistent 256-query forward takes a D = 128 problem of `total` such blocks: only where its static
+// shares come out even.  Without a mask all blocks weigh the same, so the last round of one block per CU has to be
+// nearly full (then it is 3-4 % faster than the 128-query kernel, whose K/V copies are twice as many; at 75 % full
+// already 14 % slower).  Under causal masking a work group's heavy block is paired with a light one, which comes out
+// even for exactly one pair of blocks per CU (3-6 % faster; hardware-scheduled small blocks are 13 % faster at 2.5
+// blocks per CU and 1-4 % at 8).
+bool persistent_forward_pays(int total, int n, bool causal) {
+  const int cus = (int)persistent_grid(1 << 30);
+  if (causal) return n >= 2048 && total <= 2 * cus && total * 16L >= 2 * cus * 15L;
+  const long rounds = (total + cus - 1) / cus;
+  return total * 16L >= rounds * cus * 15L;
+}
+
 template <int D, bool CAUSAL>
 int launch_forward(const void* q, const void* k, const void* v, Strides qs, Strides ks, Strides vs, void* o, void* lse,
                    int batch, int head, int n, float scale, hipStream_t stream) {
-  const int nmb = (n + kFwdBlockQ - 1) / kFwdBlockQ;
-  const int total = nmb * batch * head;
-  const unsigned grid = persistent_grid(total);
   // scale == 0 would turn the masked scores (-inf) into NaN when multiplied; a
   // tiny positive factor gives the same uniform softmax and keeps -inf * c = -inf.
   const float c = fmaxf(fabsf(scale) * kLog2e, 1e-30f);
-  if constexpr (D == 64) {
-    if (!CAUSAL || n <= kFwdBlockKernelMaxN) {  // see fmha_fwd_block_kernel
-      const hipError_t rc = launch(fmha_fwd_block_kernel<D, CAUSAL>, (unsigned)total, kFwdThreads, stream,
+  const int negate = scale < 0.f ? 1 : 0;
+  if constexpr (D == 128) {
+    const int nmb = (n + kFwdBlockQ - 1) / kFwdBlockQ, total = nmb * batch * head;
+    if (persistent_forward_pays(total, n, CAUSAL)) {
+      const hipError_t rc = launch(fmha_fwd_kernel<D, CAUSAL>, persistent_grid(total), kFwdThreads, stream,
                                    (const half_t*)q, (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o,
-                                   (float*)lse, head, n, nmb, c, scale < 0.f ? 1 : 0);
+                                   (float*)lse, head, n, nmb, total, c, negate);
       return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
     }
   }
-  const hipError_t rc = launch(fmha_fwd_kernel<D, CAUSAL>, grid, kFwdThreads, stream, (const half_t*)q,
-                               (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, total, c,
-                               scale < 0.f ? 1 : 0);
+  const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ, total = nmb * batch * head;
+  const hipError_t rc = launch(fmha_fwd_pipe_kernel<D, CAUSAL>, (unsigned)total, kPipeThreads, stream, (const half_t*)q,
+                               (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, c,
+                               negate);
   return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
 }
 

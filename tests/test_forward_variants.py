@@ -1,0 +1,90 @@
+"""The forward's work-group order, on the CPU, and its two kernels at the sizes where they can go wrong, on the GPU."""
+import os
+import subprocess
+
+import pytest
+import torch
+
+import abi
+from oracle import attention_oracle as ao
+
+
+def test_scheduled_blocks_are_a_bijection(tmp_path):
+    """csrc/block_map.h, compiled for the host: every (slice, block) once for any slice count, whole slices on one XCD
+    up to slices % 8 of them, and (heavy_first) block indices that never fall inside a group of slices."""
+    src = tmp_path / "check.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (int slices = 1; slices <= 300; slices += (slices < 150 ? 1 : 7))
+    for (int bps : {1, 2, 3, 5, 8, 12, 33})
+      for (int mode = 0; mode < 3; ++mode) {
+        const bool heavy = mode == 0, short_last = mode == 1;
+        const int total = slices * bps;
+        std::vector<int> seen(total, 0), xcd(slices, -1);
+        int prev = 0, drops = 0;
+        for (int lin = 0; lin < total; ++lin) {
+          int s = -1, b = -1;
+          fmha_scheduled_block(lin, slices, bps, heavy, short_last, s, b);
+          if (s < 0 || s >= slices || b < 0 || b >= bps || seen[s * bps + b]++) { printf("map %d %d %d %d\n", slices, bps, mode, lin); return 1; }
+          if (heavy && s < (slices & ~7)) {
+            if (xcd[s] >= 0 && xcd[s] != (lin & 7)) { printf("xcd %d %d\n", slices, bps); return 1; }
+            xcd[s] = lin & 7;
+          }
+          if (short_last && (b == bps - 1) != (lin >= slices * (bps - 1))) { printf("short %d %d\n", slices, bps); return 1; }
+          drops += heavy && b < prev;
+          prev = b;
+        }
+        if (heavy && drops > slices / 64) { printf("order %d %d\n", slices, bps); return 1; }
+      }
+  puts("ok");
+  return 0;
+}
+''')
+    exe = tmp_path / "check"
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
+def _inputs(B, N, H, D, growing):
+    """growing: the score scale rises with the key index, so that nearly every 64-key tile holds a maximum that is
+    more than 2^12 times (12 in the exp2 domain) above the earlier ones and the running maximum is raised in it."""
+    q, k, v, _ = ao.make_inputs(B, N, H, D, seed=7)
+    if growing:
+        q = q.abs() * 0.25
+        k = (k.abs() * 0.5 + torch.arange(N).view(1, N, 1, 1) // 64 * (60.0 / D)).half()
+        q = q.half()
+    return q, k, v
+
+
+def _check(B, N, H, D, causal, growing, heads=None):
+    q, k, v = _inputs(B, N, H, D, growing)
+    out, lse = abi.forward(abi.load(), q.cuda(), k.cuda(), v.cuda(), D ** -0.5 if not growing else 1.0, causal)
+    assert torch.isfinite(out).all() and torch.isfinite(lse).all()
+    pick = list(range(H)) if heads is None else heads
+    ref, ref_lse = ao.attention_forward(q[:, :, pick], k[:, :, pick], v[:, :, pick],
+                                        D ** -0.5 if not growing else 1.0, causal)
+    # the repository's bounds: fp16 probabilities and results for O of order 1, fp32 sums for the logsumexp (relative
+    # to its size: a score of size s carries the fp32 rounding of D products of size s, below 2^-20 s)
+    assert (out[:, :, pick].float().cpu() - ref.half().float()).abs().max() <= 2e-3 * max(1.0, ref.abs().max().item())
+    assert ((lse[:, pick].cpu() - ref_lse).abs() <= 2e-3 + 1e-6 * ref_lse.abs()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 32, 33, 64, 65, 96, 128, 129, 192, 193, 256, 257, 320, 449])
+def test_small_blocks(N, causal, D):
+    for growing in (False, True):
+        _check(1, N, 3, D, causal, growing)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,causal", [(5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True)])
+def test_persistent_blocks(B, H, N, causal):
+    """255 and 256 blocks of 256 queries without a mask, 504 with one: the launches the persistent kernel takes."""
+    for growing in (False, True):
+        _check(B, N, H, 128, causal, growing, heads=[0, H // 2, H - 1])
