@@ -179,7 +179,9 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
 
   const Operand qo = operand(q), ko = operand(k), vo = operand(v), go = operand(dout);
   at::Tensor od = dense(out), ld = dense(lse);
-  const size_t ws_bytes = fused_mha_backward_workspace_bytes(batch_size, num_heads, seqlen_q, head_size);
+  // head size 64 makes no use of room for dS
+  const size_t ws_bytes = (head_size == 64 ? fused_mha_backward_min_workspace_bytes : fused_mha_backward_workspace_bytes)(
+      batch_size, num_heads, seqlen_q, head_size);
   auto workspace = torch::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte));
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
   check_rc(fused_mha_backward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,

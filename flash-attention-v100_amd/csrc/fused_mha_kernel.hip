@@ -34,6 +34,7 @@
 #include <math.h>
 #include <mutex>
 #include <tuple>
+#include <utility>
 
 #include "fused_mha.h"
 #include "block_map.h"
@@ -77,9 +78,11 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // fp32, multiplying and converting back, in 2 instructions instead of 5).
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ unsigned neg_mul_to_f16x2(unsigned p_pair, float x0, float x1) {
-  unsigned r = 0;
-  asm("v_fma_mixlo_f16 %0, %1, -%2, 0 op_sel_hi:[1,0,0]" : "+v"(r) : "v"(p_pair), "v"(x0));
-  asm("v_fma_mixhi_f16 %0, %1, -%2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(r) : "v"(p_pair), "v"(x1));
+  unsigned r;
+  asm("v_fma_mixlo_f16 %0, %1, -%2, 0 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %0, %1, -%3, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+      : "=&v"(r)
+      : "v"(p_pair), "v"(x0), "v"(x1));
   return r;
 }
 // y[.] = fp16(-p[.] * x[.]) for the 8 values of one B-operand fragment
@@ -341,6 +344,15 @@ __device__ __forceinline__ void wait_vm_tiles(int later) {
 }
 template <int V>
 struct IntTag { static constexpr int value = V; };
+// f(IntTag<0>{}), f(IntTag<1>{}), .. f(IntTag<kN - 1>{}): unrolled whatever the size of the body.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_each(std::integer_sequence<int, I...>, F&& f) {
+  (f(IntTag<I>{}), ...);
+}
+template <int kN, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_each(std::make_integer_sequence<int, kN>{}, f);
+}
 
 // 16 bytes per lane to p + kOffset bytes, with the non-temporal hint (data that is read once, by a later
 // kernel).  Inline asm because the compiler keeps the hint only on the first of several stores that share
@@ -744,6 +756,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 constexpr int kPipeWaves = 4;
 constexpr int kPipeThreads = kPipeWaves * 64;
 constexpr int kPipeBlockQ = kPipeWaves * kResident;
+constexpr int kPipeBlockKeys = kPipeWaves * kResident;  // of the dK/dV pass
 // kCount copies of 1 KiB to consecutive blocks of LDS: lane l's 16 bytes of block u land at lds + 1024 * u + 16 * l.
 // The instruction's offset counts for both addresses, so they come from base + voff + 64 * u with voff lowered by
 // 960 * u.
@@ -1394,6 +1407,243 @@ fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, c
 }
 
 // ---------------------------------------------------------------------------
+// Backward for D = 64: a dQ pass and a dK/dV pass that both form S and dP themselves, 4 waves of 32 resident rows per
+// block, two blocks per CU, everything of a wave's rows inside that wave.
+//
+// At D = 64 writing and reading dS costs more than forming it twice: 4 bytes of HBM traffic per element against 256
+// FLOP, and the wave-pair kernels behind it (probabilities handed over through LDS, one block per CU) were bound by
+// latency.  Here, as in fmha_fwd_pipe_kernel, a wave's instruction stream interleaves the MFMAs of one step with the
+// vector instructions of its neighbours, in units of one MFMA whose order is pinned.  us at B16 H12 N512 / B4 H16 N1024
+// causal / B16 H16 N1024 / B4 H16 N4096 causal, against the wave-pair kernels over and without dS:
+//   dQ pass     30 / 24 / 148 / 240   (22 / 18 / 106 / 217 plus delta pass 7 / 5 / 17 / 17; 40 / 38 / 172 / 315)
+//   dK/dV pass  34 / 28 / 178 / 300   (45 / 44 / 275 / 455;                                 45 / 45 / 205 / 385)
+// What bounds them: the issue of one instruction every 4-5 cycles per wave in small problems, the power limit (clock at
+// 1.9 GHz) in large ones.  64 keys per wave with one wave per SIMD halves the LDS reads per MFMA but is slower or
+// equal everywhere (43 / 36 / 179 / 310): a lone wave cannot cover its own issue gaps.
+//
+// dQ pass.  The formulas are those of fmha_bwd_dq_kernel, and so are the results, bit for bit.
+// ---------------------------------------------------------------------------
+template <bool CAUSAL, bool STATS>
+__global__ void __launch_bounds__(kPipeThreads, 2)
+fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                        const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
+                        Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
+                        half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+  constexpr int D = 64;
+  using G = TileGeom<D>;
+  using T = SwzTile<D>;
+  constexpr int kDB = G::kDBlocks, kKS = G::kKSteps;
+  constexpr int kIPW = T::kInstrs / kPipeWaves;
+  static_assert(kIPW == T::kNC, "a wave copies the 16 rows of one block row of a tile");
+  constexpr int kSlots = 3;  // K tiles, then V tiles: the current one, the one before it, the one being copied
+  constexpr int kVOff = kSlots * T::kBytes;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * kSlots * T::kBytes];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 31, hh = lane >> 5;
+  int bh, mb;
+  fmha_scheduled_block(blockIdx.x, gridDim.x / nmb, nmb, CAUSAL, N % kPipeBlockQ != 0, bh, mb);
+  const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
+  const int b = bh / H, h = bh - b * H;
+  const int rs = H * D;  // O and dQ are dense
+  const long head_off = ((long)b * N * H + h) * D;
+  const int m0 = mblk * kPipeBlockQ;
+  const int q0w = m0 + wave * kResident;
+  const int qi = q0w + i, qrow = min(qi, N - 1);
+
+  const int nt_all = (N + kTile - 1) / kTile;
+  int nt = nt_all, ntw = q0w < N ? nt_all : 0;  // tiles the block streams; tiles this wave works on
+  if (CAUSAL) {
+    nt = min(nt, (min(m0 + kPipeBlockQ, N) - 1) / kTile + 1);
+    ntw = q0w < N ? min(nt, (min(q0w + kResident, N) - 1) / kTile + 1) : 0;
+  }
+
+  // tile copies as in fmha_fwd_pipe_kernel
+  constexpr int kBack = 960 * (kIPW - 1);
+  int k_goff, v_goff, c_past;
+  {
+    const int row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ (lane >> 4)) * 16;
+    k_goff = row * ks.n * 2 + col + kBack;
+    v_goff = row * vs.n * 2 + col + kBack;
+    c_past = max((nt_all - 1) * kTile + row - (N - 1), 0) * 2;
+  }
+  const half_t* kp = K + b * ks.b + (long)h * ks.h - kBack / 2;  // the next tile to copy
+  const half_t* vp = V + b * vs.b + (long)h * vs.h - kBack / 2;
+  const unsigned lds_w = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * (kIPW * 1024);
+  auto copy_tile = [&](int tile, int slot) __attribute__((always_inline)) {
+    if (tile == nt_all - 1) {
+      k_goff -= c_past * ks.n;
+      v_goff -= c_past * vs.n;
+    }
+    copy16_blocks<kIPW>(kp, k_goff, lds_w + slot * T::kBytes);
+    copy16_blocks<kIPW>(vp, v_goff, lds_w + kVOff + slot * T::kBytes);
+    kp += (long)kTile * ks.n;
+    vp += (long)kTile * vs.n;
+  };
+  copy_tile(0, 0);
+
+  // Resident rows and the row statistics.  dO is negated: its product with V on top of delta gives delta - dP.
+  h8 qf[kKS], gf[kKS];
+  float my_lse2, my_delta;
+  {
+    const half_t* qp = Q + b * qs.b + (long)h * qs.h + (long)qrow * qs.n + hh * 8;
+    const half_t* gp = dO + b * gs.b + (long)h * gs.h + (long)qrow * gs.n + hh * 8;
+    const long stat_at = ((long)b * H + h) * N + qrow;
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) {
+      qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
+      gf[kk] = *reinterpret_cast<const h8*>(gp + kk * 16);
+    }
+    my_lse2 = LSE[stat_at] * kLog2e;
+    if (STATS) {
+      // partial sums combined in the order of fmha_bwd_delta_kernel's shuffle tree: the same bits
+      const half_t* op = O + head_off + (long)qrow * rs + hh * 8;
+      float part[kKS];
+#pragma unroll
+      for (int kk = 0; kk < kKS; ++kk) {
+        const h8 ov = *reinterpret_cast<const h8*>(op + kk * 16);
+        part[kk] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part[kk] = fmaf((float)ov[e], (float)gf[kk][e], part[kk]);
+      }
+#pragma unroll
+      for (int stride = kKS / 2; stride > 0; stride >>= 1)
+#pragma unroll
+        for (int kk = 0; kk < stride; ++kk) part[kk] += part[kk + stride];
+      my_delta = part[0] + other_half(part[0]);
+      if (hh == 0 && qi < N) {
+        delta[stat_at] = my_delta;
+        lse2[stat_at] = my_lse2;
+      }
+    } else {
+      my_delta = delta[stat_at];
+    }
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) {
+      gf[kk] = -gf[kk];
+      asm volatile("" : "+v"(gf[kk]));  // negated here, not in the loop
+    }
+  }
+
+  int r_off[2], c_off[2];
+  swz_rows_off<D>(lane, r_off);
+  swz_cols_off<D>(lane, c_off);
+  // fragment addresses: rows in the slot of the current tile, columns in that of the tile before it
+  unsigned ra0 = opaque_lds_address(smem + r_off[0]), ra1 = opaque_lds_address(smem + r_off[1]);
+  unsigned ca0 = opaque_lds_address(smem + c_off[0]), ca1 = opaque_lds_address(smem + c_off[1]);
+
+  f16v dq[kDB], s[2], x[2], dl, zero;
+  u4v p[4], y[4];  // probabilities and dS of a tile, fp16 pairs in B-operand order
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    dl[r] = my_delta;
+    zero[r] = 0.f;
+    x[0][r] = x[1][r] = 0.f;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db) dq[db][r] = 0.f;
+  }
+#pragma unroll
+  for (int c16 = 0; c16 < 4; ++c16) p[c16] = y[c16] = u4v{0, 0, 0, 0};
+
+  constexpr int kLead = 3;
+  auto ds_pair = [&](int n) __attribute__((always_inline)) {  // pair n of 16: two neighbouring keys
+    const int c16 = n >> 2, e = (n & 3) * 2, rb = c16 >> 1, r = (c16 & 1) * 8 + e;
+    y[c16][e >> 1] = neg_mul_to_f16x2(p[c16][e >> 1], x[rb][r], x[rb][r + 1]);
+  };
+  // dQ^T += K^T dS^T, MFMA n of 8
+  auto dq_mfma = [&](h8 frag, int n) __attribute__((always_inline)) {
+    dq[n % kDB] = mfma(frag, __builtin_bit_cast(h8, y[n / kDB]), dq[n % kDB]);
+  };
+  // Tile j in 24 units of one MFMA and what is issued in its shadow:
+  //   0.. 7  S^T(j) = K(j) Q^T                     dS(j-1) = P o (dP - delta)
+  //   8..15  delta - dP^T(j) = delta - V(j) dO^T   P(j) = exp2(S c - lse2), from unit 10 (S complete) to 23
+  //  16..23  dQ^T += K(j-1)^T dS(j-1)^T
+  // so that no vector instruction waits for an MFMA of its own tile just issued, nor the other way round.
+  auto tile = [&](int j, auto masked_tag) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value != 0;
+    h8 frag[kLead];
+    const int last = (CAUSAL ? min(qi, N - 1) : N - 1) - j * kTile - 4 * hh;  // last key that counts
+    auto p_pair = [&](int n) __attribute__((always_inline)) {
+      const int c16 = n >> 2, e = (n & 3) * 2, rb = c16 >> 1, r = (c16 & 1) * 8 + e;
+      float p0 = fast_exp2(fmaf(s[rb][r], c, -my_lse2));
+      float p1 = fast_exp2(fmaf(s[rb][r + 1], c, -my_lse2));
+      if (MASKED) {
+        if (acc_row(rb, r, 0) > last) p0 = 0.f;
+        if (acc_row(rb, r + 1, 0) > last) p1 = 0.f;
+      }
+      p[c16][e >> 1] = pack_f16(p0, p1);
+    };
+    auto read = [&](int m) __attribute__((always_inline)) {
+      const int n = m % 8;
+      if (m < 8) return swz_rows_at<D>(ra0, ra1, n & 1, n >> 1);
+      if (m < 16) return swz_rows_at<D>(ra0 + kVOff, ra1 + kVOff, n & 1, n >> 1);
+      return swz_cols_at<D>(ca0, ca1, n / kDB, n % kDB);
+    };
+#pragma unroll
+    for (int m = 0; m < kLead; ++m) frag[m] = read(m);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<24>([&](auto m_tag) __attribute__((always_inline)) {
+      constexpr int m = decltype(m_tag)::value, n = m % 8;
+      if constexpr (m < 8) s[n & 1] = mfma(frag[m % kLead], qf[n >> 1], n < 2 ? zero : s[n & 1]);
+      else if constexpr (m < 16) x[n & 1] = mfma(frag[m % kLead], gf[n >> 1], n < 2 ? dl : x[n & 1]);
+      else dq_mfma(frag[m % kLead], n);
+      if constexpr (m + kLead < 24) frag[m % kLead] = read(m + kLead);
+      if constexpr (m < 8) {
+        ds_pair(2 * m);
+        ds_pair(2 * m + 1);
+      }
+      if constexpr (m >= 10) {
+        p_pair(m - 10);
+        if constexpr (m >= 22) p_pair(m - 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
+  wait_vm<0>();  // resident rows and the first tile: no wait for a register load is left to be placed in the loop
+  int slot = 0, next_slot = 1;
+  auto top = [&](int j) __attribute__((always_inline)) {
+    wait_vm<0>();
+    block_barrier();
+    if (j + 1 < nt) copy_tile(j + 1, next_slot);
+  };
+  auto next = [&](int j) __attribute__((always_inline)) {
+    const int step = (next_slot - slot) * T::kBytes;
+    ra0 += step, ra1 += step;
+    if (j > 0) {
+      const int cstep = (slot == 0 ? -(kSlots - 1) : 1) * T::kBytes;
+      ca0 += cstep, ca1 += cstep;
+    }
+    slot = next_slot;
+    next_slot = next_slot == kSlots - 1 ? 0 : next_slot + 1;
+  };
+  int j = 0;
+  for (; j + 1 < ntw; ++j) {
+    top(j);
+    tile(j, IntTag<0>{});
+    next(j);
+  }
+  if (ntw > 0) {  // the wave's last tile, the only one that can need a mask, and what is left of it
+    top(j);
+    tile(j, IntTag<1>{});
+    next(j);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) ds_pair(n);
+#pragma unroll
+    for (int n = 0; n < 8; ++n) dq_mfma(swz_cols_at<D>(ca0, ca1, n / kDB, n % kDB), n);
+    ++j;
+  }
+  for (; j < nt; ++j) {
+    top(j);
+    next(j);
+  }
+
+  block_barrier();  // every wave is done with the rings: they become the staging tiles
+  store_resident<D>(dQ + head_off, rs, q0w, N, dq, scale, lane, smem + wave * StageGeom<D>::kBytes);
+}
+
+// ---------------------------------------------------------------------------
 // Backward, dK/dV pass.  Block = 128 keys = 4 pairs of waves; a pair owns 32
 // keys and splits the work so that each wave keeps only one accumulator and one
 // of K / V in registers (two waves per SIMD fit):
@@ -1715,6 +1965,240 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   char* const stage = smem + wave * StageGeom<D>::kBytes;
   if (!role_b) store_resident<D>(dV + head_off, rs, k0w, N, acc, 1.f, lane, stage);
   else store_resident<D>(dK + head_off, rs, k0w, N, acc, scale, lane, stage);
+}
+
+// ---------------------------------------------------------------------------
+// Backward, dK/dV pass for D = 64 (see fmha_bwd_dq_pipe_kernel).  Formulas and results are those of fmha_bwd_dkdv_kernel.
+// A 64-query tile is worked on in two halves of 32 queries; the accumulation into dV and dK of a half runs during the
+// next one, so Q and dO have three slots: the tile before, the current one, the one being copied.
+// ---------------------------------------------------------------------------
+template <bool CAUSAL>
+__global__ void __launch_bounds__(kPipeThreads, 2)
+fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                          const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                          const float* __restrict__ delta, const float* __restrict__ lse2, half_t* __restrict__ dK,
+                          half_t* __restrict__ dV, int H, int N, int nnb, float c, float scale) {
+  constexpr int D = 64;
+  using G = TileGeom<D>;
+  using T = SwzTile<D>;
+  constexpr int kDB = G::kDBlocks, kKS = G::kKSteps;
+  constexpr int kIPW = T::kInstrs / kPipeWaves;
+  constexpr int kSlots = 3;                               // the current tile, the one before it, the one being copied
+  constexpr int kGOff = kSlots * T::kBytes, kStOff = 2 * kSlots * T::kBytes;
+  constexpr int kStBytes = 512;                           // 64 lse2 then 64 delta values
+  __shared__ __attribute__((aligned(1024))) char smem[kStOff + kSlots * kStBytes];
+  static_assert(kPipeWaves * StageGeom<D>::kBytes <= kStOff, "the output staging tiles fit the rings");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 31, hh = lane >> 5;
+  int bh, nblk;
+  fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kPipeBlockKeys != 0, bh, nblk);
+  const int b = bh / H, h = bh - b * H;                   // causal: low key blocks are the heavy ones and come first
+  const int rs = H * D;                                   // dK and dV are dense
+  const long head_off = ((long)b * N * H + h) * D;
+  const int n0 = nblk * kPipeBlockKeys;
+  const int k0w = n0 + wave * kResident, ki = k0w + i, krow = min(ki, N - 1);
+
+  const int nt = (N + kTile - 1) / kTile;
+  const int t_begin = CAUSAL ? n0 / kTile : 0;
+  // tiles this wave works on: from the one with the first query that sees a key of it
+  const int t_active = k0w < N ? (CAUSAL ? k0w / kTile : 0) : nt;
+
+  // tile copies as in fmha_fwd_pipe_kernel
+  constexpr int kBack = 960 * (kIPW - 1);
+  int q_goff, g_goff, c_past;
+  {
+    const int row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ (lane >> 4)) * 16;
+    q_goff = row * qs.n * 2 + col + kBack;
+    g_goff = row * gs.n * 2 + col + kBack;
+    c_past = max((nt - 1) * kTile + row - (N - 1), 0) * 2;
+  }
+  const half_t* qp = Q + b * qs.b + (long)h * qs.h + (long)t_begin * kTile * qs.n - kBack / 2;  // next tile to copy
+  const half_t* gp = dO + b * gs.b + (long)h * gs.h + (long)t_begin * kTile * gs.n - kBack / 2;
+  const float* const stat = (wave == 0 ? lse2 : delta) + ((long)b * H + h) * N;
+  const unsigned lds_w = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * (kIPW * 1024);
+  auto copy_tile = [&](int t, int slot) __attribute__((always_inline)) {
+    if (t == nt - 1) {
+      q_goff -= c_past * qs.n;
+      g_goff -= c_past * gs.n;
+    }
+    copy16_blocks<kIPW>(qp, q_goff, lds_w + slot * T::kBytes);
+    copy16_blocks<kIPW>(gp, g_goff, lds_w + kGOff + slot * T::kBytes);
+    qp += (long)kTile * qs.n;
+    gp += (long)kTile * gs.n;
+    if (wave < 2) copy4(stat, min(t * kTile + lane, N - 1) * 4, smem + kStOff + slot * kStBytes + wave * 256);
+  };
+  copy_tile(t_begin, 0);
+
+  // resident rows: K, and V negated, so that the dP product on top of delta gives delta - dP
+  h8 kf[kKS], vf[kKS];
+  {
+    const half_t* kp = K + b * ks.b + (long)h * ks.h + (long)krow * ks.n + hh * 8;
+    const half_t* vp = V + b * vs.b + (long)h * vs.h + (long)krow * vs.n + hh * 8;
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) {
+      kf[kk] = *reinterpret_cast<const h8*>(kp + kk * 16);
+      vf[kk] = *reinterpret_cast<const h8*>(vp + kk * 16);
+    }
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) {
+      vf[kk] = -vf[kk];
+      asm volatile("" : "+v"(vf[kk]));  // negated here, not in the loop
+    }
+  }
+
+  int r_off[2], c_off[2];
+  swz_rows_off<D>(lane, r_off);
+  swz_cols_off<D>(lane, c_off);
+  // fragment addresses in the slot of the current tile, and of columns in that of the tile before it
+  unsigned ra0 = opaque_lds_address(smem + r_off[0]), ra1 = opaque_lds_address(smem + r_off[1]);
+  unsigned ca0 = opaque_lds_address(smem + c_off[0]), ca1 = opaque_lds_address(smem + c_off[1]);
+  unsigned pa0 = ca0, pa1 = ca1;
+  unsigned st0 = opaque_lds_address(smem + kStOff + hh * 16);
+
+  f16v dv[kDB], dk[kDB], s, x[2], zero;
+  u4v p[2], y[2];  // [16 queries]: probabilities and dS, fp16 pairs in B-operand order
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    zero[r] = x[0][r] = x[1][r] = 0.f;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db) dv[db][r] = dk[db][r] = 0.f;
+  }
+#pragma unroll
+  for (int cc = 0; cc < 2; ++cc) p[cc] = y[cc] = u4v{0, 0, 0, 0};
+
+  auto ds_pair = [&](int n, const f16v& xx) __attribute__((always_inline)) {  // pair n of 8: two neighbouring queries
+    const int cc = n >> 2, e = (n & 3) * 2, r = cc * 8 + e;
+    y[cc][e >> 1] = neg_mul_to_f16x2(p[cc][e >> 1], xx[r], xx[r + 1]);
+  };
+  auto dv_mfma = [&](h8 frag, int n) __attribute__((always_inline)) {
+    dv[n % kDB] = mfma(frag, __builtin_bit_cast(h8, p[n / kDB]), dv[n % kDB]);
+  };
+  auto dk_mfma = [&](h8 frag, int n) __attribute__((always_inline)) {
+    dk[n % kDB] = mfma(frag, __builtin_bit_cast(h8, y[n / kDB]), dk[n % kDB]);
+  };
+  // columns of the half before the one with rows 32 hq .. of the current tile
+  auto cols_before = [&](int hq, unsigned at, int n) __attribute__((always_inline)) {
+    return hq == 0 ? swz_cols_at<D>(pa0 + at, pa1 + at, 2 + n / kDB, n % kDB)
+                   : swz_cols_at<D>(ca0 + at, ca1 + at, n / kDB, n % kDB);
+  };
+
+  constexpr int kLead = 4;
+  // Half a tile (32 queries, rows 32 hq ..) in 16 units of one MFMA and what is issued in its shadow:
+  //   0.. 7  S = Q K^T and delta - dP = delta - dO V^T in turn      dS = P o (dP - delta) of the half before
+  //   8..11  dV^T += dO^T P of the half before                      P = exp2(S c - lse2), from unit 10
+  //  12..15  dK^T += Q^T dS of the half before
+  auto half = [&](int t, auto hq_tag, auto masked_tag) __attribute__((always_inline)) {
+    constexpr int hq = decltype(hq_tag)::value;
+    constexpr bool MASKED = decltype(masked_tag)::value != 0;
+    typedef __attribute__((address_space(3))) f4v lds_f4;
+    h8 frag[kLead];
+    f16v dl;
+    f4v ls[4];
+    auto read = [&](int m) __attribute__((always_inline)) {
+      if (m < 8) return swz_rows_at<D>(ra0 + (m & 1) * kGOff, ra1 + (m & 1) * kGOff, hq, m >> 1);
+      if (m < 12) return cols_before(hq, kGOff, m - 8);
+      return cols_before(hq, 0, m - 12);
+    };
+    auto p_pair = [&](int n) __attribute__((always_inline)) {
+      const int cc = n >> 2, e = (n & 3) * 2, r = cc * 8 + e;
+      float p0 = fast_exp2(fmaf(s[r], c, -ls[r >> 2][r & 3]));
+      float p1 = fast_exp2(fmaf(s[r + 1], c, -ls[r >> 2][(r & 3) + 1]));
+      if (MASKED) {
+        const int q = t * kTile + acc_row(hq, r, hh);
+        if ((CAUSAL && ki > q) || q >= N) p0 = 0.f;
+        if ((CAUSAL && ki > q + 1) || q + 1 >= N) p1 = 0.f;
+      }
+      p[cc][e >> 1] = pack_f16(p0, p1);
+    };
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f4v d4 = *(const lds_f4*)(uintptr_t)(st0 + 256 + hq * 128 + 32 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dl[4 * g + e] = d4[e];
+    }
+#pragma unroll
+    for (int m = 0; m < kLead; ++m) frag[m] = read(m);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<16>([&](auto m_tag) __attribute__((always_inline)) {
+      constexpr int m = decltype(m_tag)::value;
+      if constexpr (m < 8) {
+        if constexpr (m % 2 == 0) s = mfma(frag[m % kLead], kf[m / 2], m == 0 ? zero : s);
+        else x[hq] = mfma(frag[m % kLead], vf[m / 2], m == 1 ? dl : x[hq]);
+      } else if constexpr (m < 12) {
+        dv_mfma(frag[m % kLead], m - 8);
+      } else {
+        dk_mfma(frag[m % kLead], m - 12);
+      }
+      if constexpr (m + kLead < 16) frag[m % kLead] = read(m + kLead);
+      if constexpr (m < 8) {
+        ds_pair(m, x[hq ^ 1]);
+        if constexpr (m % 2 == 0) ls[m / 2] = *(const lds_f4*)(uintptr_t)(st0 + hq * 128 + 16 * m);
+      }
+      // P of queries 0..15 after the last reader of the half before's (unit 9), of queries 16..31 after unit 11
+      if constexpr (m == 10 || m == 11) p_pair(m - 10);
+      if constexpr (m == 12 || m == 13) {
+        p_pair(2 * m - 22);
+        p_pair(2 * m - 21);
+      }
+      if constexpr (m >= 14) p_pair(m - 8);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
+  wait_vm<0>();
+  int slot = 0, next_slot = 1, t = t_begin;
+  auto top = [&]() __attribute__((always_inline)) {
+    wait_vm<0>();
+    block_barrier();
+    if (t + 1 < nt) copy_tile(t + 1, next_slot);
+  };
+  auto next = [&]() __attribute__((always_inline)) {
+    const int step = next_slot - slot;
+    if (t >= t_active) pa0 = ca0, pa1 = ca1;
+    ra0 += step * T::kBytes, ra1 += step * T::kBytes, ca0 += step * T::kBytes, ca1 += step * T::kBytes;
+    if (t < t_active) pa0 = ca0, pa1 = ca1;  // the first tile worked on: P and dS before it are zero, any rows will do
+    st0 += step * kStBytes;
+    slot = next_slot;
+    next_slot = next_slot == kSlots - 1 ? 0 : next_slot + 1;
+    ++t;
+  };
+  // The wave's tiles in order: not seen by its keys (copies only), then spans of masked tiles (on the diagonal, at the
+  // end of the sequence) and of unmasked ones, each in a loop of its own so that no accumulator crosses a branch.
+  const int t_diag = CAUSAL ? t_active + 1 : 0;  // first tile below the diagonal
+  const int nt_full = N / kTile;                 // tiles without rows past the end
+  while (t < min(t_active, nt)) {
+    top();
+    next();
+  }
+  while (t < nt) {
+    while (t < nt && (t < t_diag || t >= nt_full)) {
+      top();
+      half(t, IntTag<0>{}, IntTag<1>{});
+      half(t, IntTag<1>{}, IntTag<1>{});
+      next();
+    }
+    while (t >= t_diag && t < nt_full) {
+      top();
+      half(t, IntTag<0>{}, IntTag<0>{});
+      half(t, IntTag<1>{}, IntTag<0>{});
+      next();
+    }
+  }
+  if (t_active < nt) {  // what is left of the last half
+#pragma unroll
+    for (int n = 0; n < 8; ++n) ds_pair(n, x[1]);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) dv_mfma(cols_before(0, kGOff, n), n);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) dk_mfma(cols_before(0, 0, n), n);
+  }
+
+  block_barrier();  // every wave is done with the rings: they become the staging tiles
+  char* const stage = smem + wave * StageGeom<D>::kBytes;
+  store_resident<D>(dV + head_off, rs, k0w, N, dv, 1.f, lane, stage);
+  store_resident<D>(dK + head_off, rs, k0w, N, dk, scale, lane, stage);
 }
 
 // ---------------------------------------------------------------------------
@@ -2110,6 +2594,7 @@ template <int D, bool CAUSAL>
 int launch_backward(int passes, bool spill, const void* q, const void* k, const void* v, const void* o,
                     const void* d_o, Strides qs, Strides ks, Strides vs, Strides gs, const void* lse, float* delta,
                     void* dq, void* dk, void* dv, int batch, int head, int n, float scale, hipStream_t stream) {
+  if (D == 64) spill = false;  // see fmha_bwd_dq_pipe_kernel
   // Without the spill and with all three passes asked for, the dQ pass produces delta and lse2 itself.
   const bool dq_makes_stats = !spill && (passes & kPassAll) == kPassAll;
   float* lse2 = delta + (long)batch * head * n;
@@ -2124,28 +2609,43 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
   }
   const float c = scale * kLog2e;
   auto dq_pass = [&]() {
-    if (spill) {
-      // two panels per block when that leaves every work group at least two blocks (a heavy and a light one)
-      const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * batch * head;
-      if (total2 >= 2 * persistent_grid(total2))
-        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, persistent_grid(total2), ds_threads(2), stream,
-                      (const half_t*)k, ks, (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, scale);
-      const int nqb = np / kDsPanelQ, total = nqb * batch * head;
-      return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, persistent_grid(total), ds_threads(1), stream,
-                    (const half_t*)k, ks, (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, scale);
+    if constexpr (D == 64) {
+      const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ;
+      auto kernel = dq_makes_stats ? fmha_bwd_dq_pipe_kernel<CAUSAL, true> : fmha_bwd_dq_pipe_kernel<CAUSAL, false>;
+      return launch(kernel, (unsigned)nmb * batch * head, kPipeThreads, stream, (const half_t*)q, (const half_t*)k,
+                    (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
+                    (half_t*)dq, head, n, nmb, c, scale);
+    } else {
+      if (spill) {
+        // two panels per block when that leaves every work group at least two blocks (a heavy and a light one)
+        const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * batch * head;
+        if (total2 >= 2 * persistent_grid(total2))
+          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, persistent_grid(total2), ds_threads(2), stream,
+                        (const half_t*)k, ks, (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, scale);
+        const int nqb = np / kDsPanelQ, total = nqb * batch * head;
+        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, persistent_grid(total), ds_threads(1), stream,
+                      (const half_t*)k, ks, (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, scale);
+      }
+      const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;
+      auto kernel = dq_makes_stats ? fmha_bwd_dq_kernel<D, CAUSAL, true> : fmha_bwd_dq_kernel<D, CAUSAL, false>;
+      return launch(kernel, (unsigned)nmb * batch * head, kDqThreads, stream, (const half_t*)q, (const half_t*)k,
+                    (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
+                    (half_t*)dq, head, n, nmb, c, scale);
     }
-    const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;
-    auto kernel = dq_makes_stats ? fmha_bwd_dq_kernel<D, CAUSAL, true> : fmha_bwd_dq_kernel<D, CAUSAL, false>;
-    return launch(kernel, (unsigned)nmb * batch * head, kDqThreads, stream, (const half_t*)q, (const half_t*)k,
-                  (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
-                  (half_t*)dq, head, n, nmb, c, scale);
   };
   auto dkdv_pass = [&]() {
-    const int nnb = (n + kKvBlockKeys - 1) / kKvBlockKeys;
-    auto kernel = spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, true> : fmha_bwd_dkdv_kernel<D, CAUSAL, false>;
-    return launch(kernel, (unsigned)nnb * batch * head, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
-                  (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
-                  (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, c, scale);
+    if constexpr (D == 64) {
+      const int nnb = (n + kPipeBlockKeys - 1) / kPipeBlockKeys;
+      return launch(fmha_bwd_dkdv_pipe_kernel<CAUSAL>, (unsigned)nnb * batch * head, kPipeThreads, stream,
+                    (const half_t*)q, (const half_t*)k, (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs,
+                    (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n, nnb, c, scale);
+    } else {
+      const int nnb = (n + kKvBlockKeys - 1) / kKvBlockKeys;
+      auto kernel = spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, true> : fmha_bwd_dkdv_kernel<D, CAUSAL, false>;
+      return launch(kernel, (unsigned)nnb * batch * head, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
+                    (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
+                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, c, scale);
+    }
   };
   // The spilling dK/dV pass feeds the dQ pass; otherwise the dQ pass (which may make the statistics) goes first.
   if (spill) {
@@ -2170,7 +2670,7 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
   if (int rc = check_shape(batch, head, m, n, d)) return rc;
   if (!isfinite(scale)) return FUSED_MHA_ERR_BAD_SCALE;
   if (workspace_bytes < stats_bytes(batch, head, n)) return FUSED_MHA_ERR_BAD_SHAPE;
-  // A workspace with room for the dS tiles selects the spill path (5 GEMMs executed instead of 7).
+  // A workspace with room for the dS tiles selects the spill path (5 GEMMs executed instead of 7; D = 128 only).
   const bool spill = spill_bytes(batch, head, n) <= FUSED_MHA_SPILL_MAX_BYTES &&
                      workspace_bytes >= spill_offset(batch, head, n) + spill_bytes(batch, head, n);
   if (misaligned(q) || misaligned(k) || misaligned(v) || misaligned(o) || misaligned(d_o) || misaligned(lse) ||
