@@ -1,0 +1,16 @@
+// What the PyTorch extension uses of the kernel library beside its public interface (fused_mha.h).
+#ifndef FMHA_INTERNAL_H_
+#define FMHA_INTERNAL_H_
+
+#include "fused_mha.h"
+
+extern "C" {
+
+// fused_mha_forward_strided for callers without a backward pass: the logsumexp is not written.
+int fmha_forward_without_lse(const void* query_ptr, const fused_mha_strides* query_strides, const void* key_ptr,
+                             const fused_mha_strides* key_strides, const void* value_ptr,
+                             const fused_mha_strides* value_strides, void* output_ptr, int batch, int head, int n, int d,
+                             float scale, int causal, void* stream);
+
+}  // extern "C"
+#endif  // FMHA_INTERNAL_H_

@@ -15,6 +15,7 @@
 //     with wrong strides;
 //   * the arch gate asks for gfx950 instead of sm_70 (:21-23).
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -25,6 +26,7 @@
 #include <vector>
 
 #include "fused_mha.h"
+#include "fmha_internal.h"
 
 #define CHECK_DEVICE(x) TORCH_CHECK(x.is_cuda(), #x " must be on the GPU")
 #define CHECK_SHAPE(x, ...) \
@@ -45,6 +47,11 @@ void check_arch(int device) {
 
 void check_rc(int rc, const char* what) {
   TORCH_CHECK(rc == FUSED_MHA_OK, what, " failed: ", fused_mha_error_string(rc));
+}
+
+// torch.empty without the dispatcher, which costs more than the allocation itself.
+at::Tensor gpu_empty(at::IntArrayRef size, at::ScalarType dtype, const at::Tensor& like) {
+  return at::Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
 }
 
 at::Tensor dense(const at::Tensor& x) { return x.is_contiguous() ? x : x.contiguous(); }
@@ -70,10 +77,13 @@ Operand operand(const at::Tensor& x) {
 
 }  // namespace
 
-std::vector<at::Tensor> mha_fwd(const at::Tensor& q,  // batch x seqlen x heads x head_size
-                                const at::Tensor& k,  // batch x seqlen x heads x head_size
-                                const at::Tensor& v,  // batch x seqlen x heads x head_size
-                                c10::optional<at::Tensor>& out_, const float softmax_scale, bool is_causal) {
+namespace {
+
+// The forward; lse (batch x heads x seqlen, fp32) is not produced if nullptr.
+at::Tensor forward(const at::Tensor& q,  // batch x seqlen x heads x head_size
+                   const at::Tensor& k,  // batch x seqlen x heads x head_size
+                   const at::Tensor& v,  // batch x seqlen x heads x head_size
+                   const c10::optional<at::Tensor>& out_, at::Tensor* lse, const float softmax_scale, bool is_causal) {
   auto q_dtype = q.dtype();
   TORCH_CHECK(q_dtype == torch::kFloat16, "This repo only supports fp16 data type");
   TORCH_CHECK(k.dtype() == q_dtype, "query and key must have the same dtype");
@@ -108,17 +118,33 @@ std::vector<at::Tensor> mha_fwd(const at::Tensor& q,  // batch x seqlen x heads 
     TORCH_CHECK(out.is_contiguous(), "Output tensor must be contiguous");
     CHECK_SHAPE(out, batch_size, seqlen_q, num_heads, head_size);
   } else {
-    out = torch::empty({batch_size, seqlen_q, num_heads, head_size}, q.options());
+    out = gpu_empty({batch_size, seqlen_q, num_heads, head_size}, at::kHalf, q);
   }
 
   c10::DeviceGuard device_guard(q.device());
   const Operand qo = operand(q), ko = operand(k), vo = operand(v);
-  auto lse = torch::empty({batch_size, num_heads, seqlen_q}, q.options().dtype(at::kFloat));
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
-  check_rc(fused_mha_forward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
-                                     out.data_ptr(), lse.data_ptr(), batch_size, num_heads, seqlen_q, head_size,
-                                     softmax_scale, is_causal ? 1 : 0, stream),
-           "fused_mha_forward");
+  if (lse) {
+    *lse = gpu_empty({batch_size, num_heads, seqlen_q}, at::kFloat, q);
+    check_rc(fused_mha_forward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
+                                       out.data_ptr(), lse->data_ptr(), batch_size, num_heads, seqlen_q, head_size,
+                                       softmax_scale, is_causal ? 1 : 0, stream),
+             "fused_mha_forward");
+  } else {
+    check_rc(fmha_forward_without_lse(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
+                                      out.data_ptr(), batch_size, num_heads, seqlen_q, head_size, softmax_scale,
+                                      is_causal ? 1 : 0, stream),
+             "fused_mha_forward");
+  }
+  return out;
+}
+
+}  // namespace
+
+std::vector<at::Tensor> mha_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                                const c10::optional<at::Tensor>& out_, const float softmax_scale, bool is_causal) {
+  at::Tensor lse;
+  at::Tensor out = forward(q, k, v, out_, &lse, softmax_scale, is_causal);
   return {out, lse};
 }
 
@@ -173,7 +199,7 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
       TORCH_CHECK(t.sizes() == q.sizes(), name, " must have the shape of q");
       return t;
     }
-    return torch::empty({batch_size, seqlen_q, num_heads, head_size}, q.options());
+    return gpu_empty({batch_size, seqlen_q, num_heads, head_size}, at::kHalf, q);
   };
   at::Tensor dq = grad_like(dq_, "dq"), dk = grad_like(dk_, "dk"), dv = grad_like(dv_, "dv");
 
@@ -182,7 +208,7 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
   // head size 64 makes no use of room for dS
   const size_t ws_bytes = (head_size == 64 ? fused_mha_backward_min_workspace_bytes : fused_mha_backward_workspace_bytes)(
       batch_size, num_heads, seqlen_q, head_size);
-  auto workspace = torch::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte));
+  auto workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
   check_rc(fused_mha_backward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
                                       od.data_ptr(), go.t.data_ptr(), &go.st, ld.data_ptr(), workspace.data_ptr(),
@@ -204,12 +230,12 @@ class AttentionNode : public torch::autograd::Function<AttentionNode> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q_in, const at::Tensor& k_in,
                             const at::Tensor& v_in, double softmax_scale, bool is_causal) {
     const at::Tensor q = last_dim_contiguous(q_in), k = last_dim_contiguous(k_in), v = last_dim_contiguous(v_in);
-    c10::optional<at::Tensor> none;
-    auto out_lse = mha_fwd(q, k, v, none, (float)softmax_scale, is_causal);
-    ctx->save_for_backward(torch::autograd::variable_list{q, k, v, out_lse[0], out_lse[1]});
+    at::Tensor lse;
+    at::Tensor out = ::forward(q, k, v, c10::nullopt, &lse, (float)softmax_scale, is_causal);
+    ctx->save_for_backward(torch::autograd::variable_list{q, k, v, out, lse});
     ctx->saved_data["softmax_scale"] = softmax_scale;
     ctx->saved_data["causal"] = is_causal;
-    return out_lse[0];
+    return out;
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
@@ -231,9 +257,8 @@ at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
   const double scale = softmax_scale.has_value() ? *softmax_scale : std::pow((double)q.size(-1), -0.5);
   if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
     return AttentionNode::apply(q, k, v, scale, is_causal);
-  c10::optional<at::Tensor> none;
-  return mha_fwd(last_dim_contiguous(q), last_dim_contiguous(k), last_dim_contiguous(v), none, (float)scale,
-                 is_causal)[0];
+  return forward(last_dim_contiguous(q), last_dim_contiguous(k), last_dim_contiguous(v), c10::nullopt, nullptr,
+                 (float)scale, is_causal);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

@@ -37,6 +37,7 @@
 #include <utility>
 
 #include "fused_mha.h"
+#include "fmha_internal.h"
 #include "block_map.h"
 
 
@@ -714,7 +715,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
         for (int part = 0; part < D / 64; ++part)
           store_resident<64>(O + cur.o_off + part * 64, rs, q0w, N, *reinterpret_cast<const f16v(*)[2]>(&o[2 * part]),
                              inv, lane, stage);
-        if (hh == 0 && qi < N) LSE[cur.stat_off + qi] = (m_run * c + __builtin_amdgcn_logf(l_tot)) * kLn2;
+        if (LSE && hh == 0 && qi < N) LSE[cur.stat_off + qi] = (m_run * c + __builtin_amdgcn_logf(l_tot)) * kLn2;
       }
       if (lin_next < 0) break;
       lin_cur = lin_next;
@@ -1101,7 +1102,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   const float l_tot = l_run + other_half(l_run);
   const float inv = 1.f / l_tot;
   store_resident<D>(O + head_off, rs, q0w, N, o, inv, lane, smem + wave * StageGeom<D>::kBytes);
-  if (lane < 32 && qi < N) LSE[((long)b * H + h) * N + qi] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
+  if (LSE && lane < 32 && qi < N) LSE[((long)b * H + h) * N + qi] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
 }
 
 // ---------------------------------------------------------------------------
@@ -2561,9 +2562,9 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
 }
 
 int dispatch_forward(const void* q, const fused_mha_strides* q_st, const void* k, const fused_mha_strides* k_st,
-                     const void* v, const fused_mha_strides* v_st, void* o, void* lse, int batch, int head, int m,
-                     int n, int d, float scale, int causal, void* stream) {
-  if (!q || !k || !v || !o || !lse) return FUSED_MHA_ERR_NULL_POINTER;
+                     const void* v, const fused_mha_strides* v_st, void* o, void* lse, bool need_lse, int batch, int head,
+                     int m, int n, int d, float scale, int causal, void* stream) {
+  if (!q || !k || !v || !o || (need_lse && !lse)) return FUSED_MHA_ERR_NULL_POINTER;
   if (int rc = check_shape(batch, head, m, n, d)) return rc;
   if (!isfinite(scale)) return FUSED_MHA_ERR_BAD_SCALE;
   if (misaligned(q) || misaligned(k) || misaligned(v) || misaligned(o) || misaligned(lse))
@@ -2714,8 +2715,8 @@ extern "C" {
 int fused_mha_forward(const void* query_ptr, const void* key_ptr, const void* value_ptr, void* output_ptr,
                       void* lse_ptr, int batch, int head, int m, int n, int d, float scale, int causal,
                       void* stream) {
-  return dispatch_forward(query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr, lse_ptr, batch, head,
-                          m, n, d, scale, causal, stream);
+  return dispatch_forward(query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr, lse_ptr, true, batch,
+                          head, m, n, d, scale, causal, stream);
 }
 
 int fused_mha_forward_strided(const void* query_ptr, const fused_mha_strides* query_strides, const void* key_ptr,
@@ -2723,7 +2724,15 @@ int fused_mha_forward_strided(const void* query_ptr, const fused_mha_strides* qu
                               const fused_mha_strides* value_strides, void* output_ptr, void* lse_ptr, int batch,
                               int head, int n, int d, float scale, int causal, void* stream) {
   return dispatch_forward(query_ptr, query_strides, key_ptr, key_strides, value_ptr, value_strides, output_ptr,
-                          lse_ptr, batch, head, n, n, d, scale, causal, stream);
+                          lse_ptr, true, batch, head, n, n, d, scale, causal, stream);
+}
+
+int fmha_forward_without_lse(const void* query_ptr, const fused_mha_strides* query_strides, const void* key_ptr,
+                             const fused_mha_strides* key_strides, const void* value_ptr,
+                             const fused_mha_strides* value_strides, void* output_ptr, int batch, int head, int n, int d,
+                             float scale, int causal, void* stream) {
+  return dispatch_forward(query_ptr, query_strides, key_ptr, key_strides, value_ptr, value_strides, output_ptr, nullptr,
+                          false, batch, head, n, n, d, scale, causal, stream);
 }
 
 size_t fused_mha_backward_min_workspace_bytes(int batch, int head, int n, int d) {

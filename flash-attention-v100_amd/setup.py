@@ -36,8 +36,9 @@ KERNEL_LIB = os.path.join(LIB_DIR, "libfused_mha.so")
 EXT_LIB = os.path.join(HERE, "flash_attn_v100_cuda.so")
 ROCM_HOME = os.environ.get("ROCM_HOME", "/opt/rocm")
 KERNEL_SOURCES = [os.path.join(CSRC, "fused_mha_kernel.hip"), os.path.join(CSRC, "block_map.h"),
+                  os.path.join(CSRC, "fmha_internal.h"),
                   os.path.join(INCLUDE, "fused_mha.h")]
-EXT_SOURCES = [os.path.join(CSRC, "fused_mha_api.cpp"), os.path.join(INCLUDE, "fused_mha.h")]
+EXT_SOURCES = [os.path.join(CSRC, "fused_mha_api.cpp"), os.path.join(CSRC, "fmha_internal.h"), os.path.join(INCLUDE, "fused_mha.h")]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -68,7 +69,7 @@ def build_extension(out=EXT_LIB):
     lib_dir = os.path.join(os.path.dirname(out), LIB_SUBDIR)
     if not os.path.exists(os.path.join(lib_dir, "libfused_mha.so")):
         build_kernels(out=os.path.join(lib_dir, "libfused_mha.so"))
-    includes = cpp_extension.include_paths() + [INCLUDE, os.path.join(ROCM_HOME, "include"),
+    includes = cpp_extension.include_paths() + [INCLUDE, CSRC, os.path.join(ROCM_HOME, "include"),
                                                 sysconfig.get_paths()["include"]]
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wno-deprecated-declarations",
@@ -78,7 +79,7 @@ def build_extension(out=EXT_LIB):
     for inc in includes:
         cmd += ["-isystem", inc]
     cmd += [os.path.join(CSRC, "fused_mha_api.cpp"), "-o", out,
-            "-L", torch_lib, "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python",
+            "-L", torch_lib, "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python",
             "-L", lib_dir, "-lfused_mha", "-Wl,-rpath,$ORIGIN/" + LIB_SUBDIR, "-Wl,--no-as-needed"]
     _run(cmd)
     return out
