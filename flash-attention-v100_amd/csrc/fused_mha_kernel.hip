@@ -362,6 +362,11 @@ template <int kOffset>
 __device__ __forceinline__ void store16_stream(half_t* p, h8 v, IntTag<kOffset>) {
   asm volatile("global_store_dwordx4 %0, %1, off offset:%2 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
 }
+// The same without the hint.
+template <int kOffset>
+__device__ __forceinline__ void store16_keep(half_t* p, h8 v, IntTag<kOffset>) {
+  asm volatile("global_store_dwordx4 %0, %1, off offset:%2" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+}
 
 // Element strides of a (batch, n, head, d) tensor whose last dimension is
 // contiguous.  The dense layout of reference kernel/fused_mha_kernel.cu:57-59 is
@@ -1684,7 +1689,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
                      const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                      const float* __restrict__ delta, const float* __restrict__ lse2,
                      half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
-                     int nnb, float c, float scale) {
+                     int nnb, int stream_ds, float c, float scale) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kKvWaves;  // copies per wave per tile, per tensor
@@ -1704,7 +1709,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   const bool role_b = wave >= kKvPairs;
   const int i = lane & 31, hh = lane >> 5;
   int bh, nblk;
-  slice_and_block(nnb, bh, nblk);  // causal: low key blocks are the heavy ones and come first
+  // causal: low key blocks are the heavy ones and come first
+  fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kKvBlockKeys != 0, bh, nblk);
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // dK and dV are dense
   const long head_off = ((long)b * N * H + h) * D;
@@ -1845,8 +1851,10 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         }
       }
   };
+  // a pair without keys has nothing to do, except for the zeros of dS it owes the last 64-key tile
+  const bool has_keys = k0w < (SPILL ? (N + kTile - 1) / kTile * kTile : N);
   auto tile_active = [&](int it) __attribute__((always_inline)) {
-    return !CAUSAL || (t_begin + it) * kTile + kTile - 1 >= k0w;
+    return has_keys && (!CAUSAL || (t_begin + it) * kTile + kTile - 1 >= k0w);
   };
 
   // Per iteration: wait for tile `it` (issued two iterations ago; the copies of tile
@@ -1939,10 +1947,17 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         // right after the barrier: the stores go through the same path and would queue behind them.
         const int t = t_begin + it - 1;  // the query tile
         half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048;
-        store16_stream(dst, y[0], IntTag<0>{});
-        store16_stream(dst, y[1], IntTag<1024>{});
-        store16_stream(dst, y[2], IntTag<2048>{});
-        store16_stream(dst, y[3], IntTag<3072>{});
+        if (stream_ds) {
+          store16_stream(dst, y[0], IntTag<0>{});
+          store16_stream(dst, y[1], IntTag<1024>{});
+          store16_stream(dst, y[2], IntTag<2048>{});
+          store16_stream(dst, y[3], IntTag<3072>{});
+        } else {
+          store16_keep(dst, y[0], IntTag<0>{});
+          store16_keep(dst, y[1], IntTag<1024>{});
+          store16_keep(dst, y[2], IntTag<2048>{});
+          store16_keep(dst, y[3], IntTag<3072>{});
+        }
       }
       if (it < n_it && tile_active(it)) {
         const char* Gl = g_ring + (it % 3) * T::kBytes;
@@ -2241,7 +2256,7 @@ constexpr int ds_threads(int panels) { return (4 * panels + kDsCopyWaves) * 64; 
 template <int D, bool CAUSAL, int kDsPanels>
 __global__ void __launch_bounds__(ds_threads(kDsPanels), 1)
 fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
-                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, float scale) {
+                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, int stream_ds, float scale) {
   using T = SwzTile<D>;             // K tile: 64 keys x D features
   constexpr int kKIPW = T::kInstrs / 2;              // K copies per K-copying wave and tile
   constexpr int kDsWaves = 4 * kDsPanels;            // computing waves
@@ -2267,6 +2282,11 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   const int slices = total / nqb;
   const PersistentBlocks pb{total};
 
+  // With one block per work group the hardware shares the blocks out, otherwise the persistent schedule does.
+  auto locate = [&](int lin, int& bh, int& mb) __attribute__((always_inline)) {
+    if ((int)gridDim.x == total) fmha_scheduled_block(lin, slices, nqb, CAUSAL, false, bh, mb);
+    else fmha_slice_and_block(lin, slices, nqb, bh, mb);
+  };
   // A position in the work group's sequence of tiles: block (round, number), tile j of its nt.
   struct Cursor {
     int round, lin, j, nt, mblk;
@@ -2278,7 +2298,7 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
     c.round = round;
     c.lin = round >= 0 ? pb.lin(round) : 0;
     int bh, mb;
-    fmha_slice_and_block(c.lin, slices, nqb, bh, mb);
+    locate(c.lin, bh, mb);
     c.mblk = CAUSAL ? nqb - 1 - mb : mb;  // heavy blocks first
     const int b = bh / H, h = bh - b * H;
     c.j = 0;
@@ -2302,7 +2322,7 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   int n_tiles = 0;  // tiles in this work group's sequence
   for (int r = 0; r >= 0; r = pb.next_round(r)) {
     int bh, mb;
-    fmha_slice_and_block(pb.lin(r), slices, nqb, bh, mb);
+    locate(pb.lin(r), bh, mb);
     const int mblk = CAUSAL ? nqb - 1 - mb : mb;
     n_tiles += CAUSAL ? min(nt_all, 2 * kDsPanels * (mblk + 1)) : nt_all;
   }
@@ -2328,8 +2348,13 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   auto copy_s = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
     const half_t* sp = c.base + (long)c.j * (kDsPanelTileBytes / 2);  // wave-uniform
     char* dst = s_ring + slot * kDsTileBytes + cw * kSIPW * 1024;
+    if (stream_ds) {
 #pragma unroll
-    for (int u = 0; u < kSIPW; ++u) copy16_stream(sp, c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+      for (int u = 0; u < kSIPW; ++u) copy16_stream(sp, c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+    } else {
+#pragma unroll
+      for (int u = 0; u < kSIPW; ++u) copy16(sp, c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+    }
   };
   auto copy_k = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
     const int row0 = c.j * kTile;
@@ -2601,6 +2626,11 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
   float* lse2 = delta + (long)batch * head * n;
   half_t* ds = spill ? (half_t*)((char*)delta + spill_offset(batch, head, n)) : nullptr;
   const int np = padded_n(n);
+  // dS that the 256 MiB Infinity Cache can hold next to the rest stays there between the two passes if neither is told
+  // that it is used once (B1 H8 N2048, 64 MiB: backward 82 -> 77 us); at 128 MiB and above the hint is the better choice,
+  // and for a few MiB too (B2 H4 N700 causal, 5 MiB: 34.7 against 36.2 us).
+  const size_t ds_bytes = spill_bytes(batch, head, n) / (CAUSAL ? 2 : 1);
+  const int stream_ds = ds_bytes < (24u << 20) || ds_bytes > (96u << 20);
   if ((passes & kPassDelta) && !dq_makes_stats) {
     const long rows = (long)batch * n * head;
     const long threads = rows * (D / 8);
@@ -2618,14 +2648,23 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
                     (half_t*)dq, head, n, nmb, c, scale);
     } else {
       if (spill) {
-        // two panels per block when that leaves every work group at least two blocks (a heavy and a light one)
+        // Two panels per block when that leaves every CU at least two blocks (a heavy and a light one).  The persistent
+        // schedule only where its static shares come out even (pairs of blocks under causal masking, as in
+        // persistent_forward_pays); otherwise one block per work group, heaviest first (B2 H40 N2048 causal, 2.5 blocks
+        // per CU: 116 -> 95 us).
+        const int cus = (int)persistent_grid(1 << 30);
+        auto groups = [&](int total) {
+          const long per = (CAUSAL ? 2L : 1L) * cus;
+          const bool even = total * 16L >= (total + per - 1) / per * per * 15;
+          return even ? persistent_grid(total) : (unsigned)total;
+        };
         const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * batch * head;
-        if (total2 >= 2 * persistent_grid(total2))
-          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, persistent_grid(total2), ds_threads(2), stream,
-                        (const half_t*)k, ks, (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, scale);
+        if (total2 >= 2 * cus)
+          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, groups(total2), ds_threads(2), stream, (const half_t*)k, ks,
+                        (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, stream_ds, scale);
         const int nqb = np / kDsPanelQ, total = nqb * batch * head;
-        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, persistent_grid(total), ds_threads(1), stream,
-                      (const half_t*)k, ks, (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, scale);
+        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, groups(total), ds_threads(1), stream, (const half_t*)k, ks,
+                      (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, stream_ds, scale);
       }
       const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;
       auto kernel = dq_makes_stats ? fmha_bwd_dq_kernel<D, CAUSAL, true> : fmha_bwd_dq_kernel<D, CAUSAL, false>;
@@ -2645,7 +2684,7 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
       auto kernel = spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, true> : fmha_bwd_dkdv_kernel<D, CAUSAL, false>;
       return launch(kernel, (unsigned)nnb * batch * head, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
-                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, c, scale);
+                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, stream_ds, c, scale);
     }
   };
   // The spilling dK/dV pass feeds the dQ pass; otherwise the dQ pass (which may make the statistics) goes first.
