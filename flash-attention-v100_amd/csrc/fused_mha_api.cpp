@@ -20,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
@@ -205,10 +206,23 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
 
   const Operand qo = operand(q), ko = operand(k), vo = operand(v), go = operand(dout);
   at::Tensor od = dense(out), ld = dense(lse);
-  // head size 64 makes no use of room for dS
-  const size_t ws_bytes = (head_size == 64 ? fused_mha_backward_min_workspace_bytes : fused_mha_backward_workspace_bytes)(
-      batch_size, num_heads, seqlen_q, head_size);
-  auto workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);
+  // Statistics, and at head size 128 room for the dS of as many (batch, head) slices as FUSED_MHA_SPILL_MAX_BYTES
+  // allows; if the memory for it is not there, the backward runs without it.
+  const size_t min_bytes = fused_mha_backward_min_workspace_bytes(batch_size, num_heads, seqlen_q, head_size);
+  size_t ws_bytes = min_bytes;
+  if (head_size == 128) {
+    const size_t np = ((size_t)seqlen_q + 127) & ~(size_t)127, slice = np * np * 2;
+    const size_t slices = std::min((size_t)batch_size * num_heads, (size_t)FUSED_MHA_SPILL_MAX_BYTES / slice);
+    if (slices) ws_bytes = ((min_bytes + 255) & ~(size_t)255) + slices * slice;
+  }
+  at::Tensor workspace;
+  try {
+    workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);
+  } catch (const c10::OutOfMemoryError&) {
+    if (ws_bytes == min_bytes) throw;
+    ws_bytes = min_bytes;
+    workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);
+  }
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
   check_rc(fused_mha_backward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
                                       od.data_ptr(), go.t.data_ptr(), &go.st, ld.data_ptr(), workspace.data_ptr(),

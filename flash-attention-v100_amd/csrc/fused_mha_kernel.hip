@@ -1689,7 +1689,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
                      const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                      const float* __restrict__ delta, const float* __restrict__ lse2,
                      half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
-                     int nnb, int stream_ds, float c, float scale) {
+                     int nnb, int slice0, int stream_ds, float c, float scale) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kKvWaves;  // copies per wave per tile, per tensor
@@ -1711,7 +1711,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   int bh, nblk;
   // causal: low key blocks are the heavy ones and come first
   fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kKvBlockKeys != 0, bh, nblk);
-  const int b = bh / H, h = bh - b * H;
+  const int b = (slice0 + bh) / H, h = slice0 + bh - b * H;  // bh: the slice in this launch and in dS
   const int rs = H * D;  // dK and dV are dense
   const long head_off = ((long)b * N * H + h) * D;
   const half_t* Qb = Q + b * qs.b + (long)h * qs.h;
@@ -2256,7 +2256,8 @@ constexpr int ds_threads(int panels) { return (4 * panels + kDsCopyWaves) * 64; 
 template <int D, bool CAUSAL, int kDsPanels>
 __global__ void __launch_bounds__(ds_threads(kDsPanels), 1)
 fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
-                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, int stream_ds, float scale) {
+                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, int slice0,
+                         int stream_ds, float scale) {
   using T = SwzTile<D>;             // K tile: 64 keys x D features
   constexpr int kKIPW = T::kInstrs / 2;              // K copies per K-copying wave and tile
   constexpr int kDsWaves = 4 * kDsPanels;            // computing waves
@@ -2300,7 +2301,7 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
     int bh, mb;
     locate(c.lin, bh, mb);
     c.mblk = CAUSAL ? nqb - 1 - mb : mb;  // heavy blocks first
-    const int b = bh / H, h = bh - b * H;
+    const int b = (slice0 + bh) / H, h = slice0 + bh - b * H;  // bh: the slice in this launch and in dS
     c.j = 0;
     c.nt = CAUSAL ? min(nt_all, 2 * kDsPanels * (c.mblk + 1)) : nt_all;
     // the pieces of a dS-copying wave: with two panels per block one whole panel (the last block of a sequence
@@ -2611,16 +2612,30 @@ enum BwdPass { kPassDelta = 1, kPassDq = 2, kPassDkDv = 4, kPassAll = 7 };
 size_t stats_bytes(int batch, int head, int n) { return 2 * (size_t)batch * head * n * sizeof(float); }
 size_t spill_offset(int batch, int head, int n) { return (stats_bytes(batch, head, n) + 255) & ~(size_t)255; }
 int padded_n(int n) { return (n + 127) & ~127; }
-size_t spill_bytes(int batch, int head, int n) {
-  const size_t np = (size_t)padded_n(n);
-  return (size_t)batch * head * np * np * sizeof(half_t);
+size_t slice_bytes(int n) { return (size_t)padded_n(n) * padded_n(n) * sizeof(half_t); }
+size_t spill_bytes(int batch, int head, int n) { return (size_t)batch * head * slice_bytes(n); }
+// Slices whose dS tiles a workspace has room for (of at most FUSED_MHA_SPILL_MAX_BYTES).
+int spill_slices(int batch, int head, int n, size_t workspace_bytes) {
+  const size_t offset = spill_offset(batch, head, n);
+  if (workspace_bytes <= offset) return 0;
+  size_t room = workspace_bytes - offset;
+  if (room > FUSED_MHA_SPILL_MAX_BYTES) room = FUSED_MHA_SPILL_MAX_BYTES;
+  const size_t fit = room / slice_bytes(n), all = (size_t)batch * head;
+  return (int)(fit < all ? fit : all);
 }
 
 template <int D, bool CAUSAL>
-int launch_backward(int passes, bool spill, const void* q, const void* k, const void* v, const void* o,
+int launch_backward(int passes, int slices_at_once, const void* q, const void* k, const void* v, const void* o,
                     const void* d_o, Strides qs, Strides ks, Strides vs, Strides gs, const void* lse, float* delta,
                     void* dq, void* dk, void* dv, int batch, int head, int n, float scale, hipStream_t stream) {
-  if (D == 64) spill = false;  // see fmha_bwd_dq_pipe_kernel
+  // slices_at_once: how many slices' dS the workspace holds, 0 for the passes that need none
+  if (D == 64) slices_at_once = 0;  // see fmha_bwd_dq_pipe_kernel
+  // Rounds of so few slices that they leave CUs idle cost more than the GEMMs they save.
+  const int cus = (int)persistent_grid(1 << 30);
+  if (slices_at_once < batch * head && (long)slices_at_once * ((n + kKvBlockKeys - 1) / kKvBlockKeys) < 2L * cus)
+    slices_at_once = 0;
+  const bool spill = slices_at_once > 0;
+  int slice0 = 0, slices = batch * head;  // what the passes over dS are launched for
   // Without the spill and with all three passes asked for, the dQ pass produces delta and lse2 itself.
   const bool dq_makes_stats = !spill && (passes & kPassAll) == kPassAll;
   float* lse2 = delta + (long)batch * head * n;
@@ -2629,7 +2644,7 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
   // dS that the 256 MiB Infinity Cache can hold next to the rest stays there between the two passes if neither is told
   // that it is used once (B1 H8 N2048, 64 MiB: backward 82 -> 77 us); at 128 MiB and above the hint is the better choice,
   // and for a few MiB too (B2 H4 N700 causal, 5 MiB: 34.7 against 36.2 us).
-  const size_t ds_bytes = spill_bytes(batch, head, n) / (CAUSAL ? 2 : 1);
+  const size_t ds_bytes = slice_bytes(n) * (spill ? slices_at_once : 0) / (CAUSAL ? 2 : 1);
   const int stream_ds = ds_bytes < (24u << 20) || ds_bytes > (96u << 20);
   if ((passes & kPassDelta) && !dq_makes_stats) {
     const long rows = (long)batch * n * head;
@@ -2652,19 +2667,18 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
         // schedule only where its static shares come out even (pairs of blocks under causal masking, as in
         // persistent_forward_pays); otherwise one block per work group, heaviest first (B2 H40 N2048 causal, 2.5 blocks
         // per CU: 116 -> 95 us).
-        const int cus = (int)persistent_grid(1 << 30);
         auto groups = [&](int total) {
           const long per = (CAUSAL ? 2L : 1L) * cus;
           const bool even = total * 16L >= (total + per - 1) / per * per * 15;
           return even ? persistent_grid(total) : (unsigned)total;
         };
-        const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * batch * head;
+        const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * slices;
         if (total2 >= 2 * cus)
           return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, groups(total2), ds_threads(2), stream, (const half_t*)k, ks,
-                        (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, stream_ds, scale);
-        const int nqb = np / kDsPanelQ, total = nqb * batch * head;
+                        (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, slice0, stream_ds, scale);
+        const int nqb = np / kDsPanelQ, total = nqb * slices;
         return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, groups(total), ds_threads(1), stream, (const half_t*)k, ks,
-                      (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, stream_ds, scale);
+                      (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, slice0, stream_ds, scale);
       }
       const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;
       auto kernel = dq_makes_stats ? fmha_bwd_dq_kernel<D, CAUSAL, true> : fmha_bwd_dq_kernel<D, CAUSAL, false>;
@@ -2682,15 +2696,22 @@ int launch_backward(int passes, bool spill, const void* q, const void* k, const 
     } else {
       const int nnb = (n + kKvBlockKeys - 1) / kKvBlockKeys;
       auto kernel = spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, true> : fmha_bwd_dkdv_kernel<D, CAUSAL, false>;
-      return launch(kernel, (unsigned)nnb * batch * head, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
+      return launch(kernel, (unsigned)nnb * slices, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
-                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, stream_ds, c, scale);
+                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, slice0, stream_ds, c, scale);
     }
   };
   // The spilling dK/dV pass feeds the dQ pass; otherwise the dQ pass (which may make the statistics) goes first.
   if (spill) {
-    if ((passes & kPassDkDv) && dkdv_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
-    if ((passes & kPassDq) && dq_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
+    // as many slices at a time as the workspace holds dS of, in rounds of equal size
+    const int rounds = (slices + slices_at_once - 1) / slices_at_once, all = slices;
+    int per = (all + rounds - 1) / rounds;
+    if (((per + 7) & ~7) <= slices_at_once) per = (per + 7) & ~7;  // whole slices per XCD
+    for (slice0 = 0; slice0 < all; slice0 += per) {
+      slices = all - slice0 < per ? all - slice0 : per;
+      if ((passes & kPassDkDv) && dkdv_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
+      if ((passes & kPassDq) && dq_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
+    }
   } else {
     if ((passes & kPassDq) && dq_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
     if ((passes & kPassDkDv) && dkdv_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
@@ -2710,9 +2731,10 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
   if (int rc = check_shape(batch, head, m, n, d)) return rc;
   if (!isfinite(scale)) return FUSED_MHA_ERR_BAD_SCALE;
   if (workspace_bytes < stats_bytes(batch, head, n)) return FUSED_MHA_ERR_BAD_SHAPE;
-  // A workspace with room for the dS tiles selects the spill path (5 GEMMs executed instead of 7; D = 128 only).
-  const bool spill = spill_bytes(batch, head, n) <= FUSED_MHA_SPILL_MAX_BYTES &&
-                     workspace_bytes >= spill_offset(batch, head, n) + spill_bytes(batch, head, n);
+  // A workspace with room for dS tiles selects the spill path (5 GEMMs executed instead of 7; D = 128 only): with room
+  // for some of the slices in rounds, which takes all passes in one call.
+  int slices_at_once = spill_slices(batch, head, n, workspace_bytes);
+  if (slices_at_once < batch * head && (passes & kPassAll) != kPassAll) slices_at_once = 0;
   if (misaligned(q) || misaligned(k) || misaligned(v) || misaligned(o) || misaligned(d_o) || misaligned(lse) ||
       misaligned(workspace) || misaligned(dq) || misaligned(dk) || misaligned(dv))
     return FUSED_MHA_ERR_MISALIGNED;
@@ -2722,7 +2744,7 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
   const Strides qs = to_strides(q_st, head, n, d), ks = to_strides(k_st, head, n, d),
                 vs = to_strides(v_st, head, n, d), gs = to_strides(g_st, head, n, d);
 #define FMHA_BWD(DD, CC) \
-  launch_backward<DD, CC>(passes, spill, q, k, v, o, d_o, qs, ks, vs, gs, lse, delta, dq, dk, dv, batch, head, n, \
+  launch_backward<DD, CC>(passes, slices_at_once, q, k, v, o, d_o, qs, ks, vs, gs, lse, delta, dq, dk, dv, batch, head, n, \
                           scale, s)
   if (d == 128) return causal ? FMHA_BWD(128, true) : FMHA_BWD(128, false);
   return causal ? FMHA_BWD(64, true) : FMHA_BWD(64, false);

@@ -93,7 +93,7 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
                               int batch, int head, int n, int d,
                               float scale, int causal, void *stream);
 
-/* Largest dS spill (bytes) the backward will use; beyond it the recompute path runs. */
+/* Largest dS spill (bytes) the backward will use at a time. */
 #define FUSED_MHA_SPILL_MAX_BYTES ((size_t)16 << 30)
 
 /*
@@ -109,8 +109,12 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * workspace the dQ pass recomputes S and dP.  Both paths are deterministic and
  * give the same dK and dV bits; dQ differs by summation order only.
  * fused_mha_backward_workspace_bytes returns the larger size when the spill is
- * within the limit, else the minimum; any size in between selects the
- * recompute path.  Both return 0 for an invalid shape.  No counterpart in the
+ * within the limit, else the minimum.  With d = 128 a size in between is used
+ * as well: fused_mha_backward runs the two passes in rounds, for as many
+ * (batch, head) slices at a time as the dS of np * np elements each fits
+ * behind the statistics (rounded up to 256 bytes), unless rounds of so few
+ * slices would leave compute units idle; the results are the same bits as
+ * with room for all.  Both functions return 0 for an invalid shape.  No counterpart in the
  * reference, which receives delta from Python (flash_attn_interface.py:43-44).
  */
 size_t fused_mha_backward_workspace_bytes(int batch, int head, int n, int d);
