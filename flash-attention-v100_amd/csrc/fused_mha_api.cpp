@@ -269,7 +269,10 @@ class AttentionNode : public torch::autograd::Function<AttentionNode> {
 at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                      c10::optional<double> softmax_scale, bool is_causal) {
   const double scale = softmax_scale.has_value() ? *softmax_scale : std::pow((double)q.size(-1), -0.5);
-  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+  // A tangent (forward-mode differentiation) goes to the node too, whatever the grad mode: it refuses it.
+  const auto has_tangent = [](const at::Tensor& x) { return x._fw_grad(/*level=*/0).defined(); };
+  if ((at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) ||
+      has_tangent(q) || has_tangent(k) || has_tangent(v))
     return AttentionNode::apply(q, k, v, scale, is_causal);
   return forward(last_dim_contiguous(q), last_dim_contiguous(k), last_dim_contiguous(v), c10::nullopt, nullptr,
                  (float)scale, is_causal);

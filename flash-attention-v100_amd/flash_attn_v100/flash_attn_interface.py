@@ -66,5 +66,9 @@ class FlashAttnFunc(torch.autograd.Function):
 
 
 def flash_attn_func(q, k, v, softmax_scale=None, causal=False):
+    if torch._C._get_tracing_state() is not None:
+        # torch.jit.trace records a Python autograd function as a node; it would keep what the extension returns as a
+        # constant
+        return FlashAttnFunc.apply(q, k, v, softmax_scale, causal)
     # the same as FlashAttnFunc.apply, with the autograd node in the extension
     return flash_attn_cuda.attention(q, k, v, softmax_scale, causal)
