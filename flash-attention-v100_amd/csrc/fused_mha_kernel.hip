@@ -1683,13 +1683,15 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // (consecutive lanes, consecutive addresses); inside a chunk position 8*hh + e holds
 // query 8*(e >> 2) + 4*hh + (e & 3).  Rows of keys at or past n are written as zeros; (key tile, query
 // tile) pairs above the diagonal are not written (and not read) under causal masking.
-template <int D, bool CAUSAL, bool SPILL>
+// KEEP: without the non-temporal hint on those stores (rule: launch_backward).  A parameter of the template because a
+// branch around the stores inside the loop costs 1-3 %.
+template <int D, bool CAUSAL, bool SPILL, bool KEEP>
 __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                      const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                      const float* __restrict__ delta, const float* __restrict__ lse2,
                      half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
-                     int nnb, int slice0, int stream_ds, float c, float scale) {
+                     int nnb, int slice0, float c, float scale) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kKvWaves;  // copies per wave per tile, per tensor
@@ -1853,9 +1855,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   };
   // a pair without keys has nothing to do, except for the zeros of dS it owes the last 64-key tile
   const bool has_keys = k0w < (SPILL ? (N + kTile - 1) / kTile * kTile : N);
-  auto tile_active = [&](int it) __attribute__((always_inline)) {
-    return has_keys && (!CAUSAL || (t_begin + it) * kTile + kTile - 1 >= k0w);
-  };
+  const int first_active = !has_keys ? n_it : CAUSAL ? k0w / kTile - t_begin : 0;
+  auto tile_active = [&](int it) __attribute__((always_inline)) { return CAUSAL ? it >= first_active : has_keys; };
 
   // Per iteration: wait for tile `it` (issued two iterations ago; the copies of tile
   // it+1 may still be in flight), one barrier, issue the copies of tile it+2.
@@ -1947,7 +1948,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         // right after the barrier: the stores go through the same path and would queue behind them.
         const int t = t_begin + it - 1;  // the query tile
         half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048;
-        if (stream_ds) {
+        if constexpr (!KEEP) {
           store16_stream(dst, y[0], IntTag<0>{});
           store16_stream(dst, y[1], IntTag<1024>{});
           store16_stream(dst, y[2], IntTag<2048>{});
@@ -2695,10 +2696,12 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
                     (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n, nnb, c, scale);
     } else {
       const int nnb = (n + kKvBlockKeys - 1) / kKvBlockKeys;
-      auto kernel = spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, true> : fmha_bwd_dkdv_kernel<D, CAUSAL, false>;
+      auto kernel = !spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, false, false>
+                    : stream_ds ? fmha_bwd_dkdv_kernel<D, CAUSAL, true, false>
+                                : fmha_bwd_dkdv_kernel<D, CAUSAL, true, true>;
       return launch(kernel, (unsigned)nnb * slices, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
-                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, slice0, stream_ds, c, scale);
+                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, slice0, c, scale);
     }
   };
   // The spilling dK/dV pass feeds the dQ pass; otherwise the dQ pass (which may make the statistics) goes first.
