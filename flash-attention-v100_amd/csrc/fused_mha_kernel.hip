@@ -495,7 +495,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
   // state of the block being worked on
   int q0w = 0, qi = 0, ntw = 0;
   f16v o[G::kDBlocks];
-  float m_run = -INFINITY, l_run = 0.f;
+  float mc = -INFINITY, l_run = 0.f;  // running maximum times c
   f16v s[2];   // scores of the tile in flight
   h8 pf[4];    // its probabilities, fp16, B-operand order
 
@@ -526,7 +526,6 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
     }
   };
   auto exponentials = [&]() __attribute__((always_inline)) {
-    const float mc = m_run * c;
     float l0 = 0.f, l1 = 0.f;
 #pragma unroll
     for (int c16 = 0; c16 < 4; ++c16) {
@@ -556,18 +555,21 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
     }
     // Optimistic: probabilities relative to the running maximum as it stands.  If any lane's sum over its 32 keys is
     // past kRescaleSum (or not a number: no maximum yet), the maximum is brought up to date and they are formed again.
+    // A wave's last tile always brings it up to date, as in fmha_fwd_pipe_kernel: both kernels give the same bits, so
+    // that a slice's result does not depend on how many others the call has.
     float lt = exponentials();
-    if (__builtin_amdgcn_ballot_w64(!(lt <= kRescaleSum)) != 0) {
+    if (t == ntw - 1 || __builtin_amdgcn_ballot_w64(!(lt <= kRescaleSum)) != 0) {
       float mx = s[0][0];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
       mx = fmaxf(mx, other_half(mx));
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = fast_exp2((m_run - m_new) * c);
-      m_run = m_new;
+      const float mc_new = fmaxf(mc, mx * c);
+      const float alpha = fast_exp2(mc - mc_new);
+      mc = mc_new;
       l_run *= alpha;
+      asm volatile("" : "+v"(l_run));  // rounded here: contracted with the sum below the loop is 4 % slower without a mask
 #pragma unroll
       for (int db = 0; db < G::kDBlocks; ++db)
 #pragma unroll
@@ -635,7 +637,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
       for (int db = 0; db < G::kDBlocks; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-      m_run = -INFINITY;
+      mc = -INFINITY;
       l_run = 0.f;
       auto wait_and_sync = [&]() __attribute__((always_inline)) {
         if (in_flight == 2 * kIPW) wait_vm<2 * kIPW>();
@@ -720,7 +722,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
         for (int part = 0; part < D / 64; ++part)
           store_resident<64>(O + cur.o_off + part * 64, rs, q0w, N, *reinterpret_cast<const f16v(*)[2]>(&o[2 * part]),
                              inv, lane, stage);
-        if (LSE && hh == 0 && qi < N) LSE[cur.stat_off + qi] = (m_run * c + __builtin_amdgcn_logf(l_tot)) * kLn2;
+        if (LSE && hh == 0 && qi < N) LSE[cur.stat_off + qi] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
       }
       if (lin_next < 0) break;
       lin_cur = lin_next;
@@ -962,6 +964,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     const float alpha = fast_exp2(mc - mc_new);
     mc = mc_new;
     l_run *= alpha;
+    asm volatile("" : "+v"(l_run));  // rounded here, as in fmha_fwd_kernel
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -2556,13 +2559,14 @@ bool bad_strides(const fused_mha_strides* st) {
 // shares come out even.  Without a mask all blocks weigh the same, so the last round of one block per CU has to be
 // nearly full (then it is 3-4 % faster than the 128-query kernel, whose K/V copies are twice as many; at 75 % full
 // already 14 % slower).  Under causal masking a work group's heavy block is paired with a light one, which comes out
-// even for exactly one pair of blocks per CU (3-6 % faster; hardware-scheduled small blocks are 13 % faster at 2.5
-// blocks per CU and 1-4 % at 8).
+// even for one pair of blocks per CU (3-6 % faster) and, where blocks are long enough that handing them out costs
+// nothing, for two (B2 H32 N4096: 265 against 272 us; B4 H32 N2048: 153 against 151).  At 2.5 blocks per CU
+// hardware-scheduled small blocks are 13 % faster, at 8 they are as fast or faster.
 bool persistent_forward_pays(int total, int n, bool causal) {
   const int cus = (int)persistent_grid(1 << 30);
-  if (causal) return n >= 2048 && total <= 2 * cus && total * 16L >= 2 * cus * 15L;
-  const long rounds = (total + cus - 1) / cus;
-  return total * 16L >= rounds * cus * 15L;
+  if (causal && (total > 4 * cus || n < (total > 2 * cus ? 4096 : 2048))) return false;
+  const long round = causal ? 2L * cus : cus;
+  return total * 16L >= (total + round - 1) / round * round * 15L;
 }
 
 template <int D, bool CAUSAL>

@@ -88,3 +88,23 @@ def test_persistent_blocks(B, H, N, causal):
     """255 and 256 blocks of 256 queries without a mask, 504 with one: the launches the persistent kernel takes."""
     for growing in (False, True):
         _check(B, N, H, 128, causal, growing, heads=[0, H // 2, H - 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,causal", [
+    (5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True), (1, 64, 2048, True),
+    (2, 32, 4096, True),   # two pairs of blocks per compute unit
+    (1, 61, 4099, True),   # two pairs, 17 blocks a slice, the last one of three queries
+])
+def test_a_slice_alone_gives_the_same_bits(B, H, N, causal):
+    """One slice has too few blocks for the persistent kernel, the whole problem takes it (or the other one: then there
+    is nothing to tell apart)."""
+    lib = abi.load()
+    for growing in (False, True):
+        q, k, v = (t.cuda() for t in _inputs(B, N, H, 128, growing))
+        scale = 1.0 if growing else 128 ** -0.5
+        out, lse = abi.forward(lib, q, k, v, scale, causal)
+        for b, h in ((0, 0), (B - 1, H - 1), (B // 2, H // 2)):
+            one = [t[b:b + 1, :, h:h + 1].contiguous() for t in (q, k, v)]
+            o1, l1 = abi.forward(lib, *one, scale, causal)
+            assert torch.equal(o1, out[b:b + 1, :, h:h + 1]) and torch.equal(l1, lse[b:b + 1, h:h + 1])
