@@ -1019,10 +1019,16 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     top_wait();
 #pragma unroll
     for (int m = 0; m < kLead; ++m) frag[m] = read(m);
-    top_copy(j, 1 - kSlot);
+    // At D = 128 a step's eight copies, issued by all waves at once, hold them until the copy path has taken them (64
+    // bytes per clock and CU): K follows when V is through.  B1 H2 N4000: 54.6 -> 50.8 us, B3 H20 N1031: 50.4 -> 49.6.
+    // Much later (unit 28: 61.4 us) it does not arrive in time.  At D = 64 there are half as many and it changes nothing.
+    constexpr int kCopyKAt = D == 128 ? 8 : 0;
+    if (j < nt) copy_v(j, 1 - kSlot);
+    if (kCopyKAt == 0 && j + 2 < nt) copy_k(j + 2, 1 - kSlot);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int m = 0; m < kM + 2; ++m) {
+      if (kCopyKAt != 0 && m == kCopyKAt && j + 2 < nt) copy_k(j + 2, 1 - kSlot);
       if (m < kM) {
         const int ch = m / (2 * kDB), in = m % (2 * kDB);
         if (in < kDB) {
