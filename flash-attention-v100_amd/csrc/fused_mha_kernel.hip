@@ -1868,7 +1868,9 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   auto tile_active = [&](int it) __attribute__((always_inline)) { return CAUSAL ? it >= first_active : has_keys; };
 
   // Per iteration: wait for tile `it` (issued two iterations ago; the copies of tile
-  // it+1 may still be in flight), one barrier, issue the copies of tile it+2.
+  // it+1 may still be in flight), one barrier, issue the copies of tile it+2.  Role A issues its half of them at the end
+  // of the iteration and role B near its start: all at once right after the barrier they held every wave until the copy
+  // path had taken them (B2 H32 N4096 causal: 608 -> 591 us; role A after its first GEMM: 627; role B later: 609).
   auto step_wait = [&](int it) __attribute__((always_inline)) {
     if (it + 1 < n_it) {
       if (wave == 0) wait_vm<2 * kIPW + 2>();
@@ -1878,8 +1880,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     }
     block_barrier();
   };
-  auto step_sync = [&](int it) __attribute__((always_inline)) {
-    step_wait(it);
+  auto step_copy = [&](int it) __attribute__((always_inline)) {
     if (it + 2 < n_it) copy_tiles(it + 2);
   };
   // where this lane's registers of dS go (SPILL): its key's 32 bytes in chunk 0 of query tile 0 of
@@ -1890,7 +1891,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   wait_vm<0>();  // resident rows and the first copies: nothing is left for the compiler to wait on in the loops
   if (!role_b) {
     for (int it = 0; it <= n_it; ++it) {
-      step_sync(it);
+      step_wait(it);
       if (it < n_it && tile_active(it)) {
         const char* Ql = q_ring + (it & 3) * T::kBytes;
         const char* Gl = g_ring + (it % 3) * T::kBytes;
@@ -1914,6 +1915,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         }
         gemm2(Gl, y);
       }
+      step_copy(it);
     }
   } else {
     f16v x[2];  // delta - dP of the previous tile
@@ -1925,8 +1927,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       // SPILL: this wave issues its tile copies and, after the second GEMM, the four stores of dS.  The wait
       // at the top of the next iteration leaves at most as many operations in flight as those stores, the
       // newest: every copy issued so far has then landed, whatever order stores and copies complete in.
-      if (SPILL) step_wait(it);
-      else step_sync(it);
+      step_wait(it);
+      if (!SPILL) step_copy(it);
       const bool prev_active = it >= 1 && tile_active(it - 1);
       h8 y[4];
       if (prev_active) {  // the part that needs P, one tile behind
@@ -1950,7 +1952,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
           }
         }
       }
-      if (SPILL && it + 2 < n_it) copy_tiles(it + 2);
+      if (SPILL) step_copy(it);
       if (prev_active) gemm2(q_ring + ((it - 1) & 3) * T::kBytes, y);
       if (SPILL && prev_active) {
         // dS(it - 1) leaves here, between the two GEMMs and away from the tile copies, which all waves issue
