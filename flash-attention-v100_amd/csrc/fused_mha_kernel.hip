@@ -1692,8 +1692,7 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // (consecutive lanes, consecutive addresses); inside a chunk position 8*hh + e holds
 // query 8*(e >> 2) + 4*hh + (e & 3).  Rows of keys at or past n are written as zeros; (key tile, query
 // tile) pairs above the diagonal are not written (and not read) under causal masking.
-// KEEP: without the non-temporal hint on those stores (rule: launch_backward).  A parameter of the template because a
-// branch around the stores inside the loop costs 1-3 %.
+// KEEP: without the non-temporal hint on those stores (rule: launch_backward).
 template <int D, bool CAUSAL, bool SPILL, bool KEEP>
 __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,

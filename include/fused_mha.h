@@ -106,7 +106,10 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * dK/dV pass writes the dS it forms there and the dQ pass is a single GEMM over
  * them: five GEMMs are executed, as in the reference's one-pass backward
  * (kernel/fused_mha_kernel.cu:564-713), instead of seven.  With the minimum
- * workspace the dQ pass recomputes S and dP.  Both paths are deterministic and
+ * workspace the dQ pass recomputes S and dP.  With d = 64 it always does, which
+ * is the faster way there: nothing but the minimum is used, whatever the size of
+ * the workspace (the preferred size is the same for both d so that callers need
+ * not tell them apart).  Both paths are deterministic and
  * give the same dK and dV bits; dQ differs by summation order only.
  * fused_mha_backward_workspace_bytes returns the larger size when the spill is
  * within the limit, else the minimum.  With d = 128 a size in between is used
@@ -184,9 +187,9 @@ int fused_mha_backward_noalloc(const void *query_ptr, const void *key_ptr, const
  *           followed by lse * log2(e) in the same shape
  *   dq    : d_q, streaming key/value tiles per block of 128 queries
  *   dkdv  : d_k and d_v, streaming query/d_o tiles per block of 128 keys
- * With a workspace of fused_mha_backward_workspace_bytes (room for the dS
- * tiles) the dkdv pass also writes dS and the dq pass reads it: dq must then
- * run after dkdv, on the same workspace.
+ * With d = 128 and a workspace of fused_mha_backward_workspace_bytes (room for
+ * the dS tiles) the dkdv pass also writes dS and the dq pass reads it: dq must
+ * then run after dkdv, on the same workspace.
  */
 int fused_mha_backward_delta(const void *output_ptr, const void *d_output_ptr, const void *lse_ptr,
                              void *workspace, size_t workspace_bytes,
