@@ -2625,7 +2625,7 @@ size_t stats_bytes(int batch, int head, int n) { return 2 * (size_t)batch * head
 size_t spill_offset(int batch, int head, int n) { return (stats_bytes(batch, head, n) + 255) & ~(size_t)255; }
 int padded_n(int n) { return (n + 127) & ~127; }
 size_t slice_bytes(int n) { return (size_t)padded_n(n) * padded_n(n) * sizeof(half_t); }
-size_t spill_bytes(int batch, int head, int n) { return (size_t)batch * head * slice_bytes(n); }
+int key_blocks(int n) { return (n + kKvBlockKeys - 1) / kKvBlockKeys; }
 // Slices whose dS tiles a workspace has room for (of at most FUSED_MHA_SPILL_MAX_BYTES).
 int spill_slices(int batch, int head, int n, size_t workspace_bytes) {
   const size_t offset = spill_offset(batch, head, n);
@@ -2634,6 +2634,36 @@ int spill_slices(int batch, int head, int n, size_t workspace_bytes) {
   if (room > FUSED_MHA_SPILL_MAX_BYTES) room = FUSED_MHA_SPILL_MAX_BYTES;
   const size_t fit = room / slice_bytes(n), all = (size_t)batch * head;
   return (int)(fit < all ? fit : all);
+}
+// Whether rounds of that many slices keep the CUs busy: two key blocks for each.
+bool rounds_fill(int slices, int n, int cus) { return (long)slices * key_blocks(n) >= 2L * cus; }
+// The workspace of at most `room` bytes that the backward makes the best use of.  dS of all slices where that is at most
+// FUSED_MHA_SPILL_MAX_BYTES.  Otherwise rounds of eight key blocks per CU or 4 GiB, whichever is more, if there is room:
+// larger ones gain next to nothing.  Backward in ms, without dS / with the dS of rounds of so many GiB:
+//   N32768 H16 causal     13.9 / 4: 13.6, 8: 12.1, 16: 11.6 (2, 4, 8 blocks per CU)
+//   N20000 H32            20.9 / 3: 19.5, 6: 17.8, 7.5: 17.6, 16: 17.3
+//   N8192 H256 causal     14.9 / 1: 13.3, 2: 12.6, 4: 12.6, 16: 12.8 (2, 4, 8, 32 blocks per CU)
+//   N2048 H2100 causal     9.8 / 0.2: 9.3, 1: 8.7, 4: 8.7, 16: 8.6
+//   N512 H33000 causal    16.6 / 0.1: 17.9, 0.5: 16.7, 1: 16.6, 2: 16.1, 16: 16.1
+// Rounds of less than 1 GiB are not worth it (last line).  The size is that for the 256 CUs of an MI355X, whatever device
+// is current.
+size_t best_workspace(int batch, int head, int n, int d, size_t room) {
+  constexpr int kCus = 256;
+  constexpr size_t kGiB = (size_t)1 << 30;
+  const size_t least = stats_bytes(batch, head, n), offset = spill_offset(batch, head, n), slice = slice_bytes(n);
+  if (d == 64) return least;  // see fmha_bwd_dq_pipe_kernel
+  const size_t all = (size_t)batch * head;
+  size_t want = all;
+  if (all * slice > FUSED_MHA_SPILL_MAX_BYTES) {
+    const size_t blocks = (size_t)key_blocks(n);
+    want = (8 * kCus + blocks - 1) / blocks;
+    if (want * slice < 4 * kGiB) want = 4 * kGiB / slice;
+    if (want * slice > FUSED_MHA_SPILL_MAX_BYTES) want = FUSED_MHA_SPILL_MAX_BYTES / slice;
+  }
+  const size_t fit = room > offset ? (room - offset) / slice : 0;
+  if (fit < want) want = fit;
+  const bool use = want == all || (want * slice >= kGiB && rounds_fill((int)want, n, kCus));
+  return use ? offset + want * slice : least;
 }
 
 template <int D, bool CAUSAL>
@@ -2644,8 +2674,7 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   if (D == 64) slices_at_once = 0;  // see fmha_bwd_dq_pipe_kernel
   // Rounds of so few slices that they leave CUs idle cost more than the GEMMs they save.
   const int cus = (int)persistent_grid(1 << 30);
-  if (slices_at_once < batch * head && (long)slices_at_once * ((n + kKvBlockKeys - 1) / kKvBlockKeys) < 2L * cus)
-    slices_at_once = 0;
+  if (slices_at_once < batch * head && !rounds_fill(slices_at_once, n, cus)) slices_at_once = 0;
   const bool spill = slices_at_once > 0;
   int slice0 = 0, slices = batch * head;  // what the passes over dS are launched for
   // Without the spill and with all three passes asked for, the dQ pass produces delta and lse2 itself.
@@ -2706,7 +2735,7 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
                     (const half_t*)q, (const half_t*)k, (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs,
                     (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n, nnb, c, scale);
     } else {
-      const int nnb = (n + kKvBlockKeys - 1) / kKvBlockKeys;
+      const int nnb = key_blocks(n);
       auto kernel = !spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, false, false>
                     : stream_ds ? fmha_bwd_dkdv_kernel<D, CAUSAL, true, false>
                                 : fmha_bwd_dkdv_kernel<D, CAUSAL, true, true>;
@@ -2817,8 +2846,7 @@ size_t fused_mha_backward_min_workspace_bytes(int batch, int head, int n, int d)
 
 size_t fused_mha_backward_workspace_bytes(int batch, int head, int n, int d) {
   if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK) return 0;
-  if (spill_bytes(batch, head, n) > FUSED_MHA_SPILL_MAX_BYTES) return stats_bytes(batch, head, n);
-  return spill_offset(batch, head, n) + spill_bytes(batch, head, n);
+  return best_workspace(batch, head, n, d, SIZE_MAX);
 }
 
 int fused_mha_backward(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,

@@ -100,24 +100,26 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * Bytes of device scratch the backward works best with for this problem size.
  * The workspace starts with delta = rowsum(d_o * o) and lse * log2(e), both
  * fp32 of shape (batch, head, n), delta first: that much
- * (fused_mha_backward_min_workspace_bytes) is always needed.  When the
- * workspace also has room for the fp16 dS tiles (batch * head * np * np
- * elements, np = n rounded up to 128; at most FUSED_MHA_SPILL_MAX_BYTES), the
+ * (fused_mha_backward_min_workspace_bytes) is always needed.  With d = 128 and
+ * room behind it (at the next multiple of 256 bytes) for the fp16 dS tiles of
+ * all batch * head slices, np * np elements each, np = n rounded up to 128, the
  * dK/dV pass writes the dS it forms there and the dQ pass is a single GEMM over
  * them: five GEMMs are executed, as in the reference's one-pass backward
  * (kernel/fused_mha_kernel.cu:564-713), instead of seven.  With the minimum
- * workspace the dQ pass recomputes S and dP.  With d = 64 it always does, which
- * is the faster way there: nothing but the minimum is used, whatever the size of
- * the workspace (the preferred size is the same for both d so that callers need
- * not tell them apart).  Both paths are deterministic and
- * give the same dK and dV bits; dQ differs by summation order only.
- * fused_mha_backward_workspace_bytes returns the larger size when the spill is
- * within the limit, else the minimum.  With d = 128 a size in between is used
- * as well: fused_mha_backward runs the two passes in rounds, for as many
- * (batch, head) slices at a time as the dS of np * np elements each fits
- * behind the statistics (rounded up to 256 bytes), unless rounds of so few
- * slices would leave compute units idle; the results are the same bits as
- * with room for all.  Both functions return 0 for an invalid shape.  No counterpart in the
+ * workspace the dQ pass recomputes S and dP.  With room for some of the slices
+ * fused_mha_backward runs the two passes in rounds, that many slices at a time,
+ * unless rounds of so few slices would leave compute units idle; the results are
+ * the same bits as with room for all.  All paths are deterministic and give
+ * the same dK and dV bits; dQ of the recomputing pass differs by summation order.
+ * fused_mha_backward_workspace_bytes returns
+ *   - d = 64: the minimum.  The dQ pass always recomputes, which is the faster
+ *     way there, and nothing else is read or written whatever the size;
+ *   - d = 128, dS of at most FUSED_MHA_SPILL_MAX_BYTES: room for all of it;
+ *   - d = 128, more dS than that: room for rounds of enough slices to keep an
+ *     MI355X busy, at most FUSED_MHA_SPILL_MAX_BYTES behind the statistics, or
+ *     the minimum where that does not hold one slice (n > 92672).
+ * A caller that wants to spend less passes any size from the minimum on.
+ * Both functions return 0 for an invalid shape.  No counterpart in the
  * reference, which receives delta from Python (flash_attn_interface.py:43-44).
  */
 size_t fused_mha_backward_workspace_bytes(int batch, int head, int n, int d);
@@ -187,9 +189,11 @@ int fused_mha_backward_noalloc(const void *query_ptr, const void *key_ptr, const
  *           followed by lse * log2(e) in the same shape
  *   dq    : d_q, streaming key/value tiles per block of 128 queries
  *   dkdv  : d_k and d_v, streaming query/d_o tiles per block of 128 keys
- * With d = 128 and a workspace of fused_mha_backward_workspace_bytes (room for
- * the dS tiles) the dkdv pass also writes dS and the dq pass reads it: dq must
- * then run after dkdv, on the same workspace.
+ * With d = 128 and a workspace with room for the dS tiles of all slices (what
+ * fused_mha_backward_workspace_bytes returns up to FUSED_MHA_SPILL_MAX_BYTES of
+ * dS) the dkdv pass also writes dS and the dq pass reads it: dq must then run
+ * after dkdv, on the same workspace.  Rounds need all passes in one call: with
+ * room for some of the slices only, the three do what they do with the minimum.
  */
 int fused_mha_backward_delta(const void *output_ptr, const void *d_output_ptr, const void *lse_ptr,
                              void *workspace, size_t workspace_bytes,

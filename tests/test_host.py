@@ -47,15 +47,40 @@ def test_workspace_bytes(lib):
     assert small(1, 4, 100, 64) == 2 * 4 * 100 * 4  # any n > 0 is accepted
     assert small(1, 4, 0, 64) == 0
     assert small(1, 4, 128, 96) == 0
-    # the preferred workspace adds room for the fp16 dS tiles: slices * np * np elements, np = n rounded up to
-    # 128, behind the statistics rounded up to 256 bytes
+    # at head size 128 the preferred workspace adds room for the fp16 dS tiles: slices * np * np elements, np = n rounded
+    # up to 128, behind the statistics rounded up to 256 bytes
     big = lib.fused_mha_backward_workspace_bytes
     assert big(2, 32, 4096, 128) == 2 * 2 * 32 * 4096 * 4 + 64 * 4096 * 4096 * 2
-    assert big(1, 4, 100, 64) == 3328 + 4 * 128 * 128 * 2  # 3200 bytes of statistics -> 3328
+    assert big(1, 4, 100, 128) == 3328 + 4 * 128 * 128 * 2  # 3200 bytes of statistics -> 3328
     assert big(1, 4, 0, 64) == 0 and big(1, 4, 128, 96) == 0
-    # past the spill limit (16 GiB) only the statistics are asked for
-    assert big(1, 32, 16384, 128) == small(1, 32, 16384, 128) + 32 * 16384 * 16384 * 2  # 16 GiB: still spilled
-    assert big(1, 64, 16384, 128) == small(1, 64, 16384, 128)                           # 32 GiB: recompute path
+    assert big(1, 32, 16384, 128) == small(1, 32, 16384, 128) + 32 * 16384 * 16384 * 2  # 16 GiB: all slices at once
+
+
+@pytest.mark.parametrize("batch,head,n", [(1, 4, 128), (2, 3, 333), (16, 12, 512), (1, 16, 32768), (1, 64, 16384)])
+def test_workspace_bytes_head_size_64(lib, batch, head, n):
+    """The backward reads and writes nothing but the statistics there, so no more is asked for."""
+    assert (lib.fused_mha_backward_workspace_bytes(batch, head, n, 64) ==
+            lib.fused_mha_backward_min_workspace_bytes(batch, head, n, 64))
+
+
+@pytest.mark.parametrize("batch,head,n,slices", [
+    (1, 64, 16384, 16),   # 32 GiB of dS; 128 key blocks a slice: 8 blocks per compute unit are 16 slices
+    (8, 32, 8192, 32),
+    (1, 16, 32768, 8),
+    (2, 16, 20000, 14),   # 157 blocks a slice: rounded up
+    (1, 12, 45000, 4),    # 5 more blocks per unit would be past 16 GiB
+    (1, 2, 92672, 1),     # one slice is just within 16 GiB
+    (1, 2, 92673, 0),     # not even one is
+    (2, 4200, 1024, 2048),  # many short slices: 4 GiB
+    (512, 1024, 384, 14563),
+])
+def test_workspace_bytes_past_the_spill_limit(lib, batch, head, n, slices):
+    """What the preferred size has room for past 16 GiB of dS: rounds of enough slices for the launches to be full."""
+    least = lib.fused_mha_backward_min_workspace_bytes(batch, head, n, 128)
+    np_ = -(-n // 128) * 128
+    want = -(-least // 256) * 256 + slices * np_ * np_ * 2 if slices else least
+    assert batch * head * np_ * np_ * 2 > 16 << 30 and slices * np_ * np_ * 2 <= 16 << 30
+    assert lib.fused_mha_backward_workspace_bytes(batch, head, n, 128) == want
 
 
 def test_forward_validation_codes(lib):

@@ -375,14 +375,15 @@ SPILL_CASES = [  # B, H, N, D, causal
 
 @pytest.mark.parametrize("B,H,N,D,causal", SPILL_CASES)
 def test_spill_and_recompute_backward_agree(lib, B, H, N, D, causal):
-    """The backward has two paths, chosen by the size of the workspace: with room for the dS tiles the dK/dV pass
+    """At head size 128 the backward has two paths, chosen by the size of the workspace: with room for the dS tiles the dK/dV pass
     spills them and the dQ pass is one GEMM; with the minimum workspace the dQ pass recomputes S and dP.  dK and
     dV come from the same arithmetic (bit-equal); dQ sums the same products tile by tile (equal to rounding);
     both match the oracle."""
     scale = 1.0 / math.sqrt(D)
     q, k, v, do = ao.make_inputs(B, N, H, D, seed=5 * N + D)
     print(f"spill/recompute B{B} H{H} N{N} D{D} causal={causal}", flush=True)
-    assert lib.fused_mha_backward_workspace_bytes(B, H, N, D) > lib.fused_mha_backward_min_workspace_bytes(B, H, N, D)
+    room = lib.fused_mha_backward_workspace_bytes(B, H, N, D) > lib.fused_mha_backward_min_workspace_bytes(B, H, N, D)
+    assert room == (D == 128)  # at head size 64 there is only the recomputing path
     qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
     out, lse = abi.forward(lib, qg, kg, vg, scale, causal)
     dq_s, dk_s, dv_s, _ = abi.backward(lib, qg, kg, vg, out, dog, lse, scale, causal)
