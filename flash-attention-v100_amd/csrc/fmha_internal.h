@@ -12,5 +12,9 @@ int fmha_forward_without_lse(const void* query_ptr, const fused_mha_strides* que
                              const fused_mha_strides* value_strides, void* output_ptr, int batch, int head, int n, int d,
                              float scale, int causal, void* stream);
 
+// fused_mha_backward_workspace_bytes for callers that can spare `room` bytes: the size of at most that (and at least the
+// minimum) with which the backward is fastest.  0 for an invalid shape.
+size_t fmha_backward_workspace_within(int batch, int head, int n, int d, size_t room);
+
 }  // extern "C"
 #endif  // FMHA_INTERNAL_H_

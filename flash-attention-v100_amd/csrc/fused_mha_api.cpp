@@ -17,6 +17,8 @@
 #include <torch/extension.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -74,6 +76,30 @@ Operand operand(const at::Tensor& x) {
   if (ok) return {x, {sb, sn, sh}};
   at::Tensor c = x.contiguous();
   return {c, {c.stride(0), c.stride(1), c.stride(2)}};
+}
+
+// From this size on (where the backward takes about a millisecond) it is worth asking what memory there is.
+constexpr size_t kLargeWorkspace = (size_t)1 << 30;
+
+// How much of `wanted` bytes torch's allocator can hand out without giving back what it has cached: its largest free
+// block, or half of what the device has left of this process's share.  Half, because whatever is allocated next needs
+// its memory more than the backward, which only gets slower without it.  A free block of another stream counts too:
+// then, and where nothing can be said (a graph capture has a pool of its own, other allocators may not answer), the
+// allocation is tried and the caller handles its failure.  The current device must be `device`.
+size_t workspace_room(c10::DeviceIndex device, size_t wanted) {
+  namespace caching = c10::hip::HIPCachingAllocator;
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None || caching::name() != "native")
+    return wanted;
+  size_t block = 1;  // with 0 the answer would take in what the device has left
+  caching::cacheInfo(device, &block);
+  if (block >= wanted) return wanted;
+  size_t left = 0, total = 0;
+  if (hipMemGetInfo(&left, &total) != hipSuccess) return block;
+  constexpr auto kAll = static_cast<size_t>(c10::CachingAllocator::StatType::AGGREGATE);
+  const double share = caching::getMemoryFraction(device) * (double)total;
+  const double used = (double)caching::getDeviceStats(device).reserved_bytes[kAll].current;
+  left = std::min(left, (size_t)std::max(share - used, 0.0));
+  return std::min(wanted, std::max(block, left / 2));
 }
 
 }  // namespace
@@ -206,15 +232,12 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
 
   const Operand qo = operand(q), ko = operand(k), vo = operand(v), go = operand(dout);
   at::Tensor od = dense(out), ld = dense(lse);
-  // Statistics, and at head size 128 room for the dS of as many (batch, head) slices as FUSED_MHA_SPILL_MAX_BYTES
-  // allows; if the memory for it is not there, the backward runs without it.
+  // Statistics, and at head size 128 room for dS; a large one only as far as it is there for the taking.
   const size_t min_bytes = fused_mha_backward_min_workspace_bytes(batch_size, num_heads, seqlen_q, head_size);
-  size_t ws_bytes = min_bytes;
-  if (head_size == 128) {
-    const size_t np = ((size_t)seqlen_q + 127) & ~(size_t)127, slice = np * np * 2;
-    const size_t slices = std::min((size_t)batch_size * num_heads, (size_t)FUSED_MHA_SPILL_MAX_BYTES / slice);
-    if (slices) ws_bytes = ((min_bytes + 255) & ~(size_t)255) + slices * slice;
-  }
+  size_t ws_bytes = fused_mha_backward_workspace_bytes(batch_size, num_heads, seqlen_q, head_size);
+  if (ws_bytes >= kLargeWorkspace)
+    ws_bytes = fmha_backward_workspace_within(batch_size, num_heads, seqlen_q, head_size,
+                                              workspace_room(q.get_device(), ws_bytes));
   at::Tensor workspace;
   try {
     workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);

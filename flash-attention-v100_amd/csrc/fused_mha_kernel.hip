@@ -2849,6 +2849,11 @@ size_t fused_mha_backward_workspace_bytes(int batch, int head, int n, int d) {
   return best_workspace(batch, head, n, d, SIZE_MAX);
 }
 
+size_t fmha_backward_workspace_within(int batch, int head, int n, int d, size_t room) {
+  if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK) return 0;
+  return best_workspace(batch, head, n, d, room);
+}
+
 int fused_mha_backward(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,
                        const void* d_output_ptr, const void* lse_ptr, void* workspace, size_t workspace_bytes,
                        void* d_query_ptr, void* d_key_ptr, void* d_value_ptr, int batch, int head, int m, int n,

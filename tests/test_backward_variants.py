@@ -78,3 +78,104 @@ def test_backward_without_memory_for_the_spill():
             torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(grads[0][1], grads[1][1]) and torch.equal(grads[0][2], grads[1][2])
     assert (grads[0][0].float() - grads[1][0].float()).abs().max() <= 2e-3
+
+
+def _workspace_and_grads(leaves, out, do):
+    """Gradients and the bytes that the backward held at its height beside them."""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    grads = torch.autograd.grad(out, leaves, do, retain_graph=True)
+    return torch.cuda.max_memory_allocated() - before - sum(g.numel() * 2 for g in grads), grads
+
+
+@pytest.mark.gpu
+def test_backward_leaves_the_rest_of_the_memory_alone():
+    """Past 16 GiB of dS (17 here) the backward takes rounds of 8 GiB where the memory is there, smaller ones where half
+    of what is left does not hold those, none of it where that is not worth it, and never makes the allocator give back
+    what it has cached."""
+    from flash_attn_v100 import flash_attn_func
+    B, H, N, D = 1, 34, 16384, 128
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    out = flash_attn_func(*leaves, causal=True)
+    total, results = torch.cuda.get_device_properties(0).total_memory, []
+    for left, slices in ((None, 16), (7 << 30, 6), (1 << 30, 0)):
+        torch.cuda.empty_cache()
+        cached = [torch.empty(64 << 20, dtype=torch.uint8, device="cuda") for _ in range(4)]
+        del cached
+        stats = torch.cuda.memory_stats()
+        try:
+            if left:
+                grads = 3 * q.numel() * 2
+                torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + grads + left) / total)
+            took, got = _workspace_and_grads(leaves, out, do)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        after = torch.cuda.memory_stats()
+        assert after["num_alloc_retries"] == stats["num_alloc_retries"] and after["num_ooms"] == stats["num_ooms"]
+        assert after["reserved_bytes.all.current"] >= stats["reserved_bytes.all.current"]
+        assert abs(took - slices * N * N * 2 - 2 * H * N * 4) <= 16 << 20  # the allocator rounds up
+        results.append(got)
+    for got in results[1:]:
+        assert torch.equal(got[1], results[0][1]) and torch.equal(got[2], results[0][2])
+    assert torch.equal(results[1][0], results[0][0])
+    assert (results[2][0].float() - results[0][0].float()).abs().max() <= 2e-3
+
+
+@pytest.mark.gpu
+def test_backward_takes_a_cached_workspace_again():
+    """What the allocator has cached is taken although nothing is left of the process's share."""
+    from flash_attn_v100 import flash_attn_func
+    B, H, N, D = 1, 10, 8192, 128  # 1.25 GiB of dS
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    out = flash_attn_func(*leaves, causal=True)
+    torch.cuda.empty_cache()
+    took, grads = _workspace_and_grads(leaves, out, do)
+    first = [g.cpu() for g in grads]
+    del grads  # their blocks serve the second call's
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() /
+                                                   torch.cuda.get_device_properties(0).total_memory)
+        took_again, grads = _workspace_and_grads(leaves, out, do)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert took == took_again > 1 << 30
+    for a, b in zip(first, grads):
+        assert torch.equal(a, b.cpu())
+
+
+@pytest.mark.gpu
+def test_capture_with_a_large_workspace():
+    """A graph capture takes its memory from a pool of its own: 1 GiB of dS there, the eager result on every replay."""
+    from flash_attn_v100 import flash_attn_func
+    B, H, N, D = 1, 8, 8192, 128
+    static = [torch.zeros(B, N, H, D, dtype=torch.float16, device="cuda") for _ in range(4)]
+    leaves = [t.requires_grad_() for t in static[:3]]
+
+    def step():
+        return torch.autograd.grad(flash_attn_func(*leaves, causal=True), leaves, static[3])
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for seed in (1, 2, 3):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        with torch.no_grad():
+            for t in static:
+                t.copy_(torch.randn(t.shape, device="cuda", dtype=torch.float16, generator=gen))
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = [t.clone() for t in captured]
+        eager = step()
+        torch.cuda.synchronize()
+        for a, b in zip(replayed, eager):
+            assert torch.equal(a, b)

@@ -83,6 +83,28 @@ def test_workspace_bytes_past_the_spill_limit(lib, batch, head, n, slices):
     assert lib.fused_mha_backward_workspace_bytes(batch, head, n, 128) == want
 
 
+@pytest.mark.parametrize("batch,head,n,d,room,slices", [
+    (2, 32, 4096, 128, 16 << 30, 64),          # room for all
+    (2, 32, 4096, 128, (2 << 30) + (2 << 20), 64),  # just so
+    (2, 32, 4096, 128, (2 << 30) + (2 << 20) - 1, 63),
+    (2, 32, 4096, 128, (1 << 30) - 1, 0),      # rounds of less than 1 GiB are not worth it
+    (2, 4, 1024, 128, 1 << 20, 0),
+    (1, 16, 32768, 128, 9 << 30, 4),
+    (1, 16, 32768, 128, 3 << 30, 0),           # one slice is one block per compute unit
+    (1, 16, 32768, 128, 0, 0),
+    (1, 64, 16384, 128, 64 << 30, 16),         # no more than the preferred size
+    (1, 64, 16384, 64, 64 << 30, 0),
+])
+def test_workspace_within(lib, batch, head, n, d, room, slices):
+    """The size the extension takes when it can spare `room` bytes."""
+    f = lib.fmha_backward_workspace_within
+    f.argtypes, f.restype = [ctypes.c_int] * 4 + [ctypes.c_size_t], ctypes.c_size_t
+    least = lib.fused_mha_backward_min_workspace_bytes(batch, head, n, d)
+    np_ = -(-n // 128) * 128
+    assert f(batch, head, n, d, room) == (-(-least // 256) * 256 + slices * np_ * np_ * 2 if slices else least)
+    assert f(batch, head, 0, d, room) == 0
+
+
 def test_forward_validation_codes(lib):
     p = 0x1000  # never dereferenced: every call below is rejected before a launch
     f = lib.fused_mha_forward
