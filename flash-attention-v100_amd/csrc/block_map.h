@@ -66,6 +66,17 @@ FMHA_HOST_DEVICE int fmha_persistent_next_round(int r, int w, int G, int total) 
   return -1;
 }
 
+// Whether the shares of G persistent work groups come out even.  Without a mask all blocks weigh the same: the last round
+// has to be nearly full.  Under causal masking every work group has to get as many heavy blocks as light ones of the same
+// slices, which takes whole pairs of rounds and whole slices for every XCD: the shares are then equal to the tile.  Pairs of
+// rounds that are just nearly full are not enough: the largest share of 60 slices of 8 blocks (480 on 256 work groups) is
+// 1.54 times the mean, of 42 slices of 12 blocks 1.8 times, of 120 slices of 8 blocks still 1.07 times.
+FMHA_HOST_DEVICE bool fmha_even_shares(int slices, int blocks_per_slice, int G, bool causal) {
+  const long total = (long)slices * blocks_per_slice;
+  if (causal) return (slices & 7) == 0 && total % (2 * G) == 0;
+  return total * 16 >= (total + G - 1) / G * G * 15;
+}
+
 // Launches of one block per work group that the hardware hands out as CUs become free, two or more to a CU.
 // heavy_first (causal masking, blocks numbered heaviest first): the blocks of many slices are ordered block-index
 // major, so that heavy blocks start first and the launch ends with light ones.  An XCD's slices are taken in groups of

@@ -2562,18 +2562,20 @@ bool bad_strides(const fused_mha_strides* st) {
   return st->seq >= (1 << 24) || st->head >= (1LL << 31);
 }
 
-// Whether the persistent 256-query forward takes a D = 128 problem of `total` such blocks: only where its static
-// shares come out even.  Without a mask all blocks weigh the same, so the last round of one block per CU has to be
-// nearly full (then it is 3-4 % faster than the 128-query kernel, whose K/V copies are twice as many; at 75 % full
-// already 14 % slower).  Under causal masking a work group's heavy block is paired with a light one, which comes out
-// even for one pair of blocks per CU (3-6 % faster) and, where blocks are long enough that handing them out costs
-// nothing, for two (B2 H32 N4096: 265 against 272 us; B4 H32 N2048: 153 against 151).  At 2.5 blocks per CU
-// hardware-scheduled small blocks are 13 % faster, at 8 they are as fast or faster.
-bool persistent_forward_pays(int total, int n, bool causal) {
-  const int cus = (int)persistent_grid(1 << 30);
+// Whether the persistent 256-query forward takes a D = 128 problem: only where its static shares come out even.  Figures:
+// us of the 128-query kernel, then of this one, at N x slices.
+//   Without a mask the two are within 3 % of each other where the last round is nearly full (1024 x 64: 37.7, 38.4; 4096 x
+//   16: 126, 123; 4096 x 64: 492, 484; 2048 x 320: 636, 654); at 75 % full they are not (4096 x 24: 187, 205).
+//   Under causal masking one pair of blocks per CU is even at N = 2048 and gains from there on (1024 x 128: 47.5, 47.7;
+//   2048 x 64: 77.4, 77.5; 4096 x 32: 139, 136; 8192 x 16: 265, 249; 16384 x 8: 516, 479), two pairs from N = 4096 on (2048
+//   x 128: 147, 154; 4096 x 64: 276, 274 over seconds of nothing else, where the power cap rules and fewer copies of K and V
+//   count, but 262, 269 in turns of 12 ms; 8192 x 32: 498, 495; 32768 x 8: 1905, 1874), more do not (4096 x 96: 408, 419;
+//   8192 x 64: 984, 1006).  Uneven shares lose: 2048 x 60: 74, 90; 4096 x 60: 248, 292; 6144 x 42: 373, 487; 32768 x 4:
+//   1008, 1131.
+bool persistent_forward_pays(int slices, int blocks_per_slice, int n, bool causal) {
+  const int cus = (int)persistent_grid(1 << 30), total = slices * blocks_per_slice;
   if (causal && (total > 4 * cus || n < (total > 2 * cus ? 4096 : 2048))) return false;
-  const long round = causal ? 2L * cus : cus;
-  return total * 16L >= (total + round - 1) / round * round * 15L;
+  return fmha_even_shares(slices, blocks_per_slice, cus, causal);
 }
 
 template <int D, bool CAUSAL>
@@ -2585,7 +2587,7 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
   const int negate = scale < 0.f ? 1 : 0;
   if constexpr (D == 128) {
     const int nmb = (n + kFwdBlockQ - 1) / kFwdBlockQ, total = nmb * batch * head;
-    if (persistent_forward_pays(total, n, CAUSAL)) {
+    if (persistent_forward_pays(batch * head, nmb, n, CAUSAL)) {
       const hipError_t rc = launch(fmha_fwd_kernel<D, CAUSAL>, persistent_grid(total), kFwdThreads, stream,
                                    (const half_t*)q, (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o,
                                    (float*)lse, head, n, nmb, total, c, negate);

@@ -83,9 +83,11 @@ def test_small_blocks(N, causal, D):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,N,causal", [(5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True)])
+@pytest.mark.parametrize("B,H,N,causal", [(5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True),
+                                            (1, 32, 3900, True)])
 def test_persistent_blocks(B, H, N, causal):
-    """255 and 256 blocks of 256 queries without a mask, 504 with one: the launches the persistent kernel takes."""
+    """255 and 256 blocks of 256 queries without a mask, 512 with one: launches the persistent kernel takes.  504 blocks
+    with a mask do not share out evenly and go to the other kernel."""
     for growing in (False, True):
         _check(B, N, H, 128, causal, growing, heads=[0, H // 2, H - 1])
 
@@ -93,8 +95,10 @@ def test_persistent_blocks(B, H, N, causal):
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,N,causal", [
     (5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True), (1, 64, 2048, True),
-    (2, 32, 4096, True),   # two pairs of blocks per compute unit
-    (1, 61, 4099, True),   # two pairs, 17 blocks a slice, the last one of three queries
+    (2, 32, 4096, True),   # two pairs of blocks per compute unit: persistent
+    (1, 61, 4099, True),   # 17 blocks a slice, the last one of three queries
+    (1, 32, 3900, True),   # one pair per compute unit, with a ragged end: persistent
+    (1, 32, 8001, True),   # two pairs: persistent
 ])
 def test_a_slice_alone_gives_the_same_bits(B, H, N, causal):
     """One slice has too few blocks for the persistent kernel, the whole problem takes it (or the other one: then there

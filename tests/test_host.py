@@ -354,6 +354,57 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_even_shares_are_even(tmp_path):
+    """csrc/block_map.h, compiled for the host: where fmha_even_shares says so, no persistent work group's share of the
+    tiles is above the mean under causal masking, nor above 16/15 of it without a mask; launches that just about fill
+    their rounds are not called even when their shares are not."""
+    import subprocess
+
+    src = tmp_path / "check_even.cpp"
+    src.write_text(r'''
+#include <algorithm>
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+// largest share over the mean one, in tiles; blocks are numbered heaviest first
+static double largest(int slices, int bps, int G, bool causal) {
+  const int total = slices * bps, grid = total < G ? total : G;
+  std::vector<long> load(grid, 0);
+  long sum = 0;
+  for (int w = 0; w < grid; ++w)
+    for (int r = 0; r >= 0; r = fmha_persistent_next_round(r, w, grid, total)) {
+      int s, b;
+      fmha_slice_and_block(fmha_persistent_block(r, w, grid), slices, bps, s, b);
+      load[w] += causal ? bps - b : 1;
+    }
+  for (long v : load) sum += v;
+  return (double)*std::max_element(load.begin(), load.end()) * G / sum;
+}
+int main() {
+  int even[2] = {0, 0};
+  for (int G : {64, 256})
+    for (int slices = 1; slices <= 300; ++slices)
+      for (int bps = 1; bps <= 130; ++bps)
+        for (int causal = 0; causal < 2; ++causal) {
+          if (slices * bps > 16 * G || !fmha_even_shares(slices, bps, G, causal)) continue;
+          ++even[causal];
+          const double most = largest(slices, bps, G, causal);
+          if (most > (causal ? 1.0001 : 16.0001 / 15)) { printf("%d %d %d %d: %.3f\n", G, slices, bps, causal, most); return 1; }
+        }
+  if (even[0] < 1000 || even[1] < 50) { printf("few: %d %d\n", even[0], even[1]); return 1; }
+  const int uneven[][2] = {{60, 8}, {42, 12}, {120, 8}, {60, 16}, {42, 24}, {30, 32}, {4, 128}};
+  for (auto& x : uneven)
+    if (fmha_even_shares(x[0], x[1], 256, true) || largest(x[0], x[1], 256, true) < 1.05) { printf("uneven %d %d\n", x[0], x[1]); return 1; }
+  puts("ok");
+  return 0;
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    exe = tmp_path / "check_even"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
 def test_installed_distribution_imports_without_pythonpath(tmp_path):
     """`pip install .` (the wheel `python setup.py install` / `pip wheel .` build; reference setup.py:151-172,
     README.md:21-23) puts the package, the extension and the kernel library into one place, and the package
