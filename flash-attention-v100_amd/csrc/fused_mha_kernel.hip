@@ -2707,20 +2707,24 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
     } else {
       if (spill) {
         // Two panels per block when that leaves every CU at least two blocks (a heavy and a light one).  The persistent
-        // schedule only where its static shares come out even (pairs of blocks under causal masking, as in
-        // persistent_forward_pays); otherwise one block per work group, heaviest first (B2 H40 N2048 causal, 2.5 blocks
-        // per CU: 116 -> 95 us).
-        auto groups = [&](int total) {
-          const long per = (CAUSAL ? 2L : 1L) * cus;
-          const bool even = total * 16L >= (total + per - 1) / per * per * 15;
+        // schedule only where its static shares come out even, otherwise one block per work group, heaviest first (B2 H40
+        // N2048 causal, 2.5 blocks per CU: 116 -> 95 us).  Under causal masking nearly full pairs of rounds are not even
+        // (forward and backward, us of the hardware's and of the persistent schedule, N x slices: 3072 x 42: 488, 516;
+        // 4096 x 60: 1098, 1136; 8192 x 30: 2003, 2060), but up to N = 1024, where a block is a few us, they do as well (512
+        // x 120: 81, 77; 1024 x 120: 208, 204; 768 x 80: 93, 92).  Even launches are within 1 % of each other (2048 x 64:
+        // 335, 331; 4096 x 64: 1144, 1156; 8192 x 32: 2087, 2097; 16384 x 16: 3976, 3964).
+        auto groups = [&](int blocks_per_slice) {
+          const int total = blocks_per_slice * slices;
+          const bool even = CAUSAL && n <= 1024 ? fmha_even_shares(slices, blocks_per_slice, 2 * cus, false)
+                                                : fmha_even_shares(slices, blocks_per_slice, cus, CAUSAL);
           return even ? persistent_grid(total) : (unsigned)total;
         };
         const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * slices;
         if (total2 >= 2 * cus)
-          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, groups(total2), ds_threads(2), stream, (const half_t*)k, ks,
+          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, groups(nqb2), ds_threads(2), stream, (const half_t*)k, ks,
                         (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, slice0, stream_ds, scale);
         const int nqb = np / kDsPanelQ, total = nqb * slices;
-        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, groups(total), ds_threads(1), stream, (const half_t*)k, ks,
+        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, groups(nqb), ds_threads(1), stream, (const half_t*)k, ks,
                       (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, slice0, stream_ds, scale);
       }
       const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;

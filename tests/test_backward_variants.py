@@ -58,6 +58,29 @@ def test_backward_in_rounds(B, H, N, room, causal):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,N,causal", [
+    (64, 2048, True),   # dQ pass: one pair of blocks of 256 queries per compute unit, persistent
+    (60, 2048, True),   # nearly one pair, which does not share out evenly: handed out by the hardware
+    (42, 1300, True),   # the same with the half panels of a ragged end
+    (120, 512, True),   # nearly one pair of short blocks: persistent all the same
+    (62, 1031, False),  # 558 blocks, 2.2 per compute unit
+    (63, 1000, False),  # 252 blocks, nearly one per compute unit: persistent
+])
+def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
+    """One slice has too few blocks for any of the schedules the whole problem takes: the same bits."""
+    D, lib = 128, abi.load()
+    gen = torch.Generator(device="cuda").manual_seed(N + H)
+    q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+    whole = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal)[:3]
+    for h in (0, H // 2, H - 1):
+        one = [t[:, :, h:h + 1].contiguous() for t in (q, k, v, out, do)]
+        alone = abi.backward(lib, *one, lse[:, h:h + 1].clone(), D ** -0.5, causal)[:3]
+        for a, b in zip(alone, whole):
+            assert torch.equal(a, b[:, :, h:h + 1])
+
+
+@pytest.mark.gpu
 def test_backward_without_memory_for_the_spill():
     from flash_attn_v100 import flash_attn_func
     B, H, N, D = 1, 32, 4096, 128  # 1 GiB of dS
