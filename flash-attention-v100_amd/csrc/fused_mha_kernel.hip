@@ -2684,11 +2684,15 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   float* lse2 = delta + (long)batch * head * n;
   half_t* ds = spill ? (half_t*)((char*)delta + spill_offset(batch, head, n)) : nullptr;
   const int np = padded_n(n);
-  // dS that the 256 MiB Infinity Cache can hold next to the rest stays there between the two passes if neither is told
-  // that it is used once (B1 H8 N2048, 64 MiB: backward 82 -> 77 us); at 128 MiB and above the hint is the better choice,
-  // and for a few MiB too (B2 H4 N700 causal, 5 MiB: 34.7 against 36.2 us).
+  // dS stays in the 256 MiB Infinity Cache between the two passes if neither is told that it is used once: where it fits
+  // together with the six tensors the passes touch, and from 10 MiB on.  Forward and backward, us without and with the hint
+  // (dS; with the tensors, MiB): B1 H4 N1024 59.5, 60.4 (8; 14), B1 H16 N512 40.7, 39.8 (8; 14), B1 H10 N1024 causal 63.3,
+  // 65.2 (10; 25), B1 H4 N2048 causal 101, 106 (16; 28), B1 H8 N4096 causal 207, 224 (128; 176), B1 H11 N4096 causal 240,
+  // 254 (176; 242), B3 H20 N1031 203, 207 (152; 243), H224 N512 185, 179 (112; 280), H88 N1024 237, 227 (176; 308), B1 H16
+  // N4096 causal 305, 300 (256; 352), H64 N4096 causal 1217, 1161 (1024; 1408).
   const size_t ds_bytes = slice_bytes(n) * (spill ? slices_at_once : 0) / (CAUSAL ? 2 : 1);
-  const int stream_ds = ds_bytes < (24u << 20) || ds_bytes > (96u << 20);
+  const size_t touched = ds_bytes + 6 * (size_t)slices_at_once * n * D * sizeof(half_t);
+  const int stream_ds = ds_bytes < (10u << 20) || touched > (256u << 20);
   if ((passes & kPassDelta) && !dq_makes_stats) {
     const long rows = (long)batch * n * head;
     const long threads = rows * (D / 8);

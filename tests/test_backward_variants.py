@@ -81,6 +81,26 @@ def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,N,causal", [
+    (4, 1024, False), (5, 1024, False),      # 8 MiB of dS: stored with the used-once hint; 10 MiB: without
+    (5, 1025, True), (9, 1025, True),        # 6.3 and 11.4 MiB of dS
+    (63, 1031, False), (64, 1031, False),    # 255 and 259 MiB of dS and tensors
+    (71, 1031, True), (106, 1031, True),     # 197 and 294 MiB
+])
+def test_hint_on_the_stores_of_ds(H, N, causal):
+    """Both sides of the lines between dS stored with and without the hint: the gradients of the recomputing path (dQ
+    sums the same products in another order)."""
+    D, lib = 128, abi.load()
+    gen = torch.Generator(device="cuda").manual_seed(N + H)
+    q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+    want = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=True)
+    got = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal)
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    assert (got[0].float() - want[0].float()).abs().max() <= 2e-3
+
+
+@pytest.mark.gpu
 def test_backward_without_memory_for_the_spill():
     from flash_attn_v100 import flash_attn_func
     B, H, N, D = 1, 32, 4096, 128  # 1 GiB of dS
