@@ -30,6 +30,46 @@ def test_backward_d64(N, causal):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 129, 200, 321])
+def test_backward_d64_strided(N, causal):
+    """q, k, v and dout each with strides of their own: the bits of dense copies."""
+    B, H, D = 2, 3, 64
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    normal = lambda *shape: torch.randn(shape, device="cuda", dtype=torch.float16, generator=gen)
+    q = normal(B, N, 3, H, D)[:, :, 1]          # a slice of a packed projection
+    k = normal(B, H, N, D).transpose(1, 2)      # backed by (batch, heads, seqlen, head_size)
+    v = normal(B, N, H, D + 8)[..., :D]         # rows longer than the head size
+    do = normal(N, B, H, D).transpose(0, 1)     # sequence first
+    assert len({t.stride() for t in (q, k, v, do)}) == 4
+    lib, scale = abi.load(), D ** -0.5
+    dense = [t.contiguous() for t in (q, k, v, do)]
+    out, lse = abi.forward(lib, *dense[:3], scale, causal)
+    got = abi.backward_strided(lib, q, k, v, out, do, lse, scale, causal)
+    want = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 33, 64, 100, 128, 257, 500])
+def test_backward_d64_has_the_bits_of_the_general_passes(N, causal):
+    """Features that are zero add nothing to any sum, so D = 64 problems padded to D = 128 give the recomputing kernels of
+    that size the same products to add, in the order that the D = 64 kernels have to keep: bit for bit the same."""
+    B, H, D = 2, 3, 64
+    q, k, v, do = (t.cuda() for t in ao.make_inputs(B, N, H, D, seed=N))
+    lib, scale = abi.load(), D ** -0.5
+    out, lse = abi.forward(lib, q, k, v, scale, causal)
+    got = abi.backward(lib, q, k, v, out, do, lse, scale, causal)
+    wide = [torch.nn.functional.pad(t, (0, D)) for t in (q, k, v, out, do)]
+    want = abi.backward(lib, *wide, lse, scale, causal, min_workspace=True)
+    for a, b in zip(got[:3], want[:3]):
+        assert torch.equal(a, b[..., :D]) and not b[..., D:].any()
+    assert torch.equal(got[3], want[3])  # delta
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,H,N,room", [
     (1, 1025, 64, 512),   # three rounds of 344 slices, the last one smaller
     (2, 129, 129, 256),   # two rounds, the workspace one slice pair short of one

@@ -112,3 +112,37 @@ def test_a_slice_alone_gives_the_same_bits(B, H, N, causal):
             one = [t[b:b + 1, :, h:h + 1].contiguous() for t in (q, k, v)]
             o1, l1 = abi.forward(lib, *one, scale, causal)
             assert torch.equal(o1, out[b:b + 1, :, h:h + 1]) and torch.equal(l1, lse[b:b + 1, h:h + 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,D,causal", [
+    (1, 3, 449, 64, False), (1, 3, 449, 64, True), (1, 3, 449, 128, False), (1, 3, 449, 128, True),
+    (5, 17, 700, 128, False), (1, 64, 2048, 128, True),  # persistent: 255 blocks, and one pair of blocks per unit
+])
+def test_rows_that_are_not_finite(B, H, N, D, causal):
+    """Queries with a NaN or an infinity give NaN rows and make their wave raise its maximum at every tile; the finite rows
+    beside them, in the forward and in dQ, stay within the usual bounds, and other heads keep their bits."""
+    bad = [5, 40, 41, N - 1]
+    q, k, v, do = ao.make_inputs(B, N, H, D, seed=9)
+    lib, scale, h = abi.load(), D ** -0.5, 1
+    clean = q.clone()
+    q[:, bad[:2], h, 3] = float("nan")
+    q[:, bad[2:], h, 7] = float("inf")
+    qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
+    out, lse = abi.forward(lib, qg, kg, vg, scale, causal)
+    dq, dk, dv = abi.backward(lib, qg, kg, vg, out, dog, lse, scale, causal)[:3]
+    out0, lse0 = abi.forward(lib, clean.cuda(), kg, vg, scale, causal)
+    others = [i for i in range(H) if i != h]
+    assert torch.equal(out[:, :, others], out0[:, :, others]) and torch.equal(lse[:, others], lse0[:, others])
+    grads0 = abi.backward(lib, clean.cuda(), kg, vg, out0, dog, lse0, scale, causal)[:3]
+    for a, b in zip((dq, dk, dv), grads0):
+        assert torch.equal(a[:, :, others], b[:, :, others])
+    good = [i for i in range(N) if i not in bad]
+    one = [t[:, :, h:h + 1] for t in (clean, k, v, do)]
+    ref, ref_lse = ao.attention_forward(*one[:3], scale, causal)
+    ref_dq = ao.attention_backward(*one, scale, causal)[0]
+    assert torch.isnan(out[:, bad, h]).all() and torch.isnan(dq[:, bad, h]).all()
+    # the repository's bounds for O, the logsumexp and gradients of order 1
+    assert (out[:, good, h].float().cpu() - ref[:, good, 0].half().float()).abs().max() <= 2e-3
+    assert (lse[:, h, good].cpu() - ref_lse[:, 0, good]).abs().max() <= 2e-3
+    assert (dq[:, good, h].float().cpu() - ref_dq[:, good, 0].half().float()).abs().max() <= 1e-2
