@@ -80,9 +80,11 @@ FMHA_HOST_DEVICE bool fmha_even_shares(int slices, int blocks_per_slice, int G, 
 // Launches of one block per work group that the hardware hands out as CUs become free, two or more to a CU.
 // heavy_first (causal masking, blocks numbered heaviest first): the blocks of many slices are ordered block-index
 // major, so that heavy blocks start first and the launch ends with light ones.  An XCD's slices are taken in groups of
-// kScheduledSlices (the last group holds the rest too), which keeps the rows being streamed at any time within reach
-// of the L2; groups of 8 instead of 2 took 3-19 % off the causal forward from N = 512 to 4096, 16 lost some of it
-// again.  The slices % 8 that no XCD has for itself go one block per level to successive XCDs, in the last group.
+// kScheduledSlices (the last group holds the rest too): groups of 8 instead of 2 took 3-19 % off the causal forward
+// from N = 512 to 4096, 16 lost some of it again.  The rows that 8 slices stream fit the XCD's 4 MiB of L2 up to N =
+// 1024 at D = 128; past that some are read again (dK/dV pass at B2 H32 N4096: 748 MB instead of 283 come from beyond
+// the L2) for no time that could be measured: that pass is 1 % faster than with groups of 2, the dQ pass after it 2 %
+// slower.  The slices % 8 that no XCD has for itself go one block per level to successive XCDs, in the last group.
 // Otherwise (all blocks weigh the same) the order is fmha_slice_and_block's, except that with short_last the last block
 // of every slice, which has fewer rows, comes at the end of the launch.
 constexpr int kScheduledSlices = 8;

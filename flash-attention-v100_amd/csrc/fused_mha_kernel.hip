@@ -9,7 +9,9 @@
 //     MFMA B operands for the whole kernel.  The other sequence dimension is
 //     streamed through LDS in 64-row tiles shared by the waves of a block.
 //   * Tiles go global -> LDS with global_load_lds_dwordx4 (no registers in
-//     between) into a 3-slot ring, two tiles ahead of their use; one barrier
+//     between) into a ring of two to four slots, two tiles ahead of their use
+//     where one work group has the CU (256-query forward, D = 128 backward), one
+//     ahead where two share it (128-query forward, D = 64 backward); one barrier
 //     per tile.  The LDS layout is XOR-swizzled so that both the row-wise
 //     128-bit reads and the transposing ds_read_b64_tr_b16 reads are free of
 //     bank conflicts without padding.
@@ -18,8 +20,10 @@
 //     block.  Row statistics (max, sum, logsumexp, delta) are therefore plain
 //     per-lane scalars plus one exchange between the two 32-lane halves.
 //   * The accumulator registers of the first GEMM, rounded to fp16, are
-//     already laid out as the B operand of the second GEMM, so P and dS never
-//     travel through LDS.  The matching A operand (V^T, K^T, Q^T, dO^T) is read
+//     already laid out as the B operand of the second GEMM.  P and dS therefore
+//     need no shuffling; they go through LDS only in the D = 128 backward, where
+//     the waves of a pair hand P over, lane for lane, and where dS comes back from
+//     memory.  The matching A operand (V^T, K^T, Q^T, dO^T) is read
 //     transposed out of the same row-major tile.
 //   * The backward is split into a dQ pass (query-block parallel) and a dK/dV
 //     pass (key-block parallel): no atomics, no fp32 dQ scratch, deterministic.
@@ -378,7 +382,7 @@ struct Strides {
 
 // ---------------------------------------------------------------------------
 // Forward for D = 128 where blocks of 256 queries share out evenly over the CUs
-// (rule: launch_forward).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
+// (rule: persistent_forward_pays).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
 // tiles of 64 keys stream through a 3-slot LDS ring, copied asynchronously two
 // tiles ahead.
 //
@@ -744,8 +748,8 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 }
 
 // ---------------------------------------------------------------------------
-// Forward for D = 64, and for D = 128 where blocks of 256 queries would leave CUs idle (rule: launch_forward).  Block = 4
-// waves, one per SIMD, of 32 queries each; two blocks share a CU.
+// Forward for D = 64, and for D = 128 where blocks of 256 queries do not share out evenly (rule:
+// persistent_forward_pays).  Block = 4 waves, one per SIMD, of 32 queries each; two blocks share a CU.
 //
 // What bounds it: a wave issues one instruction every 4-5 cycles, so one that runs scores, softmax and accumulation one
 // after the other needs 1,800 cycles per 32 x 64 tile at D = 64 (MFMA 512, vector instructions 700) and a SIMD needs
@@ -758,8 +762,8 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 // causal 41 -> 31 us, B4 H16 N1024 D64 causal 24 -> 17 us, B16 H12 N512 D64 24 -> 20 us, B3 H20 N1031 D128 67 -> 50 us.
 // Three blocks per CU at D = 64 (168 registers) gain 2 % on the long shape and lose 2-5 % on the short ones: not taken.
 //
-// The maximum is handled as in fmha_fwd_kernel.  Bringing it up to date happens outside the main loop, so that the loop
-// itself holds nothing twice.  K and V have two slots each; a tile is copied one tile ahead of its use.
+// The maximum is handled as in fmha_fwd_kernel.  Bringing it up to date happens outside the main loop.  K and V have two
+// slots each; a tile is copied one tile ahead of its use.
 // ---------------------------------------------------------------------------
 constexpr int kPipeWaves = 4;
 constexpr int kPipeThreads = kPipeWaves * 64;
@@ -1068,7 +1072,9 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     for (int rb = 0; rb < 2; ++rb) sA[rb] = sB[rb];
     // Main loop, two tiles per round, the scores alternating between two sets of registers: those of odd tiles in
     // sA, of even ones in sB.  It is left where a tile's probabilities came out too large, so that what has to be
-    // done then costs it no registers.
+    // done then is not held twice.  At D = 128 the kernel still uses all 256 registers and spills three (16 bytes of
+    // scratch per lane): two across the whole loop, one in the path that raises the maximum, where the reload waits for
+    // the tile copies in flight.  Nothing is spilled or reloaded inside a step.
     bool odd_done = false;
     for (;;) {
       int why;
@@ -1954,8 +1960,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       if (SPILL) step_copy(it);
       if (prev_active) gemm2(q_ring + ((it - 1) & 3) * T::kBytes, y);
       if (SPILL && prev_active) {
-        // dS(it - 1) leaves here, between the two GEMMs and away from the tile copies, which all waves issue
-        // right after the barrier: the stores go through the same path and would queue behind them.
+        // dS(it - 1) leaves here, between the two GEMMs: behind this wave's tile copies by a GEMM and before those of
+        // role A, which come at the end of the iteration.  The stores go through the same path and would queue.
         const int t = t_begin + it - 1;  // the query tile
         half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048;
         if constexpr (!KEEP) {
