@@ -400,7 +400,7 @@ def test_spill_and_recompute_backward_agree(lib, B, H, N, D, causal):
     assert torch.isfinite(dq_s).all()
 
 
-TWO_PANEL_CASES = [  # B, H, N, D, causal: at least 1024 blocks of 256 queries
+TWO_PANEL_CASES = [  # B, H, N, D, causal: at least 1024 blocks of 256 queries (D = 64: recomputes with any workspace)
     (8, 32, 1024, 128, True), (7, 32, 1100, 64, True), (4, 64, 1000, 64, False), (7, 32, 1100, 128, False),
     (8, 32, 777, 128, True),
 ]
