@@ -331,6 +331,14 @@ __device__ __forceinline__ void wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt immediate");  // bits 3:0 and 15:14 of the immediate
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
+// Wait until at most n (0 to 4) of this wave's LDS reads are on their way.
+__device__ __forceinline__ void wait_lds(int n) {
+  if (n == 0) __builtin_amdgcn_s_waitcnt(0xC07F);
+  else if (n == 1) __builtin_amdgcn_s_waitcnt(0xC17F);
+  else if (n == 2) __builtin_amdgcn_s_waitcnt(0xC27F);
+  else if (n == 3) __builtin_amdgcn_s_waitcnt(0xC37F);
+  else __builtin_amdgcn_s_waitcnt(0xC47F);
+}
 __device__ __forceinline__ void block_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's LDS reads have landed
   asm volatile("" ::: "memory");       // keep LDS accesses on their side of the barrier
@@ -1008,6 +1016,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       const int ch = m / (2 * kDB), in = m % (2 * kDB);
       return in < kDB ? v_frag(at, ch * kDB + in) : k_frag(at, ch * kDB + in - kDB);
     };
+    auto reads = [](int m) { return m >= kM ? 0 : m % (2 * kDB) < kDB ? 2 : 1; };  // LDS reads of a fragment
     auto start = [&](int x) __attribute__((always_inline)) {
       const int c16 = x >> 2, e = (x & 3) * 2;
       p0 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e], c, -mc));
@@ -1033,6 +1042,15 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 #pragma unroll
     for (int m = 0; m < kM + 2; ++m) {
       if (kCopyKAt != 0 && m == kCopyKAt && j + 2 < nt) copy_k(j + 2, 1 - kSlot);
+      if (m < kM && m % 2 == 0) {
+        // One wait for the fragments of this unit and the next instead of the compiler's one before each: a wave alone on
+        // its SIMD pays for every instruction.  B1 H4 N8192 D64: 80.2 -> 79.2 us, B1 H12 N8192 D64: 217 -> 214, B1 H32
+        // N1500 D128 causal: 29.6 -> 28.8, B1 H2 N4000 D128: 51.0 -> 49.1.  At D = 128 the first MFMA may move before it
+        // (pinned: 50.0).
+        if (D == 64) __builtin_amdgcn_sched_barrier(0);
+        wait_lds(reads(m + 2));
+        if (D == 64) __builtin_amdgcn_sched_barrier(0);
+      }
       if (m < kM) {
         const int ch = m / (2 * kDB), in = m % (2 * kDB);
         if (in < kDB) {
