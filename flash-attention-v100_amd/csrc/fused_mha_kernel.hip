@@ -75,6 +75,7 @@ struct TileGeom {
 __device__ __forceinline__ f16v mfma(h8 a, h8 b, f16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ f4v mfma16(h8 a, h8 b, f4v c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -189,11 +190,12 @@ struct PersistentBlocks {
 // 4 lanes reading one 64-byte row segment.  The tile is an array of such 1 KiB
 // blocks, block (R, C) = rows 16R..16R+15, bytes 64C..64C+63 of each row.
 // Inside a block the 16-byte chunk c4 of row r16 sits at
-//     r16 * 64 + ((c4 ^ (r16 >> 2)) * 16),
-// which makes both read patterns below bank-conflict free without padding:
-//   rows:  16 lanes read the same chunk of 16 consecutive rows  (128-bit reads)
-//   cols:  16 lanes read 4 rows x 32 bytes, transposed         (ds_read_b64_tr_b16)
+//     r16 * 64 + ((c4 ^ swz(r16 >> 2)) * 16),
+// which makes all read patterns below bank-conflict free without padding:
+//   rows:  16 lanes read the same chunk of 16 rows      (128-bit reads)
+//   cols:  16 lanes read 4 rows x 32 bytes, transposed  (ds_read_b64_tr_b16)
 // ---------------------------------------------------------------------------
+__host__ __device__ constexpr int swz(int rows4) { return -rows4 & 3; }
 template <int D>
 struct SwzTile {
   static constexpr int kNC = D / 32;              // 64-byte column groups per row
@@ -208,7 +210,7 @@ template <int D>
 __device__ __forceinline__ void copy_src(int t, int lane, int row_stride, int& row, int& goff) {
   const int R = t / SwzTile<D>::kNC, C = t % SwzTile<D>::kNC;
   const int r16 = lane >> 2, pos = lane & 3;
-  const int c4 = pos ^ (r16 >> 2);
+  const int c4 = pos ^ swz(r16 >> 2);
   row = 16 * R + r16;
   goff = (row * row_stride + (4 * C + c4) * 8) * 2;  // bytes
 }
@@ -272,7 +274,7 @@ __device__ __forceinline__ void copy4(const float* base, int voff, char* lds_dst
 // Two lane offsets (kk even / odd); the rest is an immediate.
 template <int D>
 __device__ __forceinline__ void swz_rows_off(int lane, int (&off)[2]) {
-  const int i = lane & 31, hh = lane >> 5, r16 = i & 15, g = r16 >> 2;
+  const int i = lane & 31, hh = lane >> 5, r16 = i & 15, g = swz(r16 >> 2);
   const int base = (i >> 4) * SwzTile<D>::kNC * 1024 + r16 * 64;
   off[0] = base + ((hh ^ g) * 16);
   off[1] = base + (((2 + hh) ^ g) * 16);
@@ -290,7 +292,7 @@ __device__ __forceinline__ void swz_cols_off(int lane, int (&off)[2]) {
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int r16 = 8 * e + 4 * hh + (L >> 2);
-    off[e] = r16 * 64 + ((c4 ^ (r16 >> 2)) * 16) + (L & 1) * 8;
+    off[e] = r16 * 64 + ((c4 ^ swz(r16 >> 2)) * 16) + (L & 1) * 8;
   }
 }
 template <int D>
@@ -322,6 +324,103 @@ __device__ __forceinline__ h8 swz_cols_at(unsigned a0, unsigned a1, int c16, int
   s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)(a0 + o));
   s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)(a1 + o));
   return __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// ---------------------------------------------------------------------------
+// 16 x 16 x 32 MFMAs over the same tiles.  At the power cap they do 13 % more products per second than the 32 x 32 x 16
+// ones (registers only, random operands, all CUs busy: 1,766 against 1,555 TFLOP/s; with each A operand read from LDS for
+// 2 x 16 columns 1,580 against 1,400), so the kernels that run there use them.  They are twice as many instructions, which
+// a wave alone on its SIMD feels (B1 H2 N4000 forward: 51 -> 59 us), and where vector instructions are the bound they gain
+// nothing (B1 H12 N8192 D64 forward: 218 -> 223 us): those kernels keep the others.
+//
+// Both give the same bits.  One 16 x 16 x 32 MFMA adds the products of its lanes 0..31 first, then those of lanes
+// 32..63, each the way a 32 x 32 x 16 MFMA adds its 16; and the streamed rows are dealt out so that these are the same 16:
+// of 32 streamed rows kc, row block p (0 or 1) has, in MFMA row 4 g + r (held by lanes 16 g .. in register r), the row
+//     32 kc + 16 (g >> 1) + 8 p + 4 (g & 1) + r.
+// The second GEMM takes rows 32 kc .. as one step, register e = 4 p + r of lane group g as its k = 8 g + e.
+// ---------------------------------------------------------------------------
+template <int D>
+struct Geom16 {
+  static constexpr int kKS = D / 32;  // steps over the features
+  static constexpr int kDB = D / 16;  // blocks of 16 features
+};
+// first of the four streamed rows, inside 32, that lane group g holds in row block p
+__device__ __forceinline__ int acc16_row(int p, int g) { return 16 * (g >> 1) + 8 * p + 4 * (g & 1); }
+// rows pattern: lane (m, g) reads chunk g of the row of MFMA row m; two lane offsets (row block even / odd).
+template <int D>
+__device__ __forceinline__ int rows16_off(int lane, int p) {
+  const int m = lane & 15, g = lane >> 4, r16 = 8 * p + (m & 7);
+  return (m >> 3) * SwzTile<D>::kNC * 1024 + r16 * 64 + ((g ^ swz(r16 >> 2)) * 16);
+}
+template <int D>
+__device__ __forceinline__ h8 rows16_at(unsigned a_even, unsigned a_odd, int rb, int kk) {
+  typedef __attribute__((address_space(3))) h8 lds_h8;
+  return *(const lds_h8*)(uintptr_t)(((rb & 1) ? a_odd : a_even) + (unsigned)SwzTile<D>::block_off(rb & 2, kk));
+}
+// cols pattern: MFMA A operand, rows = features 16 db + (lane & 15), k = 32 streamed rows kc in accumulator order.  Two
+// lane offsets (rows +0 / +8) for even db; odd ones are 32 bytes away, one way or the other.
+template <int D>
+__device__ __forceinline__ int cols16_off(int lane, int p, int odd) {
+  const int L = lane & 15, g = lane >> 4, r16 = 8 * p + 4 * (g & 1) + (L >> 2);
+  return (g >> 1) * SwzTile<D>::kNC * 1024 + r16 * 64 + (((2 * odd + ((L & 3) >> 1)) ^ swz(r16 >> 2)) * 16) + (L & 1) * 8;
+}
+template <int D>
+struct Cols16 {
+  unsigned a[2][2];  // [rows +0 / +8][feature block even / odd]
+  __device__ __forceinline__ Cols16(const char* tile, int lane) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int odd = 0; odd < 2; ++odd) a[p][odd] = opaque_lds_address(tile + cols16_off<D>(lane, p, odd));
+  }
+  __device__ __forceinline__ h8 at(unsigned slot, int kc, int db) const {
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    const unsigned o = slot + SwzTile<D>::block_off(2 * kc, db >> 1);
+    s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)(a[0][db & 1] + o));
+    s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)(a[1][db & 1] + o));
+    return __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+};
+// Over the four lanes with the same l & 15: first the two that are 32 apart, then the others.
+__device__ __forceinline__ float max_over_groups(float x) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
+  x = fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_int(x), __float_as_int(x), false, false);
+  return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+// store_resident for accumulators of 16 x 16 blocks: acc[db][cb] has features 16 db + 4 g + 0..3 of resident position
+// 16 cb + (lane & 15), to be scaled by mul[cb].
+template <int D>
+struct Stage16 {
+  // bytes per row: the 8-byte pieces that 32 lanes write, 16 rows x 2, fall on different banks
+  static constexpr int kPitch = D * 2 + 16;
+  static constexpr int kBytes = kResident * kPitch;  // per wave
+};
+template <int D>
+__device__ __forceinline__ void store_resident16(half_t* __restrict__ base, long row_stride, int row0, int n,
+                                                 const f4v (*acc)[2], const float (&mul)[2], int lane,
+                                                 char* __restrict__ stage) {
+  constexpr int kPitch = Stage16<D>::kPitch;
+  char* mine = stage + (lane & 15) * kPitch + (lane >> 4) * 8;
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      h4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (half_t)(acc[db][cb][e] * mul[cb]);
+      *reinterpret_cast<h4*>(mine + cb * 16 * kPitch + db * 32) = v;
+    }
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own writes have landed
+  asm volatile("" ::: "memory");
+  constexpr int kLanesPerRow = D / 8, kRowsPerPass = 64 / kLanesPerRow;
+  const int r_in = lane / kLanesPerRow, ch = lane % kLanesPerRow;
+#pragma unroll
+  for (int pass = 0; pass < kResident / kRowsPerPass; ++pass) {
+    const int r = pass * kRowsPerPass + r_in;
+    const h8 v = *reinterpret_cast<const h8*>(stage + r * kPitch + ch * 16);
+    if (row0 + r < n) *reinterpret_cast<h8*>(base + (long)(row0 + r) * row_stride + ch * 8) = v;
+  }
 }
 
 // s_waitcnt vmcnt(N) with the other counters left alone.  Issued through the
@@ -397,7 +496,7 @@ struct Strides {
 // Online softmax as in reference kernel/fused_mha_kernel.cu:159-181, except that
 // no tile's maximum is looked for as long as the running one serves: the
 // probabilities of a tile are formed relative to the running maximum first, and
-// only if a lane's sum over its 32 keys of the tile exceeds kRescaleSum (so every
+// only if the sum of half of them (32 keys of a query) exceeds kRescaleSum (so every
 // single one stays far below the fp16 range) or is no number (no maximum yet) the
 // maximum is raised, O and l are rescaled, and they are formed again.  That takes
 // the 16 max instructions and the exchange between the half waves out of nearly
@@ -409,6 +508,9 @@ struct Strides {
 // 4-7 do  softmax(j-1), accumulate(j-1), scores(j).  Both need exactly K(j)
 // and V(j-1) in iteration j, so one barrier per iteration is enough, and one
 // wave's MFMA stretch coincides with the other's VALU stretch.
+//
+// What bounds it is the power cap; 16 x 16 x 32 MFMAs take less of it (Geom16).  B2 H32 N4096 D128 causal 258 -> 244 us,
+// without a mask 473 -> 442 us (1.24 PFLOP/s), B1 H16 N16384 causal 1016 -> 950.
 // ---------------------------------------------------------------------------
 constexpr float kRescaleSum = 4096.f;
 constexpr int kFwdWaves = 8;
@@ -428,20 +530,20 @@ __global__ void __launch_bounds__(kFwdThreads, 1)
 fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                 Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
                 int nmb, int total, float c, int negate_q) {
-  using G = TileGeom<D>;
+  using G = Geom16<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kFwdWaves;  // copy instructions per wave per tile
   // K ring then V ring, kRing slots each, then per wave a staging tile for 64 features of
   // its 32 output rows.  The copies into the ring are inline asm (see copy16), so slots
   // can be addressed at run time.
-  __shared__ __attribute__((aligned(1024))) char smem[2 * kRing * T::kBytes + kFwdWaves * StageGeom<64>::kBytes];
+  __shared__ __attribute__((aligned(1024))) char smem[2 * kRing * T::kBytes + kFwdWaves * Stage16<64>::kBytes];
   char* const k_ring = smem;
   char* const v_ring = smem + kRing * T::kBytes;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i = lane & 31, hh = lane >> 5;
-  char* const stage = smem + 2 * kRing * T::kBytes + wave * StageGeom<64>::kBytes;
+  const int i = lane & 15, g = lane >> 4;
+  char* const stage = smem + 2 * kRing * T::kBytes + wave * Stage16<64>::kBytes;
   const int rs = H * D;  // O is dense
   const int nt_all = (N + kTile - 1) / kTile;
   const PersistentBlocks pb{total};
@@ -493,114 +595,127 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
     }
   };
 
-  h8 qf[G::kKSteps];
+  h8 qf[G::kKS][2];
   auto load_q = [&](const Block& B) __attribute__((always_inline)) {
-    const half_t* qp = B.q + (long)min(B.m0 + wave * kResident + i, N - 1) * qs.n + hh * 8;
 #pragma unroll
-    for (int kk = 0; kk < G::kKSteps; ++kk) qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
+    for (int cb = 0; cb < 2; ++cb) {
+      const half_t* qp = B.q + (long)min(B.m0 + wave * kResident + cb * 16 + i, N - 1) * qs.n + g * 8;
+#pragma unroll
+      for (int kk = 0; kk < G::kKS; ++kk) qf[kk][cb] = *reinterpret_cast<const h8*>(qp + kk * 32);
+    }
+  };
+  auto negate = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < G::kKS; ++kk) {
+      qf[kk][0] = -qf[kk][0];
+      qf[kk][1] = -qf[kk][1];
+    }
   };
 
-  int k_off[2], v_off[2];
-  swz_rows_off<D>(lane, k_off);
-  swz_cols_off<D>(lane, v_off);
+  const int k_off0 = rows16_off<D>(lane, 0), k_off1 = rows16_off<D>(lane, 1);
 
-  // state of the block being worked on
-  int q0w = 0, qi = 0, ntw = 0;
-  f16v o[G::kDBlocks];
-  float mc = -INFINITY, l_run = 0.f;  // running maximum times c
-  f16v s[2];   // scores of the tile in flight
-  h8 pf[4];    // its probabilities, fp16, B-operand order
+  // state of the block being worked on; [2]: of this lane's queries q0w + i and q0w + 16 + i
+  int q0w = 0, ntw = 0;
+  f4v o[G::kDB][2];
+  float mc[2] = {-INFINITY, -INFINITY};  // running maximum times c
+  float l_run = 0.f;  // lanes 0..31: of query q0w + i, lanes 32..63: of q0w + 16 + i; over the keys of lane groups g and g ^ 2
+  f4v s[4][2];   // scores of the tile in flight
+  h8 pf[2][2];   // its probabilities, fp16, B-operand order
 
-  // The fragment reads of both GEMMs run kLead MFMAs ahead of their use.  The order is written out
-  // and pinned with scheduling barriers: left to itself the scheduler, once registers get scarce,
+  // The fragment reads of both GEMMs run kLead units (of one fragment and two MFMAs) ahead of their use.  The order is
+  // written out and pinned with scheduling barriers: left to itself the scheduler, once registers get scarce,
   // puts every read right before its MFMA, which then waits a full LDS round trip each time.
   constexpr int kLead = 4;
+  constexpr int kN = 4 * G::kKS;  // units of either GEMM
+  static_assert(kN == 2 * G::kDB, "");
   auto scores = [&](const char* Kl, int t) __attribute__((always_inline)) {
     if (t >= ntw) return;
-    constexpr int kN = 2 * G::kKSteps;  // MFMA n: key block rb = n & 1, feature step kk = n >> 1
-    h8 frag[kLead];
+    const unsigned a0 = opaque_lds_address(Kl + k_off0), a1 = opaque_lds_address(Kl + k_off1);
+    h8 frag[kLead];  // unit n: row block rb = n & 3, feature step kk = n >> 2
 #pragma unroll
-    for (int n = 0; n < kLead; ++n) frag[n] = swz_rows<D>(Kl, n & 1, n >> 1, k_off);
+    for (int n = 0; n < kLead; ++n) frag[n] = rows16_at<D>(a0, a1, n & 3, n >> 2);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < kN; ++n) {
-      const int rb = n & 1, kk = n >> 1;
-      if (kk == 0) {
-        f16v zero;
+      const int rb = n & 3, kk = n >> 2;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-        s[rb] = mfma(frag[n % kLead], qf[kk], zero);
-      } else {
-        s[rb] = mfma(frag[n % kLead], qf[kk], s[rb]);
-      }
-      if (n + kLead < kN) frag[n % kLead] = swz_rows<D>(Kl, (n + kLead) & 1, (n + kLead) >> 1, k_off);
+      for (int cb = 0; cb < 2; ++cb)
+        s[rb][cb] = mfma16(frag[n % kLead], qf[kk][cb], kk == 0 ? f4v{0.f, 0.f, 0.f, 0.f} : s[rb][cb]);
+      if (n + kLead < kN) frag[n % kLead] = rows16_at<D>(a0, a1, (n + kLead) & 3, (n + kLead) >> 2);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto exponentials = [&]() __attribute__((always_inline)) {
-    float l0 = 0.f, l1 = 0.f;
+  auto exponentials = [&]() __attribute__((always_inline)) {  // returns the tile's part of l_run
+    float l[2] = {0.f, 0.f};
 #pragma unroll
-    for (int c16 = 0; c16 < 4; ++c16) {
+    for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const float p0 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e], c, -mc));
-        const float p1 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e + 1], c, -mc));
-        pf[c16][e] = (half_t)p0;
-        pf[c16][e + 1] = (half_t)p1;
-        l0 += p0;
-        l1 += p1;
-      }
-    }
-    return l0 + l1;
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p = fast_exp2(fmaf(s[2 * kc + (e >> 2)][cb][e & 3], c, -mc[cb]));
+          pf[kc][cb][e] = (half_t)p;
+          l[cb] += p;
+        }
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(l[0]), __float_as_int(l[1]), false, false);
+    return __int_as_float(r[0]) + __int_as_float(r[1]);
   };
   auto softmax = [&](int t) __attribute__((always_inline)) {
     if (t < 0 || t >= ntw) return;
     const int key0 = t * kTile;
     if ((CAUSAL && key0 + kTile - 1 > q0w) || (key0 + kTile > N)) {
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
+      for (int cb = 0; cb < 2; ++cb) {
+        const int last = (CAUSAL ? min(q0w + cb * 16 + i, N - 1) : N - 1) - key0 - acc16_row(0, g);  // last key that counts
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          int key = key0 + acc_row(rb, r, hh);
-          if ((CAUSAL && key > qi) || key >= N) s[rb][r] = -INFINITY;
-        }
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if ((rb >> 1) * 32 + (rb & 1) * 8 + r > last) s[rb][cb][r] = -INFINITY;
+      }
     }
-    // Optimistic: probabilities relative to the running maximum as it stands.  If any lane's sum over its 32 keys is
-    // past kRescaleSum (or not a number: no maximum yet), the maximum is brought up to date and they are formed again.
+    // Optimistic: probabilities relative to the running maximum as it stands.  If the sum over the 32 keys of a query
+    // that lane groups g and g ^ 2 have is past kRescaleSum (or not a number: no maximum yet), the maximum is brought up to date and they are formed again.
     // A wave's last tile always brings it up to date, as in fmha_fwd_pipe_kernel: both kernels give the same bits, so
     // that a slice's result does not depend on how many others the call has.
     float lt = exponentials();
     if (t == ntw - 1 || __builtin_amdgcn_ballot_w64(!(lt <= kRescaleSum)) != 0) {
-      float mx = s[0][0];
+      float alpha[2];
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
+      for (int cb = 0; cb < 2; ++cb) {
+        float mx = s[0][cb][0];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
-      mx = fmaxf(mx, other_half(mx));
-      const float mc_new = fmaxf(mc, mx * c);
-      const float alpha = fast_exp2(mc - mc_new);
-      mc = mc_new;
-      l_run *= alpha;
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[rb][cb][r]);
+        mx = max_over_groups(mx);
+        const float mc_new = fmaxf(mc[cb], mx * c);
+        alpha[cb] = fast_exp2(mc[cb] - mc_new);
+        mc[cb] = mc_new;
+#pragma unroll
+        for (int db = 0; db < G::kDB; ++db)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[db][cb][r] *= alpha[cb];
+      }
+      l_run *= lane < 32 ? alpha[0] : alpha[1];
       asm volatile("" : "+v"(l_run));  // rounded here: contracted with the sum below the loop is 4 % slower without a mask
-#pragma unroll
-      for (int db = 0; db < G::kDBlocks; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
       lt = exponentials();
     }
     l_run += lt;
   };
   auto accumulate = [&](const char* Vl, int t) __attribute__((always_inline)) {
     if (t < 0 || t >= ntw) return;
-    constexpr int kDB = G::kDBlocks, kN = 4 * kDB;  // MFMA n: key chunk c16 = n / kDB, feature block db = n % kDB
-    h8 frag[kLead];
+    const Cols16<D> cols(Vl, lane);
+    h8 frag[kLead];  // unit n: 32 keys kc = n / kDB, feature block db = n % kDB
 #pragma unroll
-    for (int n = 0; n < kLead; ++n) frag[n] = swz_cols<D>(Vl, n / kDB, n % kDB, v_off);
+    for (int n = 0; n < kLead; ++n) frag[n] = cols.at(0, n / G::kDB, n % G::kDB);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < kN; ++n) {
-      o[n % kDB] = mfma(frag[n % kLead], pf[n / kDB], o[n % kDB]);
-      if (n + kLead < kN) frag[n % kLead] = swz_cols<D>(Vl, (n + kLead) / kDB, (n + kLead) % kDB, v_off);
+      const int kc = n / G::kDB, db = n % G::kDB;
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) o[db][cb] = mfma16(frag[n % kLead], pf[kc][cb], o[db][cb]);
+      if (n + kLead < kN) frag[n % kLead] = cols.at(0, (n + kLead) / G::kDB, (n + kLead) % G::kDB);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -639,17 +754,14 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
         nt = cur.nt;
         q0w = cur.m0 + wave * kResident;
       }
-      qi = q0w + i;
       ntw = nt;
       if (CAUSAL) {
         ntw = min(nt, (min(q0w + kResident, N) - 1) / kTile + 1);
         if (q0w >= N) ntw = 0;
       }
 #pragma unroll
-      for (int db = 0; db < G::kDBlocks; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-      mc = -INFINITY;
+      for (int db = 0; db < G::kDB; ++db) o[db][0] = o[db][1] = f4v{0.f, 0.f, 0.f, 0.f};
+      mc[0] = mc[1] = -INFINITY;
       l_run = 0.f;
       auto wait_and_sync = [&]() __attribute__((always_inline)) {
         if (in_flight == 2 * kIPW) wait_vm<2 * kIPW>();
@@ -675,10 +787,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
       int j = 0;
       for (; j + 2 < nt; ++j) {
         wait_and_sync();
-        if (j == 0 && negate_q) {
-#pragma unroll
-          for (int kk = 0; kk < G::kKSteps; ++kk) qf[kk] = -qf[kk];
-        }
+        if (j == 0 && negate_q) negate();
         copy_tile(cur_k, ks.n, c_kgoff, k_ring + s2 * T::kBytes, j + 2);
         copy_tile(cur_v, vs.n, c_vgoff, v_ring + s1 * T::kBytes, j + 1);
         in_flight = 2 * kIPW;
@@ -692,10 +801,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
         Block nxt = decode(lin_next >= 0 ? lin_next : lin_cur);
         for (; j < nt; ++j) {
           wait_and_sync();
-          if (j == 0 && negate_q) {
-#pragma unroll
-            for (int kk = 0; kk < G::kKSteps; ++kk) qf[kk] = -qf[kk];
-          }
+          if (j == 0 && negate_q) negate();
           in_flight = 0;
           const int ek = j + 2, ev = j + 1;
           if (ek < nt) {
@@ -728,13 +834,17 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
       // the block's output: O rows through this wave's staging tile, 64 features at a time
       {
         const Block cur = decode(lin_cur);
-        const float l_tot = l_run + other_half(l_run);
-        const float inv = 1.f / l_tot;
+        const auto other = __builtin_amdgcn_permlane16_swap(__float_as_int(l_run), __float_as_int(l_run), false, false);
+        const int l_sum = __float_as_int(__int_as_float(other[0]) + __int_as_float(other[1]));
+        const auto both = __builtin_amdgcn_permlane32_swap(l_sum, l_sum, false, false);
+        const float l_tot[2] = {__int_as_float(both[0]), __int_as_float(both[1])};
+        const float inv[2] = {1.f / l_tot[0], 1.f / l_tot[1]};
 #pragma unroll
         for (int part = 0; part < D / 64; ++part)
-          store_resident<64>(O + cur.o_off + part * 64, rs, q0w, N, *reinterpret_cast<const f16v(*)[2]>(&o[2 * part]),
-                             inv, lane, stage);
-        if (LSE && hh == 0 && qi < N) LSE[cur.stat_off + qi] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
+          store_resident16<64>(O + cur.o_off + part * 64, rs, q0w, N, o + 4 * part, inv, lane, stage);
+        if (LSE && lane < kResident && q0w + lane < N)
+          LSE[cur.stat_off + q0w + lane] = ((lane < 16 ? mc[0] : mc[1]) +
+                                            __builtin_amdgcn_logf(lane < 16 ? l_tot[0] : l_tot[1])) * kLn2;
       }
       if (lin_next < 0) break;
       lin_cur = lin_next;
@@ -860,7 +970,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   constexpr int kBack = 960 * (kIPW - 1);
   int k_goff, v_goff, c_past;  // c_past: how many rows past the end this lane's row of the last tile is
   {
-    const int lane = lane_now(), row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ (lane >> 4)) * 16;
+    const int lane = lane_now(), row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ swz(lane >> 4)) * 16;
     k_goff = row * ks.n * 2 + col + kBack;
     v_goff = row * vs.n * 2 + col + kBack;
     asm volatile("" : "+v"(k_goff), "+v"(v_goff));
@@ -933,6 +1043,18 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // A lane's sum over a tile has two parts.  At D = 128 the even and the odd chunks of 16 keys, which are the parts that
+  // two lanes of fmha_fwd_kernel have; at D = 64 the even and the odd keys, which wait less for each other.
+  auto add_up = [&](float& l0, float& l1, int c16, float p0, float p1) __attribute__((always_inline)) {
+    if (D == 64) {
+      l0 += p0;
+      l1 += p1;
+    } else {
+      float& l = c16 & 1 ? l1 : l0;
+      l += p0;
+      l += p1;
+    }
+  };
   auto exponentials = [&](const f16v (&s)[2]) __attribute__((always_inline)) {
     float l0 = 0.f, l1 = 0.f;
 #pragma unroll
@@ -942,8 +1064,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         const float p0 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e], c, -mc));
         const float p1 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e + 1], c, -mc));
         pf[c16][e >> 1] = pack_f16(p0, p1);
-        l0 += p0;
-        l1 += p1;
+        add_up(l0, l1, c16, p0, p1);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1024,8 +1145,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     };
     auto finish = [&](int x) __attribute__((always_inline)) {
       const int c16 = x >> 2, e = (x & 3) * 2;
-      l0 += p0;
-      l1 += p1;
+      add_up(l0, l1, c16, p0, p1);
       asm volatile("" : "+v"(l0), "+v"(l1));  // sums now, not all at the end
       pf[c16][e >> 1] = pack_f16(p0, p1);
     };
@@ -1502,7 +1622,7 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
   constexpr int kBack = 960 * (kIPW - 1);
   int k_goff, v_goff, c_past;
   {
-    const int row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ (lane >> 4)) * 16;
+    const int row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ swz(lane >> 4)) * 16;
     k_goff = row * ks.n * 2 + col + kBack;
     v_goff = row * vs.n * 2 + col + kBack;
     c_past = max((nt_all - 1) * kTile + row - (N - 1), 0) * 2;
@@ -2060,7 +2180,7 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
   constexpr int kBack = 960 * (kIPW - 1);
   int q_goff, g_goff, c_past;
   {
-    const int row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ (lane >> 4)) * 16;
+    const int row = 16 * wave + (lane >> 2), col = ((lane & 3) ^ swz(lane >> 4)) * 16;
     q_goff = row * qs.n * 2 + col + kBack;
     g_goff = row * gs.n * 2 + col + kBack;
     c_past = max((nt - 1) * kTile + row - (N - 1), 0) * 2;
