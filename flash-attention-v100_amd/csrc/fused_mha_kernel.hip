@@ -438,6 +438,12 @@ __device__ __forceinline__ void wait_lds(int n) {
   else if (n == 3) __builtin_amdgcn_s_waitcnt(0xC37F);
   else __builtin_amdgcn_s_waitcnt(0xC47F);
 }
+// The same at this place in the program, so that the compiler adds no wait of its own in front of it.
+__device__ __forceinline__ void wait_lds_pinned(int n) {
+  __builtin_amdgcn_sched_barrier(0);
+  wait_lds(n);
+  __builtin_amdgcn_sched_barrier(0);
+}
 __device__ __forceinline__ void block_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's LDS reads have landed
   asm volatile("" ::: "memory");       // keep LDS accesses on their side of the barrier
@@ -624,7 +630,8 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 
   // The fragment reads of both GEMMs run kLead units (of one fragment and two MFMAs) ahead of their use.  The order is
   // written out and pinned with scheduling barriers: left to itself the scheduler, once registers get scarce,
-  // puts every read right before its MFMA, which then waits a full LDS round trip each time.
+  // puts every read right before its MFMA, which then waits a full LDS round trip each time.  The fragments of two units
+  // are waited for together (half as many s_waitcnt: 1 % at B2 H32 N4096).
   constexpr int kLead = 4;
   constexpr int kN = 4 * G::kKS;  // units of either GEMM
   static_assert(kN == 2 * G::kDB, "");
@@ -638,6 +645,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 #pragma unroll
     for (int n = 0; n < kN; ++n) {
       const int rb = n & 3, kk = n >> 2;
+      if (n % 2 == 0) wait_lds_pinned(n + 3 < kN ? 2 : n + 2 < kN ? 1 : 0);
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb)
         s[rb][cb] = mfma16(frag[n % kLead], qf[kk][cb], kk == 0 ? f4v{0.f, 0.f, 0.f, 0.f} : s[rb][cb]);
@@ -713,6 +721,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 #pragma unroll
     for (int n = 0; n < kN; ++n) {
       const int kc = n / G::kDB, db = n % G::kDB;
+      if (n % 2 == 0) wait_lds_pinned(n + 3 < kN ? 4 : n + 2 < kN ? 2 : 0);
 #pragma unroll
       for (int cb = 0; cb < 2; ++cb) o[db][cb] = mfma16(frag[n % kLead], pf[kc][cb], o[db][cb]);
       if (n + kLead < kN) frag[n % kLead] = cols.at(0, (n + kLead) / G::kDB, (n + kLead) % G::kDB);
@@ -1167,9 +1176,8 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         // its SIMD pays for every instruction.  B1 H4 N8192 D64: 80.2 -> 79.2 us, B1 H12 N8192 D64: 217 -> 214, B1 H32
         // N1500 D128 causal: 29.6 -> 28.8, B1 H2 N4000 D128: 51.0 -> 49.1.  At D = 128 the first MFMA may move before it
         // (pinned: 50.0).
-        if (D == 64) __builtin_amdgcn_sched_barrier(0);
-        wait_lds(reads(m + 2));
-        if (D == 64) __builtin_amdgcn_sched_barrier(0);
+        if (D == 64) wait_lds_pinned(reads(m + 2));
+        else wait_lds(reads(m + 2));
       }
       if (m < kM) {
         const int ch = m / (2 * kDB), in = m % (2 * kDB);
