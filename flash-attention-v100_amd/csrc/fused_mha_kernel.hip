@@ -38,6 +38,7 @@
 #include <math.h>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 
 #include "fused_mha.h"
@@ -399,18 +400,23 @@ struct Stage16 {
 template <int D>
 __device__ __forceinline__ void store_resident16(half_t* __restrict__ base, long row_stride, int row0, int n,
                                                  const f4v (*acc)[2], const float (&mul)[2], int lane,
-                                                 char* __restrict__ stage) {
+                                                 char* __restrict__ stage, int row_of_0 = -1, int row_of_1 = -1,
+                                                 int upper_off = 16 * Stage16<D>::kPitch) {
+  // row_of_cb: the row (0..31, relative to row0) of this lane's column of block cb, when that is not 16 cb + (lane & 15);
+  // upper_off: where rows 16..31 are staged, relative to `stage`, when the staging tile is not contiguous
   constexpr int kPitch = Stage16<D>::kPitch;
-  char* mine = stage + (lane & 15) * kPitch + (lane >> 4) * 8;
 #pragma unroll
-  for (int db = 0; db < D / 16; ++db)
+  for (int cb = 0; cb < 2; ++cb) {
+    const int row = row_of_0 < 0 ? 16 * cb + (lane & 15) : cb ? row_of_1 : row_of_0;
+    char* mine = stage + (row & 15) * kPitch + (row >> 4) * upper_off + (lane >> 4) * 8;
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
+    for (int db = 0; db < D / 16; ++db) {
       h4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = (half_t)(acc[db][cb][e] * mul[cb]);
-      *reinterpret_cast<h4*>(mine + cb * 16 * kPitch + db * 32) = v;
+      *reinterpret_cast<h4*>(mine + db * 32) = v;
     }
+  }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own writes have landed
   asm volatile("" ::: "memory");
   constexpr int kLanesPerRow = D / 8, kRowsPerPass = 64 / kLanesPerRow;
@@ -418,7 +424,7 @@ __device__ __forceinline__ void store_resident16(half_t* __restrict__ base, long
 #pragma unroll
   for (int pass = 0; pass < kResident / kRowsPerPass; ++pass) {
     const int r = pass * kRowsPerPass + r_in;
-    const h8 v = *reinterpret_cast<const h8*>(stage + r * kPitch + ch * 16);
+    const h8 v = *reinterpret_cast<const h8*>(stage + (r & 15) * kPitch + (r >> 4) * upper_off + ch * 16);
     if (row0 + r < n) *reinterpret_cast<h8*>(base + (long)(row0 + r) * row_stride + ch * 8) = v;
   }
 }
@@ -1826,6 +1832,9 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
 // for lane (double-buffered).  Q tiles of 64 queries stream through a 4-slot
 // LDS ring (B still needs tile j-1), dO tiles and the tile's lse2/delta rows
 // through 3-slot rings, all copied two tiles ahead.
+// What bounds it: the MFMAs and LDS reads that the two waves of a SIMD share, and with all CUs busy the power cap, which
+// is why those launches take the 16 x 16 x 32 MFMAs (B2 H40 N2048 causal: 212 -> 201 us; B2 H32 N4096 causal, dS stored:
+// 594 -> 572 us, 957 TFLOP/s of its four products; B3 H20 N1031: 99.6 -> 96 us).
 // ---------------------------------------------------------------------------
 constexpr int kKvPairs = 4;
 constexpr int kKvWaves = 2 * kKvPairs;
@@ -1838,14 +1847,16 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // its own.  Layout per (batch, head) slice, np = n rounded up to 128:
 //   [np / 128 query blocks][np / 64 key tiles] x 16 KiB, the tile a block of 128 queries
 //   streams per 64 keys, made of 16 pieces of 1 KiB:
-//   [2 halves of 32 keys][2 query tiles of 64][4 chunks of 16 queries] x 1 KiB.
-// A 1 KiB piece is what one store instruction of wave B writes: lane l = 32 * hh + i
-// (key i, half hh) puts the 16 bytes of registers it holds for the chunk at 16 * l
-// (consecutive lanes, consecutive addresses); inside a chunk position 8*hh + e holds
-// query 8*(e >> 2) + 4*hh + (e & 3).  Rows of keys at or past n are written as zeros; (key tile, query
-// tile) pairs above the diagonal are not written (and not read) under causal masking.
+//   [2 halves of 32 keys][2 query tiles of 64][4 fragments] x 1 KiB.
+// A 1 KiB piece is what one store instruction of wave B writes: each lane puts the 16 bytes of registers it holds, an
+// operand fragment of the second GEMM, at 16 * lane (consecutive lanes, consecutive addresses).  WIDE: fragment f is
+// queries 16 f .. of the 64, lane 32 * hh + i holds key i and as element e query 8 * (e >> 2) + 4 * hh + (e & 3).
+// Otherwise fragment f is queries 32 (f >> 1) .. and keys 16 (f & 1) .., and lane 16 * g + i holds key i and as element e
+// query 16 * (g >> 1) + 8 * (e >> 2) + 4 * (g & 1) + (e & 3).  Rows of keys at or past n are written as zeros; (key tile,
+// query tile) pairs above the diagonal are not written (and not read) under causal masking.
 // KEEP: without the non-temporal hint on those stores (rule: launch_backward).
-template <int D, bool CAUSAL, bool SPILL, bool KEEP>
+// WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: launch_backward).
+template <int D, bool CAUSAL, bool SPILL, bool KEEP, bool WIDE>
 __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                      const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
@@ -1853,6 +1864,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
                      half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
                      int nnb, int slice0, float c, float scale) {
   using G = TileGeom<D>;
+  using G16 = Geom16<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kKvWaves;  // copies per wave per tile, per tensor
   // Q ring (4), dO ring (3), per stats slot 64 lse2 then 64 delta values (1 KiB, half
@@ -1869,7 +1881,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int pair = wave & (kKvPairs - 1);
   const bool role_b = wave >= kKvPairs;
-  const int i = lane & 31, hh = lane >> 5;
+  const int i = WIDE ? lane & 31 : lane & 15;        // resident position of this lane's columns, and
+  const int g = WIDE ? lane >> 5 : lane >> 4;        // which streamed rows it has
   int bh, nblk;
   // causal: low key blocks are the heavy ones and come first
   fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kKvBlockKeys != 0, bh, nblk);
@@ -1883,8 +1896,6 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 
   const int n0 = nblk * kKvBlockKeys;
   const int k0w = n0 + pair * kResident;
-  const int ki = k0w + i;
-  const int krow = min(ki, N - 1);
 
   const int nt = (N + kTile - 1) / kTile;
   const int t_begin = CAUSAL ? n0 / kTile : 0;
@@ -1932,86 +1943,156 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   copy_tiles(0);
   if (n_it > 1) copy_tiles(1);
 
-  // resident rows of this wave: K for role A, V for role B
+  // resident rows of this wave: K for role A, V for role B; [feature step] of key k0w + i, or [feature step][cb] of keys
+  // k0w + 16 cb + i
   h8 rf[G::kKSteps];
-  {
-    const half_t* rp = (role_b ? V + b * vs.b + (long)h * vs.h + (long)krow * vs.n
-                               : K + b * ks.b + (long)h * ks.h + (long)krow * ks.n) + hh * 8;
 #pragma unroll
-    for (int kk = 0; kk < G::kKSteps; ++kk) {
-      rf[kk] = *reinterpret_cast<const h8*>(rp + kk * 16);
+  for (int cb = 0; cb < (WIDE ? 1 : 2); ++cb) {
+    const int krow = min(k0w + 16 * cb + i, N - 1);
+    const half_t* rp = (role_b ? V + b * vs.b + (long)h * vs.h + (long)krow * vs.n
+                               : K + b * ks.b + (long)h * ks.h + (long)krow * ks.n) + g * 8;
+#pragma unroll
+    for (int kk = 0; kk < (WIDE ? G::kKSteps : G16::kKS); ++kk) {
+      h8& r = rf[WIDE ? kk : 2 * kk + cb];
+      r = *reinterpret_cast<const h8*>(rp + kk * (WIDE ? 16 : 32));
       // Role B works with -V: its first GEMM then gives delta - dP on top of
       // accumulators loaded with delta, with no subtraction afterwards.
-      if (role_b) rf[kk] = -rf[kk];
+      if (role_b) r = -r;
     }
   }
 
   int r_off[2], c_off[2];
-  swz_rows_off<D>(lane, r_off);
-  swz_cols_off<D>(lane, c_off);
-  const int st_off = hh * 16 + (role_b ? 256 : 0);   // + (rb * 32 + 8 * g) * 4: this role's quad
-  char* const p_mine = p_xchg + pair * 4096 + lane * 16;  // + buffer * kPBytes + rb * 2048 + half * 1024
+  if constexpr (WIDE) {
+    swz_rows_off<D>(lane, r_off);
+    swz_cols_off<D>(lane, c_off);
+  } else {
+    r_off[0] = rows16_off<D>(lane, 0);
+    r_off[1] = rows16_off<D>(lane, 1);
+  }
+  // this role's statistics of the four rows at + 4 * stat_row(quad)
+  const int st_off = (WIDE ? 4 * g : acc16_row(0, g)) * 4 + (role_b ? 256 : 0);
+  constexpr int kQuads = WIDE ? 8 : 4;
+  constexpr auto stat_row = [](int quad) { return WIDE ? 8 * quad : 32 * (quad >> 1) + 8 * (quad & 1); };
+  char* const p_mine = p_xchg + pair * 4096 + lane * 16;  // + buffer * kPBytes + 1024 * fragment
 
-  f16v acc[G::kDBlocks];  // dV^T (role A) or dK^T (role B)
+  // Products of 64 streamed rows and the 32 resident ones, and the accumulator of the second GEMM: dV^T (role A) or dK^T
+  // (role B).  Either way 32 registers of the one, in the order of the fragments of the second GEMM, and 64 of the other.
+  typedef typename std::conditional<WIDE, f16v[2], f4v[4][2]>::type Product;
+  typename std::conditional<WIDE, f16v[G::kDBlocks], f4v[G16::kDB][2]>::type acc;
+  auto clear = [](auto& x) __attribute__((always_inline)) {
+    if constexpr (WIDE) {
 #pragma unroll
-  for (int db = 0; db < G::kDBlocks; ++db)
+      for (auto& v : x)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+        for (int r = 0; r < 16; ++r) v[r] = 0.f;
+    } else {
+#pragma unroll
+      for (auto& row : x) row[0] = row[1] = f4v{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  // element e of 8 of fragment f of 4: 16 streamed rows f, or 32 streamed rows f >> 1 and resident block f & 1
+  auto element = [](const Product& x, int f, int e) __attribute__((always_inline)) {
+    if constexpr (WIDE) return x[f >> 1][(f & 1) * 8 + e];
+    else return x[2 * (f >> 1) + (e >> 2)][f & 1][e & 3];
+  };
+  clear(acc);
 
+  // Two waves of a SIMD that both have MFMAs ready do not take turns: one runs, the other waits, and which one is up to the
+  // priorities.  The products that an iteration begins with go first: those that would be held up meet the next ones too.
+  // (B2 H40 N2048 causal: 212 us without priorities, 206 with one for all, 201 with these, B3 H20 N1031: 102, 100, 96.  32 x
+  // 32 MFMAs: no difference.)
+  auto priority = [&](auto b_tag, auto a_tag) __attribute__((always_inline)) {
+    if constexpr (!WIDE) {
+      if (role_b) __builtin_amdgcn_s_setprio(decltype(b_tag)::value);
+      else __builtin_amdgcn_s_setprio(decltype(a_tag)::value);
+    }
+  };
   // first GEMM of a tile: rows of Q (role A) or dO (role B) against the resident
   // rows, on top of what x holds
   // Both GEMMs read their LDS fragments kLead MFMAs ahead of their use, in an order that is written out and
   // pinned (see the forward: scheduling hints alone are dropped when registers get scarce).
-  constexpr int kLead = 4;
-  auto gemm1 = [&](const char* tile_lds, f16v (&x)[2]) __attribute__((always_inline)) {
+  constexpr int kLead = 4, kN = 2 * G::kKSteps;  // units of one fragment; both GEMMs have as many
+  static_assert(kN == 4 * G::kDBlocks, "");
+  auto gemm1 = [&](const char* tile_lds, Product& x) __attribute__((always_inline)) {
     const unsigned a0 = opaque_lds_address(tile_lds + r_off[0]), a1 = opaque_lds_address(tile_lds + r_off[1]);
-    constexpr int kN = 2 * G::kKSteps;  // MFMA n: row block rb = n & 1, feature step kk = n >> 1
+    // unit n: row block n & 1 and feature step n >> 1, or row block n & 3 and feature step n >> 2
+    auto read = [&](int n) __attribute__((always_inline)) {
+      if constexpr (WIDE) return swz_rows_at<D>(a0, a1, n & 1, n >> 1);
+      else return rows16_at<D>(a0, a1, n & 3, n >> 2);
+    };
     h8 frag[kLead];
 #pragma unroll
-    for (int n = 0; n < kLead; ++n) frag[n] = swz_rows_at<D>(a0, a1, n & 1, n >> 1);
+    for (int n = 0; n < kLead; ++n) frag[n] = read(n);
+    priority(IntTag<1>{}, IntTag<2>{});
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < kN; ++n) {
-      x[n & 1] = mfma(frag[n % kLead], rf[n >> 1], x[n & 1]);
-      if (n + kLead < kN) frag[n % kLead] = swz_rows_at<D>(a0, a1, (n + kLead) & 1, (n + kLead) >> 1);
+      if constexpr (WIDE) {
+        x[n & 1] = mfma(frag[n % kLead], rf[n >> 1], x[n & 1]);
+      } else {
+        if (n % 2 == 0) wait_lds_pinned(n + 3 < kN ? 2 : n + 2 < kN ? 1 : 0);
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) x[n & 3][cb] = mfma16(frag[n % kLead], rf[2 * (n >> 2) + cb], x[n & 3][cb]);
+      }
+      if (n + kLead < kN) frag[n % kLead] = read(n + kLead);
       __builtin_amdgcn_sched_barrier(0);
     }
+    priority(IntTag<0>{}, IntTag<0>{});
   };
   // second GEMM: columns of dO (role A) or Q (role B) against the fp16 operand y
   auto gemm2 = [&](const char* tile_lds, const h8 (&y)[4]) __attribute__((always_inline)) {
-    const unsigned a0 = opaque_lds_address(tile_lds + c_off[0]), a1 = opaque_lds_address(tile_lds + c_off[1]);
-    constexpr int kDB = G::kDBlocks, kN = 4 * kDB;  // MFMA n: chunk c16 = n / kDB, feature block db = n % kDB
-    h8 frag[kLead];
+    auto run = [&](auto read) __attribute__((always_inline)) {
+      h8 frag[kLead];
 #pragma unroll
-    for (int n = 0; n < kLead; ++n) frag[n] = swz_cols_at<D>(a0, a1, n / kDB, n % kDB);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int n = 0; n < kN; ++n) {
-      acc[n % kDB] = mfma(frag[n % kLead], y[n / kDB], acc[n % kDB]);
-      if (n + kLead < kN) frag[n % kLead] = swz_cols_at<D>(a0, a1, (n + kLead) / kDB, (n + kLead) % kDB);
+      for (int n = 0; n < kLead; ++n) frag[n] = read(n);
+      priority(IntTag<3>{}, IntTag<2>{});
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < kN; ++n) {
+        if constexpr (WIDE) {
+          constexpr int kDB = G::kDBlocks;
+          acc[n % kDB] = mfma(frag[n % kLead], y[n / kDB], acc[n % kDB]);
+        } else {
+          constexpr int kDB = G16::kDB;
+          if (n % 2 == 0) wait_lds_pinned(n + 3 < kN ? 4 : n + 2 < kN ? 2 : 0);
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) acc[n % kDB][cb] = mfma16(frag[n % kLead], y[2 * (n / kDB) + cb], acc[n % kDB][cb]);
+        }
+        if (n + kLead < kN) frag[n % kLead] = read(n + kLead);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      priority(IntTag<0>{}, IntTag<0>{});
+    };
+    // unit n: 16 streamed rows n / 4 and feature block n % 4, or 32 streamed rows n / 8 and feature block n % 8
+    if constexpr (WIDE) {
+      const unsigned a0 = opaque_lds_address(tile_lds + c_off[0]), a1 = opaque_lds_address(tile_lds + c_off[1]);
+      run([&](int n) __attribute__((always_inline)) { return swz_cols_at<D>(a0, a1, n / G::kDBlocks, n % G::kDBlocks); });
+    } else {
+      const Cols16<D> cols(tile_lds, lane);
+      run([&](int n) __attribute__((always_inline)) { return cols.at(0, n / G16::kDB, n % G16::kDB); });
     }
   };
   // P = exp2(S*c - lse2), fp16, in B-operand order.  MASKED tiles straddle the
   // diagonal or the end of the sequence.
-  auto probabilities = [&](const f16v (&x)[2], h8 (&y)[4], const char* Sl, int q0, auto masked_tag)
+  auto probabilities = [&](const Product& x, h8 (&y)[4], const char* Sl, int q0, auto masked_tag)
                            __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value != 0;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int quad = 0; quad < kQuads; ++quad) {
+      const f4v l4 = *reinterpret_cast<const f4v*>(Sl + stat_row(quad) * 4);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f4v l4 = *reinterpret_cast<const f4v*>(Sl + (rb * 32 + 8 * g) * 4);
+      for (int cb = 0; cb < (WIDE ? 1 : 2); ++cb)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float p = fast_exp2(fmaf(x[rb][4 * g + e], c, -l4[e]));
+        for (int r = 0; r < 4; ++r) {
+          const int f = WIDE ? quad >> 1 : 2 * (quad >> 1) + cb, e = (quad & 1) * 4 + r;
+          float p = fast_exp2(fmaf(element(x, f, e), c, -l4[r]));
           if (MASKED) {
-            const int q = q0 + rb * 32 + 8 * g + 4 * hh + e;
-            if ((CAUSAL && ki > q) || q >= N) p = 0.f;
+            const int q = q0 + stat_row(quad) + (WIDE ? 4 * g : acc16_row(0, g)) + r;
+            if ((CAUSAL && k0w + 16 * cb + i > q) || q >= N) p = 0.f;
           }
-          y[rb * 2 + (g >> 1)][(g & 1) * 4 + e] = (half_t)p;
+          y[f][e] = (half_t)p;
         }
-      }
+    }
   };
   // a pair without keys has nothing to do, except for the zeros of dS it owes the last 64-key tile
   const bool has_keys = k0w < (SPILL ? (N + kTile - 1) / kTile * kTile : N);
@@ -2049,31 +2130,22 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         const char* Sl = st_ring + (it % 3) * kStBytes + st_off;
         const int q0 = (t_begin + it) * kTile;
         const bool masked = (CAUSAL && q0 < k0w + kResident - 1) || (q0 + kTile > N);
-        f16v x[2];
+        Product x;
         h8 y[4];
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) x[rb][r] = 0.f;
+        clear(x);
         gemm1(Ql, x);
         if (masked) probabilities(x, y, Sl, q0, IntTag<1>{});
         else probabilities(x, y, Sl, q0, IntTag<0>{});
         char* pw = p_mine + (it & 1) * kPBytes;
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-          *reinterpret_cast<h8*>(pw + rb * 2048) = y[rb * 2];
-          *reinterpret_cast<h8*>(pw + rb * 2048 + 1024) = y[rb * 2 + 1];
-        }
+        for (int f = 0; f < 4; ++f) *reinterpret_cast<h8*>(pw + f * 1024) = y[f];
         gemm2(Gl, y);
       }
       step_copy(it);
     }
   } else {
-    f16v x[2];  // delta - dP of the previous tile
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) x[rb][r] = 0.f;
+    Product x;  // delta - dP of the previous tile
+    clear(x);
     for (int it = 0; it <= n_it; ++it) {
       // SPILL: this wave issues its tile copies and, after the second GEMM, the four stores of dS.  The wait
       // at the top of the next iteration leaves at most as many operations in flight as those stores, the
@@ -2085,22 +2157,17 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       if (prev_active) {  // the part that needs P, one tile behind
         const char* pr = p_mine + ((it - 1) & 1) * kPBytes;
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-          const h8 p0 = *reinterpret_cast<const h8*>(pr + rb * 2048);
-          const h8 p1 = *reinterpret_cast<const h8*>(pr + rb * 2048 + 1024);
-          float xr[16];
+        for (int f = 0; f < 4; ++f) {
+          const h8 p = *reinterpret_cast<const h8*>(pr + f * 1024);
+          float xr[8];
 #pragma unroll
-          for (int e = 0; e < 16; ++e) xr[e] = x[rb][e];
-          y[rb * 2] = neg_mul_to_f16x8(p0, xr);
-          y[rb * 2 + 1] = neg_mul_to_f16x8(p1, xr + 8);
+          for (int e = 0; e < 8; ++e) xr[e] = element(x, f, e);
+          y[f] = neg_mul_to_f16x8(p, xr);
         }
-        if (SPILL) {
-          if (k0w + kResident > N && ki >= N) {  // keys past the end contribute nothing to dQ
+        if (SPILL && k0w + kResident > N) {  // keys past the end contribute nothing to dQ
 #pragma unroll
-            for (int c16 = 0; c16 < 4; ++c16)
-#pragma unroll
-              for (int e = 0; e < 8; ++e) y[c16][e] = (half_t)0.f;
-          }
+          for (int f = 0; f < 4; ++f)
+            if (k0w + (WIDE ? 0 : 16 * (f & 1)) + i >= N) y[f] = h8{};
         }
       }
       if (SPILL) step_copy(it);
@@ -2110,40 +2177,42 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
         // role A, which come at the end of the iteration.  The stores go through the same path and would queue.
         const int t = t_begin + it - 1;  // the query tile
         half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048;
-        if constexpr (!KEEP) {
-          store16_stream(dst, y[0], IntTag<0>{});
-          store16_stream(dst, y[1], IntTag<1024>{});
-          store16_stream(dst, y[2], IntTag<2048>{});
-          store16_stream(dst, y[3], IntTag<3072>{});
-        } else {
-          store16_keep(dst, y[0], IntTag<0>{});
-          store16_keep(dst, y[1], IntTag<1024>{});
-          store16_keep(dst, y[2], IntTag<2048>{});
-          store16_keep(dst, y[3], IntTag<3072>{});
-        }
+        static_for<4>([&](auto f_tag) __attribute__((always_inline)) {
+          constexpr int f = decltype(f_tag)::value, at = f * 1024;
+          if constexpr (!KEEP) store16_stream(dst, y[f], IntTag<at>{});
+          else store16_keep(dst, y[f], IntTag<at>{});
+        });
       }
       if (it < n_it && tile_active(it)) {
         const char* Gl = g_ring + (it % 3) * T::kBytes;
         const char* Sl = st_ring + (it % 3) * kStBytes + st_off;
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
+        for (int quad = 0; quad < kQuads; ++quad) {
+          const f4v d4 = *reinterpret_cast<const f4v*>(Sl + stat_row(quad) * 4);
+          if constexpr (WIDE) {
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const f4v d4 = *reinterpret_cast<const f4v*>(Sl + (rb * 32 + 8 * g) * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[rb][4 * g + e] = d4[e];
+            for (int r = 0; r < 4; ++r) x[quad >> 2][4 * (quad & 3) + r] = d4[r];
+          } else {
+            x[quad][0] = x[quad][1] = d4;
           }
+        }
         __builtin_amdgcn_sched_barrier(0);  // keep the delta loads out of the GEMM's read/MFMA pipeline
         gemm1(Gl, x);
       }
     }
   }
 
-  static_assert(kKvWaves * StageGeom<D>::kBytes <= 7 * T::kBytes, "the output staging tiles fit the rings");
+  static_assert(kKvWaves * Stage16<D>::kBytes <= 7 * T::kBytes && kKvWaves * StageGeom<D>::kBytes <= 7 * T::kBytes,
+                "the output staging tiles fit the rings");
   block_barrier();  // every wave is done with the rings: they become the staging tiles
-  char* const stage = smem + wave * StageGeom<D>::kBytes;
-  if (!role_b) store_resident<D>(dV + head_off, rs, k0w, N, acc, 1.f, lane, stage);
-  else store_resident<D>(dK + head_off, rs, k0w, N, acc, scale, lane, stage);
+  half_t* const out = (role_b ? dK : dV) + head_off;
+  const float mul = role_b ? scale : 1.f;
+  if constexpr (WIDE) {
+    store_resident<D>(out, rs, k0w, N, acc, mul, lane, smem + wave * StageGeom<D>::kBytes);
+  } else {
+    const float both[2] = {mul, mul};
+    store_resident16<D>(out, rs, k0w, N, acc, both, lane, smem + wave * Stage16<D>::kBytes);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2404,8 +2473,10 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
 //     that a CU has in flight, a K tile takes as long to arrive as they do, L2 hit or not;
 //   * the LDS is full with that, so the epilogue stages a wave's output rows in the 4 KiB of the block's last dS
 //     tile that hold the wave's own queries and that no other wave reads.
-// The queries of a chunk sit in the order the dK/dV pass's registers held them (bits
-// 2 and 3 of the position inside 16 swapped); the epilogue puts the rows back in place.
+// The queries of a fragment sit in the order the dK/dV pass's registers held them; the epilogue puts the rows back in
+// place.  WIDE as in that pass.  The 16 x 16 MFMAs take less of the power that the copies also need (B2 H40 N2048 causal:
+// 97 -> 88 us, B2 H32 N4096 causal 242 -> 229 us); more copying waves, deeper rings or K fragments read further ahead
+// change nothing.
 // (formula: reference kernel/fused_mha_kernel.cu:680-683.)
 // ---------------------------------------------------------------------------
 constexpr int kDsCopyWaves = 4;    // waves that only copy tiles: two for dS, two for K
@@ -2416,7 +2487,7 @@ constexpr int kDsPanelTileBytes = kTile * kDsPanelQ * 2;
 constexpr int kDsStageD = 32;          // features staged at a time in the epilogue
 constexpr int ds_threads(int panels) { return (4 * panels + kDsCopyWaves) * 64; }
 
-template <int D, bool CAUSAL, int kDsPanels>
+template <int D, bool CAUSAL, int kDsPanels, bool WIDE>
 __global__ void __launch_bounds__(ds_threads(kDsPanels), 1)
 fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
                          half_t* __restrict__ dQ, int H, int N, int nqb, int total, int slice0,
@@ -2427,8 +2498,8 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   constexpr int kDsBlockQ = kDsPanels * kDsPanelQ;
   constexpr int kDsTileBytes = kDsPanels * kDsPanelTileBytes;
   constexpr int kSIPW = kDsTileBytes / 1024 / 2;     // dS copies per dS-copying wave and tile: half of the pieces
-  constexpr int kDB = D / 32;       // 32-feature blocks
-  static_assert(16 * StageGeom<kDsStageD>::kPitch <= 2048, "half a staging tile must fit into two dS pieces");
+  static_assert(16 * StageGeom<kDsStageD>::kPitch <= 2048 && 16 * Stage16<kDsStageD>::kPitch <= 2048,
+                "half a staging tile must fit into two dS pieces");
   __shared__ __attribute__((aligned(1024))) char smem[kDsRingS * kDsTileBytes + kDsRingK * T::kBytes];
   char* const s_ring = smem;
   char* const k_ring = smem + kDsRingS * kDsTileBytes;
@@ -2439,7 +2510,6 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   const int qb = wave & (kDsWaves - 1);              // computing wave: its 32 queries of the block
   const bool copies_k = wave >= kDsWaves + 2;
   const int cw = wave & 1;                           // copying wave: which half of its tensor's copies
-  const int i = lane & 31;
   const int rs = H * D;  // dQ is dense
   const int nt_all = (N + kTile - 1) / kTile;
   const int n_panels = np / kDsPanelQ;
@@ -2492,10 +2562,10 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   }
 
   // K copies: this wave's half of a tile (as in the other kernels).  dS copies: this wave's kSIPW pieces of
-  // 1 KiB, lane l fetching 16 bytes.  In memory a piece is [2 halves][32 keys] x 16 bytes; in LDS it
-  // becomes [32 keys][2 halves] x 16 bytes (rows of 16 queries), and the pieces of odd query chunks land rotated
-  // by 128 bytes (LDS offset o holds row-major byte (o - 128) mod 1024), which keeps the two halves of a 32-lane
-  // transposing read on different banks.
+  // 1 KiB, lane l fetching 16 bytes, in an order in which the 32 lanes of a transposing read fall on different banks.
+  // WIDE: in memory a piece is [2 halves][32 keys] x 16 bytes; in LDS it becomes [32 keys][2 halves] x 16 bytes (rows of 16
+  // queries), and the pieces of odd query chunks land rotated by 128 bytes (LDS offset o holds row-major byte (o - 128) mod
+  // 1024).  Otherwise a piece is [4 lane groups j][16 keys] x 16 bytes, and in LDS the keys of odd j are 8 further (modulo 16).
   int c_row[kKIPW], c_kgoff[kKIPW], c_kblk[kKIPW];
 #pragma unroll
   for (int u = 0; u < kKIPW; ++u) {
@@ -2504,10 +2574,12 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
     c_kblk[u] = t * 1024;
   }
   int c_sgoff[2];  // even and odd pieces; + piece * 1024
-  {
+  if constexpr (WIDE) {
     const int at = (lane - 8) & 63;  // position (key, half) = (at >> 1, at & 1) in LDS of what lane l fetches of an odd piece
     c_sgoff[0] = ((lane & 1) * 32 + (lane >> 1)) * 16;
     c_sgoff[1] = ((at & 1) * 32 + (at >> 1)) * 16;
+  } else {
+    c_sgoff[0] = c_sgoff[1] = (lane ^ ((lane >> 4 & 1) * 8)) * 16;
   }
   auto copy_s = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
     const half_t* sp = c.base + (long)c.j * (kDsPanelTileBytes / 2);  // wave-uniform
@@ -2536,39 +2608,56 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
     }
   };
 
-  // LDS offsets of this lane's transposing reads.  K tile: as in the other kernels.  dS tile: key step kc,
-  // read e: key row (kc & 1) * 16 + 8 * e + 4 * hhk + (L >> 2) of the piece [panel][(kc >> 1)][query tile][chunk
-  // 2 * (qb & 1) + lane bit 4], 8 bytes at (L & 3) * 8 of its 32-byte row, plus the rotation of odd chunks.
-  int c_off[2];
-  swz_cols_off<D>(lane, c_off);
   // the first of this wave's pieces of a dS tile: two adjacent ones per 32 keys
   const int own_pieces = (qb >> 2) * kDsPanelTileBytes + (((qb >> 1) & 1) * 4 + 2 * (qb & 1)) * 1024;
-  int s_off[2][2];
+  // LDS offsets of this lane's transposing reads.  WIDE: key step kc, read e: key row (kc & 1) * 16 + 8 * e + 4 * g +
+  // (L >> 2), with g = lane >> 5, of the piece [panel][(kc >> 1)][query tile][chunk 2 * (qb & 1) + lane bit 4], 8 bytes at
+  // (L & 3) * 8 of its 32-byte row, plus the rotation of odd chunks.
+  // Otherwise lane 16 g + L reads 8 bytes, 4 queries, of lane group j = L & 3 of the key 16 (g >> 1) + 8 p + 4 (g & 1) + (L >> 2), and then holds query L of 16 of the four keys.  The 16 bytes of a key
+  // and j are queries 16 (j >> 1) + 4 (j & 1) + 0..3 and the same + 8; query block nb takes the first half of j = 0, 1
+  // and the second of j = 2, 3, or the other way round: so its reads touch all banks.
+  int s_off[2][2];  // WIDE: [kc & 1][e], otherwise [nb][p]
   {
-    const int L = lane & 15, odd = (lane >> 4) & 1, hhk = lane >> 5;
+    const int L = lane & 15;
 #pragma unroll
-    for (int kcl = 0; kcl < 2; ++kcl)
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        const int in_piece = (kcl * 16 + 8 * e + 4 * hhk + (L >> 2)) * 32 + (L & 3) * 8;
-        s_off[kcl][e] = own_pieces + odd * 1024 + ((in_piece + odd * 128) & 1023);
+        if constexpr (WIDE) {
+          const int odd = (lane >> 4) & 1, in_piece = (u * 16 + 8 * e + 4 * (lane >> 5) + (L >> 2)) * 32 + (L & 3) * 8;
+          s_off[u][e] = own_pieces + odd * 1024 + ((in_piece + odd * 128) & 1023);
+        } else {
+          const int g = lane >> 4, j = L & 3;
+          s_off[u][e] = own_pieces + (g >> 1) * 1024 + (16 * j + ((8 * e + 4 * (g & 1) + (L >> 2)) ^ (8 * (j & 1)))) * 16 +
+                        ((j >> 1) ^ u) * 8;
+        }
       }
   }
-  auto s_frag = [&](const char* tile, int kc) __attribute__((always_inline)) {
+  int c_off[2];
+  swz_cols_off<D>(lane, c_off);
+  auto s_frag = [&](const char* tile, int f) __attribute__((always_inline)) {  // 16 keys f, or 32 keys f >> 1 and nb = f & 1
     typedef __attribute__((address_space(3))) s4 lds_s4;
-    const char* p = tile + (kc >> 1) * 8192;
-    s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + s_off[kc & 1][0]));
-    s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + s_off[kc & 1][1]));
+    const char* at = tile + (f >> 1) * 8192;
+    s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(at + s_off[f & 1][0]));
+    s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(at + s_off[f & 1][1]));
     return __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
-  f16v acc[kDB];
+  typename std::conditional<WIDE, f16v[TileGeom<D>::kDBlocks], f4v[Geom16<D>::kDB][2]>::type acc;
+  auto clear = [&](int part) __attribute__((always_inline)) {
+    if constexpr (WIDE) {
 #pragma unroll
-  for (int db = 0; db < kDB; ++db)
+      for (int r = 0; r < 16; ++r) acc[part][r] = 0.f;
+    } else {
+      acc[2 * part][0] = acc[2 * part][1] = acc[2 * part + 1][0] = acc[2 * part + 1][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    }
+  };
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
-  // column i of the accumulator is the query at position i of the wave's 32: bits 2 and 3 swapped
-  const int my_row = (i & 0x13) | ((i & 8) >> 1) | ((i & 4) << 1);
+  for (int part = 0; part < D / kDsStageD; ++part) clear(part);
+  // The query, of the wave's 32, of this lane's column.  WIDE: that at position i of the 32, bits 2 and 3 swapped;
+  // otherwise that of block nb is my_row ^ (8 * nb).
+  const int my_row = WIDE ? (lane & 0x13) | ((lane & 8) >> 1) | ((lane & 4) << 1)
+                          : 24 * ((lane >> 3) & 1) + 4 * ((lane >> 2) & 1) + (lane & 3);
 
   constexpr int kAheadS = kDsRingS - 1, kAheadK = kDsRingK - 1;
   // the copying waves run ahead of the sequence: kAhead tiles are issued before the first is used
@@ -2602,20 +2691,38 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
     if (computes && cur.j < jend) {
       const char* Kl = k_ring + slot_k * T::kBytes;
       const char* Sl = s_ring + slot_s * kDsTileBytes;
-      // MFMA n: key step kc = n / kDB, feature block db = n % kDB; the K fragments are read kLead MFMAs ahead, the
-      // four dS fragments up front (order pinned, see the forward)
-      constexpr int kN = 4 * kDB, kLead = 4;
+      // unit n: 16 keys n / 4 and feature block n % 4, or 32 keys n / 8 and feature block n % 8; the K fragments are read
+      // kLead units ahead, the four dS fragments up front (order pinned, see the forward)
+      constexpr int kN = D / 8, kLead = 4;
       h8 bfrag[4], afrag[kLead];
 #pragma unroll
-      for (int kc = 0; kc < 4; ++kc) bfrag[kc] = s_frag(Sl, kc);
+      for (int f = 0; f < 4; ++f) bfrag[f] = s_frag(Sl, f);
+      auto run = [&](auto read) __attribute__((always_inline)) {
 #pragma unroll
-      for (int n = 0; n < kLead; ++n) afrag[n] = swz_cols<D>(Kl, n / kDB, n % kDB, c_off);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int n = 0; n < kN; ++n) {
-        acc[n % kDB] = mfma(afrag[n % kLead], bfrag[n / kDB], acc[n % kDB]);
-        if (n + kLead < kN) afrag[n % kLead] = swz_cols<D>(Kl, (n + kLead) / kDB, (n + kLead) % kDB, c_off);
+        for (int n = 0; n < kLead; ++n) afrag[n] = read(n);
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < kN; ++n) {
+          if constexpr (WIDE) {
+            constexpr int kDB = TileGeom<D>::kDBlocks;
+            acc[n % kDB] = mfma(afrag[n % kLead], bfrag[n / kDB], acc[n % kDB]);
+          } else {
+            constexpr int kDB = Geom16<D>::kDB;
+            if (n % 2 == 0) wait_lds_pinned(n + 3 < kN ? 4 : n + 2 < kN ? 2 : 0);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) acc[n % kDB][nb] = mfma16(afrag[n % kLead], bfrag[2 * (n / kDB) + nb], acc[n % kDB][nb]);
+          }
+          if (n + kLead < kN) afrag[n % kLead] = read(n + kLead);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      if constexpr (WIDE) {
+        run([&](int n) __attribute__((always_inline)) {
+          return swz_cols<D>(Kl, n / TileGeom<D>::kDBlocks, n % TileGeom<D>::kDBlocks, c_off);
+        });
+      } else {
+        const Cols16<D> cols(Kl, lane);
+        run([&](int n) __attribute__((always_inline)) { return cols.at(0, n / Geom16<D>::kDB, n % Geom16<D>::kDB); });
       }
     }
     if (computes && cur.j == cur.nt - 1) {
@@ -2626,11 +2733,16 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
       half_t* out = dQ + cur.out_off;
       const int row0 = cur.mblk * kDsBlockQ + qb * kResident;
 #pragma unroll
-      for (int part = 0; part < kDB; ++part) {
-        store_resident<kDsStageD>(out + part * kDsStageD, rs, row0, N, *reinterpret_cast<const f16v(*)[1]>(&acc[part]),
-                                  scale, lane, stage, my_row, 8192);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[part][r] = 0.f;
+      for (int part = 0; part < D / kDsStageD; ++part) {
+        if constexpr (WIDE) {
+          store_resident<kDsStageD>(out + part * kDsStageD, rs, row0, N, *reinterpret_cast<const f16v(*)[1]>(&acc[part]),
+                                    scale, lane, stage, my_row, 8192);
+        } else {
+          const float mul[2] = {scale, scale};
+          store_resident16<kDsStageD>(out + part * kDsStageD, rs, row0, N, acc + 2 * part, mul, lane, stage, my_row,
+                                      my_row ^ 8, 8192);
+        }
+        clear(part);
       }
     }
     advance(cur, false);
@@ -2853,6 +2965,14 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
       return FUSED_MHA_ERR_LAUNCH;
   }
   const float c = scale * kLog2e;
+  // Which MFMAs the D = 128 passes use, both the same, since it decides the order of dS in the workspace: 16 x 16 where the
+  // chip runs at its power cap, 32 x 32 where a good part of the CUs has nothing to do and a wave's own instructions are
+  // what takes the time.  us of the dK/dV pass with 32 x 32 and with 16 x 16 MFMAs, N x slices (blocks per CU): without a
+  // mask 1031 x 16 31.4, 33.1 (0.56); 4096 x 5 105.8, 104.2 (0.63); 1031 x 20 33.9, 33.8 (0.70); 1031 x 28 41.8, 41.2; 4096 x 8
+  // 139, 134 (1); 512 x 64 25.2, 24.0.  Causal, where a block is half as much work: 4096 x 6 94.0, 100.8 (0.75); 16384 x 2
+  // 398, 405 (1); 4096 x 10 111.1, 111.2 (1.25); 16384 x 3 477, 469 (1.5); 2048 x 32 83.7, 80.1 (2); 2048 x 80 212, 201.  dQ
+  // pass over dS: 1031 x 8 11.5, 12.8; 4096 x 4 causal 33.0, 35.6; 1031 x 60 42, 40.5; 2048 x 80 causal 97, 88.
+  auto wide = [&]() { return (long)key_blocks(n) * slices * (CAUSAL ? 1 : 2) * 4 < 5 * cus; };
   auto dq_pass = [&]() {
     if constexpr (D == 64) {
       const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ;
@@ -2876,11 +2996,12 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
           return even ? persistent_grid(total) : (unsigned)total;
         };
         const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * slices;
-        if (total2 >= 2 * cus)
-          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2>, groups(nqb2), ds_threads(2), stream, (const half_t*)k, ks,
+        if (total2 >= 2 * cus)  // so many blocks are never `wide`
+          return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2, false>, groups(nqb2), ds_threads(2), stream, (const half_t*)k, ks,
                         (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, slice0, stream_ds, scale);
         const int nqb = np / kDsPanelQ, total = nqb * slices;
-        return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 1>, groups(nqb), ds_threads(1), stream, (const half_t*)k, ks,
+        auto kernel = wide() ? fmha_bwd_dq_spill_kernel<D, CAUSAL, 1, true> : fmha_bwd_dq_spill_kernel<D, CAUSAL, 1, false>;
+        return launch(kernel, groups(nqb), ds_threads(1), stream, (const half_t*)k, ks,
                       (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, slice0, stream_ds, scale);
       }
       const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;
@@ -2898,9 +3019,13 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
                     (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n, nnb, c, scale);
     } else {
       const int nnb = key_blocks(n);
-      auto kernel = !spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, false, false>
-                    : stream_ds ? fmha_bwd_dkdv_kernel<D, CAUSAL, true, false>
-                                : fmha_bwd_dkdv_kernel<D, CAUSAL, true, true>;
+      auto pick = [&](auto wide_tag) {
+        constexpr bool kWide = decltype(wide_tag)::value != 0;
+        return !spill ? fmha_bwd_dkdv_kernel<D, CAUSAL, false, false, kWide>
+               : stream_ds ? fmha_bwd_dkdv_kernel<D, CAUSAL, true, false, kWide>
+                           : fmha_bwd_dkdv_kernel<D, CAUSAL, true, true, kWide>;
+      };
+      auto kernel = wide() ? pick(IntTag<1>{}) : pick(IntTag<0>{});
       return launch(kernel, (unsigned)nnb * slices, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
                     (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, slice0, c, scale);

@@ -121,6 +121,27 @@ def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200])
+def test_backward_d128_with_either_mfma(N, causal):
+    """A launch that has just enough blocks takes the passes with 16 x 16 MFMAs, a slice of it those with 32 x 32 ones: the
+    same bits, with and without the workspace for dS."""
+    D, lib = 128, abi.load()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H = -(-5 * cus // (4 if causal else 8) // (-(-N // 128))) + 1
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+    for least in (False, True):
+        whole = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=least)[:3]
+        for h in (0, H - 1):
+            one = [t[:, :, h:h + 1].contiguous() for t in (q, k, v, out, do)]
+            alone = abi.backward(lib, *one, lse[:, h:h + 1].clone(), D ** -0.5, causal, min_workspace=least)[:3]
+            for a, b in zip(alone, whole):
+                assert torch.equal(a, b[:, :, h:h + 1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,N,causal", [
     (4, 1024, False), (5, 1024, False),      # 8 MiB of dS: stored with the used-once hint; 10 MiB: without
     (5, 1025, True), (9, 1025, True),        # 6.3 and 11.4 MiB of dS
