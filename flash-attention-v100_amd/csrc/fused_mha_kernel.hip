@@ -943,7 +943,15 @@ __device__ __forceinline__ unsigned pack_f16(float lo, float hi) {
   return r;
 }
 
-template <int D, bool CAUSAL>
+// Of two waves that share a SIMD one goes first whenever both could issue: the one in an odd wave slot (bits 0 to 3 of the
+// register say which slot a wave has).  Rule and figures: half_round_left.
+__device__ __forceinline__ void odd_slots_first() {
+  int slot;
+  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID, 0, 4)" : "=s"(slot));
+  if (slot & 1) __builtin_amdgcn_s_setprio(1);
+}
+
+template <int D, bool CAUSAL, bool ODD_FIRST>
 __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                      Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
@@ -957,6 +965,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   __shared__ __attribute__((aligned(1024))) char smem[4 * T::kBytes];
   constexpr int kVOff = 2 * T::kBytes;
 
+  if (ODD_FIRST) odd_slots_first();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // what depends on the lane is worked out again where it is needed, not kept in registers across the main loop
   auto lane_now = []() __attribute__((always_inline)) {
@@ -1596,7 +1605,7 @@ fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, c
 //
 // dQ pass.  The formulas are those of fmha_bwd_dq_kernel, and so are the results, bit for bit.
 // ---------------------------------------------------------------------------
-template <bool CAUSAL, bool STATS>
+template <bool CAUSAL, bool STATS, bool ODD_FIRST>
 __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                         const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
@@ -1612,6 +1621,7 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
   constexpr int kVOff = kSlots * T::kBytes;
   __shared__ __attribute__((aligned(1024))) char smem[2 * kSlots * T::kBytes];
 
+  if (ODD_FIRST) odd_slots_first();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 31, hh = lane >> 5;
@@ -2220,7 +2230,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 // A 64-query tile is worked on in two halves of 32 queries; the accumulation into dV and dK of a half runs during the
 // next one, so Q and dO have three slots: the tile before, the current one, the one being copied.
 // ---------------------------------------------------------------------------
-template <bool CAUSAL>
+template <bool CAUSAL, bool ODD_FIRST>
 __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                           const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
@@ -2237,6 +2247,7 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
   __shared__ __attribute__((aligned(1024))) char smem[kStOff + kSlots * kStBytes];
   static_assert(kPipeWaves * StageGeom<D>::kBytes <= kStOff, "the output staging tiles fit the rings");
 
+  if (ODD_FIRST) odd_slots_first();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 31, hh = lane >> 5;
@@ -2842,6 +2853,21 @@ bool persistent_forward_pays(int slices, int blocks_per_slice, int n, bool causa
   return fmha_even_shares(slices, blocks_per_slice, cus, causal);
 }
 
+// Whether a launch of equal blocks, two to a CU, has work for at most half of the places in its last round, the second one or
+// (up to max_rounds) the third.  Two blocks that share a CU evenly end together, and the last ones then run alone, at little
+// over half the rate of a pair; with one of the two going first (odd_slots_first) its place is free sooner, and the last
+// blocks run beside the others.  us without and with that, D = 64, N x slices (rounds), forward, then backward: 1024 x 66
+// (1.03) 31.1, 29.6; 92.1, 90.6.  1024 x 96 (1.5) 34.3, 33.1; 102.8, 102.7.  2048 x 40 (1.25) 56.2, 53.3; 174, 170.  8192 x 12
+// (1.5) 218, 211; 725, 703.  2048 x 66 (2.06) 89.7, 88.7; 279, 271.  1024 x 160 (2.5) 54.7, 55.2; 166, 164.  2048 x 80 (2.5)
+// 96.7, 96.8; 300, 297.  Forward D = 128: 1031 x 60 (1.05) 48.9, 46.8; 2048 x 40 91.8, 90.1; 4096 x 20 174, 170.
+// Short blocks have nothing to gain (512 x 192: 21.6, 21.5; 61.1, 62.2.  256 x 320: 14.1, 14.3; 39.2, 39.4), nor has a fuller
+// last round (1024 x 112, 1.75: 41.2, 42.2; dK/dV 69.1, 70.1.  1024 x 192, 3: 65.5, 65.6; dK/dV 110, 118), nor more rounds
+// (1024 x 288, 4.5: 96.9, 98.4), nor a causal launch, where the blocks differ (1024 x 64 forward: 16.4, 18.2).
+bool half_round_left(long blocks, int n, int max_rounds) {
+  const long places = 2 * (long)persistent_grid(1 << 30), rounds = blocks / places, left = blocks % places;
+  return n >= 1024 && rounds >= 1 && rounds < max_rounds && left > 0 && 2 * left <= places;
+}
+
 template <int D, bool CAUSAL>
 int launch_forward(const void* q, const void* k, const void* v, Strides qs, Strides ks, Strides vs, void* o, void* lse,
                    int batch, int head, int n, float scale, hipStream_t stream) {
@@ -2859,7 +2885,10 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
     }
   }
   const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ, total = nmb * batch * head;
-  const hipError_t rc = launch(fmha_fwd_pipe_kernel<D, CAUSAL>, (unsigned)total, kPipeThreads, stream, (const half_t*)q,
+  auto kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false>;
+  if constexpr (!CAUSAL)
+    if (half_round_left(total, n, 2)) kernel = fmha_fwd_pipe_kernel<D, CAUSAL, true>;
+  const hipError_t rc = launch(kernel, (unsigned)total, kPipeThreads, stream, (const half_t*)q,
                                (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, c,
                                negate);
   return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
@@ -2976,7 +3005,14 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   auto dq_pass = [&]() {
     if constexpr (D == 64) {
       const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ;
-      auto kernel = dq_makes_stats ? fmha_bwd_dq_pipe_kernel<CAUSAL, true> : fmha_bwd_dq_pipe_kernel<CAUSAL, false>;
+      auto pick = [&](auto odd_first) {
+        constexpr bool kOddFirst = decltype(odd_first)::value != 0;
+        return dq_makes_stats ? fmha_bwd_dq_pipe_kernel<CAUSAL, true, kOddFirst>
+                              : fmha_bwd_dq_pipe_kernel<CAUSAL, false, kOddFirst>;
+      };
+      auto kernel = pick(IntTag<0>{});
+      if constexpr (!CAUSAL)
+        if (half_round_left((long)nmb * batch * head, n, 3)) kernel = pick(IntTag<1>{});
       return launch(kernel, (unsigned)nmb * batch * head, kPipeThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
                     (half_t*)dq, head, n, nmb, c, scale);
@@ -3014,7 +3050,10 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   auto dkdv_pass = [&]() {
     if constexpr (D == 64) {
       const int nnb = (n + kPipeBlockKeys - 1) / kPipeBlockKeys;
-      return launch(fmha_bwd_dkdv_pipe_kernel<CAUSAL>, (unsigned)nnb * batch * head, kPipeThreads, stream,
+      auto kernel = fmha_bwd_dkdv_pipe_kernel<CAUSAL, false>;
+      if constexpr (!CAUSAL)
+        if (half_round_left((long)nnb * batch * head, n, 3)) kernel = fmha_bwd_dkdv_pipe_kernel<CAUSAL, true>;
+      return launch(kernel, (unsigned)nnb * batch * head, kPipeThreads, stream,
                     (const half_t*)q, (const half_t*)k, (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs,
                     (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n, nnb, c, scale);
     } else {

@@ -142,6 +142,28 @@ def test_backward_d128_with_either_mfma(N, causal):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,N,D", [
+    (65, 1024, 64), (57, 1031, 64),    # 520 and 513 blocks on 512 places
+    (65, 1024, 128), (57, 1031, 128),  # the forward alone
+    (129, 1024, 64), (128, 1025, 64),  # 1032 blocks, and 1152, whose last ones have one row each
+])
+def test_a_nearly_empty_last_round(H, N, D):
+    """Launches in which every other wave slot goes first: the bits of a slice alone, which has no second round."""
+    lib = abi.load()
+    gen = torch.Generator(device="cuda").manual_seed(N + H)
+    q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, False)
+    whole = [out] + list(abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, False)[:3])
+    for h in (0, H // 2, H - 1):
+        q1, k1, v1, do1 = (t[:, :, h:h + 1].contiguous() for t in (q, k, v, do))
+        out1, lse1 = abi.forward(lib, q1, k1, v1, D ** -0.5, False)
+        alone = [out1] + list(abi.backward(lib, q1, k1, v1, out1, do1, lse1, D ** -0.5, False)[:3])
+        assert torch.equal(lse1, lse[:, h:h + 1])
+        for a, b in zip(alone, whole):
+            assert torch.equal(a, b[:, :, h:h + 1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,N,causal", [
     (4, 1024, False), (5, 1024, False),      # 8 MiB of dS: stored with the used-once hint; 10 MiB: without
     (5, 1025, True), (9, 1025, True),        # 6.3 and 11.4 MiB of dS
