@@ -115,4 +115,20 @@ FMHA_HOST_DEVICE void fmha_scheduled_block(int lin, int slices, int blocks_per_s
   const int p = idx - blk * level;
   slice = (p >> 3) < count ? (lin & 7) * q + first + (p >> 3) : 8 * q + (p - 8 * count);
 }
+
+// The same launches, two blocks to a CU: work groups w and w + kCus start on the same CU, so with the second kCus taken in
+// reverse (inside each XCD, which keeps a block on the XCD of its slice) a CU starts with one heavy and one light block
+// instead of the k-th heaviest of either half.  Returns the position in the order above that work group `lin` takes.  us
+// before and after, forward, then backward (D = 64, N x slices, blocks per CU): 512 x 128 (2) 14.2, 12.1; 38.3, 33.9.  1024 x
+// 64 (2) 16.3, 15.5; 47.2, 45.6.  4096 x 16 (2) 48.6, 47.2; 154.8, 146.7.  1024 x 40 (1.25) 14.7, 14.5; 41.4, 41.0.  1024 x
+// 66 17.8, 17.4; 50.1, 46.8.  1024 x 96 (3) 23.5, 23.1; 70.1, 66.4.  1024 x 128 (4) 30.5, 28.9; 87.1, 84.7.  8192 x 12 (3)
+// 126, 124; 388, 382.  2048 x 64 (4) 45.4, 45.6; 141, 139.  Forward, D = 128: 1500 x 32 (1.5) 29.5, 27.9; 2048 x 80 (5) 95.6,
+// 95.0.  Later blocks go where a place is free: the fourth kCus reversed as well loses (1024 x 128 29.6; 86.8).
+constexpr int kCus = 256;  // of an MI355X; on any other number of CUs this is just another order
+FMHA_HOST_DEVICE int fmha_paired_block(int lin, int total) {
+  if (lin < kCus || lin >= 2 * kCus) return lin;
+  const int xcd = lin & 7, end = total < 2 * kCus ? total : 2 * kCus;
+  const int slots = (end - xcd + 7) >> 3;  // work groups below `end` on this XCD
+  return ((kCus / 8 + slots - 1 - (lin >> 3)) << 3) + xcd;
+}
 #endif  // FMHA_BLOCK_MAP_H_

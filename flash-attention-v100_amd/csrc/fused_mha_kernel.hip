@@ -974,7 +974,8 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     return t & 63;
   };
   int bh, mb;
-  fmha_scheduled_block(blockIdx.x, gridDim.x / nmb, nmb, CAUSAL, N % kPipeBlockQ != 0, bh, mb);
+  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
+                       N % kPipeBlockQ != 0, bh, mb);
   const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O is dense
@@ -1626,7 +1627,8 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 31, hh = lane >> 5;
   int bh, mb;
-  fmha_scheduled_block(blockIdx.x, gridDim.x / nmb, nmb, CAUSAL, N % kPipeBlockQ != 0, bh, mb);
+  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
+                       N % kPipeBlockQ != 0, bh, mb);
   const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O and dQ are dense
@@ -2252,7 +2254,8 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 31, hh = lane >> 5;
   int bh, nblk;
-  fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kPipeBlockKeys != 0, bh, nblk);
+  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nnb, nnb, CAUSAL,
+                       N % kPipeBlockKeys != 0, bh, nblk);
   const int b = bh / H, h = bh - b * H;                   // causal: low key blocks are the heavy ones and come first
   const int rs = H * D;                                   // dK and dV are dense
   const long head_off = ((long)b * N * H + h) * D;
@@ -2943,7 +2946,6 @@ bool rounds_fill(int slices, int n, int cus) { return (long)slices * key_blocks(
 // Rounds of less than 1 GiB are not worth it (last line).  The size is that for the 256 CUs of an MI355X, whatever device
 // is current.
 size_t best_workspace(int batch, int head, int n, int d, size_t room) {
-  constexpr int kCus = 256;
   constexpr size_t kGiB = (size_t)1 << 30;
   const size_t least = stats_bytes(batch, head, n), offset = spill_offset(batch, head, n), slice = slice_bytes(n);
   if (d == 64) return least;  // see fmha_bwd_dq_pipe_kernel

@@ -49,6 +49,35 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_paired_blocks_are_a_bijection(tmp_path):
+    """csrc/block_map.h: every block once and on the same XCD for any number of blocks, and with two blocks to a CU those
+    that share one weigh the same together."""
+    src = tmp_path / "check.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (int total = 1; total <= 1100; ++total) {
+    std::vector<int> seen(total, 0);
+    for (int lin = 0; lin < total; ++lin) {
+      const int at = fmha_paired_block(lin, total);
+      if (at < 0 || at >= total || seen[at]++ || (at & 7) != (lin & 7)) { printf("%d of %d\n", lin, total); return 1; }
+      if ((lin < kCus || lin >= 2 * kCus) && at != lin) { printf("moved %d of %d\n", lin, total); return 1; }
+    }
+  }
+  for (int w = 0; w < kCus; ++w)
+    if ((w >> 3) + (fmha_paired_block(w + kCus, 2 * kCus) >> 3) != 2 * kCus / 8 - 1) { printf("pair %d\n", w); return 1; }
+  puts("ok");
+  return 0;
+}
+''')
+    exe = tmp_path / "check"
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
 def _inputs(B, N, H, D, growing):
     """growing: the score scale rises with the key index, so that nearly every 64-key tile holds a maximum that is
     more than 2^12 times (12 in the exp2 domain) above the earlier ones and the running maximum is raised in it."""
