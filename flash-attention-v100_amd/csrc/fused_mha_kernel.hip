@@ -2840,20 +2840,31 @@ bool bad_strides(const fused_mha_strides* st) {
   return st->seq >= (1 << 24) || st->head >= (1LL << 31);
 }
 
-// Whether the persistent 256-query forward takes a D = 128 problem: only where its static shares come out even.  Figures:
-// us of the 128-query kernel, then of this one, at N x slices.
-//   Without a mask the two are within 3 % of each other where the last round is nearly full (1024 x 64: 37.7, 38.4; 4096 x
-//   16: 126, 123; 4096 x 64: 492, 484; 2048 x 320: 636, 654); at 75 % full they are not (4096 x 24: 187, 205).
-//   Under causal masking one pair of blocks per CU is even at N = 2048 and gains from there on (1024 x 128: 47.5, 47.7;
-//   2048 x 64: 77.4, 77.5; 4096 x 32: 139, 136; 8192 x 16: 265, 249; 16384 x 8: 516, 479), two pairs from N = 4096 on (2048
-//   x 128: 147, 154; 4096 x 64: 276, 274 over seconds of nothing else, where the power cap rules and fewer copies of K and V
-//   count, but 262, 269 in turns of 12 ms; 8192 x 32: 498, 495; 32768 x 8: 1905, 1874), more do not (4096 x 96: 408, 419;
-//   8192 x 64: 984, 1006).  Uneven shares lose: 2048 x 60: 74, 90; 4096 x 60: 248, 292; 6144 x 42: 373, 487; 32768 x 4:
-//   1008, 1131.
+// Whether the persistent 256-query forward takes a D = 128 problem.  It does up to 10 % more per second than the 128-query
+// kernel where all CUs are busy, but a CU takes or leaves a whole block of 256.  Figures: us of the 128-query kernel, then of
+// this one, at N x slices.
+//   Without a mask, from N = 1152 on, where the last round of the 128-query kernel (two blocks to a CU, so that half a round
+//   costs it 0.6 of one) is more than half full and this one needs no more rounds: 4096 x 64: 497, 455; 4096 x 16 128, 117;
+//   8192 x 7 224, 205; 2048 x 26 (0.81 rounds) 59.1, 56.3; 1500 x 32 (0.73) 44.9, 44.5; 4096 x 25 (1.56) 224, 205; 1792 x 64
+//   (1.75) 109, 105; 2048 x 84 (2.6) 182, 169; 2048 x 116 (3.6) 246, 230.  Not with half a round or less: 4096 x 24 (1.5) 189,
+//   211; 2048 x 80 (2.5) 162, 168; 2048 x 104 (3.25) 218, 228; 2048 x 168 (5.25) 356, 365; 16384 x 5 (1.25) 651, 780; nor where
+//   N is just past a multiple of 256: 1152 x 84 (1.5) 60.3, 71.3; 1031 x 120 (1.9; 2.3 of this kernel's) 82.8, 99.1.  Shorter
+//   sequences, where it is ahead by less, only where its last round is nearly full: 1024 x 64 37.7, 37.6; 512 x 128 25.2, 24.0;
+//   256 x 512 34.6, 31.3; not 1024 x 224 (3.5) 121, 132.
+//   Under causal masking only where its static shares come out even, and the fewer pairs of rounds the longer they have to
+//   be, because the 128-query kernel hands out more and smaller blocks.  One or two pairs: 2048 x 64 75.6, 77.5; 4096 x 32
+//   133, 129; 8192 x 16 255, 237; 2048 x 128 150, 156; 4096 x 64 265, 266 in turns of 12 ms, 261, 253 over longer ones, where
+//   the power cap rules; 8192 x 32 501, 471; 32768 x 8 1917, 1760.  Three: 4096 x 96 402, 413; 6144 x 64 567, 586; 8192 x 48
+//   745, 733.  More: 4096 x 128 539, 554; 8192 x 64 986, 1003; 8192 x 96 1608, 1510; 8192 x 128 1986, 2016; 16384 x 32 1937,
+//   1811; 16384 x 64 4040, 3868; 32768 x 16 3823, 3533.  Uneven shares lose: 2048 x 60: 72.9, 92.4; 4096 x 60: 249, 285; 2048 x
+//   80 95, 123.
 bool persistent_forward_pays(int slices, int blocks_per_slice, int n, bool causal) {
-  const int cus = (int)persistent_grid(1 << 30), total = slices * blocks_per_slice;
-  if (causal && (total > 4 * cus || n < (total > 2 * cus ? 4096 : 2048))) return false;
-  return fmha_even_shares(slices, blocks_per_slice, cus, causal);
+  const int cus = (int)persistent_grid(1 << 30);
+  const long total = (long)slices * blocks_per_slice;
+  if (causal && (n < 4096 || (n < 16384 && total > (n < 8192 ? 4 : 6) * cus))) return false;
+  if (causal || n < 1152) return fmha_even_shares(slices, blocks_per_slice, cus, causal);
+  const long rows = (long)slices * n, round = (long)cus * kFwdBlockQ, left = rows % round;
+  return (left == 0 || 2 * left > round) && (total + cus - 1) / cus <= (rows + round - 1) / round;
 }
 
 // Whether a launch of equal blocks, two to a CU, has work for at most half of the places in its last round, the second one or

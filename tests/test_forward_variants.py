@@ -122,6 +122,24 @@ def test_persistent_blocks(B, H, N, causal):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,N,causal", [
+    (26, 2048, False), (25, 4096, False), (44, 1153, False), (37, 1500, False),  # last rounds of 208, 144, 220 and 222 blocks
+    (48, 8192, True), (24, 16384, True),                                         # three pairs of rounds of work groups
+])
+def test_a_slice_alone_where_the_last_round_is_half_full(H, N, causal):
+    """The persistent kernel without even shares and with many rounds: the bits of the 128-query kernel, which takes a slice
+    alone."""
+    D, lib = 128, abi.load()
+    gen = torch.Generator(device="cuda").manual_seed(N + H)
+    q, k, v = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(3))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+    for h in (0, H // 2, H - 1):
+        one = [t[:, :, h:h + 1].contiguous() for t in (q, k, v)]
+        out1, lse1 = abi.forward(lib, *one, D ** -0.5, causal)
+        assert torch.equal(out1, out[:, :, h:h + 1]) and torch.equal(lse1, lse[:, h:h + 1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,H,N,causal", [
     (5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True), (1, 64, 2048, True),
     (2, 32, 4096, True),   # two pairs of blocks per compute unit: persistent
