@@ -1751,13 +1751,12 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
     const int last = (CAUSAL ? min(qi, N - 1) : N - 1) - j * kTile - 4 * hh;  // last key that counts
     auto p_pair = [&](int n) __attribute__((always_inline)) {
       const int c16 = n >> 2, e = (n & 3) * 2, rb = c16 >> 1, r = (c16 & 1) * 8 + e;
-      float p0 = fast_exp2(fmaf(s[rb][r], c, -my_lse2));
-      float p1 = fast_exp2(fmaf(s[rb][r + 1], c, -my_lse2));
+      float a0 = fmaf(s[rb][r], c, -my_lse2), a1 = fmaf(s[rb][r + 1], c, -my_lse2);
       if (MASKED) {
-        if (acc_row(rb, r, 0) > last) p0 = 0.f;
-        if (acc_row(rb, r + 1, 0) > last) p1 = 0.f;
+        if (acc_row(rb, r, 0) > last) a0 = -INFINITY;
+        if (acc_row(rb, r + 1, 0) > last) a1 = -INFINITY;
       }
-      p[c16][e >> 1] = pack_f16(p0, p1);
+      p[c16][e >> 1] = pack_f16(fast_exp2(a0), fast_exp2(a1));
     };
     auto read = [&](int m) __attribute__((always_inline)) {
       const int n = m % 8;
@@ -1804,20 +1803,26 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
     next_slot = next_slot == kSlots - 1 ? 0 : next_slot + 1;
   };
   int j = 0;
-  for (; j + 1 < ntw; ++j) {
+  // Only the wave's last tile can need a mask, under which it is a third longer.  The mask goes on the exponent: on the
+  // probabilities it keeps the compiler from converting two at a time.  Both: B16 H12 N512 26.9 -> 26.4 us (eight tiles a
+  // block, none masked now), B4 H16 N1024 causal 21.1 -> 20.8 us; in the dK/dV pass 25.2 -> 24.9 us.
+  const int plain = CAUSAL || N % kTile != 0 ? ntw - 1 : ntw;
+  for (; j < plain; ++j) {
     top(j);
     tile(j, IntTag<0>{});
     next(j);
   }
-  if (ntw > 0) {  // the wave's last tile, the only one that can need a mask, and what is left of it
+  if (j < ntw) {
     top(j);
     tile(j, IntTag<1>{});
     next(j);
+    ++j;
+  }
+  if (ntw > 0) {  // what is left of the wave's last tile
 #pragma unroll
     for (int n = 0; n < 16; ++n) ds_pair(n);
 #pragma unroll
     for (int n = 0; n < 8; ++n) dq_mfma(swz_cols_at<D>(ca0, ca1, n / kDB, n % kDB), n);
-    ++j;
   }
   for (; j < nt; ++j) {
     top(j);
@@ -2356,6 +2361,7 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
     constexpr bool MASKED = decltype(masked_tag)::value != 0;
     typedef __attribute__((address_space(3))) f4v lds_f4;
     h8 frag[kLead];
+    const int first_q = ki - t * kTile - 4 * hh, end_q = N - t * kTile - 4 * hh;  // queries that count, as acc_row(hq, r, 0)
     f16v dl;
     f4v ls[4];
     auto read = [&](int m) __attribute__((always_inline)) {
@@ -2365,14 +2371,13 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
     };
     auto p_pair = [&](int n) __attribute__((always_inline)) {
       const int cc = n >> 2, e = (n & 3) * 2, r = cc * 8 + e;
-      float p0 = fast_exp2(fmaf(s[r], c, -ls[r >> 2][r & 3]));
-      float p1 = fast_exp2(fmaf(s[r + 1], c, -ls[r >> 2][(r & 3) + 1]));
+      float a0 = fmaf(s[r], c, -ls[r >> 2][r & 3]), a1 = fmaf(s[r + 1], c, -ls[r >> 2][(r & 3) + 1]);
       if (MASKED) {
-        const int q = t * kTile + acc_row(hq, r, hh);
-        if ((CAUSAL && ki > q) || q >= N) p0 = 0.f;
-        if ((CAUSAL && ki > q + 1) || q + 1 >= N) p1 = 0.f;
+        const int q = acc_row(hq, r, 0);
+        if ((CAUSAL && q < first_q) || q >= end_q) a0 = -INFINITY;
+        if ((CAUSAL && q + 1 < first_q) || q + 1 >= end_q) a1 = -INFINITY;
       }
-      p[cc][e >> 1] = pack_f16(p0, p1);
+      p[cc][e >> 1] = pack_f16(fast_exp2(a0), fast_exp2(a1));
     };
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
