@@ -3,7 +3,9 @@
 // Takes the place of the reference's kernel/fused_mha_kernel.cu (forward
 // :20-323, backward :325-735, launchers :891-916) with a different design:
 //
-//   * Every GEMM runs on v_mfma_f32_32x32x16_f16 with fp32 accumulation.
+//   * Every GEMM runs on v_mfma_f32_32x32x16_f16 or, where all CUs are busy long
+//     enough to meet the power cap, v_mfma_f32_16x16x32_f16 (Geom16), with fp32
+//     accumulation; either gives the same bits.
 //   * A wave owns 32 "resident" sequence positions (queries in the forward and
 //     in the dQ pass, keys in the dK/dV pass).  Their rows stay in registers as
 //     MFMA B operands for the whole kernel.  The other sequence dimension is
@@ -17,8 +19,8 @@
 //     bank conflicts without padding.
 //   * The first GEMM is computed transposed, tile^T[streamed][resident], so a
 //     lane holds 16 streamed positions of ONE resident position per 32x32
-//     block.  Row statistics (max, sum, logsumexp, delta) are therefore plain
-//     per-lane scalars plus one exchange between the two 32-lane halves.
+//     block (16 x 16 MFMAs: of two).  Row statistics (max, sum, logsumexp, delta)
+//     are therefore plain per-lane scalars plus one exchange between lane groups.
 //   * The accumulator registers of the first GEMM, rounded to fp16, are
 //     already laid out as the B operand of the second GEMM.  P and dS therefore
 //     need no shuffling; they go through LDS only in the D = 128 backward, where
@@ -500,7 +502,7 @@ struct Strides {
 };
 
 // ---------------------------------------------------------------------------
-// Forward for D = 128 where blocks of 256 queries share out evenly over the CUs
+// Forward for D = 128 where blocks of 256 queries share out well over the CUs
 // (rule: persistent_forward_pays).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
 // tiles of 64 keys stream through a 3-slot LDS ring, copied asynchronously two
 // tiles ahead.
@@ -1885,7 +1887,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kKvWaves;  // copies per wave per tile, per tensor
   // Q ring (4), dO ring (3), per stats slot 64 lse2 then 64 delta values (1 KiB, half
-  // unused), and the P exchange: 2 buffers x per pair two 32x32 fp16 blocks (two 16-byte halves per lane each, in separate 1 KiB planes so that the 16-byte accesses are free of bank conflicts).
+  // unused), and the P exchange: 2 buffers x per pair the four fragments of P, 16 bytes per lane each, in separate 1 KiB
+  // planes so that the accesses are free of bank conflicts.
   constexpr int kStBytes = 1024;
   constexpr int kPBytes = kKvPairs * 2 * 2048;
   __shared__ __attribute__((aligned(1024))) char smem[7 * T::kBytes + 3 * kStBytes + 2 * kPBytes];
@@ -2132,8 +2135,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   auto step_copy = [&](int it) __attribute__((always_inline)) {
     if (it + 2 < n_it) copy_tiles(it + 2);
   };
-  // where this lane's registers of dS go (SPILL): its key's 32 bytes in chunk 0 of query tile 0 of
-  // query block 0; per query tile t: + (t >> 1) * np * 128 + (t & 1) * 2048, per chunk + 512 (elements)
+  // where this lane's registers of dS go (SPILL): its 16 bytes of fragment 0 of query tile 0 of
+  // query block 0; per query tile t: + (t >> 1) * np * 128 + (t & 1) * 2048, per fragment + 512 (elements)
   half_t* const ds_lane = SPILL ? dS + ((long)bh * (np >> 7)) * np * 128 + (long)(k0w >> 6) * 8192 +
                                       ((k0w >> 5) & 1) * 4096 + lane * 8
                                 : nullptr;
