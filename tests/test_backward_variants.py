@@ -164,6 +164,28 @@ def test_a_nearly_empty_last_round(H, N, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("H,N", [(3, n) for n in (1, 32, 33, 64, 65, 96, 97, 128, 129, 257, 320)] + [(260, 300), (130, 600)])
+def test_dq_ignores_dS_that_no_query_needs(H, N, causal):
+    """The workspace holds NaN where the dK/dV pass writes nothing.  dQ is that of the recomputing path, which sums the same
+    products in another order."""
+    D, lib = 128, abi.load()
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+    want = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=True)[:3]
+    nbytes = lib.fused_mha_backward_workspace_bytes(1, H, N, D)
+    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
+    got = [torch.full_like(q, float("nan")) for _ in range(3)]
+    rc = lib.fused_mha_backward(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), lse.data_ptr(),
+                                ws.data_ptr(), nbytes, *(g.data_ptr() for g in got), 1, H, N, N, D, D ** -0.5,
+                                int(causal), torch.cuda.current_stream().cuda_stream)
+    assert rc == abi.OK
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    assert (got[0].float() - want[0].float()).abs().max() <= 2e-3
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,N,causal", [
     (4, 1024, False), (5, 1024, False),      # 8 MiB of dS: stored with the used-once hint; 10 MiB: without
     (5, 1025, True), (9, 1025, True),        # 6.3 and 11.4 MiB of dS
