@@ -2895,8 +2895,9 @@ bool persistent_forward_pays(int slices, int blocks_per_slice, int n, bool causa
 // last round (1024 x 112, 1.75: 41.2, 42.2; dK/dV 69.1, 70.1.  1024 x 192, 3: 65.5, 65.6; dK/dV 110, 118), nor more rounds
 // (1024 x 288, 4.5: 96.9, 98.4), nor a causal launch, where the blocks differ (1024 x 64 forward: 16.4, 18.2).
 bool half_round_left(long blocks, int n, int max_rounds) {
+  if (n < 1024) return false;
   const long places = 2 * (long)persistent_grid(1 << 30), rounds = blocks / places, left = blocks % places;
-  return n >= 1024 && rounds >= 1 && rounds < max_rounds && left > 0 && 2 * left <= places;
+  return rounds >= 1 && rounds < max_rounds && left > 0 && 2 * left <= places;
 }
 
 template <int D, bool CAUSAL>
