@@ -2113,7 +2113,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 
   // Per iteration: wait for tile `it` (issued two iterations ago; the copies of tile
   // it+1 may still be in flight), one barrier, issue the copies of tile it+2.  Role A issues its half of them at the end
-  // of the iteration and role B near its start: all at once right after the barrier they held every wave until the copy
+  // of the iteration and role B earlier in it: all at once right after the barrier they held every wave until the copy
   // path had taken them (B2 H32 N4096 causal: 608 -> 591 us; role A after its first GEMM: 627; role B later: 609).
   auto step_wait = [&](int it) __attribute__((always_inline)) {
     if (it + 1 < n_it) {
@@ -2159,11 +2159,13 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     Product x;  // delta - dP of the previous tile
     clear(x);
     for (int it = 0; it <= n_it; ++it) {
-      // SPILL: this wave issues its tile copies and, after the second GEMM, the four stores of dS.  The wait
-      // at the top of the next iteration leaves at most as many operations in flight as those stores, the
-      // newest: every copy issued so far has then landed, whatever order stores and copies complete in.
+      // After the second GEMM this wave issues the four stores of dS (SPILL) and then its copies of tile it + 2.  The wait
+      // at the top of the next iteration leaves at most as many operations in flight as those copies, the newest:
+      // every earlier copy has then landed, whatever order stores and copies complete in.  (Copies before the second GEMM,
+      // where the wait is for them too: B2 H40 N2048 causal 198.6 us against 195.7, B2 H32 N4096 causal 566.7 against
+      // 560.6, B3 H20 N1031 94.7 against 91.9.  After the GEMM and before the stores 200.1, 569.0, 91.9; at the end of the
+      // iteration 201.7, 573.6, 95.0.)
       step_wait(it);
-      if (!SPILL) step_copy(it);
       const bool prev_active = it >= 1 && tile_active(it - 1);
       h8 y[4];
       if (prev_active) {  // the part that needs P, one tile behind
@@ -2182,11 +2184,10 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
             if (k0w + (WIDE ? 0 : 16 * (f & 1)) + i >= N) y[f] = h8{};
         }
       }
-      if (SPILL) step_copy(it);
       if (prev_active) gemm2(q_ring + ((it - 1) & 3) * T::kBytes, y);
       if (SPILL && prev_active) {
-        // dS(it - 1) leaves here, between the two GEMMs: behind this wave's tile copies by a GEMM and before those of
-        // role A, which come at the end of the iteration.  The stores go through the same path and would queue.
+        // dS(it - 1) leaves here, between the two GEMMs, before the tile copies of role A, which come at the end of the
+        // iteration: the stores go through the same path and would queue.
         const int t = t_begin + it - 1;  // the query tile
         half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048;
         static_for<4>([&](auto f_tag) __attribute__((always_inline)) {
@@ -2195,6 +2196,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
           else store16_keep(dst, y[f], IntTag<at>{});
         });
       }
+      step_copy(it);
       if (it < n_it && tile_active(it)) {
         const char* Gl = g_ring + (it % 3) * T::kBytes;
         const char* Sl = st_ring + (it % 3) * kStBytes + st_off;
