@@ -131,4 +131,12 @@ FMHA_HOST_DEVICE int fmha_paired_block(int lin, int total) {
   const int slots = (end - xcd + 7) >> 3;  // work groups below `end` on this XCD
   return ((kCus / 8 + slots - 1 - (lin >> 3)) << 3) + xcd;
 }
+
+// Row statistics: blocks of consecutive rows, numbered through all slices, taken from `chains` runs of `chain` blocks by
+// turns.  With a run about as long as a slice, work groups that follow each other read the same positions of different heads,
+// which lie side by side.  A launch has chain * chains work groups, those past the last block have nothing to do.
+FMHA_HOST_DEVICE unsigned fmha_interleaved_block(unsigned lin, unsigned chain, unsigned chains) {
+  const unsigned step = lin / chains;
+  return (lin - step * chains) * chain + step;
+}
 #endif  // FMHA_BLOCK_MAP_H_

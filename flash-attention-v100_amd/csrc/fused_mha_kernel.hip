@@ -1303,22 +1303,39 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 // flash_attn_interface.py:43-44 (which work in fp16).  Also writes the
 // logsumexp scaled to the exp2 domain, lse2 = lse * log2(e), behind delta in
 // the workspace, so the dK/dV pass gets both row statistics with one copy.
-// A block takes consecutive rows of one slice, so that the only divisions are of the block number, by the scalar unit, and
-// its statistics are written together.  D = 128: B2 H40 N2048 20.2 -> 17.7 us (4.7 TB/s), B3 H20 N1031 8.5 -> 7.4 us, B4 H16
-// N512 5.1 -> 4.8 us against rows numbered through with three 64-bit divisions per thread; two or four rows per thread are
-// at most 0.8 us faster at the largest and slower at the others (17.0, 17.1; 7.5, 7.9; 5.0, 5.5).
+// Bound by its bytes (5.6-6.1 TB/s on tensors used again and again; small problems take 7 us to start and end).  Rows are
+// numbered through slice by slice, which is the order of the statistics: a block writes its 16 (D = 64: 32) together, and
+// none of it idles where sequences are short.  Slice and row come from divisions of the block's first row by the scalar unit;
+// only threads past the end of that slice divide again.  Blocks in flight at a time are those of the same positions of
+// different heads (fmha_interleaved_block), so that O and dO are read through: in the order of the rows, 256 bytes of each
+// position, strides that are a power of two can meet in a few channels.  D = 128, us: rows in the order of O with three 64-bit
+// divisions a thread; blocks one after the other in this order, with an end at each slice; and as it is: B1024 H32 N1 7.2,
+// 11.9, 6.9; B256 H32 N17 14.8, 18.9, 14.3; B3 H20 N1031 7.1, 6.9, 6.9; B64 H16 N512 52.9, 46.1, 45.8; B2 H40 N2048 18.1, 15.2,
+// 15.4; B2 H32 N4096 25.4, 28.6, 23.6; B1 H64 N8192 44.7, 45 or 68 by where the tensors lie, 44.8; B1 H16 N32768 52, 46, 43.
 // ---------------------------------------------------------------------------
 constexpr int delta_rows(int d) { return 256 * 8 / d; }  // of a block
 template <int D>
 __global__ void __launch_bounds__(256)
 fmha_bwd_delta_kernel(const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides gs,
-                      const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, int H, int N,
-                      int nb, int first_slice) {
-  constexpr int kLanesPerRow = D / 8;
-  const int in_launch = blockIdx.x / nb, slice = first_slice + in_launch, b = slice / H, h = slice - b * H;
-  const int n = (blockIdx.x - in_launch * nb) * delta_rows(D) + threadIdx.x / kLanesPerRow, c = threadIdx.x % kLanesPerRow;
+                      const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, unsigned H,
+                      unsigned N, unsigned first, unsigned end, unsigned chain, unsigned chains) {
+  constexpr unsigned kLanesPerRow = D / 8;
+  const unsigned row0 = first + fmha_interleaved_block(blockIdx.x, chain, chains) * delta_rows(D);  // rows first .. end - 1
+  const unsigned slice0 = row0 / N, b0 = slice0 / H;
+  const unsigned in_block = threadIdx.x / kLanesPerRow, row = row0 + in_block, c = threadIdx.x % kLanesPerRow;
+  unsigned n = row0 - slice0 * N + in_block, h = slice0 - b0 * H, b = b0;
+  if (n >= N) {  // past the end of the slice that the block starts in
+    const unsigned later = n / N;
+    n -= later * N;
+    h += later;
+    if (h >= H) {
+      const unsigned batches = h / H;
+      b += batches;
+      h -= batches * H;
+    }
+  }
   float acc = 0.f;
-  if (n < N) {  // O is dense, dO has its own strides
+  if (row < end) {  // O is dense, dO has its own strides
     const h8 a = *reinterpret_cast<const h8*>(O + (((long)b * N + n) * H + h) * D + c * 8);
     const h8 g = *reinterpret_cast<const h8*>(dO + b * gs.b + (long)n * gs.n + (long)h * gs.h + c * 8);
 #pragma unroll
@@ -1326,10 +1343,9 @@ fmha_bwd_delta_kernel(const half_t* __restrict__ O, const half_t* __restrict__ d
   }
 #pragma unroll
   for (int off = kLanesPerRow / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-  if (n < N && c == 0) {
-    const long at = (long)slice * N + n;
-    delta[at] = acc;
-    lse2[at] = LSE[at] * kLog2e;
+  if (row < end && c == 0) {
+    delta[row] = acc;
+    lse2[row] = LSE[row] * kLog2e;
   }
 }
 
@@ -3027,12 +3043,15 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   const size_t touched = ds_bytes + 6 * (size_t)slices_at_once * n * D * sizeof(half_t);
   const int stream_ds = ds_bytes < (10u << 20) || touched > (256u << 20);
   if ((passes & kPassDelta) && !dq_makes_stats) {
-    const int nb = (n + delta_rows(D) - 1) / delta_rows(D);
-    const int fit = ((1 << 24) - 1) / nb, most = fit > 0 ? fit : 1;  // slices of a launch of fewer than 2^32 threads
-    for (int first = 0; first < slices; first += most) {
-      const int count = slices - first < most ? slices - first : most;
-      if (launch(fmha_bwd_delta_kernel<D>, (unsigned)(nb * count), 256, stream, (const half_t*)o, (const half_t*)d_o, gs,
-                 (const float*)lse, delta, lse2, head, n, nb, first) != hipSuccess)
+    const unsigned rows = (unsigned)slices * n;              // fewer than 2^32 / (D / 8): check_shape
+    const unsigned most = (1u << 23) * delta_rows(D);        // a launch of fewer than 2^32 threads: fewer than twice the blocks
+    for (unsigned first = 0; first < rows; first += most) {
+      const unsigned end = rows - first < most ? rows : first + most;
+      const unsigned blocks = (end - first + delta_rows(D) - 1) / delta_rows(D);
+      const unsigned per_slice = (unsigned)(n + delta_rows(D) - 1) / delta_rows(D);
+      const unsigned chain = per_slice < blocks ? per_slice : blocks, chains = (blocks + chain - 1) / chain;
+      if (launch(fmha_bwd_delta_kernel<D>, chain * chains, 256, stream, (const half_t*)o, (const half_t*)d_o, gs,
+                 (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains) != hipSuccess)
         return FUSED_MHA_ERR_LAUNCH;
     }
   }

@@ -327,3 +327,26 @@ def test_capture_with_a_large_workspace():
         torch.cuda.synchronize()
         for a, b in zip(replayed, eager):
             assert torch.equal(a, b)
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,N", [
+    (3, 5, 1), (67, 3, 1), (9, 7, 2), (5, 1, 7), (2, 5, 15), (2, 3, 16), (3, 3, 17),  # blocks with rows of many slices and batches
+    (2, 3, 31), (2, 3, 32), (3, 2, 33), (2, 4, 100), (1, 3, 1031), (2, 8, 512),
+])
+def test_row_statistics(B, H, N, D):
+    """delta and lse * log2(e) of every row, whatever rows share a block, and nothing behind them."""
+    lib = abi.load()
+    gen = torch.Generator(device="cuda").manual_seed(B * H * N)
+    out, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(2))
+    lse = torch.randn(B, H, N, device="cuda", generator=gen)
+    nbytes, rows = lib.fused_mha_backward_min_workspace_bytes(B, H, N, D), B * H * N
+    ws = torch.full((nbytes // 4 + 64,), float("nan"), device="cuda")
+    assert lib.fused_mha_backward_delta(out.data_ptr(), do.data_ptr(), lse.data_ptr(), ws.data_ptr(), nbytes, B, H, N, D,
+                                        torch.cuda.current_stream().cuda_stream) == abi.OK
+    products = (out.double() * do.double()).permute(0, 2, 1, 3)
+    error = (ws[:rows].view(B, H, N) - products.sum(-1)).abs()
+    assert (error <= D * 2.0 ** -24 * products.abs().sum(-1)).all()  # D roundings of partial sums in fp32
+    want = lse.double() / torch.log(torch.tensor(2.0, dtype=torch.float64))
+    assert ((ws[rows:2 * rows].view(B, H, N) - want).abs() <= 2.0 ** -22 * want.abs()).all()  # the constant's and the product's
+    assert nbytes == 8 * rows and torch.isnan(ws[2 * rows:]).all()

@@ -405,6 +405,36 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_interleaved_blocks_are_a_bijection(tmp_path):
+    """csrc/block_map.h: the row statistics' work groups take every block of a launch once, and few more than there are."""
+    import subprocess
+
+    src = tmp_path / "check_rows.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (unsigned blocks = 1; blocks <= 700; ++blocks)
+    for (unsigned chain = 1; chain <= blocks; chain += (chain < 40 ? 1 : 13)) {
+      const unsigned chains = (blocks + chain - 1) / chain;
+      if (chain * chains >= blocks + chain) { printf("many %u %u\n", blocks, chain); return 1; }
+      std::vector<int> seen(chain * chains, 0);
+      for (unsigned lin = 0; lin < chain * chains; ++lin) {
+        const unsigned at = fmha_interleaved_block(lin, chain, chains);
+        if (at >= seen.size() || seen[at]++) { printf("%u %u %u\n", blocks, chain, lin); return 1; }
+      }
+    }
+  puts("ok");
+  return 0;
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    exe = tmp_path / "check_rows"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
 def test_installed_distribution_imports_without_pythonpath(tmp_path):
     """`pip install .` (the wheel `python setup.py install` / `pip wheel .` build; reference setup.py:151-172,
     README.md:21-23) puts the package, the extension and the kernel library into one place, and the package
