@@ -77,6 +77,41 @@ FMHA_HOST_DEVICE bool fmha_even_shares(int slices, int blocks_per_slice, int G, 
   return total * 16 >= (total + G - 1) / G * G * 15;
 }
 
+// Whether the persistent 256-query forward takes a D = 128 problem.  It does up to 10 % more per second than the 128-query
+// kernel where all CUs are busy, but a CU takes or leaves a whole block of 256.  Figures: us of the 128-query kernel, then of
+// this one, at N x slices, over stretches of 0.15 s in turn.  The chip is at its power cap and what one kernel draws slows the
+// others, so a call counts with what else runs: "+" with its backward behind.  Cards differ: A and B.
+//   Under causal masking where its static shares come out even, whatever the number of rounds, from N = 4096 on, where a block
+// has 32 tiles on average.  A: 4096 x 64 265, 261, + 1108, 1104; x 96 413, 399, + 1674, 1660; x 128 548, 541, + 2244, 2246; x
+// 192 828, 806, + 3355, 3343; 6144 x 64 581, 565, + 2350, 2345; 8192 x 64 1012, 967, + 4081, 4032; x 96 1686, 1441, + 6458,
+// 6207; x 128 2060, 1947, + 8249, 8178.  B: 4096 x 64 264, 247, + 1153, 1085; x 96 412, 384, + 1698, 1633; x 128 549, 514, +
+// 2240, 2207; x 512 2164, 2063, + 8890, 8768; 8192 x 96 1641, 1397, + 6283, 5996; 8001 x 64 957, 923, + 3881, 3852; 16384 x
+// 64 4104, 3518, + 15367, 14829.  In turns of 12 ms each has the clock that both together leave, which favours the one that
+// draws more: 4096 x 96 397, 396; x 192 790, 809; 8192 x 128 1963, 1915.  Not at N = 2048, where card A shows nothing (x 64 76.2,
+// 74.7, + 319, 323; x 128 148, 149, + 651, 653) though B does (x 128 147, 146, + 681, 646); nor with uneven shares: 4100 x
+// 128 571, 669; 5120 x 64 415, 450; 7168 x 64 787, 890.
+//   Without a mask, from N = 1152 on, where the last round of the 128-query kernel (two blocks to a CU, so that half a round
+// costs it 0.6 of one) is more than half full and this one needs no more rounds.  A: 4096 x 16 126, 114, + 499, 488; x 64 485,
+// 448, + 1974, 1945; x 25 (1.56 rounds) 220, 198, + 883, 888; x 42 (2.6) 343, 314, + 1356, 1346; 8192 x 13 434, 387, + 1722,
+// 1700; 2048 x 30 (0.94) 64.3, 59.9, + 260, 258; 2048 x 64 129, 122, + 534, 530; 3000 x 20 90.1, 82.7, + 367, 365; 1500 x 42
+// 51.9, 48.3, + 211, 210; 1500 x 69 (1.6) 89.7, 87.7, + 380, 386.  Not with half a round or less: the idle CUs leave the others
+// a higher clock when nothing else runs, but not beside a backward that is at the cap.  4096 x 24 (1.5) 188, 197; x 56 (3.5)
+// 428, 415, + 1736, 1748; x 68 (4.25) 530, 520, + 2173, 2187; x 100 (6.25) 779, 753, + 3191, 3192; 8192 x 28 (3.5) 842, 801,
+// + 3337, 3369; x 42 (5.25) 1280, 1228, + 5118, 5166; 16384 x 17 (4.25) 2062, 1998, + 8134, 8289; 2048 x 168 (5.25) 361, 353,
+// + 1440, 1451.  (B: 4096 x 56 + 1768, 1721; x 100 + 3165, 3148; 8192 x 42 + 4961, 4997.)  Nor where N is just past a multiple
+// of 256: 1152 x 84 (1.5) 60.3, 71.3; 1031 x 120 (1.9; 2.3 of this kernel's) 82.8, 99.1.  Shorter sequences only where the last
+// round is nearly full, as good alone, not with a backward: 1024 x 64 38.1, 36.2, + 154, 158; 512 x 128 24.1, 23.9, + 98, 103;
+// 256 x 512 32.0, 30.8, + 139, 142; not 1024 x 224 (3.5) 121, 132.
+constexpr int kPersistentForwardRows = 256;  // queries of a block
+FMHA_HOST_DEVICE bool fmha_persistent_forward_pays(int slices, int n, int cus, bool causal) {
+  const int blocks_per_slice = (n + kPersistentForwardRows - 1) / kPersistentForwardRows;
+  if (causal) return n >= 4096 && fmha_even_shares(slices, blocks_per_slice, cus, true);
+  if (n < 1152) return fmha_even_shares(slices, blocks_per_slice, cus, false);
+  const long total = (long)slices * blocks_per_slice;
+  const long rows = (long)slices * n, round = (long)cus * kPersistentForwardRows, left = rows % round;
+  return (left == 0 || 2 * left > round) && (total + cus - 1) / cus <= (rows + round - 1) / round;
+}
+
 // Launches of one block per work group that the hardware hands out as CUs become free, two or more to a CU.
 // heavy_first (causal masking, blocks numbered heaviest first): the blocks of many slices are ordered block-index
 // major, so that heavy blocks start first and the launch ends with light ones.  An XCD's slices are taken in groups of

@@ -537,7 +537,7 @@ struct Strides {
 
 // ---------------------------------------------------------------------------
 // Forward for D = 128 where blocks of 256 queries share out well over the CUs
-// (rule: persistent_forward_pays).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
+// (rule: fmha_persistent_forward_pays).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
 // tiles of 64 keys stream through a 3-slot LDS ring, copied asynchronously two
 // tiles ahead.
 //
@@ -564,6 +564,7 @@ constexpr float kRescaleSum = 4096.f;
 constexpr int kFwdWaves = 8;
 constexpr int kFwdThreads = kFwdWaves * 64;
 constexpr int kFwdBlockQ = kFwdWaves * kResident;
+static_assert(kFwdBlockQ == kPersistentForwardRows, "");
 constexpr int kRing = 3;
 
 // The kernel is persistent: the launch has one work group per CU (fewer for small
@@ -925,7 +926,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 
 // ---------------------------------------------------------------------------
 // Forward for D = 64, and for D = 128 where blocks of 256 queries do not share out evenly (rule:
-// persistent_forward_pays).  Block = 4 waves, one per SIMD, of 32 queries each; two blocks share a CU.
+// fmha_persistent_forward_pays).  Block = 4 waves, one per SIMD, of 32 queries each; two blocks share a CU.
 //
 // What bounds it: a wave issues one instruction every 4-5 cycles, so one that runs scores, softmax and accumulation one
 // after the other needs 1,800 cycles per 32 x 64 tile at D = 64 (MFMA 512, vector instructions 700) and a SIMD needs
@@ -2882,33 +2883,6 @@ bool bad_strides(const fused_mha_strides* st) {
   return st->seq >= (1 << 24) || st->head >= (1LL << 31);
 }
 
-// Whether the persistent 256-query forward takes a D = 128 problem.  It does up to 10 % more per second than the 128-query
-// kernel where all CUs are busy, but a CU takes or leaves a whole block of 256.  Figures: us of the 128-query kernel, then of
-// this one, at N x slices.
-//   Without a mask, from N = 1152 on, where the last round of the 128-query kernel (two blocks to a CU, so that half a round
-//   costs it 0.6 of one) is more than half full and this one needs no more rounds: 4096 x 64: 497, 455; 4096 x 16 128, 117;
-//   8192 x 7 224, 205; 2048 x 26 (0.81 rounds) 59.1, 56.3; 1500 x 32 (0.73) 44.9, 44.5; 4096 x 25 (1.56) 224, 205; 1792 x 64
-//   (1.75) 109, 105; 2048 x 84 (2.6) 182, 169; 2048 x 116 (3.6) 246, 230.  Not with half a round or less: 4096 x 24 (1.5) 189,
-//   211; 2048 x 80 (2.5) 162, 168; 2048 x 104 (3.25) 218, 228; 2048 x 168 (5.25) 356, 365; 16384 x 5 (1.25) 651, 780; nor where
-//   N is just past a multiple of 256: 1152 x 84 (1.5) 60.3, 71.3; 1031 x 120 (1.9; 2.3 of this kernel's) 82.8, 99.1.  Shorter
-//   sequences, where it is ahead by less, only where its last round is nearly full: 1024 x 64 37.7, 37.6; 512 x 128 25.2, 24.0;
-//   256 x 512 34.6, 31.3; not 1024 x 224 (3.5) 121, 132.
-//   Under causal masking only where its static shares come out even, and the fewer pairs of rounds the longer they have to
-//   be, because the 128-query kernel hands out more and smaller blocks.  One or two pairs: 2048 x 64 75.6, 77.5; 4096 x 32
-//   133, 129; 8192 x 16 255, 237; 2048 x 128 150, 156; 4096 x 64 265, 266 in turns of 12 ms, 261, 253 over longer ones, where
-//   the power cap rules; 8192 x 32 501, 471; 32768 x 8 1917, 1760.  Three: 4096 x 96 402, 413; 6144 x 64 567, 586; 8192 x 48
-//   745, 733.  More: 4096 x 128 539, 554; 8192 x 64 986, 1003; 8192 x 96 1608, 1510; 8192 x 128 1986, 2016; 16384 x 32 1937,
-//   1811; 16384 x 64 4040, 3868; 32768 x 16 3823, 3533.  Uneven shares lose: 2048 x 60: 72.9, 92.4; 4096 x 60: 249, 285; 2048 x
-//   80 95, 123.
-bool persistent_forward_pays(int slices, int blocks_per_slice, int n, bool causal) {
-  const int cus = (int)persistent_grid(1 << 30);
-  const long total = (long)slices * blocks_per_slice;
-  if (causal && (n < 4096 || (n < 16384 && total > (n < 8192 ? 4 : 6) * cus))) return false;
-  if (causal || n < 1152) return fmha_even_shares(slices, blocks_per_slice, cus, causal);
-  const long rows = (long)slices * n, round = (long)cus * kFwdBlockQ, left = rows % round;
-  return (left == 0 || 2 * left > round) && (total + cus - 1) / cus <= (rows + round - 1) / round;
-}
-
 // Whether a launch of equal blocks, two to a CU, has work for at most half of the places in its last round, the second one or
 // (up to max_rounds) the third.  Two blocks that share a CU evenly end together, and the last ones then run alone, at little
 // over half the rate of a pair; with one of the two going first (odd_slots_first) its place is free sooner, and the last
@@ -2934,7 +2908,7 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
   const int negate = scale < 0.f ? 1 : 0;
   if constexpr (D == 128) {
     const int nmb = (n + kFwdBlockQ - 1) / kFwdBlockQ, total = nmb * batch * head;
-    if (persistent_forward_pays(batch * head, nmb, n, CAUSAL)) {
+    if (fmha_persistent_forward_pays(batch * head, n, (int)persistent_grid(1 << 30), CAUSAL)) {
       const hipError_t rc = launch(fmha_fwd_kernel<D, CAUSAL>, persistent_grid(total), kFwdThreads, stream,
                                    (const half_t*)q, (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o,
                                    (float*)lse, head, n, nmb, total, c, negate);

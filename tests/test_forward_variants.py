@@ -78,6 +78,41 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def _persistent(tmp_path, shapes):
+    """Which of the (slices, N, causal) problems the 256-query kernel takes on 256 compute units: the rule of
+    csrc/block_map.h, compiled for the host."""
+    src, exe = tmp_path / "rule.cpp", tmp_path / "rule"
+    src.write_text(r'''
+#include <cstdio>
+#include <cstdlib>
+#include "block_map.h"
+int main(int argc, char** argv) {
+  for (int i = 1; i + 2 < argc; i += 3)
+    putchar(fmha_persistent_forward_pays(atoi(argv[i]), atoi(argv[i + 1]), 256, atoi(argv[i + 2])) ? '1' : '0');
+  return 0;
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    out = subprocess.check_output([str(exe)] + [str(int(x)) for s in shapes for x in s]).decode()
+    assert len(out) == len(shapes)
+    return [c == "1" for c in out]
+
+
+def test_rule_between_the_forward_kernels(tmp_path):
+    """Causal launches with even shares: by the length alone, however many rounds they have.  Without a mask: by the last
+    round."""
+    pairs = [(n, 512 // (-(-n // 256)) * k) for n in (1024, 2048, 4095, 4096, 8001, 8192, 16384) for k in range(1, 9)]
+    assert all(slices % 8 == 0 for _, slices in pairs)
+    assert _persistent(tmp_path, [(slices, n, True) for n, slices in pairs]) == [n >= 4096 for n, _ in pairs]
+    uneven = [(60, 2048), (60, 4096), (128, 4100), (64, 5120), (64, 7168), (4, 32768)]
+    assert not any(_persistent(tmp_path, [(s, n, True) for s, n in uneven]))
+    taken = [(64, 4096), (25, 4096), (42, 4096), (13, 8192), (30, 2048), (32, 1500), (128, 512), (256, 256)]
+    left = [(24, 4096), (56, 4096), (84, 4096), (100, 4096), (28, 8192), (42, 8192), (84, 1152), (120, 1031), (224, 1024)]
+    assert all(_persistent(tmp_path, [(s, n, False) for s, n in taken]))
+    assert not any(_persistent(tmp_path, [(s, n, False) for s, n in left]))
+
+
 def _inputs(B, N, H, D, growing):
     """growing: the score scale rises with the key index, so that nearly every 64-key tile holds a maximum that is
     more than 2^12 times (12 in the exp2 domain) above the earlier ones and the running maximum is raised in it."""
