@@ -6,6 +6,7 @@ compiled from here."""
 import ctypes
 import os
 import re
+import subprocess
 
 import torch  # noqa: F401  (load order matters)
 
@@ -31,6 +32,17 @@ class Strides(ctypes.Structure):
 
 
 _sp = ctypes.POINTER(Strides)
+
+
+def host_rule(tmp_path, expression, cases):
+    """The truth of an expression in csrc/block_map.h, compiled for the host, at x = each case (whole numbers)."""
+    src, exe = tmp_path / "rule.cpp", tmp_path / "rule"
+    rows = ", ".join("{%s}" % ", ".join(str(int(v)) for v in case) for case in cases)
+    src.write_text('#include <cstdio>\n#include "block_map.h"\nint main() {\n  const int cases[][%d] = {%s};\n'
+                   "  for (auto& x : cases) putchar(%s ? '1' : '0');\n}\n" % (len(cases[0]), rows, expression))
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "flash-attention-v100_amd", "csrc"), str(src),
+                           "-o", str(exe)])
+    return [c == "1" for c in subprocess.check_output([str(exe)]).decode()]
 
 
 def declared_symbols():

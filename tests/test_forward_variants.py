@@ -79,24 +79,8 @@ int main() {
 
 
 def _persistent(tmp_path, shapes):
-    """Which of the (slices, N, causal) problems the 256-query kernel takes on 256 compute units: the rule of
-    csrc/block_map.h, compiled for the host."""
-    src, exe = tmp_path / "rule.cpp", tmp_path / "rule"
-    src.write_text(r'''
-#include <cstdio>
-#include <cstdlib>
-#include "block_map.h"
-int main(int argc, char** argv) {
-  for (int i = 1; i + 2 < argc; i += 3)
-    putchar(fmha_persistent_forward_pays(atoi(argv[i]), atoi(argv[i + 1]), 256, atoi(argv[i + 2])) ? '1' : '0');
-  return 0;
-}
-''')
-    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
-    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
-    out = subprocess.check_output([str(exe)] + [str(int(x)) for s in shapes for x in s]).decode()
-    assert len(out) == len(shapes)
-    return [c == "1" for c in out]
+    """Which of the (slices, N, causal) problems the 256-query kernel takes."""
+    return abi.host_rule(tmp_path, "fmha_persistent_forward_pays(x[0], x[1], 256, x[2])", shapes)
 
 
 def test_rule_between_the_forward_kernels(tmp_path):
@@ -146,21 +130,41 @@ def test_small_blocks(N, causal, D):
         _check(1, N, 3, D, causal, growing)
 
 
+PERSISTENT = [  # B, H, N, causal: launches of the 256-query kernel
+    (5, 17, 700, False), (1, 256, 250, False),  # 255 and 256 blocks
+    (1, 32, 4096, True), (1, 16, 8001, True),   # one pair of blocks per compute unit
+]
+FULL = [  # launches of the other kernel with as many queries
+    (1, 63, 2000, True),                        # 504 blocks of 256: no even shares
+    (1, 32, 3900, True), (1, 64, 2048, True),   # even ones, too short
+]
+
+
+def test_shapes_take_the_kernel_they_are_meant_for(tmp_path):
+    """On 256 compute units."""
+    several = [(2, 32, 4096, True), (1, 32, 8001, True)]
+    assert all(_persistent(tmp_path, [(B * H, N, causal) for B, H, N, causal in PERSISTENT + several] +
+                           [(H, N, causal) for H, N, causal in MANY_ROUNDS] +
+                           [(B * H, N, causal) for B, H, N, _, causal in NOT_FINITE_PERSISTENT]))
+    assert not any(_persistent(tmp_path, [(B * H, N, causal) for B, H, N, causal in FULL + [(1, 61, 4099, True)]]))
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,N,causal", [(5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True),
-                                            (1, 32, 3900, True)])
+@pytest.mark.parametrize("B,H,N,causal", PERSISTENT + FULL)
 def test_persistent_blocks(B, H, N, causal):
-    """255 and 256 blocks of 256 queries without a mask, 512 with one: launches the persistent kernel takes.  504 blocks
-    with a mask do not share out evenly and go to the other kernel."""
+    """Launches the persistent kernel takes and such that it nearly takes."""
     for growing in (False, True):
         _check(B, N, H, 128, causal, growing, heads=[0, H // 2, H - 1])
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("H,N,causal", [
+MANY_ROUNDS = [
     (26, 2048, False), (25, 4096, False), (44, 1153, False), (37, 1500, False),  # last rounds of 208, 144, 220 and 222 blocks
-    (48, 8192, True), (24, 16384, True),                                         # three pairs of rounds of work groups
-])
+    (48, 8192, True), (24, 16384, True), (96, 4096, True),                       # three pairs of rounds of work groups
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,N,causal", MANY_ROUNDS)
 def test_a_slice_alone_where_the_last_round_is_half_full(H, N, causal):
     """The persistent kernel without even shares and with many rounds: the bits of the 128-query kernel, which takes a slice
     alone."""
@@ -175,12 +179,10 @@ def test_a_slice_alone_where_the_last_round_is_half_full(H, N, causal):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,N,causal", [
-    (5, 17, 700, False), (1, 256, 250, False), (1, 63, 2000, True), (1, 64, 2048, True),
+@pytest.mark.parametrize("B,H,N,causal", PERSISTENT + FULL + [
     (2, 32, 4096, True),   # two pairs of blocks per compute unit: persistent
     (1, 61, 4099, True),   # 17 blocks a slice, the last one of three queries
-    (1, 32, 3900, True),   # one pair per compute unit, with a ragged end: persistent
-    (1, 32, 8001, True),   # two pairs: persistent
+    (1, 32, 8001, True),   # two pairs, with a ragged end: persistent
 ])
 def test_a_slice_alone_gives_the_same_bits(B, H, N, causal):
     """One slice has too few blocks for the persistent kernel, the whole problem takes it (or the other one: then there
@@ -196,10 +198,12 @@ def test_a_slice_alone_gives_the_same_bits(B, H, N, causal):
             assert torch.equal(o1, out[b:b + 1, :, h:h + 1]) and torch.equal(l1, lse[b:b + 1, h:h + 1])
 
 
+NOT_FINITE_PERSISTENT = [(5, 17, 700, 128, False), (1, 32, 4096, 128, True), (1, 16, 8001, 128, True)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,N,D,causal", [
-    (1, 3, 449, 64, False), (1, 3, 449, 64, True), (1, 3, 449, 128, False), (1, 3, 449, 128, True),
-    (5, 17, 700, 128, False), (1, 64, 2048, 128, True),  # persistent: 255 blocks, and one pair of blocks per unit
+@pytest.mark.parametrize("B,H,N,D,causal", NOT_FINITE_PERSISTENT + [
+    (1, 3, 449, 64, False), (1, 3, 449, 64, True), (1, 3, 449, 128, False), (1, 3, 449, 128, True), (1, 64, 2048, 128, True),
 ])
 def test_rows_that_are_not_finite(B, H, N, D, causal):
     """Queries with a NaN or an infinity give NaN rows and make their wave raise its maximum at every tile; the finite rows
