@@ -3030,14 +3030,7 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
     }
   }
   const float c = scale * kLog2e;
-  // Which MFMAs the D = 128 passes use, both the same, since it decides the order of dS in the workspace: 16 x 16 where the
-  // chip runs at its power cap, 32 x 32 where a good part of the CUs has nothing to do and a wave's own instructions are
-  // what takes the time.  us of the dK/dV pass with 32 x 32 and with 16 x 16 MFMAs, N x slices (blocks per CU): without a
-  // mask 1031 x 16 31.4, 33.1 (0.56); 4096 x 5 105.8, 104.2 (0.63); 1031 x 20 33.9, 33.8 (0.70); 1031 x 28 41.8, 41.2; 4096 x 8
-  // 139, 134 (1); 512 x 64 25.2, 24.0.  Causal, where a block is half as much work: 4096 x 6 94.0, 100.8 (0.75); 16384 x 2
-  // 398, 405 (1); 4096 x 10 111.1, 111.2 (1.25); 16384 x 3 477, 469 (1.5); 2048 x 32 83.7, 80.1 (2); 2048 x 80 212, 201.  dQ
-  // pass over dS: 1031 x 8 11.5, 12.8; 4096 x 4 causal 33.0, 35.6; 1031 x 60 42, 40.5; 2048 x 80 causal 97, 88.
-  auto wide = [&]() { return (long)key_blocks(n) * slices * (CAUSAL ? 1 : 2) * 4 < 5 * cus; };
+  auto wide = [&]() { return fmha_wide_mfmas((long)key_blocks(n) * slices, cus, CAUSAL); };
   auto dq_pass = [&]() {
     if constexpr (D == 64) {
       const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ;

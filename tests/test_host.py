@@ -405,6 +405,17 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_full_launches_take_the_kernels_they_are_meant_for(tmp_path):
+    """On 256 compute units."""
+    from test_parity_gpu import FULL_LAUNCHES
+
+    wide = "fmha_wide_mfmas((long)((x[1] + 127) / 128) * x[0], 256, x[2])"
+    shapes = [(B * H, N, causal) for B, H, N, causal in FULL_LAUNCHES]
+    assert not any(abi.host_rule(tmp_path, wide, shapes))
+    assert abi.host_rule(tmp_path, "fmha_persistent_forward_pays(x[0], x[1], 256, x[2])", shapes) == [True] * 3 + [False] * 2
+    assert all(abi.host_rule(tmp_path, wide, [(31, 520, False), (63, 520, True), (4, 320, True)]))
+
+
 def test_interleaved_blocks_are_a_bijection(tmp_path):
     """csrc/block_map.h: the row statistics' work groups take every block of a launch once, and few more than there are."""
     import subprocess

@@ -305,6 +305,55 @@ def test_strided_inputs_c_abi(lib, B, H, N, D, causal):
         assert torch.equal(dq, dq_d) and torch.equal(dk, dk_d) and torch.equal(dv, dv_d), name
 
 
+FULL_LAUNCHES = [  # B, H, N, causal at head size 128: launches of the kernels with 16 x 16 MFMAs
+    (16, 32, 250, False), (1, 32, 4096, True), (1, 16, 8001, True),  # the 256-query forward too
+    (2, 20, 520, False), (4, 20, 520, True),                         # both backward passes
+]
+
+
+@pytest.mark.parametrize("B,H,N,causal", FULL_LAUNCHES)
+def test_strided_inputs_of_full_launches(lib, B, H, N, causal):
+    """As above where the problem fills the chip, and with strides that differ between the tensors."""
+    D, scale = 128, 1.0 / math.sqrt(128)
+    (q, k, v, do), cases = _strided_cases(B, N, H, D, seed=N)
+    packed, heads_first, wide = cases["packed_qkv"], cases["heads_first"], cases["wide_rows"]
+    cases["mixed"] = (packed[0], heads_first[1], wide[2], heads_first[3])
+    cases["mixed_the_other_way"] = (heads_first[0], wide[1], packed[2], wide[3])
+    dense = [t.cuda() for t in (q, k, v, do)]
+    out_d, lse_d = abi.forward(lib, *dense[:3], scale, causal)
+    grads_d = abi.backward(lib, *dense[:3], out_d, dense[3], lse_d, scale, causal)[:3]
+    for name, (qs, ks, vs, gs) in cases.items():
+        out, lse = abi.forward_strided(lib, qs, ks, vs, scale, causal)
+        grads = abi.backward_strided(lib, qs, ks, vs, out, gs, lse, scale, causal)
+        assert torch.equal(out, out_d) and torch.equal(lse, lse_d), name
+        for a, b in zip(grads, grads_d):
+            assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("B,H,N,causal", FULL_LAUNCHES)
+def test_negative_scale_of_full_launches(lib, B, H, N, causal):
+    """A negative scale is the positive one with -q, and dQ changes its sign.  The forward negates the queries itself: the
+    same bits.  The backward has the scale behind S, and the matrix cores do not round S of q and of -q alike: fp32 scores
+    differ in the last bit, here and there P or dS in the last of fp16, which is no more than another order of the sums
+    changes.  Against the oracle on three heads."""
+    D, scale = 128, -0.11
+    q, k, v, do = ao.make_inputs(B, N, H, D, seed=N + 1)
+    qg, kg, vg, dog = (t.cuda() for t in (q, k, v, do))
+    out, lse = abi.forward(lib, qg, kg, vg, scale, causal)
+    dq, dk, dv = abi.backward(lib, qg, kg, vg, out, dog, lse, scale, causal)[:3]
+    out2, lse2 = abi.forward(lib, -qg, kg, vg, -scale, causal)
+    dq2, dk2, dv2 = abi.backward(lib, -qg, kg, vg, out2, dog, lse2, -scale, causal)[:3]
+    assert torch.equal(out, out2) and torch.equal(lse, lse2)
+    for a, b in ((dq, -dq2), (dk, dk2), (dv, dv2)):
+        assert (a.float() - b.float()).abs().max() <= 2e-3 * max(1.0, b.abs().max().item())
+    for b, h in ((0, 0), (B // 2, H // 2), (B - 1, H - 1)):
+        one = [t[b:b + 1, :, h:h + 1] for t in (q, k, v, do)]
+        refs = (ao.attention_forward(*one[:3], scale, causal)[0],) + tuple(ao.attention_backward(*one, scale, causal))
+        for got, want, tol in zip((out, dq, dk, dv), refs, (O_TOL, G_TOL, G_TOL, G_TOL)):
+            # the results are fp16: the bound grows with them, as for the random shapes
+            assert _err(got[b:b + 1, :, h:h + 1], want) <= tol * max(1.0, want.abs().max().item())
+
+
 def test_strided_inputs_python_api():
     """flash_attn_func on views of a packed QKV tensor: gradients flow back into the packed tensor."""
     from flash_attn_v100 import flash_attn_func
