@@ -557,8 +557,9 @@ struct Strides {
 // and V(j-1) in iteration j, so one barrier per iteration is enough, and one
 // wave's MFMA stretch coincides with the other's VALU stretch.
 //
-// What bounds it is the power cap; 16 x 16 x 32 MFMAs take less of it (Geom16).  B2 H32 N4096 D128 causal 258 -> 244 us,
-// without a mask 473 -> 442 us (1.24 PFLOP/s), B1 H16 N16384 causal 1016 -> 950.
+// What bounds it is the power cap; 16 x 16 x 32 MFMAs take less of it (Geom16).  With them, one wait for the fragments of two
+// units and half of the waves copying late (below), against the kernel without the three, in turn: B2 H32 N4096 D128 causal 267
+// -> 251 us, without a mask 486 -> 450 us (1.22 PFLOP/s), B1 H16 N16384 causal 965 -> 895.
 // ---------------------------------------------------------------------------
 constexpr float kRescaleSum = 4096.f;
 constexpr int kFwdWaves = 8;
@@ -826,9 +827,9 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
         const char* Kl = k_ring + s0 * T::kBytes;
         const char* Vl = v_ring + s2 * T::kBytes;
         // The first group issues its half of the tile copies at the end of the iteration, the second at its start: all at
-        // once after the barrier they held every wave until the copy path had taken them.  B2 H32 N4096 without a mask
-        // 460 -> 446 us, causal 254 -> 250, B1 H16 N32768 causal 3642 -> 3509; other places 0.5-1 % slower than this, both
-        // at the end 0.5 % slower than before.
+        // once after the barrier they held every wave until the copy path had taken them.  This alone, 16 x 16 MFMAs and merged
+        // waits in place, on one card: B2 H32 N4096 causal 254 -> 250 us, without a mask 460 -> 446, B1 H16 N32768
+        // causal 3642 -> 3509; other places 0.5-1 % slower than this, both at the end 0.5 % slower than before.
         if (kFirst) {
           accumulate(Vl, j - 1);
           if (!kDrain) { scores(Kl, j); softmax(j); }
@@ -1877,8 +1878,9 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
 // LDS ring (B still needs tile j-1), dO tiles and the tile's lse2/delta rows
 // through 3-slot rings, all copied two tiles ahead.
 // What bounds it: the MFMAs and LDS reads that the two waves of a SIMD share, and with all CUs busy the power cap, which
-// is why those launches take the 16 x 16 x 32 MFMAs (B2 H40 N2048 causal: 212 -> 201 us; B2 H32 N4096 causal, dS stored:
-// 594 -> 572 us, 957 TFLOP/s of its four products; B3 H20 N1031: 99.6 -> 96 us).
+// is why those launches take the 16 x 16 x 32 MFMAs.  With them and the copies as they are placed now, against 32 x 32 ones, in
+// turn: B2 H40 N2048 causal 211 -> 203 us; B2 H32 N4096 causal, dS stored: 597 -> 574 us, 958 TFLOP/s of its four products; B3
+// H20 N1031: 98.7 -> 94.5 us.
 // ---------------------------------------------------------------------------
 constexpr int kKvPairs = 4;
 constexpr int kKvWaves = 2 * kKvPairs;
@@ -2035,8 +2037,10 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 
   // Two waves of a SIMD that both have MFMAs ready do not take turns: one runs, the other waits, and which one is up to the
   // priorities.  The products that an iteration begins with go first: those that would be held up meet the next ones too.
-  // (B2 H40 N2048 causal: 212 us without priorities, 206 with one for all, 201 with these, B3 H20 N1031: 102, 100, 96.  32 x
-  // 32 MFMAs: no difference.)
+  // That gained 5 % while role B copied before its second product (B2 H40 N2048 causal: 212 us without priorities, 201 with
+  // these); since it copies later, it is B3 H20 N1031 alone that gains, on three cards 94.4 -> 94.0, 96.8 -> 94.9, 98.0 -> 95.2,
+  // others lose up to 1.5 % (B2 H40 N2048 201.8, 202.0; 200.2, 201.6; 196.9, 198.2; B1 H12 N8192 without a mask 765, 777).
+  // Kernels of another stream do not run any slower for it: half_round_left.  32 x 32 MFMAs: no difference.
   auto priority = [&](auto b_tag, auto a_tag) __attribute__((always_inline)) {
     if constexpr (!WIDE) {
       if (role_b) __builtin_amdgcn_s_setprio(decltype(b_tag)::value);
@@ -2137,8 +2141,9 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 
   // Per iteration: wait for tile `it` (issued two iterations ago; the copies of tile
   // it+1 may still be in flight), one barrier, issue the copies of tile it+2.  Role A issues its half of them at the end
-  // of the iteration and role B earlier in it: all at once right after the barrier they held every wave until the copy
-  // path had taken them (B2 H32 N4096 causal: 608 -> 591 us; role A after its first GEMM: 627; role B later: 609).
+  // of the iteration and role B after the stores of dS: all at once right after the barrier they held every wave until the
+  // copy path had taken them (32 x 32 MFMAs, B2 H32 N4096 causal: 608 us, role A at the end 591, role A after its first GEMM
+  // 627; 16 x 16 ones, role B's places: below).
   auto step_wait = [&](int it) __attribute__((always_inline)) {
     if (it + 1 < n_it) {
       if (wave == 0) wait_vm<2 * kIPW + 2>();
@@ -2893,6 +2898,12 @@ bool bad_strides(const fused_mha_strides* st) {
 // Short blocks have nothing to gain (512 x 192: 21.6, 21.5; 61.1, 62.2.  256 x 320: 14.1, 14.3; 39.2, 39.4), nor has a fuller
 // last round (1024 x 112, 1.75: 41.2, 42.2; dK/dV 69.1, 70.1.  1024 x 192, 3: 65.5, 65.6; dK/dV 110, 118), nor more rounds
 // (1024 x 288, 4.5: 96.9, 98.4), nor a causal launch, where the blocks differ (1024 x 64 forward: 16.4, 18.2).
+// A wave keeps its priority to its end, also before waves of another stream on the same CU.  Those take no longer for it: us of
+// a 128 MiB elementwise kernel, of one of 4 MiB and of a 4096 cubed fp16 product on a second stream, without and with it:
+// beside the forward 8192 x 12 59.3, 58.3; 10.7, 10.7; 234, 228; beside its backward 57.7, 55.3; 10.3, 10.3; 220, 217; beside
+// the forward 1031 x 60 67.1, 65.7; 13.1, 13.1; 148, 149; beside the D = 128 backward, where the dK/dV pass has priorities of
+// its own, 2048 x 80 72.6, 73.0; 11.0, 11.0; 212, 211.  (The D = 64 backward itself gives way more: 960, 1057 beside the first
+// kernel; both streams' work together is done as early, 46.1, 45.4 ms.)
 bool half_round_left(long blocks, int n, int max_rounds) {
   if (n < 1024) return false;
   const long places = 2 * (long)persistent_grid(1 << 30), rounds = blocks / places, left = blocks % places;
