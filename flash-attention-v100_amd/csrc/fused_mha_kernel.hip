@@ -1978,11 +1978,10 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     }
   };
 
-  copy_tiles(0);
-  if (n_it > 1) copy_tiles(1);
-
   // resident rows of this wave: K for role A, V for role B; [feature step] of key k0w + i, or [feature step][cb] of keys
-  // k0w + 16 cb + i
+  // k0w + 16 cb + i.  They and the first tile are all that the loops need to start; the second tile is asked for when these
+  // are there, not waited for with them (B3 H20 N1031 step 193.9 -> 192.7 us, B2 H40 N2048 causal 434.6 -> 432.0, B2 H32 N4096
+  // causal 1129 -> 1125).
   h8 rf[G::kKSteps];
 #pragma unroll
   for (int cb = 0; cb < (WIDE ? 1 : 2); ++cb) {
@@ -1990,14 +1989,10 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     const half_t* rp = (role_b ? V + b * vs.b + (long)h * vs.h + (long)krow * vs.n
                                : K + b * ks.b + (long)h * ks.h + (long)krow * ks.n) + g * 8;
 #pragma unroll
-    for (int kk = 0; kk < (WIDE ? G::kKSteps : G16::kKS); ++kk) {
-      h8& r = rf[WIDE ? kk : 2 * kk + cb];
-      r = *reinterpret_cast<const h8*>(rp + kk * (WIDE ? 16 : 32));
-      // Role B works with -V: its first GEMM then gives delta - dP on top of
-      // accumulators loaded with delta, with no subtraction afterwards.
-      if (role_b) r = -r;
-    }
+    for (int kk = 0; kk < (WIDE ? G::kKSteps : G16::kKS); ++kk)
+      rf[WIDE ? kk : 2 * kk + cb] = *reinterpret_cast<const h8*>(rp + kk * (WIDE ? 16 : 32));
   }
+  copy_tiles(0);
 
   int r_off[2], c_off[2];
   if constexpr (WIDE) {
@@ -2161,7 +2156,16 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   half_t* const ds_lane = SPILL ? dS + ((long)bh * (np >> 7)) * np * 128 + (long)(k0w >> 6) * 8192 +
                                       ((k0w >> 5) & 1) * 4096 + lane * 8
                                 : nullptr;
-  wait_vm<0>();  // resident rows and the first copies: nothing is left for the compiler to wait on in the loops
+  wait_vm<0>();  // resident rows and the first tile: nothing is left for the compiler to wait on in the loops
+  // Role B works with -V: its first GEMM then gives delta - dP on top of accumulators loaded with delta, with no
+  // subtraction afterwards.
+  const unsigned sign = role_b ? 0x80008000u : 0u;
+#pragma unroll
+  for (h8& r : rf) {
+    r = __builtin_bit_cast(h8, __builtin_bit_cast(u4v, r) ^ u4v{sign, sign, sign, sign});
+    asm volatile("" : "+v"(r));  // here, not in the loop
+  }
+  if (n_it > 1) copy_tiles(1);
   if (!role_b) {
     for (int it = 0; it <= n_it; ++it) {
       step_wait(it);
