@@ -1634,12 +1634,13 @@ fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, c
 //
 // dQ pass.  The formulas are those of fmha_bwd_dq_kernel, and so are the results, bit for bit.
 // ---------------------------------------------------------------------------
-template <bool CAUSAL, bool STATS, bool ODD_FIRST>
-__global__ void __launch_bounds__(kPipeThreads, 2)
-fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                        const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
-                        Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
-                        half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+constexpr int kDqPipeLds = 2 * 3 * SwzTile<64>::kBytes;
+template <bool CAUSAL, bool STATS>
+__device__ __forceinline__ void
+bwd_dq_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                  const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
+                  Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
+                  half_t* __restrict__ dQ, int H, int N, float c, float scale, char* smem, int bh, int mblk) {
   constexpr int D = 64;
   using G = TileGeom<D>;
   using T = SwzTile<D>;
@@ -1648,16 +1649,11 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
   static_assert(kIPW == T::kNC, "a wave copies the 16 rows of one block row of a tile");
   constexpr int kSlots = 3;  // K tiles, then V tiles: the current one, the one before it, the one being copied
   constexpr int kVOff = kSlots * T::kBytes;
-  __shared__ __attribute__((aligned(1024))) char smem[2 * kSlots * T::kBytes];
+  static_assert(kDqPipeLds == 2 * kSlots * T::kBytes, "");
 
-  if (ODD_FIRST) odd_slots_first();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 31, hh = lane >> 5;
-  int bh, mb;
-  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
-                       N % kPipeBlockQ != 0, bh, mb);
-  const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O and dQ are dense
   const long head_off = ((long)b * N * H + h) * D;
@@ -1859,6 +1855,21 @@ fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__
 
   block_barrier();  // every wave is done with the rings: they become the staging tiles
   store_resident<D>(dQ + head_off, rs, q0w, N, dq, scale, lane, smem + wave * StageGeom<D>::kBytes);
+}
+
+template <bool CAUSAL, bool STATS, bool ODD_FIRST>
+__global__ void __launch_bounds__(kPipeThreads, 2)
+fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                        const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
+                        Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
+                        half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+  __shared__ __attribute__((aligned(1024))) char smem[kDqPipeLds];
+  if (ODD_FIRST) odd_slots_first();
+  int bh, mb;
+  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
+                       N % kPipeBlockQ != 0, bh, mb);
+  bwd_dq_pipe_block<CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
+                                   CAUSAL ? nmb - 1 - mb : mb);  // heavy blocks first
 }
 
 // ---------------------------------------------------------------------------
@@ -2267,12 +2278,16 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 // A 64-query tile is worked on in two halves of 32 queries; the accumulation into dV and dK of a half runs during the
 // next one, so Q and dO have three slots: the tile before, the current one, the one being copied.
 // ---------------------------------------------------------------------------
-template <bool CAUSAL, bool ODD_FIRST>
-__global__ void __launch_bounds__(kPipeThreads, 2)
-fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                          const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
-                          const float* __restrict__ delta, const float* __restrict__ lse2, half_t* __restrict__ dK,
-                          half_t* __restrict__ dV, int H, int N, int nnb, float c, float scale) {
+// STATS: the row statistics of every tile are formed here, from O, dO and LSE, a tile ahead; delta and lse2 are not read.
+constexpr int kDkDvPipeStBytes = 512;                     // 64 lse2 then 64 delta values
+constexpr int kDkDvPipeLds = 3 * (2 * SwzTile<64>::kBytes + kDkDvPipeStBytes);
+template <bool CAUSAL, bool STATS>
+__device__ __forceinline__ void
+bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                    const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                    const float* __restrict__ LSE, const float* __restrict__ delta, const float* __restrict__ lse2,
+                    half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, float c, float scale, char* smem, int bh,
+                    int nblk) {
   constexpr int D = 64;
   using G = TileGeom<D>;
   using T = SwzTile<D>;
@@ -2280,18 +2295,14 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
   constexpr int kIPW = T::kInstrs / kPipeWaves;
   constexpr int kSlots = 3;                               // the current tile, the one before it, the one being copied
   constexpr int kGOff = kSlots * T::kBytes, kStOff = 2 * kSlots * T::kBytes;
-  constexpr int kStBytes = 512;                           // 64 lse2 then 64 delta values
-  __shared__ __attribute__((aligned(1024))) char smem[kStOff + kSlots * kStBytes];
+  constexpr int kStBytes = kDkDvPipeStBytes;
+  static_assert(kDkDvPipeLds == kStOff + kSlots * kStBytes, "");
   static_assert(kPipeWaves * StageGeom<D>::kBytes <= kStOff, "the output staging tiles fit the rings");
 
-  if (ODD_FIRST) odd_slots_first();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 31, hh = lane >> 5;
-  int bh, nblk;
-  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nnb, nnb, CAUSAL,
-                       N % kPipeBlockKeys != 0, bh, nblk);
-  const int b = bh / H, h = bh - b * H;                   // causal: low key blocks are the heavy ones and come first
+  const int b = bh / H, h = bh - b * H;
   const int rs = H * D;                                   // dK and dV are dense
   const long head_off = ((long)b * N * H + h) * D;
   const int n0 = nblk * kPipeBlockKeys;
@@ -2313,7 +2324,7 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
   }
   const half_t* qp = Q + b * qs.b + (long)h * qs.h + (long)t_begin * kTile * qs.n - kBack / 2;  // next tile to copy
   const half_t* gp = dO + b * gs.b + (long)h * gs.h + (long)t_begin * kTile * gs.n - kBack / 2;
-  const float* const stat = (wave == 0 ? lse2 : delta) + ((long)b * H + h) * N;
+  const float* const stat = STATS ? nullptr : (wave == 0 ? lse2 : delta) + ((long)b * H + h) * N;
   const unsigned lds_w = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * (kIPW * 1024);
   auto copy_tile = [&](int t, int slot) __attribute__((always_inline)) {
     if (t == nt - 1) {
@@ -2324,9 +2335,52 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
     copy16_blocks<kIPW>(gp, g_goff, lds_w + kGOff + slot * T::kBytes);
     qp += (long)kTile * qs.n;
     gp += (long)kTile * gs.n;
-    if (wave < 2) copy4(stat, min(t * kTile + lane, N - 1) * 4, smem + kStOff + slot * kStBytes + wave * 256);
+    if (!STATS && wave < 2) copy4(stat, min(t * kTile + lane, N - 1) * 4, smem + kStOff + slot * kStBytes + wave * 256);
   };
   copy_tile(t_begin, 0);
+
+  // Statistics of a tile: eight lanes to a row, two rows each, in the order of fmha_bwd_delta_kernel.  The rows are asked for
+  // two tiles ahead, into registers, and summed up one tile ahead.
+  h8 st_o[2], st_g[2];
+  float st_l[2];
+  const half_t* op = O + head_off + (long)t_begin * kTile * rs;  // the next tile to ask for
+  const half_t* dop = dO + b * gs.b + (long)h * gs.h + (long)t_begin * kTile * gs.n;
+  const float* lp = LSE + ((long)b * H + h) * N + t_begin * kTile;
+  const int st_row = threadIdx.x >> 3, st_col = (threadIdx.x & 7) * 16;
+  int st_oo = st_row * rs * 2 + st_col, st_go = st_row * gs.n * 2 + st_col, st_lo = st_row * 4;
+  auto load_stats = [&](int t) __attribute__((always_inline)) {
+    const auto at = [](const void* base, int off) { return reinterpret_cast<const char*>(base) + (unsigned)off; };
+    const bool end = t == nt - 1;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const half_t *ou = op + 32 * u * (long)rs, *gu = dop + 32 * u * (long)gs.n;
+      const float* lu = lp + 32 * u;
+      if (end) {  // rows past the end re-read row N-1
+        const int row = min(32 * u + st_row, N - 1 - t * kTile);
+        ou = op, gu = dop, lu = lp;
+        st_oo = row * rs * 2 + st_col, st_go = row * gs.n * 2 + st_col, st_lo = row * 4;
+      }
+      st_o[u] = *reinterpret_cast<const h8*>(at(ou, st_oo));
+      st_g[u] = *reinterpret_cast<const h8*>(at(gu, st_go));
+      st_l[u] = *reinterpret_cast<const float*>(at(lu, st_lo));
+    }
+    op += kTile * (long)rs, dop += kTile * (long)gs.n, lp += kTile;
+  };
+  auto make_stats = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float a = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a = fmaf((float)st_o[u][e], (float)st_g[u][e], a);
+      a += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(a), (4 << 10) | 31));        // of the lane at ^ 4
+      a += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0x4E, 15, 15, true));       // ^ 2
+      a += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0xB1, 15, 15, true));       // ^ 1
+      float* const mine = reinterpret_cast<float*>(smem + kStOff + slot * kStBytes) + 32 * u + st_row;
+      mine[0] = st_l[u] * kLog2e;  // the same from all eight lanes
+      mine[64] = a;
+    }
+  };
+  if (STATS) load_stats(t_begin);
 
   // resident rows: K, and V negated, so that the dP product on top of delta gives delta - dP
   h8 kf[kKS], vf[kKS];
@@ -2444,12 +2498,22 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
     });
   };
 
+  if (STATS) {
+    make_stats(0);
+    if (t_begin + 1 < nt) load_stats(t_begin + 1);
+  }
   wait_vm<0>();
   int slot = 0, next_slot = 1, t = t_begin;
   auto top = [&]() __attribute__((always_inline)) {
     wait_vm<0>();
     block_barrier();
-    if (t + 1 < nt) copy_tile(t + 1, next_slot);
+    if (t + 1 < nt) {
+      copy_tile(t + 1, next_slot);
+      if (STATS) {
+        make_stats(next_slot);
+        if (t + 2 < nt) load_stats(t + 2);
+      }
+    }
   };
   auto next = [&]() __attribute__((always_inline)) {
     const int step = next_slot - slot;
@@ -2496,6 +2560,46 @@ fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict
   char* const stage = smem + wave * StageGeom<D>::kBytes;
   store_resident<D>(dV + head_off, rs, k0w, N, dv, 1.f, lane, stage);
   store_resident<D>(dK + head_off, rs, k0w, N, dk, scale, lane, stage);
+}
+
+template <bool CAUSAL, bool ODD_FIRST>
+__global__ void __launch_bounds__(kPipeThreads, 2)
+fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                          const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                          const float* __restrict__ delta, const float* __restrict__ lse2, half_t* __restrict__ dK,
+                          half_t* __restrict__ dV, int H, int N, int nnb, float c, float scale) {
+  __shared__ __attribute__((aligned(1024))) char smem[kDkDvPipeLds];
+  if (ODD_FIRST) odd_slots_first();
+  int bh, nblk;  // causal: low key blocks are the heavy ones and come first
+  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nnb, nnb, CAUSAL,
+                       N % kPipeBlockKeys != 0, bh, nblk);
+  bwd_dkdv_pipe_block<CAUSAL, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, H, N, c, scale, smem,
+                                     bh, nblk);
+}
+
+// Both passes in one launch: neither waits for the other, and a launch that leaves places empty (two blocks to a CU), or whose
+// last round does, takes the blocks of the other pass along.  STATS: every block makes the row statistics it needs, otherwise
+// they come from fmha_bwd_delta_kernel.  The blocks are those of the two kernels above, and so are the results, bit for bit.
+// Rules and both sides: fmha_passes_at_once, fmha_blocks_make_stats.
+static_assert(kPipeBlockQ == kPipeBlockKeys, "as many blocks of either pass");
+template <bool CAUSAL, bool STATS>
+__global__ void __launch_bounds__(kPipeThreads, 2)
+fmha_bwd_both_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                          const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
+                          Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
+                          half_t* __restrict__ dQ, half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, int nb, float c,
+                          float scale) {
+  constexpr int kLds = kDkDvPipeLds > kDqPipeLds ? kDkDvPipeLds : kDqPipeLds;
+  __shared__ __attribute__((aligned(1024))) char smem[kLds];
+  int bh, blk;
+  bool dq;
+  fmha_two_pass_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / (2 * nb), nb, CAUSAL,
+                      N % kPipeBlockQ != 0, bh, blk, dq);
+  if (dq)
+    bwd_dq_pipe_block<CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
+                                    CAUSAL ? nb - 1 - blk : blk);
+  else
+    bwd_dkdv_pipe_block<CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dK, dV, H, N, c, scale, smem, bh, blk);
 }
 
 // ---------------------------------------------------------------------------
@@ -3031,7 +3135,7 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   const size_t ds_bytes = slice_bytes(n) * (spill ? slices_at_once : 0) / (CAUSAL ? 2 : 1);
   const size_t touched = ds_bytes + 6 * (size_t)slices_at_once * n * D * sizeof(half_t);
   const int stream_ds = ds_bytes < (10u << 20) || touched > (256u << 20);
-  if ((passes & kPassDelta) && !dq_makes_stats) {
+  auto delta_pass = [&]() {
     const unsigned rows = (unsigned)slices * n;              // fewer than 2^32 / (D / 8): check_shape
     const unsigned most = (1u << 23) * delta_rows(D);        // a launch of fewer than 2^32 threads: fewer than twice the blocks
     for (unsigned first = 0; first < rows; first += most) {
@@ -3039,12 +3143,26 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
       const unsigned blocks = (end - first + delta_rows(D) - 1) / delta_rows(D);
       const unsigned per_slice = (unsigned)(n + delta_rows(D) - 1) / delta_rows(D);
       const unsigned chain = per_slice < blocks ? per_slice : blocks, chains = (blocks + chain - 1) / chain;
-      if (launch(fmha_bwd_delta_kernel<D>, chain * chains, 256, stream, (const half_t*)o, (const half_t*)d_o, gs,
-                 (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains) != hipSuccess)
-        return FUSED_MHA_ERR_LAUNCH;
+      const hipError_t rc = launch(fmha_bwd_delta_kernel<D>, chain * chains, 256, stream, (const half_t*)o, (const half_t*)d_o,
+                                   gs, (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains);
+      if (rc != hipSuccess) return rc;
+    }
+    return hipSuccess;
+  };
+  const float c = scale * kLog2e;
+  if constexpr (D == 64) {
+    const int nb = (n + kPipeBlockQ - 1) / kPipeBlockQ;
+    if ((passes & kPassAll) == kPassAll && fmha_passes_at_once((long)nb * batch * head, n, cus, CAUSAL)) {
+      const bool stats = fmha_blocks_make_stats(n, CAUSAL);
+      if (!stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
+      const hipError_t rc = launch(stats ? fmha_bwd_both_pipe_kernel<CAUSAL, true> : fmha_bwd_both_pipe_kernel<CAUSAL, false>,
+                                   2u * nb * batch * head, kPipeThreads, stream, (const half_t*)q, (const half_t*)k,
+                                   (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse,
+                                   delta, lse2, (half_t*)dq, (half_t*)dk, (half_t*)dv, head, n, nb, c, scale);
+      return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
     }
   }
-  const float c = scale * kLog2e;
+  if ((passes & kPassDelta) && !dq_makes_stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
   auto wide = [&]() { return fmha_wide_mfmas((long)key_blocks(n) * slices, cus, CAUSAL); };
   auto dq_pass = [&]() {
     if constexpr (D == 64) {

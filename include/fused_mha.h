@@ -179,7 +179,8 @@ int fused_mha_backward_noalloc(const void *query_ptr, const void *key_ptr, const
                                float scale, int causal, void *stream);
 
 /*
- * The three passes fused_mha_backward enqueues, one entry point each, so a
+ * The three passes of fused_mha_backward (which with d = 64 may put several
+ * into one launch, with the same results), one entry point each, so a
  * caller can time them separately or, with the minimum workspace, put the dQ
  * pass and the dK/dV pass (then independent of each other, both depend on the
  * delta pass) on different streams.  Same conventions and workspace as fused_mha_backward.  No

@@ -1,6 +1,9 @@
 """The D = 64 backward kernels at the sizes where they can go wrong: edges of 32-row waves, 64-row tiles and 128-row
 blocks, one tile and less, several tiles with a partial last one.  The D = 128 backward with a workspace that holds the
 dS of some of the slices."""
+import os
+import subprocess
+
 import pytest
 import torch
 
@@ -350,3 +353,79 @@ def test_row_statistics(B, H, N, D):
     want = lse.double() / torch.log(torch.tensor(2.0, dtype=torch.float64))
     assert ((ws[rows:2 * rows].view(B, H, N) - want).abs() <= 2.0 ** -22 * want.abs()).all()  # the constant's and the product's
     assert nbytes == 8 * rows and torch.isnan(ws[2 * rows:]).all()
+
+
+def test_blocks_of_two_passes_are_a_bijection(tmp_path):
+    """csrc/block_map.h, compiled for the host: every block of either pass once, whole slices on one XCD, heavy blocks first or
+    short ones last; and launches of both passes at once stay within the number of threads that a launch can have."""
+    src = tmp_path / "check.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (int slices = 1; slices <= 300; slices += (slices < 80 ? 1 : 7))
+    for (int nb : {1, 2, 3, 8, 33})
+      for (int mode = 0; mode < 3; ++mode) {
+        const bool heavy = mode == 0, short_last = mode == 1;
+        const int total = 2 * slices * nb;
+        std::vector<int> seen(total, 0), xcd(slices, -1);
+        int prev = 0, drops = 0;
+        for (int lin = 0; lin < total; ++lin) {
+          int s = -1, b = -1;
+          bool second = false;
+          fmha_two_pass_block(lin, slices, nb, heavy, short_last, s, b, second);
+          if (s < 0 || s >= slices || b < 0 || b >= nb || seen[2 * (s * nb + b) + second]++) {
+            printf("map %d %d %d %d\n", slices, nb, mode, lin);
+            return 1;
+          }
+          if (!short_last && s < (slices & ~7)) {
+            if (xcd[s] >= 0 && xcd[s] != (lin & 7)) { printf("xcd %d %d\n", slices, nb); return 1; }
+            xcd[s] = lin & 7;
+          }
+          if (short_last && (b == nb - 1) != (lin >= 2 * slices * (nb - 1))) { printf("short %d %d\n", slices, nb); return 1; }
+          drops += heavy && b < prev;
+          prev = b;
+        }
+        if (heavy && drops > slices / 64) { printf("order %d %d\n", slices, nb); return 1; }
+      }
+  for (int causal = 0; causal < 2; ++causal)
+    for (int n = 1; n <= 8192; n = n < 600 ? n + 1 : n * 2)
+      for (long slices = 1; slices < 1 << 23; slices += 1 + slices / 9) {
+        const long blocks = slices * ((n + 127) / 128);
+        if (fmha_passes_at_once(blocks, n, 256, causal) && 2 * blocks * 256 >= 1L << 32) { printf("threads %d\n", n); return 1; }
+      }
+  puts("ok");
+  return 0;
+}
+''')
+    exe = tmp_path / "check"
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,causal", [
+    # one launch, statistics made by the blocks: one tile, edges of tiles and blocks, two rounds and more
+    (1, 1, 1, False), (3, 5, 64, True), (2, 3, 65, False), (1, 3, 512, False), (2, 4, 511, True), (1, 5, 1024, True),
+    (16, 40, 129, False), (1, 70, 1000, True),
+    # one launch behind the kernel for the statistics
+    (1, 3, 513, False), (2, 2, 1025, True), (1, 5, 1031, False), (1, 3, 1536, True), (3, 20, 1031, False),
+    # two launches
+    (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False),
+])
+def test_backward_d64_in_one_launch(B, H, N, causal):
+    """Whatever goes in one launch, gradients and delta are those of the passes one by one, bit for bit, also with strides."""
+    D, lib = 64, abi.load()
+    scale = D ** -0.5
+    gen = torch.Generator(device="cuda").manual_seed(N + H)
+    packed = torch.randn(B, N, 4, H, D, device="cuda", dtype=torch.float16, generator=gen)
+    dense = [packed[:, :, i].contiguous() for i in range(4)]
+    out, lse = abi.forward(lib, *dense[:3], scale, causal)
+    want = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal, split=True)
+    got = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal)
+    strided = abi.backward_strided(lib, *(packed[:, :, i] for i in range(3)), out, packed[:, :, 3], lse, scale, causal)
+    for a, b, c in zip(got, want, strided):
+        assert torch.equal(a, b) and torch.equal(c, b)
+    assert torch.equal(got[3], want[3])
