@@ -199,24 +199,40 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
   second_pass = v & 1;
 }
 
-// Whether the D = 64 backward does both passes, `blocks` blocks of 128 rows each, in one launch of 2 * blocks.  With fewer
-// blocks than places (two to a CU) the passes one after the other leave most of the chip idle; with a few more, each has a
-// nearly empty last round of its own.  Full rounds have nothing to gain and pay for the statistics, which the dQ pass makes
-// on the side when it goes first.  us of two launches, and of one with the statistics made by the blocks or, behind "+", by a
-// kernel of their own first (fmha_blocks_make_stats), N x slices (rounds of one pass):
-//   Without a mask 128 x 32 12.9, 8.1; 128 x 512 (1) 22.7, 20.7; 128 x 1024 44.4, 34.6; 128 x 2048 (4) 75.4, 69.1; 256 x 64
-// 16.4, 10.4; 256 x 320 (1.25) 38.8, 33.6; 256 x 640 (2.5) 64.6, 60.4; 256 x 768 (3) 73.3, 77.0.  512 x 32 22.5, 14.9; 512 x
+// Whether the backward does both passes, `blocks` blocks of 128 rows each, in one launch of 2 * blocks.  With fewer blocks
+// than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few more,
+// each has a nearly empty last round of its own.  Full rounds have nothing to gain and pay for the statistics, which the D =
+// 64 dQ pass makes on the side when it goes first, or, at D = 128, for forming S and dP twice.  us of the launches one after
+// the other, and of one with the statistics made by the blocks or, behind "+", by a kernel of their own first
+// (fmha_blocks_make_stats), N x slices (rounds of one pass):
+// D = 64, without a mask.  128 x 32 12.9, 8.1; 128 x 512 (1) 22.7, 20.7; 128 x 1024 44.4, 34.6; 128 x 2048 (4) 75.4, 69.1; 256 x
+// 64 16.4, 10.4; 256 x 320 (1.25) 38.8, 33.6; 256 x 640 (2.5) 64.6, 60.4; 256 x 768 (3) 73.3, 77.0.  512 x 32 22.5, 14.9; 512 x
 // 64 (0.5) 24.0, 23.2; 512 x 96 (0.75) 37.3, 33.7; 512 x 112 39.3, 40.9; 512 x 128 (1) 42.0, 44.2; 512 x 136 54.8, 50.8; 512 x
 // 160 (1.25) 55.9, 53.5; 512 x 176 57.5, 60.8; 512 x 208 (1.63) 70.4, 70.3.  1024 x 16 36.3, + 24.4; 2048 x 4 62.1, + 37.4;
 // 4096 x 4 (0.25) 118, + 75.5; 4096 x 6 120, + 115; 2048 x 16 (0.5) 71.0, + 69.7; 2048 x 24 (0.75) 110, + 103; 2048 x 28 118, +
 // 126; 2048 x 32 (1) 128, + 134; 2048 x 40 (1.25) 173, + 168; 2048 x 44 179, + 190; 4096 x 26 (1.63) 440, + 424; 4096 x 28 449,
 // + 438; 4096 x 30 462, + 484; 4096 x 36 (2.25) 554, + 561.
-//   Causal 128 x 128 14.6, 9.0; 256 x 256 (1) 26.1, 26.0; 256 x 768 (3) 68.7, 59.9; 256 x 1024 (4) 84.9, 84.6; 512 x 64 24.5,
-// 17.8; 512 x 192 (1.5) 48.6, 46.0; 512 x 320 (2.5) 72.3, 70.0; 512 x 512 (4) 110, 117; 1024 x 32 (0.5) 37.9, 27.3; 1024 x 64
-// (1) 46.4, 43.4; 1024 x 104 74.4, 70.1; 1024 x 128 (2) 86.3, 85.7.  2048 x 12 63.2, + 41.0; 2048 x 32 (1) 79.9, + 74.3; 2048 x
+// D = 64, causal.  128 x 128 14.6, 9.0; 256 x 256 (1) 26.1, 26.0; 256 x 768 (3) 68.7, 59.9; 256 x 1024 (4) 84.9, 84.6; 512 x 64
+// 24.5, 17.8; 512 x 192 (1.5) 48.6, 46.0; 512 x 320 (2.5) 72.3, 70.0; 512 x 512 (4) 110, 117; 1024 x 32 (0.5) 37.9, 27.3; 1024 x
+// 64 (1) 46.4, 43.4; 1024 x 104 74.4, 70.1; 1024 x 128 (2) 86.3, 85.7.  2048 x 12 63.2, + 41.0; 2048 x 32 (1) 79.9, + 74.3; 2048 x
 // 60 136, + 135; 2048 x 64 (2) 141, + 145; 4096 x 16 (1) 148, + 134; 4096 x 30 242, + 240; 8192 x 4 (0.5) 220, + 155; 8192 x 8
 // (1) 283, + 256; 8192 x 15 464, + 459; 8192 x 32 (4) 946, + 963.
-FMHA_HOST_DEVICE bool fmha_passes_at_once(long blocks, int n, int cus, bool causal) {
+// D = 128, without a mask.  128 x 8 16.0, 9.4; 128 x 128 (0.5) 18.6, 11.7; 128 x 144 19.7, 20.1; 128 x 192 21.6, 20.4; 128 x 320
+// 37.3, 31.1; 128 x 512 (2) 46.8, 44.7; 256 x 16 20.0, 13.4; 256 x 64 (0.5) 23.1, 16.0; 256 x 72 24.0, 27.3; 256 x 128 (1) 29.6,
+// 31.6; 256 x 136 44.2, 42.4; 256 x 192 (1.5) 47.6, 46.7; 256 x 224 51.5, 58.5.  512 x 8 27.0, + 19.2; 512 x 32 (0.5) 31.7, +
+// 24.0; 512 x 36 32.2, + 39.2; 1024 x 8 42.1, + 30.9; 1024 x 16 (0.5) 46.0, + 37.5; 2048 x 8 (0.5) 75.4, + 64.5; 4096 x 2 124, +
+// 96.9; 4096 x 4 (0.5) 131, + 122; 4096 x 5 145, + 209; 8192 x 2 (0.5) 280, + 235; 512 x 68 (1.06) 61.9, + 61.8; 2048 x 18 166, +
+// 176.
+// D = 128, causal.  128 x 32 17.5, 10.4; 128 x 192 22.4, 21.2; 256 x 64 (0.5) 23.3, 15.3; 256 x 128 (1) 28.9, 26.5; 256 x 192
+// (1.5) 44.5, 39.2; 256 x 224 46.0, 48.2.  512 x 32 (0.5) 31.0, + 21.7; 512 x 64 (1) 37.7, + 34.2; 512 x 68 41.5, + 43.2; 1024 x 24
+// 47.8, + 38.0; 1024 x 32 (1) 54.0, + 48.1; 2048 x 8 (0.5) 71.3, + 54.2; 2048 x 16 (1) 84.9, + 76.0; 2048 x 18 91.6, + 89.2; 2048 x
+// 20 91.1, + 98.1; 4096 x 8 (1) 153, + 133; 4096 x 10 159, + 169; 8192 x 4 (1) 303, + 267; 8192 x 5 315, + 318.
+FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bool causal) {
+  if (d == 128) {
+    if (n <= 128) return blocks <= 2L * cus;
+    if (causal) return 2 * blocks <= (n <= 256 ? 3L : 2L) * cus;
+    return 2 * blocks <= cus || (n <= 256 && blocks > cus && 2 * blocks <= 3L * cus);
+  }
   const long places = 2L * cus;
   if (causal) return n <= 512 ? blocks * n <= places * (2L * n + 256) : blocks < 2 * places;
   if (n <= 256) return blocks * n <= places * (n + 384L);  // the start and the end of a launch are a good part of it
@@ -224,12 +240,16 @@ FMHA_HOST_DEVICE bool fmha_passes_at_once(long blocks, int n, int cus, bool caus
   return 4 * blocks <= 3 * places || (blocks > places && blocks < 2 * places && left > 0 && 2 * left <= places);
 }
 
-// Whether the blocks of such a launch make the row statistics themselves, which adds a tenth to the tiles of the dK/dV
-// blocks, or a kernel before it does, which takes 2 to 5 us and more where there are many rows.  Figures as above, blocks,
-// then kernel: without a mask 256 x 64 10.4, 12.1; 512 x 32 14.9, 15.9; 512 x 160 53.5, 53.2; 1024 x 16 24.9, 24.4; 1024 x 48
-// 59.8, 56.9; 4096 x 4 85.3, 75.5.  Causal 512 x 64 17.8, 18.9; 1024 x 16 24.1, 23.5; 1024 x 64 43.4, 45.2; 1024 x 104 70.1, 73.5;
-// 2048 x 12 44.5, 41.0; 8192 x 4 172, 155.
-FMHA_HOST_DEVICE bool fmha_blocks_make_stats(int n, bool causal) { return n <= (causal ? 1024 : 512); }
+// Whether the blocks of such a launch make the row statistics themselves, which adds a tenth and more to the tiles of the
+// dK/dV blocks, or a kernel before it does, which takes 2 to 5 us and more where there are many rows.  Figures as above,
+// blocks, then kernel.  D = 64: 256 x 64 10.4, 12.1; 512 x 32 14.9, 15.9; 512 x 160 53.5, 53.2; 1024 x 16 24.9, 24.4; 1024 x 48
+// 59.8, 56.9; 4096 x 4 85.3, 75.5; causal 512 x 64 17.8, 18.9; 1024 x 16 24.1, 23.5; 1024 x 64 43.4, 45.2; 1024 x 104 70.1, 73.5;
+// 2048 x 12 44.5, 41.0; 8192 x 4 172, 155.  D = 128: 128 x 32 9.7, 10.9; 256 x 16 13.4, 13.8; 256 x 64 16.0, 17.4; 512 x 8 21.0,
+// 19.2; 512 x 32 24.1, 24.0; 1024 x 8 36.5, 30.9; causal 256 x 64 15.3, 16.5; 512 x 8 21.3, 20.0; 512 x 40 24.6, 25.0; 1024 x 16
+// 37.0, 32.4.
+FMHA_HOST_DEVICE bool fmha_blocks_make_stats(int d, int n, bool causal) {
+  return n <= (d == 128 ? 384 : causal ? 1024 : 512);
+}
 
 // Row statistics: blocks of consecutive rows, numbered through all slices, taken from `chains` runs of `chain` blocks by
 // turns.  With a run about as long as a slice, work groups that follow each other read the same positions of different heads,

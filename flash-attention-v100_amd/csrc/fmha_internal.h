@@ -16,5 +16,9 @@ int fmha_forward_without_lse(const void* query_ptr, const fused_mha_strides* que
 // minimum) with which the backward is fastest.  0 for an invalid shape.
 size_t fmha_backward_workspace_within(int batch, int head, int n, int d, size_t room);
 
+// fused_mha_backward_workspace_bytes for one backward: the minimum where that does both passes in one launch, which needs no
+// room for dS.
+size_t fmha_backward_workspace_for(int batch, int head, int n, int d, int causal);
+
 }  // extern "C"
 #endif  // FMHA_INTERNAL_H_

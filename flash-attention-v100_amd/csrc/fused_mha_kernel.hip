@@ -535,6 +535,59 @@ struct Strides {
   int n, h;
 };
 
+// Row statistics of 64-row tiles for a work group of 4 * D threads: D / 8 lanes to a row, two rows each, in the order of
+// fmha_bwd_delta_kernel.  load asks for the rows of a tile, one tile after the other; make sums up what was asked for.
+template <int D>
+struct TileStats {
+  static constexpr int kLanes = D / 8;
+  h8 o[2], g[2];
+  float l[2];
+  const half_t *op, *gp;  // the next tile to ask for
+  const float* lp;
+  int o_stride, g_stride, row, col, o_off, g_off, l_off;
+  __device__ __forceinline__ TileStats(const half_t* O, const half_t* dO, const float* LSE, int rs, int gs_n, int tile) {
+    op = O + (long)tile * kTile * rs, gp = dO + (long)tile * kTile * gs_n, lp = LSE + tile * kTile;
+    o_stride = rs, g_stride = gs_n;
+    row = threadIdx.x / kLanes, col = threadIdx.x % kLanes * 16;
+    o_off = row * rs * 2 + col, g_off = row * gs_n * 2 + col, l_off = row * 4;
+  }
+  __device__ __forceinline__ void load(int last_row) {  // last_row: of the tile, N - 1 if it holds that; 63 or more if not
+    const auto at = [](const void* base, int off) { return reinterpret_cast<const char*>(base) + (unsigned)off; };
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const half_t *ou = op + 32 * u * (long)o_stride, *gu = gp + 32 * u * (long)g_stride;
+      const float* lu = lp + 32 * u;
+      if (last_row < kTile - 1) {  // rows past the end re-read row N-1
+        const int r = min(32 * u + row, last_row);
+        ou = op, gu = gp, lu = lp;
+        o_off = r * o_stride * 2 + col, g_off = r * g_stride * 2 + col, l_off = r * 4;
+      }
+      o[u] = *reinterpret_cast<const h8*>(at(ou, o_off));
+      g[u] = *reinterpret_cast<const h8*>(at(gu, g_off));
+      l[u] = *reinterpret_cast<const float*>(at(lu, l_off));
+    }
+    op += kTile * (long)o_stride, gp += kTile * (long)g_stride, lp += kTile;
+  }
+  __device__ __forceinline__ void make(char* slot) const {  // 64 lse * log2(e), then 64 delta values
+    const auto dpp = [](float x, auto ctrl) __attribute__((always_inline)) {
+      return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), decltype(ctrl)::value, 15, 15, true));
+    };
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float a = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a = fmaf((float)o[u][e], (float)g[u][e], a);
+      if (kLanes == 16) a += dpp(a, IntTag<0x128>{});                                       // of the lane at ^ 8 (of 16)
+      a += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(a), (4 << 10) | 31));  // ^ 4
+      a += dpp(a, IntTag<0x4E>{});                                                          // ^ 2
+      a += dpp(a, IntTag<0xB1>{});                                                          // ^ 1
+      float* const mine = reinterpret_cast<float*>(slot) + 32 * u + row;
+      mine[0] = l[u] * kLog2e;  // the same from all lanes of the row
+      mine[kTile] = a;
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Forward for D = 128 where blocks of 256 queries share out well over the CUs
 // (rule: fmha_persistent_forward_pays).  Block = 8 waves = 256 queries, wave = 32 queries; K/V
@@ -1376,18 +1429,20 @@ constexpr int kDqBlockQ = kDqPairs * kResident;
 // them and stores them in the workspace for the dK/dV pass (which must then be
 // launched after this one); fmha_bwd_delta_kernel is not needed in that case.
 // Otherwise delta is read from the workspace.
+template <int D>
+constexpr int dq_lds() { return 7 * SwzTile<D>::kBytes + 2 * kDqPairs * 4096; }
 template <int D, bool CAUSAL, bool STATS>
-__global__ void __launch_bounds__(kDqThreads, 1)
-fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                   const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
-                   Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
-                   half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+__device__ __forceinline__ void
+bwd_dq_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+             const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+             const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ, int H,
+             int N, float c, float scale, char* smem, int bh, int mblk) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kDqWaves;  // copies per wave per tile, per tensor
   // K ring (4), V ring (3), then two buffers of per pair a 64x32 fp16 block (4 KiB) of P^T
   constexpr int kPBytes = kDqPairs * 4096;
-  __shared__ __attribute__((aligned(1024))) char smem[7 * T::kBytes + 2 * kPBytes];
+  static_assert(dq_lds<D>() == 7 * T::kBytes + 2 * kPBytes, "");
   char* const k_ring = smem;
   char* const v_ring = smem + 4 * T::kBytes;
   char* const p_xchg = smem + 7 * T::kBytes;
@@ -1397,9 +1452,6 @@ fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, c
   const int pair = wave & (kDqPairs - 1);
   const bool role_b = wave >= kDqPairs;
   const int i = lane & 31, hh = lane >> 5;
-  int bh, mb;
-  slice_and_block(nmb, bh, mb);
-  const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O and dQ are dense
   const long head_off = ((long)b * N * H + h) * D;
@@ -1615,6 +1667,19 @@ fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, c
   static_assert(kDqPairs * StageGeom<D>::kBytes <= 7 * T::kBytes, "the output staging tiles fit the rings");
   block_barrier();  // every wave is done with the rings: they become the staging tiles
   if (role_b) store_resident<D>(dQ + head_off, rs, q0w, N, dq, scale, lane, smem + pair * StageGeom<D>::kBytes);
+}
+
+template <int D, bool CAUSAL, bool STATS>
+__global__ void __launch_bounds__(kDqThreads, 1)
+fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                   const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
+                   Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
+                   half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+  __shared__ __attribute__((aligned(1024))) char smem[dq_lds<D>()];
+  int bh, mb;
+  slice_and_block(nmb, bh, mb);
+  bwd_dq_block<D, CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
+                                 CAUSAL ? nmb - 1 - mb : mb);  // heavy blocks first
 }
 
 // ---------------------------------------------------------------------------
@@ -1913,13 +1978,17 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // query tile) pairs above the diagonal are not written (and not read) under causal masking.
 // KEEP: without the non-temporal hint on those stores (rule: launch_backward).
 // WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: launch_backward).
-template <int D, bool CAUSAL, bool SPILL, bool KEEP, bool WIDE>
-__global__ void __launch_bounds__(kKvThreads, 1)
-fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                     const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
-                     const float* __restrict__ delta, const float* __restrict__ lse2,
-                     half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
-                     int nnb, int slice0, float c, float scale) {
+// STATS: the row statistics of every tile are formed here, from O, dO and LSE, a tile ahead; delta and lse2 are not read.
+constexpr int kKvStBytes = 1024;
+template <int D>
+constexpr int dkdv_lds() { return 7 * SwzTile<D>::kBytes + 3 * kKvStBytes + 2 * kKvPairs * 2 * 2048; }
+template <int D, bool CAUSAL, bool SPILL, bool KEEP, bool WIDE, bool STATS>
+__device__ __forceinline__ void
+bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+               const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+               const float* __restrict__ LSE, const float* __restrict__ delta, const float* __restrict__ lse2,
+               half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N, int slice0,
+               float c, float scale, char* smem, int bh, int nblk) {
   using G = TileGeom<D>;
   using G16 = Geom16<D>;
   using T = SwzTile<D>;
@@ -1927,9 +1996,9 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   // Q ring (4), dO ring (3), per stats slot 64 lse2 then 64 delta values (1 KiB, half
   // unused), and the P exchange: 2 buffers x per pair the four fragments of P, 16 bytes per lane each, in separate 1 KiB
   // planes so that the accesses are free of bank conflicts.
-  constexpr int kStBytes = 1024;
+  constexpr int kStBytes = kKvStBytes;
   constexpr int kPBytes = kKvPairs * 2 * 2048;
-  __shared__ __attribute__((aligned(1024))) char smem[7 * T::kBytes + 3 * kStBytes + 2 * kPBytes];
+  static_assert(dkdv_lds<D>() == 7 * T::kBytes + 3 * kStBytes + 2 * kPBytes, "");
   char* const q_ring = smem;
   char* const g_ring = smem + 4 * T::kBytes;
   char* const st_ring = smem + 7 * T::kBytes;
@@ -1941,16 +2010,13 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   const bool role_b = wave >= kKvPairs;
   const int i = WIDE ? lane & 31 : lane & 15;        // resident position of this lane's columns, and
   const int g = WIDE ? lane >> 5 : lane >> 4;        // which streamed rows it has
-  int bh, nblk;
-  // causal: low key blocks are the heavy ones and come first
-  fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kKvBlockKeys != 0, bh, nblk);
   const int b = (slice0 + bh) / H, h = slice0 + bh - b * H;  // bh: the slice in this launch and in dS
   const int rs = H * D;  // dK and dV are dense
   const long head_off = ((long)b * N * H + h) * D;
   const half_t* Qb = Q + b * qs.b + (long)h * qs.h;
   const half_t* dOb = dO + b * gs.b + (long)h * gs.h;
-  const float* delta_b = delta + ((long)b * H + h) * N;
-  const float* lse2_b = lse2 + ((long)b * H + h) * N;
+  const float* delta_b = STATS ? nullptr : delta + ((long)b * H + h) * N;
+  const float* lse2_b = STATS ? nullptr : lse2 + ((long)b * H + h) * N;
 
   const int n0 = nblk * kKvBlockKeys;
   const int k0w = n0 + pair * kResident;
@@ -1982,7 +2048,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       copy16_blocks<kIPW>(qp, c_qgoff - back * qs.n * 2, qdst);
       copy16_blocks<kIPW>(gp, c_ggoff - back * gs.n * 2, gdst);
     }
-    if (wave == 0) {  // lane l: lse2 and delta of row row0 + l (rows past the end re-read row N-1)
+    if (!STATS && wave == 0) {  // lane l: lse2 and delta of row row0 + l (rows past the end re-read row N-1)
       const int at = min(row0 + lane, N - 1) * 4;
       copy4(lse2_b, at, st_ring + (it % 3) * kStBytes);
       copy4(delta_b, at, st_ring + (it % 3) * kStBytes + 256);
@@ -2004,6 +2070,14 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
       rf[WIDE ? kk : 2 * kk + cb] = *reinterpret_cast<const h8*>(rp + kk * (WIDE ? 16 : 32));
   }
   copy_tiles(0);
+
+  // statistics: the rows are asked for two tiles ahead, into registers, and summed up one tile ahead
+  TileStats<D> stats(O + head_off, dOb, LSE + ((long)b * H + h) * N, rs, gs.n, t_begin);
+  auto stats_ahead = [&](int it) __attribute__((always_inline)) {  // of tile it + 1; those of tile it + 2 are asked for
+    if (it + 1 < n_it) stats.make(st_ring + (it + 1) % 3 * kStBytes);
+    if (it + 2 < n_it) stats.load(N - 1 - (t_begin + it + 2) * kTile);
+  };
+  if (STATS) stats.load(N - 1 - t_begin * kTile);
 
   int r_off[2], c_off[2];
   if constexpr (WIDE) {
@@ -2151,13 +2225,14 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   // copy path had taken them (32 x 32 MFMAs, B2 H32 N4096 causal: 608 us, role A at the end 591, role A after its first GEMM
   // 627; 16 x 16 ones, role B's places: below).
   auto step_wait = [&](int it) __attribute__((always_inline)) {
-    if (it + 1 < n_it) {
+    if (!STATS && it + 1 < n_it) {
       if (wave == 0) wait_vm<2 * kIPW + 2>();
       else wait_vm<2 * kIPW>();
     } else {
       wait_vm<0>();
     }
     block_barrier();
+    if (STATS) stats_ahead(it);
   };
   auto step_copy = [&](int it) __attribute__((always_inline)) {
     if (it + 2 < n_it) copy_tiles(it + 2);
@@ -2167,6 +2242,7 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   half_t* const ds_lane = SPILL ? dS + ((long)bh * (np >> 7)) * np * 128 + (long)(k0w >> 6) * 8192 +
                                       ((k0w >> 5) & 1) * 4096 + lane * 8
                                 : nullptr;
+  if (STATS) stats_ahead(-1);
   wait_vm<0>();  // resident rows and the first tile: nothing is left for the compiler to wait on in the loops
   // Role B works with -V: its first GEMM then gives delta - dP on top of accumulators loaded with delta, with no
   // subtraction afterwards.
@@ -2273,6 +2349,46 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   }
 }
 
+template <int D, bool CAUSAL, bool SPILL, bool KEEP, bool WIDE>
+__global__ void __launch_bounds__(kKvThreads, 1)
+fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                     const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                     const float* __restrict__ delta, const float* __restrict__ lse2,
+                     half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
+                     int nnb, int slice0, float c, float scale) {
+  __shared__ __attribute__((aligned(1024))) char smem[dkdv_lds<D>()];
+  int bh, nblk;
+  // causal: low key blocks are the heavy ones and come first
+  fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kKvBlockKeys != 0, bh, nblk);
+  bwd_dkdv_block<D, CAUSAL, SPILL, KEEP, WIDE, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
+                                                      H, N, slice0, c, scale, smem, bh, nblk);
+}
+
+// The dK/dV pass and the dQ pass that recomputes S and dP in one launch, for problems of so few blocks that neither fills the
+// chip: dS is not stored.  STATS as in fmha_bwd_both_pipe_kernel.  The blocks are those of the kernels for either pass, and so
+// are the results, bit for bit; those over dS give them too.  Rules and both sides: fmha_passes_at_once,
+// fmha_blocks_make_stats.
+static_assert(kDqBlockQ == kKvBlockKeys && kDqThreads == kKvThreads, "as many blocks of either pass, of the same size");
+template <bool CAUSAL, bool STATS>
+__global__ void __launch_bounds__(kKvThreads, 1)
+fmha_bwd_both_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                     const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                     const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ,
+                     half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, int nb, float c, float scale) {
+  constexpr int D = 128;
+  constexpr int kLds = dkdv_lds<D>() > dq_lds<D>() ? dkdv_lds<D>() : dq_lds<D>();
+  __shared__ __attribute__((aligned(1024))) char smem[kLds];
+  int bh, blk;
+  bool dq;
+  fmha_two_pass_block(blockIdx.x, gridDim.x / (2 * nb), nb, CAUSAL, N % kKvBlockKeys != 0, bh, blk, dq);
+  if (dq)
+    bwd_dq_block<D, CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
+                                   CAUSAL ? nb - 1 - blk : blk);
+  else
+    bwd_dkdv_block<D, CAUSAL, false, false, true, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dK, dV, nullptr, 0, H,
+                                                         N, 0, c, scale, smem, bh, blk);
+}
+
 // ---------------------------------------------------------------------------
 // Backward, dK/dV pass for D = 64 (see fmha_bwd_dq_pipe_kernel).  Formulas and results are those of fmha_bwd_dkdv_kernel.
 // A 64-query tile is worked on in two halves of 32 queries; the accumulation into dV and dK of a half runs during the
@@ -2339,47 +2455,10 @@ bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, 
   };
   copy_tile(t_begin, 0);
 
-  // Statistics of a tile: eight lanes to a row, two rows each, in the order of fmha_bwd_delta_kernel.  The rows are asked for
-  // two tiles ahead, into registers, and summed up one tile ahead.
-  h8 st_o[2], st_g[2];
-  float st_l[2];
-  const half_t* op = O + head_off + (long)t_begin * kTile * rs;  // the next tile to ask for
-  const half_t* dop = dO + b * gs.b + (long)h * gs.h + (long)t_begin * kTile * gs.n;
-  const float* lp = LSE + ((long)b * H + h) * N + t_begin * kTile;
-  const int st_row = threadIdx.x >> 3, st_col = (threadIdx.x & 7) * 16;
-  int st_oo = st_row * rs * 2 + st_col, st_go = st_row * gs.n * 2 + st_col, st_lo = st_row * 4;
-  auto load_stats = [&](int t) __attribute__((always_inline)) {
-    const auto at = [](const void* base, int off) { return reinterpret_cast<const char*>(base) + (unsigned)off; };
-    const bool end = t == nt - 1;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const half_t *ou = op + 32 * u * (long)rs, *gu = dop + 32 * u * (long)gs.n;
-      const float* lu = lp + 32 * u;
-      if (end) {  // rows past the end re-read row N-1
-        const int row = min(32 * u + st_row, N - 1 - t * kTile);
-        ou = op, gu = dop, lu = lp;
-        st_oo = row * rs * 2 + st_col, st_go = row * gs.n * 2 + st_col, st_lo = row * 4;
-      }
-      st_o[u] = *reinterpret_cast<const h8*>(at(ou, st_oo));
-      st_g[u] = *reinterpret_cast<const h8*>(at(gu, st_go));
-      st_l[u] = *reinterpret_cast<const float*>(at(lu, st_lo));
-    }
-    op += kTile * (long)rs, dop += kTile * (long)gs.n, lp += kTile;
-  };
-  auto make_stats = [&](int slot) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      float a = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) a = fmaf((float)st_o[u][e], (float)st_g[u][e], a);
-      a += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(a), (4 << 10) | 31));        // of the lane at ^ 4
-      a += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0x4E, 15, 15, true));       // ^ 2
-      a += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0xB1, 15, 15, true));       // ^ 1
-      float* const mine = reinterpret_cast<float*>(smem + kStOff + slot * kStBytes) + 32 * u + st_row;
-      mine[0] = st_l[u] * kLog2e;  // the same from all eight lanes
-      mine[64] = a;
-    }
-  };
+  // statistics: the rows are asked for two tiles ahead, into registers, and summed up one tile ahead
+  TileStats<D> stats(O + head_off, dO + b * gs.b + (long)h * gs.h, LSE + ((long)b * H + h) * N, rs, gs.n, t_begin);
+  auto load_stats = [&](int t) __attribute__((always_inline)) { stats.load(N - 1 - t * kTile); };
+  auto make_stats = [&](int slot) __attribute__((always_inline)) { stats.make(smem + kStOff + slot * kStBytes); };
   if (STATS) load_stats(t_begin);
 
   // resident rows: K, and V negated, so that the dP product on top of delta gives delta - dP
@@ -3150,17 +3229,24 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
     return hipSuccess;
   };
   const float c = scale * kLog2e;
-  if constexpr (D == 64) {
-    const int nb = (n + kPipeBlockQ - 1) / kPipeBlockQ;
-    if ((passes & kPassAll) == kPassAll && fmha_passes_at_once((long)nb * batch * head, n, cus, CAUSAL)) {
-      const bool stats = fmha_blocks_make_stats(n, CAUSAL);
-      if (!stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
-      const hipError_t rc = launch(stats ? fmha_bwd_both_pipe_kernel<CAUSAL, true> : fmha_bwd_both_pipe_kernel<CAUSAL, false>,
-                                   2u * nb * batch * head, kPipeThreads, stream, (const half_t*)q, (const half_t*)k,
-                                   (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse,
-                                   delta, lse2, (half_t*)dq, (half_t*)dk, (half_t*)dv, head, n, nb, c, scale);
-      return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
+  const int nb = (n + 127) / 128;
+  if ((passes & kPassAll) == kPassAll && fmha_passes_at_once(D, (long)nb * slices, n, cus, CAUSAL)) {
+    const bool stats = fmha_blocks_make_stats(D, n, CAUSAL);
+    if (!stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
+    auto both = [&](auto kernel, int threads) {
+      return launch(kernel, 2u * nb * slices, threads, stream, (const half_t*)q, (const half_t*)k, (const half_t*)v,
+                    (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2, (half_t*)dq, (half_t*)dk,
+                    (half_t*)dv, head, n, nb, c, scale);
+    };
+    hipError_t rc;
+    if constexpr (D == 64) {
+      static_assert(kPipeBlockQ == 128 && kPipeBlockKeys == 128, "");
+      rc = both(stats ? fmha_bwd_both_pipe_kernel<CAUSAL, true> : fmha_bwd_both_pipe_kernel<CAUSAL, false>, kPipeThreads);
+    } else {
+      static_assert(kDqBlockQ == 128 && kKvBlockKeys == 128, "");
+      rc = both(stats ? fmha_bwd_both_kernel<CAUSAL, true> : fmha_bwd_both_kernel<CAUSAL, false>, kKvThreads);
     }
+    return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
   }
   if ((passes & kPassDelta) && !dq_makes_stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
   auto wide = [&]() { return fmha_wide_mfmas((long)key_blocks(n) * slices, cus, CAUSAL); };
@@ -3340,6 +3426,13 @@ size_t fused_mha_backward_workspace_bytes(int batch, int head, int n, int d) {
 size_t fmha_backward_workspace_within(int batch, int head, int n, int d, size_t room) {
   if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK) return 0;
   return best_workspace(batch, head, n, d, room);
+}
+
+size_t fmha_backward_workspace_for(int batch, int head, int n, int d, int causal) {
+  if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK) return 0;
+  const int cus = (int)persistent_grid(1 << 30);
+  if (fmha_passes_at_once(d, (long)key_blocks(n) * batch * head, n, cus, causal != 0)) return stats_bytes(batch, head, n);
+  return best_workspace(batch, head, n, d, SIZE_MAX);
 }
 
 int fused_mha_backward(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,

@@ -389,11 +389,11 @@ int main() {
         }
         if (heavy && drops > slices / 64) { printf("order %d %d\n", slices, nb); return 1; }
       }
-  for (int causal = 0; causal < 2; ++causal)
+  for (int causal = 0; causal < 4; ++causal)
     for (int n = 1; n <= 8192; n = n < 600 ? n + 1 : n * 2)
       for (long slices = 1; slices < 1 << 23; slices += 1 + slices / 9) {
         const long blocks = slices * ((n + 127) / 128);
-        if (fmha_passes_at_once(blocks, n, 256, causal) && 2 * blocks * 256 >= 1L << 32) { printf("threads %d\n", n); return 1; }
+        if (fmha_passes_at_once(causal & 2 ? 64 : 128, blocks, n, 256, causal & 1) && 2 * blocks * 512 >= 1L << 32) { printf("threads %d\n", n); return 1; }
       }
   puts("ok");
   return 0;
@@ -406,7 +406,7 @@ int main() {
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,N,causal", [
+@pytest.mark.parametrize("D,B,H,N,causal", [(64, *case) for case in [
     # one launch, statistics made by the blocks: one tile, edges of tiles and blocks, two rounds and more
     (1, 1, 1, False), (3, 5, 64, True), (2, 3, 65, False), (1, 3, 512, False), (2, 4, 511, True), (1, 5, 1024, True),
     (16, 40, 129, False), (1, 70, 1000, True),
@@ -414,10 +414,16 @@ int main() {
     (1, 3, 513, False), (2, 2, 1025, True), (1, 5, 1031, False), (1, 3, 1536, True), (3, 20, 1031, False),
     # two launches
     (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False),
-])
-def test_backward_d64_in_one_launch(B, H, N, causal):
-    """Whatever goes in one launch, gradients and delta are those of the passes one by one, bit for bit, also with strides."""
-    D, lib = 64, abi.load()
+]] + [(128, *case) for case in [
+    (1, 1, 1, True), (3, 5, 33, False), (2, 3, 64, True), (2, 3, 65, False), (1, 100, 128, True), (5, 100, 77, False),
+    (2, 30, 255, False), (1, 70, 256, True), (1, 140, 256, False), (3, 7, 384, True), (1, 9, 321, False),
+    (1, 3, 385, False), (2, 2, 1031, True), (1, 9, 1031, False), (1, 30, 1000, True), (1, 2, 2049, False),
+    (1, 140, 250, False), (1, 70, 250, False), (1, 70, 400, True), (1, 20, 1031, False),
+]])
+def test_backward_in_one_launch(D, B, H, N, causal):
+    """Whatever goes in one launch, gradients and delta are those of the passes one by one, bit for bit, also with strides
+    and with the least workspace (at D = 128 the passes one by one store dS, the launch forms it twice)."""
+    lib = abi.load()
     scale = D ** -0.5
     gen = torch.Generator(device="cuda").manual_seed(N + H)
     packed = torch.randn(B, N, 4, H, D, device="cuda", dtype=torch.float16, generator=gen)
@@ -426,6 +432,7 @@ def test_backward_d64_in_one_launch(B, H, N, causal):
     want = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal, split=True)
     got = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal)
     strided = abi.backward_strided(lib, *(packed[:, :, i] for i in range(3)), out, packed[:, :, 3], lse, scale, causal)
-    for a, b, c in zip(got, want, strided):
-        assert torch.equal(a, b) and torch.equal(c, b)
-    assert torch.equal(got[3], want[3])
+    least = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal, min_workspace=True)
+    for a, b, c, d in zip(got, want, strided, least):
+        assert torch.equal(a, b) and torch.equal(c, b) and torch.equal(d, b)
+    assert torch.equal(got[3], want[3]) and torch.equal(least[3], want[3])
