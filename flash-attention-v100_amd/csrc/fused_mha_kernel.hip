@@ -2019,7 +2019,15 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   const float* lse2_b = STATS ? nullptr : lse2 + ((long)b * H + h) * N;
 
   const int n0 = nblk * kKvBlockKeys;
-  const int k0w = n0 + pair * kResident;
+  // In a last block of at most 32 keys all four pairs own those: each takes one half of the rows of the even or of the odd
+  // tiles, and their sums are put together at the end.  One pair alone took 23 us for such a block where four take 40 for a
+  // whole one (N = 1031, dS stored), its two waves on one SIMD and the others idle; now 17 us.  dK/dV pass, us, before and after:
+  // 1031 x 60 100.8, 88.0; x 32 63.5, 57.3; x 64 100.9, 93; 2053 x 60 295, 290; 4097 x 30 515, 504; 140 x 640 62.6, 60.5.  Two
+  // pairs each for up to 64 keys gain nothing (1080 x 60 100.3, 99.2; x 32 63.9, 66.1).  The rule is one of N and the mask alone,
+  // so the bits of a slice don't depend on the size of the call.  Under causal masking such a block has one tile.
+  const bool shared = !CAUSAL && nblk > 0 && N - n0 <= kResident;
+  const int group = shared ? 0 : pair;  // which 32 keys of the block
+  const int k0w = n0 + group * kResident;
 
   const int nt = (N + kTile - 1) / kTile;
   const int t_begin = CAUSAL ? n0 / kTile : 0;
@@ -2089,13 +2097,14 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   }
   // this role's statistics of the four rows at + 4 * stat_row(quad)
   const int st_off = (WIDE ? 4 * g : acc16_row(0, g)) * 4 + (role_b ? 256 : 0);
-  constexpr int kQuads = WIDE ? 8 : 4;
   constexpr auto stat_row = [](int quad) { return WIDE ? 8 * quad : 32 * (quad >> 1) + 8 * (quad & 1); };
   char* const p_mine = p_xchg + pair * 4096 + lane * 16;  // + buffer * kPBytes + 1024 * fragment
 
-  // Products of 64 streamed rows and the 32 resident ones, and the accumulator of the second GEMM: dV^T (role A) or dK^T
-  // (role B).  Either way 32 registers of the one, in the order of the fragments of the second GEMM, and 64 of the other.
+  // Products of 64 (or, sharing, 32) streamed rows and the 32 resident ones, and the accumulator of the second GEMM: dV^T
+  // (role A) or dK^T (role B).  Either way 32 (16) registers of the one, in the order of the fragments of the second GEMM,
+  // and 64 of the other.
   typedef typename std::conditional<WIDE, f16v[2], f4v[4][2]>::type Product;
+  typedef typename std::conditional<WIDE, f16v[1], f4v[2][2]>::type HalfProduct;
   typename std::conditional<WIDE, f16v[G::kDBlocks], f4v[G16::kDB][2]>::type acc;
   auto clear = [](auto& x) __attribute__((always_inline)) {
     if constexpr (WIDE) {
@@ -2109,7 +2118,7 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
     }
   };
   // element e of 8 of fragment f of 4: 16 streamed rows f, or 32 streamed rows f >> 1 and resident block f & 1
-  auto element = [](const Product& x, int f, int e) __attribute__((always_inline)) {
+  auto element = [](const auto& x, int f, int e) __attribute__((always_inline)) {
     if constexpr (WIDE) return x[f >> 1][(f & 1) * 8 + e];
     else return x[2 * (f >> 1) + (e >> 2)][f & 1][e & 3];
   };
@@ -2131,14 +2140,15 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   // rows, on top of what x holds
   // Both GEMMs read their LDS fragments kLead MFMAs ahead of their use, in an order that is written out and
   // pinned (see the forward: scheduling hints alone are dropped when registers get scarce).
-  constexpr int kLead = 4, kN = 2 * G::kKSteps;  // units of one fragment; both GEMMs have as many
-  static_assert(kN == 4 * G::kDBlocks, "");
-  auto gemm1 = [&](const char* tile_lds, Product& x) __attribute__((always_inline)) {
+  constexpr int kLead = 4, kUnits = 2 * G::kKSteps;  // units of one fragment of a whole tile; both GEMMs have as many
+  static_assert(kUnits == 4 * G::kDBlocks, "");
+  auto gemm1 = [&](const char* tile_lds, auto& x) __attribute__((always_inline)) {
+    constexpr int kN = kUnits * sizeof(x) / sizeof(Product), kRB = kN / (WIDE ? G::kKSteps : G16::kKS);  // row blocks
     const unsigned a0 = opaque_lds_address(tile_lds + r_off[0]), a1 = opaque_lds_address(tile_lds + r_off[1]);
-    // unit n: row block n & 1 and feature step n >> 1, or row block n & 3 and feature step n >> 2
+    // unit n: row block n % kRB and feature step n / kRB
     auto read = [&](int n) __attribute__((always_inline)) {
-      if constexpr (WIDE) return swz_rows_at<D>(a0, a1, n & 1, n >> 1);
-      else return rows16_at<D>(a0, a1, n & 3, n >> 2);
+      if constexpr (WIDE) return swz_rows_at<D>(a0, a1, n % kRB, n / kRB);
+      else return rows16_at<D>(a0, a1, n % kRB, n / kRB);
     };
     h8 frag[kLead];
 #pragma unroll
@@ -2148,11 +2158,12 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
 #pragma unroll
     for (int n = 0; n < kN; ++n) {
       if constexpr (WIDE) {
-        x[n & 1] = mfma(frag[n % kLead], rf[n >> 1], x[n & 1]);
+        x[n % kRB] = mfma(frag[n % kLead], rf[n / kRB], x[n % kRB]);
       } else {
         if (n % 2 == 0) wait_lds_pinned(n + 3 < kN ? 2 : n + 2 < kN ? 1 : 0);
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb) x[n & 3][cb] = mfma16(frag[n % kLead], rf[2 * (n >> 2) + cb], x[n & 3][cb]);
+        for (int cb = 0; cb < 2; ++cb)
+          x[n % kRB][cb] = mfma16(frag[n % kLead], rf[2 * (n / kRB) + cb], x[n % kRB][cb]);
       }
       if (n + kLead < kN) frag[n % kLead] = read(n + kLead);
       __builtin_amdgcn_sched_barrier(0);
@@ -2160,7 +2171,8 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
     priority(IntTag<0>{}, IntTag<0>{});
   };
   // second GEMM: columns of dO (role A) or Q (role B) against the fp16 operand y
-  auto gemm2 = [&](const char* tile_lds, const h8 (&y)[4]) __attribute__((always_inline)) {
+  auto gemm2 = [&](const char* tile_lds, const auto& y) __attribute__((always_inline)) {
+    constexpr int kN = kUnits * sizeof(y) / sizeof(h8[4]);
     auto run = [&](auto read) __attribute__((always_inline)) {
       h8 frag[kLead];
 #pragma unroll
@@ -2194,9 +2206,9 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   };
   // P = exp2(S*c - lse2), fp16, in B-operand order.  MASKED tiles straddle the
   // diagonal or the end of the sequence.
-  auto probabilities = [&](const Product& x, h8 (&y)[4], const char* Sl, int q0, auto masked_tag)
-                           __attribute__((always_inline)) {
+  auto probabilities = [&](const auto& x, auto& y, const char* Sl, int q0, auto masked_tag) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value != 0;
+    constexpr int kQuads = sizeof(x) / (WIDE ? 16 : 32);
 #pragma unroll
     for (int quad = 0; quad < kQuads; ++quad) {
       const f4v l4 = *reinterpret_cast<const f4v*>(Sl + stat_row(quad) * 4);
@@ -2217,7 +2229,9 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   // a pair without keys has nothing to do, except for the zeros of dS it owes the last 64-key tile
   const bool has_keys = k0w < (SPILL ? (N + kTile - 1) / kTile * kTile : N);
   const int first_active = !has_keys ? n_it : CAUSAL ? k0w / kTile - t_begin : 0;
-  auto tile_active = [&](int it) __attribute__((always_inline)) { return CAUSAL ? it >= first_active : has_keys; };
+  auto tile_active = [&](int it) __attribute__((always_inline)) {
+    return CAUSAL ? it >= first_active : has_keys && (!shared || (it & 1) == pair >> 1);
+  };
 
   // Per iteration: wait for tile `it` (issued two iterations ago; the copies of tile
   // it+1 may still be in flight), one barrier, issue the copies of tile it+2.  Role A issues its half of them at the end
@@ -2253,92 +2267,131 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
     asm volatile("" : "+v"(r));  // here, not in the loop
   }
   if (n_it > 1) copy_tiles(1);
-  if (!role_b) {
-    for (int it = 0; it <= n_it; ++it) {
-      step_wait(it);
-      if (it < n_it && tile_active(it)) {
-        const char* Ql = q_ring + (it & 3) * T::kBytes;
-        const char* Gl = g_ring + (it % 3) * T::kBytes;
-        const char* Sl = st_ring + (it % 3) * kStBytes + st_off;
-        const int q0 = (t_begin + it) * kTile;
-        const bool masked = (CAUSAL && q0 < k0w + kResident - 1) || (q0 + kTile > N);
-        Product x;
-        h8 y[4];
-        clear(x);
-        gemm1(Ql, x);
-        if (masked) probabilities(x, y, Sl, q0, IntTag<1>{});
-        else probabilities(x, y, Sl, q0, IntTag<0>{});
-        char* pw = p_mine + (it & 1) * kPBytes;
-#pragma unroll
-        for (int f = 0; f < 4; ++f) *reinterpret_cast<h8*>(pw + f * 1024) = y[f];
-        gemm2(Gl, y);
-      }
-      step_copy(it);
-    }
-  } else {
-    Product x;  // delta - dP of the previous tile
-    clear(x);
-    for (int it = 0; it <= n_it; ++it) {
-      // After the second GEMM this wave issues the four stores of dS (SPILL) and then its copies of tile it + 2.  The wait
-      // at the top of the next iteration leaves at most as many operations in flight as those copies, the newest:
-      // every earlier copy has then landed, whatever order stores and copies complete in.  (Copies before the second GEMM,
-      // where the wait is for them too: B2 H40 N2048 causal 198.6 us against 195.7, B2 H32 N4096 causal 566.7 against
-      // 560.6, B3 H20 N1031 94.7 against 91.9.  After the GEMM and before the stores 200.1, 569.0, 91.9; at the end of the
-      // iteration 201.7, 573.6, 95.0.)
-      step_wait(it);
-      const bool prev_active = it >= 1 && tile_active(it - 1);
-      h8 y[4];
-      if (prev_active) {  // the part that needs P, one tile behind
-        const char* pr = p_mine + ((it - 1) & 1) * kPBytes;
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          const h8 p = *reinterpret_cast<const h8*>(pr + f * 1024);
-          float xr[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xr[e] = element(x, f, e);
-          y[f] = neg_mul_to_f16x8(p, xr);
+  // half_tag: the pairs share their keys, and each works on 32 rows of a tile.
+  auto run = [&](auto half_tag) __attribute__((always_inline)) {
+    constexpr bool HALF = decltype(half_tag)::value != 0;
+    constexpr int kFrags = HALF ? 2 : 4;
+    typedef typename std::conditional<HALF, HalfProduct, Product>::type Rows;
+    const int half = HALF ? pair & 1 : 0, rows_at = half * (T::kBytes / 2);
+    if (!role_b) {
+      for (int it = 0; it <= n_it; ++it) {
+        step_wait(it);
+        if (it < n_it && tile_active(it)) {
+          const char* Ql = q_ring + (it & 3) * T::kBytes + rows_at;
+          const char* Gl = g_ring + (it % 3) * T::kBytes + rows_at;
+          const char* Sl = st_ring + (it % 3) * kStBytes + st_off + half * 128;
+          const int q0 = (t_begin + it) * kTile + half * 32;
+          const bool masked = (CAUSAL && q0 < k0w + kResident - 1) || (q0 + (HALF ? 32 : kTile) > N);
+          Rows x;
+          h8 y[kFrags];
+          clear(x);
+          gemm1(Ql, x);
+          if (masked) probabilities(x, y, Sl, q0, IntTag<1>{});
+          else probabilities(x, y, Sl, q0, IntTag<0>{});
+          char* pw = p_mine + (it & 1) * kPBytes;
+  #pragma unroll
+          for (int f = 0; f < kFrags; ++f) *reinterpret_cast<h8*>(pw + f * 1024) = y[f];
+          gemm2(Gl, y);
         }
-        if (SPILL && k0w + kResident > N) {  // keys past the end contribute nothing to dQ
-#pragma unroll
-          for (int f = 0; f < 4; ++f)
-            if (k0w + (WIDE ? 0 : 16 * (f & 1)) + i >= N) y[f] = h8{};
-        }
+        step_copy(it);
       }
-      if (prev_active) gemm2(q_ring + ((it - 1) & 3) * T::kBytes, y);
-      if (SPILL && prev_active) {
-        // dS(it - 1) leaves here, between the two GEMMs, before the tile copies of role A, which come at the end of the
-        // iteration: the stores go through the same path and would queue.
-        const int t = t_begin + it - 1;  // the query tile
-        half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048;
-        static_for<4>([&](auto f_tag) __attribute__((always_inline)) {
-          constexpr int f = decltype(f_tag)::value, at = f * 1024;
-          if constexpr (!KEEP) store16_stream(dst, y[f], IntTag<at>{});
-          else store16_keep(dst, y[f], IntTag<at>{});
-        });
-      }
-      step_copy(it);
-      if (it < n_it && tile_active(it)) {
-        const char* Gl = g_ring + (it % 3) * T::kBytes;
-        const char* Sl = st_ring + (it % 3) * kStBytes + st_off;
-#pragma unroll
-        for (int quad = 0; quad < kQuads; ++quad) {
-          const f4v d4 = *reinterpret_cast<const f4v*>(Sl + stat_row(quad) * 4);
-          if constexpr (WIDE) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[quad >> 2][4 * (quad & 3) + r] = d4[r];
-          } else {
-            x[quad][0] = x[quad][1] = d4;
+    } else {
+      Rows x;  // delta - dP of the previous tile
+      clear(x);
+      for (int it = 0; it <= n_it; ++it) {
+        // After the second GEMM this wave issues the four stores of dS (SPILL) and then its copies of tile it + 2.  The wait
+        // at the top of the next iteration leaves at most as many operations in flight as those copies, the newest:
+        // every earlier copy has then landed, whatever order stores and copies complete in.  (Copies before the second GEMM,
+        // where the wait is for them too: B2 H40 N2048 causal 198.6 us against 195.7, B2 H32 N4096 causal 566.7 against
+        // 560.6, B3 H20 N1031 94.7 against 91.9.  After the GEMM and before the stores 200.1, 569.0, 91.9; at the end of the
+        // iteration 201.7, 573.6, 95.0.)
+        step_wait(it);
+        const bool prev_active = it >= 1 && tile_active(it - 1);
+        h8 y[kFrags];
+        if (prev_active) {  // the part that needs P, one tile behind
+          const char* pr = p_mine + ((it - 1) & 1) * kPBytes;
+  #pragma unroll
+          for (int f = 0; f < kFrags; ++f) {
+            const h8 p = *reinterpret_cast<const h8*>(pr + f * 1024);
+            float xr[8];
+  #pragma unroll
+            for (int e = 0; e < 8; ++e) xr[e] = element(x, f, e);
+            y[f] = neg_mul_to_f16x8(p, xr);
+          }
+          if (SPILL && k0w + kResident > N) {  // keys past the end contribute nothing to dQ
+  #pragma unroll
+            for (int f = 0; f < kFrags; ++f)
+              if (k0w + (WIDE ? 0 : 16 * (f & 1)) + i >= N) y[f] = h8{};
           }
         }
-        __builtin_amdgcn_sched_barrier(0);  // keep the delta loads out of the GEMM's read/MFMA pipeline
-        gemm1(Gl, x);
+        if (prev_active) gemm2(q_ring + ((it - 1) & 3) * T::kBytes + rows_at, y);
+        if (SPILL && prev_active) {
+          // dS(it - 1) leaves here, between the two GEMMs, before the tile copies of role A, which come at the end of the
+          // iteration: the stores go through the same path and would queue.
+          const int t = t_begin + it - 1;  // the query tile
+          half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048 + half * 1024;
+          static_for<kFrags>([&](auto f_tag) __attribute__((always_inline)) {
+            constexpr int f = decltype(f_tag)::value, at = f * 1024;
+            if constexpr (!KEEP) store16_stream(dst, y[f], IntTag<at>{});
+            else store16_keep(dst, y[f], IntTag<at>{});
+          });
+          if (HALF) {  // the zeros that the other 32 keys of the last 64-key tile owe
+            static_for<kFrags>([&](auto f_tag) __attribute__((always_inline)) {
+              constexpr int at = decltype(f_tag)::value * 1024;
+              if constexpr (!KEEP) store16_stream(dst + 4096, h8{}, IntTag<at>{});
+              else store16_keep(dst + 4096, h8{}, IntTag<at>{});
+            });
+          }
+        }
+        step_copy(it);
+        if (it < n_it && tile_active(it)) {
+          const char* Gl = g_ring + (it % 3) * T::kBytes + rows_at;
+          const char* Sl = st_ring + (it % 3) * kStBytes + st_off + half * 128;
+  #pragma unroll
+          for (int quad = 0; quad < (int)sizeof(Rows) / (WIDE ? 16 : 32); ++quad) {
+            const f4v d4 = *reinterpret_cast<const f4v*>(Sl + stat_row(quad) * 4);
+            if constexpr (WIDE) {
+  #pragma unroll
+              for (int r = 0; r < 4; ++r) x[quad >> 2][4 * (quad & 3) + r] = d4[r];
+            } else {
+              x[quad][0] = x[quad][1] = d4;
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);  // keep the delta loads out of the GEMM's read/MFMA pipeline
+          gemm1(Gl, x);
+        }
       }
     }
-  }
+  };
+  if (shared) run(IntTag<1>{});
+  else run(IntTag<0>{});
 
   static_assert(kKvWaves * Stage16<D>::kBytes <= 7 * T::kBytes && kKvWaves * StageGeom<D>::kBytes <= 7 * T::kBytes,
                 "the output staging tiles fit the rings");
   block_barrier();  // every wave is done with the rings: they become the staging tiles
+  if (shared) {  // the sums of the four pairs, added in the order of the pairs by the first one
+    constexpr int kSums = sizeof(acc) / 16, kBytes = kSums * 1024;  // per wave, 16 bytes of a lane at a time
+    static_assert(2 * (kKvPairs - 1) * kBytes <= 7 * T::kBytes, "the sums of three pairs fit the rings");
+    f4v* const sums = reinterpret_cast<f4v*>(&acc);
+    char* const first = smem + (role_b ? kKvPairs - 1 : 0) * kBytes + lane * 16;  // + (pair - 1) * kBytes
+    if (pair > 0) {
+#pragma unroll
+      for (int u = 0; u < kSums; ++u) *reinterpret_cast<f4v*>(first + (pair - 1) * kBytes + u * 1024) = sums[u];
+    }
+    block_barrier();
+    if (pair == 0) {
+      for (int other = 0; other < kKvPairs - 1; ++other) {
+#pragma unroll
+        for (int u = 0; u < kSums; ++u) {
+          const f4v x = *reinterpret_cast<const f4v*>(first + other * kBytes + u * 1024);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sums[u][r] += x[r];
+        }
+      }
+    }
+    block_barrier();
+    if (pair > 0) return;
+  }
   half_t* const out = (role_b ? dK : dV) + head_off;
   const float mul = role_b ? scale : 1.f;
   if constexpr (WIDE) {
