@@ -200,42 +200,61 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 }
 
 // Whether the backward does both passes, `blocks` blocks of 128 rows each, in one launch of 2 * blocks.  With fewer blocks
-// than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few more,
-// each has a nearly empty last round of its own.  Full rounds have nothing to gain and pay for the statistics, which the D =
-// 64 dQ pass makes on the side when it goes first, or, at D = 128, for forming S and dP twice.  us of the launches one after
-// the other, and of one with the statistics made by the blocks or, behind "+", by a kernel of their own first
-// (fmha_blocks_make_stats), N x slices (rounds of one pass):
-// D = 64, without a mask.  128 x 32 12.9, 8.1; 128 x 512 (1) 22.7, 20.7; 128 x 1024 44.4, 34.6; 128 x 2048 (4) 75.4, 69.1; 256 x
-// 64 16.4, 10.4; 256 x 320 (1.25) 38.8, 33.6; 256 x 640 (2.5) 64.6, 60.4; 256 x 768 (3) 73.3, 77.0.  512 x 32 22.5, 14.9; 512 x
-// 64 (0.5) 24.0, 23.2; 512 x 96 (0.75) 37.3, 33.7; 512 x 112 39.3, 40.9; 512 x 128 (1) 42.0, 44.2; 512 x 136 54.8, 50.8; 512 x
-// 160 (1.25) 55.9, 53.5; 512 x 176 57.5, 60.8; 512 x 208 (1.63) 70.4, 70.3.  1024 x 16 36.3, + 24.4; 2048 x 4 62.1, + 37.4;
-// 4096 x 4 (0.25) 118, + 75.5; 4096 x 6 120, + 115; 2048 x 16 (0.5) 71.0, + 69.7; 2048 x 24 (0.75) 110, + 103; 2048 x 28 118, +
-// 126; 2048 x 32 (1) 128, + 134; 2048 x 40 (1.25) 173, + 168; 2048 x 44 179, + 190; 4096 x 26 (1.63) 440, + 424; 4096 x 28 449,
-// + 438; 4096 x 30 462, + 484; 4096 x 36 (2.25) 554, + 561.
-// D = 64, causal.  128 x 128 14.6, 9.0; 256 x 256 (1) 26.1, 26.0; 256 x 768 (3) 68.7, 59.9; 256 x 1024 (4) 84.9, 84.6; 512 x 64
-// 24.5, 17.8; 512 x 192 (1.5) 48.6, 46.0; 512 x 320 (2.5) 72.3, 70.0; 512 x 512 (4) 110, 117; 1024 x 32 (0.5) 37.9, 27.3; 1024 x
-// 64 (1) 46.4, 43.4; 1024 x 104 74.4, 70.1; 1024 x 128 (2) 86.3, 85.7.  2048 x 12 63.2, + 41.0; 2048 x 32 (1) 79.9, + 74.3; 2048 x
-// 60 136, + 135; 2048 x 64 (2) 141, + 145; 4096 x 16 (1) 148, + 134; 4096 x 30 242, + 240; 8192 x 4 (0.5) 220, + 155; 8192 x 8
-// (1) 283, + 256; 8192 x 15 464, + 459; 8192 x 32 (4) 946, + 963.
-// D = 128, without a mask.  128 x 8 16.0, 9.4; 128 x 128 (0.5) 18.6, 11.7; 128 x 144 19.7, 20.1; 128 x 192 21.6, 20.4; 128 x 320
-// 37.3, 31.1; 128 x 512 (2) 46.8, 44.7; 256 x 16 20.0, 13.4; 256 x 64 (0.5) 23.1, 16.0; 256 x 72 24.0, 27.3; 256 x 128 (1) 29.6,
-// 31.6; 256 x 136 44.2, 42.4; 256 x 192 (1.5) 47.6, 46.7; 256 x 224 51.5, 58.5.  512 x 8 27.0, + 19.2; 512 x 32 (0.5) 31.7, +
-// 24.0; 512 x 36 32.2, + 39.2; 1024 x 8 42.1, + 30.9; 1024 x 16 (0.5) 46.0, + 37.5; 2048 x 8 (0.5) 75.4, + 64.5; 4096 x 2 124, +
-// 96.9; 4096 x 4 (0.5) 131, + 122; 4096 x 5 145, + 209; 8192 x 2 (0.5) 280, + 235; 512 x 68 (1.06) 61.9, + 61.8; 2048 x 18 166, +
-// 176.
-// D = 128, causal.  128 x 32 17.5, 10.4; 128 x 192 22.4, 21.2; 256 x 64 (0.5) 23.3, 15.3; 256 x 128 (1) 28.9, 26.5; 256 x 192
-// (1.5) 44.5, 39.2; 256 x 224 46.0, 48.2.  512 x 32 (0.5) 31.0, + 21.7; 512 x 64 (1) 37.7, + 34.2; 512 x 68 41.5, + 43.2; 1024 x 24
-// 47.8, + 38.0; 1024 x 32 (1) 54.0, + 48.1; 2048 x 8 (0.5) 71.3, + 54.2; 2048 x 16 (1) 84.9, + 76.0; 2048 x 18 91.6, + 89.2; 2048 x
-// 20 91.1, + 98.1; 4096 x 8 (1) 153, + 133; 4096 x 10 159, + 169; 8192 x 4 (1) 303, + 267; 8192 x 5 315, + 318.
+// than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few
+// more, each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together
+// it saves one start and one end, and pays for the statistics, which the D = 64 dQ pass makes on the side when it goes first,
+// or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  The lines are those of 7,000 launches
+// of 124 lengths timed both ways in turn.  us of the launches one after the other, and of one with the statistics made by the
+// blocks or, behind "+", by a kernel of their own first (fmha_blocks_make_stats), N x slices (blocks per CU), on both sides
+// of the lines:
+// D = 64, without a mask, up to 256 rows.  56 x 512 (2) equal, 48 x 512 13.8, 12.5; 64 x 486 (1.9) 14.3, 13.5; 64 x 512 14.0,
+// 15.0; 80 x 384 (1.5) 17.2, 16.2; 80 x 448 (1.75) 17.7, 18.7; 120 x 384 19.7, 19.2; 120 x 512 22.0, 23.9; 120 x 538 (2.1)
+// 28.9, 24.8; 128 x 512 23.0, 20.6; 192 x 256 (2) 24.0, 24.0; 210 x 243 (1.9) 27.9, 28.2; 210 x 269 36.9, 33.0.  Many blocks:
+// 24 x 3840 (15) 58.8, 58.5; 24 x 5120 75.4, 76.7; 40 x 3840 64.7, 63.3; 40 x 4096 (16) 68.5, 71.6; 64 x 2048 (8) 44.3, 42.9;
+// 64 x 2432 53.0, 55.1; 64 x 3584 69.4, 74.5; 80 x 2048 56.4, 57.6; 80 x 2560 68.5, 71.9; 128 x 2048 74.4, 69.3; 256 x 640
+// (5) 64.6, 60.4; 256 x 768 73.3, 77.0.
+// Longer: 512 x 32 22.5, 14.9; 512 x 96 (1.5) 37.3, 33.7; 512 x 112 39.3, 40.9; 512 x 128 (2) 42.0, 44.2; 512 x 136 54.8,
+// 50.8; 512 x 160 (2.5) 55.9, 53.5; 512 x 176 57.5, 60.8; 512 x 208 (3.25) 70.4, 70.3.  4096 x 4 (0.5) 118, + 75.5; 2048 x 24
+// (1.5) 110, + 103; 2048 x 28 118, + 126; 2048 x 32 (2) 128, + 134; 2048 x 40 (2.5) 173, + 168; 2048 x 44 179, + 190; 4096 x
+// 26 (3.25) 440, + 424; 4096 x 28 449, + 438; 4096 x 30 462, + 484; 4096 x 36 (4.5) 554, + 561.
+// D = 64, causal.  1 x 4096 (16) 57.2, 56.9; 1 x 5120 69.9, 70.3; 25 x 5120 (20) 82.7, 81.4; 140 x 1024 (8) 61.7, 56.2; 450 x
+// 320 (5) 69.5, 66.3; 450 x 352 72.5, 73.3; 512 x 512 (8) 110, 117; 777 x 144 (3.95) 70.4, 66.3; 1024 x 32 37.9, 27.3; 1024 x
+// 128 (4) 86.3, 85.7; 2048 x 32 (2) 79.9, + 74.3; 2048 x 60 136, + 135; 2048 x 64 (4) 141, + 145; 8192 x 8 (2) 283, + 256;
+// 8192 x 15 464, + 459; 8192 x 32 946, + 963.
+// D = 128, without a mask.  33 x 128 (0.5) 14.1, 7.8; 33 x 256 (1) 14.7, 13.3; 64 x 230 (0.9) 15.8, 15.5; 64 x 256 15.5,
+// 16.9; 64 x 264 23.9, 22.5; 64 x 384 (1.5) 25.8, 24.6; 64 x 397 27.2, 30.4; 110 x 128 18.7, 13.2; 110 x 136 19.0, 22.0; 110
+// x 256 24.1, 26.1; 110 x 264 35.1, 34.8; 110 x 384 38.4, 38.1; 110 x 410 39.7, 46.1.  128 x 128 19.0, 12.2; 128 x 141 (0.55)
+// 19.6, 20.8; 128 x 192 (0.75) 22.2, 21.1; 128 x 256 24.8, 24.2; 128 x 384 40.3, 34.5; 128 x 410 41.5, 43.7; 128 x 448 (1.75)
+// 44.2, 42.6; 128 x 512 47.0, 44.8.  140 x 64 (0.5) 19.6, 12.8; 140 x 68 20.1, 20.5; 140 x 128 (1) 23.7, 24.7; 140 x 141
+// 33.2, 33.9; 140 x 166 (1.3) 35.9, 34.3; 140 x 192 37.0, 36.3; 200 x 64 22.6, 16.4; 200 x 68 22.9, 27.5; 200 x 141 41.0,
+// 42.5; 256 x 132 (1.03) 43.8, 43.0; 256 x 192 46.7, 45.4; 256 x 205 48.5, 57.3.  350 x 38 (0.45) 26.9, 20.1; 350 x 43 27.2,
+// 34.6; 1200 x 11 (0.43) 49.6, + 40.1; 1200 x 13 49.4, + 67.8; 2048 x 8 (0.5) 75.4, + 64.5; 4096 x 4 (0.5) 131, + 122; 4096 x
+// 5 145, + 209.
+// D = 128, causal.  24 x 384 (1.5) 23.1, 18.0; 24 x 410 23.3, 22.8; 24 x 486 (1.9) 22.3, 23.2; 40 x 384 24.4, 20.2; 40 x 410
+// 24.7, 25.3; 40 x 486 24.1, 25.8; 64 x 410 28.1, 27.7; 64 x 512 (2) 30.7, 28.2; 110 x 410 40.0, 40.2; 110 x 512 45.5, 43.3;
+// 129 x 128 (1) 21.7, 21.5; 129 x 192 33.0, 30.5; 200 x 192 (1.5) 41.5, 35.9; 200 x 218 42.2, 43.3; 512 x 64 (1) 37.7, +
+// 34.2; 512 x 68 41.5, + 43.2; 777 x 33 (0.9) 42.0, + 37.8; 2048 x 16 (1) 84.9, + 76.0; 2048 x 18 91.6, + 89.2; 2048 x 20
+// 91.1, + 98.1; 4096 x 8 (1) 153, + 133; 4096 x 10 159, + 169; 8192 x 5 315, + 318.
 FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bool causal) {
   if (d == 128) {
-    if (n <= 128) return blocks <= 2L * cus;
-    if (causal) return 2 * blocks <= (n <= 256 ? 3L : 2L) * cus;
-    return 2 * blocks <= cus || (n <= 256 && blocks > cus && 2 * blocks <= 3L * cus);
+    if (blocks > 2L * cus) return false;
+    if (causal) {
+      if (n > 256) return blocks <= cus;
+      return 2 * blocks <= 3L * cus || n <= 24 || (n >= 52 && n <= 128);
+    }
+    if (2 * blocks <= cus) return true;                                      // one round instead of two
+    if (blocks > cus && 2 * blocks <= 3L * cus) return n < 160 || n == 256;  // three rounds instead of four
+    if (n <= 64) return 10 * blocks <= (n <= 48 ? 10L : 9L) * cus;
+    const long left = 2 * blocks % cus;
+    return n == 128 && (left == 0 || 2 * left >= cus);
   }
   const long places = 2L * cus;
-  if (causal) return n <= 512 ? blocks * n <= places * (2L * n + 256) : blocks < 2 * places;
-  if (n <= 256) return blocks * n <= places * (n + 384L);  // the start and the end of a launch are a good part of it
+  if (causal) return n <= 512 ? blocks <= 10 * places && blocks * n <= places * (2L * n + 256) : blocks < 2 * places;
+  if (n <= 256) {
+    if (4 * blocks > 3 * places && blocks <= places)  // two rounds either way
+      return n <= 56 || (n <= 64 && 20 * blocks <= 19 * places) || (n >= 128 && n <= 192);
+    return 2 * blocks <= (n <= 60 ? 15 : 8) * places && blocks * n <= places * (n + 384L);
+  }
   const long left = 2 * blocks % places;
   return 4 * blocks <= 3 * places || (blocks > places && blocks < 2 * places && left > 0 && 2 * left <= places);
 }

@@ -434,6 +434,25 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_one_launch_only_where_it_is_faster(tmp_path):
+    """D, N, slices, causal of launches timed both ways on 256 compute units."""
+    rule = "fmha_passes_at_once(x[0], (long)((x[1] + 127) / 128) * x[2], x[1], 256, x[3])"
+    faster_apart = [
+        (128, 64, 256, 0), (128, 64, 512, 0), (128, 77, 136, 0), (128, 100, 256, 0), (128, 120, 141, 0), (128, 110, 512, 0),
+        (128, 128, 141, 0), (128, 128, 410, 0), (128, 140, 128, 0), (128, 200, 141, 0), (128, 40, 486, 1), (128, 300, 90, 1),
+        (64, 64, 512, 0), (64, 64, 3584, 0), (64, 80, 448, 0), (64, 100, 512, 0), (64, 120, 512, 0), (64, 80, 2560, 0),
+        (64, 5, 5120, 0), (64, 210, 250, 0), (64, 512, 128, 0), (64, 5, 8192, 1),
+    ]
+    faster_at_once = [
+        (128, 33, 256, 0), (128, 64, 230, 0), (128, 110, 128, 0), (128, 77, 384, 0), (128, 128, 192, 0), (128, 128, 512, 0),
+        (128, 140, 166, 0), (128, 256, 192, 0), (128, 64, 512, 1), (128, 24, 410, 1), (128, 200, 192, 1), (128, 1031, 28, 1),
+        (64, 48, 512, 0), (64, 64, 486, 0), (64, 120, 384, 0), (64, 120, 538, 0), (64, 128, 512, 0), (64, 24, 3840, 0),
+        (64, 128, 2048, 0), (64, 512, 96, 0), (64, 1, 4096, 1), (64, 140, 900, 1), (64, 1024, 64, 1),
+    ]
+    assert not any(abi.host_rule(tmp_path, rule, faster_apart))
+    assert all(abi.host_rule(tmp_path, rule, faster_at_once))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,B,H,N,causal", [(64, *case) for case in [
     # one launch, statistics made by the blocks: one tile, edges of tiles and blocks, two rounds and more
