@@ -1976,7 +1976,7 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // Otherwise fragment f is queries 32 (f >> 1) .. and keys 16 (f & 1) .., and lane 16 * g + i holds key i and as element e
 // query 16 * (g >> 1) + 8 * (e >> 2) + 4 * (g & 1) + (e & 3).  Rows of keys at or past n are written as zeros; (key tile,
 // query tile) pairs above the diagonal are not written (and not read) under causal masking.
-// KEEP: without the non-temporal hint on those stores (rule: launch_backward).
+// KEEP: without the non-temporal hint on those stores (rule: fmha_ds_used_once).
 // WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: launch_backward).
 // STATS: the row statistics of every tile are formed here, from O, dO and LSE, a tile ahead; delta and lse2 are not read.
 constexpr int kKvStBytes = 1024;
@@ -3258,15 +3258,9 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   float* lse2 = delta + (long)batch * head * n;
   half_t* ds = spill ? (half_t*)((char*)delta + spill_offset(batch, head, n)) : nullptr;
   const int np = padded_n(n);
-  // dS stays in the 256 MiB Infinity Cache between the two passes if neither is told that it is used once: where it fits
-  // together with the six tensors the passes touch, and from 10 MiB on.  Forward and backward, us without and with the hint
-  // (dS; with the tensors, MiB): B1 H4 N1024 59.5, 60.4 (8; 14), B1 H16 N512 40.7, 39.8 (8; 14), B1 H10 N1024 causal 63.3,
-  // 65.2 (10; 25), B1 H4 N2048 causal 101, 106 (16; 28), B1 H8 N4096 causal 207, 224 (128; 176), B1 H11 N4096 causal 240,
-  // 254 (176; 242), B3 H20 N1031 203, 207 (152; 243), H224 N512 185, 179 (112; 280), H88 N1024 237, 227 (176; 308), B1 H16
-  // N4096 causal 305, 300 (256; 352), H64 N4096 causal 1217, 1161 (1024; 1408).
   const size_t ds_bytes = slice_bytes(n) * (spill ? slices_at_once : 0) / (CAUSAL ? 2 : 1);
   const size_t touched = ds_bytes + 6 * (size_t)slices_at_once * n * D * sizeof(half_t);
-  const int stream_ds = ds_bytes < (10u << 20) || touched > (256u << 20);
+  const int stream_ds = fmha_ds_used_once(ds_bytes, touched, n, CAUSAL);
   auto delta_pass = [&]() {
     const unsigned rows = (unsigned)slices * n;              // fewer than 2^32 / (D / 8): check_shape
     const unsigned most = (1u << 23) * delta_rows(D);        // a launch of fewer than 2^32 threads: fewer than twice the blocks

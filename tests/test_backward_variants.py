@@ -217,14 +217,29 @@ def test_dq_ignores_dS_that_no_query_needs(H, N, causal):
     assert (got[0].float() - want[0].float()).abs().max() <= 2e-3
 
 
+HINT_ON_DS = [  # H, N, causal, whether the passes are called one by one, whether dS is told to be used once
+    (127, 256, False, False, True), (128, 256, False, False, False),   # 15.9 and 16 MiB of dS
+    (511, 127, False, False, True), (512, 127, False, False, False),
+    (511, 50, True, False, True), (513, 50, True, False, False),       # 7.98 and 8.02 MiB
+    (4, 1024, False, True, True), (5, 1024, False, True, False),       # 8 and 10 MiB
+    (5, 1025, True, True, True), (9, 1025, True, True, False),         # 6.3 and 11.4 MiB
+    (63, 1031, False, False, False), (64, 1031, False, False, True),   # 255 and 259 MiB of dS and tensors
+    (71, 1031, True, False, False), (106, 1031, True, False, True),    # 197 and 294 MiB
+]
+
+
+def test_hint_on_ds_cases(tmp_path):
+    """The cases below store dS on 256 compute units, with the hint or without as they say."""
+    once = "fmha_passes_at_once(128, (long)((x[1] + 127) / 128) * x[0], x[1], 256, x[2])"
+    ds = "(unsigned long)x[0] * ((x[1] + 127) / 128 * 128) * ((x[1] + 127) / 128 * 128) * 2 / (x[2] ? 2 : 1)"
+    hint = f"fmha_ds_used_once({ds}, {ds} + 6ul * x[0] * x[1] * 256, x[1], x[2])"
+    assert not any(abi.host_rule(tmp_path, once, [c[:3] for c in HINT_ON_DS if not c[3]]))
+    assert abi.host_rule(tmp_path, hint, HINT_ON_DS) == [c[4] for c in HINT_ON_DS]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,N,causal", [
-    (4, 1024, False), (5, 1024, False),      # 8 MiB of dS: stored with the used-once hint; 10 MiB: without
-    (5, 1025, True), (9, 1025, True),        # 6.3 and 11.4 MiB of dS
-    (63, 1031, False), (64, 1031, False),    # 255 and 259 MiB of dS and tensors
-    (71, 1031, True), (106, 1031, True),     # 197 and 294 MiB
-])
-def test_hint_on_the_stores_of_ds(H, N, causal):
+@pytest.mark.parametrize("H,N,causal,one_by_one,hint", HINT_ON_DS)
+def test_hint_on_the_stores_of_ds(H, N, causal, one_by_one, hint):
     """Both sides of the lines between dS stored with and without the hint: the gradients of the recomputing path (dQ
     sums the same products in another order)."""
     D, lib = 128, abi.load()
@@ -232,7 +247,7 @@ def test_hint_on_the_stores_of_ds(H, N, causal):
     q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
     out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
     want = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=True)
-    got = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal)
+    got = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=one_by_one)
     assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
     assert (got[0].float() - want[0].float()).abs().max() <= 2e-3
 
