@@ -2419,8 +2419,8 @@ fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 
 // The dK/dV pass and the dQ pass that recomputes S and dP in one launch, for problems of so few blocks that neither fills the
 // chip: dS is not stored.  STATS as in fmha_bwd_both_pipe_kernel.  The blocks are those of the kernels for either pass, and so
-// are the results, bit for bit; those over dS give them too.  Rules and both sides: fmha_passes_at_once,
-// fmha_blocks_make_stats.
+// are the results, bit for bit; the dQ pass over dS adds the same dS up in the same order and gives them too.  Rules and both
+// sides: fmha_passes_at_once, fmha_blocks_make_stats.
 static_assert(kDqBlockQ == kKvBlockKeys && kDqThreads == kKvThreads, "as many blocks of either pass, of the same size");
 template <bool CAUSAL, bool STATS>
 __global__ void __launch_bounds__(kKvThreads, 1)

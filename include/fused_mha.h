@@ -109,8 +109,10 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * workspace the dQ pass recomputes S and dP.  With room for some of the slices
  * fused_mha_backward runs the two passes in rounds, that many slices at a time,
  * unless rounds of so few slices would leave compute units idle; the results are
- * the same bits as with room for all.  All paths are deterministic and give
- * the same dK and dV bits; dQ of the recomputing pass differs by summation order.
+ * the same bits as with room for all.  All paths are deterministic and, from
+ * finite inputs, give the same bits of d_q, d_k and d_v: a (batch, head) slice's
+ * gradients depend neither on the workspace nor on how many other slices the
+ * call has.
  * fused_mha_backward_workspace_bytes returns
  *   - d = 64: the minimum.  The dQ pass always recomputes, which is the faster
  *     way there, and nothing else is read or written whatever the size;
@@ -183,8 +185,8 @@ int fused_mha_backward_noalloc(const void *query_ptr, const void *key_ptr, const
                                float scale, int causal, void *stream);
 
 /*
- * The three passes of fused_mha_backward (which with d = 64 may put several
- * into one launch, with the same results), one entry point each, so a
+ * The three passes of fused_mha_backward (which may put several into one
+ * launch, with the same bits as results), one entry point each, so a
  * caller can time them separately or, with the minimum workspace, put the dQ
  * pass and the dK/dV pass (then independent of each other, both depend on the
  * delta pass) on different streams.  Same conventions and workspace as fused_mha_backward.  No
