@@ -204,7 +204,7 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 // more, each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together
 // it saves one start and one end, and pays for the statistics, which the D = 64 dQ pass makes on the side when it goes first,
 // or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  The lines are those of 7,000 launches
-// of 124 lengths timed both ways in turn.  us of the launches one after the other, and of one with the statistics made by the
+// of 106 lengths timed both ways in turn.  us of the launches one after the other, and of one with the statistics made by the
 // blocks or, behind "+", by a kernel of their own first (fmha_blocks_make_stats), N x slices (blocks per CU), on both sides
 // of the lines:
 // D = 64, without a mask, up to 256 rows.  56 x 512 (2) equal, 48 x 512 13.8, 12.5; 64 x 486 (1.9) 14.3, 13.5; 64 x 512 14.0,

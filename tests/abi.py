@@ -94,14 +94,19 @@ def forward(lib, q, k, v, scale, causal, stream=None):
     return out, lse
 
 
-def backward(lib, q, k, v, out, dout, lse, scale, causal, stream=None, split=False, min_workspace=False):
+def backward(lib, q, k, v, out, dout, lse, scale, causal, stream=None, split=False, min_workspace=False, poison=False):
     """min_workspace: pass only delta + lse2 (the dQ pass then recomputes S and dP) instead of the
-    workspace with room for the dS tiles (the dK/dV pass spills dS, the dQ pass is one GEMM)."""
+    workspace with room for the dS tiles (the dK/dV pass spills dS, the dQ pass is one GEMM).
+    split: the passes one by one, which with that room store dS also where fused_mha_backward goes in one launch.
+    poison: workspace and gradients hold NaN before the call."""
     B, N, H, D = q.shape
     nbytes = (lib.fused_mha_backward_min_workspace_bytes if min_workspace else
               lib.fused_mha_backward_workspace_bytes)(B, H, N, D)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
+    if poison:
+        for t in (ws, *(g.view(torch.uint8) for g in (dq, dk, dv))):
+            t.fill_(255)
     s = torch.cuda.current_stream().cuda_stream if stream is None else stream
     if split:
         rc = lib.fused_mha_backward_delta(out.data_ptr(), dout.data_ptr(), lse.data_ptr(), ws.data_ptr(), nbytes, B, H, N, D, s)

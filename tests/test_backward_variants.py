@@ -120,23 +120,38 @@ def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
             assert torch.equal(a, b[:, :, h:h + 1])
 
 
+EITHER_MFMA = [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200]
+
+
+def _slices_of_a_busy_launch(N, causal, cus):
+    return -(-5 * cus // (4 if causal else 8) // (-(-N // 128))) + 1
+
+
+def test_mfmas_of_the_cases_below(tmp_path):
+    """16 x 16 ones for the whole launch and 32 x 32 ones for a slice of it, on 256 compute units."""
+    wide = "fmha_wide_mfmas((long)((x[0] + 127) / 128) * x[1], 256, x[2])"
+    cases = [(N, _slices_of_a_busy_launch(N, causal, 256), causal) for N in EITHER_MFMA for causal in (False, True)]
+    assert not any(abi.host_rule(tmp_path, wide, cases))
+    assert all(abi.host_rule(tmp_path, wide, [(N, 1, causal) for N, _, causal in cases]))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("N", [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200])
+@pytest.mark.parametrize("N", EITHER_MFMA)
 def test_backward_d128_with_either_mfma(N, causal):
     """A launch that has just enough blocks takes the passes with 16 x 16 MFMAs, a slice of it those with 32 x 32 ones: the
-    same bits, with and without the workspace for dS."""
+    same bits, with and without the workspace for dS.  The passes are called one by one: together, launches of this size
+    go in one."""
     D, lib = 128, abi.load()
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    H = -(-5 * cus // (4 if causal else 8) // (-(-N // 128))) + 1
+    H = _slices_of_a_busy_launch(N, causal, torch.cuda.get_device_properties(0).multi_processor_count)
     gen = torch.Generator(device="cuda").manual_seed(N)
     q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
     out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
     for least in (False, True):
-        whole = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=least)[:3]
+        whole = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=least, split=True)[:3]
         for h in (0, H - 1):
             one = [t[:, :, h:h + 1].contiguous() for t in (q, k, v, out, do)]
-            alone = abi.backward(lib, *one, lse[:, h:h + 1].clone(), D ** -0.5, causal, min_workspace=least)[:3]
+            alone = abi.backward(lib, *one, lse[:, h:h + 1].clone(), D ** -0.5, causal, min_workspace=least, split=True)[:3]
             for a, b in zip(alone, whole):
                 assert torch.equal(a, b[:, :, h:h + 1])
 
@@ -153,16 +168,9 @@ def test_backward_d128_short_last_block_of_keys(N):
     out, lse = abi.forward(lib, qg, kg, vg, scale, False)
     ref = ao.attention_backward(q, k, v, do, scale, False)
     least = abi.backward(lib, qg, kg, vg, out, dog, lse, scale, False, min_workspace=True)[:3]
-    split = abi.backward(lib, qg, kg, vg, out, dog, lse, scale, False, split=True)[:3]
-    nbytes = lib.fused_mha_backward_workspace_bytes(B, 60 * H, N, D)
+    split = abi.backward(lib, qg, kg, vg, out, dog, lse, scale, False, split=True, poison=True)[:3]
     many = [t.repeat(1, 1, 60, 1) for t in (qg, kg, vg, out, dog)]  # enough slices for the passes over dS
-    many_lse = lse.repeat(1, 60, 1)
-    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
-    spill = [torch.full_like(many[0], float("nan")) for _ in range(3)]
-    rc = lib.fused_mha_backward(*(t.data_ptr() for t in many), many_lse.data_ptr(), ws.data_ptr(), nbytes,
-                                *(g.data_ptr() for g in spill), B, 60 * H, N, N, D, scale, 0,
-                                torch.cuda.current_stream().cuda_stream)
-    assert rc == abi.OK
+    spill = abi.backward(lib, *many, lse.repeat(1, 60, 1), scale, False, poison=True)[:3]
     for i, want in enumerate(ref):
         for got in (least[i], split[i], spill[i][:, :, :H], spill[i][:, :, -H:]):
             # fp16 roundings of P, dS, delta's O and the result: the repository's bound for gradients of order 1
@@ -170,47 +178,73 @@ def test_backward_d128_short_last_block_of_keys(N):
             assert torch.equal(got, least[i])
 
 
+LAST_ROUND = [  # H, N, D, whether fused_mha_backward goes in one launch
+    (65, 1024, 64, True), (57, 1031, 64, True),      # 520 and 513 blocks on 512 places
+    (65, 1024, 128, False), (57, 1031, 128, False),  # the forward alone
+    (90, 1024, 64, False), (75, 1031, 64, False),    # 720 and 675
+    (129, 1024, 64, False), (128, 1025, 64, False),  # 1032 blocks, and 1152, whose last ones have one row each
+]
+
+
+def test_launches_of_the_cases_below(tmp_path):
+    """On 256 compute units, and that the passes' own launches have at most half a round behind full ones."""
+    once = "fmha_passes_at_once(x[2], (long)((x[1] + 127) / 128) * x[0], x[1], 256, 0)"
+    assert abi.host_rule(tmp_path, once, LAST_ROUND) == [c[3] for c in LAST_ROUND]
+    for H, N, D, _ in LAST_ROUND:
+        if D == 64:
+            rounds, left = divmod(H * -(-N // 128), 512)
+            assert 1 <= rounds < 3 and 0 < left <= 256
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,N,D", [
-    (65, 1024, 64), (57, 1031, 64),    # 520 and 513 blocks on 512 places
-    (65, 1024, 128), (57, 1031, 128),  # the forward alone
-    (129, 1024, 64), (128, 1025, 64),  # 1032 blocks, and 1152, whose last ones have one row each
-])
-def test_a_nearly_empty_last_round(H, N, D):
-    """Launches in which every other wave slot goes first: the bits of a slice alone, which has no second round."""
+@pytest.mark.parametrize("H,N,D,once", LAST_ROUND)
+def test_a_nearly_empty_last_round(H, N, D, once):
+    """Launches in which every other wave slot goes first: the bits of a slice alone, which has no second round.  The
+    passes of the D = 64 backward take them one by one, and together unless all of it goes in one launch."""
     lib = abi.load()
     gen = torch.Generator(device="cuda").manual_seed(N + H)
     q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
     out, lse = abi.forward(lib, q, k, v, D ** -0.5, False)
     whole = [out] + list(abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, False)[:3])
+    split = [out] + list(abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, False, split=True)[:3])
     for h in (0, H // 2, H - 1):
         q1, k1, v1, do1 = (t[:, :, h:h + 1].contiguous() for t in (q, k, v, do))
         out1, lse1 = abi.forward(lib, q1, k1, v1, D ** -0.5, False)
         alone = [out1] + list(abi.backward(lib, q1, k1, v1, out1, do1, lse1, D ** -0.5, False)[:3])
         assert torch.equal(lse1, lse[:, h:h + 1])
-        for a, b in zip(alone, whole):
-            assert torch.equal(a, b[:, :, h:h + 1])
+        for a, b, c in zip(alone, whole, split):
+            assert torch.equal(a, b[:, :, h:h + 1]) and torch.equal(a, c[:, :, h:h + 1])
+
+
+DS_IN_ONE_CALL = [(260, 300), (130, 600), (50, 300), (100, 300)]  # H, N: dS is stored, without a mask or under one
+
+
+def test_dS_in_one_call(tmp_path):
+    """Of the cases below on 256 compute units, and that it is by passes with 32 x 32 MFMAs too."""
+    expression = "!fmha_passes_at_once(128, (long)((x[1] + 127) / 128) * x[0], x[1], 256, x[2])"
+    wide = "fmha_wide_mfmas((long)((x[1] + 127) / 128) * x[0], 256, x[2])"
+    no_mask, causal = ([(*case, mask) for case in DS_IN_ONE_CALL] for mask in (0, 1))
+    assert abi.host_rule(tmp_path, expression, no_mask) == [True] * 4
+    assert abi.host_rule(tmp_path, expression, causal) == [True, True, False, True]
+    assert abi.host_rule(tmp_path, wide, no_mask) == [False, False, True, False]
+    assert abi.host_rule(tmp_path, wide, causal) == [False, False, True, True]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("H,N", [(3, n) for n in (1, 32, 33, 64, 65, 96, 97, 128, 129, 257, 320)] + [(260, 300), (130, 600)])
+@pytest.mark.parametrize("H,N", [(3, n) for n in (1, 32, 33, 64, 65, 96, 97, 128, 129, 257, 320)] + DS_IN_ONE_CALL)
 def test_dq_ignores_dS_that_no_query_needs(H, N, causal):
-    """The workspace holds NaN where the dK/dV pass writes nothing.  dQ is that of the recomputing path, bit for bit."""
+    """The workspace holds NaN where the dK/dV pass writes nothing.  dQ is that of the recomputing path, bit for bit.  By the
+    passes one by one, which store dS in every case."""
     D, lib = 128, abi.load()
     gen = torch.Generator(device="cuda").manual_seed(N)
     q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
     out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
     want = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=True)[:3]
-    nbytes = lib.fused_mha_backward_workspace_bytes(1, H, N, D)
-    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
-    got = [torch.full_like(q, float("nan")) for _ in range(3)]
-    rc = lib.fused_mha_backward(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), lse.data_ptr(),
-                                ws.data_ptr(), nbytes, *(g.data_ptr() for g in got), 1, H, N, N, D, D ** -0.5,
-                                int(causal), torch.cuda.current_stream().cuda_stream)
-    assert rc == abi.OK
-    for a, b in zip(got[:3], want[:3]):
-        assert torch.equal(a, b)
+    for split in (True, False):
+        got = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=split, poison=True)[:3]
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
 
 
 HINT_ON_DS = [  # H, N, causal, whether the passes are called one by one, whether dS is told to be used once
@@ -462,21 +496,46 @@ def test_one_launch_only_where_it_is_faster(tmp_path):
     assert all(abi.host_rule(tmp_path, rule, faster_at_once))
 
 
+ONE_LAUNCH = {  # B, H, N, causal by head size and by what fused_mha_backward does
+    (64, "one launch, statistics made by the blocks"): [
+        (1, 1, 1, False), (3, 5, 64, True), (2, 3, 65, False), (1, 3, 512, False), (2, 4, 511, True), (1, 5, 1024, True),
+        (16, 40, 129, False), (1, 70, 1000, True), (1, 480, 60, False), (1, 900, 127, False),
+    ],
+    (64, "one launch behind the kernel for the statistics"): [
+        (1, 3, 513, False), (2, 2, 1025, True), (1, 5, 1031, False), (1, 3, 1536, True), (3, 20, 1031, False),
+    ],
+    (64, "the passes one after the other"): [
+        (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False), (1, 3900, 33, False), (1, 512, 64, False),
+        (1, 500, 65, False), (1, 250, 193, False), (1, 3100, 65, True), (1, 600, 511, True), (1, 120, 1031, True),
+    ],
+    (128, "one launch, statistics made by the blocks"): [
+        (1, 1, 1, True), (3, 5, 33, False), (2, 3, 64, True), (2, 3, 65, False), (1, 100, 128, True), (3, 100, 77, False),
+        (2, 30, 255, False), (1, 70, 256, True), (1, 140, 256, False), (3, 7, 384, True), (1, 9, 321, False),
+        (5, 100, 64, True),
+    ],
+    (128, "one launch behind the kernel for the statistics"): [
+        (1, 3, 385, False), (2, 2, 1031, True), (1, 9, 1031, False), (1, 30, 1000, True), (1, 2, 2049, False),
+    ],
+    (128, "the passes one after the other"): [
+        (5, 100, 77, False), (1, 140, 250, False), (1, 70, 250, False), (1, 70, 400, True), (1, 20, 1031, False),
+        (1, 400, 33, False), (1, 513, 64, True), (1, 400, 40, True), (1, 150, 65, False), (1, 140, 128, False),
+    ],
+}
+
+
+def test_launches_of_the_backward(tmp_path):
+    """The cases below on 256 compute units."""
+    shape = "x[0], (long)((x[3] + 127) / 128) * x[1] * x[2], x[3], 256, x[4]"
+    for (D, what), cases in ONE_LAUNCH.items():
+        cases = [(D, *case) for case in cases]
+        assert abi.host_rule(tmp_path, f"fmha_passes_at_once({shape})", cases) == [what.startswith("one launch")] * len(cases)
+        if what.startswith("one launch"):
+            blocks = abi.host_rule(tmp_path, "fmha_blocks_make_stats(x[0], x[3], x[4])", cases)
+            assert blocks == [what.endswith("by the blocks")] * len(cases)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("D,B,H,N,causal", [(64, *case) for case in [
-    # one launch, statistics made by the blocks: one tile, edges of tiles and blocks, two rounds and more
-    (1, 1, 1, False), (3, 5, 64, True), (2, 3, 65, False), (1, 3, 512, False), (2, 4, 511, True), (1, 5, 1024, True),
-    (16, 40, 129, False), (1, 70, 1000, True),
-    # one launch behind the kernel for the statistics
-    (1, 3, 513, False), (2, 2, 1025, True), (1, 5, 1031, False), (1, 3, 1536, True), (3, 20, 1031, False),
-    # two launches
-    (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False),
-]] + [(128, *case) for case in [
-    (1, 1, 1, True), (3, 5, 33, False), (2, 3, 64, True), (2, 3, 65, False), (1, 100, 128, True), (5, 100, 77, False),
-    (2, 30, 255, False), (1, 70, 256, True), (1, 140, 256, False), (3, 7, 384, True), (1, 9, 321, False),
-    (1, 3, 385, False), (2, 2, 1031, True), (1, 9, 1031, False), (1, 30, 1000, True), (1, 2, 2049, False),
-    (1, 140, 250, False), (1, 70, 250, False), (1, 70, 400, True), (1, 20, 1031, False),
-]])
+@pytest.mark.parametrize("D,B,H,N,causal", [(D, *case) for (D, _), cases in ONE_LAUNCH.items() for case in cases])
 def test_backward_in_one_launch(D, B, H, N, causal):
     """Whatever goes in one launch, gradients and delta are those of the passes one by one, bit for bit, also with strides
     and with the least workspace (at D = 128 the passes one by one store dS, the launch forms it twice)."""

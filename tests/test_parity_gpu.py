@@ -419,14 +419,16 @@ def test_hip_graph_capture_and_replay():
 SPILL_CASES = [  # B, H, N, D, causal
     (1, 2, 64, 128, True), (2, 3, 333, 64, True), (1, 2, 70, 128, False), (1, 2, 40, 64, True),
     (1, 2, 1031, 128, True), (2, 4, 512, 64, False), (1, 20, 384, 128, True), (1, 9, 1500, 64, False),
+    (1, 100, 384, 128, True), (1, 50, 300, 128, False),  # enough blocks that dS is stored in one call too
 ]
 
 
 @pytest.mark.parametrize("B,H,N,D,causal", SPILL_CASES)
 def test_spill_and_recompute_backward_agree(lib, B, H, N, D, causal):
     """At head size 128 the backward has two paths, chosen by the size of the workspace: with room for the dS tiles the dK/dV pass
-    spills them and the dQ pass is one GEMM; with the minimum workspace the dQ pass recomputes S and dP.  All three
-    gradients are sums of the same products in the same order (bit-equal); both match the oracle."""
+    spills them and the dQ pass is one GEMM; with the minimum workspace the dQ pass recomputes S and dP.  (With as few
+    blocks as in the first cases one call takes the second path whatever the size; the passes one by one spill.)  All
+    three gradients are sums of the same products in the same order (bit-equal); both match the oracle."""
     scale = 1.0 / math.sqrt(D)
     q, k, v, do = ao.make_inputs(B, N, H, D, seed=5 * N + D)
     print(f"spill/recompute B{B} H{H} N{N} D{D} causal={causal}", flush=True)
