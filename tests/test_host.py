@@ -105,6 +105,19 @@ def test_workspace_within(lib, batch, head, n, d, room, slices):
     assert f(batch, head, 0, d, room) == 0
 
 
+@pytest.mark.parametrize("batch,head,n,d,causal,room", [
+    (2, 32, 4096, 128, 1, True), (1, 8, 4096, 128, 1, False), (1, 8, 4096, 128, 0, True), (1, 4, 4096, 128, 0, False),
+    (1, 400, 100, 128, 0, True), (1, 100, 100, 128, 0, False), (1, 4, 128, 64, 0, False), (1, 64, 4096, 64, 1, False),
+])
+def test_workspace_for(lib, batch, head, n, d, causal, room):
+    """The size the extension takes for one backward: none for dS where both passes go in one launch (256 compute units)."""
+    f = lib.fmha_backward_workspace_for
+    f.argtypes, f.restype = [ctypes.c_int] * 5, ctypes.c_size_t
+    which = lib.fused_mha_backward_workspace_bytes if room else lib.fused_mha_backward_min_workspace_bytes
+    assert f(batch, head, n, d, causal) == which(batch, head, n, d)
+    assert f(batch, head, 0, d, causal) == 0
+
+
 def test_forward_validation_codes(lib):
     p = 0x1000  # never dereferenced: every call below is rejected before a launch
     f = lib.fused_mha_forward
