@@ -203,16 +203,18 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 // than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few
 // more, each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together
 // it saves one start and one end, and pays for the statistics, which the D = 64 dQ pass makes on the side when it goes first,
-// or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  The lines are those of 7,000 launches
-// of 106 lengths timed both ways in turn.  us of the launches one after the other, and of one with the statistics made by the
+// or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  Timed both ways, 9,700 launches of 108
+// lengths lose 0.2 to 0.7 % on average against the better way, D = 128 without a mask 1.1 % before the lines were drawn between
+// lengths of 128 x 2^k; most of that is one launch being faster past the lines (128 x 537 at D = 128, 128 x 3584 at D = 64:
+// 0.8 of the time).  us of the launches one after the other, and of one with the statistics made by the
 // blocks or, behind "+", by a kernel of their own first (fmha_blocks_make_stats), N x slices (blocks per CU), on both sides
 // of the lines:
 // D = 64, without a mask, up to 256 rows.  56 x 512 (2) equal, 48 x 512 13.8, 12.5; 64 x 486 (1.9) 14.3, 13.5; 64 x 512 14.0,
 // 15.0; 80 x 384 (1.5) 17.2, 16.2; 80 x 448 (1.75) 17.7, 18.7; 120 x 384 19.7, 19.2; 120 x 512 22.0, 23.9; 120 x 538 (2.1)
-// 28.9, 24.8; 128 x 512 23.0, 20.6; 192 x 256 (2) 24.0, 24.0; 210 x 243 (1.9) 27.9, 28.2; 210 x 269 36.9, 33.0.  Many blocks:
-// 24 x 3840 (15) 58.8, 58.5; 24 x 5120 75.4, 76.7; 40 x 3840 64.7, 63.3; 40 x 4096 (16) 68.5, 71.6; 64 x 2048 (8) 44.3, 42.9;
-// 64 x 2432 53.0, 55.1; 64 x 3584 69.4, 74.5; 80 x 2048 56.4, 57.6; 80 x 2560 68.5, 71.9; 128 x 2048 74.4, 69.3; 256 x 640
-// (5) 64.6, 60.4; 256 x 768 73.3, 77.0.
+// 28.9, 24.8; 128 x 512 23.0, 20.6; 192 x 256 (2) 24.0, 24.0; 204 x 256 30.7, 29.0; 216 x 256 30.5, 29.9; 255 x 256 equal.
+// Many blocks: 24 x 3840 (15) 58.8, 58.5; 24 x 5120 75.4, 76.7; 40 x 3840 64.7, 63.3; 40 x 4096 (16) 68.5, 71.6; 64 x 2048 (8)
+// 44.3, 42.9; 64 x 2432 53.0, 55.1; 64 x 3584 69.4, 74.5; 80 x 2048 56.4, 57.6; 80 x 2560 68.5, 71.9; 128 x 2048 74.4, 69.3;
+// 256 x 640 (5) 64.6, 60.4; 256 x 768 73.3, 77.0.
 // Longer: 512 x 32 22.5, 14.9; 512 x 96 (1.5) 37.3, 33.7; 512 x 112 39.3, 40.9; 512 x 128 (2) 42.0, 44.2; 512 x 136 54.8,
 // 50.8; 512 x 160 (2.5) 55.9, 53.5; 512 x 176 57.5, 60.8; 512 x 208 (3.25) 70.4, 70.3.  4096 x 4 (0.5) 118, + 75.5; 2048 x 24
 // (1.5) 110, + 103; 2048 x 28 118, + 126; 2048 x 32 (2) 128, + 134; 2048 x 40 (2.5) 173, + 168; 2048 x 44 179, + 190; 4096 x
@@ -252,7 +254,7 @@ FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bo
   if (causal) return n <= 512 ? blocks <= 10 * places && blocks * n <= places * (2L * n + 256) : blocks < 2 * places;
   if (n <= 256) {
     if (4 * blocks > 3 * places && blocks <= places)  // two rounds either way
-      return n <= 56 || (n <= 64 && 20 * blocks <= 19 * places) || (n >= 128 && n <= 192);
+      return n <= 56 || (n <= 64 && 20 * blocks <= 19 * places) || n >= 128;
     return 2 * blocks <= (n <= 60 ? 15 : 8) * places && blocks * n <= places * (n + 384L);
   }
   const long left = 2 * blocks % places;

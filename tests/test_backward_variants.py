@@ -484,13 +484,14 @@ def test_one_launch_only_where_it_is_faster(tmp_path):
         (128, 64, 256, 0), (128, 64, 512, 0), (128, 77, 136, 0), (128, 100, 256, 0), (128, 120, 141, 0), (128, 110, 512, 0),
         (128, 128, 141, 0), (128, 128, 410, 0), (128, 140, 128, 0), (128, 200, 141, 0), (128, 40, 486, 1), (128, 300, 90, 1),
         (64, 64, 512, 0), (64, 64, 3584, 0), (64, 80, 448, 0), (64, 100, 512, 0), (64, 120, 512, 0), (64, 80, 2560, 0),
-        (64, 5, 5120, 0), (64, 210, 250, 0), (64, 512, 128, 0), (64, 5, 8192, 1),
+        (64, 5, 5120, 0), (64, 512, 128, 0), (64, 5, 8192, 1),
     ]
     faster_at_once = [
         (128, 33, 256, 0), (128, 64, 230, 0), (128, 110, 128, 0), (128, 77, 384, 0), (128, 128, 192, 0), (128, 128, 512, 0),
         (128, 140, 166, 0), (128, 256, 192, 0), (128, 64, 512, 1), (128, 24, 410, 1), (128, 200, 192, 1), (128, 1031, 28, 1),
         (64, 48, 512, 0), (64, 64, 486, 0), (64, 120, 384, 0), (64, 120, 538, 0), (64, 128, 512, 0), (64, 24, 3840, 0),
-        (64, 128, 2048, 0), (64, 512, 96, 0), (64, 1, 4096, 1), (64, 140, 900, 1), (64, 1024, 64, 1),
+        (64, 128, 2048, 0), (64, 204, 256, 0), (64, 220, 243, 0), (64, 512, 96, 0), (64, 1, 4096, 1), (64, 140, 900, 1),
+        (64, 1024, 64, 1),
     ]
     assert not any(abi.host_rule(tmp_path, rule, faster_apart))
     assert all(abi.host_rule(tmp_path, rule, faster_at_once))
@@ -499,14 +500,14 @@ def test_one_launch_only_where_it_is_faster(tmp_path):
 ONE_LAUNCH = {  # B, H, N, causal by head size and by what fused_mha_backward does
     (64, "one launch, statistics made by the blocks"): [
         (1, 1, 1, False), (3, 5, 64, True), (2, 3, 65, False), (1, 3, 512, False), (2, 4, 511, True), (1, 5, 1024, True),
-        (16, 40, 129, False), (1, 70, 1000, True), (1, 480, 60, False), (1, 900, 127, False),
+        (16, 40, 129, False), (1, 70, 1000, True), (1, 480, 60, False), (1, 900, 127, False), (1, 250, 193, False),
     ],
     (64, "one launch behind the kernel for the statistics"): [
         (1, 3, 513, False), (2, 2, 1025, True), (1, 5, 1031, False), (1, 3, 1536, True), (3, 20, 1031, False),
     ],
     (64, "the passes one after the other"): [
         (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False), (1, 3900, 33, False), (1, 512, 64, False),
-        (1, 500, 65, False), (1, 250, 193, False), (1, 3100, 65, True), (1, 600, 511, True), (1, 120, 1031, True),
+        (1, 500, 65, False), (1, 800, 193, False), (1, 3100, 65, True), (1, 600, 511, True), (1, 120, 1031, True),
     ],
     (128, "one launch, statistics made by the blocks"): [
         (1, 1, 1, True), (3, 5, 33, False), (2, 3, 64, True), (2, 3, 65, False), (1, 100, 128, True), (3, 100, 77, False),
