@@ -112,16 +112,18 @@ FMHA_HOST_DEVICE bool fmha_persistent_forward_pays(int slices, int n, int cus, b
   return (left == 0 || 2 * left > round) && (total + cus - 1) / cus <= (rows + round - 1) / round;
 }
 
-// Which MFMAs both passes of the D = 128 backward use, the same in both, since it decides the order of dS in the workspace:
-// 16 x 16 where the chip runs at its power cap, 32 x 32 where a good part of the CUs has nothing to do and a wave's own
-// instructions are what takes the time.  us of the dK/dV pass with 32 x 32 and with 16 x 16 MFMAs, N x slices (blocks per
-// CU): without a mask 1031 x 16 31.4, 33.1 (0.56); 4096 x 5 105.8, 104.2 (0.63); 1031 x 20 33.9, 33.8 (0.70); 1031 x 28
-// 41.8, 41.2; 4096 x 8 139, 134 (1); 512 x 64 25.2, 24.0.  Causal, where a block is half as much work: 4096 x 6 94.0, 100.8
-// (0.75); 16384 x 2 398, 405 (1); 4096 x 10 111.1, 111.2 (1.25); 16384 x 3 477, 469 (1.5); 2048 x 32 83.7, 80.1 (2); 2048 x
-// 80 212, 201.  dQ pass over dS: 1031 x 8 11.5, 12.8; 4096 x 4 causal 33.0, 35.6; 1031 x 60 42, 40.5; 2048 x 80 causal 97,
-// 88.
+// Which MFMAs both passes of the D = 128 backward use, the same in both, since it decides the order of dS in the workspace: 16
+// x 16 where the chip runs at its power cap, 32 x 32 where a good part of the CUs has nothing to do and a wave's own
+// instructions are what takes the time.  Only passes called one by one have so few blocks: fused_mha_backward sends those into
+// one launch, with 32 x 32 MFMAs, up to the same number of blocks or more (fmha_passes_at_once).  us of the backward
+// (statistics, both passes, dS stored) with 32 x 32 and with 16 x 16 MFMAs, N x slices (blocks per CU): without a mask 4096 x
+// 2 (0.25) 125, 130; 1031 x 9 (0.32) 45.9, 46.7; 4096 x 4 (0.5) 132, 134; 1031 x 15 (0.53) 47.1, 47.6; 1024 x 18 (0.56) 47.3,
+// 46.8; 2048 x 9 76.6, 76.9; 1024 x 19 (0.59) 48.9, 47.9; 4096 x 5 (0.63) 145, 140; 2048 x 10 80.2, 78.3; 1031 x 20 (0.7)
+// 52.9, 50.6; 512 x 64 (1) 43.8, 40.1; 1024 x 32 66.3, 59.7.  Causal, where a block is half as much work: 8192 x 2 (0.5) 236,
+// 246; 4096 x 6 (0.75) 134, 135; 2048 x 14 (0.88) 78.8, 79.5; 1031 x 28 (0.98) 52.5, 52.3; 2048 x 16 (1) 82.1, 82.2; 4096 x 8
+// 147, 146; 2048 x 18 (1.13) 88.0, 86.3; 4096 x 10 (1.25) 163, 160; 4096 x 12 (1.5) 182, 176.
 FMHA_HOST_DEVICE bool fmha_wide_mfmas(long key_blocks, int cus, bool causal) {  // blocks of 128 keys of a launch
-  return key_blocks * (causal ? 1 : 2) * 4 < 5L * cus;
+  return key_blocks * (causal ? 1 : 2) <= cus;
 }
 
 // Launches of one block per work group that the hardware hands out as CUs become free, two or more to a CU.

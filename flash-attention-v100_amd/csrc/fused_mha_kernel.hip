@@ -1977,7 +1977,7 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // query 16 * (g >> 1) + 8 * (e >> 2) + 4 * (g & 1) + (e & 3).  Rows of keys at or past n are written as zeros; (key tile,
 // query tile) pairs above the diagonal are not written (and not read) under causal masking.
 // KEEP: without the non-temporal hint on those stores (rule: fmha_ds_used_once).
-// WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: launch_backward).
+// WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: fmha_wide_mfmas).
 // STATS: the row statistics of every tile are formed here, from O, dO and LSE, a tile ahead; delta and lse2 are not read.
 constexpr int kKvStBytes = 1024;
 template <int D>

@@ -124,7 +124,7 @@ EITHER_MFMA = [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200]
 
 
 def _slices_of_a_busy_launch(N, causal, cus):
-    return -(-5 * cus // (4 if causal else 8) // (-(-N // 128))) + 1
+    return cus // (1 if causal else 2) // (-(-N // 128)) + 1
 
 
 def test_mfmas_of_the_cases_below(tmp_path):
@@ -220,14 +220,14 @@ DS_IN_ONE_CALL = [(260, 300), (130, 600), (50, 300), (100, 300)]  # H, N: dS is 
 
 
 def test_dS_in_one_call(tmp_path):
-    """Of the cases below on 256 compute units, and that it is by passes with 32 x 32 MFMAs too."""
-    expression = "!fmha_passes_at_once(128, (long)((x[1] + 127) / 128) * x[0], x[1], 256, x[2])"
+    """Of the cases below on 256 compute units, which are by passes with 16 x 16 MFMAs then: no call stores dS by the others."""
+    at_once = "fmha_passes_at_once(128, (long)((x[1] + 127) / 128) * x[0], x[1], 256, x[2])"
     wide = "fmha_wide_mfmas((long)((x[1] + 127) / 128) * x[0], 256, x[2])"
     no_mask, causal = ([(*case, mask) for case in DS_IN_ONE_CALL] for mask in (0, 1))
-    assert abi.host_rule(tmp_path, expression, no_mask) == [True] * 4
-    assert abi.host_rule(tmp_path, expression, causal) == [True, True, False, True]
-    assert abi.host_rule(tmp_path, wide, no_mask) == [False, False, True, False]
-    assert abi.host_rule(tmp_path, wide, causal) == [False, False, True, True]
+    assert abi.host_rule(tmp_path, at_once, no_mask) == [False] * 4
+    assert abi.host_rule(tmp_path, at_once, causal) == [False, False, True, False]
+    every = [(H, N, mask) for N in (1, 20, 40, 64, 65, 128, 129, 200, 256, 257, 1031, 4096) for H in range(1, 600) for mask in (0, 1)]
+    assert not any(abi.host_rule(tmp_path, f"!{at_once} && {wide}", every))
 
 
 @pytest.mark.gpu
@@ -241,7 +241,7 @@ def test_dq_ignores_dS_that_no_query_needs(H, N, causal):
     q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
     out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
     want = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, min_workspace=True)[:3]
-    for split in (True, False):
+    for split in (True, False):  # H = 3 one by one: 32 x 32 MFMAs
         got = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=split, poison=True)[:3]
         for a, b in zip(got, want):
             assert torch.equal(a, b)

@@ -426,7 +426,7 @@ def test_full_launches_take_the_kernels_they_are_meant_for(tmp_path):
     shapes = [(B * H, N, causal) for B, H, N, causal in FULL_LAUNCHES]
     assert not any(abi.host_rule(tmp_path, wide, shapes))
     assert abi.host_rule(tmp_path, "fmha_persistent_forward_pays(x[0], x[1], 256, x[2])", shapes) == [True] * 3 + [False] * 2
-    assert all(abi.host_rule(tmp_path, wide, [(31, 520, False), (63, 520, True), (4, 320, True)]))
+    assert all(abi.host_rule(tmp_path, wide, [(25, 520, False), (51, 520, True), (4, 320, True)]))
 
 
 def test_interleaved_blocks_are_a_bijection(tmp_path):
