@@ -276,19 +276,20 @@ FMHA_HOST_DEVICE bool fmha_blocks_make_stats(int d, int n, bool causal) {
 
 // Whether the D = 128 passes over dS are told that it is used once.  Without that dS stays in the 256 MiB Infinity Cache
 // between the two: better where it fits together with the six tensors the passes touch, and is not small.  Small is less than
-// 16 MiB without a mask up to 256 rows, 8 MiB (of half the square) under causal masking and 10 MiB else.  Fewer blocks than
+// 16 MiB without a mask up to 384 rows, 8 MiB (of half the square) under causal masking and 10 MiB else.  Fewer blocks than
 // those of the figures go in one launch that stores no dS, unless the passes are called one by one, as the ones with "*" are.
 // us of the backward without and with the hint, N x slices (MiB of dS; with the tensors):
-// Lower line: 66 x 230 (7; 29) 20.3, 19.0; 110 x 256 (8; 49) 24.7, 24.4; 77 x 430 (13; 62) 36.5, 35.9; 140 x 79 (10; 26)
-// 20.7, 20.3; 140 x 120 (15; 40) 23.2, 22.3; 200 x 110 (14; 46) 26.8, 26.5; 256 x 100 (13; 50) 27.0, 26.8; 256 x 128 (16; 64)
-// 30.4, 30.7; 200 x 135 (17; 56) 42.1, 42.2; 110 x 520 (16; 100) 57.6, 58.5; 128 x 520 (16; 114) 61.3, 62.6; 350 x 86 (24;
-// 68) 51.8, 53.6; causal 33 x 500 (8; 32) 24.0, 23.5; 50 x 500 (8; 44) 26.7, 26.5; 64 x 530 (8; 58) 43.4, 43.4; 128 x 513 (8;
-// 104) 59.3, 61.0; 128 x 600 (9; 122) 64.3, 65.3; 512 x 75 (19; 75) 45.0, 47.7.  Forward and backward: 512 x 16 * (8; 20)
-// 40.8, 39.8; 1024 x 5 * (10; 18) 59.8, 61.8.
+// Lower line: 66 x 230 (7; 29) 20.3, 19.0; 110 x 256 (8; 49) 24.7, 24.4; 77 x 430 (13; 62) 36.5, 35.9; 140 x 79 (10; 26) 20.7,
+// 20.3; 140 x 120 (15; 40) 23.2, 22.3; 200 x 110 (14; 46) 26.8, 26.5; 256 x 100 (13; 50) 27.0, 26.8; 256 x 128 (16; 64) 30.4,
+// 30.7; 257 x 46 (13; 30) 25.2, 24.2; 384 x 46 (13; 39) 28.2, 27.9; 384 x 64 (18; 54) 29.9, 29.9; 384 x 85 (24; 72) 33.3,
+// 34.0; 200 x 135 (17; 56) 42.1, 42.2; 110 x 520 (16; 100) 57.6, 58.5; 128 x 520 (16; 114) 61.3, 62.6; 350 x 86 (24; 68) 51.8,
+// 53.6; causal 33 x 500 (8; 32) 24.0, 23.5; 50 x 500 (8; 44) 26.7, 26.5; 64 x 530 (8; 58) 43.4, 43.4; 128 x 513 (8; 104) 59.3,
+// 61.0; 128 x 600 (9; 122) 64.3, 65.3; 512 x 75 (19; 75) 45.0, 47.7.  Forward and backward: 512 x 16 * (8; 20) 40.8, 39.8;
+// 1024 x 5 * (10; 18) 59.8, 61.8.
 // Upper line, forward and backward: 1031 x 60 (152; 243) 203, 207; 4096 x 11 causal (176; 242) 240, 254; 512 x 224 (112; 280)
 // 185, 179; 1024 x 88 (176; 308) 237, 227; 4096 x 16 causal (256; 352) 305, 300; 4096 x 64 causal (1024; 1408) 1217, 1161.
 FMHA_HOST_DEVICE bool fmha_ds_used_once(unsigned long ds_bytes, unsigned long touched, int n, bool causal) {
-  const unsigned long small = causal ? 8 : n <= 256 ? 16 : 10;  // MiB
+  const unsigned long small = causal ? 8 : n <= 384 ? 16 : 10;  // MiB
   return ds_bytes < (small << 20) || touched > (256ul << 20);
 }
 

@@ -250,6 +250,7 @@ def test_dq_ignores_dS_that_no_query_needs(H, N, causal):
 HINT_ON_DS = [  # H, N, causal, whether the passes are called one by one, whether dS is told to be used once
     (127, 256, False, False, True), (128, 256, False, False, False),   # 15.9 and 16 MiB of dS
     (511, 127, False, False, True), (512, 127, False, False, False),
+    (56, 384, False, False, True), (57, 384, False, False, False),     # 15.8 and 16.03
     (511, 50, True, False, True), (513, 50, True, False, False),       # 7.98 and 8.02 MiB
     (4, 1024, False, True, True), (5, 1024, False, True, False),       # 8 and 10 MiB
     (5, 1025, True, True, True), (9, 1025, True, True, False),         # 6.3 and 11.4 MiB
