@@ -1426,9 +1426,10 @@ constexpr int kDqBlockQ = kDqPairs * kResident;
 
 // STATS: the kernel also produces the two row statistics of the backward,
 // delta = rowsum(dO o O) and lse2 = lse * log2(e), for its own queries, uses
-// them and stores them in the workspace for the dK/dV pass (which must then be
-// launched after this one); fmha_bwd_delta_kernel is not needed in that case.
-// Otherwise delta is read from the workspace.
+// them and stores them in the workspace; fmha_bwd_delta_kernel is not needed in
+// that case.  A dK/dV pass that reads them must be launched after this one; the
+// dK/dV blocks that share a launch with these (fmha_bwd_both_kernel) form their
+// own.  Otherwise delta is read from the workspace.
 template <int D>
 constexpr int dq_lds() { return 7 * SwzTile<D>::kBytes + 2 * kDqPairs * 4096; }
 template <int D, bool CAUSAL, bool STATS>
@@ -2065,8 +2066,8 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
 
   // resident rows of this wave: K for role A, V for role B; [feature step] of key k0w + i, or [feature step][cb] of keys
   // k0w + 16 cb + i.  They and the first tile are all that the loops need to start; the second tile is asked for when these
-  // are there, not waited for with them (B3 H20 N1031 step 193.9 -> 192.7 us, B2 H40 N2048 causal 434.6 -> 432.0, B2 H32 N4096
-  // causal 1129 -> 1125).
+  // are there, not waited for with them.  What that gives, 0.2 to 0.8 % of B3 H20 N1031, B2 H40 N2048 causal and B2 H32 N4096
+  // causal, is within what runs of one side differ by.
   h8 rf[G::kKSteps];
 #pragma unroll
   for (int cb = 0; cb < (WIDE ? 1 : 2); ++cb) {
@@ -3501,9 +3502,10 @@ int fused_mha_backward_noalloc(const void* query_ptr, const void* key_ptr, const
   if (rows > (size_t)FUSED_MHA_NOALLOC_MAX_ROWS) return FUSED_MHA_ERR_SCRATCH_LIMIT;
   void* ws = nullptr;
   if (int rc = scratch_for_device(&ws)) return rc;
-  // Every workspace element the dK/dV pass reads is written by the dQ pass of
-  // the same call (rows 0 .. batch*head*n-1 of both halves), so nothing from
-  // an earlier call is ever read and nothing needs clearing.
+  // Every workspace element that a pass reads is written before it by the same
+  // call, by the dQ pass or the kernel for the statistics (rows 0 ..
+  // batch*head*n-1 of both halves; launches whose blocks all make their own read
+  // none), so nothing from an earlier call is ever read and nothing needs clearing.
   return dispatch_backward(kPassAll, query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr,
                            d_output_ptr, nullptr, lse_ptr, ws, 2 * rows * sizeof(float), d_query_ptr, d_key_ptr,
                            d_value_ptr, batch, head, m, n, d, scale, causal, stream);

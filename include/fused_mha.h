@@ -122,8 +122,11 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  *     the minimum where that does not hold one slice (n > 92672).
  * Problems of so few blocks of 128 rows that neither pass fills the device
  * (with d = 128 at most one per compute unit under causal masking, one for two
- * without; somewhat more up to n = 256) need no room for dS: there both passes
- * go into one launch and form S and dP twice, whatever the size.
+ * without; somewhat more up to n = 256) use no room for dS: there both passes
+ * go into one launch and form S and dP twice, whatever the size.  That depends
+ * on the mask and the device, which this function does not know, so it returns
+ * room for dS for those too (2 GiB for one causal slice of n = 32768); the
+ * minimum is as fast for them.
  * A caller that wants to spend less passes any size from the minimum on.
  * Both functions return 0 for an invalid shape.  No counterpart in the
  * reference, which receives delta from Python (flash_attn_interface.py:43-44).
