@@ -205,12 +205,12 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 // than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few
 // more, each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together
 // it saves one start and one end, and pays for the statistics, which the D = 64 dQ pass makes on the side when it goes first,
-// or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  Timed both ways, 9,700 launches of 108
-// lengths lose 0.2 to 0.7 % on average against the better way, D = 128 without a mask 1.1 % before the lines were drawn between
-// lengths of 128 x 2^k; most of that is one launch being faster past the lines (128 x 537 at D = 128, 128 x 3584 at D = 64:
-// 0.8 of the time).  us of the launches one after the other, and of one with the statistics made by the
-// blocks or, behind "+", by a kernel of their own first (fmha_blocks_make_stats), N x slices (blocks per CU), on both sides
-// of the lines:
+// or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  Of 9,620 launches of 107 lengths timed
+// both ways the rule loses 0.2 to 0.6 % on average against the better way (D = 128 without a mask 0.2; 1.1 with lines that had
+// been read off lengths of 128 x 2^k), nearly all of it past the rounds it goes to, where the one launch would be ahead (128 x
+// 537 at D = 128, 128 x 3584 at D = 64: 0.8 of the time).  us of the launches one after the other, and of one with the
+// statistics made by the blocks or, behind "+", by a kernel of their own first (fmha_blocks_make_stats), N x slices (blocks
+// per CU), on both sides of the lines:
 // D = 64, without a mask, up to 256 rows.  56 x 512 (2) equal, 48 x 512 13.8, 12.5; 64 x 486 (1.9) 14.3, 13.5; 64 x 512 14.0,
 // 15.0; 80 x 384 (1.5) 17.2, 16.2; 80 x 448 (1.75) 17.7, 18.7; 120 x 384 19.7, 19.2; 120 x 512 22.0, 23.9; 120 x 538 (2.1)
 // 28.9, 24.8; 128 x 512 23.0, 20.6; 192 x 256 (2) 24.0, 24.0; 204 x 256 30.7, 29.0; 216 x 256 30.5, 29.9; 255 x 256 equal.
