@@ -239,7 +239,11 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 // 129 x 128 (1) 21.7, 21.5; 129 x 192 33.0, 30.5; 200 x 192 (1.5) 41.5, 35.9; 200 x 218 42.2, 43.3; 512 x 64 (1) 37.7, +
 // 34.2; 512 x 68 41.5, + 43.2; 777 x 33 (0.9) 42.0, + 37.8; 2048 x 16 (1) 84.9, + 76.0; 2048 x 18 91.6, + 89.2; 2048 x 20
 // 91.1, + 98.1; 4096 x 8 (1) 153, + 133; 4096 x 10 159, + 169; 8192 x 5 315, + 318.
-FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bool causal) {
+// room: whether the workspace holds dS.  If not, the D = 128 passes one after the other form S and dP twice as well, and
+// without a mask every round saved counts: 128 x 396 (1.55) 45.2, 41.5; 160 x 192 (1.5) 41.6, 36.7; 230 x 192 50.4, 47.8; 1031
+// x 42 121, 106; 4096 x 9 (1.1) 388, 318; 16384 x 3 1554, 1326.  Under causal masking the lines are those with room, though
+// the one launch is ahead past them: 1024 x 48 (1.5) 76.8, 72.1; 1024 x 64 (2) equal; 2048 x 24 117, 108.
+FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bool causal, bool room = true) {
   if (d == 128) {
     if (blocks > 2L * cus) return false;
     if (causal) {
@@ -247,10 +251,10 @@ FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bo
       return 2 * blocks <= 3L * cus || n <= 24 || (n >= 52 && n <= 128);
     }
     if (2 * blocks <= cus) return true;                                      // one round instead of two
-    if (blocks > cus && 2 * blocks <= 3L * cus) return n < 160 || n == 256;  // three rounds instead of four
+    if (blocks > cus && 2 * blocks <= 3L * cus) return n < 160 || n == 256 || !room;  // three rounds instead of four
     if (n <= 64) return 10 * blocks <= (n <= 48 ? 10L : 9L) * cus;
     const long left = 2 * blocks % cus;
-    return n == 128 && (left == 0 || 2 * left >= cus);
+    return n == 128 && (left == 0 || 2 * left >= cus || !room);
   }
   const long places = 2L * cus;
   if (causal) return n <= 512 ? blocks <= 10 * places && blocks * n <= places * (2L * n + 256) : blocks < 2 * places;

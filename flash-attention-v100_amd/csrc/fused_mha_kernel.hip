@@ -3278,7 +3278,7 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   };
   const float c = scale * kLog2e;
   const int nb = (n + 127) / 128;
-  if ((passes & kPassAll) == kPassAll && fmha_passes_at_once(D, (long)nb * slices, n, cus, CAUSAL)) {
+  if ((passes & kPassAll) == kPassAll && fmha_passes_at_once(D, (long)nb * slices, n, cus, CAUSAL, spill)) {
     const bool stats = fmha_blocks_make_stats(D, n, CAUSAL);
     if (!stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
     auto both = [&](auto kernel, int threads) {

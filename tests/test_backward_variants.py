@@ -496,6 +496,13 @@ def test_one_launch_only_where_it_is_faster(tmp_path):
     ]
     assert not any(abi.host_rule(tmp_path, rule, faster_apart))
     assert all(abi.host_rule(tmp_path, rule, faster_at_once))
+    without_room = rule.replace("x[3])", "x[3], false)")  # for dS
+    faster_at_once = [(128, 128, 396, 0), (128, 160, 192, 0), (128, 230, 166, 0), (128, 192, 132, 0), (128, 1031, 42, 0)]
+    faster_apart = [(128, 64, 256, 0), (128, 110, 256, 0), (128, 120, 141, 0), (128, 230, 256, 0),
+                    (128, 40, 486, 1), (128, 1024, 20, 0), (128, 4096, 15, 0)]
+    assert not any(abi.host_rule(tmp_path, rule, faster_at_once))
+    assert all(abi.host_rule(tmp_path, without_room, faster_at_once))
+    assert not any(abi.host_rule(tmp_path, without_room, faster_apart))
 
 
 ONE_LAUNCH = {  # B, H, N, causal by head size and by what fused_mha_backward does
@@ -521,6 +528,7 @@ ONE_LAUNCH = {  # B, H, N, causal by head size and by what fused_mha_backward do
     (128, "the passes one after the other"): [
         (5, 100, 77, False), (1, 140, 250, False), (1, 70, 250, False), (1, 70, 400, True), (1, 20, 1031, False),
         (1, 400, 33, False), (1, 513, 64, True), (1, 400, 40, True), (1, 150, 65, False), (1, 140, 128, False),
+        (1, 396, 128, False), (1, 192, 160, False), (1, 90, 300, False), (1, 31, 1031, False),  # one launch without room for dS
     ],
 }
 
