@@ -3135,7 +3135,8 @@ bool bad_strides(const fused_mha_strides* st) {
 // blocks run beside the others.  us without and with that, D = 64, N x slices (rounds), forward, then backward: 1024 x 66
 // (1.03) 31.1, 29.6; 92.1, 90.6.  1024 x 96 (1.5) 34.3, 33.1; 102.8, 102.7.  2048 x 40 (1.25) 56.2, 53.3; 174, 170.  8192 x 12
 // (1.5) 218, 211; 725, 703.  2048 x 66 (2.06) 89.7, 88.7; 279, 271.  1024 x 160 (2.5) 54.7, 55.2; 166, 164.  2048 x 80 (2.5)
-// 96.7, 96.8; 300, 297.  Forward D = 128: 1031 x 60 (1.05) 48.9, 46.8; 2048 x 40 91.8, 90.1; 4096 x 20 174, 170.
+// 96.7, 96.8; 300, 297.  (Backwards of 1 to 1.25 rounds go in one launch, unless their passes are called one by one:
+// fmha_passes_at_once.)  Forward D = 128: 1031 x 60 (1.05) 48.9, 46.8; 2048 x 40 91.8, 90.1; 4096 x 20 174, 170.
 // Short blocks have nothing to gain (512 x 192: 21.6, 21.5; 61.1, 62.2.  256 x 320: 14.1, 14.3; 39.2, 39.4), nor has a fuller
 // last round (1024 x 112, 1.75: 41.2, 42.2; dK/dV 69.1, 70.1.  1024 x 192, 3: 65.5, 65.6; dK/dV 110, 118), nor more rounds
 // (1024 x 288, 4.5: 96.9, 98.4), nor a causal launch, where the blocks differ (1024 x 64 forward: 16.4, 18.2).
