@@ -114,16 +114,18 @@ FMHA_HOST_DEVICE bool fmha_persistent_forward_pays(int slices, int n, int cus, b
 
 // Which MFMAs both passes of the D = 128 backward use, the same in both, since it decides the order of dS in the workspace: 16
 // x 16 where the chip runs at its power cap, 32 x 32 where a good part of the CUs has nothing to do and a wave's own
-// instructions are what takes the time.  Only passes called one by one have so few blocks: fused_mha_backward sends those into
-// one launch, with 32 x 32 MFMAs, up to the same number of blocks or more (fmha_passes_at_once).  us of the backward
-// (statistics, both passes, dS stored) with 32 x 32 and with 16 x 16 MFMAs, N x slices (blocks per CU): without a mask 4096 x
-// 2 (0.25) 125, 130; 1031 x 9 (0.32) 45.9, 46.7; 4096 x 4 (0.5) 132, 134; 1031 x 15 (0.53) 47.1, 47.6; 1024 x 18 (0.56) 47.3,
-// 46.8; 2048 x 9 76.6, 76.9; 1024 x 19 (0.59) 48.9, 47.9; 4096 x 5 (0.63) 145, 140; 2048 x 10 80.2, 78.3; 1031 x 20 (0.7)
-// 52.9, 50.6; 512 x 64 (1) 43.8, 40.1; 1024 x 32 66.3, 59.7.  Causal, where a block is half as much work: 8192 x 2 (0.5) 236,
-// 246; 4096 x 6 (0.75) 134, 135; 2048 x 14 (0.88) 78.8, 79.5; 1031 x 28 (0.98) 52.5, 52.3; 2048 x 16 (1) 82.1, 82.2; 4096 x 8
-// 147, 146; 2048 x 18 (1.13) 88.0, 86.3; 4096 x 10 (1.25) 163, 160; 4096 x 12 (1.5) 182, 176.
+// instructions are what takes the time.  fused_mha_backward has so few blocks only without a mask, from one for two CUs on:
+// fewer, and all under causal masking, go in one launch, with 32 x 32 MFMAs (fmha_passes_at_once), unless the passes are
+// called one by one.  us of the backward (statistics, both passes, dS stored) with 32 x 32 and with 16 x 16 MFMAs, N x slices
+// (blocks per CU): without a mask 4096 x 2 (0.25) 125, 130; 1031 x 9 (0.32) 45.9, 46.7; 4096 x 4 (0.5) 132, 134; 1031 x 15
+// (0.53) 47.1, 47.6; 1024 x 18 (0.56) 47.3, 46.8; 2048 x 9 76.6, 76.9; 1024 x 19 (0.59) 48.9, 47.9; 4096 x 5 (0.63) 145, 140;
+// 2048 x 10 80.2, 78.3; 1031 x 20 (0.7) 52.9, 50.6; 512 x 64 (1) 43.8, 40.1; 1024 x 32 66.3, 59.7; 32 x 32 ahead by 0.7 % in
+// the median of 11 more lengths between 0.5 and 0.63, by 0.4 % of 31 without room for dS (1439 x 13 75.2, 76.4).  Causal,
+// where a block is half as much work: 8192 x 2 (0.5) 236, 246; 4096 x 6 (0.75) 134, 135; 2048 x 14 (0.88) 78.8, 79.5; 1031 x
+// 28 (0.98) 52.5, 52.3; 2048 x 16 (1) 82.1, 82.2; 4096 x 8 147, 146; 2048 x 18 (1.13) 88.0, 86.3; 4096 x 10 (1.25) 163, 160;
+// 4096 x 12 (1.5) 182, 176.
 FMHA_HOST_DEVICE bool fmha_wide_mfmas(long key_blocks, int cus, bool causal) {  // blocks of 128 keys of a launch
-  return key_blocks * (causal ? 1 : 2) <= cus;
+  return causal ? key_blocks <= cus : 8 * key_blocks < 5L * cus;
 }
 
 // Launches of one block per work group that the hardware hands out as CUs become free, two or more to a CU.
@@ -202,21 +204,23 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 }
 
 // Whether the backward does both passes, `blocks` blocks of 128 rows each, in one launch of 2 * blocks.  With fewer blocks
-// than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few
-// more, each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together
-// it saves one start and one end, and pays for the statistics, which the D = 64 dQ pass makes on the side when it goes first,
-// or, at D = 128, for forming S and dP twice; most where the last tile is not whole.  Of 9,620 launches of 107 lengths timed
-// both ways the rule loses 0.2 to 0.6 % on average against the better way (D = 128 without a mask 0.2; 1.1 with lines that had
-// been read off lengths of 128 x 2^k), nearly all of it past the rounds it goes to, where the one launch would be ahead (128 x
-// 537 at D = 128, 128 x 3584 at D = 64: 0.8 of the time).  us of the launches one after the other, and of one with the
-// statistics made by the blocks or, behind "+", by a kernel of their own first (fmha_blocks_make_stats), N x slices (blocks
-// per CU), on both sides of the lines:
-// D = 64, without a mask, up to 256 rows.  56 x 512 (2) equal, 48 x 512 13.8, 12.5; 64 x 486 (1.9) 14.3, 13.5; 64 x 512 14.0,
-// 15.0; 80 x 384 (1.5) 17.2, 16.2; 80 x 448 (1.75) 17.7, 18.7; 120 x 384 19.7, 19.2; 120 x 512 22.0, 23.9; 120 x 538 (2.1)
-// 28.9, 24.8; 128 x 512 23.0, 20.6; 192 x 256 (2) 24.0, 24.0; 204 x 256 30.7, 29.0; 216 x 256 30.5, 29.9; 255 x 256 equal.
-// Many blocks: 24 x 3840 (15) 58.8, 58.5; 24 x 5120 75.4, 76.7; 40 x 3840 64.7, 63.3; 40 x 4096 (16) 68.5, 71.6; 64 x 2048 (8)
-// 44.3, 42.9; 64 x 2432 53.0, 55.1; 64 x 3584 69.4, 74.5; 80 x 2048 56.4, 57.6; 80 x 2560 68.5, 71.9; 128 x 2048 74.4, 69.3;
-// 256 x 640 (5) 64.6, 60.4; 256 x 768 73.3, 77.0.
+// than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few more,
+// each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together it
+// saves launches, and pays for the statistics, which the D = 64 dQ pass makes on the side when it goes first, or, at D = 128,
+// for forming S and dP twice; most where the last tile is not whole.  The launches it saves are one at D = 64, two and the
+// room for dS at D = 128: 4 and 7 us of the host, and a program that calls these functions from Python waits for the host
+// unless forward and backward have 40 us of kernels or, more often, 70.  us of the two through autograd, one launch and apart:
+// D = 128 N = 64 x 256 slices 71, 79 (kernels of the backward 16.9, 15.5); 100 x 256 73, 79; 40 x 448 73, 79; 100 x 448 75, 80
+// (kernels 44.4, 39.6); 180 x 192 73, 80; causal 40 x 480 73, 79; D = 64 64 x 512 72, 77; 80 x 448 73, 76.  So short launches
+// go in one also where their kernels lose by it, up to 3 us, and at D = 128 without a mask from 65 to 127 rows past one and a
+// half blocks per CU 4 to 8; the lines lie where a call waits for its kernels, or where they lose more.
+// us of the kernels one after the other, and of one launch with the statistics made by the blocks or, behind "+", by a kernel
+// of their own first (fmha_blocks_make_stats), N x slices (blocks per CU), on both sides of the lines:
+// D = 64, without a mask, up to 256 rows.  64 x 512 (2) 14.0, 15.0; 80 x 448 (1.75) 17.7, 18.7; 120 x 512 22.0, 23.9; 120 x
+// 538 (2.1) 28.9, 24.8; 128 x 512 23.0, 20.6; 204 x 256 30.7, 29.0; 255 x 256 equal.  Many blocks: 24 x 3840 (15) 58.8, 58.5;
+// 24 x 5120 75.4, 76.7; 40 x 3840 64.7, 63.3; 40 x 4096 (16) 68.5, 71.6; 64 x 2048 (8) 44.3, 42.9; 64 x 2432 53.0, 55.1; 64 x
+// 3584 69.4, 74.5; 80 x 2048 56.4, 57.6; 80 x 2560 68.5, 71.9; 128 x 2048 74.4, 69.3; 256 x 640 (5) 64.6, 60.4; 256 x 768
+// 73.3, 77.0.
 // Longer: 512 x 32 22.5, 14.9; 512 x 96 (1.5) 37.3, 33.7; 512 x 112 39.3, 40.9; 512 x 128 (2) 42.0, 44.2; 512 x 136 54.8,
 // 50.8; 512 x 160 (2.5) 55.9, 53.5; 512 x 176 57.5, 60.8; 512 x 208 (3.25) 70.4, 70.3.  4096 x 4 (0.5) 118, + 75.5; 2048 x 24
 // (1.5) 110, + 103; 2048 x 28 118, + 126; 2048 x 32 (2) 128, + 134; 2048 x 40 (2.5) 173, + 168; 2048 x 44 179, + 190; 4096 x
@@ -225,44 +229,35 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 // 320 (5) 69.5, 66.3; 450 x 352 72.5, 73.3; 512 x 512 (8) 110, 117; 777 x 144 (3.95) 70.4, 66.3; 1024 x 32 37.9, 27.3; 1024 x
 // 128 (4) 86.3, 85.7; 2048 x 32 (2) 79.9, + 74.3; 2048 x 60 136, + 135; 2048 x 64 (4) 141, + 145; 8192 x 8 (2) 283, + 256;
 // 8192 x 15 464, + 459; 8192 x 32 946, + 963.
-// D = 128, without a mask.  33 x 128 (0.5) 14.1, 7.8; 33 x 256 (1) 14.7, 13.3; 64 x 230 (0.9) 15.8, 15.5; 64 x 256 15.5,
-// 16.9; 64 x 264 23.9, 22.5; 64 x 384 (1.5) 25.8, 24.6; 64 x 397 27.2, 30.4; 110 x 128 18.7, 13.2; 110 x 136 19.0, 22.0; 110
-// x 256 24.1, 26.1; 110 x 264 35.1, 34.8; 110 x 384 38.4, 38.1; 110 x 410 39.7, 46.1.  128 x 128 19.0, 12.2; 128 x 141 (0.55)
-// 19.6, 20.8; 128 x 192 (0.75) 22.2, 21.1; 128 x 256 24.8, 24.2; 128 x 384 40.3, 34.5; 128 x 410 41.5, 43.7; 128 x 448 (1.75)
-// 44.2, 42.6; 128 x 512 47.0, 44.8.  140 x 64 (0.5) 19.6, 12.8; 140 x 68 20.1, 20.5; 140 x 128 (1) 23.7, 24.7; 140 x 141
-// 33.2, 33.9; 140 x 166 (1.3) 35.9, 34.3; 140 x 192 37.0, 36.3; 200 x 64 22.6, 16.4; 200 x 68 22.9, 27.5; 200 x 141 41.0,
-// 42.5; 256 x 132 (1.03) 43.8, 43.0; 256 x 192 46.7, 45.4; 256 x 205 48.5, 57.3.  350 x 38 (0.45) 26.9, 20.1; 350 x 43 27.2,
-// 34.6; 1200 x 11 (0.43) 49.6, + 40.1; 1200 x 13 49.4, + 67.8; 2048 x 8 (0.5) 75.4, + 64.5; 4096 x 4 (0.5) 131, + 122; 4096 x
-// 5 145, + 209.
-// D = 128, causal.  24 x 384 (1.5) 23.1, 18.0; 24 x 410 23.3, 22.8; 24 x 486 (1.9) 22.3, 23.2; 40 x 384 24.4, 20.2; 40 x 410
-// 24.7, 25.3; 40 x 486 24.1, 25.8; 64 x 410 28.1, 27.7; 64 x 512 (2) 30.7, 28.2; 110 x 410 40.0, 40.2; 110 x 512 45.5, 43.3;
-// 129 x 128 (1) 21.7, 21.5; 129 x 192 33.0, 30.5; 200 x 192 (1.5) 41.5, 35.9; 200 x 218 42.2, 43.3; 512 x 64 (1) 37.7, +
-// 34.2; 512 x 68 41.5, + 43.2; 777 x 33 (0.9) 42.0, + 37.8; 2048 x 16 (1) 84.9, + 76.0; 2048 x 18 91.6, + 89.2; 2048 x 20
-// 91.1, + 98.1; 4096 x 8 (1) 153, + 133; 4096 x 10 159, + 169; 8192 x 5 315, + 318.
+// D = 128, without a mask.  33 x 128 (0.5) 14.1, 7.8; 33 x 256 (1) 14.7, 13.3; 64 x 256 15.5, 16.9; 64 x 264 23.9, 22.5; 64 x
+// 397 (1.55) 27.2, 30.4; 48 x 486 (1.9) 25.3, 28.4; 64 x 512 (2) 29.2, 32.1; 64 x 537 41.4, 37.2; 110 x 128 18.7, 13.2; 120 x
+// 140 (0.55) 19.8, 23.1; 110 x 256 24.1, 26.1; 110 x 384 (1.5) 38.4, 38.1; 80 x 396 33.9, 40.2; 110 x 410 39.7, 46.1; 120 x
+// 512 45.5, 50.8.  128 x 128 19.0, 12.2; 128 x 141 19.6, 20.8; 128 x 256 24.8, 24.2; 128 x 384 40.3, 34.5; 128 x 410 41.5,
+// 43.7; 128 x 512 47.0, 44.8; 128 x 537 61.2, 53.5.  140 x 64 (0.5) 19.6, 12.8; 140 x 68 20.1, 20.5; 140 x 128 (1) 23.7, 24.7;
+// 140 x 141 33.2, 33.9; 140 x 192 (1.5) 37.0, 36.3; 200 x 64 22.6, 16.4; 200 x 68 22.9, 27.5; 200 x 141 41.0, 42.5; 230 x 192
+// 47.5, 48.5; 200 x 198 (1.55) 46.4, 56.9; 256 x 132 43.8, 43.0; 256 x 192 46.7, 45.4; 256 x 205 48.5, 57.3.  350 x 38 (0.45)
+// 26.9, 20.1; 350 x 43 27.2, 34.6; 1200 x 11 (0.43) 49.6, + 40.1; 1200 x 13 49.4, + 67.8; 2048 x 8 (0.5) 75.4, + 64.5; 4096 x
+// 4 (0.5) 131, + 122; 4096 x 5 145, + 209.
+// D = 128, causal.  24 x 384 (1.5) 23.1, 18.0; 24 x 410 23.3, 22.8; 40 x 486 (1.9) 24.1, 25.8; 64 x 512 (2) 30.7, 28.2; 64 x
+// 537 43.3, 34.3; 110 x 410 40.0, 40.2; 110 x 512 45.5, 43.3; 129 x 128 (1) 21.7, 21.5; 129 x 192 33.0, 30.5; 200 x 192 (1.5)
+// 41.5, 35.9; 200 x 218 42.2, 43.3; 512 x 64 (1) 37.7, + 34.2; 512 x 68 41.5, + 43.2; 777 x 33 (0.9) 42.0, + 37.8; 2048 x 16
+// (1) 84.9, + 76.0; 2048 x 18 91.6, + 89.2; 2048 x 20 91.1, + 98.1; 4096 x 8 (1) 153, + 133; 4096 x 10 159, + 169; 8192 x 5
+// 315, + 318.
 // room: whether the workspace holds dS.  If not, the D = 128 passes one after the other form S and dP twice as well, and
-// without a mask every round saved counts: 128 x 396 (1.55) 45.2, 41.5; 160 x 192 (1.5) 41.6, 36.7; 230 x 192 50.4, 47.8; 1031
-// x 42 121, 106; 4096 x 9 (1.1) 388, 318; 16384 x 3 1554, 1326.  Under causal masking the lines are those with room, though
-// the one launch is ahead past them: 1024 x 48 (1.5) 76.8, 72.1; 1024 x 64 (2) equal; 2048 x 24 117, 108.
+// without a mask a round saved counts at any length: 1031 x 42 (1.5) 121, 106; 4096 x 9 (1.1) 388, 318; 16384 x 3 1554, 1326.
+// Under causal masking the lines are those with room, though the one launch is ahead past them: 1024 x 48 (1.5) 76.8, 72.1;
+// 1024 x 64 (2) equal; 2048 x 24 117, 108.
 FMHA_HOST_DEVICE bool fmha_passes_at_once(int d, long blocks, int n, int cus, bool causal, bool room = true) {
   if (d == 128) {
     if (blocks > 2L * cus) return false;
-    if (causal) {
-      if (n > 256) return blocks <= cus;
-      return 2 * blocks <= 3L * cus || n <= 24 || (n >= 52 && n <= 128);
-    }
-    if (2 * blocks <= cus) return true;                                      // one round instead of two
-    if (blocks > cus && 2 * blocks <= 3L * cus) return n < 160 || n == 256 || !room;  // three rounds instead of four
-    if (n <= 64) return 10 * blocks <= (n <= 48 ? 10L : 9L) * cus;
-    const long left = 2 * blocks % cus;
-    return n == 128 && (left == 0 || 2 * left >= cus || !room);
+    if (n <= 128) return true;
+    if (causal) return 2 * blocks <= (n <= 256 ? 3L : 2L) * cus;
+    const bool three_rounds_for_four = blocks > cus && 2 * blocks <= 3L * cus;
+    return 2 * blocks <= cus || (three_rounds_for_four && (n <= 256 || !room));
   }
   const long places = 2L * cus;
   if (causal) return n <= 512 ? blocks <= 10 * places && blocks * n <= places * (2L * n + 256) : blocks < 2 * places;
-  if (n <= 256) {
-    if (4 * blocks > 3 * places && blocks <= places)  // two rounds either way
-      return n <= 56 || (n <= 64 && 20 * blocks <= 19 * places) || n >= 128;
-    return 2 * blocks <= (n <= 60 ? 15 : 8) * places && blocks * n <= places * (n + 384L);
-  }
+  if (n <= 256) return 2 * blocks < (n <= 60 ? 15 : 10) * places && blocks * n <= places * (n + 384L);
   const long left = 2 * blocks % places;
   return 4 * blocks <= 3 * places || (blocks > places && blocks < 2 * places && left > 0 && 2 * left <= places);
 }
@@ -283,13 +278,13 @@ FMHA_HOST_DEVICE bool fmha_blocks_make_stats(int d, int n, bool causal) {
 // 16 MiB without a mask up to 384 rows, 8 MiB (of half the square) under causal masking and 10 MiB else.  Fewer blocks than
 // those of the figures go in one launch that stores no dS, unless the passes are called one by one, as the ones with "*" are.
 // us of the backward without and with the hint, N x slices (MiB of dS; with the tensors):
-// Lower line: 66 x 230 (7; 29) 20.3, 19.0; 110 x 256 (8; 49) 24.7, 24.4; 77 x 430 (13; 62) 36.5, 35.9; 140 x 79 (10; 26) 20.7,
-// 20.3; 140 x 120 (15; 40) 23.2, 22.3; 200 x 110 (14; 46) 26.8, 26.5; 256 x 100 (13; 50) 27.0, 26.8; 256 x 128 (16; 64) 30.4,
-// 30.7; 257 x 46 (13; 30) 25.2, 24.2; 384 x 46 (13; 39) 28.2, 27.9; 384 x 64 (18; 54) 29.9, 29.9; 384 x 85 (24; 72) 33.3,
-// 34.0; 200 x 135 (17; 56) 42.1, 42.2; 110 x 520 (16; 100) 57.6, 58.5; 128 x 520 (16; 114) 61.3, 62.6; 350 x 86 (24; 68) 51.8,
-// 53.6; causal 33 x 500 (8; 32) 24.0, 23.5; 50 x 500 (8; 44) 26.7, 26.5; 64 x 530 (8; 58) 43.4, 43.4; 128 x 513 (8; 104) 59.3,
-// 61.0; 128 x 600 (9; 122) 64.3, 65.3; 512 x 75 (19; 75) 45.0, 47.7.  Forward and backward: 512 x 16 * (8; 20) 40.8, 39.8;
-// 1024 x 5 * (10; 18) 59.8, 61.8.
+// Lower line: 66 x 230 * (7; 29) 20.3, 19.0; 110 x 256 * (8; 49) 24.7, 24.4; 77 x 430 * (13; 62) 36.5, 35.9; 140 x 79 (10; 26)
+// 20.7, 20.3; 140 x 120 (15; 40) 23.2, 22.3; 200 x 110 (14; 46) 26.8, 26.5; 256 x 100 (13; 50) 27.0, 26.8; 256 x 128 (16; 64)
+// 30.4, 30.7; 257 x 46 (13; 30) 25.2, 24.2; 384 x 46 (13; 39) 28.2, 27.9; 384 x 64 (18; 54) 29.9, 29.9; 384 x 85 (24; 72)
+// 33.3, 34.0; 200 x 135 (17; 56) 42.1, 42.2; 110 x 520 (16; 100) 57.6, 58.5; 128 x 520 (16; 114) 61.3, 62.6; 350 x 86 (24; 68)
+// 51.8, 53.6; causal 33 x 500 * (8; 32) 24.0, 23.5; 50 x 500 * (8; 44) 26.7, 26.5; 64 x 530 (8; 58) 43.4, 43.4; 128 x 513 (8;
+// 104) 59.3, 61.0; 128 x 600 (9; 122) 64.3, 65.3; 512 x 75 (19; 75) 45.0, 47.7.  Forward and backward: 512 x 16 * (8; 20)
+// 40.8, 39.8; 1024 x 5 * (10; 18) 59.8, 61.8.
 // Upper line, forward and backward: 1031 x 60 (152; 243) 203, 207; 4096 x 11 causal (176; 242) 240, 254; 512 x 224 (112; 280)
 // 185, 179; 1024 x 88 (176; 308) 237, 227; 4096 x 16 causal (256; 352) 305, 300; 4096 x 64 causal (1024; 1408) 1217, 1161.
 FMHA_HOST_DEVICE bool fmha_ds_used_once(unsigned long ds_bytes, unsigned long touched, int n, bool causal) {

@@ -124,7 +124,8 @@ EITHER_MFMA = [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200]
 
 
 def _slices_of_a_busy_launch(N, causal, cus):
-    return cus // (1 if causal else 2) // (-(-N // 128)) + 1
+    blocks = cus if causal else -(-5 * cus // 8)
+    return blocks // (-(-N // 128)) + 1
 
 
 def test_mfmas_of_the_cases_below(tmp_path):
@@ -220,13 +221,14 @@ DS_IN_ONE_CALL = [(260, 300), (130, 600), (50, 300), (100, 300)]  # H, N: dS is 
 
 
 def test_dS_in_one_call(tmp_path):
-    """Of the cases below on 256 compute units, which are by passes with 16 x 16 MFMAs then: no call stores dS by the others."""
+    """Of the cases below on 256 compute units, and that it is by passes with 32 x 32 MFMAs too, though never under a mask."""
     at_once = "fmha_passes_at_once(128, (long)((x[1] + 127) / 128) * x[0], x[1], 256, x[2])"
     wide = "fmha_wide_mfmas((long)((x[1] + 127) / 128) * x[0], 256, x[2])"
     no_mask, causal = ([(*case, mask) for case in DS_IN_ONE_CALL] for mask in (0, 1))
     assert abi.host_rule(tmp_path, at_once, no_mask) == [False] * 4
     assert abi.host_rule(tmp_path, at_once, causal) == [False, False, True, False]
-    every = [(H, N, mask) for N in (1, 20, 40, 64, 65, 128, 129, 200, 256, 257, 1031, 4096) for H in range(1, 600) for mask in (0, 1)]
+    assert abi.host_rule(tmp_path, wide, no_mask) == [False, False, True, False]
+    every = [(H, N, 1) for N in (1, 20, 40, 64, 65, 128, 129, 200, 256, 257, 1031, 4096) for H in range(1, 600)]
     assert not any(abi.host_rule(tmp_path, f"!{at_once} && {wide}", every))
 
 
@@ -249,9 +251,9 @@ def test_dq_ignores_dS_that_no_query_needs(H, N, causal):
 
 HINT_ON_DS = [  # H, N, causal, whether the passes are called one by one, whether dS is told to be used once
     (127, 256, False, False, True), (128, 256, False, False, False),   # 15.9 and 16 MiB of dS
-    (511, 127, False, False, True), (512, 127, False, False, False),
+    (511, 127, False, True, True), (512, 127, False, True, False),
     (56, 384, False, False, True), (57, 384, False, False, False),     # 15.8 and 16.03
-    (511, 50, True, False, True), (513, 50, True, False, False),       # 7.98 and 8.02 MiB
+    (511, 50, True, True, True), (513, 50, True, False, False),        # 7.98 and 8.02 MiB
     (4, 1024, False, True, True), (5, 1024, False, True, False),       # 8 and 10 MiB
     (5, 1025, True, True, True), (9, 1025, True, True, False),         # 6.3 and 11.4 MiB
     (63, 1031, False, False, False), (64, 1031, False, False, True),   # 255 and 259 MiB of dS and tensors
@@ -478,57 +480,58 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
-def test_one_launch_only_where_it_is_faster(tmp_path):
+def test_one_launch_only_where_it_is_worth_it(tmp_path):
     """D, N, slices, causal of launches timed both ways on 256 compute units."""
     rule = "fmha_passes_at_once(x[0], (long)((x[1] + 127) / 128) * x[2], x[1], 256, x[3])"
-    faster_apart = [
-        (128, 64, 256, 0), (128, 64, 512, 0), (128, 77, 136, 0), (128, 100, 256, 0), (128, 120, 141, 0), (128, 110, 512, 0),
-        (128, 128, 141, 0), (128, 128, 410, 0), (128, 140, 128, 0), (128, 200, 141, 0), (128, 40, 486, 1), (128, 300, 90, 1),
-        (64, 64, 512, 0), (64, 64, 3584, 0), (64, 80, 448, 0), (64, 100, 512, 0), (64, 120, 512, 0), (64, 80, 2560, 0),
-        (64, 5, 5120, 0), (64, 512, 128, 0), (64, 5, 8192, 1),
+    apart = [
+        (128, 77, 520, 0), (128, 128, 513, 0), (128, 140, 128, 0), (128, 140, 68, 0),
+        (128, 200, 198, 0), (128, 257, 89, 0), (128, 1031, 20, 0), (128, 300, 90, 1), (128, 200, 218, 1), (128, 33, 520, 0),
+        (64, 64, 3584, 0), (64, 80, 2560, 0), (64, 5, 5120, 0), (64, 512, 128, 0), (64, 5, 8192, 1),
     ]
-    faster_at_once = [
-        (128, 33, 256, 0), (128, 64, 230, 0), (128, 110, 128, 0), (128, 77, 384, 0), (128, 128, 192, 0), (128, 128, 512, 0),
-        (128, 140, 166, 0), (128, 256, 192, 0), (128, 64, 512, 1), (128, 24, 410, 1), (128, 200, 192, 1), (128, 1031, 28, 1),
-        (64, 48, 512, 0), (64, 64, 486, 0), (64, 120, 384, 0), (64, 120, 538, 0), (64, 128, 512, 0), (64, 24, 3840, 0),
-        (64, 128, 2048, 0), (64, 204, 256, 0), (64, 220, 243, 0), (64, 512, 96, 0), (64, 1, 4096, 1), (64, 140, 900, 1),
+    at_once = [
+        (128, 33, 256, 0), (128, 64, 256, 0), (128, 64, 512, 0), (128, 110, 128, 0), (128, 100, 448, 0), (128, 77, 384, 0),
+        (128, 128, 141, 0), (128, 128, 512, 0), (128, 140, 166, 0), (128, 180, 192, 0), (128, 256, 192, 0), (128, 64, 512, 1),
+        (128, 40, 486, 1), (128, 200, 192, 1), (128, 1031, 28, 1), (128, 1031, 14, 0),
+        (64, 48, 512, 0), (64, 64, 512, 0), (64, 80, 448, 0), (64, 120, 512, 0), (64, 128, 512, 0), (64, 24, 3800, 0),
+        (64, 64, 2400, 0), (64, 128, 2048, 0), (64, 204, 256, 0), (64, 512, 96, 0), (64, 1, 4096, 1), (64, 140, 900, 1),
         (64, 1024, 64, 1),
     ]
-    assert not any(abi.host_rule(tmp_path, rule, faster_apart))
-    assert all(abi.host_rule(tmp_path, rule, faster_at_once))
+    assert not any(abi.host_rule(tmp_path, rule, apart))
+    assert all(abi.host_rule(tmp_path, rule, at_once))
     without_room = rule.replace("x[3])", "x[3], false)")  # for dS
-    faster_at_once = [(128, 128, 396, 0), (128, 160, 192, 0), (128, 230, 166, 0), (128, 192, 132, 0), (128, 1031, 42, 0)]
-    faster_apart = [(128, 64, 256, 0), (128, 110, 256, 0), (128, 120, 141, 0), (128, 230, 256, 0),
-                    (128, 40, 486, 1), (128, 1024, 20, 0), (128, 4096, 15, 0)]
-    assert not any(abi.host_rule(tmp_path, rule, faster_at_once))
-    assert all(abi.host_rule(tmp_path, without_room, faster_at_once))
-    assert not any(abi.host_rule(tmp_path, without_room, faster_apart))
+    at_once = [(128, 300, 90, 0), (128, 512, 96, 0), (128, 1031, 42, 0), (128, 4096, 9, 0)]
+    apart = [(128, 110, 520, 0), (128, 230, 256, 0), (128, 1024, 20, 0), (128, 1024, 50, 0), (128, 4096, 15, 0)]
+    assert not any(abi.host_rule(tmp_path, rule, at_once))
+    assert all(abi.host_rule(tmp_path, without_room, at_once))
+    assert not any(abi.host_rule(tmp_path, without_room, apart))
 
 
 ONE_LAUNCH = {  # B, H, N, causal by head size and by what fused_mha_backward does
     (64, "one launch, statistics made by the blocks"): [
         (1, 1, 1, False), (3, 5, 64, True), (2, 3, 65, False), (1, 3, 512, False), (2, 4, 511, True), (1, 5, 1024, True),
         (16, 40, 129, False), (1, 70, 1000, True), (1, 480, 60, False), (1, 900, 127, False), (1, 250, 193, False),
+        (1, 512, 64, False), (1, 500, 65, False),
     ],
     (64, "one launch behind the kernel for the statistics"): [
         (1, 3, 513, False), (2, 2, 1025, True), (1, 5, 1031, False), (1, 3, 1536, True), (3, 20, 1031, False),
     ],
     (64, "the passes one after the other"): [
-        (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False), (1, 3900, 33, False), (1, 512, 64, False),
-        (1, 500, 65, False), (1, 800, 193, False), (1, 3100, 65, True), (1, 600, 511, True), (1, 120, 1031, True),
+        (1, 64, 1024, False), (1, 130, 1024, True), (1, 800, 256, False), (1, 3900, 33, False), (1, 2600, 64, False),
+        (1, 2600, 65, False), (1, 800, 193, False), (1, 3100, 65, True), (1, 600, 511, True), (1, 120, 1031, True),
     ],
     (128, "one launch, statistics made by the blocks"): [
         (1, 1, 1, True), (3, 5, 33, False), (2, 3, 64, True), (2, 3, 65, False), (1, 100, 128, True), (3, 100, 77, False),
         (2, 30, 255, False), (1, 70, 256, True), (1, 140, 256, False), (3, 7, 384, True), (1, 9, 321, False),
-        (5, 100, 64, True),
+        (5, 100, 64, True), (1, 140, 250, False), (1, 400, 33, False), (1, 400, 40, True), (1, 150, 65, False),
+        (1, 140, 128, False), (1, 396, 128, False), (1, 192, 160, False), (5, 100, 77, False), (1, 400, 65, False),
     ],
     (128, "one launch behind the kernel for the statistics"): [
         (1, 3, 385, False), (2, 2, 1031, True), (1, 9, 1031, False), (1, 30, 1000, True), (1, 2, 2049, False),
     ],
     (128, "the passes one after the other"): [
-        (5, 100, 77, False), (1, 140, 250, False), (1, 70, 250, False), (1, 70, 400, True), (1, 20, 1031, False),
-        (1, 400, 33, False), (1, 513, 64, True), (1, 400, 40, True), (1, 150, 65, False), (1, 140, 128, False),
-        (1, 396, 128, False), (1, 192, 160, False), (1, 90, 300, False), (1, 31, 1031, False),  # one launch without room for dS
+        (6, 100, 77, False), (1, 70, 250, False), (1, 70, 400, True), (1, 20, 1031, False), (1, 520, 33, False),
+        (1, 513, 64, True), (1, 520, 40, True), (1, 520, 65, False), (1, 520, 128, False), (1, 200, 200, False),
+        (1, 90, 300, False), (1, 31, 1031, False),  # one launch without room for dS
     ],
 }
 

@@ -107,7 +107,7 @@ def test_workspace_within(lib, batch, head, n, d, room, slices):
 
 @pytest.mark.parametrize("batch,head,n,d,causal,room", [
     (2, 32, 4096, 128, 1, True), (1, 8, 4096, 128, 1, False), (1, 8, 4096, 128, 0, True), (1, 4, 4096, 128, 0, False),
-    (1, 400, 100, 128, 0, True), (1, 100, 100, 128, 0, False), (1, 4, 128, 64, 0, False), (1, 64, 4096, 64, 1, False),
+    (1, 600, 100, 128, 0, True), (1, 400, 100, 128, 0, False), (1, 4, 128, 64, 0, False), (1, 64, 4096, 64, 1, False),
 ])
 def test_workspace_for(lib, batch, head, n, d, causal, room):
     """The size the extension takes for one backward: none for dS where both passes go in one launch (256 compute units)."""
@@ -426,7 +426,7 @@ def test_full_launches_take_the_kernels_they_are_meant_for(tmp_path):
     shapes = [(B * H, N, causal) for B, H, N, causal in FULL_LAUNCHES]
     assert not any(abi.host_rule(tmp_path, wide, shapes))
     assert abi.host_rule(tmp_path, "fmha_persistent_forward_pays(x[0], x[1], 256, x[2])", shapes) == [True] * 3 + [False] * 2
-    assert all(abi.host_rule(tmp_path, wide, [(25, 520, False), (51, 520, True), (4, 320, True)]))
+    assert all(abi.host_rule(tmp_path, wide, [(31, 520, False), (51, 520, True), (4, 320, True)]))
 
 
 def test_interleaved_blocks_are_a_bijection(tmp_path):
