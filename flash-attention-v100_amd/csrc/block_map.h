@@ -203,6 +203,53 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
   second_pass = v & 1;
 }
 
+// A launch of all blocks of the dK/dV pass and then all of the dQ pass over the dS that it stores, nb each per slice, either
+// in the order of a launch of its own (the short last blocks of sequences without a mask in their places: what comes last
+// are the dQ blocks, and they wait for whole slices).  The second part begins at a multiple of 8, so that a slice stays on its
+// XCD; the up to 7 work groups before that have no block.
+FMHA_HOST_DEVICE int fmha_ds_launch_blocks(int slices, int nb) { return ((slices * nb + 7) & ~7) + slices * nb; }
+FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool heavy_first, int& slice, int& blk, bool& second_pass) {
+  const int blocks = slices * nb, second = (blocks + 7) & ~7;
+  second_pass = lin >= second;
+  if (second_pass) lin -= second;
+  if (lin >= blocks) return false;
+  fmha_scheduled_block(lin, slices, nb, heavy_first, false, slice, blk);
+  return true;
+}
+
+// Whether such a launch takes the place of the two passes one after the other.  It gains where the last round of one of them is
+// far from full, and with few rounds, and a launch where these are short; it loses where a dQ block of 128 queries is much
+// slower than the one of 256 that the dQ pass alone takes then (half of the copies of K), which long sequences feel.  us of the
+// backward, passes apart and in one launch, N x slices (rounds of blocks of 128 rows):
+// Up to 768 rows.  64 x 520 (2.0) 40.3, 30.4; 64 x 1200 (4.7) 59.5, 59.4; 100 x 300 (1.2) 44.2, 34.9; 100 x 3000 (11.7) 226, 235;
+// 128 x 600 63.1, 50.9; 128 x 2000 (7.8) 177, 174; 200 x 200 46.0, 37.3; 256 x 256 (2) 52.5, 51.5; 300 x 86 (1.0) 42.3, 32.5; 384 x
+// 400 (4.7) 159, 144; 512 x 64 (1) 38.2, 35.7; 512 x 100 63.4, 54.9; 512 x 192 (3) 107, 103; 512 x 256 (4) 140, 141; 512 x 600
+// (9.4) 346, 345; 640 x 128 (2.5) 112, 97; 640 x 300 (5.9) 251, 243.  Causal: 64 x 600 43.5, 33.9; 64 x 2000 (7.8) 98.0, 98.2; 128
+// x 1200 (4.7) 117, 99; 200 x 400 69.9, 58.3; 200 x 1000 (7.8) 153, 157; 256 x 300 62.5, 50.7; 256 x 1000 191, 184; 512 x 80
+// 42.4, 37.6; 512 x 192 (3) 86.7, 78.2; 512 x 400 (6.3) 176, 171; 640 x 200 (3.9) 123, 114.
+// Longer, without a mask.  One round or less: 1024 x 32 59.2, 55.5; 1280 x 20 59.6, 57.6; 2048 x 16 97.0, 95.9; 4096 x 8 185,
+// 193.  777 x 40 (1.1) 69.4, 58.2; 777 x 100 (2.7) 136, 125; 1024 x 48 (1.5) 96.2, 86.0; 1024 x 64 (2) 107, 106; 1024 x 96 (3) 165,
+// 167; 1031 x 60 (2.1) 129, 114; 1500 x 24 (1.1) 123, 105; 1500 x 48 (2.3) 204, 177; 1500 x 64 (3) 232, 234; 1500 x 100 (4.7)
+// 374, 375; 2048 x 20 (1.3) 158, 135; 2048 x 28 (1.8) 189, 186; 2048 x 56 (3.5) 368, 353; 2048 x 64 (4) 397, 404; 2048 x 130 (8.1)
+// 872, 839; 2048 x 170 (10.6) 1089, 1100; 3000 x 12 (1.1) 230, 195; 3000 x 50 (4.7) 664, 677; 4096 x 10 (1.3) 309, 263; 4096 x
+// 20 (2.5) 506, 482; 4096 x 32 (4) 710, 739; 4096 x 42 (5.3) 1002, 992; 4096 x 52 (6.5) 1230, 1239; 6000 x 6 (1.1) 435, 435;
+// 6000 x 8 (1.5) 470, 473; 6000 x 12 (2.2) 705, 618; 8192 x 5 (1.3) 574, 582; 8192 x 9 (2.3) 909, 828; 8192 x 17 (4.3) 1606,
+// 1540; 16384 x 3 1189, 1211.
+// Longer, causal.  777 x 64 (1.8) 58.0, 54.8; 777 x 300 (8.2) 267, 262; 1024 x 40 54.6, 50.4; 1024 x 128 (4) 144, 146; 1024 x 150
+// 190, 176; 1024 x 220 (6.9) 276, 264; 1280 x 100 (3.9) 176, 170; 1500 x 48 (2.3) 118, 108; 1500 x 80 (3.8) 189, 181; 2048 x 20 85.3,
+// 81.0; 2048 x 56 (3.5) 213, 208; 2048 x 64 (4) 232, 237; 2048 x 80 (5) 296, 299; 4096 x 9 (1.1) 149, 140; 4096 x 11 (1.4) 159,
+// 153; 4096 x 12 (1.5) 169, 171; 4096 x 16 (2) 207, 210; 8192 x 6 323, 324; 8192 x 12 (3) 586, 594; 16384 x 16 (8) 2820, 2919.
+FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool causal) {
+  const long blocks = (long)slices * ((n + 127) / 128), left = blocks % cus;
+  if (n <= 768) return 2 * blocks <= 15L * cus;
+  if (causal) return n <= 1024 ? blocks <= 7L * cus : n <= 2048 ? blocks < 4L * cus : n <= 4096 && 2 * blocks < 3L * cus;
+  if (blocks <= cus) return n <= 2048;
+  if (left == 0) return false;
+  if (n <= 1024) return 4 * left <= 3L * cus && blocks <= 9L * cus;
+  if (n <= 4096) return 2 * left <= cus && blocks <= (n <= 2048 ? 9L : 6L) * cus;
+  return n <= 8192 && 4 * left <= cus && blocks > 2L * cus && blocks < 5L * cus;
+}
+
 // Whether the backward does both passes, `blocks` blocks of 128 rows each, in one launch of 2 * blocks.  With fewer blocks
 // than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few more,
 // each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together it

@@ -234,10 +234,13 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
   at::Tensor od = dense(out), ld = dense(lse);
   // Statistics, and at head size 128 room for dS; a large one only as far as it is there for the taking.
   const size_t min_bytes = fused_mha_backward_min_workspace_bytes(batch_size, num_heads, seqlen_q, head_size);
-  size_t ws_bytes = fmha_backward_workspace_for(batch_size, num_heads, seqlen_q, head_size, is_causal ? 1 : 0);
+  const size_t wanted = fmha_backward_workspace_for(batch_size, num_heads, seqlen_q, head_size, is_causal ? 1 : 0);
+  size_t ws_bytes = wanted;
   if (ws_bytes >= kLargeWorkspace)
     ws_bytes = fmha_backward_workspace_within(batch_size, num_heads, seqlen_q, head_size,
                                               workspace_room(q.get_device(), ws_bytes));
+  if (ws_bytes == wanted)
+    ws_bytes += fmha_backward_count_bytes(batch_size, num_heads, seqlen_q, head_size, is_causal ? 1 : 0);
   at::Tensor workspace;
   try {
     workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);

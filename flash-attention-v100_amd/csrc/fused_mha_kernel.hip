@@ -241,8 +241,9 @@ __device__ __forceinline__ void copy16(const half_t* tile_base, int voff, char* 
       : "v"(voff), "s"(tile_base), "s"(lds_addr)
       : "memory");
 }
-// The same for data that is read once (the non-temporal hint keeps it from displacing
-// the tiles other work groups re-read out of the L2).
+// The same for dS, which other work groups of the launch may have written (sc1: not out of this XCD's L2, see
+// store16_stream), with the hint that it is read once, which keeps it from displacing the tiles other work groups re-read
+// out of the L2, and without.
 __device__ __forceinline__ void copy16_stream(const half_t* tile_base, int voff, char* lds_block) {
   const unsigned lds_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds_block;
   unsigned saved_m0;
@@ -250,7 +251,20 @@ __device__ __forceinline__ void copy16_stream(const half_t* tile_base, int voff,
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %3\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2 nt\n\t"
+      "global_load_lds_dwordx4 %1, %2 sc1 nt\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved_m0)
+      : "v"(voff), "s"(tile_base), "s"(lds_addr)
+      : "memory");
+}
+__device__ __forceinline__ void copy16_shared(const half_t* tile_base, int voff, char* lds_block) {
+  const unsigned lds_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds_block;
+  unsigned saved_m0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %3\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2 sc1\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved_m0)
       : "v"(voff), "s"(tile_base), "s"(lds_addr)
@@ -514,17 +528,19 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_each(std::make_integer_sequence<int, kN>{}, f);
 }
 
-// 16 bytes per lane to p + kOffset bytes, with the non-temporal hint (data that is read once, by a later
-// kernel).  Inline asm because the compiler keeps the hint only on the first of several stores that share
+// 16 bytes per lane to p + kOffset bytes, with the non-temporal hint (data that is read once, by other work groups of this
+// launch or of a later one).  sc1: past the XCD's L2, so that work groups of any XCD see it once the store is done; with
+// the hint that costs nothing (64 x 4096 x 128 causal, both passes: 795.9 us without, 796.6 with).  Inline asm because
+// the compiler keeps the hint only on the first of several stores that share
 // a base address; like the tile copies it is therefore invisible to the compiler's wait counts.
 template <int kOffset>
 __device__ __forceinline__ void store16_stream(half_t* p, h8 v, IntTag<kOffset>) {
-  asm volatile("global_store_dwordx4 %0, %1, off offset:%2 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
 }
 // The same without the hint.
 template <int kOffset>
 __device__ __forceinline__ void store16_keep(half_t* p, h8 v, IntTag<kOffset>) {
-  asm volatile("global_store_dwordx4 %0, %1, off offset:%2" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
 }
 
 // Element strides of a (batch, n, head, d) tensor whose last dimension is
@@ -1373,8 +1389,10 @@ template <int D>
 __global__ void __launch_bounds__(256)
 fmha_bwd_delta_kernel(const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides gs,
                       const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, unsigned H,
-                      unsigned N, unsigned first, unsigned end, unsigned chain, unsigned chains) {
+                      unsigned N, unsigned first, unsigned end, unsigned chain, unsigned chains, unsigned* __restrict__ clear,
+                      unsigned words) {
   constexpr unsigned kLanesPerRow = D / 8;
+  for (unsigned at = blockIdx.x * 256 + threadIdx.x; at < words; at += gridDim.x * 256) clear[at] = 0;  // for a later kernel
   const unsigned row0 = first + fmha_interleaved_block(blockIdx.x, chain, chains) * delta_rows(D);  // rows first .. end - 1
   const unsigned slice0 = row0 / N, b0 = slice0 / H;
   const unsigned in_block = threadIdx.x / kLanesPerRow, row = row0 + in_block, c = threadIdx.x % kLanesPerRow;
@@ -1980,6 +1998,7 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // KEEP: without the non-temporal hint on those stores (rule: fmha_ds_used_once).
 // WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: fmha_wide_mfmas).
 // STATS: the row statistics of every tile are formed here, from O, dO and LSE, a tile ahead; delta and lse2 are not read.
+// stored: counts the waves that have stored all of their dS, kKvPairs of every block (fmha_bwd_both_spill_kernel).
 constexpr int kKvStBytes = 1024;
 template <int D>
 constexpr int dkdv_lds() { return 7 * SwzTile<D>::kBytes + 3 * kKvStBytes + 2 * kKvPairs * 2 * 2048; }
@@ -1989,7 +2008,7 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
                const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                const float* __restrict__ LSE, const float* __restrict__ delta, const float* __restrict__ lse2,
                half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N, int slice0,
-               float c, float scale, char* smem, int bh, int nblk) {
+               float c, float scale, char* smem, int bh, int nblk, unsigned* stored = nullptr) {
   using G = TileGeom<D>;
   using G16 = Geom16<D>;
   using T = SwzTile<D>;
@@ -2370,6 +2389,10 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   static_assert(kKvWaves * Stage16<D>::kBytes <= 7 * T::kBytes && kKvWaves * StageGeom<D>::kBytes <= 7 * T::kBytes,
                 "the output staging tiles fit the rings");
   block_barrier();  // every wave is done with the rings: they become the staging tiles
+  if (SPILL && stored && role_b) {  // this wave's dS is where every work group of the launch can read it
+    wait_vm<0>();
+    if (lane == 0) __hip_atomic_fetch_add(stored, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   if (shared) {  // the sums of the four pairs, added in the order of the pairs by the first one
     constexpr int kSums = sizeof(acc) / 16, kBytes = kSums * 1024;  // per wave, 16 bytes of a lane at a time
     static_assert(2 * (kKvPairs - 1) * kBytes <= 7 * T::kBytes, "the sums of three pairs fit the rings");
@@ -2780,11 +2803,32 @@ __device__ __forceinline__ const half_t* wave_uniform(const half_t* p) {
   return (const half_t*)((uint64_t)hi << 32 | lo);
 }
 
-template <int D, bool CAUSAL, int kDsPanels, bool WIDE>
-__global__ void __launch_bounds__(ds_threads(kDsPanels), 1)
-fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
-                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, int slice0,
-                         int stream_ds, float scale) {
+// The blocks of a launch of this pass alone.  With one block per work group the hardware shares them out, otherwise the
+// persistent schedule does.
+template <bool CAUSAL>
+struct DsBlocks {
+  int total, nqb;
+  __device__ __forceinline__ int next_round(int r) const { return PersistentBlocks{total}.next_round(r); }
+  __device__ __forceinline__ void locate(int round, int& bh, int& mb) const {
+    const int lin = round >= 0 ? PersistentBlocks{total}.lin(round) : 0, slices = total / nqb;
+    if ((int)gridDim.x == total) fmha_scheduled_block(lin, slices, nqb, CAUSAL, false, bh, mb);
+    else fmha_slice_and_block(lin, slices, nqb, bh, mb);
+  }
+};
+// One block that is known already.
+struct DsBlock {
+  int bh, mb;
+  __device__ __forceinline__ int next_round(int) const { return -1; }
+  __device__ __forceinline__ void locate(int, int& bh_, int& mb_) const { bh_ = bh, mb_ = mb; }
+};
+
+template <int D, int kDsPanels>
+constexpr int ds_lds() { return kDsRingS * kDsPanels * kDsPanelTileBytes + kDsRingK * SwzTile<D>::kBytes; }
+template <int D, bool CAUSAL, int kDsPanels, bool WIDE, typename Blocks>
+__device__ __forceinline__ void
+bwd_dq_spill_blocks(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
+                    half_t* __restrict__ dQ, int H, int N, int nqb, int slice0, int stream_ds, float scale, char* smem,
+                    const Blocks blocks) {
   using T = SwzTile<D>;             // K tile: 64 keys x D features
   constexpr int kKIPW = T::kInstrs / 2;              // K copies per K-copying wave and tile
   constexpr int kDsWaves = 4 * kDsPanels;            // computing waves
@@ -2793,7 +2837,7 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   constexpr int kSIPW = kDsTileBytes / 1024 / 2;     // dS copies per dS-copying wave and tile: half of the pieces
   static_assert(16 * StageGeom<kDsStageD>::kPitch <= 2048 && 16 * Stage16<kDsStageD>::kPitch <= 2048,
                 "half a staging tile must fit into two dS pieces");
-  __shared__ __attribute__((aligned(1024))) char smem[kDsRingS * kDsTileBytes + kDsRingK * T::kBytes];
+  static_assert(ds_lds<D, kDsPanels>() == kDsRingS * kDsTileBytes + kDsRingK * T::kBytes, "");
   char* const s_ring = smem;
   char* const k_ring = smem + kDsRingS * kDsTileBytes;
 
@@ -2806,26 +2850,18 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   const int rs = H * D;  // dQ is dense
   const int nt_all = (N + kTile - 1) / kTile;
   const int n_panels = np / kDsPanelQ;
-  const int slices = total / nqb;
-  const PersistentBlocks pb{total};
 
-  // With one block per work group the hardware shares the blocks out, otherwise the persistent schedule does.
-  auto locate = [&](int lin, int& bh, int& mb) __attribute__((always_inline)) {
-    if ((int)gridDim.x == total) fmha_scheduled_block(lin, slices, nqb, CAUSAL, false, bh, mb);
-    else fmha_slice_and_block(lin, slices, nqb, bh, mb);
-  };
   // A position in the work group's sequence of tiles: block (round, number), tile j of its nt.
   struct Cursor {
-    int round, lin, j, nt, mblk;
+    int round, j, nt, mblk;
     const half_t* base;  // dS copies: this wave's pieces of the block's tile 0; K copies: the slice's K rows
     long out_off;        // consumer: element offset of the slice in dQ
   };
   auto open = [&](int round, bool for_k) __attribute__((always_inline)) {
     Cursor c;
     c.round = round;
-    c.lin = round >= 0 ? pb.lin(round) : 0;
     int bh, mb;
-    locate(c.lin, bh, mb);
+    blocks.locate(round, bh, mb);
     c.mblk = CAUSAL ? nqb - 1 - mb : mb;  // heavy blocks first
     const int b = (slice0 + bh) / H, h = slice0 + bh - b * H;  // bh: the slice in this launch and in dS
     c.j = 0;
@@ -2841,15 +2877,15 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   };
   auto advance = [&](Cursor& c, bool for_k) __attribute__((always_inline)) {  // to the next tile of the sequence
     if (++c.j == c.nt) {
-      const int r = pb.next_round(c.round);
+      const int r = blocks.next_round(c.round);
       if (r >= 0) c = open(r, for_k);
       else c.round = -1;  // past the end
     }
   };
   int n_tiles = 0;  // tiles in this work group's sequence
-  for (int r = 0; r >= 0; r = pb.next_round(r)) {
+  for (int r = 0; r >= 0; r = blocks.next_round(r)) {
     int bh, mb;
-    locate(pb.lin(r), bh, mb);
+    blocks.locate(r, bh, mb);
     const int mblk = CAUSAL ? nqb - 1 - mb : mb;
     n_tiles += CAUSAL ? min(nt_all, 2 * kDsPanels * (mblk + 1)) : nt_all;
   }
@@ -2892,7 +2928,7 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
       for (int u = 0; u < kSIPW; ++u) copy16_stream(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
     } else {
 #pragma unroll
-      for (int u = 0; u < kSIPW; ++u) copy16(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+      for (int u = 0; u < kSIPW; ++u) copy16_shared(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
     }
   };
   auto copy_k = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
@@ -3056,6 +3092,73 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
   }
 }
 
+template <int D, bool CAUSAL, int kDsPanels, bool WIDE>
+__global__ void __launch_bounds__(ds_threads(kDsPanels), 1)
+fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
+                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, int slice0,
+                         int stream_ds, float scale) {
+  __shared__ __attribute__((aligned(1024))) char smem[ds_lds<D, kDsPanels>()];
+  bwd_dq_spill_blocks<D, CAUSAL, kDsPanels, WIDE>(K, ks, dS, np, dQ, H, N, nqb, slice0, stream_ds, scale, smem,
+                                                  DsBlocks<CAUSAL>{total, nqb});
+}
+
+// ---------------------------------------------------------------------------
+// The dK/dV pass that stores dS and the dQ pass over it in one launch: first all blocks of the former, then those of the
+// latter, one to a work group.  One after the other, each pass leaves CUs idle in its last round and the second starts when
+// the first has drained; here the dQ blocks of slices that are finished fill the places that the dK/dV blocks leave.  What
+// that gives, and where the passes still go one by one: fmha_ds_in_one_launch.
+//
+// A dQ block waits for the dS of its slice: every wave that stores some counts itself when its stores are done, and the
+// block starts when the count is whole.  dS is stored and read past the XCDs' L2s (store16_stream), so that is all it takes,
+// on whatever XCD the blocks are; a release of everything written (an L2 write-back per block) takes 8 % longer.  Each count
+// has a cache line of its own and is asked for about once a microsecond: with the counts of 32 slices in one line the work
+// groups that ask hold up those that work (24 x 2048 x 128 causal, 111 us; a line each 89).
+// The wait ends by itself: dK/dV blocks wait for nobody and come first, and should they not be done within kReadyTicks,
+// whatever the reason, the block forms S and dP itself, as fmha_bwd_dq_kernel does, with the same bits as result.
+// ---------------------------------------------------------------------------
+constexpr unsigned kReadyTicks = 5000000;  // of the 100 MHz clock: 50 ms
+constexpr int kReadyStride = 32;           // words from one slice's count to the next
+template <bool CAUSAL, bool KEEP>
+__global__ void __launch_bounds__(kKvThreads, 1)
+fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                           const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                           const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ,
+                           half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* dS, unsigned* ready, int np, int H, int N,
+                           int nb, int slices, unsigned ticks, float c, float scale) {
+  constexpr int D = 128;
+  static_assert(ds_threads(1) == kKvThreads && kDqThreads == kKvThreads && kDsPanelQ == kKvBlockKeys, "one grid for all");
+  constexpr int kLds = dkdv_lds<D>() > dq_lds<D>() ? dkdv_lds<D>() : dq_lds<D>();
+  static_assert(ds_lds<D, 1>() <= kLds, "");
+  __shared__ __attribute__((aligned(1024))) char smem[kLds];
+  int bh, blk;
+  bool dq;
+  if (!fmha_ds_launch_block(blockIdx.x, slices, nb, CAUSAL, bh, blk, dq)) return;
+  if (!dq) {
+    bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
+                                                        H, N, 0, c, scale, smem, bh, blk, ready + (long)bh * kReadyStride);
+    return;
+  }
+  if (threadIdx.x == 0) {
+    const unsigned long long start = wall_clock64();
+    int whole;
+    for (;;) {
+      whole = __hip_atomic_load(ready + (long)bh * kReadyStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+              (unsigned)(kKvPairs * nb);
+      if (whole || wall_clock64() - start >= ticks) break;
+      __builtin_amdgcn_s_sleep(32);  // 2048 cycles
+    }
+    *reinterpret_cast<volatile int*>(smem) = whole;
+  }
+  block_barrier();
+  const int whole = __builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile int*>(smem));
+  block_barrier();  // the answer is read: the tiles may go where it was
+  if (whole)
+    bwd_dq_spill_blocks<D, CAUSAL, 1, false>(K, ks, dS, np, dQ, H, N, nb, 0, !KEEP, scale, smem, DsBlock{bh, blk});
+  else
+    bwd_dq_block<D, CAUSAL, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
+                                   CAUSAL ? nb - 1 - blk : blk);  // blocks are numbered heaviest first
+}
+
 // ---------------------------------------------------------------------------
 // Host side: validation and launches.
 // ---------------------------------------------------------------------------
@@ -3214,6 +3317,8 @@ int spill_slices(int batch, int head, int n, size_t workspace_bytes) {
   const size_t fit = room / slice_bytes(n), all = (size_t)batch * head;
   return (int)(fit < all ? fit : all);
 }
+// Behind the dS of all slices: the counts of fmha_bwd_both_spill_kernel.
+size_t ready_bytes(int slices) { return (size_t)slices * kReadyStride * sizeof(unsigned); }
 // Whether rounds of that many slices keep the CUs busy: two key blocks for each.
 bool rounds_fill(int slices, int n, int cus) { return (long)slices * key_blocks(n) >= 2L * cus; }
 // The workspace of at most `room` bytes that the backward makes the best use of.  dS of all slices where that is at most
@@ -3245,10 +3350,11 @@ size_t best_workspace(int batch, int head, int n, int d, size_t room) {
 }
 
 template <int D, bool CAUSAL>
-int launch_backward(int passes, int slices_at_once, const void* q, const void* k, const void* v, const void* o,
+int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsigned ticks, const void* q, const void* k, const void* v, const void* o,
                     const void* d_o, Strides qs, Strides ks, Strides vs, Strides gs, const void* lse, float* delta,
                     void* dq, void* dk, void* dv, int batch, int head, int n, float scale, hipStream_t stream) {
-  // slices_at_once: how many slices' dS the workspace holds, 0 for the passes that need none
+  // slices_at_once: how many slices' dS the workspace holds, 0 for the passes that need none; ticks: how long a block may wait
+  // for another's dS
   if (D == 64) slices_at_once = 0;  // see fmha_bwd_dq_pipe_kernel
   // Rounds of so few slices that they leave CUs idle cost more than the GEMMs they save.
   const int cus = (int)persistent_grid(1 << 30);
@@ -3263,6 +3369,14 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
   const size_t ds_bytes = slice_bytes(n) * (spill ? slices_at_once : 0) / (CAUSAL ? 2 : 1);
   const size_t touched = ds_bytes + 6 * (size_t)slices_at_once * n * D * sizeof(half_t);
   const int stream_ds = fmha_ds_used_once(ds_bytes, touched, n, CAUSAL);
+  // Both passes over dS in one launch, where the workspace has room for the counts behind the dS of all slices.
+  unsigned* ready = nullptr;
+  if constexpr (D == 128) {
+    const size_t at = spill_offset(batch, head, n) + (size_t)slices * slice_bytes(n);
+    if (spill && slices_at_once == slices && (passes & kPassAll) == kPassAll && workspace_bytes >= at + ready_bytes(slices) &&
+        fmha_ds_in_one_launch(slices, n, cus, CAUSAL))
+      ready = (unsigned*)((char*)delta + at);
+  }
   auto delta_pass = [&]() {
     const unsigned rows = (unsigned)slices * n;              // fewer than 2^32 / (D / 8): check_shape
     const unsigned most = (1u << 23) * delta_rows(D);        // a launch of fewer than 2^32 threads: fewer than twice the blocks
@@ -3272,7 +3386,8 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
       const unsigned per_slice = (unsigned)(n + delta_rows(D) - 1) / delta_rows(D);
       const unsigned chain = per_slice < blocks ? per_slice : blocks, chains = (blocks + chain - 1) / chain;
       const hipError_t rc = launch(fmha_bwd_delta_kernel<D>, chain * chains, 256, stream, (const half_t*)o, (const half_t*)d_o,
-                                   gs, (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains);
+                                   gs, (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains, ready,
+                                   ready ? (unsigned)(ready_bytes(slices) / 4) : 0u);
       if (rc != hipSuccess) return rc;
     }
     return hipSuccess;
@@ -3367,6 +3482,15 @@ int launch_backward(int passes, int slices_at_once, const void* q, const void* k
                     (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, slice0, c, scale);
     }
   };
+  if constexpr (D == 128) {
+    if (ready) {
+      auto kernel = stream_ds ? fmha_bwd_both_spill_kernel<CAUSAL, false> : fmha_bwd_both_spill_kernel<CAUSAL, true>;
+      const hipError_t rc = launch(kernel, (unsigned)fmha_ds_launch_blocks(slices, nb), kKvThreads, stream, (const half_t*)q,
+                                   (const half_t*)k, (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
+                                   (half_t*)dq, (half_t*)dk, (half_t*)dv, ds, ready, np, head, n, nb, slices, ticks, c, scale);
+      return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
+    }
+  }
   // The spilling dK/dV pass feeds the dQ pass; otherwise the dQ pass (which may make the statistics) goes first.
   if (spill) {
     // as many slices at a time as the workspace holds dS of, in rounds of equal size
@@ -3389,7 +3513,7 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
                       const fused_mha_strides* k_st, const void* v, const fused_mha_strides* v_st, const void* o,
                       const void* d_o, const fused_mha_strides* g_st, const void* lse, void* workspace,
                       size_t workspace_bytes, void* dq, void* dk, void* dv, int batch, int head, int m, int n, int d,
-                      float scale, int causal, void* stream) {
+                      float scale, int causal, void* stream, unsigned ticks = kReadyTicks) {
   const bool need_o = passes & kPassDelta, need_dq = passes & kPassDq, need_dkdv = passes & kPassDkDv;
   if (!d_o || !workspace || !lse || (need_o && !o) || ((need_dq || need_dkdv) && (!q || !k || !v)) ||
       (need_dq && !dq) || (need_dkdv && (!dk || !dv)))
@@ -3410,7 +3534,7 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
   const Strides qs = to_strides(q_st, head, n, d), ks = to_strides(k_st, head, n, d),
                 vs = to_strides(v_st, head, n, d), gs = to_strides(g_st, head, n, d);
 #define FMHA_BWD(DD, CC) \
-  launch_backward<DD, CC>(passes, slices_at_once, q, k, v, o, d_o, qs, ks, vs, gs, lse, delta, dq, dk, dv, batch, head, n, \
+  launch_backward<DD, CC>(passes, slices_at_once, workspace_bytes, ticks, q, k, v, o, d_o, qs, ks, vs, gs, lse, delta, dq, dk, dv, batch, head, n, \
                           scale, s)
   if (d == 128) return causal ? FMHA_BWD(128, true) : FMHA_BWD(128, false);
   return causal ? FMHA_BWD(64, true) : FMHA_BWD(64, false);
@@ -3483,6 +3607,24 @@ size_t fmha_backward_workspace_for(int batch, int head, int n, int d, int causal
   const int cus = (int)persistent_grid(1 << 30);
   if (fmha_passes_at_once(d, (long)key_blocks(n) * batch * head, n, cus, causal != 0)) return stats_bytes(batch, head, n);
   return best_workspace(batch, head, n, d, SIZE_MAX);
+}
+
+size_t fmha_backward_count_bytes(int batch, int head, int n, int d, int causal) {
+  if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK || d == 64) return 0;
+  const int cus = (int)persistent_grid(1 << 30), slices = batch * head;
+  if (fmha_passes_at_once(d, (long)key_blocks(n) * slices, n, cus, causal != 0) ||
+      slices * slice_bytes(n) > FUSED_MHA_SPILL_MAX_BYTES || !fmha_ds_in_one_launch(slices, n, cus, causal != 0))
+    return 0;
+  return ready_bytes(slices);
+}
+
+int fmha_backward_waiting(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,
+                          const void* d_output_ptr, const void* lse_ptr, void* workspace, size_t workspace_bytes,
+                          void* d_query_ptr, void* d_key_ptr, void* d_value_ptr, int batch, int head, int n, int d, float scale,
+                          int causal, unsigned ticks, void* stream) {
+  return dispatch_backward(kPassAll, query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr, d_output_ptr, nullptr,
+                           lse_ptr, workspace, workspace_bytes, d_query_ptr, d_key_ptr, d_value_ptr, batch, head, n, n, d, scale,
+                           causal, stream, ticks);
 }
 
 int fused_mha_backward(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,

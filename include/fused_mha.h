@@ -127,6 +127,10 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * on the mask and the device, which this function does not know, so it returns
  * room for dS for those too (2 GiB for one causal slice of n = 32768); the
  * minimum is as fast for them.
+ * With d = 128 and, behind room for the dS of all slices, another 128 bytes for
+ * each (batch, head) slice, both passes go in one launch where that is faster
+ * (many problems of up to a few blocks of 128 rows per compute unit); the
+ * results are the same bits.
  * A caller that wants to spend less passes any size from the minimum on.
  * Both functions return 0 for an invalid shape.  No counterpart in the
  * reference, which receives delta from Python (flash_attn_interface.py:43-44).

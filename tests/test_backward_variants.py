@@ -1,6 +1,7 @@
 """The D = 64 backward kernels at the sizes where they can go wrong: edges of 32-row waves, 64-row tiles and 128-row
 blocks, one tile and less, several tiles with a partial last one.  The D = 128 backward with a workspace that holds the
 dS of some of the slices."""
+import ctypes
 import os
 import subprocess
 
@@ -118,6 +119,39 @@ def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
         alone = abi.backward(lib, *one, lse[:, h:h + 1].clone(), D ** -0.5, causal)[:3]
         for a, b in zip(alone, whole):
             assert torch.equal(a, b[:, :, h:h + 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ticks", [5000000, 0])
+@pytest.mark.parametrize("H,N,causal", [
+    (520, 64, False), (515, 100, True), (517, 128, True),  # a block per slice and pass
+    (261, 129, False), (200, 160, False), (200, 161, True),  # last blocks of 1, 32 and 33 rows
+    (100, 384, True), (65, 512, False),
+    (60, 1031, False), (37, 1056, False), (33, 1023, True),
+    (18, 2047, True), (9, 4096, False),
+])
+def test_both_passes_over_ds_in_one_launch(H, N, causal, ticks):
+    """The bits of the passes one after the other, also (ticks) where no block waits for the dS of another."""
+    B, D, lib = 1, 128, abi.load()
+    lib.fmha_backward_count_bytes.argtypes, lib.fmha_backward_count_bytes.restype = [ctypes.c_int] * 5, ctypes.c_size_t
+    lib.fmha_backward_waiting.argtypes = ([ctypes.c_void_p] * 7 + [ctypes.c_size_t] + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 +
+                                          [ctypes.c_float, ctypes.c_int, ctypes.c_uint, ctypes.c_void_p])
+    gen = torch.Generator(device="cuda").manual_seed(N + H)
+    q, k, v, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+    apart = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=True)[:3]
+    counts = lib.fmha_backward_count_bytes(B, H, N, D, int(causal))
+    assert counts == 128 * H
+    nbytes = lib.fused_mha_backward_workspace_bytes(B, H, N, D) + counts
+    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
+    for _ in range(2):
+        got = [torch.full_like(q, float("nan")) for _ in range(3)]
+        rc = lib.fmha_backward_waiting(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), lse.data_ptr(),
+                                       ws.data_ptr(), nbytes, *(g.data_ptr() for g in got), B, H, N, D, D ** -0.5, int(causal),
+                                       ticks, torch.cuda.current_stream().cuda_stream)
+        assert rc == abi.OK
+        for a, b in zip(got, apart):
+            assert torch.equal(a, b)
 
 
 EITHER_MFMA = [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200]

@@ -429,6 +429,59 @@ def test_full_launches_take_the_kernels_they_are_meant_for(tmp_path):
     assert all(abi.host_rule(tmp_path, wide, [(31, 520, False), (51, 520, True), (4, 320, True)]))
 
 
+def test_blocks_of_the_launch_over_ds(tmp_path):
+    """csrc/block_map.h: every block of both passes once, a dQ block behind all dK/dV blocks, slices on one XCD where the order
+    of either pass keeps them there."""
+    import subprocess
+
+    src = tmp_path / "check_ds.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (int slices = 1; slices <= 200; slices += slices < 40 ? 1 : 7)
+    for (int nb = 1; nb <= 40; ++nb)
+      for (int causal = 0; causal < 2; ++causal) {
+        const int total = fmha_ds_launch_blocks(slices, nb), blocks = slices * nb;
+        std::vector<int> seen(2 * blocks, -1);
+        int idle = 0;
+        for (int lin = 0; lin < total; ++lin) {
+          int s, b;
+          bool dq;
+          if (!fmha_ds_launch_block(lin, slices, nb, causal, s, b, dq)) { ++idle; continue; }
+          if (s < 0 || s >= slices || b < 0 || b >= nb || dq != (lin >= blocks) || seen[dq * blocks + s * nb + b] >= 0) {
+            printf("%d %d %d: %d\n", slices, nb, causal, lin);
+            return 1;
+          }
+          seen[dq * blocks + s * nb + b] = lin;
+        }
+        if (idle > 7 || total != 2 * blocks + idle) return 2;
+        for (int at = 0; at < blocks; ++at)
+          if ((seen[at] ^ seen[blocks + at]) & 7) return 3;  // the dQ block is where the dK/dV block of the same number was
+      }
+  puts("ok");
+  return 0;
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    exe = tmp_path / "check_ds"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
+def test_count_bytes(lib):
+    """What the extension adds behind the dS of all slices, on 256 compute units: 128 bytes a slice where one launch does both
+    passes, nothing elsewhere."""
+    f = lib.fmha_backward_count_bytes
+    f.argtypes, f.restype = [ctypes.c_int] * 5, ctypes.c_size_t
+    assert f(3, 20, 1031, 128, 0) == 60 * 128 and f(16, 12, 512, 128, 1) == 192 * 128 and f(1, 600, 64, 128, 0) == 600 * 128
+    assert f(2, 32, 4096, 128, 1) == 0    # the dQ pass alone has blocks of 256 queries there
+    assert f(1, 4, 1031, 128, 0) == 0     # few blocks: one launch that forms S and dP twice
+    assert f(16, 12, 512, 64, 0) == 0 and f(1, 0, 512, 128, 0) == 0
+    assert f(1, 33000, 512, 128, 0) == 0  # dS in rounds
+
+
 def test_interleaved_blocks_are_a_bijection(tmp_path):
     """csrc/block_map.h: the row statistics' work groups take every block of a launch once, and few more than there are."""
     import subprocess
