@@ -250,6 +250,49 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
   return n <= 8192 && 4 * left <= cus && blocks > 2L * cus && blocks < 5L * cus;
 }
 
+// Whether the backward takes a work group for each slice (fmha_bwd_slice_kernel, one to a CU), before all of the below.  It
+// forms S and dP once, as the D = 128 passes over dS do, but needs no room for dS, makes the statistics and is one launch; and it
+// reads Q, K, V and dO once.  It loses where slices leave CUs idle that blocks of 128 rows would fill: with few slices, and with
+// a last round that is far from full, the more so the longer a round is and under causal masking, where half of the blocks of a
+// slice are light, which the other launches pair with heavy ones.  At D = 64 up to 128 rows half of its waves have no keys, and
+// blocks of 128 rows, two to a CU, are ahead (64 x 256 equal, 128 x 256 and 128 x 1024 lose 4 and 18 %).
+// us of the kernels of the backward, without it and with it, N x slices:
+// D = 128, without a mask.  One round: 40 x 128 7.5, 8.9; 40 x 160 12.9, 9.1; 200 x 128 25.5, 26.8; 256 x 136 43.0, 30.1; 256 x 256
+// 51.9, 37.4.  Two: 17 x 264 16.8, 11.9; 100 x 264 32.8, 28.6; 160 x 288 42.8, 46.0; 160 x 320 47.8, 45.8; 256 x 288 56.5, 60.8;
+// 256 x 320 61.2, 61.8; 256 x 512 100.3, 77.7.  More: 33 x 514 24.7, 23.9; 50 x 528 27.8, 27.6; 100 x 528 41.9, 44.2; 100 x 640
+// 48.2, 45.0; 100 x 800 59.7, 61.0; 100 x 1030 73.0, 75.8; 100 x 1600 120.8, 114.0; 256 x 528 106.2, 99.8; 256 x 1024 206, 163.
+// D = 128, causal.  160 x 128 22.1, 18.4 but 200 x 128 25.4, 24.3 and 100 x 128 slower; 256 x 160 35.8, 28.6; 256 x 256 43.5, 32.5;
+// 160 x 288 37.4, 35.5; 256 x 288 48.5, 55.3; 256 x 336 56.3, 57.5; 256 x 352 58.4, 58.0; 256 x 512 86.0, 64.9; 100 x 514 40.1,
+// 42.5; 100 x 640 48.8, 43.9; 256 x 528 90.9, 89.7.
+// D = 64, without a mask.  256 x 128 15.7, 18.8; 145 x 144 15.8, 12.9; 256 x 144 21.2, 19.1; 300 x 168 30.2, 32.1; 300 x
+// 192 34.3, 32.7; 512 x 192 60.9, 52.8; 512 x 256 78.5, 61.8; 300 x 352 60.1, 61.7; 300 x 384 61.2, 62.2; 300 x
+// 400 62.9, 62.7; 512 x 384 115, 110; 512 x 448 131, 115; 300 x 560 85.2, 92.2; 300 x 600 92.6, 92.5; 512 x 560 173, 177; 512 x
+// 620 191, 180; 300 x 770 115, 123; 300 x 900 135, 129; 300 x 1030 157, 159; 512 x 1030 339, 299; 512 x 1300 427, 362.
+// D = 64, causal.  129 x 160 12.6, 13.1; 129 x 168 14.5, 13.1; 160 x 256 19.1, 15.1; 145 x 416 26.9, 26.6; 145 x 448 28.1, 27.3; 145
+// x 600 35.9, 39.0; 180 x 208 16.8, 16.3; 200 x 230 20.1, 18.7; 256 x 240 22.0, 22.1; 300 x 208 27.3, 29.2; 300 x 230 31.3, 29.3;
+// 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512 x 432 93.7,
+// 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512 x 900 217, 198;
+// 512 x 1030 247, 246; 300 x 1030 124, 141.
+FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, bool causal) {
+  if (n > 32768 / d) return false;  // LDS and registers hold no more keys
+  const long rounds = ((long)slices + cus - 1) / cus, last = slices - (rounds - 1) * cus;
+  if (d == 128) {
+    if (rounds == 1) return 2 * last > cus;
+    if (n <= 64) return true;
+    if (n <= 128) return rounds == 2 || rounds > 6 || 2 * last >= cus;
+    return rounds > 2 || (causal && n > 160 ? 3 : 4) * last >= cus;
+  }
+  if (n <= 128) return false;
+  if (!causal) {
+    if (rounds == 1) return n <= 256 ? 2 * last > cus : 4 * last >= 3L * cus;
+    return rounds > 5 || rounds * last > cus;
+  }
+  if (n <= 160) return rounds == 1 ? 3 * last >= 2L * cus : rounds == 2 && 4 * last >= 3L * cus;
+  if (n <= 256) return n <= 200 && rounds == 1 && 8 * last >= 7L * cus;
+  if (n <= 384) return 16 * last >= (rounds == 1 ? 14L : 15L) * cus;
+  return rounds > 4 || 8 * last >= (rounds == 1 ? 7L : 6L) * cus;
+}
+
 // Whether the backward does both passes, `blocks` blocks of 128 rows each, in one launch of 2 * blocks.  With fewer blocks
 // than places (D = 64: two to a CU, D = 128: one) the passes one after the other leave most of the chip idle; with a few more,
 // each has a nearly empty last round of its own.  Where the one launch takes as many rounds as the two passes together it

@@ -3160,6 +3160,492 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
 }
 
 // ---------------------------------------------------------------------------
+// Backward of a whole slice in one work group, for slices that a CU can hold: K, all dK and dV, and the dS of 32 queries
+// ---------------------------------------------------------------------------
+// A wave owns 32 keys (D = 64 past 256 rows: twice 32, blocks w and 15 - w, which under causal masking are together as heavy as
+// any other two).  It keeps their dK and dV and their rows of V, negated, in registers.  K lies in LDS whole.  The work group
+// walks the queries 32 at a time: Q, dO and O come by copies to LDS that are two tiles ahead, delta is made from them as
+// fmha_bwd_delta_kernel makes it, each wave forms S, P, dP and dS of its keys (32 x 32 MFMAs, as bwd_dkdv_block), adds to dV and dK,
+// and leaves dS in LDS; behind the next barrier the waves share out the 16 x 16 tiles of dQ of those 32 queries and add up all
+// keys in order.  So S and dP are formed once and neither dS nor partial dQ leaves the CU, each input is read once, and there is
+// one barrier for 32 queries.  All sums are in the order of the other paths, which give the same bits.
+// Bound by the LDS and by issue: at D = 64 with two blocks of keys a wave reads 24 KiB of Q, dO and K for 32 MFMAs of 32 x 32 x 16
+// and 32 KiB of K and dS for 16 of 16 x 16 x 32, which for 8 waves is 1.5 times as long as a SIMD's MFMAs take, and with two
+// waves to a SIMD the vector work on S and P hardly overlaps with another wave's MFMAs.  (dQ in front of the rest of a tile in all waves, or behind it in half of them, so that the two kinds
+// of work meet: no difference, and the first needs fewer registers.  dQ steps between those of dK: slower.)  Fragments are read
+// two to four MFMA groups ahead; one ahead costs 6 %.  512 x 192 slices, D = 64: 52.7 us, 610 TFLOP/s on the 192 CUs that have
+// work; two passes that form S and dP twice: 61.  256 x 256, D = 128: 37.4 us, 574 TFLOP/s; over dS in memory: 51.9.
+// At D = 128 without a mask 129 to 160 rows have four idle waves and one of up to 32 keys.  bwd_dkdv_block shares such keys between
+// its four pairs of waves, tile j to pair j mod 4, and adds the four sums up at the end; to have its bits the idle waves do the
+// same here.
+constexpr int kSliceWaves = 8;
+constexpr int kSliceThreads = kSliceWaves * 64;
+template <int D, int KB>
+struct SliceGeom {
+  static constexpr int kRows = kSliceWaves * KB * kResident;  // the longest slice
+  static constexpr int kTileBytes = kResident * D * 2;        // 32 rows of Q or dO
+  static constexpr int kExchange = kRows * kResident * 2;     // dS of 32 queries
+  static constexpr int kRingOff = kRows * D * 2;              // behind K
+  static constexpr int kOOff = kRingOff + 3 * 2 * kTileBytes;
+  static constexpr int kStOff = kOOff + kTileBytes;
+  static constexpr int kExOff = kStOff + 2 * kRows * 4;
+  static constexpr int kLds = kExOff + 2 * kExchange;
+};
+template <int D, int KB, bool CAUSAL>
+__global__ void __launch_bounds__(kSliceThreads, 1)
+fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
+                      const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
+                      const float* __restrict__ LSE, float* __restrict__ Delta, float* __restrict__ LSE2, half_t* __restrict__ dQ,
+                      half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, float c, float scale) {
+  using Geo = SliceGeom<D, KB>;
+  using T = SwzTile<D>;
+  constexpr int kKS = TileGeom<D>::kKSteps, kDB = TileGeom<D>::kDBlocks;
+  constexpr int kC = 2 * T::kNC / 4;  // copies of a wave per 32-row tile
+  __shared__ __attribute__((aligned(1024))) char smem[Geo::kLds];
+  char* const ring = smem + Geo::kRingOff;
+  float* const st_lse = reinterpret_cast<float*>(smem + Geo::kStOff);
+  float* const st_delta = st_lse + Geo::kRows;
+
+  // what depends on the lane is worked out again where it is needed, not kept in registers across the loop
+  auto thread_now = []() __attribute__((always_inline)) {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+  };
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bh = blockIdx.x, b = bh / H, h = bh - b * H;
+  const int rs = H * D;
+  const long head_off = ((long)b * N * H + h) * D;
+  const int nj = (N + kResident - 1) / kResident;  // 32-query tiles, 32-key blocks
+  const half_t* const Qb = Q + b * qs.b + (long)h * qs.h;
+  const half_t* const Gb = dO + b * gs.b + (long)h * gs.h;
+  const half_t* const Kb = K + b * ks.b + (long)h * ks.h;
+  int blk[KB];  // this wave's key blocks
+  blk[0] = wave;
+  const bool shared = D == 128 && !CAUSAL && nj == 5;  // waves 4 to 7 own block 4, each every fourth tile
+  if (shared && wave > 4) blk[0] = 4;
+  if constexpr (KB == 2) blk[KB - 1] = 2 * kSliceWaves - 1 - wave;
+
+  // Q (waves 0-3) or dO (4-7) of 32 rows
+  const bool copies_q = wave < 4;
+  const half_t* const c_base = copies_q ? Qb : Gb;
+  const int c_stride = copies_q ? qs.n : gs.n;
+  char* const c_dst = ring + (copies_q ? 0 : Geo::kTileBytes) + (wave & 3) * kC * 1024;
+  auto copy_tile = [&](int j, int slot) __attribute__((always_inline)) {
+    const int row0 = j * kResident;
+    const half_t* const base = c_base + (long)row0 * c_stride;
+    const int lane = thread_now() & 63;
+#pragma unroll
+    for (int u = 0; u < kC; ++u) {
+      int row, off;
+      copy_src<D>((wave & 3) * kC + u, lane, c_stride, row, off);
+      const int back = max(row0 + row - (N - 1), 0);  // rows past the end re-read row N-1
+      copy16(base, off - back * c_stride * 2, c_dst + slot * 2 * Geo::kTileBytes + u * 1024);
+    }
+  };
+  {  // K, all of it
+    constexpr int kPer = T::kInstrs / kSliceWaves;
+    int row[kPer], off[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) copy_src<D>(wave * kPer + u, threadIdx.x & 63, ks.n, row[u], off[u]);
+    for (int t = 0; t * kTile < N; ++t) {
+      const half_t* const base = Kb + (long)t * kTile * ks.n;
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        const int back = max(t * kTile + row[u] - (N - 1), 0);
+        copy16(base, off[u] - back * ks.n * 2, smem + t * T::kBytes + (wave * kPer + u) * 1024);
+      }
+    }
+  }
+  copy_tile(0, 0);
+
+  // V rows, negated
+  h8 vf[KB][kKS];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int lane = thread_now() & 63;
+    const half_t* const vp = V + b * vs.b + (long)h * vs.h + (long)min(blk[kb] * kResident + (lane & 31), N - 1) * vs.n +
+                             (lane >> 5) * 8;
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) vf[kb][kk] = *reinterpret_cast<const h8*>(vp + kk * 16);
+  }
+  // Row statistics of 32 rows, in the order of fmha_bwd_delta_kernel, by the first D / 16 waves.  The rows of O that a wave
+  // adds up it copies itself, 1 KiB of them, for its lanes to read back.
+  constexpr int kLanes = D / 8;
+  const bool makes_stats = wave < D / 16;
+  char* const o_mine = smem + Geo::kOOff + (wave & (D / 16 - 1)) * 1024;
+  char* const o_second = smem + Geo::kExOff + Geo::kExchange + (wave & (D / 16 - 1)) * 1024;  // free until dS of tile 1
+  auto stats_load = [&](int j, char* to) __attribute__((always_inline)) {
+    if (makes_stats) {
+      const int t = thread_now(), row0 = j * kResident;
+      copy16(O + head_off + (long)row0 * rs, (min(t / kLanes, N - 1 - row0) * rs + t % kLanes * 8) * 2, to);
+    }
+  };
+  auto stats_make = [&](int j, int slot, const char* from) __attribute__((always_inline)) {
+    if (makes_stats) {
+      const int t = thread_now(), st_row = t / kLanes, st_col = t % kLanes;
+      const h8 o8 = *reinterpret_cast<const h8*>(from + (t & 63) * 16);
+      // chunk st_col of row st_row of the tile of dO (SwzTile)
+      const h8 g8 = *reinterpret_cast<const h8*>(ring + slot * 2 * Geo::kTileBytes + Geo::kTileBytes +
+                                                 T::block_off(st_row >> 4, st_col >> 2) + (st_row & 15) * 64 +
+                                                 (((st_col & 3) ^ swz((st_row & 15) >> 2)) * 16));
+      float a = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a = fmaf((float)o8[e], (float)g8[e], a);
+      const auto dpp = [](float x, auto ctrl) __attribute__((always_inline)) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), decltype(ctrl)::value, 15, 15, true));
+      };
+      if (kLanes == 16) a += dpp(a, IntTag<0x128>{});                                       // of the lane at ^ 8 (of 16)
+      a += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(a), (4 << 10) | 31));  // ^ 4
+      a += dpp(a, IntTag<0x4E>{});                                                          // ^ 2
+      a += dpp(a, IntTag<0xB1>{});                                                          // ^ 1
+      const int at = j * kResident + st_row;
+      if (st_col == 0) {
+        st_delta[at] = a;
+        if (at < N) Delta[(long)bh * N + at] = a;
+      }
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the rows of O are read, others may take their place
+      asm volatile("" ::: "memory");
+    }
+  };
+  stats_load(0, o_mine);
+  if (nj > 1) {
+    copy_tile(1, 1);
+    stats_load(1, o_second);
+  }
+  if ((int)threadIdx.x < Geo::kRows) {
+    const int at = min((int)threadIdx.x, N - 1);
+    const float l2 = LSE[(long)bh * N + at] * kLog2e;
+    st_lse[threadIdx.x] = l2;
+    LSE2[(long)bh * N + at] = l2;  // rows past the end write that of row N-1 again
+  }
+
+  // LDS addresses of this lane's fragments: rows and columns of Q (+ kTileBytes: of dO) in slot 0, rows of this wave's K, and for
+  // dQ columns of K and dS: features 16 db .. and 16 of the 32 queries (D = 128: both halves).  Odd fragments of rows are at ^
+  // kOddRows, the upper eight rows of a fragment of columns at ^ kUpper, those of dS at + 256.
+  constexpr unsigned kOddRows = 32, kUpper = 512 + 32;
+  constexpr int kQB = D == 128 ? 2 : 1;
+  const int db = D == 128 ? wave : wave & 3, qb0 = D == 128 ? 0 : wave >> 2;
+  unsigned ra, ca, kr[KB], ka, ea;
+  {
+    const int lane = threadIdx.x & 63, L = lane & 15, g = lane >> 4, m = L & 3;
+    int r_off[2], t_off[2];
+    swz_rows_off<D>(lane, r_off);
+    swz_cols_off<D>(lane, t_off);
+    ra = opaque_lds_address(ring + r_off[0]);
+    ca = opaque_lds_address(ring + t_off[0]);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      kr[kb] = opaque_lds_address(smem + (blk[kb] >> 1) * T::kBytes + (blk[kb] & 1) * T::block_off(2, 0) + r_off[0]);
+    ka = opaque_lds_address(smem + cols16_off<D>(lane, 0, db & 1) + T::block_off(0, db >> 1));
+    ea = opaque_lds_address(smem + Geo::kExOff + qb0 * 1024 + (16 * (g >> 1) + 4 * (g & 1) + (L >> 2)) * 32 + (m & 1) * 16 +
+                            (m >> 1) * 8);
+  }
+
+  f16v dv[KB][kDB], dk[KB][kDB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+    for (int d = 0; d < kDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dv[kb][d][r] = dk[kb][d][r] = 0.f;
+
+  f16v zero;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+  wait_vm<0>();
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) {
+      vf[kb][kk] = -vf[kb][kk];
+      asm volatile("" : "+v"(vf[kb][kk]));  // negated here, not in the loop
+    }
+
+  // Fragments of LDS are read kLead units ahead of the MFMAs that take them, in an order that is written out and pinned.
+  auto in_order = [&](auto units_tag, auto lead_tag, auto read, auto use) __attribute__((always_inline)) {
+    constexpr int kUnits = decltype(units_tag)::value, kLead = decltype(lead_tag)::value;
+    decltype(read(0)) frag[kLead];
+#pragma unroll
+    for (int n = 0; n < kLead; ++n) frag[n] = read(n);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < kUnits; ++n) {
+      use(n, frag[n % kLead]);
+      if (n + kLead < kUnits) frag[n % kLead] = read(n + kLead);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // dQ of tile j
+  auto queries = [&](int j) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    struct Pair { h8 a, b[kQB]; };
+    const unsigned ex = ea + (j & 1) * Geo::kExchange;
+    const int n_blocks = CAUSAL ? j + 1 : nj;
+    f4v dq[kQB];
+#pragma unroll
+    for (int n = 0; n < kQB; ++n) dq[n] = f4v{0.f, 0.f, 0.f, 0.f};
+    auto both = [](unsigned a0, unsigned a1) __attribute__((always_inline)) {
+      const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)a0);
+      const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(uintptr_t)a1);
+      return __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    // every address is one of these and a constant
+    const unsigned k_lo = ka, k_hi = ka ^ kUpper;
+    auto read = [&](int kb) __attribute__((always_inline)) {
+      Pair f;
+      const unsigned kt = (kb >> 1) * T::kBytes + (kb & 1) * T::block_off(2, 0), et = kb * 2048;
+      f.a = both(k_lo + kt, k_hi + kt);
+#pragma unroll
+      for (int n = 0; n < kQB; ++n) f.b[n] = both(ex + (et + n * 1024), ex + (et + n * 1024 + 256));
+      return f;
+    };
+    auto use = [&](const Pair& f) __attribute__((always_inline)) {
+#pragma unroll
+      for (int n = 0; n < kQB; ++n) dq[n] = mfma16(f.a, f.b[n], dq[n]);
+    };
+    constexpr int kLead = 4, kMost = kSliceWaves * KB;
+    Pair frag[kLead];
+#pragma unroll
+    for (int u = 0; u < kLead; ++u) frag[u] = read(u);  // also past the last block: of no use then
+    __builtin_amdgcn_sched_barrier(0);
+    bool more = true;
+#pragma unroll
+    for (int kb = 0; kb < kMost; kb += kLead) {
+      if (!more) continue;
+      more = kb + kLead <= n_blocks;
+      if (more) {
+#pragma unroll
+        for (int u = 0; u < kLead; ++u) {
+          use(frag[u]);
+          if (kb + kLead < kMost) frag[u] = read(kb + kLead + u);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < kLead - 1; ++u)
+          if (kb + u < n_blocks) use(frag[u]);
+      }
+    }
+    const int lane = thread_now() & 63;
+#pragma unroll
+    for (int n = 0; n < kQB; ++n) {
+      const int q = j * kResident + 16 * (qb0 + n) + (lane & 15);
+      h4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (half_t)(dq[n][e] * scale);
+      if (q < N) *reinterpret_cast<h4*>(dQ + head_off + (long)q * rs + 16 * db + 4 * (lane >> 4)) = v;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // tile j, NB of this wave's key blocks
+  auto work = [&](int j, int slot, auto nb_tag, auto masked_tag) __attribute__((always_inline)) {
+    constexpr int NB = decltype(nb_tag)::value;
+    constexpr bool MASKED = decltype(masked_tag)::value != 0;
+    struct Rows { h8 a, k[NB]; };
+    const unsigned at = slot * 2 * Geo::kTileBytes;
+    const int q0 = j * kResident, lane = thread_now() & 63, i = lane & 31, hh = lane >> 5;
+    const char* const st = smem + Geo::kStOff + (q0 + 4 * hh) * 4;
+    f16v s[NB];
+    h8 y[NB][2];
+    {
+      const unsigned qa0 = ra + at, qa1 = qa0 ^ kOddRows;
+      in_order(IntTag<kKS>{}, IntTag<2>{}, [&](int kk) __attribute__((always_inline)) {
+        Rows f;
+        f.a = swz_rows_at<D>(qa0, qa1, 0, kk);
+#pragma unroll
+        for (int n = 0; n < NB; ++n) f.k[n] = swz_rows_at<D>(kr[n], kr[n] ^ kOddRows, 0, kk);
+        return f;
+      }, [&](int kk, const Rows& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) s[n] = mfma(f.a, f.k[n], kk == 0 ? zero : s[n]);
+      });
+    }
+    auto p_quad = [&](int quad) __attribute__((always_inline)) {
+      const f4v l4 = *reinterpret_cast<const f4v*>(st + 32 * quad);
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float p = fast_exp2(fmaf(s[n][4 * quad + r], c, -l4[r]));
+          if (MASKED) {
+            const int q = q0 + 8 * quad + 4 * hh + r;
+            if ((CAUSAL && blk[n] * kResident + i > q) || q >= N) p = 0.f;
+          }
+          y[n][quad >> 1][(quad & 1) * 4 + r] = (half_t)p;
+        }
+    };
+    p_quad(0);
+    p_quad(1);
+    __builtin_amdgcn_sched_barrier(0);
+    {  // the products with the first 16 queries while P of the others is formed
+      const unsigned a0 = ca + Geo::kTileBytes + at, a1 = a0 ^ kUpper;
+      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) { return swz_cols_at<D>(a0, a1, n / kDB, n % kDB); },
+               [&](int u, h8 f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) dv[n][u % kDB] = mfma(f, y[n][u / kDB], dv[n][u % kDB]);
+        if (u == 0) p_quad(2);
+        if (u == kDB / 2) p_quad(3);
+      });
+    }
+    f16v x[NB];
+    const char* const st2 = smem + Geo::kStOff + Geo::kRows * 4 + (q0 + 4 * ((thread_now() & 63) >> 5)) * 4;
+#pragma unroll
+    for (int quad = 0; quad < 4; ++quad) {
+      const f4v d4 = *reinterpret_cast<const f4v*>(st2 + 32 * quad);
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[n][4 * quad + r] = d4[r];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      const unsigned a0 = ra + Geo::kTileBytes + at, a1 = a0 ^ kOddRows;
+      in_order(IntTag<kKS>{}, IntTag<3>{}, [&](int kk) __attribute__((always_inline)) { return swz_rows_at<D>(a0, a1, 0, kk); },
+               [&](int kk, h8 f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) x[n] = mfma(f, vf[n][kk], x[n]);
+      });
+    }
+    // neg_mul_to_f16x8 is inline asm: the compiler leaves no time in front of it for the last MFMA's results to arrive
+    if constexpr (NB == 1) asm volatile("s_nop 15\n\ts_nop 7" : "+v"(x[0]));
+    else asm volatile("s_nop 15\n\ts_nop 7" : "+v"(x[0]), "+v"(x[NB - 1]));
+    __builtin_amdgcn_sched_barrier(0);
+    const int lane2 = thread_now() & 63, i2 = lane2 & 31;
+    char* const ex = smem + Geo::kExOff + (j & 1) * Geo::kExchange + (2 * i2 + (lane2 >> 5)) * 16;
+    auto ds_half = [&](int cc) __attribute__((always_inline)) {
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        float xr[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xr[e] = x[n][8 * cc + e];
+        y[n][cc] = neg_mul_to_f16x8(y[n][cc], xr);
+        if (blk[n] * kResident + kResident > N && blk[n] * kResident + i2 >= N) y[n][cc] = h8{};  // keys past the end: no dQ
+        *reinterpret_cast<h8*>(ex + blk[n] * 2048 + cc * 1024) = y[n][cc];
+      }
+    };
+    ds_half(0);
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      const unsigned a0 = ca + at, a1 = a0 ^ kUpper;
+      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) { return swz_cols_at<D>(a0, a1, n / kDB, n % kDB); },
+               [&](int u, h8 f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) dk[n][u % kDB] = mfma(f, y[n][u / kDB], dk[n][u % kDB]);
+        if (u == 0) ds_half(1);
+      });
+    }
+  };
+
+  block_barrier();
+  stats_make(0, 0, o_mine);
+  if (nj > 1) stats_make(1, 1, o_second);
+  int slot = 0, j = 0;
+  auto top = [&]() __attribute__((always_inline)) {
+    wait_vm<0>();  // tile j + 1 and its rows of O, asked for an iteration ago
+    block_barrier();
+    if (j > 0 && j + 1 < nj) stats_make(j + 1, slot == 2 ? 0 : slot + 1, o_mine);
+    if (j + 2 < nj) {
+      stats_load(j + 2, o_mine);
+      copy_tile(j + 2, slot == 0 ? 2 : slot - 1);
+    }
+    if (j > 0) queries(j - 1);
+  };
+  auto next = [&]() __attribute__((always_inline)) {
+    ++j;
+    slot = slot == 2 ? 0 : slot + 1;
+  };
+  // Tiles in which none, one or both of this wave's key blocks count; those on the diagonal of one and at the end of the slice
+  // with the mask, each in a loop of its own so that no accumulator crosses a branch.
+  const int whole = N / kResident;
+  auto span = [&](int end, int diag, auto nb_tag) __attribute__((always_inline)) {  // up to `end`, with a diagonal tile `diag`
+    while (j < end) {
+      while (j < end && (j == diag || j >= whole)) {
+        top();
+        work(j, slot, nb_tag, IntTag<1>{});
+        next();
+      }
+      while (j < end && j != diag && j < whole) {
+        top();
+        work(j, slot, nb_tag, IntTag<0>{});
+        next();
+      }
+    }
+  };
+  const int first = blk[0] >= nj ? nj : CAUSAL ? blk[0] : 0, second = blk[KB - 1] >= nj ? nj : CAUSAL ? blk[KB - 1] : 0;
+  while (j < first) {
+    top();
+    next();
+  }
+  if constexpr (D == 128 && !CAUSAL) {
+    if (shared && wave >= 4) {
+      for (int mine = wave - 4; mine < nj; mine += 4) {
+        while (j < mine) {
+          top();
+          next();
+        }
+        top();
+        work(j, slot, IntTag<1>{}, IntTag<1>{});
+        next();
+      }
+      while (j < nj) {
+        top();
+        next();
+      }
+    }
+  }
+  if constexpr (KB == 1) {
+    span(nj, CAUSAL ? blk[0] : -1, IntTag<1>{});
+  } else {
+    span(second, CAUSAL ? blk[0] : -1, IntTag<1>{});
+    span(nj, CAUSAL ? blk[1] : -1, IntTag<2>{});
+  }
+  top();
+
+  static_assert(kSliceWaves * StageGeom<D>::kBytes <= Geo::kExOff, "the output staging tiles do not reach the dS of a tile");
+  block_barrier();
+  char* const stage = smem + wave * StageGeom<D>::kBytes;
+  const int lane = thread_now() & 63;
+  if constexpr (D == 128 && !CAUSAL) {
+    if (shared) {  // the sums of the four waves, added in their order by the first one
+      constexpr int kQuads = kDB * 4, kOff = kSliceWaves * StageGeom<D>::kBytes;  // four sums of a lane at a time
+      static_assert(kOff + 3 * kQuads * 1024 <= Geo::kLds, "the sums of three waves fit, of dV and then of dK");
+      auto add = [&](f16v (&acc)[KB][kDB]) __attribute__((always_inline)) {
+        char* const at = smem + kOff + lane * 16;
+        if (wave > 4) {
+#pragma unroll
+          for (int u = 0; u < kQuads; ++u) {
+            f4v x;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = acc[0][u >> 2][4 * (u & 3) + r];
+            *reinterpret_cast<f4v*>(at + ((wave - 5) * kQuads + u) * 1024) = x;
+          }
+        }
+        block_barrier();
+        if (wave == 4) {
+          for (int other = 0; other < 3; ++other)
+#pragma unroll
+            for (int u = 0; u < kQuads; ++u) {
+              const f4v x = *reinterpret_cast<const f4v*>(at + (other * kQuads + u) * 1024);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[0][u >> 2][4 * (u & 3) + r] += x[r];
+            }
+        }
+        block_barrier();
+      };
+      add(dv);
+      add(dk);
+      if (wave > 4) return;
+    }
+  }
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    store_resident<D>(dV + head_off, rs, blk[kb] * kResident, N, dv[kb], 1.f, lane, stage);
+    store_resident<D>(dK + head_off, rs, blk[kb] * kResident, N, dk[kb], scale, lane, stage);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Host side: validation and launches.
 // ---------------------------------------------------------------------------
 // Limits of the 32-bit arithmetic in the kernels and of what a launch can take:
@@ -3298,7 +3784,7 @@ int dispatch_forward(const void* q, const fused_mha_strides* q_st, const void* k
 #undef FMHA_FWD
 }
 
-enum BwdPass { kPassDelta = 1, kPassDq = 2, kPassDkDv = 4, kPassAll = 7 };
+enum BwdPass { kPassDelta = 1, kPassDq = 2, kPassDkDv = 4, kPassAll = 7, kNotBySlice = 8 /* by the passes in any case */ };
 
 // Workspace of the backward: delta and lse * log2(e), fp32 (batch, head, n) each; then, for
 // the spill path, at the next multiple of 256 bytes, the fp16 dS tiles
@@ -3394,6 +3880,13 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
   };
   const float c = scale * kLog2e;
   const int nb = (n + 127) / 128;
+  if ((passes & kPassAll) == kPassAll && !(passes & kNotBySlice) && fmha_backward_by_slice(D, n, slices, cus, CAUSAL)) {
+    auto kernel = n <= 256 ? fmha_bwd_slice_kernel<D, 1, CAUSAL> : fmha_bwd_slice_kernel<D, D == 64 ? 2 : 1, CAUSAL>;
+    const hipError_t rc = launch(kernel, (unsigned)slices, kSliceThreads, stream, (const half_t*)q, (const half_t*)k, (const half_t*)v,
+                                 (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2, (half_t*)dq,
+                                 (half_t*)dk, (half_t*)dv, head, n, c, scale);
+    return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
+  }
   if ((passes & kPassAll) == kPassAll && fmha_passes_at_once(D, (long)nb * slices, n, cus, CAUSAL, spill)) {
     const bool stats = fmha_blocks_make_stats(D, n, CAUSAL);
     if (!stats && delta_pass() != hipSuccess) return FUSED_MHA_ERR_LAUNCH;
@@ -3605,6 +4098,7 @@ size_t fmha_backward_workspace_for(int batch, int head, int n, int d, int causal
   if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK) return 0;
   if (d == 64) return stats_bytes(batch, head, n);  // whatever the launches: the device is not asked
   const int cus = (int)persistent_grid(1 << 30);
+  if (fmha_backward_by_slice(d, n, batch * head, cus, causal != 0)) return stats_bytes(batch, head, n);
   if (fmha_passes_at_once(d, (long)key_blocks(n) * batch * head, n, cus, causal != 0)) return stats_bytes(batch, head, n);
   return best_workspace(batch, head, n, d, SIZE_MAX);
 }
@@ -3612,7 +4106,8 @@ size_t fmha_backward_workspace_for(int batch, int head, int n, int d, int causal
 size_t fmha_backward_count_bytes(int batch, int head, int n, int d, int causal) {
   if (check_shape(batch, head, n, n, d) != FUSED_MHA_OK || d == 64) return 0;
   const int cus = (int)persistent_grid(1 << 30), slices = batch * head;
-  if (fmha_passes_at_once(d, (long)key_blocks(n) * slices, n, cus, causal != 0) ||
+  if (fmha_backward_by_slice(d, n, slices, cus, causal != 0) ||
+      fmha_passes_at_once(d, (long)key_blocks(n) * slices, n, cus, causal != 0) ||
       slices * slice_bytes(n) > FUSED_MHA_SPILL_MAX_BYTES || !fmha_ds_in_one_launch(slices, n, cus, causal != 0))
     return 0;
   return ready_bytes(slices);
@@ -3622,8 +4117,8 @@ int fmha_backward_waiting(const void* query_ptr, const void* key_ptr, const void
                           const void* d_output_ptr, const void* lse_ptr, void* workspace, size_t workspace_bytes,
                           void* d_query_ptr, void* d_key_ptr, void* d_value_ptr, int batch, int head, int n, int d, float scale,
                           int causal, unsigned ticks, void* stream) {
-  return dispatch_backward(kPassAll, query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr, d_output_ptr, nullptr,
-                           lse_ptr, workspace, workspace_bytes, d_query_ptr, d_key_ptr, d_value_ptr, batch, head, n, n, d, scale,
+  return dispatch_backward(kPassAll | kNotBySlice, query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr,
+                           d_output_ptr, nullptr, lse_ptr, workspace, workspace_bytes, d_query_ptr, d_key_ptr, d_value_ptr, batch, head, n, n, d, scale,
                            causal, stream, ticks);
 }
 

@@ -126,7 +126,9 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * go into one launch and form S and dP twice, whatever the size.  That depends
  * on the mask and the device, which this function does not know, so it returns
  * room for dS for those too (2 GiB for one causal slice of n = 32768); the
- * minimum is as fast for them.
+ * minimum is as fast for them.  The same goes for many problems of at least
+ * half as many slices as the device has compute units and n <= 32768 / d, of
+ * which one compute unit does a whole slice, with S and dP formed once.
  * With d = 128 and, behind room for the dS of all slices, another 128 bytes for
  * each (batch, head) slice, both passes go in one launch where that is faster
  * (many problems of up to a few blocks of 128 rows per compute unit); the

@@ -75,7 +75,8 @@ def test_backward_d64_has_the_bits_of_the_general_passes(N, causal):
 @pytest.mark.gpu
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,H,N,room", [
-    (1, 1025, 64, 512),   # three rounds of 344 slices, the last one smaller
+    (1, 1025, 64, 512),   # three rounds of 344 slices, the last one smaller: had a slice not a work group of its own
+    (1, 1030, 100, 512),  # the same where it has not
     (2, 129, 129, 256),   # two rounds, the workspace one slice pair short of one
     (7, 57, 300, 200),    # two rounds that do not end at a batch, the full room used
     (3, 100, 300, 170),   # rounds of fewer than two blocks per compute unit: recomputes instead
@@ -121,6 +122,53 @@ def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
             assert torch.equal(a, b[:, :, h:h + 1])
 
 
+BY_SLICE = [(D, N, causal) for causal in (False, True) for D, Ns in (
+    (128, (1, 2, 31, 32, 33, 63, 64, 65, 96, 100, 127, 128, 129, 130, 159, 160, 161, 192, 193, 223, 224, 225, 255, 256)),
+    (64, (129, 159, 160, 161, 192, 193, 200, 256, 257, 287, 288, 289, 320, 383, 384, 385, 449, 480, 481, 511, 512)))
+            for N in Ns if not (D == 64 and causal and 200 < N <= 256)]
+
+
+def test_by_slice_cases(tmp_path):
+    """The cases below have a work group for each of 256 slices on 256 compute units."""
+    assert all(abi.host_rule(tmp_path, "fmha_backward_by_slice(x[0], x[1], 256, 256, x[2])", BY_SLICE))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,N,causal", BY_SLICE)
+def test_a_work_group_for_each_slice(D, N, causal):
+    """The bits of the passes one by one, delta too, also with strides and with the least workspace; every element of the
+    gradients and none of the workspace but the statistics is written."""
+    B, lib, scale = 2, abi.load(), D ** -0.5
+    H = torch.cuda.get_device_properties(0).multi_processor_count // B
+    gen = torch.Generator(device="cuda").manual_seed(N + D)
+    packed = torch.randn(B, N, 4, H, D, device="cuda", dtype=torch.float16, generator=gen)
+    dense = [packed[:, :, i].contiguous() for i in range(4)]
+    out, lse = abi.forward(lib, *dense[:3], scale, causal)
+    want = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal, split=True)
+    got = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal, poison=True)
+    least = abi.backward(lib, *dense[:3], out, dense[3], lse, scale, causal, poison=True, min_workspace=True)
+    strided = abi.backward_strided(lib, *(packed[:, :, i] for i in range(3)), out, packed[:, :, 3], lse, scale, causal)
+    for a, b, c in zip(got, want, least):
+        assert torch.equal(a, b) and torch.equal(c, b)
+    for a, b in zip(strided, want):
+        assert torch.equal(a, b)
+    ref = ao.attention_backward(*(t[:1, :, :2].cpu() for t in dense), scale, causal)
+    for a, b in zip(got, ref):
+        # fp16 roundings of P, dS, delta's O and the result: the repository's bound for gradients of order 1
+        assert (a[:1, :, :2].float().cpu() - b.half().float()).abs().max() <= 1e-2
+    words = 2 * B * H * N  # delta and lse * log2(e)
+    ws = torch.full((words + 64,), float("nan"), device="cuda")
+    grads = [torch.full_like(g, float("nan")) for g in got[:3]]
+    rc = lib.fused_mha_backward(*(t.data_ptr() for t in (*dense[:3], out, dense[3], lse, ws)), 4 * ws.numel(),
+                                *(g.data_ptr() for g in grads), B, H, N, N, D, scale, int(causal),
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == abi.OK
+    assert not torch.isnan(ws[:words]).any() and torch.isnan(ws[words:]).all()
+    assert torch.equal(ws[words // 2:words], (lse * torch.tensor(1.4426950408889634, device="cuda")).flatten())
+    for a, b in zip(grads, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ticks", [5000000, 0])
 @pytest.mark.parametrize("H,N,causal", [
@@ -133,16 +181,13 @@ def test_a_slice_alone_gives_the_same_gradients(H, N, causal):
 def test_both_passes_over_ds_in_one_launch(H, N, causal, ticks):
     """The bits of the passes one after the other, also (ticks) where no block waits for the dS of another."""
     B, D, lib = 1, 128, abi.load()
-    lib.fmha_backward_count_bytes.argtypes, lib.fmha_backward_count_bytes.restype = [ctypes.c_int] * 5, ctypes.c_size_t
     lib.fmha_backward_waiting.argtypes = ([ctypes.c_void_p] * 7 + [ctypes.c_size_t] + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 +
                                           [ctypes.c_float, ctypes.c_int, ctypes.c_uint, ctypes.c_void_p])
     gen = torch.Generator(device="cuda").manual_seed(N + H)
     q, k, v, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
     out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
     apart = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=True)[:3]
-    counts = lib.fmha_backward_count_bytes(B, H, N, D, int(causal))
-    assert counts == 128 * H
-    nbytes = lib.fused_mha_backward_workspace_bytes(B, H, N, D) + counts
+    nbytes = lib.fused_mha_backward_workspace_bytes(B, H, N, D) + 128 * H  # room for the counts of this launch
     ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
     for _ in range(2):
         got = [torch.full_like(q, float("nan")) for _ in range(3)]
@@ -288,6 +333,7 @@ HINT_ON_DS = [  # H, N, causal, whether the passes are called one by one, whethe
     (511, 127, False, True, True), (512, 127, False, True, False),
     (56, 384, False, False, True), (57, 384, False, False, False),     # 15.8 and 16.03
     (511, 50, True, True, True), (513, 50, True, False, False),        # 7.98 and 8.02 MiB
+    (513, 50, True, True, False),                                      # one by one: whole, it has a work group for each slice
     (4, 1024, False, True, True), (5, 1024, False, True, False),       # 8 and 10 MiB
     (5, 1025, True, True, True), (9, 1025, True, True, False),         # 6.3 and 11.4 MiB
     (63, 1031, False, False, False), (64, 1031, False, False, True),   # 255 and 259 MiB of dS and tensors

@@ -470,14 +470,38 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_backward_by_slice(tmp_path, lib):
+    """D, N, slices, causal of backwards timed both ways on 256 compute units; and what the extension takes for them."""
+    rule = "fmha_backward_by_slice(x[0], x[1], x[2], 256, x[3])"
+    slices = [
+        (128, 1, 129, 0), (128, 256, 129, 1), (128, 256, 256, 0), (128, 100, 257, 0), (128, 200, 320, 0), (128, 160, 320, 1),
+        (128, 256, 342, 1), (128, 33, 514, 0), (128, 100, 640, 1), (128, 256, 514, 0), (128, 100, 1600, 0), (128, 64, 3000, 1),
+        (64, 129, 129, 0), (64, 257, 192, 0), (64, 512, 192, 0), (64, 300, 400, 0), (64, 512, 600, 0), (64, 512, 1300, 0),
+        (64, 129, 171, 1), (64, 160, 448, 1), (64, 200, 224, 1), (64, 384, 256, 1), (64, 512, 224, 1), (64, 512, 448, 1),
+        (64, 512, 1030, 1),
+    ]
+    other = [
+        (128, 1, 128, 0), (128, 257, 200, 0), (128, 256, 319, 0), (128, 256, 330, 1), (128, 100, 528, 0), (128, 100, 1030, 1),
+        (64, 128, 256, 0), (64, 129, 128, 0), (64, 257, 176, 0), (64, 300, 384, 0), (64, 512, 590, 0), (64, 513, 256, 0),
+        (64, 129, 160, 1), (64, 201, 256, 1), (64, 200, 480, 1), (64, 300, 480, 1), (64, 512, 208, 1), (64, 512, 640, 1),
+        (64, 300, 1030, 1), (64, 512, 96, 0), (128, 1, 1, 0), (64, 1, 1 << 23, 0),
+    ]
+    assert all(abi.host_rule(tmp_path, rule, slices)) and not any(abi.host_rule(tmp_path, rule, other))
+    f = lib.fmha_backward_workspace_for
+    f.argtypes, f.restype = [ctypes.c_int] * 5, ctypes.c_size_t
+    for D, N, S, causal in slices:  # no room for dS
+        assert f(1, S, N, D, causal) == lib.fused_mha_backward_min_workspace_bytes(1, S, N, D)
+
+
 def test_count_bytes(lib):
     """What the extension adds behind the dS of all slices, on 256 compute units: 128 bytes a slice where one launch does both
     passes, nothing elsewhere."""
     f = lib.fmha_backward_count_bytes
     f.argtypes, f.restype = [ctypes.c_int] * 5, ctypes.c_size_t
-    assert f(3, 20, 1031, 128, 0) == 60 * 128 and f(16, 12, 512, 128, 1) == 192 * 128 and f(1, 600, 64, 128, 0) == 600 * 128
+    assert f(3, 20, 1031, 128, 0) == 60 * 128 and f(16, 12, 512, 128, 1) == 192 * 128 and f(1, 600, 100, 128, 0) == 600 * 128
     assert f(2, 32, 4096, 128, 1) == 0    # the dQ pass alone has blocks of 256 queries there
     assert f(1, 4, 1031, 128, 0) == 0     # few blocks: one launch that forms S and dP twice
+    assert f(1, 600, 64, 128, 0) == 0     # a work group for each slice
     assert f(16, 12, 512, 64, 0) == 0 and f(1, 0, 512, 128, 0) == 0
     assert f(1, 33000, 512, 128, 0) == 0  # dS in rounds
 
