@@ -183,6 +183,39 @@ FMHA_HOST_DEVICE int fmha_paired_block(int lin, int total) {
   return ((kCus / 8 + slots - 1 - (lin >> 3)) << 3) + xcd;
 }
 
+// The 128-query forward without a mask where the last block of every slice has up to 32 queries: those of `per` (2 or 4) slices
+// can go to one block, a wave each (fwd_tail_rows), in front of all others; as many blocks as a multiple of 8, so that the others
+// stay on the XCD of their slice.  Work group `lin` and wave -> slice; one past the last means none.
+FMHA_HOST_DEVICE int fmha_tail_blocks(int slices, int per) { return ((slices + per - 1) / per + 7) & ~7; }
+FMHA_HOST_DEVICE int fmha_tail_slice(int lin, int wave, int tails, int per) {
+  return per * ((lin & 7) * (tails >> 3) + (lin >> 3)) + wave;  // an XCD has slices next to each other here too
+}
+
+// Whether they do: 0, or how many to a block.  Blocks of the same length are done in layers of one to a CU, and it pays where
+// there are fewer of those.  Two to a block where that gives as few as four does, since four streams of K and V are slow beside
+// another block.  us of the forward with a block for each, two and four to a block, N x slices (layers):
+// D = 64.  129 x 230 (2, 2, 2) 7.8, 8.0, 8.3; 129 x 300 (3, 2, 2) 11.5, 8.7, 8.7; 129 x 400 (4, 3, 2) 13.9, 11.8, 9.5; 129 x 512
+// (4, 3, 3) 16.4, 12.1, 12.8; 129 x 4000 (32, 24, 20) 99.0, 80.2, 77.8; 257 x 100 (2, 1, 1) 9.6, 7.7, 7.8; 257 x 400 (5, 4, 4)
+// 24.9, 22.1, 21.8; 520 x 110 (3, 2, 2) 21.8, 17.1, 18.1; 520 x 120 (3, 3, 2) 22.0, 22.1, 18.4; 520 x 150 (3, 3, 3) 24.0, 24.4,
+// 23.4; 660 x 90 (3, 2, 2) 24.9, 19.8, 20.7; 1031 x 56 (2, 2, 2) 26.5, 27.2, 27.9; 1031 x 60 (3, 2, 2) 31.8, 27.9, 28.5; 1031 x 230
+// (9, 8, 8) 98.5, 94.6, 92.4; 2070 x 31 (3, 2, 2) 54.5, 48.8, 49.7; 2070 x 200 (14, 13, 13) 276, 275, 268.
+// D = 128.  129 x 230 (2, 2, 2) 13.7, 11.9, 13.7; 129 x 300 (3, 2, 2) 19.6, 13.2, 14.8; 257 x 200 (3, 2, 2) 23.9, 20.2, 21.8; 257 x
+// 700 (9, 7, 7) 67.2, 60.4, 57.2; 520 x 56 (2, 1, 1) 20.9, 17.9, 18.8; 520 x 64 (2, 2, 2) 21.9, 23.1, 24.4; 520 x 600 (12, 11, 10)
+// 138, 136, 130; 1031 x 56 (2, 2, 2) 41.9, 44.2, 46.0; 1031 x 60 (3, 2, 2) 50.1, 46.0, 48.0; 1031 x 120 (5, 4, 4) 87.9, 82.7, 81.0;
+// 1300 x 48 (3, 2, 2) 58.2, 53.8, 56.8; 2070 x 31 (3, 2, 2) 88.6, 81.8, 84.2.
+// Not past three rounds of longer ones at D = 128: 1031 x 200 (8, 7, 7) 146, 150, 150; 2070 x 230 (16, 15, 15) 550, 579, 539.
+// Nor from two layers to one where it is the wave on its own that takes the time: D = 64 660 x 45 15.6, 13.8, 15.4; 1031 x 30
+// 20.4, 20.6, 21.7; 1300 x 24 23.8, 24.9, 25.9; and with four to a block 900 x 34 18.7, 21.7, 19.5.  D = 128 1031 x 30 31.8, 29.1,
+// 31.7; 900 x 34 28.8, 32.8, 28.8.
+FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus) {
+  if (n <= 128 || (n - 1) % 128 >= 32) return 0;
+  const long full = (long)slices * ((n - 1) / 128);
+  const long now = (full + slices + cus - 1) / cus, two = (full + fmha_tail_blocks(slices, 2) + cus - 1) / cus,
+             four = (full + fmha_tail_blocks(slices, 4) + cus - 1) / cus;
+  if (n > 768 && ((d == 128 && now > 6) || (now == 2 && (d == 64 || two == 2)))) return 0;
+  return two < now && two <= four ? 2 : four < now ? 4 : 0;
+}
+
 // A launch of two passes with `nb` blocks each per slice: the blocks of both in turn, ordered as one pass's are (heaviest of
 // both first, or the short last ones of both at the end).
 FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heavy_first, bool short_last, int& slice, int& blk,

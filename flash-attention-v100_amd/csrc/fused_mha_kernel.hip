@@ -1007,6 +1007,7 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
 // the chip runs at its power limit (B1 H12 N8192 D64: 263 -> 220 us).
 // Small blocks cost twice the K/V copies per query of 256-query blocks and are worth it for balance: B1 H32 N1500 D128
 // causal 41 -> 31 us, B4 H16 N1024 D64 causal 24 -> 17 us, B16 H12 N512 D64 24 -> 20 us, B3 H20 N1031 D128 67 -> 50 us.
+// Where the last block of a slice has up to 32 queries, one wave of four works: fwd_tail_rows.
 // Three blocks per CU at D = 64 (168 registers) gain 2 % on the long shape and lose 2-5 % on the short ones: not taken.
 //
 // The maximum is handled as in fmha_fwd_kernel.  Bringing it up to date happens outside the main loop.  K and V have two
@@ -1032,11 +1033,174 @@ __device__ __forceinline__ void odd_slots_first() {
   if (slot & 1) __builtin_amdgcn_s_setprio(1);
 }
 
-template <int D, bool CAUSAL, bool ODD_FIRST>
+// The last, up to 32, queries of a slice by one wave for itself, with no other wave or barrier (rule: fmha_tails_per_block).  As
+// a block of their own they take a whole place of a CU for three waves that do nothing; here two or four slices share one.  K and V
+// of 64 keys take turns in a tile of LDS that is the wave's own: K(t + 1) comes while the scores of tile t are formed from
+// registers and goes to registers, V(t) then comes while the softmax is.  Not interleaved further: at D = 128 the registers are
+// used up.  A tile takes 2,500 cycles (kernel below: 1,850 for a wave alone), of which the MFMAs take 2,048; all that counts
+// is that the block ends before the others of its round, so its waves go first wherever they could issue (a tail that is
+// still there when the others have ended: 4100 x 20 slices, D = 128, 186 us without, 170 with).  Two tiles of LDS to a wave, so that
+// copies are under way longer: nothing gained.  All sums are those of the kernel below, in the same order.
+template <int D>
+__device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, const half_t* __restrict__ K,
+                                              const half_t* __restrict__ V, Strides qs, Strides ks, Strides vs,
+                                              half_t* __restrict__ O, float* __restrict__ LSE, int H, int N, int bh, float c,
+                                              int negate_q, char* ring) {
+  using G = TileGeom<D>;
+  using T = SwzTile<D>;
+  constexpr int kKS = G::kKSteps, kDB = G::kDBlocks;
+  __builtin_amdgcn_s_setprio(3);
+  const int lane = threadIdx.x & 63, i = lane & 31, hh = lane >> 5;
+  const int b = bh / H, h = bh - b * H, nt = (N + kTile - 1) / kTile, q0 = (N - 1) / kPipeBlockQ * kPipeBlockQ;
+  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+  auto copy = [&](const half_t* base, int stride, int t) __attribute__((always_inline)) {
+    constexpr int kBack = 960 * (T::kNC - 1);  // see copy16_blocks
+    base += (long)t * kTile * stride - kBack / 2;
+    const int r16 = lane >> 2, col = ((lane & 3) ^ swz(r16 >> 2)) * 16 + kBack;
+#pragma unroll
+    for (int R = 0; R < 4; ++R) {
+      const int row = 16 * R + r16, back = max(t * kTile + row - (N - 1), 0);  // rows past the end re-read row N-1
+      copy16_blocks<T::kNC>(base, (row - back) * stride * 2 + col, lds + T::block_off(R, 0));
+    }
+  };
+  const half_t* const Kb = K + b * ks.b + (long)h * ks.h;
+  const half_t* const Vb = V + b * vs.b + (long)h * vs.h;
+  copy(Kb, ks.n, 0);
+  h8 qf[kKS];
+  {
+    const half_t* const qp = Q + b * qs.b + (long)h * qs.h + (long)min(q0 + i, N - 1) * qs.n + hh * 8;
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk) {
+      qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
+      if (negate_q) qf[kk] = -qf[kk];
+    }
+  }
+  unsigned ka0, ka1, va0, va1;
+  {
+    int k_off[2], v_off[2];
+    swz_rows_off<D>(lane, k_off);
+    swz_cols_off<D>(lane, v_off);
+    ka0 = opaque_lds_address(ring + k_off[0]);
+    ka1 = opaque_lds_address(ring + k_off[1]);
+    va0 = opaque_lds_address(ring + v_off[0]);
+    va1 = opaque_lds_address(ring + v_off[1]);
+  }
+  f16v o[kDB], s[2], zero;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+#pragma unroll
+  for (int db = 0; db < kDB; ++db) o[db] = zero;
+  float mc = -INFINITY, l_run = 0.f;
+  u4v pf[4];
+  auto exponentials = [&]() __attribute__((always_inline)) {
+    float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+    for (int c16 = 0; c16 < 4; ++c16) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float p0 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e], c, -mc));
+        const float p1 = fast_exp2(fmaf(s[c16 >> 1][(c16 & 1) * 8 + e + 1], c, -mc));
+        pf[c16][e >> 1] = pack_f16(p0, p1);
+        if (D == 64) {
+          l0 += p0;
+          l1 += p1;
+        } else {
+          float& l = c16 & 1 ? l1 : l0;
+          l += p0;
+          l += p1;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return l0 + l1;
+  };
+  auto lds_read = []() __attribute__((always_inline)) {  // the tile is read: another may take its place
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  h8 kf[2][kKS];
+  auto read_k = [&]() __attribute__((always_inline)) {
+    wait_vm<0>();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) kf[rb][kk] = swz_rows_at<D>(ka0, ka1, rb, kk);
+    lds_read();
+  };
+  read_k();
+  if (nt > 1) copy(Kb, ks.n, 1);
+  for (int t = 0; t < nt; ++t) {
+#pragma unroll
+    for (int kk = 0; kk < kKS; ++kk)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) s[rb] = mfma(kf[rb][kk], qf[kk], kk == 0 ? zero : s[rb]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 < nt) read_k();
+    copy(Vb, vs.n, t);
+    __builtin_amdgcn_sched_barrier(0);
+    if (t == nt - 1) {  // the only tile with keys that do not count
+      const int last = N - 1 - t * kTile - 4 * hh;
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (acc_row(rb, r, 0) > last) s[rb][r] = -INFINITY;
+    }
+    float lt = 0.f;
+    bool raise = t == 0 || t == nt - 1;
+    if (!raise) {
+      lt = exponentials();
+      raise = __builtin_amdgcn_ballot_w64(!(lt <= kRescaleSum)) != 0;
+    }
+    if (raise) {  // the maximum is brought up to date, as by raise_max of the kernel below
+      float mx = s[0][0];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
+      mx = fmaxf(mx, other_half(mx));
+      const float mc_new = fmaxf(mc, mx * c);
+      const float alpha = fast_exp2(mc - mc_new);
+      mc = mc_new;
+      l_run *= alpha;
+      asm volatile("" : "+v"(l_run));
+#pragma unroll
+      for (int db = 0; db < kDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+      lt = exponentials();
+    }
+    l_run += lt;
+    wait_vm<0>();
+    asm volatile("" ::: "memory");
+    {
+      constexpr int kLead = 4, kNP = 4 * kDB;
+      h8 frag[kLead];
+#pragma unroll
+      for (int n = 0; n < kLead; ++n) frag[n] = swz_cols_at<D>(va0, va1, n / kDB, n % kDB);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < kNP; ++n) {
+        o[n % kDB] = mfma(frag[n % kLead], __builtin_bit_cast(h8, pf[n / kDB]), o[n % kDB]);
+        if (n + kLead < kNP) frag[n % kLead] = swz_cols_at<D>(va0, va1, (n + kLead) / kDB, (n + kLead) % kDB);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    lds_read();
+    if (t + 2 < nt) copy(Kb, ks.n, t + 2);
+  }
+  const float l_tot = l_run + other_half(l_run);
+  store_resident<D>(O + ((long)b * N * H + h) * D, H * D, q0, N, o, 1.f / l_tot, lane, ring);
+  if (LSE && lane < 32 && q0 + i < N) LSE[((long)b * H + h) * N + q0 + i] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
+}
+
+template <int D, bool CAUSAL, bool ODD_FIRST, bool TAIL>
 __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                      Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
-                     int nmb, float c, int negate_q) {
+                     int nmb, int slices, int tails_per_block, float c, int negate_q) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
   constexpr int kDB = G::kDBlocks;
@@ -1055,8 +1219,18 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     return t & 63;
   };
   int bh, mb;
-  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
-                       N % kPipeBlockQ != 0, bh, mb);
+  if constexpr (TAIL) {
+    const int tails = fmha_tail_blocks(slices, tails_per_block);
+    if ((int)blockIdx.x < tails) {
+      bh = fmha_tail_slice(blockIdx.x, wave, tails, tails_per_block);
+      if (wave < tails_per_block && bh < slices) fwd_tail_rows<D>(Q, K, V, qs, ks, vs, O, LSE, H, N, bh, c, negate_q, smem + wave * T::kBytes);
+      return;
+    }
+    fmha_slice_and_block(blockIdx.x - tails, slices, nmb - 1, bh, mb);
+  } else {
+    fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
+                         N % kPipeBlockQ != 0, bh, mb);
+  }
   const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O is dense
@@ -3758,12 +3932,23 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
     }
   }
   const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ, total = nmb * batch * head;
-  auto kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false>;
-  if constexpr (!CAUSAL)
-    if (half_round_left(total, n, 2)) kernel = fmha_fwd_pipe_kernel<D, CAUSAL, true>;
-  const hipError_t rc = launch(kernel, (unsigned)total, kPipeThreads, stream, (const half_t*)q,
-                               (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, c,
-                               negate);
+  const int slices = batch * head;
+  int tails_per_block = 0;
+  auto kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, false>;
+  unsigned blocks = total;
+  if constexpr (!CAUSAL) {
+    static_assert(kPipeBlockQ == 128 && kResident == 32, "as fmha_tails_per_block has it");
+    tails_per_block = fmha_tails_per_block(D, n, slices, (int)persistent_grid(1 << 30));
+    if (tails_per_block) blocks = fmha_tail_blocks(slices, tails_per_block) + slices * (nmb - 1);
+    const bool odd_first = half_round_left(blocks, n, 2);
+    if (tails_per_block)
+      kernel = odd_first ? fmha_fwd_pipe_kernel<D, CAUSAL, true, true> : fmha_fwd_pipe_kernel<D, CAUSAL, false, true>;
+    else if (odd_first)
+      kernel = fmha_fwd_pipe_kernel<D, CAUSAL, true, false>;
+  }
+  const hipError_t rc = launch(kernel, blocks, kPipeThreads, stream, (const half_t*)q,
+                               (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, slices,
+                               tails_per_block, c, negate);
   return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
 }
 

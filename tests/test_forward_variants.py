@@ -232,3 +232,81 @@ def test_rows_that_are_not_finite(B, H, N, D, causal):
     assert (out[:, good, h].float().cpu() - ref[:, good, 0].half().float()).abs().max() <= 2e-3
     assert (lse[:, h, good].cpu() - ref_lse[:, 0, good]).abs().max() <= 2e-3
     assert (dq[:, good, h].float().cpu() - ref_dq[:, good, 0].half().float()).abs().max() <= 1e-2
+
+
+TAILS = [  # D, slices, N, how many slices' last rows go to one block
+    (64, 300, 129, 2), (64, 401, 150, 4), (64, 100, 257, 2), (64, 110, 520, 2), (64, 118, 544, 4), (64, 59, 1031, 2),
+    (64, 61, 1537, 2), (128, 300, 160, 2), (128, 181, 130, 4), (128, 203, 257, 2), (128, 150, 400, 4), (128, 57, 1056, 2),
+    (128, 122, 1025, 4), (64, 62, 1550, 4),
+]
+
+
+def test_blocks_with_the_last_rows_of_slices(tmp_path):
+    """The cases below on 256 compute units and others left alone; every slice's last rows once, on few XCDs."""
+    rule = "fmha_tails_per_block(x[0], x[2], x[1], 256) == x[3]"
+    alone = [(64, 300, 128, 0), (64, 300, 161, 0), (64, 230, 129, 0), (64, 256, 257, 0), (64, 30, 1031, 0), (64, 34, 900, 0),
+             (128, 56, 1031, 0), (128, 200, 1031, 0), (128, 34, 900, 0), (128, 1, 129, 0), (64, 1, 1, 0), (128, 230, 2070, 0)]
+    assert all(abi.host_rule(tmp_path, rule, TAILS + alone))
+    src, exe = tmp_path / "tails.cpp", tmp_path / "tails"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (int per = 2; per <= 4; per += 2)
+    for (int slices = 1; slices <= 900; ++slices) {
+      const int tails = fmha_tail_blocks(slices, per);
+      std::vector<int> seen(slices, 0);
+      for (int lin = 0; lin < tails; ++lin)
+        for (int wave = 0; wave < per; ++wave) {
+          const int s = fmha_tail_slice(lin, wave, tails, per);
+          if (s < 0 || (s < slices && seen[s]++)) { printf("slice %d %d %d\n", per, slices, lin); return 1; }
+        }
+      for (int s = 0; s < slices; ++s)
+        if (!seen[s]) { printf("none %d %d %d\n", per, slices, s); return 1; }
+      if (tails % 8 || per * tails >= slices + 8 * per) { printf("many %d %d\n", per, slices); return 1; }
+    }
+  for (int d = 64; d <= 128; d += 64)
+    for (int n = 1; n <= 1200; ++n)
+      for (int slices = 1; slices <= 700; slices += 3) {
+        const int per = fmha_tails_per_block(d, n, slices, 256);
+        if (per && per != 2 && per != 4) return 1;
+        if (per && fmha_tail_blocks(slices, per) >= slices) { printf("gain %d %d\n", n, slices); return 1; }
+      }
+  puts("ok");
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,H,N,per", TAILS)
+def test_last_rows_of_several_slices_in_one_block(D, H, N, per):
+    """The bits of launches of a few slices, in which each has a block for its last rows, without a mask; with maxima that are
+    raised at nearly every tile, with strides and a negative scale, with rows that are not finite."""
+    lib = abi.load()
+    last = (N - 1) // 128 * 128
+    for kind in ("plain", "growing", "strided", "not finite"):
+        q, k, v = (t.cuda() for t in _inputs(1, N, H, D, kind == "growing"))
+        scale = {"growing": 1.0, "strided": -(D ** -0.5)}.get(kind, D ** -0.5)
+        if kind == "not finite":
+            q[:, last, 1, 3], q[:, N - 1, H // 2, 5], k[:, N - 1, H - 1, 0] = float("nan"), float("inf"), float("inf")
+        if kind == "strided":
+            q, k, v = torch.stack((q, k, v), dim=2).unbind(2)
+            out, lse = abi.forward_strided(lib, q, k, v, scale, False)
+        else:
+            out, lse = abi.forward(lib, q, k, v, scale, False)
+        for h in range(0, H, 13):
+            few = [t[:, :, h:h + 13].contiguous() for t in (q, k, v)]
+            o, l = abi.forward(lib, *few, scale, False)
+            assert torch.equal(o.view(torch.int16), out[:, :, h:h + 13].contiguous().view(torch.int16)) or (
+                kind == "not finite" and torch.equal(o.isnan(), out[:, :, h:h + 13].isnan()) and
+                torch.equal(o.nan_to_num(), out[:, :, h:h + 13].nan_to_num()))
+            assert torch.equal(l.nan_to_num(), lse[:, h:h + 13].nan_to_num())
+            if h == 0 and kind in ("plain", "growing"):
+                ref, ref_lse = ao.attention_forward(*(t[:, :, :2].cpu() for t in few), scale, False)
+                # the bounds of _check
+                assert (o[:, :, :2].float().cpu() - ref.half().float()).abs().max() <= 2e-3 * max(1.0, ref.abs().max().item())
+                assert ((l[:, :2].cpu() - ref_lse).abs() <= 2e-3 + 1e-6 * ref_lse.abs()).all()
