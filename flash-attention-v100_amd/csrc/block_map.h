@@ -183,7 +183,7 @@ FMHA_HOST_DEVICE int fmha_paired_block(int lin, int total) {
   return ((kCus / 8 + slots - 1 - (lin >> 3)) << 3) + xcd;
 }
 
-// The 128-query forward without a mask where the last block of every slice has up to 32 queries: those of `per` (2 or 4) slices
+// The 128-query forward where the last block of every slice has up to 32 queries: those of `per` (2 or 4) slices
 // can go to one block, a wave each (fwd_tail_rows), in front of all others; as many blocks as a multiple of 8, so that the others
 // stay on the XCD of their slice.  Work group `lin` and wave -> slice; one past the last means none.
 FMHA_HOST_DEVICE int fmha_tail_blocks(int slices, int per) { return ((slices + per - 1) / per + 7) & ~7; }
@@ -207,11 +207,23 @@ FMHA_HOST_DEVICE int fmha_tail_slice(int lin, int wave, int tails, int per) {
 // Nor from two layers to one where it is the wave on its own that takes the time: D = 64 660 x 45 15.6, 13.8, 15.4; 1031 x 30
 // 20.4, 20.6, 21.7; 1300 x 24 23.8, 24.9, 25.9; and with four to a block 900 x 34 18.7, 21.7, 19.5.  D = 128 1031 x 30 31.8, 29.1,
 // 31.7; 900 x 34 28.8, 32.8, 28.8.
-FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus) {
+// Under causal masking these rows have more keys than any others, and go first anyhow.  Up to 160 rows, where that makes two
+// kinds of block alike, by the layers too (D = 64 129 x 300 40, 129 x 400 13 and 57 % faster; D = 128 150 x 300 29 and 15, 150 x 256
+// (2, 2, 2) 7 and 11 slower).  Longer ones: a launch must last longer than a wave for itself takes, and the fewer blocks of a
+// slice the more there is to gain; with a block for each and four to a block: D = 64 257 x 230 14.0, 12.3; 400 x 200 17.8, 15.8;
+// 520 x 180 1 % better, 520 x 512 5 %, 520 x 100 11 % worse; D = 128 257 x 219 19.5, 16.0; 288 x 376 29.8, 26.8; 385 x 216 27.1, 24.9; 410
+// x 181 22.3, 22.3; 530 x 170 29.4, 28.1; 520 x 100 17 % worse.  Past 576 rows 1 to 2 % in the mean, with losses among them; and
+// hardly anything, or less, where the blocks are just past full layers: D = 128 410 x 264 (5) 31.8, 33.2;
+// 257 x 257 (4) 21.2, 21.9; D = 64 410 x 257 (5) 20.3, 20.6.
+FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus, bool causal) {
   if (n <= 128 || (n - 1) % 128 >= 32) return 0;
   const long full = (long)slices * ((n - 1) / 128);
   const long now = (full + slices + cus - 1) / cus, two = (full + fmha_tail_blocks(slices, 2) + cus - 1) / cus,
              four = (full + fmha_tail_blocks(slices, 4) + cus - 1) / cus;
+  if (causal && n > 160) {
+    const long blocks = full + slices, left = blocks % cus;
+    return n <= 576 && 480 * blocks >= (900L + n) * cus && 16 * left >= (d == 64 ? 1 : 5) * cus ? 4 : 0;
+  }
   if (n > 768 && ((d == 128 && now > 6) || (now == 2 && (d == 64 || two == 2)))) return 0;
   return two < now && two <= four ? 2 : four < now ? 4 : 0;
 }

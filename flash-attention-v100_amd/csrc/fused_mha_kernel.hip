@@ -1041,7 +1041,7 @@ __device__ __forceinline__ void odd_slots_first() {
 // is that the block ends before the others of its round, so its waves go first wherever they could issue (a tail that is
 // still there when the others have ended: 4100 x 20 slices, D = 128, 186 us without, 170 with).  Two tiles of LDS to a wave, so that
 // copies are under way longer: nothing gained.  All sums are those of the kernel below, in the same order.
-template <int D>
+template <int D, bool CAUSAL>
 __device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, const half_t* __restrict__ K,
                                               const half_t* __restrict__ V, Strides qs, Strides ks, Strides vs,
                                               half_t* __restrict__ O, float* __restrict__ LSE, int H, int N, int bh, float c,
@@ -1141,7 +1141,7 @@ __device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, cons
     copy(Vb, vs.n, t);
     __builtin_amdgcn_sched_barrier(0);
     if (t == nt - 1) {  // the only tile with keys that do not count
-      const int last = N - 1 - t * kTile - 4 * hh;
+      const int last = (CAUSAL ? min(q0 + i, N - 1) : N - 1) - t * kTile - 4 * hh;
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -1219,19 +1219,21 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     return t & 63;
   };
   int bh, mb;
+  const int lin = CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x;
+  const int nb = nmb - (TAIL ? 1 : 0);
   if constexpr (TAIL) {
     const int tails = fmha_tail_blocks(slices, tails_per_block);
-    if ((int)blockIdx.x < tails) {
-      bh = fmha_tail_slice(blockIdx.x, wave, tails, tails_per_block);
-      if (wave < tails_per_block && bh < slices) fwd_tail_rows<D>(Q, K, V, qs, ks, vs, O, LSE, H, N, bh, c, negate_q, smem + wave * T::kBytes);
+    if (lin < tails) {
+      bh = fmha_tail_slice(lin, wave, tails, tails_per_block);
+      if (wave < tails_per_block && bh < slices)
+        fwd_tail_rows<D, CAUSAL>(Q, K, V, qs, ks, vs, O, LSE, H, N, bh, c, negate_q, smem + wave * T::kBytes);
       return;
     }
-    fmha_slice_and_block(blockIdx.x - tails, slices, nmb - 1, bh, mb);
+    fmha_scheduled_block(lin - tails, slices, nb, CAUSAL, false, bh, mb);
   } else {
-    fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
-                         N % kPipeBlockQ != 0, bh, mb);
+    fmha_scheduled_block(lin, slices, nb, CAUSAL, N % kPipeBlockQ != 0, bh, mb);
   }
-  const int mblk = CAUSAL ? nmb - 1 - mb : mb;  // heavy blocks first
+  const int mblk = CAUSAL ? nb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O is dense
   const long head_off = ((long)b * N * H + h) * D;
@@ -3936,15 +3938,15 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
   int tails_per_block = 0;
   auto kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, false>;
   unsigned blocks = total;
+  static_assert(kPipeBlockQ == 128 && kResident == 32, "as fmha_tails_per_block has it");
+  tails_per_block = fmha_tails_per_block(D, n, slices, (int)persistent_grid(1 << 30), CAUSAL);
+  if (tails_per_block) {
+    blocks = fmha_tail_blocks(slices, tails_per_block) + slices * (nmb - 1);
+    kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, true>;
+  }
   if constexpr (!CAUSAL) {
-    static_assert(kPipeBlockQ == 128 && kResident == 32, "as fmha_tails_per_block has it");
-    tails_per_block = fmha_tails_per_block(D, n, slices, (int)persistent_grid(1 << 30));
-    if (tails_per_block) blocks = fmha_tail_blocks(slices, tails_per_block) + slices * (nmb - 1);
-    const bool odd_first = half_round_left(blocks, n, 2);
-    if (tails_per_block)
-      kernel = odd_first ? fmha_fwd_pipe_kernel<D, CAUSAL, true, true> : fmha_fwd_pipe_kernel<D, CAUSAL, false, true>;
-    else if (odd_first)
-      kernel = fmha_fwd_pipe_kernel<D, CAUSAL, true, false>;
+    if (half_round_left(blocks, n, 2))
+      kernel = tails_per_block ? fmha_fwd_pipe_kernel<D, CAUSAL, true, true> : fmha_fwd_pipe_kernel<D, CAUSAL, true, false>;
   }
   const hipError_t rc = launch(kernel, blocks, kPipeThreads, stream, (const half_t*)q,
                                (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, slices,

@@ -234,18 +234,22 @@ def test_rows_that_are_not_finite(B, H, N, D, causal):
     assert (dq[:, good, h].float().cpu() - ref_dq[:, good, 0].half().float()).abs().max() <= 1e-2
 
 
-TAILS = [  # D, slices, N, how many slices' last rows go to one block
-    (64, 300, 129, 2), (64, 401, 150, 4), (64, 100, 257, 2), (64, 110, 520, 2), (64, 118, 544, 4), (64, 59, 1031, 2),
-    (64, 61, 1537, 2), (128, 300, 160, 2), (128, 181, 130, 4), (128, 203, 257, 2), (128, 150, 400, 4), (128, 57, 1056, 2),
-    (128, 122, 1025, 4), (64, 62, 1550, 4),
+TAILS = [  # D, slices, N, causal, how many slices' last rows go to one block
+    (64, 300, 129, 0, 2), (64, 401, 150, 0, 4), (64, 100, 257, 0, 2), (64, 110, 520, 0, 2), (64, 118, 544, 0, 4),
+    (64, 59, 1031, 0, 2), (64, 61, 1537, 0, 2), (64, 62, 1550, 0, 4), (128, 300, 160, 0, 2), (128, 181, 130, 0, 4),
+    (128, 203, 257, 0, 2), (128, 150, 400, 0, 4), (128, 57, 1056, 0, 2), (128, 122, 1025, 0, 4),
+    (64, 300, 129, 1, 2), (64, 401, 160, 1, 4), (64, 231, 288, 1, 4), (64, 199, 416, 1, 4), (64, 173, 513, 1, 4),
+    (128, 150, 130, 1, 2), (128, 399, 150, 1, 4), (128, 230, 257, 1, 4), (128, 215, 385, 1, 4), (128, 170, 544, 1, 4),
 ]
 
 
 def test_blocks_with_the_last_rows_of_slices(tmp_path):
     """The cases below on 256 compute units and others left alone; every slice's last rows once, on few XCDs."""
-    rule = "fmha_tails_per_block(x[0], x[2], x[1], 256) == x[3]"
-    alone = [(64, 300, 128, 0), (64, 300, 161, 0), (64, 230, 129, 0), (64, 256, 257, 0), (64, 30, 1031, 0), (64, 34, 900, 0),
-             (128, 56, 1031, 0), (128, 200, 1031, 0), (128, 34, 900, 0), (128, 1, 129, 0), (64, 1, 1, 0), (128, 230, 2070, 0)]
+    rule = "fmha_tails_per_block(x[0], x[2], x[1], 256, x[3]) == x[4]"
+    alone = [(64, 300, 128), (64, 300, 161), (64, 230, 129), (64, 256, 257), (64, 30, 1031), (64, 34, 900), (128, 56, 1031),
+             (128, 200, 1031), (128, 34, 900), (128, 1, 129), (64, 1, 1), (128, 230, 2070)]
+    causal = [(64, 256, 150), (128, 256, 129), (64, 100, 520), (64, 257, 410), (128, 264, 410), (128, 100, 520), (128, 200, 1031)]
+    alone = [(*case, 0, 0) for case in alone] + [(*case, 1, 0) for case in causal]
     assert all(abi.host_rule(tmp_path, rule, TAILS + alone))
     src, exe = tmp_path / "tails.cpp", tmp_path / "tails"
     src.write_text(r'''
@@ -268,8 +272,8 @@ int main() {
     }
   for (int d = 64; d <= 128; d += 64)
     for (int n = 1; n <= 1200; ++n)
-      for (int slices = 1; slices <= 700; slices += 3) {
-        const int per = fmha_tails_per_block(d, n, slices, 256);
+      for (int slices = 1; slices <= 700; slices += 5) {
+        const int per = fmha_tails_per_block(d, n, slices, 256, slices & 1);
         if (per && per != 2 && per != 4) return 1;
         if (per && fmha_tail_blocks(slices, per) >= slices) { printf("gain %d %d\n", n, slices); return 1; }
       }
@@ -282,9 +286,9 @@ int main() {
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("D,H,N,per", TAILS)
-def test_last_rows_of_several_slices_in_one_block(D, H, N, per):
-    """The bits of launches of a few slices, in which each has a block for its last rows, without a mask; with maxima that are
+@pytest.mark.parametrize("D,H,N,causal,per", TAILS)
+def test_last_rows_of_several_slices_in_one_block(D, H, N, causal, per):
+    """The bits of launches of a few slices, in which each has a block for its last rows; with maxima that are
     raised at nearly every tile, with strides and a negative scale, with rows that are not finite."""
     lib = abi.load()
     last = (N - 1) // 128 * 128
@@ -295,18 +299,18 @@ def test_last_rows_of_several_slices_in_one_block(D, H, N, per):
             q[:, last, 1, 3], q[:, N - 1, H // 2, 5], k[:, N - 1, H - 1, 0] = float("nan"), float("inf"), float("inf")
         if kind == "strided":
             q, k, v = torch.stack((q, k, v), dim=2).unbind(2)
-            out, lse = abi.forward_strided(lib, q, k, v, scale, False)
+            out, lse = abi.forward_strided(lib, q, k, v, scale, causal)
         else:
-            out, lse = abi.forward(lib, q, k, v, scale, False)
+            out, lse = abi.forward(lib, q, k, v, scale, causal)
         for h in range(0, H, 13):
             few = [t[:, :, h:h + 13].contiguous() for t in (q, k, v)]
-            o, l = abi.forward(lib, *few, scale, False)
+            o, l = abi.forward(lib, *few, scale, causal)
             assert torch.equal(o.view(torch.int16), out[:, :, h:h + 13].contiguous().view(torch.int16)) or (
                 kind == "not finite" and torch.equal(o.isnan(), out[:, :, h:h + 13].isnan()) and
                 torch.equal(o.nan_to_num(), out[:, :, h:h + 13].nan_to_num()))
             assert torch.equal(l.nan_to_num(), lse[:, h:h + 13].nan_to_num())
             if h == 0 and kind in ("plain", "growing"):
-                ref, ref_lse = ao.attention_forward(*(t[:, :, :2].cpu() for t in few), scale, False)
+                ref, ref_lse = ao.attention_forward(*(t[:, :, :2].cpu() for t in few), scale, bool(causal))
                 # the bounds of _check
                 assert (o[:, :, :2].float().cpu() - ref.half().float()).abs().max() <= 2e-3 * max(1.0, ref.abs().max().item())
                 assert ((l[:, :2].cpu() - ref_lse).abs() <= 2e-3 + 1e-6 * ref_lse.abs()).all()
