@@ -3924,9 +3924,12 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
   // tiny positive factor gives the same uniform softmax and keeps -inf * c = -inf.
   const float c = fmaxf(fabsf(scale) * kLog2e, 1e-30f);
   const int negate = scale < 0.f ? 1 : 0;
+  const bool short_tail = n > kPipeBlockQ && (n - 1) % kPipeBlockQ < kResident;
+  // the number of CUs is a question to the runtime, which small calls feel: not asked where no rule needs it
+  const int cus = D == 128 || short_tail ? (int)persistent_grid(1 << 30) : 0;
   if constexpr (D == 128) {
     const int nmb = (n + kFwdBlockQ - 1) / kFwdBlockQ, total = nmb * batch * head;
-    if (fmha_persistent_forward_pays(batch * head, n, (int)persistent_grid(1 << 30), CAUSAL)) {
+    if (fmha_persistent_forward_pays(batch * head, n, cus, CAUSAL)) {
       const hipError_t rc = launch(fmha_fwd_kernel<D, CAUSAL>, persistent_grid(total), kFwdThreads, stream,
                                    (const half_t*)q, (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o,
                                    (float*)lse, head, n, nmb, total, c, negate);
@@ -3939,7 +3942,7 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
   auto kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, false>;
   unsigned blocks = total;
   static_assert(kPipeBlockQ == 128 && kResident == 32, "as fmha_tails_per_block has it");
-  tails_per_block = fmha_tails_per_block(D, n, slices, (int)persistent_grid(1 << 30), CAUSAL);
+  if (short_tail) tails_per_block = fmha_tails_per_block(D, n, slices, cus, CAUSAL);
   if (tails_per_block) {
     blocks = fmha_tail_blocks(slices, tails_per_block) + slices * (nmb - 1);
     kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, true>;
