@@ -204,6 +204,7 @@ NOT_FINITE_PERSISTENT = [(5, 17, 700, 128, False), (1, 32, 4096, 128, True), (1,
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,N,D,causal", NOT_FINITE_PERSISTENT + [
     (1, 3, 449, 64, False), (1, 3, 449, 64, True), (1, 3, 449, 128, False), (1, 3, 449, 128, True), (1, 64, 2048, 128, True),
+    (1, 200, 449, 64, False), (1, 256, 449, 64, True), (1, 130, 150, 128, False), (1, 130, 200, 128, True),  # a work group per slice
 ])
 def test_rows_that_are_not_finite(B, H, N, D, causal):
     """Queries with a NaN or an infinity give NaN rows and make their wave raise its maximum at every tile; the finite rows
