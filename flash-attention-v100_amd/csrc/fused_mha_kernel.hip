@@ -241,34 +241,27 @@ __device__ __forceinline__ void copy16(const half_t* tile_base, int voff, char* 
       : "v"(voff), "s"(tile_base), "s"(lds_addr)
       : "memory");
 }
-// The same for dS, which other work groups of the launch may have written (sc1: not out of this XCD's L2, see
-// store16_stream), with the hint that it is read once, which keeps it from displacing the tiles other work groups re-read
-// out of the L2, and without.
-__device__ __forceinline__ void copy16_stream(const half_t* tile_base, int voff, char* lds_block) {
+// The same for dS.  STREAM: with the hint that it is read once, which keeps it from displacing the tiles other work groups
+// re-read out of the L2.  SHARED: other work groups of the launch have written it (sc1: not out of this XCD's L2, see store_ds).
+template <bool SHARED, bool STREAM>
+__device__ __forceinline__ void copy16_ds(const half_t* tile_base, int voff, char* lds_block) {
   const unsigned lds_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds_block;
   unsigned saved_m0;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2 sc1 nt\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved_m0)
-      : "v"(voff), "s"(tile_base), "s"(lds_addr)
-      : "memory");
-}
-__device__ __forceinline__ void copy16_shared(const half_t* tile_base, int voff, char* lds_block) {
-  const unsigned lds_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds_block;
-  unsigned saved_m0;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2 sc1\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved_m0)
-      : "v"(voff), "s"(tile_base), "s"(lds_addr)
-      : "memory");
+#define FMHA_COPY16(HINTS)                            \
+  asm volatile(                                       \
+      "s_mov_b32 %0, m0\n\t"                          \
+      "s_mov_b32 m0, %3\n\t"                          \
+      "s_nop 0\n\t"                                   \
+      "global_load_lds_dwordx4 %1, %2" HINTS "\n\t"   \
+      "s_mov_b32 m0, %0"                              \
+      : "=&s"(saved_m0)                               \
+      : "v"(voff), "s"(tile_base), "s"(lds_addr)      \
+      : "memory")
+  if constexpr (SHARED && STREAM) FMHA_COPY16(" sc1 nt");
+  else if constexpr (SHARED) FMHA_COPY16(" sc1");
+  else if constexpr (STREAM) FMHA_COPY16(" nt");
+  else FMHA_COPY16("");
+#undef FMHA_COPY16
 }
 
 // kCount copies of 1 KiB to consecutive blocks of LDS: lane l's 16 bytes of block u land at lds + 1024 * u + 16 * l.
@@ -528,19 +521,17 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_each(std::make_integer_sequence<int, kN>{}, f);
 }
 
-// 16 bytes per lane to p + kOffset bytes, with the non-temporal hint (data that is read once, by other work groups of this
-// launch or of a later one).  sc1: past the XCD's L2, so that work groups of any XCD see it once the store is done; with
-// the hint that costs nothing (64 x 4096 x 128 causal, both passes: 795.9 us without, 796.6 with).  Inline asm because
-// the compiler keeps the hint only on the first of several stores that share
-// a base address; like the tile copies it is therefore invisible to the compiler's wait counts.
-template <int kOffset>
-__device__ __forceinline__ void store16_stream(half_t* p, h8 v, IntTag<kOffset>) {
-  asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
-}
-// The same without the hint.
-template <int kOffset>
-__device__ __forceinline__ void store16_keep(half_t* p, h8 v, IntTag<kOffset>) {
-  asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+// 16 bytes of dS per lane to p + kOffset bytes.  KEEP: without the non-temporal hint (data that is read once, by other work
+// groups of this launch or of a later one).  SHARED: work groups of this launch read it, so it goes past the XCD's L2 (sc1) and
+// those of any XCD see it once the store is done.  Not where a later launch reads it, which finds it in the caches otherwise (forward
+// and backward, 80 x 2048 x 128 causal: 397 us without sc1 on either side, 429 with).  Inline asm because the compiler keeps the hint only on the first of several
+// stores that share a base address; like the tile copies it is therefore invisible to the compiler's wait counts.
+template <bool SHARED, bool KEEP, int kOffset>
+__device__ __forceinline__ void store_ds(half_t* p, h8 v, IntTag<kOffset>) {
+  if constexpr (SHARED && !KEEP) asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+  else if constexpr (SHARED) asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+  else if constexpr (!KEEP) asm volatile("global_store_dwordx4 %0, %1, off offset:%2 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+  else asm volatile("global_store_dwordx4 %0, %1, off offset:%2" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
 }
 
 // Element strides of a (batch, n, head, d) tensor whose last dimension is
@@ -2174,11 +2165,12 @@ constexpr int kKvBlockKeys = kKvPairs * kResident;
 // KEEP: without the non-temporal hint on those stores (rule: fmha_ds_used_once).
 // WIDE: 32 x 32 x 16 MFMAs instead of 16 x 16 x 32 ones (same bits; rule and both times: fmha_wide_mfmas).
 // STATS: the row statistics of every tile are formed here, from O, dO and LSE, a tile ahead; delta and lse2 are not read.
-// stored: counts the waves that have stored all of their dS, kKvPairs of every block (fmha_bwd_both_spill_kernel).
+// SHARED: work groups of this launch read dS; stored counts the waves that have stored all of theirs, kKvPairs of every block
+// (fmha_bwd_both_spill_kernel).
 constexpr int kKvStBytes = 1024;
 template <int D>
 constexpr int dkdv_lds() { return 7 * SwzTile<D>::kBytes + 3 * kKvStBytes + 2 * kKvPairs * 2 * 2048; }
-template <int D, bool CAUSAL, bool SPILL, bool KEEP, bool WIDE, bool STATS>
+template <int D, bool CAUSAL, bool SPILL, bool KEEP, bool WIDE, bool STATS, bool SHARED = false>
 __device__ __forceinline__ void
 bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
@@ -2528,14 +2520,12 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
           half_t* dst = ds_lane + (long)(t >> 1) * np * 128 + (t & 1) * 2048 + half * 1024;
           static_for<kFrags>([&](auto f_tag) __attribute__((always_inline)) {
             constexpr int f = decltype(f_tag)::value, at = f * 1024;
-            if constexpr (!KEEP) store16_stream(dst, y[f], IntTag<at>{});
-            else store16_keep(dst, y[f], IntTag<at>{});
+            store_ds<SHARED, KEEP>(dst, y[f], IntTag<at>{});
           });
           if (HALF) {  // the zeros that the other 32 keys of the last 64-key tile owe
             static_for<kFrags>([&](auto f_tag) __attribute__((always_inline)) {
               constexpr int at = decltype(f_tag)::value * 1024;
-              if constexpr (!KEEP) store16_stream(dst + 4096, h8{}, IntTag<at>{});
-              else store16_keep(dst + 4096, h8{}, IntTag<at>{});
+              store_ds<SHARED, KEEP>(dst + 4096, h8{}, IntTag<at>{});
             });
           }
         }
@@ -2565,7 +2555,7 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   static_assert(kKvWaves * Stage16<D>::kBytes <= 7 * T::kBytes && kKvWaves * StageGeom<D>::kBytes <= 7 * T::kBytes,
                 "the output staging tiles fit the rings");
   block_barrier();  // every wave is done with the rings: they become the staging tiles
-  if (SPILL && stored && role_b) {  // this wave's dS is where every work group of the launch can read it
+  if (SHARED && role_b) {  // this wave's dS is where every work group of the launch can read it
     wait_vm<0>();
     if (lane == 0) __hip_atomic_fetch_add(stored, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -2983,6 +2973,7 @@ __device__ __forceinline__ const half_t* wave_uniform(const half_t* p) {
 // persistent schedule does.
 template <bool CAUSAL>
 struct DsBlocks {
+  static constexpr bool kShared = false;  // a launch before this one has stored dS
   int total, nqb;
   __device__ __forceinline__ int next_round(int r) const { return PersistentBlocks{total}.next_round(r); }
   __device__ __forceinline__ void locate(int round, int& bh, int& mb) const {
@@ -2993,6 +2984,7 @@ struct DsBlocks {
 };
 // One block that is known already.
 struct DsBlock {
+  static constexpr bool kShared = true;
   int bh, mb;
   __device__ __forceinline__ int next_round(int) const { return -1; }
   __device__ __forceinline__ void locate(int, int& bh_, int& mb_) const { bh_ = bh, mb_ = mb; }
@@ -3101,10 +3093,10 @@ bwd_dq_spill_blocks(const half_t* __restrict__ K, Strides ks, const half_t* __re
     char* dst = s_ring + slot * kDsTileBytes + cw * kSIPW * 1024;
     if (stream_ds) {
 #pragma unroll
-      for (int u = 0; u < kSIPW; ++u) copy16_stream(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+      for (int u = 0; u < kSIPW; ++u) copy16_ds<Blocks::kShared, true>(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
     } else {
 #pragma unroll
-      for (int u = 0; u < kSIPW; ++u) copy16_shared(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+      for (int u = 0; u < kSIPW; ++u) copy16_ds<Blocks::kShared, false>(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
     }
   };
   auto copy_k = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
@@ -3285,7 +3277,7 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
 // that gives, and where the passes still go one by one: fmha_ds_in_one_launch.
 //
 // A dQ block waits for the dS of its slice: every wave that stores some counts itself when its stores are done, and the
-// block starts when the count is whole.  dS is stored and read past the XCDs' L2s (store16_stream), so that is all it takes,
+// block starts when the count is whole.  dS is stored and read past the XCDs' L2s (store_ds), so that is all it takes,
 // on whatever XCD the blocks are; a release of everything written (an L2 write-back per block) takes 8 % longer.  Each count
 // has a cache line of its own and is asked for about once a microsecond: with the counts of 32 slices in one line the work
 // groups that ask hold up those that work (24 x 2048 x 128 causal, 111 us; a line each 89).
@@ -3310,7 +3302,7 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
   bool dq;
   if (!fmha_ds_launch_block(blockIdx.x, slices, nb, CAUSAL, bh, blk, dq)) return;
   if (!dq) {
-    bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
+    bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false, true>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
                                                         H, N, 0, c, scale, smem, bh, blk, ready + (long)bh * kReadyStride);
     return;
   }
