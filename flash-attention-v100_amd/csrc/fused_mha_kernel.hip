@@ -523,8 +523,8 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // 16 bytes of dS per lane to p + kOffset bytes.  KEEP: without the non-temporal hint (data that is read once, by other work
 // groups of this launch or of a later one).  SHARED: work groups of this launch read it, so it goes past the XCD's L2 (sc1) and
-// those of any XCD see it once the store is done.  Not where a later launch reads it, which finds it in the caches otherwise (forward
-// and backward, 80 x 2048 x 128 causal: 397 us without sc1 on either side, 429 with).  Inline asm because the compiler keeps the hint only on the first of several
+// those of any XCD see it once the store is done.  Not where a later launch reads it (forward and backward, 80 x 2048 x 128
+// causal: 397 us, with sc1 on either side 429).  Inline asm because the compiler keeps the hint only on the first of several
 // stores that share a base address; like the tile copies it is therefore invisible to the compiler's wait counts.
 template <bool SHARED, bool KEEP, int kOffset>
 __device__ __forceinline__ void store_ds(half_t* p, h8 v, IntTag<kOffset>) {
