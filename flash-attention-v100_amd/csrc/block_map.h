@@ -284,6 +284,9 @@ FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool hea
 // 190, 176; 1024 x 220 (6.9) 276, 264; 1280 x 100 (3.9) 176, 170; 1500 x 48 (2.3) 118, 108; 1500 x 80 (3.8) 189, 181; 2048 x 20 85.3,
 // 81.0; 2048 x 56 (3.5) 213, 208; 2048 x 64 (4) 232, 237; 2048 x 80 (5) 296, 299; 4096 x 9 (1.1) 149, 140; 4096 x 11 (1.4) 159,
 // 153; 4096 x 12 (1.5) 169, 171; 4096 x 16 (2) 207, 210; 8192 x 6 323, 324; 8192 x 12 (3) 586, 594; 16384 x 16 (8) 2820, 2919.
+// Past six rounds the figures above leave out what the one launch pays for dS past the L2s when others follow; forward and backward
+// as calls, no mask: 1500 x 110 (5.2) 589, 572; 1500 x 155 (7.3) 814, 800; 2048 x 84 (5.3) 757, 741; 2048 x 100 (6.3) 912, 915; 2048
+// x 114 (7.1) 1017, 1020; 2048 x 130 (8.1) 1178, 1191; 4096 x 42 (5.3) 1390, 1373.
 FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool causal) {
   const long blocks = (long)slices * ((n + 127) / 128), left = blocks % cus;
   if (n <= 768) return 2 * blocks <= 15L * cus;
@@ -291,7 +294,7 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
   if (blocks <= cus) return n <= 2048;
   if (left == 0) return false;
   if (n <= 1024) return 4 * left <= 3L * cus && blocks <= 9L * cus;
-  if (n <= 4096) return 2 * left <= cus && blocks <= (n <= 2048 ? 9L : 6L) * cus;
+  if (n <= 4096) return 2 * left <= cus && blocks <= (n <= 1536 ? 8L : 6L) * cus;
   return n <= 8192 && 4 * left <= cus && blocks > 2L * cus && blocks < 5L * cus;
 }
 
