@@ -262,6 +262,13 @@ FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool hea
   return true;
 }
 
+// How long a dQ block of that launch waits for the dS of its slice before it forms S and dP itself, in ticks of 10 ns.  Blocks
+// are handed out in order inside an XCD only, and a slice that no XCD has for itself (slices % 8) has blocks on several.  With
+// launches on more than one stream, dQ blocks of one that wait can so hold all CUs that dK/dV blocks of another need, and the
+// other way round.  So a block waits long only for dK/dV blocks that have all started: these wait for nobody and take 16 ns a
+// row of the slice.  For others it waits about as long as it takes to do without them.
+FMHA_HOST_DEVICE unsigned fmha_ds_wait_ticks(int n, bool started) { return (500u + 2u * (unsigned)n) * (started ? 32u : 1u); }
+
 // Whether such a launch takes the place of the two passes one after the other.  It gains where the last round of one of them is
 // far from full, and with few rounds, and a launch where these are short; it loses where a dQ block of 128 queries is much
 // slower than the one of 256 that the dQ pass alone takes then (half of the copies of K), which long sequences feel.  us of the

@@ -24,8 +24,10 @@ size_t fmha_backward_workspace_for(int batch, int head, int n, int d, int causal
 // it does not.
 size_t fmha_backward_count_bytes(int batch, int head, int n, int d, int causal);
 
-// fused_mha_backward by its passes also where that takes a work group for each slice, and with a limit, in ticks of 10 ns, to how
-// long a block of a launch of both passes over dS waits for another's dS before it forms S and dP itself.
+// fused_mha_backward by its passes also where that takes a work group for each slice, and with a limit of the caller's, in ticks
+// of 10 ns, to how long a block of a launch of both passes over dS waits for another's dS before it forms S and dP itself.  The
+// counts behind the dS are, per slice, the waves that have stored dS, the dK/dV blocks that have started (of the last slices % 8
+// only) and the dQ blocks that have done without, then 29 zeros.
 int fmha_backward_waiting(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,
                           const void* d_output_ptr, const void* lse_ptr, void* workspace, size_t workspace_bytes,
                           void* d_query_ptr, void* d_key_ptr, void* d_value_ptr, int batch, int head, int n, int d, float scale,

@@ -3278,14 +3278,19 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
 //
 // A dQ block waits for the dS of its slice: every wave that stores some counts itself when its stores are done, and the
 // block starts when the count is whole.  dS is stored and read past the XCDs' L2s (store_ds), so that is all it takes,
-// on whatever XCD the blocks are; a release of everything written (an L2 write-back per block) takes 8 % longer.  Each count
-// has a cache line of its own and is asked for about once a microsecond: with the counts of 32 slices in one line the work
-// groups that ask hold up those that work (24 x 2048 x 128 causal, 111 us; a line each 89).
-// The wait ends by itself: dK/dV blocks wait for nobody and come first, and should they not be done within kReadyTicks,
-// whatever the reason, the block forms S and dP itself, as fmha_bwd_dq_kernel does, with the same bits as result.
+// on whatever XCD the blocks are; a release of everything written (an L2 write-back per block) takes 8 % longer.  The counts
+// of a slice have a cache line of their own and are asked for about once a microsecond: with those of 32 slices in one line
+// the work groups that ask hold up those that work (24 x 2048 x 128 causal, 111 us; a line each 89).
+// The wait ends by itself: past fmha_ds_wait_ticks, which is longer once all dK/dV blocks of the slice have started, the
+// block forms S and dP itself, as fmha_bwd_dq_kernel does, with the same bits as result.  Counting what has started costs up
+// to 0.8 us of a launch (520 x 64), so only the slices that need it do.
 // ---------------------------------------------------------------------------
-constexpr unsigned kReadyTicks = 5000000;  // of the 100 MHz clock: 50 ms
-constexpr int kReadyStride = 32;           // words from one slice's count to the next
+constexpr int kReadyStride = 32;  // words from one slice's counts to the next
+enum ReadyWord {
+  kWavesStored,
+  kBlocksStarted,  // of the dK/dV pass, where they are not all on one XCD
+  kBlocksAlone     // of the dQ pass, that have not waited to the end
+};
 template <bool CAUSAL, bool KEEP>
 __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
@@ -3301,20 +3306,27 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
   int bh, blk;
   bool dq;
   if (!fmha_ds_launch_block(blockIdx.x, slices, nb, CAUSAL, bh, blk, dq)) return;
+  unsigned* const counts = ready + (long)bh * kReadyStride;
+  auto count = [&](int word) { __hip_atomic_fetch_add(counts + word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  const bool one_xcd = bh < (slices & ~7);  // all blocks of the slice: the dK/dV blocks have then started before this dQ block
   if (!dq) {
+    if (!one_xcd && threadIdx.x == 0) count(kBlocksStarted);
     bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false, true>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
-                                                        H, N, 0, c, scale, smem, bh, blk, ready + (long)bh * kReadyStride);
+                                                        H, N, 0, c, scale, smem, bh, blk, counts + kWavesStored);
     return;
   }
   if (threadIdx.x == 0) {
     const unsigned long long start = wall_clock64();
+    auto read = [&](int word) { return __hip_atomic_load(counts + word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     int whole;
     for (;;) {
-      whole = __hip_atomic_load(ready + (long)bh * kReadyStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-              (unsigned)(kKvPairs * nb);
-      if (whole || wall_clock64() - start >= ticks) break;
+      whole = read(kWavesStored) == (unsigned)(kKvPairs * nb);
+      if (whole) break;
+      const unsigned long long most = fmha_ds_wait_ticks(N, one_xcd || read(kBlocksStarted) == (unsigned)nb);
+      if (wall_clock64() - start >= (most < ticks ? most : ticks)) break;
       __builtin_amdgcn_s_sleep(32);  // 2048 cycles
     }
+    if (!whole) count(kBlocksAlone);
     *reinterpret_cast<volatile int*>(smem) = whole;
   }
   block_barrier();
@@ -4021,8 +4033,8 @@ template <int D, bool CAUSAL>
 int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsigned ticks, const void* q, const void* k, const void* v, const void* o,
                     const void* d_o, Strides qs, Strides ks, Strides vs, Strides gs, const void* lse, float* delta,
                     void* dq, void* dk, void* dv, int batch, int head, int n, float scale, hipStream_t stream) {
-  // slices_at_once: how many slices' dS the workspace holds, 0 for the passes that need none; ticks: how long a block may wait
-  // for another's dS
+  // slices_at_once: how many slices' dS the workspace holds, 0 for the passes that need none; ticks: the most that a block may
+  // wait for another's dS, fmha_ds_wait_ticks if that is less
   if (D == 64) slices_at_once = 0;  // see fmha_bwd_dq_pipe_kernel
   // Rounds of so few slices that they leave CUs idle cost more than the GEMMs they save.
   const int cus = (int)persistent_grid(1 << 30);
@@ -4188,7 +4200,7 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
                       const fused_mha_strides* k_st, const void* v, const fused_mha_strides* v_st, const void* o,
                       const void* d_o, const fused_mha_strides* g_st, const void* lse, void* workspace,
                       size_t workspace_bytes, void* dq, void* dk, void* dv, int batch, int head, int m, int n, int d,
-                      float scale, int causal, void* stream, unsigned ticks = kReadyTicks) {
+                      float scale, int causal, void* stream, unsigned ticks = ~0u) {
   const bool need_o = passes & kPassDelta, need_dq = passes & kPassDq, need_dkdv = passes & kPassDkDv;
   if (!d_o || !workspace || !lse || (need_o && !o) || ((need_dq || need_dkdv) && (!q || !k || !v)) ||
       (need_dq && !dq) || (need_dkdv && (!dk || !dv)))

@@ -199,6 +199,44 @@ def test_both_passes_over_ds_in_one_launch(H, N, causal, ticks):
             assert torch.equal(a, b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,N,causal", [(60, 1031, False), (33, 1023, True), (15, 4609, False), (22, 5889, False)])
+def test_launches_over_ds_on_two_streams(H, N, causal):
+    """Launches of both passes over dS at once, with slices whose blocks are on several XCDs: the bits of one alone, and no wait
+    for blocks that cannot start (of the two longest, waiting blocks of either can hold all of an XCD)."""
+    D, lib = 128, abi.load()
+    nbytes = lib.fused_mha_backward_workspace_bytes(1, H, N, D) + 128 * H
+    calls = []
+    for seed in range(2):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        q, k, v, do = (torch.randn(1, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+        out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+        want = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal)[:3]
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        calls.append(((q, k, v, out, do, lse), ws, [torch.empty_like(q) for _ in range(3)], want, torch.cuda.Stream()))
+    for _ in range(5):
+        for _, ws, got, _, _ in calls:
+            for t in (ws.view(torch.int16), *got):
+                t.fill_(-1)
+        torch.cuda.synchronize()
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for inputs, ws, got, _, stream in calls:
+            stream.wait_event(begin)
+            rc = lib.fused_mha_backward(*(t.data_ptr() for t in inputs), ws.data_ptr(), nbytes, *(g.data_ptr() for g in got),
+                                        1, H, N, N, D, D ** -0.5, int(causal), stream.cuda_stream)
+            assert rc == abi.OK
+        for *_, stream in calls:
+            torch.cuda.current_stream().wait_stream(stream)
+        end.record()
+        torch.cuda.synchronize()
+        for _, ws, got, want, _ in calls:
+            assert (ws[-128 * H:].view(torch.int32).view(H, 32)[:, 0] == 4 * (-(-N // 128))).all()  # the launch with counts
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
+        assert begin.elapsed_time(end) < 20  # ms; about 1.5 each
+
+
 EITHER_MFMA = [1, 15, 16, 17, 32, 49, 64, 79, 128, 129, 200]
 
 

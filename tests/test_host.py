@@ -470,6 +470,91 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_launches_over_ds_at_once_do_not_hold_each_other_up(tmp_path):
+    """csrc/block_map.h: launches of both passes over dS on several streams, on 8 XCDs of 32 compute units that hand out the
+    blocks of a launch in order and prefer different launches.  A dQ block that waits keeps its compute unit, and the dK/dV
+    blocks that it waits for may be behind such blocks of another launch, on another XCD.  The waits leave the whole no
+    more than 1.4 times as long as the launches one after the other, and nobody gives up in a launch alone."""
+    import subprocess
+
+    src = tmp_path / "at_once.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <vector>
+#include "block_map.h"
+struct Block { int slice; bool dq; };
+struct Cu { bool busy = false, waiting = false; int launch; Block block; double since, end; };
+// us until `launches` of them are done; alone: how many dQ blocks have formed S and dP themselves
+double run(int slices, int n, int launches, bool mixed, int& alone) {
+  const int nb = (n + 127) / 128;
+  const double block = 0.016 * n;  // us of a dK/dV block; a dQ block over dS takes half of that, one without it 1.1 times
+  std::vector<Block> queue[8];
+  std::vector<int> home(slices, -1);
+  for (int lin = 0; lin < fmha_ds_launch_blocks(slices, nb); ++lin) {
+    int s, b;
+    bool dq;
+    if (!fmha_ds_launch_block(lin, slices, nb, false, s, b, dq)) continue;
+    queue[lin & 7].push_back({s, dq});
+    if (s < (slices & ~7)) {  // the kernel counts on its dK/dV blocks having started
+      if (home[s] >= 0 && home[s] != (lin & 7)) printf("%d x %d: slice %d on two XCDs\n", n, slices, s);
+      home[s] = lin & 7;
+    }
+  }
+  std::vector<std::vector<size_t>> next(launches, std::vector<size_t>(8));
+  std::vector<std::vector<int>> started(launches, std::vector<int>(slices)), stored = started;
+  Cu cus[8][32];
+  alone = 0;
+  for (double t = 0;; t += block / 16) {
+    bool any = false;
+    for (auto& xcd : cus)
+      for (Cu& c : xcd)
+        if (c.busy && !c.waiting && c.end <= t) {
+          c.busy = false;
+          if (!c.block.dq) ++stored[c.launch][c.block.slice];
+        }
+    for (int x = 0; x < 8; ++x)
+      for (Cu& c : cus[x]) {
+        if (c.busy && c.waiting) {
+          const int s = c.block.slice;
+          const bool whole = stored[c.launch][s] == nb;
+          if (whole || t - c.since >= 0.01 * fmha_ds_wait_ticks(n, started[c.launch][s] == nb)) {
+            c.waiting = false;
+            c.end = t + (whole ? 0.5 : 1.1) * block;
+            alone += !whole;
+          }
+        }
+        for (int k = 0; k < launches && !c.busy; ++k) {
+          const int l = mixed ? (x + k) % launches : k;
+          if (next[l][x] == queue[x].size()) continue;
+          const Block b = queue[x][next[l][x]++];
+          c = {true, b.dq, l, b, t, t + block};
+          if (!b.dq) ++started[l][b.slice];
+        }
+        any |= c.busy;
+      }
+    if (!any) return t;
+  }
+}
+int main() {
+  const int shapes[][2] = {{60, 1031}, {9, 4096}, {15, 4609}, {22, 5889}, {23, 5633}, {18, 8192}};
+  for (auto& shape : shapes) {
+    int alone;
+    run(shape[0], shape[1], 1, false, alone);
+    if (alone) printf("%d x %d alone: %d\n", shape[1], shape[0], alone);
+    for (int launches = 2; launches <= 4; ++launches) {
+      const double apart = launches * run(shape[0], shape[1], 1, false, alone), mixed = run(shape[0], shape[1], launches, true, alone);
+      if (mixed > 1.4 * apart) printf("%d x %d, %d launches: %.0f us, %.0f\n", shape[1], shape[0], launches, apart, mixed);
+    }
+  }
+  puts("ok");
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    exe = tmp_path / "at_once"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
 def test_backward_by_slice(tmp_path, lib):
     """D, N, slices, causal of backwards timed both ways on 256 compute units; and what the extension takes for them."""
     rule = "fmha_backward_by_slice(x[0], x[1], x[2], 256, x[3])"
