@@ -328,6 +328,15 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 // 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512 x 432 93.7,
 // 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512 x 900 217, 198;
 // 512 x 1030 247, 246; 300 x 1030 124, 141.
+// From 257 to 384 rows at D = 64 the line depends on the last tile of 64 rows too, of which the other launches do all even if
+// only half of it has rows (257 to 288 and 321 to 352 rows).  us of forward and backward, without it and with it, N x slices:
+// last tile whole, no mask: 290 x 448 99.7, 95.1; 384 x 448 119.6, 116.1; 290 x 704 144.3, 142.8; 304 x 960 195, 192; 384 x 1216
+// 317, 305; 290 x 1216 242, 245; 290 x 1440 294, 293; 320 x 1440 307, 300; 289 x 1576 329, 331; 304 x 1704 366, 351; but 384 x 385
+// 100, 103; 290 x 598 124, 127; 290 x 833 160, 167; 320 x 1076 218, 225; 290 x 1352 269, 281; 304 x 1544 330, 337.  Causal: 320 x 248
+// 47.6, 45.2; 384 x 248 54.3, 53.2; 384 x 496 102, 100; 320 x 1264 216, 215; 289 x 1520 260, 251; but 320 x 224 43.0, 43.7; 384 x 224
+// 49.7, 51.2; 384 x 752 143, 150; 320 x 1014 160, 168.
+// Last tile half empty, no mask: 264 x 608 121, 116; 264 x 840 155, 153; 352 x 400 105, 102; 352 x 840 201, 201; 352 x 1080 262, 263;
+// 264 x 1336 244, 235; 352 x 1320 332, 321.  Causal: 264 x 232 44.1, 39.0; 352 x 224 48.7, 47.9; 264 x 752 116, 106; 352 x 1008 191, 187.
 FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, bool causal) {
   if (n > 32768 / d) return false;  // LDS and registers hold no more keys
   const long rounds = ((long)slices + cus - 1) / cus, last = slices - (rounds - 1) * cus;
@@ -338,13 +347,15 @@ FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, 
     return rounds > 2 || (causal && n > 160 ? 3 : 4) * last >= cus;
   }
   if (n <= 128) return false;
+  const bool whole_tiles = (n - 1) % 64 >= 32;
   if (!causal) {
     if (rounds == 1) return n <= 256 ? 2 * last > cus : 4 * last >= 3L * cus;
+    if (n > 256 && n <= 384 && whole_tiles) return 8 * last >= (rounds < 6 ? 6L : rounds == 6 ? 5L : 1L) * cus;
     return rounds > 5 || rounds * last > cus;
   }
   if (n <= 160) return rounds == 1 ? 3 * last >= 2L * cus : rounds == 2 && 4 * last >= 3L * cus;
   if (n <= 256) return n <= 200 && rounds == 1 && 8 * last >= 7L * cus;
-  if (n <= 384) return 16 * last >= (rounds == 1 ? 14L : 15L) * cus;
+  if (n <= 384) return whole_tiles ? rounds != 3 && rounds != 4 && 16 * last >= 15L * cus : 16 * last >= (rounds == 1 ? 14L : 15L) * cus;
   return rounds > 4 || 8 * last >= (rounds == 1 ? 7L : 6L) * cus;
 }
 

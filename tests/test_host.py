@@ -561,13 +561,17 @@ def test_backward_by_slice(tmp_path, lib):
     slices = [
         (128, 1, 129, 0), (128, 256, 129, 1), (128, 256, 256, 0), (128, 100, 257, 0), (128, 200, 320, 0), (128, 160, 320, 1),
         (128, 256, 342, 1), (128, 33, 514, 0), (128, 100, 640, 1), (128, 256, 514, 0), (128, 100, 1600, 0), (128, 64, 3000, 1),
-        (64, 129, 129, 0), (64, 257, 192, 0), (64, 512, 192, 0), (64, 300, 400, 0), (64, 512, 600, 0), (64, 512, 1300, 0),
+        (64, 129, 129, 0), (64, 257, 192, 0), (64, 512, 192, 0), (64, 300, 448, 0), (64, 512, 600, 0), (64, 512, 1300, 0),
+        (64, 264, 608, 0), (64, 352, 840, 0), (64, 384, 1216, 0), (64, 290, 1440, 0), (64, 304, 1704, 0), (64, 320, 1264, 1),
+        (64, 264, 1264, 1),
         (64, 129, 171, 1), (64, 160, 448, 1), (64, 200, 224, 1), (64, 384, 256, 1), (64, 512, 224, 1), (64, 512, 448, 1),
         (64, 512, 1030, 1),
     ]
     other = [
         (128, 1, 128, 0), (128, 257, 200, 0), (128, 256, 319, 0), (128, 256, 330, 1), (128, 100, 528, 0), (128, 100, 1030, 1),
         (64, 128, 256, 0), (64, 129, 128, 0), (64, 257, 176, 0), (64, 300, 384, 0), (64, 512, 590, 0), (64, 513, 256, 0),
+        (64, 300, 400, 0), (64, 384, 385, 0), (64, 290, 598, 0), (64, 290, 833, 0), (64, 320, 1076, 0), (64, 290, 1352, 0),
+        (64, 304, 1544, 0), (64, 320, 224, 1), (64, 384, 224, 1), (64, 384, 752, 1), (64, 320, 1014, 1),  # whole tiles of 64 rows
         (64, 129, 160, 1), (64, 201, 256, 1), (64, 200, 480, 1), (64, 300, 480, 1), (64, 512, 208, 1), (64, 512, 640, 1),
         (64, 300, 1030, 1), (64, 512, 96, 0), (128, 1, 1, 0), (64, 1, 1 << 23, 0),
     ]
