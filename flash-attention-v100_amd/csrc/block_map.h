@@ -328,6 +328,9 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 // 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512 x 432 93.7,
 // 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512 x 900 217, 198;
 // 512 x 1030 247, 246; 300 x 1030 124, 141.
+// Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 27.0, 26.4; 161 x 256 27.3, 27.4;
+// 170 x 236 27.4, 26.5; 180 x 224 27.3, 27.2; 180 x 244 27.7, 27.4; 192 x 224 27.0, 27.5; 192 x 236 27.6, 27.1; 192 x 250 27.7, 28.1;
+// 193 x 224 29.3, 30.4; 193 x 250 30.5, 31.0; 200 x 230 29.9, 30.4; 200 x 240 30.3, 30.6; 200 x 256 32.0, 30.7.
 // From 257 to 384 rows at D = 64 the line depends on the last tile of 64 rows too, of which the other launches do all even if
 // only half of it has rows (257 to 288 and 321 to 352 rows).  us of forward and backward, without it and with it, N x slices:
 // last tile whole, no mask: 290 x 448 99.7, 95.1; 384 x 448 119.6, 116.1; 290 x 704 144.3, 142.8; 304 x 960 195, 192; 384 x 1216
@@ -354,7 +357,7 @@ FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, 
     return rounds > 5 || rounds * last > cus;
   }
   if (n <= 160) return rounds == 1 ? 3 * last >= 2L * cus : rounds == 2 && 4 * last >= 3L * cus;
-  if (n <= 256) return n <= 200 && rounds == 1 && 8 * last >= 7L * cus;
+  if (n <= 256) return n <= 200 && rounds == 1 && 16 * last >= (n <= 184 ? 14L : 16L) * cus;
   if (n <= 384) return whole_tiles ? rounds != 3 && rounds != 4 && 16 * last >= 15L * cus : 16 * last >= (rounds == 1 ? 14L : 15L) * cus;
   return rounds > 4 || 8 * last >= (rounds == 1 ? 7L : 6L) * cus;
 }

@@ -564,8 +564,8 @@ def test_backward_by_slice(tmp_path, lib):
         (64, 129, 129, 0), (64, 257, 192, 0), (64, 512, 192, 0), (64, 300, 448, 0), (64, 512, 600, 0), (64, 512, 1300, 0),
         (64, 264, 608, 0), (64, 352, 840, 0), (64, 384, 1216, 0), (64, 290, 1440, 0), (64, 304, 1704, 0), (64, 320, 1264, 1),
         (64, 264, 1264, 1),
-        (64, 129, 171, 1), (64, 160, 448, 1), (64, 200, 224, 1), (64, 384, 256, 1), (64, 512, 224, 1), (64, 512, 448, 1),
-        (64, 512, 1030, 1),
+        (64, 129, 171, 1), (64, 160, 448, 1), (64, 180, 224, 1), (64, 200, 256, 1), (64, 384, 256, 1),
+        (64, 512, 224, 1), (64, 512, 448, 1), (64, 512, 1030, 1),
     ]
     other = [
         (128, 1, 128, 0), (128, 257, 200, 0), (128, 256, 319, 0), (128, 256, 330, 1), (128, 100, 528, 0), (128, 100, 1030, 1),
@@ -573,6 +573,7 @@ def test_backward_by_slice(tmp_path, lib):
         (64, 300, 400, 0), (64, 384, 385, 0), (64, 290, 598, 0), (64, 290, 833, 0), (64, 320, 1076, 0), (64, 290, 1352, 0),
         (64, 304, 1544, 0), (64, 320, 224, 1), (64, 384, 224, 1), (64, 384, 752, 1), (64, 320, 1014, 1),  # whole tiles of 64 rows
         (64, 129, 160, 1), (64, 201, 256, 1), (64, 200, 480, 1), (64, 300, 480, 1), (64, 512, 208, 1), (64, 512, 640, 1),
+        (64, 192, 224, 1), (64, 193, 224, 1), (64, 200, 230, 1),
         (64, 300, 1030, 1), (64, 512, 96, 0), (128, 1, 1, 0), (64, 1, 1 << 23, 0),
     ]
     assert all(abi.host_rule(tmp_path, rule, slices)) and not any(abi.host_rule(tmp_path, rule, other))
