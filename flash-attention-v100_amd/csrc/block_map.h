@@ -328,6 +328,10 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 // 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512 x 432 93.7,
 // 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512 x 900 217, 198;
 // 512 x 1030 247, 246; 300 x 1030 124, 141.
+// Causal, D = 128, a second round of slices just past 96 rows (four tiles of 32 queries instead of three), us of forward and
+// backward, without it and with it: 97 x 257 37.1, 37.7; 97 x 266 37.8, 39.9; 97 x 296 39.2, 39.8; 97 x 320 39.8, 39.6; 105 x 266
+// 38.9, 40.3; 105 x 306 40.4, 40.2; 112 x 266 40.0, 40.6; 112 x 306 41.5, 40.5; 116 x 266 40.7, 40.7; 128 x 266 42.3, 41.4; and 96 x
+// 257 36.4, 33.4.
 // Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 27.0, 26.4; 161 x 256 27.3, 27.4;
 // 170 x 236 27.4, 26.5; 180 x 224 27.3, 27.2; 180 x 244 27.7, 27.4; 192 x 224 27.0, 27.5; 192 x 236 27.6, 27.1; 192 x 250 27.7, 28.1;
 // 193 x 224 29.3, 30.4; 193 x 250 30.5, 31.0; 200 x 230 29.9, 30.4; 200 x 240 30.3, 30.6; 200 x 256 32.0, 30.7.
@@ -346,6 +350,7 @@ FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, 
   if (d == 128) {
     if (rounds == 1) return 2 * last > cus;
     if (n <= 64) return true;
+    if (rounds == 2 && causal && n > 96 && n <= 112) return 5 * last >= cus;
     if (n <= 128) return rounds == 2 || rounds > 6 || 2 * last >= cus;
     return rounds > 2 || (causal && n > 160 ? 3 : 4) * last >= cus;
   }
