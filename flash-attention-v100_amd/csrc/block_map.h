@@ -215,6 +215,11 @@ FMHA_HOST_DEVICE int fmha_tail_slice(int lin, int wave, int tails, int per) {
 // x 181 22.3, 22.3; 530 x 170 29.4, 28.1; 520 x 100 17 % worse.  Past 576 rows 1 to 2 % in the mean, with losses among them; and
 // hardly anything, or less, where the blocks are just past full layers: D = 128 410 x 264 (5) 31.8, 33.2;
 // 257 x 257 (4) 21.2, 21.9; D = 64 410 x 257 (5) 20.3, 20.6.
+// And the more rounds (in brackets) the less: D = 128 257 x 624 (7.3) 42.3, 40.0; 288 x 625 (7.3) 43.5, 42.2; 257 x 641 (7.5) 43.5,
+// 43.0; 288 x 641 (7.5) 44.8, 46.0; 257 x 737 (8.6) 48.6, 49.0; 288 x 737 (8.6) 50.1, 52.2; 385 x 441 (6.9) 46.4, 45.5; 400 x 417 (6.5)
+// 45.6, 46.1; 400 x 481 (7.5) 51.3, 52.0; 400 x 537 (8.4) 56.3, 56.8; 416 x 249 (3.9) 30.5, 29.0; 416 x 276 (4.3) 32.1, 32.7; 416 x
+// 353 (5.5) 39.7, 41.4; 416 x 417 (6.5) 45.6, 46.6; 513 x 301 (5.9) 47.0, 45.9; 544 x 289 (5.6) 46.2, 46.5; 513 x 324 (6.3) 48.6, 49.8;
+// 544 x 385 (7.5) 58.2, 61.5; 513 x 455 (8.9) 67.2, 69.2; D = 64 416 x 489 (7.6) 33.7, 32.2.
 FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus, bool causal) {
   if (n <= 128 || (n - 1) % 128 >= 32) return 0;
   const long full = (long)slices * ((n - 1) / 128);
@@ -222,6 +227,8 @@ FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus, boo
              four = (full + fmha_tail_blocks(slices, 4) + cus - 1) / cus;
   if (causal && n > 160) {
     const long blocks = full + slices, left = blocks % cus;
+    const int most = n <= 288 ? 15 : n <= 400 ? 14 : n <= 512 ? 8 : 12;  // half rounds of blocks
+    if (d == 128 && 2 * blocks >= (long)most * cus) return 0;
     return n <= 576 && 480 * blocks >= (900L + n) * cus && 16 * left >= (d == 64 ? 1 : 5) * cus ? 4 : 0;
   }
   if (n > 768 && ((d == 128 && now > 6) || (now == 2 && (d == 64 || two == 2)))) return 0;

@@ -240,6 +240,7 @@ TAILS = [  # D, slices, N, causal, how many slices' last rows go to one block
     (64, 59, 1031, 0, 2), (64, 61, 1537, 0, 2), (64, 62, 1550, 0, 4), (128, 300, 160, 0, 2), (128, 181, 130, 0, 4),
     (128, 203, 257, 0, 2), (128, 150, 400, 0, 4), (128, 57, 1056, 0, 2), (128, 122, 1025, 0, 4),
     (64, 300, 129, 1, 2), (64, 401, 160, 1, 4), (64, 231, 288, 1, 4), (64, 199, 416, 1, 4), (64, 173, 513, 1, 4),
+    (128, 625, 288, 1, 4), (128, 301, 513, 1, 4),  # nearly as many rounds as it pays for
     (128, 150, 130, 1, 2), (128, 399, 150, 1, 4), (128, 230, 257, 1, 4), (128, 215, 385, 1, 4), (128, 170, 544, 1, 4),
 ]
 
@@ -249,7 +250,8 @@ def test_blocks_with_the_last_rows_of_slices(tmp_path):
     rule = "fmha_tails_per_block(x[0], x[2], x[1], 256, x[3]) == x[4]"
     alone = [(64, 300, 128), (64, 300, 161), (64, 230, 129), (64, 256, 257), (64, 30, 1031), (64, 34, 900), (128, 56, 1031),
              (128, 200, 1031), (128, 34, 900), (128, 1, 129), (64, 1, 1), (128, 230, 2070)]
-    causal = [(64, 256, 150), (128, 256, 129), (64, 100, 520), (64, 257, 410), (128, 264, 410), (128, 100, 520), (128, 200, 1031)]
+    causal = [(64, 256, 150), (128, 256, 129), (64, 100, 520), (64, 257, 410), (128, 264, 410), (128, 100, 520), (128, 200, 1031),
+              (128, 641, 288), (128, 710, 288), (128, 481, 400), (128, 276, 416), (128, 353, 416), (128, 324, 513), (128, 385, 544)]
     alone = [(*case, 0, 0) for case in alone] + [(*case, 1, 0) for case in causal]
     assert all(abi.host_rule(tmp_path, rule, TAILS + alone))
     src, exe = tmp_path / "tails.cpp", tmp_path / "tails"
