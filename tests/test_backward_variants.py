@@ -169,27 +169,39 @@ def test_a_work_group_for_each_slice(D, N, causal):
         assert torch.equal(a, b)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("ticks", [5000000, 0])
-@pytest.mark.parametrize("H,N,causal", [
+OVER_DS_AT_ONCE = [  # H, N, causal
     (520, 64, False), (515, 100, True), (517, 128, True),  # a block per slice and pass
     (261, 129, False), (200, 160, False), (200, 161, True),  # last blocks of 1, 32 and 33 rows
     (100, 384, True), (65, 512, False),
     (60, 1031, False), (37, 1056, False), (33, 1023, True),
     (18, 2047, True), (9, 4096, False),
-])
+]
+
+
+def test_launches_over_ds_of_the_cases_below(tmp_path):
+    """Both passes over dS go in one launch on 256 compute units, once it is not by slices."""
+    blocks = "(long)((x[1] + 127) / 128) * x[0], x[1], 256, x[2]"
+    assert all(abi.host_rule(tmp_path, f"fmha_ds_in_one_launch(x[0], x[1], 256, x[2]) && !fmha_passes_at_once(128, {blocks})",
+                             OVER_DS_AT_ONCE))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ticks", [5000000, 0])
+@pytest.mark.parametrize("H,N,causal", OVER_DS_AT_ONCE)
 def test_both_passes_over_ds_in_one_launch(H, N, causal, ticks):
-    """The bits of the passes one after the other, also (ticks) where no block waits for the dS of another."""
+    """The bits of the passes one after the other, also (ticks) where no block waits for the dS of another; what the blocks
+    have counted; nothing is left over from the call before, with other inputs."""
     B, D, lib = 1, 128, abi.load()
     lib.fmha_backward_waiting.argtypes = ([ctypes.c_void_p] * 7 + [ctypes.c_size_t] + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 +
                                           [ctypes.c_float, ctypes.c_int, ctypes.c_uint, ctypes.c_void_p])
     gen = torch.Generator(device="cuda").manual_seed(N + H)
-    q, k, v, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
-    out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
-    apart = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=True)[:3]
     nbytes = lib.fused_mha_backward_workspace_bytes(B, H, N, D) + 128 * H  # room for the counts of this launch
     ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
+    blocks, spread = -(-N // 128), H % 8  # of a slice; slices with blocks on several XCDs, the last ones
     for _ in range(2):
+        q, k, v, do = (torch.randn(B, N, H, D, device="cuda", dtype=torch.float16, generator=gen) for _ in range(4))
+        out, lse = abi.forward(lib, q, k, v, D ** -0.5, causal)
+        apart = abi.backward(lib, q, k, v, out, do, lse, D ** -0.5, causal, split=True)[:3]
         got = [torch.full_like(q, float("nan")) for _ in range(3)]
         rc = lib.fmha_backward_waiting(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), lse.data_ptr(),
                                        ws.data_ptr(), nbytes, *(g.data_ptr() for g in got), B, H, N, D, D ** -0.5, int(causal),
@@ -197,6 +209,12 @@ def test_both_passes_over_ds_in_one_launch(H, N, causal, ticks):
         assert rc == abi.OK
         for a, b in zip(got, apart):
             assert torch.equal(a, b)
+        counts = ws[-128 * H:].view(torch.int32).view(H, 32)
+        assert (counts[:, 0] == 4 * blocks).all()  # waves that have stored dS
+        assert (counts[:H - spread, 1] == 0).all() and (counts[H - spread:, 1] == blocks).all()  # dK/dV blocks that have started
+        if ticks:  # dQ blocks that have formed S and dP themselves
+            assert (counts[:H - spread, 2] == 0).all()
+        assert (counts[:, 2] <= blocks).all() and (counts[:, 3:] == 0).all()
 
 
 @pytest.mark.gpu

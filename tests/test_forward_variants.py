@@ -238,6 +238,7 @@ def test_rows_that_are_not_finite(B, H, N, D, causal):
 TAILS = [  # D, slices, N, causal, how many slices' last rows go to one block
     (64, 300, 129, 0, 2), (64, 401, 150, 0, 4), (64, 100, 257, 0, 2), (64, 110, 520, 0, 2), (64, 118, 544, 0, 4),
     (64, 59, 1031, 0, 2), (64, 61, 1537, 0, 2), (64, 62, 1550, 0, 4), (128, 300, 160, 0, 2), (128, 181, 130, 0, 4),
+    (128, 90, 1025, 0, 2),  # with every other wave slot first
     (128, 203, 257, 0, 2), (128, 150, 400, 0, 4), (128, 57, 1056, 0, 2), (128, 122, 1025, 0, 4),
     (64, 300, 129, 1, 2), (64, 401, 160, 1, 4), (64, 231, 288, 1, 4), (64, 199, 416, 1, 4), (64, 173, 513, 1, 4),
     (128, 625, 288, 1, 4), (128, 301, 513, 1, 4),  # nearly as many rounds as it pays for
