@@ -183,9 +183,9 @@ FMHA_HOST_DEVICE int fmha_paired_block(int lin, int total) {
   return ((kCus / 8 + slots - 1 - (lin >> 3)) << 3) + xcd;
 }
 
-// The 128-query forward where the last block of every slice has up to 32 queries: those of `per` (2 or 4) slices
-// can go to one block, a wave each (fwd_tail_rows), in front of all others; as many blocks as a multiple of 8, so that the others
-// stay on the XCD of their slice.  Work group `lin` and wave -> slice; one past the last means none.
+// The 128-query forward where the last block of every slice has up to 32 queries: those of `per` (2 or 4) slices can go to one
+// block, a wave each (fwd_tail_rows), in front of all others; as many blocks as a multiple of 8, so that the others stay on the
+// XCD of their slice.  Work group `lin` and wave -> slice; one past the last means none.
 FMHA_HOST_DEVICE int fmha_tail_blocks(int slices, int per) { return ((slices + per - 1) / per + 7) & ~7; }
 FMHA_HOST_DEVICE int fmha_tail_slice(int lin, int wave, int tails, int per) {
   return per * ((lin & 7) * (tails >> 3) + (lin >> 3)) + wave;  // an XCD has slices next to each other here too
@@ -194,32 +194,32 @@ FMHA_HOST_DEVICE int fmha_tail_slice(int lin, int wave, int tails, int per) {
 // Whether they do: 0, or how many to a block.  Blocks of the same length are done in layers of one to a CU, and it pays where
 // there are fewer of those.  Two to a block where that gives as few as four does, since four streams of K and V are slow beside
 // another block.  us of the forward with a block for each, two and four to a block, N x slices (layers):
-// D = 64.  129 x 230 (2, 2, 2) 7.8, 8.0, 8.3; 129 x 300 (3, 2, 2) 11.5, 8.7, 8.7; 129 x 400 (4, 3, 2) 13.9, 11.8, 9.5; 129 x 512
-// (4, 3, 3) 16.4, 12.1, 12.8; 129 x 4000 (32, 24, 20) 99.0, 80.2, 77.8; 257 x 100 (2, 1, 1) 9.6, 7.7, 7.8; 257 x 400 (5, 4, 4)
-// 24.9, 22.1, 21.8; 520 x 110 (3, 2, 2) 21.8, 17.1, 18.1; 520 x 120 (3, 3, 2) 22.0, 22.1, 18.4; 520 x 150 (3, 3, 3) 24.0, 24.4,
-// 23.4; 660 x 90 (3, 2, 2) 24.9, 19.8, 20.7; 1031 x 56 (2, 2, 2) 26.5, 27.2, 27.9; 1031 x 60 (3, 2, 2) 31.8, 27.9, 28.5; 1031 x 230
-// (9, 8, 8) 98.5, 94.6, 92.4; 2070 x 31 (3, 2, 2) 54.5, 48.8, 49.7; 2070 x 200 (14, 13, 13) 276, 275, 268.
-// D = 128.  129 x 230 (2, 2, 2) 13.7, 11.9, 13.7; 129 x 300 (3, 2, 2) 19.6, 13.2, 14.8; 257 x 200 (3, 2, 2) 23.9, 20.2, 21.8; 257 x
-// 700 (9, 7, 7) 67.2, 60.4, 57.2; 520 x 56 (2, 1, 1) 20.9, 17.9, 18.8; 520 x 64 (2, 2, 2) 21.9, 23.1, 24.4; 520 x 600 (12, 11, 10)
-// 138, 136, 130; 1031 x 56 (2, 2, 2) 41.9, 44.2, 46.0; 1031 x 60 (3, 2, 2) 50.1, 46.0, 48.0; 1031 x 120 (5, 4, 4) 87.9, 82.7, 81.0;
-// 1300 x 48 (3, 2, 2) 58.2, 53.8, 56.8; 2070 x 31 (3, 2, 2) 88.6, 81.8, 84.2.
+// D = 64.  129 x 230 (2, 2, 2) 7.8, 8.0, 8.3; 129 x 300 (3, 2, 2) 11.5, 8.7, 8.7; 129 x 400 (4, 3, 2) 13.9, 11.8, 9.5; 129 x
+// 512 (4, 3, 3) 16.4, 12.1, 12.8; 129 x 4000 (32, 24, 20) 99.0, 80.2, 77.8; 257 x 100 (2, 1, 1) 9.6, 7.7, 7.8; 257 x 400 (5, 4,
+// 4) 24.9, 22.1, 21.8; 520 x 110 (3, 2, 2) 21.8, 17.1, 18.1; 520 x 120 (3, 3, 2) 22.0, 22.1, 18.4; 520 x 150 (3, 3, 3) 24.0,
+// 24.4, 23.4; 660 x 90 (3, 2, 2) 24.9, 19.8, 20.7; 1031 x 56 (2, 2, 2) 26.5, 27.2, 27.9; 1031 x 60 (3, 2, 2) 31.8, 27.9, 28.5;
+// 1031 x 230 (9, 8, 8) 98.5, 94.6, 92.4; 2070 x 31 (3, 2, 2) 54.5, 48.8, 49.7; 2070 x 200 (14, 13, 13) 276, 275, 268.
+// D = 128.  129 x 230 (2, 2, 2) 13.7, 11.9, 13.7; 129 x 300 (3, 2, 2) 19.6, 13.2, 14.8; 257 x 200 (3, 2, 2) 23.9, 20.2, 21.8;
+// 257 x 700 (9, 7, 7) 67.2, 60.4, 57.2; 520 x 56 (2, 1, 1) 20.9, 17.9, 18.8; 520 x 64 (2, 2, 2) 21.9, 23.1, 24.4; 520 x 600
+// (12, 11, 10) 138, 136, 130; 1031 x 56 (2, 2, 2) 41.9, 44.2, 46.0; 1031 x 60 (3, 2, 2) 50.1, 46.0, 48.0; 1031 x 120 (5, 4, 4)
+// 87.9, 82.7, 81.0; 1300 x 48 (3, 2, 2) 58.2, 53.8, 56.8; 2070 x 31 (3, 2, 2) 88.6, 81.8, 84.2.
 // Not past three rounds of longer ones at D = 128: 1031 x 200 (8, 7, 7) 146, 150, 150; 2070 x 230 (16, 15, 15) 550, 579, 539.
 // Nor from two layers to one where it is the wave on its own that takes the time: D = 64 660 x 45 15.6, 13.8, 15.4; 1031 x 30
-// 20.4, 20.6, 21.7; 1300 x 24 23.8, 24.9, 25.9; and with four to a block 900 x 34 18.7, 21.7, 19.5.  D = 128 1031 x 30 31.8, 29.1,
-// 31.7; 900 x 34 28.8, 32.8, 28.8.
+// 20.4, 20.6, 21.7; 1300 x 24 23.8, 24.9, 25.9; and with four to a block 900 x 34 18.7, 21.7, 19.5.  D = 128 1031 x 30 31.8,
+// 29.1, 31.7; 900 x 34 28.8, 32.8, 28.8.
 // Under causal masking these rows have more keys than any others, and go first anyhow.  Up to 160 rows, where that makes two
-// kinds of block alike, by the layers too (D = 64 129 x 300 40, 129 x 400 13 and 57 % faster; D = 128 150 x 300 29 and 15, 150 x 256
-// (2, 2, 2) 7 and 11 slower).  Longer ones: a launch must last longer than a wave for itself takes, and the fewer blocks of a
-// slice the more there is to gain; with a block for each and four to a block: D = 64 257 x 230 14.0, 12.3; 400 x 200 17.8, 15.8;
-// 520 x 180 1 % better, 520 x 512 5 %, 520 x 100 11 % worse; D = 128 257 x 219 19.5, 16.0; 288 x 376 29.8, 26.8; 385 x 216 27.1, 24.9; 410
-// x 181 22.3, 22.3; 530 x 170 29.4, 28.1; 520 x 100 17 % worse.  Past 576 rows 1 to 2 % in the mean, with losses among them; and
-// hardly anything, or less, where the blocks are just past full layers: D = 128 410 x 264 (5) 31.8, 33.2;
-// 257 x 257 (4) 21.2, 21.9; D = 64 410 x 257 (5) 20.3, 20.6.
-// And the more rounds (in brackets) the less: D = 128 257 x 624 (7.3) 42.3, 40.0; 288 x 625 (7.3) 43.5, 42.2; 257 x 641 (7.5) 43.5,
-// 43.0; 288 x 641 (7.5) 44.8, 46.0; 257 x 737 (8.6) 48.6, 49.0; 288 x 737 (8.6) 50.1, 52.2; 385 x 441 (6.9) 46.4, 45.5; 400 x 417 (6.5)
-// 45.6, 46.1; 400 x 481 (7.5) 51.3, 52.0; 400 x 537 (8.4) 56.3, 56.8; 416 x 249 (3.9) 30.5, 29.0; 416 x 276 (4.3) 32.1, 32.7; 416 x
-// 353 (5.5) 39.7, 41.4; 416 x 417 (6.5) 45.6, 46.6; 513 x 301 (5.9) 47.0, 45.9; 544 x 289 (5.6) 46.2, 46.5; 513 x 324 (6.3) 48.6, 49.8;
-// 544 x 385 (7.5) 58.2, 61.5; 513 x 455 (8.9) 67.2, 69.2; D = 64 416 x 489 (7.6) 33.7, 32.2.
+// kinds of block alike, by the layers too (D = 64 129 x 300 40, 129 x 400 13 and 57 % faster; D = 128 150 x 300 29 and 15, 150
+// x 256 (2, 2, 2) 7 and 11 slower).  Longer ones: a launch must last longer than a wave for itself takes, and the fewer blocks
+// of a slice the more there is to gain; with a block for each and four to a block: D = 64 257 x 230 14.0, 12.3; 400 x 200 17.8,
+// 15.8; 520 x 180 1 % better, 520 x 512 5 %, 520 x 100 11 % worse; D = 128 257 x 219 19.5, 16.0; 288 x 376 29.8, 26.8; 385 x
+// 216 27.1, 24.9; 410 x 181 22.3, 22.3; 530 x 170 29.4, 28.1; 520 x 100 17 % worse.  Past 576 rows 1 to 2 % in the mean, with
+// losses among them; and hardly anything, or less, where the blocks are just past full layers: D = 128 410 x 264 (5) 31.8,
+// 33.2; 257 x 257 (4) 21.2, 21.9; D = 64 410 x 257 (5) 20.3, 20.6.
+// And the more rounds (in brackets) the less: D = 128 257 x 624 (7.3) 42.3, 40.0; 288 x 625 (7.3) 43.5, 42.2; 257 x 641 (7.5)
+// 43.5, 43.0; 288 x 641 (7.5) 44.8, 46.0; 257 x 737 (8.6) 48.6, 49.0; 288 x 737 (8.6) 50.1, 52.2; 385 x 441 (6.9) 46.4, 45.5;
+// 400 x 417 (6.5) 45.6, 46.1; 400 x 481 (7.5) 51.3, 52.0; 400 x 537 (8.4) 56.3, 56.8; 416 x 249 (3.9) 30.5, 29.0; 416 x 276
+// (4.3) 32.1, 32.7; 416 x 353 (5.5) 39.7, 41.4; 416 x 417 (6.5) 45.6, 46.6; 513 x 301 (5.9) 47.0, 45.9; 544 x 289 (5.6) 46.2,
+// 46.5; 513 x 324 (6.3) 48.6, 49.8; 544 x 385 (7.5) 58.2, 61.5; 513 x 455 (8.9) 67.2, 69.2; D = 64 416 x 489 (7.6) 33.7, 32.2.
 FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus, bool causal) {
   if (n <= 128 || (n - 1) % 128 >= 32) return 0;
   const long full = (long)slices * ((n - 1) / 128);
@@ -255,12 +255,13 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
   second_pass = v & 1;
 }
 
-// A launch of all blocks of the dK/dV pass and then all of the dQ pass over the dS that it stores, nb each per slice, either
-// in the order of a launch of its own (the short last blocks of sequences without a mask in their places: what comes last
-// are the dQ blocks, and they wait for whole slices).  The second part begins at a multiple of 8, so that a slice stays on its
-// XCD; the up to 7 work groups before that have no block.
+// A launch of all blocks of the dK/dV pass and then all of the dQ pass over the dS that it stores, nb each per slice, either in
+// the order of a launch of its own (the short last blocks of sequences without a mask in their places: what comes last are the
+// dQ blocks, and they wait for whole slices).  The second part begins at a multiple of 8, so that a slice stays on its XCD; the
+// up to 7 work groups before that have no block.
 FMHA_HOST_DEVICE int fmha_ds_launch_blocks(int slices, int nb) { return ((slices * nb + 7) & ~7) + slices * nb; }
-FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool heavy_first, int& slice, int& blk, bool& second_pass) {
+FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool heavy_first, int& slice, int& blk,
+                                           bool& second_pass) {
   const int blocks = slices * nb, second = (blocks + 7) & ~7;
   second_pass = lin >= second;
   if (second_pass) lin -= second;
@@ -280,27 +281,32 @@ FMHA_HOST_DEVICE unsigned fmha_ds_wait_ticks(int n, bool started) { return (500u
 // far from full, and with few rounds, and a launch where these are short; it loses where a dQ block of 128 queries is much
 // slower than the one of 256 that the dQ pass alone takes then (half of the copies of K), which long sequences feel.  us of the
 // backward, passes apart and in one launch, N x slices (rounds of blocks of 128 rows):
-// Up to 768 rows.  64 x 520 (2.0) 40.3, 30.4; 64 x 1200 (4.7) 59.5, 59.4; 100 x 300 (1.2) 44.2, 34.9; 100 x 3000 (11.7) 226, 235;
-// 128 x 600 63.1, 50.9; 128 x 2000 (7.8) 177, 174; 200 x 200 46.0, 37.3; 256 x 256 (2) 52.5, 51.5; 300 x 86 (1.0) 42.3, 32.5; 384 x
-// 400 (4.7) 159, 144; 512 x 64 (1) 38.2, 35.7; 512 x 100 63.4, 54.9; 512 x 192 (3) 107, 103; 512 x 256 (4) 140, 141; 512 x 600
-// (9.4) 346, 345; 640 x 128 (2.5) 112, 97; 640 x 300 (5.9) 251, 243.  Causal: 64 x 600 43.5, 33.9; 64 x 2000 (7.8) 98.0, 98.2; 128
-// x 1200 (4.7) 117, 99; 200 x 400 69.9, 58.3; 200 x 1000 (7.8) 153, 157; 256 x 300 62.5, 50.7; 256 x 1000 191, 184; 512 x 80
-// 42.4, 37.6; 512 x 192 (3) 86.7, 78.2; 512 x 400 (6.3) 176, 171; 640 x 200 (3.9) 123, 114.
+// Up to 768 rows.  64 x 520 (2.0) 40.3, 30.4; 64 x 1200 (4.7) 59.5, 59.4; 100 x 300 (1.2) 44.2, 34.9; 100 x 3000 (11.7) 226,
+// 235; 128 x 600 63.1, 50.9; 128 x 2000 (7.8) 177, 174; 200 x 200 46.0, 37.3; 256 x 256 (2) 52.5, 51.5; 300 x 86 (1.0) 42.3,
+// 32.5; 384 x 400 (4.7) 159, 144; 512 x 64 (1) 38.2, 35.7; 512 x 100 63.4, 54.9; 512 x 192 (3) 107, 103; 512 x 256 (4) 140,
+// 141; 512 x 600 (9.4) 346, 345; 640 x 128 (2.5) 112, 97; 640 x 300 (5.9) 251, 243.  Causal: 64 x 600 43.5, 33.9; 64 x 2000
+// (7.8) 98.0, 98.2; 128 x 1200 (4.7) 117, 99; 200 x 400 69.9, 58.3; 200 x 1000 (7.8) 153, 157; 256 x 300 62.5, 50.7; 256 x 1000
+// 191, 184; 512 x 80 42.4, 37.6; 512 x 192 (3) 86.7, 78.2; 512 x 400 (6.3) 176, 171; 640 x 200 (3.9) 123, 114.
 // Longer, without a mask.  One round or less: 1024 x 32 59.2, 55.5; 1280 x 20 59.6, 57.6; 2048 x 16 97.0, 95.9; 4096 x 8 185,
-// 193.  777 x 40 (1.1) 69.4, 58.2; 777 x 100 (2.7) 136, 125; 1024 x 48 (1.5) 96.2, 86.0; 1024 x 64 (2) 107, 106; 1024 x 96 (3) 165,
-// 167; 1031 x 60 (2.1) 129, 114; 1500 x 24 (1.1) 123, 105; 1500 x 48 (2.3) 204, 177; 1500 x 64 (3) 232, 234; 1500 x 100 (4.7)
-// 374, 375; 2048 x 20 (1.3) 158, 135; 2048 x 28 (1.8) 189, 186; 2048 x 56 (3.5) 368, 353; 2048 x 64 (4) 397, 404; 2048 x 130 (8.1)
-// 872, 839; 2048 x 170 (10.6) 1089, 1100; 3000 x 12 (1.1) 230, 195; 3000 x 50 (4.7) 664, 677; 4096 x 10 (1.3) 309, 263; 4096 x
-// 20 (2.5) 506, 482; 4096 x 32 (4) 710, 739; 4096 x 42 (5.3) 1002, 992; 4096 x 52 (6.5) 1230, 1239; 6000 x 6 (1.1) 435, 435;
-// 6000 x 8 (1.5) 470, 473; 6000 x 12 (2.2) 705, 618; 8192 x 5 (1.3) 574, 582; 8192 x 9 (2.3) 909, 828; 8192 x 17 (4.3) 1606,
-// 1540; 16384 x 3 1189, 1211.
-// Longer, causal.  777 x 64 (1.8) 58.0, 54.8; 777 x 300 (8.2) 267, 262; 1024 x 40 54.6, 50.4; 1024 x 128 (4) 144, 146; 1024 x 150
-// 190, 176; 1024 x 220 (6.9) 276, 264; 1280 x 100 (3.9) 176, 170; 1500 x 48 (2.3) 118, 108; 1500 x 80 (3.8) 189, 181; 2048 x 20 85.3,
-// 81.0; 2048 x 56 (3.5) 213, 208; 2048 x 64 (4) 232, 237; 2048 x 80 (5) 296, 299; 4096 x 9 (1.1) 149, 140; 4096 x 11 (1.4) 159,
-// 153; 4096 x 12 (1.5) 169, 171; 4096 x 16 (2) 207, 210; 8192 x 6 323, 324; 8192 x 12 (3) 586, 594; 16384 x 16 (8) 2820, 2919.
-// Past six rounds the figures above leave out what the one launch pays for dS past the L2s when others follow; forward and backward
-// as calls, no mask: 1500 x 110 (5.2) 589, 572; 1500 x 155 (7.3) 814, 800; 2048 x 84 (5.3) 757, 741; 2048 x 100 (6.3) 912, 915; 2048
-// x 114 (7.1) 1017, 1020; 2048 x 130 (8.1) 1178, 1191; 4096 x 42 (5.3) 1390, 1373.
+// 193.  777 x 40 (1.1) 69.4, 58.2; 777 x 100 (2.7) 136, 125; 1024 x 48 (1.5) 96.2, 86.0; 1024 x 64 (2) 107, 106; 1024 x 96 (3)
+// 165, 167; 1031 x 60 (2.1) 129, 114; 1500 x 24 (1.1) 123, 105; 1500 x 48 (2.3) 204, 177; 1500 x 64 (3) 232, 234; 1500 x 100
+// (4.7) 374, 375; 2048 x 20 (1.3) 158, 135; 2048 x 28 (1.8) 189, 186; 2048 x 56 (3.5) 368, 353; 2048 x 64 (4) 397, 404; 2048 x
+// 130 (8.1) 872, 839; 2048 x 170 (10.6) 1089, 1100; 3000 x 12 (1.1) 230, 195; 3000 x 50 (4.7) 664, 677; 4096 x 10 (1.3) 309,
+// 263; 4096 x 20 (2.5) 506, 482; 4096 x 32 (4) 710, 739; 4096 x 42 (5.3) 1002, 992; 4096 x 52 (6.5) 1230, 1239; 6000 x 6 (1.1)
+// 435, 435; 6000 x 8 (1.5) 470, 473; 6000 x 12 (2.2) 705, 618; 8192 x 5 (1.3) 574, 582; 8192 x 9 (2.3) 909, 828; 8192 x 17
+// (4.3) 1606, 1540; 16384 x 3 1189, 1211.
+// Longer, causal.  777 x 64 (1.8) 58.0, 54.8; 777 x 300 (8.2) 267, 262; 1024 x 40 54.6, 50.4; 1024 x 128 (4) 144, 146; 1024 x
+// 150 190, 176; 1024 x 220 (6.9) 276, 264; 1280 x 100 (3.9) 176, 170; 1500 x 48 (2.3) 118, 108; 1500 x 80 (3.8) 189, 181; 2048
+// x 20 85.3, 81.0; 2048 x 56 (3.5) 213, 208; 2048 x 64 (4) 232, 237; 2048 x 80 (5) 296, 299; 4096 x 9 (1.1) 149, 140; 4096 x 11
+// (1.4) 159, 153; 4096 x 12 (1.5) 169, 171; 4096 x 16 (2) 207, 210; 8192 x 6 323, 324; 8192 x 12 (3) 586, 594; 16384 x 16 (8)
+// 2820, 2919.
+// Past six rounds the figures above leave out what the one launch pays for dS past the L2s when others follow; us of forward
+// and backward as calls, in two launches and in one, no mask: 260 x 631 (7.4) 241, 230; 384 x 631 (7.4) 316, 313; 400 x 473
+// (7.4) 295, 294; 768 x 315 (7.4) 462, 456; 777 x 230 (6.3) 383, 377; 777 x 303 (8.3) 520, 512; 1000 x 265 (8.3) 666, 634; 1024
+// x 265 (8.3) 656, 638; 1500 x 110 (5.2) 589, 572; 1500 x 155 (7.3) 814, 800; 2048 x 84 (5.3) 757, 741; 2048 x 100 (6.3) 912,
+// 915; 2048 x 114 (7.1) 1017, 1020; 2048 x 130 (8.1) 1178, 1191; 4096 x 42 (5.3) 1390, 1373.  Causal: 400 x 473 (7.4) 223, 223;
+// 700 x 268 (6.3) 245, 246; 768 x 315 (7.4) 322, 317; 900 x 198 (6.2) 277, 281; 1000 x 220 (6.9) 352, 351; 1024 x 220 (6.9)
+// 353, 350.
 FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool causal) {
   const long blocks = (long)slices * ((n + 127) / 128), left = blocks % cus;
   if (n <= 768) return 2 * blocks <= 15L * cus;
@@ -313,44 +319,48 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 }
 
 // Whether the backward takes a work group for each slice (fmha_bwd_slice_kernel, one to a CU), before all of the below.  It
-// forms S and dP once, as the D = 128 passes over dS do, but needs no room for dS, makes the statistics and is one launch; and it
-// reads Q, K, V and dO once.  It loses where slices leave CUs idle that blocks of 128 rows would fill: with few slices, and with
-// a last round that is far from full, the more so the longer a round is and under causal masking, where half of the blocks of a
-// slice are light, which the other launches pair with heavy ones.  At D = 64 up to 128 rows half of its waves have no keys, and
-// blocks of 128 rows, two to a CU, are ahead (64 x 256 equal, 128 x 256 and 128 x 1024 lose 4 and 18 %).
+// forms S and dP once, as the D = 128 passes over dS do, but needs no room for dS, makes the statistics and is one launch; and
+// it reads Q, K, V and dO once.  It loses where slices leave CUs idle that blocks of 128 rows would fill: with few slices, and
+// with a last round that is far from full, the more so the longer a round is and under causal masking, where half of the blocks
+// of a slice are light, which the other launches pair with heavy ones.  At D = 64 up to 128 rows half of its waves have no
+// keys, and blocks of 128 rows, two to a CU, are ahead (64 x 256 equal, 128 x 256 and 128 x 1024 lose 4 and 18 %).
 // us of the kernels of the backward, without it and with it, N x slices:
-// D = 128, without a mask.  One round: 40 x 128 7.5, 8.9; 40 x 160 12.9, 9.1; 200 x 128 25.5, 26.8; 256 x 136 43.0, 30.1; 256 x 256
-// 51.9, 37.4.  Two: 17 x 264 16.8, 11.9; 100 x 264 32.8, 28.6; 160 x 288 42.8, 46.0; 160 x 320 47.8, 45.8; 256 x 288 56.5, 60.8;
-// 256 x 320 61.2, 61.8; 256 x 512 100.3, 77.7.  More: 33 x 514 24.7, 23.9; 50 x 528 27.8, 27.6; 100 x 528 41.9, 44.2; 100 x 640
-// 48.2, 45.0; 100 x 800 59.7, 61.0; 100 x 1030 73.0, 75.8; 100 x 1600 120.8, 114.0; 256 x 528 106.2, 99.8; 256 x 1024 206, 163.
-// D = 128, causal.  160 x 128 22.1, 18.4 but 200 x 128 25.4, 24.3 and 100 x 128 slower; 256 x 160 35.8, 28.6; 256 x 256 43.5, 32.5;
-// 160 x 288 37.4, 35.5; 256 x 288 48.5, 55.3; 256 x 336 56.3, 57.5; 256 x 352 58.4, 58.0; 256 x 512 86.0, 64.9; 100 x 514 40.1,
-// 42.5; 100 x 640 48.8, 43.9; 256 x 528 90.9, 89.7.
-// D = 64, without a mask.  256 x 128 15.7, 18.8; 145 x 144 15.8, 12.9; 256 x 144 21.2, 19.1; 300 x 168 30.2, 32.1; 300 x
-// 192 34.3, 32.7; 512 x 192 60.9, 52.8; 512 x 256 78.5, 61.8; 300 x 352 60.1, 61.7; 300 x 384 61.2, 62.2; 300 x
-// 400 62.9, 62.7; 512 x 384 115, 110; 512 x 448 131, 115; 300 x 560 85.2, 92.2; 300 x 600 92.6, 92.5; 512 x 560 173, 177; 512 x
-// 620 191, 180; 300 x 770 115, 123; 300 x 900 135, 129; 300 x 1030 157, 159; 512 x 1030 339, 299; 512 x 1300 427, 362.
-// D = 64, causal.  129 x 160 12.6, 13.1; 129 x 168 14.5, 13.1; 160 x 256 19.1, 15.1; 145 x 416 26.9, 26.6; 145 x 448 28.1, 27.3; 145
-// x 600 35.9, 39.0; 180 x 208 16.8, 16.3; 200 x 230 20.1, 18.7; 256 x 240 22.0, 22.1; 300 x 208 27.3, 29.2; 300 x 230 31.3, 29.3;
-// 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512 x 432 93.7,
-// 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512 x 900 217, 198;
-// 512 x 1030 247, 246; 300 x 1030 124, 141.
+// D = 128, without a mask.  One round: 40 x 128 7.5, 8.9; 40 x 160 12.9, 9.1; 200 x 128 25.5, 26.8; 256 x 136 43.0, 30.1; 256 x
+// 256 51.9, 37.4.  Two: 17 x 264 16.8, 11.9; 100 x 264 32.8, 28.6; 160 x 288 42.8, 46.0; 160 x 320 47.8, 45.8; 256 x 288 56.5,
+// 60.8; 256 x 320 61.2, 61.8; 256 x 512 100.3, 77.7.  More: 33 x 514 24.7, 23.9; 50 x 528 27.8, 27.6; 100 x 528 41.9, 44.2; 100
+// x 640 48.2, 45.0; 100 x 800 59.7, 61.0; 100 x 1030 73.0, 75.8; 100 x 1600 120.8, 114.0; 256 x 528 106.2, 99.8; 256 x 1024
+// 206, 163.
+// D = 128, causal.  160 x 128 22.1, 18.4 but 200 x 128 25.4, 24.3 and 100 x 128 slower; 256 x 160 35.8, 28.6; 256 x 256 43.5,
+// 32.5; 160 x 288 37.4, 35.5; 256 x 288 48.5, 55.3; 256 x 336 56.3, 57.5; 256 x 352 58.4, 58.0; 256 x 512 86.0, 64.9; 100 x 514
+// 40.1, 42.5; 100 x 640 48.8, 43.9; 256 x 528 90.9, 89.7.
+// D = 64, without a mask.  256 x 128 15.7, 18.8; 145 x 144 15.8, 12.9; 256 x 144 21.2, 19.1; 300 x 168 30.2, 32.1; 300 x 192
+// 34.3, 32.7; 512 x 192 60.9, 52.8; 512 x 256 78.5, 61.8; 300 x 352 60.1, 61.7; 300 x 384 61.2, 62.2; 300 x 400 62.9, 62.7; 512
+// x 384 115, 110; 512 x 448 131, 115; 300 x 560 85.2, 92.2; 300 x 600 92.6, 92.5; 512 x 560 173, 177; 512 x 620 191, 180; 300 x
+// 770 115, 123; 300 x 900 135, 129; 300 x 1030 157, 159; 512 x 1030 339, 299; 512 x 1300 427, 362.
+// D = 64, causal.  129 x 160 12.6, 13.1; 129 x 168 14.5, 13.1; 160 x 256 19.1, 15.1; 145 x 416 26.9, 26.6; 145 x 448 28.1,
+// 27.3; 145 x 600 35.9, 39.0; 180 x 208 16.8, 16.3; 200 x 230 20.1, 18.7; 256 x 240 22.0, 22.1; 300 x 208 27.3, 29.2; 300 x 230
+// 31.3, 29.3; 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512
+// x 432 93.7, 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512
+// x 900 217, 198; 512 x 1030 247, 246; 300 x 1030 124, 141.
+// D = 64 without a mask, 385 to 512 rows, one round: the line is at the fewest slices that were timed, not where the passes are
+// as fast.  A round takes as long with fewer (512 rows: 52.7), and the passes 57.5 for 512 x 176.
 // Causal, D = 128, a second round of slices just past 96 rows (four tiles of 32 queries instead of three), us of forward and
-// backward, without it and with it: 97 x 257 37.1, 37.7; 97 x 266 37.8, 39.9; 97 x 296 39.2, 39.8; 97 x 320 39.8, 39.6; 105 x 266
-// 38.9, 40.3; 105 x 306 40.4, 40.2; 112 x 266 40.0, 40.6; 112 x 306 41.5, 40.5; 116 x 266 40.7, 40.7; 128 x 266 42.3, 41.4; and 96 x
-// 257 36.4, 33.4.
-// Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 27.0, 26.4; 161 x 256 27.3, 27.4;
-// 170 x 236 27.4, 26.5; 180 x 224 27.3, 27.2; 180 x 244 27.7, 27.4; 192 x 224 27.0, 27.5; 192 x 236 27.6, 27.1; 192 x 250 27.7, 28.1;
-// 193 x 224 29.3, 30.4; 193 x 250 30.5, 31.0; 200 x 230 29.9, 30.4; 200 x 240 30.3, 30.6; 200 x 256 32.0, 30.7.
+// backward, without it and with it: 97 x 257 37.1, 37.7; 97 x 266 37.8, 39.9; 97 x 296 39.2, 39.8; 97 x 320 39.8, 39.6; 105 x
+// 266 38.9, 40.3; 105 x 306 40.4, 40.2; 112 x 266 40.0, 40.6; 112 x 306 41.5, 40.5; 116 x 266 40.7, 40.7; 128 x 266 42.3, 41.4;
+// and 96 x 257 36.4, 33.4.
+// Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 27.0, 26.4; 161 x 256 27.3,
+// 27.4; 170 x 236 27.4, 26.5; 180 x 224 27.3, 27.2; 180 x 244 27.7, 27.4; 192 x 224 27.0, 27.5; 192 x 236 27.6, 27.1; 192 x 250
+// 27.7, 28.1; 193 x 224 29.3, 30.4; 193 x 250 30.5, 31.0; 200 x 230 29.9, 30.4; 200 x 240 30.3, 30.6; 200 x 256 32.0, 30.7.
 // From 257 to 384 rows at D = 64 the line depends on the last tile of 64 rows too, of which the other launches do all even if
 // only half of it has rows (257 to 288 and 321 to 352 rows).  us of forward and backward, without it and with it, N x slices:
-// last tile whole, no mask: 290 x 448 99.7, 95.1; 384 x 448 119.6, 116.1; 290 x 704 144.3, 142.8; 304 x 960 195, 192; 384 x 1216
-// 317, 305; 290 x 1216 242, 245; 290 x 1440 294, 293; 320 x 1440 307, 300; 289 x 1576 329, 331; 304 x 1704 366, 351; but 384 x 385
-// 100, 103; 290 x 598 124, 127; 290 x 833 160, 167; 320 x 1076 218, 225; 290 x 1352 269, 281; 304 x 1544 330, 337.  Causal: 320 x 248
-// 47.6, 45.2; 384 x 248 54.3, 53.2; 384 x 496 102, 100; 320 x 1264 216, 215; 289 x 1520 260, 251; but 320 x 224 43.0, 43.7; 384 x 224
-// 49.7, 51.2; 384 x 752 143, 150; 320 x 1014 160, 168.
-// Last tile half empty, no mask: 264 x 608 121, 116; 264 x 840 155, 153; 352 x 400 105, 102; 352 x 840 201, 201; 352 x 1080 262, 263;
-// 264 x 1336 244, 235; 352 x 1320 332, 321.  Causal: 264 x 232 44.1, 39.0; 352 x 224 48.7, 47.9; 264 x 752 116, 106; 352 x 1008 191, 187.
+// last tile whole, no mask: 290 x 448 99.7, 95.1; 384 x 448 119.6, 116.1; 290 x 704 144.3, 142.8; 304 x 960 195, 192; 384 x
+// 1216 317, 305; 290 x 1216 242, 245; 290 x 1440 294, 293; 320 x 1440 307, 300; 289 x 1576 329, 331; 304 x 1704 366, 351; but
+// 384 x 385 100, 103; 290 x 598 124, 127; 290 x 833 160, 167; 320 x 1076 218, 225; 290 x 1352 269, 281; 304 x 1544 330, 337.
+// Causal: 320 x 248 47.6, 45.2; 384 x 248 54.3, 53.2; 384 x 496 102, 100; 320 x 1264 216, 215; 289 x 1520 260, 251; but 320 x
+// 224 43.0, 43.7; 384 x 224 49.7, 51.2; 384 x 752 143, 150; 320 x 1014 160, 168.
+// Last tile half empty, no mask: 264 x 608 121, 116; 264 x 840 155, 153; 352 x 400 105, 102; 352 x 840 201, 201; 352 x 1080
+// 262, 263; 264 x 1336 244, 235; 352 x 1320 332, 321.  Causal: 264 x 232 44.1, 39.0; 352 x 224 48.7, 47.9; 264 x 752 116, 106;
+// 352 x 1008 191, 187.
 FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, bool causal) {
   if (n > 32768 / d) return false;  // LDS and registers hold no more keys
   const long rounds = ((long)slices + cus - 1) / cus, last = slices - (rounds - 1) * cus;
@@ -370,7 +380,8 @@ FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, 
   }
   if (n <= 160) return rounds == 1 ? 3 * last >= 2L * cus : rounds == 2 && 4 * last >= 3L * cus;
   if (n <= 256) return n <= 200 && rounds == 1 && 16 * last >= (n <= 184 ? 14L : 16L) * cus;
-  if (n <= 384) return whole_tiles ? rounds != 3 && rounds != 4 && 16 * last >= 15L * cus : 16 * last >= (rounds == 1 ? 14L : 15L) * cus;
+  if (n <= 384 && whole_tiles) return rounds != 3 && rounds != 4 && 16 * last >= 15L * cus;
+  if (n <= 384) return 16 * last >= (rounds == 1 ? 14L : 15L) * cus;
   return rounds > 4 || 8 * last >= (rounds == 1 ? 7L : 6L) * cus;
 }
 

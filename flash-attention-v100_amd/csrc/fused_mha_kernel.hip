@@ -528,10 +528,13 @@ __device__ __forceinline__ void static_for(F&& f) {
 // stores that share a base address; like the tile copies it is therefore invisible to the compiler's wait counts.
 template <bool SHARED, bool KEEP, int kOffset>
 __device__ __forceinline__ void store_ds(half_t* p, h8 v, IntTag<kOffset>) {
-  if constexpr (SHARED && !KEEP) asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
-  else if constexpr (SHARED) asm volatile("global_store_dwordx4 %0, %1, off offset:%2 sc1" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
-  else if constexpr (!KEEP) asm volatile("global_store_dwordx4 %0, %1, off offset:%2 nt" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
-  else asm volatile("global_store_dwordx4 %0, %1, off offset:%2" : : "v"(p), "v"(v), "n"(kOffset) : "memory");
+#define FMHA_STORE16(HINTS) \
+  asm volatile("global_store_dwordx4 %0, %1, off offset:%2" HINTS : : "v"(p), "v"(v), "n"(kOffset) : "memory")
+  if constexpr (SHARED && !KEEP) FMHA_STORE16(" sc1 nt");
+  else if constexpr (SHARED) FMHA_STORE16(" sc1");
+  else if constexpr (!KEEP) FMHA_STORE16(" nt");
+  else FMHA_STORE16("");
+#undef FMHA_STORE16
 }
 
 // Element strides of a (batch, n, head, d) tensor whose last dimension is
@@ -1024,14 +1027,14 @@ __device__ __forceinline__ void odd_slots_first() {
   if (slot & 1) __builtin_amdgcn_s_setprio(1);
 }
 
-// The last, up to 32, queries of a slice by one wave for itself, with no other wave or barrier (rule: fmha_tails_per_block).  As
-// a block of their own they take a whole place of a CU for three waves that do nothing; here two or four slices share one.  K and V
-// of 64 keys take turns in a tile of LDS that is the wave's own: K(t + 1) comes while the scores of tile t are formed from
-// registers and goes to registers, V(t) then comes while the softmax is.  Not interleaved further: at D = 128 the registers are
-// used up.  A tile takes 2,500 cycles (kernel below: 1,850 for a wave alone), of which the MFMAs take 2,048; all that counts
-// is that the block ends before the others of its round, so its waves go first wherever they could issue (a tail that is
-// still there when the others have ended: 4100 x 20 slices, D = 128, 186 us without, 170 with).  Two tiles of LDS to a wave, so that
-// copies are under way longer: nothing gained.  All sums are those of the kernel below, in the same order.
+// The last, up to 32, queries of a slice by one wave for itself, with no other wave or barrier (rule: fmha_tails_per_block).
+// As a block of their own they take a whole place of a CU for three waves that do nothing; here two or four slices share one.
+// K and V of 64 keys take turns in a tile of LDS that is the wave's own: K(t + 1) comes while the scores of tile t are formed
+// from registers and goes to registers, V(t) then comes while the softmax is.  Not interleaved further: at D = 128 the
+// registers are used up.  At D = 128 a tile takes 2,500 cycles (kernel below: 2,000), of which the MFMAs take 1,024; all that
+// counts is that the block ends before the others of its round, so its waves go first wherever they could issue (a tail that is
+// still there when the others have ended: 4100 x 20 slices, D = 128, 186 us without, 170 with).  Two tiles of LDS to a wave, so
+// that copies are under way longer: nothing gained.  All sums are those of the kernel below, in the same order.
 template <int D, bool CAUSAL>
 __device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, const half_t* __restrict__ K,
                                               const half_t* __restrict__ V, Strides qs, Strides ks, Strides vs,
@@ -3093,10 +3096,12 @@ bwd_dq_spill_blocks(const half_t* __restrict__ K, Strides ks, const half_t* __re
     char* dst = s_ring + slot * kDsTileBytes + cw * kSIPW * 1024;
     if (stream_ds) {
 #pragma unroll
-      for (int u = 0; u < kSIPW; ++u) copy16_ds<Blocks::kShared, true>(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+      for (int u = 0; u < kSIPW; ++u)
+        copy16_ds<Blocks::kShared, true>(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
     } else {
 #pragma unroll
-      for (int u = 0; u < kSIPW; ++u) copy16_ds<Blocks::kShared, false>(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
+      for (int u = 0; u < kSIPW; ++u)
+        copy16_ds<Blocks::kShared, false>(sp[(u >> 1) & 3], c_sgoff[u & 1] + u * 1024, dst + u * 1024);
     }
   };
   auto copy_k = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
@@ -3272,18 +3277,18 @@ fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t*
 
 // ---------------------------------------------------------------------------
 // The dK/dV pass that stores dS and the dQ pass over it in one launch: first all blocks of the former, then those of the
-// latter, one to a work group.  One after the other, each pass leaves CUs idle in its last round and the second starts when
-// the first has drained; here the dQ blocks of slices that are finished fill the places that the dK/dV blocks leave.  What
-// that gives, and where the passes still go one by one: fmha_ds_in_one_launch.
+// latter, one to a work group.  One after the other, each pass leaves CUs idle in its last round and the second starts when the
+// first has drained; here the dQ blocks of slices that are finished fill the places that the dK/dV blocks leave.  What that
+// gives, and where the passes still go one by one: fmha_ds_in_one_launch.
 //
-// A dQ block waits for the dS of its slice: every wave that stores some counts itself when its stores are done, and the
-// block starts when the count is whole.  dS is stored and read past the XCDs' L2s (store_ds), so that is all it takes,
-// on whatever XCD the blocks are; a release of everything written (an L2 write-back per block) takes 8 % longer.  The counts
-// of a slice have a cache line of their own and are asked for about once a microsecond: with those of 32 slices in one line
-// the work groups that ask hold up those that work (24 x 2048 x 128 causal, 111 us; a line each 89).
-// The wait ends by itself: past fmha_ds_wait_ticks, which is longer once all dK/dV blocks of the slice have started, the
-// block forms S and dP itself, as fmha_bwd_dq_kernel does, with the same bits as result.  Counting what has started costs up
-// to 0.8 us of a launch (520 x 64), so only the slices that need it do.
+// A dQ block waits for the dS of its slice: every wave that stores some counts itself when its stores are done, and the block
+// starts when the count is whole.  dS is stored and read past the XCDs' L2s (store_ds), so that is all it takes, on whatever
+// XCD the blocks are; a release of everything written (an L2 write-back per block) takes 8 % longer.  The counts of a slice
+// have a cache line of their own and are asked for about once a microsecond: with those of 32 slices in one line the work
+// groups that ask hold up those that work (24 x 2048 x 128 causal, 111 us; a line each 89).  The wait ends by itself: past
+// fmha_ds_wait_ticks, which is longer once all dK/dV blocks of the slice have started, the block forms S and dP itself, as
+// fmha_bwd_dq_kernel does, with the same bits as result.  Counting what has started costs up to 0.8 us of a launch (520 x 64),
+// so only the slices that need it do.
 // ---------------------------------------------------------------------------
 constexpr int kReadyStride = 32;  // words from one slice's counts to the next
 enum ReadyWord {
@@ -3295,9 +3300,9 @@ template <bool CAUSAL, bool KEEP>
 __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                            const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
-                           const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ,
-                           half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* dS, unsigned* ready, int np, int H, int N,
-                           int nb, int slices, unsigned ticks, float c, float scale) {
+                           const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
+                           half_t* __restrict__ dQ, half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* dS, unsigned* ready,
+                           int np, int H, int N, int nb, int slices, unsigned ticks, float c, float scale) {
   constexpr int D = 128;
   static_assert(ds_threads(1) == kKvThreads && kDqThreads == kKvThreads && kDsPanelQ == kKvBlockKeys, "one grid for all");
   constexpr int kLds = dkdv_lds<D>() > dq_lds<D>() ? dkdv_lds<D>() : dq_lds<D>();
@@ -3311,8 +3316,8 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
   const bool one_xcd = bh < (slices & ~7);  // all blocks of the slice: the dK/dV blocks have then started before this dQ block
   if (!dq) {
     if (!one_xcd && threadIdx.x == 0) count(kBlocksStarted);
-    bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false, true>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
-                                                        H, N, 0, c, scale, smem, bh, blk, counts + kWavesStored);
+    bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false, true>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS,
+                                                              np, H, N, 0, c, scale, smem, bh, blk, counts + kWavesStored);
     return;
   }
   if (threadIdx.x == 0) {
@@ -3345,19 +3350,20 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
 // A wave owns 32 keys (D = 64 past 256 rows: twice 32, blocks w and 15 - w, which under causal masking are together as heavy as
 // any other two).  It keeps their dK and dV and their rows of V, negated, in registers.  K lies in LDS whole.  The work group
 // walks the queries 32 at a time: Q, dO and O come by copies to LDS that are two tiles ahead, delta is made from them as
-// fmha_bwd_delta_kernel makes it, each wave forms S, P, dP and dS of its keys (32 x 32 MFMAs, as bwd_dkdv_block), adds to dV and dK,
-// and leaves dS in LDS; behind the next barrier the waves share out the 16 x 16 tiles of dQ of those 32 queries and add up all
-// keys in order.  So S and dP are formed once and neither dS nor partial dQ leaves the CU, each input is read once, and there is
-// one barrier for 32 queries.  All sums are in the order of the other paths, which give the same bits.
-// Bound by the LDS and by issue: at D = 64 with two blocks of keys a wave reads 24 KiB of Q, dO and K for 32 MFMAs of 32 x 32 x 16
-// and 32 KiB of K and dS for 16 of 16 x 16 x 32, which for 8 waves is 1.5 times as long as a SIMD's MFMAs take, and with two
-// waves to a SIMD the vector work on S and P hardly overlaps with another wave's MFMAs.  (dQ in front of the rest of a tile in all waves, or behind it in half of them, so that the two kinds
-// of work meet: no difference, and the first needs fewer registers.  dQ steps between those of dK: slower.)  Fragments are read
-// two to four MFMA groups ahead; one ahead costs 6 %.  512 x 192 slices, D = 64: 52.7 us, 610 TFLOP/s on the 192 CUs that have
-// work; two passes that form S and dP twice: 61.  256 x 256, D = 128: 37.4 us, 574 TFLOP/s; over dS in memory: 51.9.
-// At D = 128 without a mask 129 to 160 rows have four idle waves and one of up to 32 keys.  bwd_dkdv_block shares such keys between
-// its four pairs of waves, tile j to pair j mod 4, and adds the four sums up at the end; to have its bits the idle waves do the
-// same here.
+// fmha_bwd_delta_kernel makes it, each wave forms S, P, dP and dS of its keys (32 x 32 MFMAs, as bwd_dkdv_block), adds to dV
+// and dK, and leaves dS in LDS; behind the next barrier the waves share out the 16 x 16 tiles of dQ of those 32 queries and add
+// up all keys in order.  So S and dP are formed once and neither dS nor partial dQ leaves the CU, each input is read once, and
+// there is one barrier for 32 queries.  All sums are in the order of the other paths, which give the same bits.
+// Bound by the LDS and by issue: at D = 64 with two blocks of keys a wave reads 24 KiB of Q, dO and K for 32 MFMAs of 32 x 32 x
+// 16 and 32 KiB of K and dS for 16 of 16 x 16 x 32, which for 8 waves is 1.5 times as long as a SIMD's MFMAs take, and with two
+// waves to a SIMD the vector work on S and P hardly overlaps with another wave's MFMAs.  (dQ in front of the rest of a tile in
+// all waves, or behind it in half of them, so that the two kinds of work meet: no difference, and the first needs fewer
+// registers.  dQ steps between those of dK: slower.)  Fragments are read two to four MFMA groups ahead; one ahead costs 6 %.
+// 512 x 192 slices, D = 64: 52.7 us, 610 TFLOP/s on the 192 CUs that have work; two passes that form S and dP twice: 61.  256 x
+// 256, D = 128: 37.4 us, 574 TFLOP/s; over dS in memory: 51.9.
+// At D = 128 without a mask 129 to 160 rows have four idle waves and one of up to 32 keys.  bwd_dkdv_block shares such keys
+// between its four pairs of waves, tile j to pair j mod 4, and adds the four sums up at the end; to have its bits the idle
+// waves do the same here.
 constexpr int kSliceWaves = 8;
 constexpr int kSliceThreads = kSliceWaves * 64;
 template <int D, int KB>
@@ -3660,8 +3666,9 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
     __builtin_amdgcn_sched_barrier(0);
     {  // the products with the first 16 queries while P of the others is formed
       const unsigned a0 = ca + Geo::kTileBytes + at, a1 = a0 ^ kUpper;
-      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) { return swz_cols_at<D>(a0, a1, n / kDB, n % kDB); },
-               [&](int u, h8 f) __attribute__((always_inline)) {
+      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) {
+        return swz_cols_at<D>(a0, a1, n / kDB, n % kDB);
+      }, [&](int u, h8 f) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < NB; ++n) dv[n][u % kDB] = mfma(f, y[n][u / kDB], dv[n][u % kDB]);
         if (u == 0) p_quad(2);
@@ -3708,8 +3715,9 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
     __builtin_amdgcn_sched_barrier(0);
     {
       const unsigned a0 = ca + at, a1 = a0 ^ kUpper;
-      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) { return swz_cols_at<D>(a0, a1, n / kDB, n % kDB); },
-               [&](int u, h8 f) __attribute__((always_inline)) {
+      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) {
+        return swz_cols_at<D>(a0, a1, n / kDB, n % kDB);
+      }, [&](int u, h8 f) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < NB; ++n) dk[n][u % kDB] = mfma(f, y[n][u / kDB], dk[n][u % kDB]);
         if (u == 0) ds_half(1);
@@ -4030,8 +4038,8 @@ size_t best_workspace(int batch, int head, int n, int d, size_t room) {
 }
 
 template <int D, bool CAUSAL>
-int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsigned ticks, const void* q, const void* k, const void* v, const void* o,
-                    const void* d_o, Strides qs, Strides ks, Strides vs, Strides gs, const void* lse, float* delta,
+int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsigned ticks, const void* q, const void* k,
+                    const void* v, const void* o, const void* d_o, Strides qs, Strides ks, Strides vs, Strides gs, const void* lse, float* delta,
                     void* dq, void* dk, void* dv, int batch, int head, int n, float scale, hipStream_t stream) {
   // slices_at_once: how many slices' dS the workspace holds, 0 for the passes that need none; ticks: the most that a block may
   // wait for another's dS, fmha_ds_wait_ticks if that is less
@@ -4066,8 +4074,8 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
       const unsigned per_slice = (unsigned)(n + delta_rows(D) - 1) / delta_rows(D);
       const unsigned chain = per_slice < blocks ? per_slice : blocks, chains = (blocks + chain - 1) / chain;
       const hipError_t rc = launch(fmha_bwd_delta_kernel<D>, chain * chains, 256, stream, (const half_t*)o, (const half_t*)d_o,
-                                   gs, (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains, ready,
-                                   ready ? (unsigned)(ready_bytes(slices) / 4) : 0u);
+                                   gs, (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains,
+                                   ready, ready ? (unsigned)(ready_bytes(slices) / 4) : 0u);
       if (rc != hipSuccess) return rc;
     }
     return hipSuccess;
@@ -4221,8 +4229,8 @@ int dispatch_backward(int passes, const void* q, const fused_mha_strides* q_st, 
   const Strides qs = to_strides(q_st, head, n, d), ks = to_strides(k_st, head, n, d),
                 vs = to_strides(v_st, head, n, d), gs = to_strides(g_st, head, n, d);
 #define FMHA_BWD(DD, CC) \
-  launch_backward<DD, CC>(passes, slices_at_once, workspace_bytes, ticks, q, k, v, o, d_o, qs, ks, vs, gs, lse, delta, dq, dk, dv, batch, head, n, \
-                          scale, s)
+  launch_backward<DD, CC>(passes, slices_at_once, workspace_bytes, ticks, q, k, v, o, d_o, qs, ks, vs, gs, lse, delta, dq, dk, \
+                          dv, batch, head, n, scale, s)
   if (d == 128) return causal ? FMHA_BWD(128, true) : FMHA_BWD(128, false);
   return causal ? FMHA_BWD(64, true) : FMHA_BWD(64, false);
 #undef FMHA_BWD
@@ -4312,8 +4320,8 @@ int fmha_backward_waiting(const void* query_ptr, const void* key_ptr, const void
                           void* d_query_ptr, void* d_key_ptr, void* d_value_ptr, int batch, int head, int n, int d, float scale,
                           int causal, unsigned ticks, void* stream) {
   return dispatch_backward(kPassAll | kNotBySlice, query_ptr, nullptr, key_ptr, nullptr, value_ptr, nullptr, output_ptr,
-                           d_output_ptr, nullptr, lse_ptr, workspace, workspace_bytes, d_query_ptr, d_key_ptr, d_value_ptr, batch, head, n, n, d, scale,
-                           causal, stream, ticks);
+                           d_output_ptr, nullptr, lse_ptr, workspace, workspace_bytes, d_query_ptr, d_key_ptr, d_value_ptr,
+                           batch, head, n, n, d, scale, causal, stream, ticks);
 }
 
 int fused_mha_backward(const void* query_ptr, const void* key_ptr, const void* value_ptr, const void* output_ptr,

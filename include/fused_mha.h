@@ -97,7 +97,8 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
 #define FUSED_MHA_SPILL_MAX_BYTES ((size_t)16 << 30)
 
 /*
- * Bytes of device scratch the backward works best with for this problem size.
+ * Bytes of device scratch that the backward works best with for this problem
+ * size, but for the counts described at the end.
  * The workspace starts with delta = rowsum(d_o * o) and lse * log2(e), both
  * fp32 of shape (batch, head, n), delta first: that much
  * (fused_mha_backward_min_workspace_bytes) is always needed.  With d = 128 and
@@ -114,8 +115,9 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * gradients depend neither on the workspace nor on how many other slices the
  * call has.
  * fused_mha_backward_workspace_bytes returns
- *   - d = 64: the minimum.  The dQ pass always recomputes, which is the faster
- *     way there, and nothing else is read or written whatever the size;
+ *   - d = 64: the minimum.  No launch stores dS in memory there (the dQ pass
+ *     recomputes, the work group of a whole slice keeps it), and nothing else
+ *     is read or written whatever the size;
  *   - d = 128, dS of at most FUSED_MHA_SPILL_MAX_BYTES: room for all of it;
  *   - d = 128, more dS than that: room for rounds of enough slices to keep an
  *     MI355X busy, at most FUSED_MHA_SPILL_MAX_BYTES behind the statistics, or
@@ -129,10 +131,13 @@ int fused_mha_forward_strided(const void *query_ptr, const fused_mha_strides *qu
  * minimum is as fast for them.  The same goes for many problems of at least
  * half as many slices as the device has compute units and n <= 32768 / d, of
  * which one compute unit does a whole slice, with S and dP formed once.
- * With d = 128 and, behind room for the dS of all slices, another 128 bytes for
- * each (batch, head) slice, both passes go in one launch where that is faster
- * (many problems of up to a few blocks of 128 rows per compute unit); the
- * results are the same bits.
+ * Counts: with d = 128 and, behind room for the dS of all slices, another 128
+ * bytes for each (batch, head) slice, both passes go in one launch where that
+ * is faster (many problems of up to a few blocks of 128 rows per compute unit,
+ * by up to a quarter of the backward); the results are the same bits.
+ * fused_mha_backward_workspace_bytes does not include them: where dS is at
+ * most FUSED_MHA_SPILL_MAX_BYTES, add (size_t)batch * head * 128 to it to have
+ * that launch.  Without them the passes are launched one after the other.
  * A caller that wants to spend less passes any size from the minimum on.
  * Both functions return 0 for an invalid shape.  No counterpart in the
  * reference, which receives delta from Python (flash_attn_interface.py:43-44).
