@@ -305,12 +305,16 @@ FMHA_HOST_DEVICE unsigned fmha_ds_wait_ticks(int n, bool started) { return (500u
 // (7.4) 295, 294; 768 x 315 (7.4) 462, 456; 777 x 230 (6.3) 383, 377; 777 x 303 (8.3) 520, 512; 1000 x 265 (8.3) 666, 634; 1024
 // x 265 (8.3) 656, 638; 1500 x 110 (5.2) 589, 572; 1500 x 155 (7.3) 814, 800; 2048 x 84 (5.3) 757, 741; 2048 x 100 (6.3) 912,
 // 915; 2048 x 114 (7.1) 1017, 1020; 2048 x 130 (8.1) 1178, 1191; 4096 x 42 (5.3) 1390, 1373.  Causal: 400 x 473 (7.4) 223, 223;
-// 700 x 268 (6.3) 245, 246; 768 x 315 (7.4) 322, 317; 900 x 198 (6.2) 277, 281; 1000 x 220 (6.9) 352, 351; 1024 x 220 (6.9)
-// 353, 350.
+// 700 x 268 (6.3) 245, 246; 768 x 315 (7.4) 322, 317; 777 x 193 (5.3) 214, 210; 777 x 239 (6.5) 268, 268; 896 x 193 (5.3) 247,
+// 244; 896 x 239 (6.5) 315, 309; 900 x 129 (4.0) 184, 182; 1024 x 129 (4.0) 207, 203; but 900 x 145 (4.5) 201, 202; 900 x 169
+// (5.3) 231, 235; 960 x 161 (5.0) 231, 232; 960 x 185 (5.8) 266, 269; 1024 x 185 (5.8) 294, 296; 1024 x 220 (6.9) 353, 350.
 FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool causal) {
   const long blocks = (long)slices * ((n + 127) / 128), left = blocks % cus;
   if (n <= 768) return 2 * blocks <= 15L * cus;
-  if (causal) return n <= 1024 ? blocks <= 7L * cus : n <= 2048 ? blocks < 4L * cus : n <= 4096 && 2 * blocks < 3L * cus;
+  if (causal) {
+    if (n <= 1024) return 8 * blocks <= (n <= 896 ? 56L : 33L) * cus;
+    return n <= 2048 ? blocks < 4L * cus : n <= 4096 && 2 * blocks < 3L * cus;
+  }
   if (blocks <= cus) return n <= 2048;
   if (left == 0) return false;
   if (n <= 1024) return 4 * left <= 3L * cus && blocks <= 9L * cus;

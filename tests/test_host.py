@@ -595,6 +595,8 @@ def test_count_bytes(lib):
     assert f(1, 600, 64, 128, 0) == 0     # a work group for each slice
     assert f(16, 12, 512, 64, 0) == 0 and f(1, 0, 512, 128, 0) == 0
     assert f(1, 33000, 512, 128, 0) == 0  # dS in rounds
+    assert f(1, 239, 896, 128, 1) == 239 * 128 and f(1, 129, 1024, 128, 1) == 129 * 128
+    assert f(1, 169, 900, 128, 1) == f(1, 161, 960, 128, 1) == f(1, 185, 1024, 128, 1) == 0  # the passes one by one are faster
 
 
 def test_interleaved_blocks_are_a_bijection(tmp_path):
