@@ -352,6 +352,9 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 // backward, without it and with it: 97 x 257 37.1, 37.7; 97 x 266 37.8, 39.9; 97 x 296 39.2, 39.8; 97 x 320 39.8, 39.6; 105 x
 // 266 38.9, 40.3; 105 x 306 40.4, 40.2; 112 x 266 40.0, 40.6; 112 x 306 41.5, 40.5; 116 x 266 40.7, 40.7; 128 x 266 42.3, 41.4;
 // and 96 x 257 36.4, 33.4.
+// D = 64 without a mask, 161 to 176 rows, us of forward and backward, without it and with it: 161 x 598 63.0, 63.9; 161 x 612
+// 63.6, 65.1; 161 x 652 69.0, 66.9; 176 x 612 65.2, 65.2; 176 x 652 69.2, 67.3; 161 x 1812 166, 172; 161 x 1892 174, 174; 161 x
+// 1932 179, 177; 176 x 1812 173, 175; 176 x 1932 187, 182; 161 x 2068 190, 194; 176 x 2068 199, 200.
 // Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 27.0, 26.4; 161 x 256 27.3,
 // 27.4; 170 x 236 27.4, 26.5; 180 x 224 27.3, 27.2; 180 x 244 27.7, 27.4; 192 x 224 27.0, 27.5; 192 x 236 27.6, 27.1; 192 x 250
 // 27.7, 28.1; 193 x 224 29.3, 30.4; 193 x 250 30.5, 31.0; 200 x 230 29.9, 30.4; 200 x 240 30.3, 30.6; 200 x 256 32.0, 30.7.
@@ -380,6 +383,7 @@ FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, 
   if (!causal) {
     if (rounds == 1) return n <= 256 ? 2 * last > cus : 4 * last >= 3L * cus;
     if (n > 256 && n <= 384 && whole_tiles) return 8 * last >= (rounds < 6 ? 6L : rounds == 6 ? 5L : 1L) * cus;
+    if (n > 160 && n <= 176 && (rounds == 3 || rounds == 8 || rounds == 9)) return 5 * last >= 2L * cus;
     return rounds > 5 || rounds * last > cus;
   }
   if (n <= 160) return rounds == 1 ? 3 * last >= 2L * cus : rounds == 2 && 4 * last >= 3L * cus;

@@ -562,6 +562,7 @@ def test_backward_by_slice(tmp_path, lib):
         (128, 1, 129, 0), (128, 256, 129, 1), (128, 256, 256, 0), (128, 100, 257, 0), (128, 200, 320, 0), (128, 160, 320, 1),
         (128, 96, 257, 1), (128, 97, 320, 1), (128, 116, 266, 1), (128, 97, 257, 0), (128, 256, 342, 1), (128, 33, 514, 0), (128, 100, 640, 1), (128, 256, 514, 0), (128, 100, 1600, 0), (128, 64, 3000, 1),
         (64, 129, 129, 0), (64, 257, 192, 0), (64, 512, 192, 0), (64, 300, 448, 0), (64, 512, 600, 0), (64, 512, 1300, 0),
+        (64, 161, 652, 0), (64, 176, 652, 0), (64, 161, 1932, 0), (64, 177, 612, 0), (64, 160, 598, 0),
         (64, 264, 608, 0), (64, 352, 840, 0), (64, 384, 1216, 0), (64, 290, 1440, 0), (64, 304, 1704, 0), (64, 320, 1264, 1),
         (64, 264, 1264, 1),
         (64, 129, 171, 1), (64, 160, 448, 1), (64, 180, 224, 1), (64, 200, 256, 1), (64, 384, 256, 1),
@@ -571,6 +572,7 @@ def test_backward_by_slice(tmp_path, lib):
         (128, 97, 257, 1), (128, 97, 296, 1), (128, 105, 266, 1), (128, 112, 266, 1),
         (128, 1, 128, 0), (128, 257, 200, 0), (128, 256, 319, 0), (128, 256, 330, 1), (128, 100, 528, 0), (128, 100, 1030, 1),
         (64, 128, 256, 0), (64, 129, 128, 0), (64, 257, 176, 0), (64, 300, 384, 0), (64, 512, 590, 0), (64, 513, 256, 0),
+        (64, 161, 598, 0), (64, 161, 612, 0), (64, 161, 1812, 0), (64, 176, 1812, 0),
         (64, 300, 400, 0), (64, 384, 385, 0), (64, 290, 598, 0), (64, 290, 833, 0), (64, 320, 1076, 0), (64, 290, 1352, 0),
         (64, 304, 1544, 0), (64, 320, 224, 1), (64, 384, 224, 1), (64, 384, 752, 1), (64, 320, 1014, 1),  # whole tiles of 64 rows
         (64, 129, 160, 1), (64, 201, 256, 1), (64, 200, 480, 1), (64, 300, 480, 1), (64, 512, 208, 1), (64, 512, 640, 1),
