@@ -5,9 +5,32 @@
 
 #if defined(__HIPCC__)
 #define FMHA_HOST_DEVICE __host__ __device__ inline
+#define FMHA_HOST __host__
 #else
 #define FMHA_HOST_DEVICE inline
+#define FMHA_HOST
 #endif
+
+// A divisor that is the same for a whole launch.  A kernel divides by it with a multiplication, an addition and a shift; a
+// division by an int is a chain of some 40 instructions, 250 cycles in which the work group has nothing else to do, and to
+// find its block and its rows takes three to five of them.  Where a work group spends a few thousand cycles on its tiles that
+// counts: figures at FmhaOrder.  Good for 0 <= n < 2^31: with mul = floor(2^32 (2^shift - d) / d) + 1, 2^32 + mul exceeds 2^(32 +
+// shift) / d by at most 1, hence the quotient n (2^32 + mul) / 2^(32 + shift) exceeds n / d by less than 1 / d
+// (Granlund and Montgomery, Division by Invariant Integers using Multiplication, 1994).
+struct FmhaDivisor {
+  int d;
+  unsigned mul, shift;
+  FmhaDivisor() = default;
+  FMHA_HOST FmhaDivisor(int by) : d(by), shift(0) {
+    while ((1ull << shift) < (unsigned long long)by) ++shift;
+    mul = (unsigned)((((1ull << shift) - (unsigned long long)by) << 32) / (unsigned long long)by + 1);
+  }
+  FMHA_HOST_DEVICE operator int() const { return d; }
+};
+FMHA_HOST_DEVICE int operator/(int n, const FmhaDivisor& by) {
+  const unsigned high = (unsigned)(((unsigned long long)(unsigned)n * by.mul) >> 32);
+  return (int)((high + (unsigned)n) >> by.shift);
+}
 
 // Work-group id -> (batch*head slice, block inside the slice).  Consecutive
 // work-group ids go round-robin over the 8 XCDs, each with a private L2; the
@@ -26,17 +49,16 @@
 #define FMHA_SLICES_IN_FLIGHT 2
 #endif
 constexpr int kSlicesInFlight = FMHA_SLICES_IN_FLIGHT;
-FMHA_HOST_DEVICE void fmha_slice_and_block(int lin, int slices, int blocks_per_slice, int& slice,
-                                                            int& blk) {
+template <typename Int>  // int or FmhaDivisor
+FMHA_HOST_DEVICE void fmha_slice_and_block(int lin, int slices, const Int& blocks_per_slice, int& slice, int& blk) {
   const int q = slices >> 3, r = slices & 7;
   const int main_blocks = 8 * q * blocks_per_slice;
   if (lin < main_blocks) {
     const int xcd = lin & 7, slot = lin >> 3;  // slot: 0 .. q * blocks_per_slice - 1 inside the XCD
-    const int group_blocks = kSlicesInFlight * blocks_per_slice;
-    const int group = slot / group_blocks, within = slot - group * group_blocks;
+    const int group = slot / kSlicesInFlight / blocks_per_slice, within = slot - group * (kSlicesInFlight * blocks_per_slice);
     const int first = group * kSlicesInFlight;
     const int g = (q - first < kSlicesInFlight ? q - first : kSlicesInFlight);  // slices in this group
-    blk = within / g;
+    blk = g == kSlicesInFlight ? within / kSlicesInFlight : kSlicesInFlight == 2 ? within : within / g;
     slice = xcd * q + first + (within - blk * g);
   } else {
     const int rem = lin - main_blocks, n_rem = r * blocks_per_slice;
@@ -139,32 +161,44 @@ FMHA_HOST_DEVICE bool fmha_wide_mfmas(long key_blocks, int cus, bool causal) {  
 // Otherwise (all blocks weigh the same) the order is fmha_slice_and_block's, except that with short_last the last block
 // of every slice, which has fewer rows, comes at the end of the launch.
 constexpr int kScheduledSlices = 8;
-FMHA_HOST_DEVICE void fmha_scheduled_block(int lin, int slices, int blocks_per_slice, bool heavy_first, bool short_last,
-                                           int& slice, int& blk) {
+// `run`: the blocks of a slice that go in order (not its short last one); `last_level`: fmha_last_level.
+template <typename Int>  // int or FmhaDivisor
+FMHA_HOST_DEVICE void fmha_ordered_block(int lin, int slices, const Int& run, const Int& last_level, bool heavy_first,
+                                         bool short_last, int& slice, int& blk) {
   if (!heavy_first) {
-    const int full = blocks_per_slice - 1;
-    if (!short_last) {
-      fmha_slice_and_block(lin, slices, blocks_per_slice, slice, blk);
-    } else if (lin < slices * full) {
-      fmha_slice_and_block(lin, slices, full, slice, blk);
+    if (!short_last || lin < slices * run) {
+      fmha_slice_and_block(lin, slices, run, slice, blk);
     } else {
-      slice = lin - slices * full;
-      blk = full;
+      slice = lin - slices * run;
+      blk = run;
     }
     return;
   }
-  const int q = slices >> 3, r = slices & 7;
+  const int q = slices >> 3;
   const int groups = q < kScheduledSlices ? 1 : q / kScheduledSlices;
-  int group = lin / (8 * kScheduledSlices * blocks_per_slice);
+  int group = lin / (8 * kScheduledSlices) / run;
   if (group > groups - 1) group = groups - 1;
   const int first = group * kScheduledSlices;
   const bool last = group == groups - 1;
   const int count = last ? q - first : kScheduledSlices;  // slices per XCD in this group
-  const int level = 8 * count + (last ? r : 0);           // blocks of one index in this group
-  const int idx = lin - 8 * first * blocks_per_slice;
-  blk = idx / level;
+  const int level = last ? (int)last_level : 8 * kScheduledSlices;  // blocks of one index in this group
+  const int idx = lin - 8 * first * run;
+  blk = last ? idx / last_level : idx / (8 * kScheduledSlices);
   const int p = idx - blk * level;
   slice = (p >> 3) < count ? (lin & 7) * q + first + (p >> 3) : 8 * q + (p - 8 * count);
+}
+// Blocks of one index in the last group, which has the slices % 8 too.
+FMHA_HOST_DEVICE int fmha_last_level(int slices) {
+  const int q = slices >> 3, groups = q < kScheduledSlices ? 1 : q / kScheduledSlices;
+  return slices - 8 * kScheduledSlices * (groups - 1);
+}
+FMHA_HOST_DEVICE int fmha_blocks_in_order(int blocks_per_slice, bool heavy_first, bool short_last) {
+  return !heavy_first && short_last && blocks_per_slice > 1 ? blocks_per_slice - 1 : blocks_per_slice;
+}
+FMHA_HOST_DEVICE void fmha_scheduled_block(int lin, int slices, int blocks_per_slice, bool heavy_first, bool short_last,
+                                           int& slice, int& blk) {
+  const int run = fmha_blocks_in_order(blocks_per_slice, heavy_first, short_last);
+  fmha_ordered_block(lin, slices, run, fmha_last_level(slices), heavy_first, run < blocks_per_slice, slice, blk);
 }
 
 // The same launches, two blocks to a CU: work groups w and w + kCus start on the same CU, so with the second kCus taken in
@@ -237,22 +271,24 @@ FMHA_HOST_DEVICE int fmha_tails_per_block(int d, int n, int slices, int cus, boo
 
 // A launch of two passes with `nb` blocks each per slice: the blocks of both in turn, ordered as one pass's are (heaviest of
 // both first, or the short last ones of both at the end).
-FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heavy_first, bool short_last, int& slice, int& blk,
-                                          bool& second_pass) {
-  const int full = 2 * (nb - 1);
+// `run`, last_level: as in fmha_ordered_block, of 2 * nb blocks, the last two short ones.
+template <typename Int>
+FMHA_HOST_DEVICE void fmha_two_pass_ordered_block(int lin, int slices, const Int& run, const Int& last_level, bool heavy_first,
+                                                  bool short_last, int& slice, int& blk, bool& second_pass) {
   int v;
-  if (heavy_first) {
-    fmha_scheduled_block(lin, slices, 2 * nb, true, false, slice, v);
-  } else if (!short_last) {
-    fmha_slice_and_block(lin, slices, 2 * nb, slice, v);
-  } else if (lin < slices * full) {
-    fmha_slice_and_block(lin, slices, full, slice, v);
+  if (heavy_first || !short_last || lin < slices * run) {
+    fmha_ordered_block(lin, slices, run, last_level, heavy_first, false, slice, v);
   } else {
-    slice = (lin - slices * full) >> 1;
-    v = full + ((lin - slices * full) & 1);
+    slice = (lin - slices * run) >> 1;
+    v = run + ((lin - slices * run) & 1);
   }
   blk = v >> 1;
   second_pass = v & 1;
+}
+FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heavy_first, bool short_last, int& slice, int& blk,
+                                          bool& second_pass) {
+  const int run = 2 * fmha_blocks_in_order(nb, heavy_first, short_last);
+  fmha_two_pass_ordered_block(lin, slices, run, fmha_last_level(slices), heavy_first, run < 2 * nb, slice, blk, second_pass);
 }
 
 // A launch of all blocks of the dK/dV pass and then all of the dQ pass over the dS that it stores, nb each per slice, either in
@@ -260,15 +296,35 @@ FMHA_HOST_DEVICE void fmha_two_pass_block(int lin, int slices, int nb, bool heav
 // dQ blocks, and they wait for whole slices).  The second part begins at a multiple of 8, so that a slice stays on its XCD; the
 // up to 7 work groups before that have no block.
 FMHA_HOST_DEVICE int fmha_ds_launch_blocks(int slices, int nb) { return ((slices * nb + 7) & ~7) + slices * nb; }
-FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool heavy_first, int& slice, int& blk,
-                                           bool& second_pass) {
+template <typename Int>
+FMHA_HOST_DEVICE bool fmha_ds_launch_ordered_block(int lin, int slices, const Int& nb, const Int& last_level, bool heavy_first,
+                                                   int& slice, int& blk, bool& second_pass) {
   const int blocks = slices * nb, second = (blocks + 7) & ~7;
   second_pass = lin >= second;
   if (second_pass) lin -= second;
   if (lin >= blocks) return false;
-  fmha_scheduled_block(lin, slices, nb, heavy_first, false, slice, blk);
+  fmha_ordered_block(lin, slices, nb, last_level, heavy_first, false, slice, blk);
   return true;
 }
+FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool heavy_first, int& slice, int& blk,
+                                           bool& second_pass) {
+  return fmha_ds_launch_ordered_block(lin, slices, nb, fmha_last_level(slices), heavy_first, slice, blk, second_pass);
+}
+
+// What the kernels take of a launch whose blocks are numbered in one of the orders above.
+// us of forward and backward kernels with the divisions of ints, then with these, in graphs of 20 calls, N x slices: D = 64
+// 77 x 8 causal 5.61, 5.51 and 6.78, 6.63; 300 x 80 causal 7.52, 7.44 and 13.09, 12.95; 256 x 256 9.67, 9.62 and 21.8, 21.5; 3000
+// x 20 causal 33.9 both and 98.1, 97.1; D = 128 200 x 48 causal 9.41, 9.28 and 14.71, 14.51; 2048 x 80 causal 93.9 both and 290.6,
+// 287.7; 1031 x 60 42.0, 42.3 and 118.8, 117.8.
+struct FmhaOrder {
+  FmhaDivisor run, last_level;
+  int slices;
+  bool short_last;  // the short last blocks come at the end
+  FmhaOrder() = default;
+  FMHA_HOST FmhaOrder(int slices_, int blocks_per_slice, bool heavy_first, bool short_last_, int passes = 1)
+      : run(passes * fmha_blocks_in_order(blocks_per_slice, heavy_first, short_last_)), last_level(fmha_last_level(slices_)),
+        slices(slices_), short_last((int)run < passes * blocks_per_slice) {}
+};
 
 // How long a dQ block of that launch waits for the dS of its slice before it forms S and dP itself, in ticks of 10 ns.  Blocks
 // are handed out in order inside an XCD only, and a slice that no XCD has for itself (slices % 8) has blocks on several.  With
@@ -485,8 +541,9 @@ FMHA_HOST_DEVICE bool fmha_ds_used_once(unsigned long ds_bytes, unsigned long to
 // Row statistics: blocks of consecutive rows, numbered through all slices, taken from `chains` runs of `chain` blocks by
 // turns.  With a run about as long as a slice, work groups that follow each other read the same positions of different heads,
 // which lie side by side.  A launch has chain * chains work groups, those past the last block have nothing to do.
-FMHA_HOST_DEVICE unsigned fmha_interleaved_block(unsigned lin, unsigned chain, unsigned chains) {
-  const unsigned step = lin / chains;
+template <typename Int>  // int or FmhaDivisor
+FMHA_HOST_DEVICE int fmha_interleaved_block(int lin, int chain, const Int& chains) {
+  const int step = lin / chains;
   return (lin - step * chains) * chain + step;
 }
 #endif  // FMHA_BLOCK_MAP_H_

@@ -172,10 +172,6 @@ __device__ __forceinline__ void store_resident(half_t* __restrict__ base, long r
   }
 }
 
-__device__ __forceinline__ void slice_and_block(int blocks_per_slice, int& slice, int& blk) {
-  fmha_slice_and_block(blockIdx.x, gridDim.x / blocks_per_slice, blocks_per_slice, slice, blk);
-}
-
 // Blocks of a persistent work group (schedule: block_map.h).
 struct PersistentBlocks {
   int total;
@@ -641,8 +637,8 @@ constexpr int kRing = 3;
 template <int D, bool CAUSAL>
 __global__ void __launch_bounds__(kFwdThreads, 1)
 fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
-                int nmb, int total, float c, int negate_q) {
+                Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, FmhaDivisor H, int N,
+                FmhaDivisor nmb, int slices, float c, int negate_q) {
   using G = Geom16<D>;
   using T = SwzTile<D>;
   constexpr int kIPW = T::kInstrs / kFwdWaves;  // copy instructions per wave per tile
@@ -659,8 +655,8 @@ fmha_fwd_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, cons
   char* const stage = smem + 2 * kRing * T::kBytes + wave * Stage16<64>::kBytes;
   const int rs = H * D;  // O is dense
   const int nt_all = (N + kTile - 1) / kTile;
+  const int total = slices * nmb;
   const PersistentBlocks pb{total};
-  const int slices = total / nmb;
 
   struct Block {
     const half_t *q, *k, *v;  // first row of the (batch, head) slice
@@ -1038,7 +1034,7 @@ __device__ __forceinline__ void odd_slots_first() {
 template <int D, bool CAUSAL>
 __device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, const half_t* __restrict__ K,
                                               const half_t* __restrict__ V, Strides qs, Strides ks, Strides vs,
-                                              half_t* __restrict__ O, float* __restrict__ LSE, int H, int N, int bh, float c,
+                                              half_t* __restrict__ O, float* __restrict__ LSE, FmhaDivisor H, int N, int bh, float c,
                                               int negate_q, char* ring) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
@@ -1193,8 +1189,8 @@ __device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, cons
 template <int D, bool CAUSAL, bool ODD_FIRST, bool TAIL>
 __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
-                     Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, int H, int N,
-                     int nmb, int slices, int tails_per_block, float c, int negate_q) {
+                     Strides qs, Strides ks, Strides vs, half_t* __restrict__ O, float* __restrict__ LSE, FmhaDivisor H, int N,
+                     FmhaOrder order, int nb, int tails, int tails_per_block, float c, int negate_q) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
   constexpr int kDB = G::kDBlocks;
@@ -1214,19 +1210,16 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   };
   int bh, mb;
   const int lin = CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  const int nb = nmb - (TAIL ? 1 : 0);
   if constexpr (TAIL) {
-    const int tails = fmha_tail_blocks(slices, tails_per_block);
     if (lin < tails) {
       bh = fmha_tail_slice(lin, wave, tails, tails_per_block);
-      if (wave < tails_per_block && bh < slices)
+      if (wave < tails_per_block && bh < order.slices)
         fwd_tail_rows<D, CAUSAL>(Q, K, V, qs, ks, vs, O, LSE, H, N, bh, c, negate_q, smem + wave * T::kBytes);
       return;
     }
-    fmha_scheduled_block(lin - tails, slices, nb, CAUSAL, false, bh, mb);
-  } else {
-    fmha_scheduled_block(lin, slices, nb, CAUSAL, N % kPipeBlockQ != 0, bh, mb);
   }
+  fmha_ordered_block(TAIL ? lin - tails : lin, order.slices, order.run, order.last_level, CAUSAL,
+                     !TAIL && order.short_last, bh, mb);
   const int mblk = CAUSAL ? nb - 1 - mb : mb;  // heavy blocks first
   const int b = bh / H, h = bh - b * H;
   const int rs = H * D;  // O is dense
@@ -1558,21 +1551,21 @@ constexpr int delta_rows(int d) { return 256 * 8 / d; }  // of a block
 template <int D>
 __global__ void __launch_bounds__(256)
 fmha_bwd_delta_kernel(const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides gs,
-                      const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, unsigned H,
-                      unsigned N, unsigned first, unsigned end, unsigned chain, unsigned chains, unsigned* __restrict__ clear,
+                      const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, FmhaDivisor H,
+                      FmhaDivisor N, int first, int end, int chain, FmhaDivisor chains, unsigned* __restrict__ clear,
                       unsigned words) {
-  constexpr unsigned kLanesPerRow = D / 8;
+  constexpr int kLanesPerRow = D / 8;
   for (unsigned at = blockIdx.x * 256 + threadIdx.x; at < words; at += gridDim.x * 256) clear[at] = 0;  // for a later kernel
-  const unsigned row0 = first + fmha_interleaved_block(blockIdx.x, chain, chains) * delta_rows(D);  // rows first .. end - 1
-  const unsigned slice0 = row0 / N, b0 = slice0 / H;
-  const unsigned in_block = threadIdx.x / kLanesPerRow, row = row0 + in_block, c = threadIdx.x % kLanesPerRow;
-  unsigned n = row0 - slice0 * N + in_block, h = slice0 - b0 * H, b = b0;
+  const int row0 = first + fmha_interleaved_block((int)blockIdx.x, chain, chains) * delta_rows(D);  // rows first .. end - 1
+  const int slice0 = row0 / N, b0 = slice0 / H;
+  const int in_block = threadIdx.x / kLanesPerRow, row = row0 + in_block, c = threadIdx.x % kLanesPerRow;
+  int n = row0 - slice0 * N + in_block, h = slice0 - b0 * H, b = b0;
   if (n >= N) {  // past the end of the slice that the block starts in
-    const unsigned later = n / N;
+    const int later = n / N;
     n -= later * N;
     h += later;
     if (h >= H) {
-      const unsigned batches = h / H;
+      const int batches = h / H;
       b += batches;
       h -= batches * H;
     }
@@ -1624,7 +1617,7 @@ template <int D, bool CAUSAL, bool STATS>
 __device__ __forceinline__ void
 bwd_dq_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
              const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
-             const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ, int H,
+             const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ, FmhaDivisor H,
              int N, float c, float scale, char* smem, int bh, int mblk) {
   using G = TileGeom<D>;
   using T = SwzTile<D>;
@@ -1863,10 +1856,10 @@ __global__ void __launch_bounds__(kDqThreads, 1)
 fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                    const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
                    Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
-                   half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+                   half_t* __restrict__ dQ, FmhaDivisor H, int N, FmhaDivisor nmb, int slices, float c, float scale) {
   __shared__ __attribute__((aligned(1024))) char smem[dq_lds<D>()];
   int bh, mb;
-  slice_and_block(nmb, bh, mb);
+  fmha_slice_and_block(blockIdx.x, slices, nmb, bh, mb);
   bwd_dq_block<D, CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
                                  CAUSAL ? nmb - 1 - mb : mb);  // heavy blocks first
 }
@@ -1894,7 +1887,7 @@ __device__ __forceinline__ void
 bwd_dq_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                   const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
                   Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
-                  half_t* __restrict__ dQ, int H, int N, float c, float scale, char* smem, int bh, int mblk) {
+                  half_t* __restrict__ dQ, FmhaDivisor H, int N, float c, float scale, char* smem, int bh, int mblk) {
   constexpr int D = 64;
   using G = TileGeom<D>;
   using T = SwzTile<D>;
@@ -2116,12 +2109,12 @@ __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_bwd_dq_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                         const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
                         Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
-                        half_t* __restrict__ dQ, int H, int N, int nmb, float c, float scale) {
+                        half_t* __restrict__ dQ, FmhaDivisor H, int N, FmhaOrder order, int nmb, float c, float scale) {
   __shared__ __attribute__((aligned(1024))) char smem[kDqPipeLds];
   if (ODD_FIRST) odd_slots_first();
   int bh, mb;
-  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nmb, nmb, CAUSAL,
-                       N % kPipeBlockQ != 0, bh, mb);
+  fmha_ordered_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, order.slices, order.run, order.last_level,
+                     CAUSAL, order.short_last, bh, mb);
   bwd_dq_pipe_block<CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
                                    CAUSAL ? nmb - 1 - mb : mb);  // heavy blocks first
 }
@@ -2178,7 +2171,7 @@ __device__ __forceinline__ void
 bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                const float* __restrict__ LSE, const float* __restrict__ delta, const float* __restrict__ lse2,
-               half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N, int slice0,
+               half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, FmhaDivisor H, int N, int slice0,
                float c, float scale, char* smem, int bh, int nblk, unsigned* stored = nullptr) {
   using G = TileGeom<D>;
   using G16 = Geom16<D>;
@@ -2600,12 +2593,12 @@ __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_dkdv_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                      const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                      const float* __restrict__ delta, const float* __restrict__ lse2,
-                     half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, int H, int N,
-                     int nnb, int slice0, float c, float scale) {
+                     half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* __restrict__ dS, int np, FmhaDivisor H, int N,
+                     FmhaOrder order, int slice0, float c, float scale) {
   __shared__ __attribute__((aligned(1024))) char smem[dkdv_lds<D>()];
   int bh, nblk;
   // causal: low key blocks are the heavy ones and come first
-  fmha_scheduled_block(blockIdx.x, gridDim.x / nnb, nnb, CAUSAL, N % kKvBlockKeys != 0, bh, nblk);
+  fmha_ordered_block(blockIdx.x, order.slices, order.run, order.last_level, CAUSAL, order.short_last, bh, nblk);
   bwd_dkdv_block<D, CAUSAL, SPILL, KEEP, WIDE, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS, np,
                                                       H, N, slice0, c, scale, smem, bh, nblk);
 }
@@ -2620,13 +2613,14 @@ __global__ void __launch_bounds__(kKvThreads, 1)
 fmha_bwd_both_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                      const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                      const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2, half_t* __restrict__ dQ,
-                     half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, int nb, float c, float scale) {
+                     half_t* __restrict__ dK, half_t* __restrict__ dV, FmhaDivisor H, int N, FmhaOrder order, int nb, float c,
+                     float scale) {
   constexpr int D = 128;
   constexpr int kLds = dkdv_lds<D>() > dq_lds<D>() ? dkdv_lds<D>() : dq_lds<D>();
   __shared__ __attribute__((aligned(1024))) char smem[kLds];
   int bh, blk;
   bool dq;
-  fmha_two_pass_block(blockIdx.x, gridDim.x / (2 * nb), nb, CAUSAL, N % kKvBlockKeys != 0, bh, blk, dq);
+  fmha_two_pass_ordered_block(blockIdx.x, order.slices, order.run, order.last_level, CAUSAL, order.short_last, bh, blk, dq);
   if (dq)
     bwd_dq_block<D, CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
                                    CAUSAL ? nb - 1 - blk : blk);
@@ -2648,7 +2642,7 @@ __device__ __forceinline__ void
 bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                     const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                     const float* __restrict__ LSE, const float* __restrict__ delta, const float* __restrict__ lse2,
-                    half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, float c, float scale, char* smem, int bh,
+                    half_t* __restrict__ dK, half_t* __restrict__ dV, FmhaDivisor H, int N, float c, float scale, char* smem, int bh,
                     int nblk) {
   constexpr int D = 64;
   using G = TileGeom<D>;
@@ -2892,12 +2886,12 @@ __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_bwd_dkdv_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                           const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                           const float* __restrict__ delta, const float* __restrict__ lse2, half_t* __restrict__ dK,
-                          half_t* __restrict__ dV, int H, int N, int nnb, float c, float scale) {
+                          half_t* __restrict__ dV, FmhaDivisor H, int N, FmhaOrder order, float c, float scale) {
   __shared__ __attribute__((aligned(1024))) char smem[kDkDvPipeLds];
   if (ODD_FIRST) odd_slots_first();
   int bh, nblk;  // causal: low key blocks are the heavy ones and come first
-  fmha_scheduled_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / nnb, nnb, CAUSAL,
-                       N % kPipeBlockKeys != 0, bh, nblk);
+  fmha_ordered_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, order.slices, order.run, order.last_level,
+                     CAUSAL, order.short_last, bh, nblk);
   bwd_dkdv_pipe_block<CAUSAL, false>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, H, N, c, scale, smem,
                                      bh, nblk);
 }
@@ -2912,14 +2906,14 @@ __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_bwd_both_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                           const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs,
                           Strides gs, const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
-                          half_t* __restrict__ dQ, half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, int nb, float c,
-                          float scale) {
+                          half_t* __restrict__ dQ, half_t* __restrict__ dK, half_t* __restrict__ dV, FmhaDivisor H, int N,
+                          FmhaOrder order, int nb, float c, float scale) {
   constexpr int kLds = kDkDvPipeLds > kDqPipeLds ? kDkDvPipeLds : kDqPipeLds;
   __shared__ __attribute__((aligned(1024))) char smem[kLds];
   int bh, blk;
   bool dq;
-  fmha_two_pass_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, gridDim.x / (2 * nb), nb, CAUSAL,
-                      N % kPipeBlockQ != 0, bh, blk, dq);
+  fmha_two_pass_ordered_block(CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x, order.slices, order.run,
+                              order.last_level, CAUSAL, order.short_last, bh, blk, dq);
   if (dq)
     bwd_dq_pipe_block<CAUSAL, STATS>(Q, K, V, O, dO, qs, ks, vs, gs, LSE, delta, lse2, dQ, H, N, c, scale, smem, bh,
                                     CAUSAL ? nb - 1 - blk : blk);
@@ -2977,12 +2971,13 @@ __device__ __forceinline__ const half_t* wave_uniform(const half_t* p) {
 template <bool CAUSAL>
 struct DsBlocks {
   static constexpr bool kShared = false;  // a launch before this one has stored dS
-  int total, nqb;
+  const FmhaOrder& order;
+  int total;
   __device__ __forceinline__ int next_round(int r) const { return PersistentBlocks{total}.next_round(r); }
   __device__ __forceinline__ void locate(int round, int& bh, int& mb) const {
-    const int lin = round >= 0 ? PersistentBlocks{total}.lin(round) : 0, slices = total / nqb;
-    if ((int)gridDim.x == total) fmha_scheduled_block(lin, slices, nqb, CAUSAL, false, bh, mb);
-    else fmha_slice_and_block(lin, slices, nqb, bh, mb);
+    const int lin = round >= 0 ? PersistentBlocks{total}.lin(round) : 0;
+    if ((int)gridDim.x == total) fmha_ordered_block(lin, order.slices, order.run, order.last_level, CAUSAL, false, bh, mb);
+    else fmha_slice_and_block(lin, order.slices, order.run, bh, mb);
   }
 };
 // One block that is known already.
@@ -2998,7 +2993,7 @@ constexpr int ds_lds() { return kDsRingS * kDsPanels * kDsPanelTileBytes + kDsRi
 template <int D, bool CAUSAL, int kDsPanels, bool WIDE, typename Blocks>
 __device__ __forceinline__ void
 bwd_dq_spill_blocks(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
-                    half_t* __restrict__ dQ, int H, int N, int nqb, int slice0, int stream_ds, float scale, char* smem,
+                    half_t* __restrict__ dQ, FmhaDivisor H, int N, int nqb, int slice0, int stream_ds, float scale, char* smem,
                     const Blocks blocks) {
   using T = SwzTile<D>;             // K tile: 64 keys x D features
   constexpr int kKIPW = T::kInstrs / 2;              // K copies per K-copying wave and tile
@@ -3268,11 +3263,11 @@ bwd_dq_spill_blocks(const half_t* __restrict__ K, Strides ks, const half_t* __re
 template <int D, bool CAUSAL, int kDsPanels, bool WIDE>
 __global__ void __launch_bounds__(ds_threads(kDsPanels), 1)
 fmha_bwd_dq_spill_kernel(const half_t* __restrict__ K, Strides ks, const half_t* __restrict__ dS, int np,
-                         half_t* __restrict__ dQ, int H, int N, int nqb, int total, int slice0,
-                         int stream_ds, float scale) {
+                         half_t* __restrict__ dQ, FmhaDivisor H, int N, FmhaOrder order, int slice0, int stream_ds,
+                         float scale) {
   __shared__ __attribute__((aligned(1024))) char smem[ds_lds<D, kDsPanels>()];
-  bwd_dq_spill_blocks<D, CAUSAL, kDsPanels, WIDE>(K, ks, dS, np, dQ, H, N, nqb, slice0, stream_ds, scale, smem,
-                                                  DsBlocks<CAUSAL>{total, nqb});
+  bwd_dq_spill_blocks<D, CAUSAL, kDsPanels, WIDE>(K, ks, dS, np, dQ, H, N, order.run, slice0, stream_ds, scale, smem,
+                                                  DsBlocks<CAUSAL>{order, order.slices * order.run});
 }
 
 // ---------------------------------------------------------------------------
@@ -3302,7 +3297,7 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
                            const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                            const float* __restrict__ LSE, float* __restrict__ delta, float* __restrict__ lse2,
                            half_t* __restrict__ dQ, half_t* __restrict__ dK, half_t* __restrict__ dV, half_t* dS, unsigned* ready,
-                           int np, int H, int N, int nb, int slices, unsigned ticks, float c, float scale) {
+                           int np, FmhaDivisor H, int N, FmhaOrder order, unsigned ticks, float c, float scale) {
   constexpr int D = 128;
   static_assert(ds_threads(1) == kKvThreads && kDqThreads == kKvThreads && kDsPanelQ == kKvBlockKeys, "one grid for all");
   constexpr int kLds = dkdv_lds<D>() > dq_lds<D>() ? dkdv_lds<D>() : dq_lds<D>();
@@ -3310,10 +3305,11 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
   __shared__ __attribute__((aligned(1024))) char smem[kLds];
   int bh, blk;
   bool dq;
-  if (!fmha_ds_launch_block(blockIdx.x, slices, nb, CAUSAL, bh, blk, dq)) return;
+  const int nb = order.run;
+  if (!fmha_ds_launch_ordered_block(blockIdx.x, order.slices, order.run, order.last_level, CAUSAL, bh, blk, dq)) return;
   unsigned* const counts = ready + (long)bh * kReadyStride;
   auto count = [&](int word) { __hip_atomic_fetch_add(counts + word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  const bool one_xcd = bh < (slices & ~7);  // all blocks of the slice: the dK/dV blocks have then started before this dQ block
+  const bool one_xcd = bh < (order.slices & ~7);  // all blocks of the slice: the dK/dV blocks have then started before this dQ block
   if (!dq) {
     if (!one_xcd && threadIdx.x == 0) count(kBlocksStarted);
     bwd_dkdv_block<D, CAUSAL, true, KEEP, false, false, true>(Q, K, V, nullptr, dO, qs, ks, vs, gs, nullptr, delta, lse2, dK, dV, dS,
@@ -3382,7 +3378,7 @@ __global__ void __launch_bounds__(kSliceThreads, 1)
 fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
                       const half_t* __restrict__ O, const half_t* __restrict__ dO, Strides qs, Strides ks, Strides vs, Strides gs,
                       const float* __restrict__ LSE, float* __restrict__ Delta, float* __restrict__ LSE2, half_t* __restrict__ dQ,
-                      half_t* __restrict__ dK, half_t* __restrict__ dV, int H, int N, float c, float scale) {
+                      half_t* __restrict__ dK, half_t* __restrict__ dV, FmhaDivisor H, int N, float c, float scale) {
   using Geo = SliceGeom<D, KB>;
   using T = SwzTile<D>;
   constexpr int kKS = TileGeom<D>::kKSteps, kDB = TileGeom<D>::kDBlocks;
@@ -3944,19 +3940,21 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
     if (fmha_persistent_forward_pays(batch * head, n, cus, CAUSAL)) {
       const hipError_t rc = launch(fmha_fwd_kernel<D, CAUSAL>, persistent_grid(total), kFwdThreads, stream,
                                    (const half_t*)q, (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o,
-                                   (float*)lse, head, n, nmb, total, c, negate);
+                                   (float*)lse, head, n, nmb, batch * head, c, negate);
       return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
     }
   }
   const int nmb = (n + kPipeBlockQ - 1) / kPipeBlockQ, total = nmb * batch * head;
   const int slices = batch * head;
-  int tails_per_block = 0;
+  int tails_per_block = 0, tails = 0, nb = nmb;  // nb: blocks of a slice beside the one with the tail
   auto kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, false>;
   unsigned blocks = total;
   static_assert(kPipeBlockQ == 128 && kResident == 32, "as fmha_tails_per_block has it");
   if (short_tail) tails_per_block = fmha_tails_per_block(D, n, slices, cus, CAUSAL);
   if (tails_per_block) {
-    blocks = fmha_tail_blocks(slices, tails_per_block) + slices * (nmb - 1);
+    tails = fmha_tail_blocks(slices, tails_per_block);
+    nb = nmb - 1;
+    blocks = tails + slices * nb;
     kernel = fmha_fwd_pipe_kernel<D, CAUSAL, false, true>;
   }
   if constexpr (!CAUSAL) {
@@ -3964,8 +3962,9 @@ int launch_forward(const void* q, const void* k, const void* v, Strides qs, Stri
       kernel = tails_per_block ? fmha_fwd_pipe_kernel<D, CAUSAL, true, true> : fmha_fwd_pipe_kernel<D, CAUSAL, true, false>;
   }
   const hipError_t rc = launch(kernel, blocks, kPipeThreads, stream, (const half_t*)q,
-                               (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n, nmb, slices,
-                               tails_per_block, c, negate);
+                               (const half_t*)k, (const half_t*)v, qs, ks, vs, (half_t*)o, (float*)lse, head, n,
+                               FmhaOrder(slices, nb, CAUSAL, !tails && n % kPipeBlockQ != 0), nb, tails, tails_per_block, c,
+                               negate);
   return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
 }
 
@@ -4074,7 +4073,7 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
       const unsigned per_slice = (unsigned)(n + delta_rows(D) - 1) / delta_rows(D);
       const unsigned chain = per_slice < blocks ? per_slice : blocks, chains = (blocks + chain - 1) / chain;
       const hipError_t rc = launch(fmha_bwd_delta_kernel<D>, chain * chains, 256, stream, (const half_t*)o, (const half_t*)d_o,
-                                   gs, (const float*)lse, delta, lse2, (unsigned)head, (unsigned)n, first, end, chain, chains,
+                                   gs, (const float*)lse, delta, lse2, head, n, (int)first, (int)end, (int)chain, (int)chains,
                                    ready, ready ? (unsigned)(ready_bytes(slices) / 4) : 0u);
       if (rc != hipSuccess) return rc;
     }
@@ -4095,7 +4094,7 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
     auto both = [&](auto kernel, int threads) {
       return launch(kernel, 2u * nb * slices, threads, stream, (const half_t*)q, (const half_t*)k, (const half_t*)v,
                     (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2, (half_t*)dq, (half_t*)dk,
-                    (half_t*)dv, head, n, nb, c, scale);
+                    (half_t*)dv, head, n, FmhaOrder(slices, nb, CAUSAL, n % 128 != 0, 2), nb, c, scale);
     };
     hipError_t rc;
     if constexpr (D == 64) {
@@ -4122,7 +4121,7 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
         if (half_round_left((long)nmb * batch * head, n, 3)) kernel = pick(IntTag<1>{});
       return launch(kernel, (unsigned)nmb * batch * head, kPipeThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
-                    (half_t*)dq, head, n, nmb, c, scale);
+                    (half_t*)dq, head, n, FmhaOrder(batch * head, nmb, CAUSAL, n % kPipeBlockQ != 0), nmb, c, scale);
     } else {
       if (spill) {
         // Two panels per block when that leaves every CU at least two blocks (a heavy and a light one).  The persistent
@@ -4141,17 +4140,17 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
         const int nqb2 = (n + 2 * kDsPanelQ - 1) / (2 * kDsPanelQ), total2 = nqb2 * slices;
         if (total2 >= 2 * cus)  // so many blocks are never `wide`
           return launch(fmha_bwd_dq_spill_kernel<D, CAUSAL, 2, false>, groups(nqb2), ds_threads(2), stream, (const half_t*)k, ks,
-                        (const half_t*)ds, np, (half_t*)dq, head, n, nqb2, total2, slice0, stream_ds, scale);
-        const int nqb = np / kDsPanelQ, total = nqb * slices;
+                        (const half_t*)ds, np, (half_t*)dq, head, n, FmhaOrder(slices, nqb2, CAUSAL, false), slice0, stream_ds, scale);
+        const int nqb = np / kDsPanelQ;
         auto kernel = wide() ? fmha_bwd_dq_spill_kernel<D, CAUSAL, 1, true> : fmha_bwd_dq_spill_kernel<D, CAUSAL, 1, false>;
         return launch(kernel, groups(nqb), ds_threads(1), stream, (const half_t*)k, ks,
-                      (const half_t*)ds, np, (half_t*)dq, head, n, nqb, total, slice0, stream_ds, scale);
+                      (const half_t*)ds, np, (half_t*)dq, head, n, FmhaOrder(slices, nqb, CAUSAL, false), slice0, stream_ds, scale);
       }
       const int nmb = (n + kDqBlockQ - 1) / kDqBlockQ;
       auto kernel = dq_makes_stats ? fmha_bwd_dq_kernel<D, CAUSAL, true> : fmha_bwd_dq_kernel<D, CAUSAL, false>;
       return launch(kernel, (unsigned)nmb * batch * head, kDqThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)o, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
-                    (half_t*)dq, head, n, nmb, c, scale);
+                    (half_t*)dq, head, n, nmb, batch * head, c, scale);
     }
   };
   auto dkdv_pass = [&]() {
@@ -4162,7 +4161,8 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
         if (half_round_left((long)nnb * batch * head, n, 3)) kernel = fmha_bwd_dkdv_pipe_kernel<CAUSAL, true>;
       return launch(kernel, (unsigned)nnb * batch * head, kPipeThreads, stream,
                     (const half_t*)q, (const half_t*)k, (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs,
-                    (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n, nnb, c, scale);
+                    (const float*)delta, (const float*)lse2, (half_t*)dk, (half_t*)dv, head, n,
+                    FmhaOrder(batch * head, nnb, CAUSAL, n % kPipeBlockKeys != 0), c, scale);
     } else {
       const int nnb = key_blocks(n);
       auto pick = [&](auto wide_tag) {
@@ -4174,7 +4174,8 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
       auto kernel = wide() ? pick(IntTag<1>{}) : pick(IntTag<0>{});
       return launch(kernel, (unsigned)nnb * slices, kKvThreads, stream, (const half_t*)q, (const half_t*)k,
                     (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)delta, (const float*)lse2,
-                    (half_t*)dk, (half_t*)dv, ds, np, head, n, nnb, slice0, c, scale);
+                    (half_t*)dk, (half_t*)dv, ds, np, head, n, FmhaOrder(slices, nnb, CAUSAL, n % kKvBlockKeys != 0), slice0, c,
+                    scale);
     }
   };
   if constexpr (D == 128) {
@@ -4182,7 +4183,8 @@ int launch_backward(int passes, int slices_at_once, size_t workspace_bytes, unsi
       auto kernel = stream_ds ? fmha_bwd_both_spill_kernel<CAUSAL, false> : fmha_bwd_both_spill_kernel<CAUSAL, true>;
       const hipError_t rc = launch(kernel, (unsigned)fmha_ds_launch_blocks(slices, nb), kKvThreads, stream, (const half_t*)q,
                                    (const half_t*)k, (const half_t*)v, (const half_t*)d_o, qs, ks, vs, gs, (const float*)lse, delta, lse2,
-                                   (half_t*)dq, (half_t*)dk, (half_t*)dv, ds, ready, np, head, n, nb, slices, ticks, c, scale);
+                                   (half_t*)dq, (half_t*)dk, (half_t*)dv, ds, ready, np, head, n, FmhaOrder(slices, nb, CAUSAL, false), ticks, c,
+                                   scale);
       return rc == hipSuccess ? FUSED_MHA_OK : FUSED_MHA_ERR_LAUNCH;
     }
   }

@@ -298,6 +298,89 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_divisors_of_a_launch(tmp_path):
+    """csrc/block_map.h: FmhaDivisor gives the quotients of whole numbers below 2^31, and the orders of blocks that take it are
+    those that take an int."""
+    import subprocess
+
+    src = tmp_path / "check_divisors.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <initializer_list>
+#include <vector>
+#include "block_map.h"
+int main() {
+  const int most = 0x7fffffff;
+  auto wrong = [&](int d) {
+    const FmhaDivisor by(d);
+    auto bad = [&](long n) { return n >= 0 && n <= most && (int)n / by != (int)n / d; };
+    for (long k : {0L, 1L, 2L, 3L, (long)most / d / 2, (long)most / d - 1, (long)most / d, (long)most / d + 1})
+      for (long e = -2; e <= 2; ++e)
+        if (bad(k * d + e)) return true;
+    for (long n = 1; n <= most; n = n * 21 / 13 + 1)
+      if (bad(n) || bad(most - n)) return true;
+    return bad(most);
+  };
+  for (int d = 1; d <= 5000; ++d)
+    if (wrong(d)) { printf("divisor %d\n", d); return 1; }
+  for (long d = 5001; d <= most; d = d * 9 / 8 + 7)
+    if (wrong((int)d)) { printf("divisor %ld\n", d); return 1; }
+  for (int bit = 12; bit < 31; ++bit)
+    for (int e = -1; e <= 1; ++e)
+      if (wrong((1 << bit) + e)) { printf("divisor 2^%d %+d\n", bit, e); return 1; }
+  if (wrong(most) || wrong(most - 1)) { puts("largest"); return 1; }
+  for (int slices : {1, 3, 7, 8, 9, 60, 64, 71, 72, 80, 127, 128, 131, 200})
+    for (int blocks : {1, 2, 3, 5, 8, 9, 16, 31})
+      for (bool heavy : {false, true})
+        for (bool last : {false, true}) {
+          const FmhaOrder one(slices, blocks, heavy, last), two(slices, blocks, heavy, last, 2), ds(slices, blocks, heavy, false);
+          auto differ = [&](int lin) {
+            int s = -1, b = -1, t = -1, c = -1;
+            bool p = false, q = false;
+            if (lin < slices * blocks) {
+              fmha_scheduled_block(lin, slices, blocks, heavy, last, s, b);
+              fmha_ordered_block(lin, one.slices, one.run, one.last_level, heavy, one.short_last, t, c);
+              if (s != t || b != c || s < 0 || s >= slices || b < 0 || b >= blocks) return true;
+              fmha_slice_and_block(lin, slices, blocks, s, b);
+              fmha_slice_and_block(lin, slices, FmhaDivisor(blocks), t, c);
+              if (s != t || b != c) return true;
+            }
+            if (lin < 2 * slices * blocks) {
+              fmha_two_pass_block(lin, slices, blocks, heavy, last, s, b, p);
+              fmha_two_pass_ordered_block(lin, two.slices, two.run, two.last_level, heavy, two.short_last, t, c, q);
+              if (s != t || b != c || p != q || s < 0 || s >= slices || b < 0 || b >= blocks) return true;
+            }
+            s = t = b = c = -1;
+            const bool some = fmha_ds_launch_block(lin, slices, blocks, heavy, s, b, p);
+            return some != fmha_ds_launch_ordered_block(lin, ds.slices, ds.run, ds.last_level, heavy, t, c, q) || s != t || b != c ||
+                   p != q;
+          };
+          std::vector<int> seen(3 * slices * blocks, 0);
+          for (int lin = 0; lin < 2 * slices * blocks; ++lin) {
+            int s, b;
+            bool second = false;
+            if (lin < slices * blocks) {
+              fmha_scheduled_block(lin, slices, blocks, heavy, last, s, b);
+              ++seen[s * blocks + b];
+            }
+            fmha_two_pass_block(lin, slices, blocks, heavy, last, s, b, second);
+            ++seen[((second ? 2 : 1) * slices + s) * blocks + b];
+          }
+          for (int n : seen)
+            if (n != 1) { printf("%d x %d, %d %d: a block %d times\n", blocks, slices, heavy, last, n); return 1; }
+          for (int lin = 0; lin < fmha_ds_launch_blocks(slices, blocks); ++lin)
+            if (differ(lin)) { printf("%d x %d, %d %d: %d\n", blocks, slices, heavy, last, lin); return 1; }
+        }
+  puts("ok");
+  return 0;
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    exe = tmp_path / "check_divisors"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
 def test_persistent_schedule_covers_every_block_once_and_balances(tmp_path):
     """csrc/block_map.h, compiled for the host: the rounds of the persistent work groups visit every block exactly
     once, a work group's blocks stay on its XCD (block number mod 8), and under causal masking the static
