@@ -127,6 +127,42 @@ __device__ __forceinline__ int acc_row(int rb, int r, int hh) {
 // row0 + i; per 32-feature block it holds features 8*g + 4*hh + 0..3 for g = 0..3.
 // The caller makes sure (with a block barrier) that nobody still reads what the
 // staging tile overwrites.
+// The rows of a staging tile as they leave.  All of them are asked for before the first is stored, and only a block with rows
+// past the end looks at each: one after the other, as read, wait, test and store, they take 200 cycles each.
+// Kernels in graphs of 20 calls, us one after the other and as it is, forward, then backward, N x slices: D = 64 77 x 8 causal
+// 5.51, 5.42 and 6.64, 6.40; 128 x 4 4.96, 4.88 and 6.25, 6.07; 1024 x 64 causal 15.7 both and 42.7, 42.1; D = 128 200 x 48
+// causal 9.27, 9.14 and 14.5 both; 2048 x 80 causal 93.9, 93.5 and 291, 289.
+template <int D, int kPitch, typename Piece>
+__device__ __forceinline__ void store_staged(half_t* __restrict__ base, int row_stride, int row0, int n, int lane,
+                                             const char* __restrict__ stage, int upper_off) {
+  constexpr int kLanesPerRow = D / 8, kRowsPerPass = 64 / kLanesPerRow, kPasses = kResident / kRowsPerPass;
+  const int r_in = lane / kLanesPerRow, ch = lane % kLanesPerRow;
+  union Row {
+    Piece piece[16 / sizeof(Piece)];
+    h8 v;
+  } rows[kPasses];
+#pragma unroll
+  for (int pass = 0; pass < kPasses; ++pass) {
+    const int r = pass * kRowsPerPass + r_in;
+    const char* const src = stage + (r & 15) * kPitch + (r >> 4) * upper_off + ch * 16;
+#pragma unroll
+    for (int e = 0; e < (int)(16 / sizeof(Piece)); ++e) rows[pass].piece[e] = *reinterpret_cast<const Piece*>(src + e * sizeof(Piece));
+  }
+  char* const out = reinterpret_cast<char*>(base + (long)row0 * row_stride);
+  const unsigned off = r_in * row_stride * 2 + ch * 16;
+  auto store = [&](int pass) __attribute__((always_inline)) {
+    *reinterpret_cast<h8*>(out + (long)pass * kRowsPerPass * 2 * row_stride + off) = rows[pass].v;
+  };
+  if (row0 + kResident <= n) {
+#pragma unroll
+    for (int pass = 0; pass < kPasses; ++pass) store(pass);
+  } else {
+#pragma unroll
+    for (int pass = 0; pass < kPasses; ++pass)
+      if (row0 + pass * kRowsPerPass + r_in < n) store(pass);
+  }
+}
+
 template <int D>
 struct StageGeom {
   // bytes per row: a row plus 8, so that the lanes of a half wave, which write 8 bytes each to
@@ -137,7 +173,7 @@ struct StageGeom {
   static constexpr int kBytes = kResident * kPitch;  // per wave
 };
 template <int D>
-__device__ __forceinline__ void store_resident(half_t* __restrict__ base, long row_stride, int row0, int n,
+__device__ __forceinline__ void store_resident(half_t* __restrict__ base, int row_stride, int row0, int n,
                                                const f16v (&acc)[TileGeom<D>::kDBlocks], float mul, int lane,
                                                char* __restrict__ stage, int my_row = -1,
                                                int upper_off = 16 * StageGeom<D>::kPitch) {
@@ -159,17 +195,7 @@ __device__ __forceinline__ void store_resident(half_t* __restrict__ base, long r
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own writes have landed
   asm volatile("" ::: "memory");
-  constexpr int kLanesPerRow = D / 8, kRowsPerPass = 64 / kLanesPerRow;
-  const int r_in = lane / kLanesPerRow, ch = lane % kLanesPerRow;
-#pragma unroll
-  for (int pass = 0; pass < kResident / kRowsPerPass; ++pass) {
-    const int r = pass * kRowsPerPass + r_in;
-    const char* src = stage + (r & 15) * kPitch + (r >> 4) * upper_off + ch * 16;
-    const h4 lo = *reinterpret_cast<const h4*>(src);
-    const h4 hi = *reinterpret_cast<const h4*>(src + 8);
-    const h8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    if (row0 + r < n) *reinterpret_cast<h8*>(base + (long)(row0 + r) * row_stride + ch * 8) = v;
-  }
+  store_staged<D, kPitch, h4>(base, row_stride, row0, n, lane, stage, upper_off);
 }
 
 // Blocks of a persistent work group (schedule: block_map.h).
@@ -437,7 +463,7 @@ struct Stage16 {
   static constexpr int kBytes = kResident * kPitch;  // per wave
 };
 template <int D>
-__device__ __forceinline__ void store_resident16(half_t* __restrict__ base, long row_stride, int row0, int n,
+__device__ __forceinline__ void store_resident16(half_t* __restrict__ base, int row_stride, int row0, int n,
                                                  const f4v (*acc)[2], const float (&mul)[2], int lane,
                                                  char* __restrict__ stage, int row_of_0 = -1, int row_of_1 = -1,
                                                  int upper_off = 16 * Stage16<D>::kPitch) {
@@ -458,14 +484,7 @@ __device__ __forceinline__ void store_resident16(half_t* __restrict__ base, long
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's own writes have landed
   asm volatile("" ::: "memory");
-  constexpr int kLanesPerRow = D / 8, kRowsPerPass = 64 / kLanesPerRow;
-  const int r_in = lane / kLanesPerRow, ch = lane % kLanesPerRow;
-#pragma unroll
-  for (int pass = 0; pass < kResident / kRowsPerPass; ++pass) {
-    const int r = pass * kRowsPerPass + r_in;
-    const h8 v = *reinterpret_cast<const h8*>(stage + (r & 15) * kPitch + (r >> 4) * upper_off + ch * 16);
-    if (row0 + r < n) *reinterpret_cast<h8*>(base + (long)(row0 + r) * row_stride + ch * 8) = v;
-  }
+  store_staged<D, kPitch, h8>(base, row_stride, row0, n, lane, stage, upper_off);
 }
 
 // s_waitcnt vmcnt(N) with the other counters left alone.  Issued through the
