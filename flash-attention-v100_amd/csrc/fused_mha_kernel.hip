@@ -3369,13 +3369,19 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
 // and dK, and leaves dS in LDS; behind the next barrier the waves share out the 16 x 16 tiles of dQ of those 32 queries and add
 // up all keys in order.  So S and dP are formed once and neither dS nor partial dQ leaves the CU, each input is read once, and
 // there is one barrier for 32 queries.  All sums are in the order of the other paths, which give the same bits.
-// Bound by the LDS and by issue: at D = 64 with two blocks of keys a wave reads 24 KiB of Q, dO and K for 32 MFMAs of 32 x 32 x
-// 16 and 32 KiB of K and dS for 16 of 16 x 16 x 32, which for 8 waves is 1.5 times as long as a SIMD's MFMAs take, and with two
-// waves to a SIMD the vector work on S and P hardly overlaps with another wave's MFMAs.  (dQ in front of the rest of a tile in
-// all waves, or behind it in half of them, so that the two kinds of work meet: no difference, and the first needs fewer
-// registers.  dQ steps between those of dK: slower.)  Fragments are read two to four MFMA groups ahead; one ahead costs 6 %.
-// 512 x 192 slices, D = 64: 52.7 us, 610 TFLOP/s on the 192 CUs that have work; two passes that form S and dP twice: 61.  256 x
-// 256, D = 128: 37.4 us, 574 TFLOP/s; over dS in memory: 51.9.
+// Bound by the chain of a wave from one barrier to the next: at D = 64 with two blocks of keys a tile takes 5,300 cycles, of which
+// the MFMAs of the two waves of a SIMD take 2,560; with one wave to a SIMD doing its work it still takes 4,800.  A wave reads
+// 24 to 32 KiB of Q, dO and K for 32 MFMAs of 32 x 32 x 16 and 32 KiB of K and dS for 16 of 16 x 16 x 32, 120 instructions, each
+// of which holds it for 15 cycles; the CU's LDS is busy half of the time.  What helps is fewer instructions between two
+// barriers, and MFMAs above all vector work: the products of a tile in an order in which P and dS are formed in the shadow of
+// others (work), no copies of fragments between registers (queries), what depends on the lane worked out once.  us without and
+// with these, backward, N x slices: D = 64 512 x 192 52.7, 50.0; 300 x 256 33.9, 32.4; 256 x 256 22.0, 20.9; causal 384 x 256 36.6,
+// 32.7; 160 x 256 14.7, 13.7; D = 128 256 x 256 36.0, 34.6; causal 31.9, 30.3; 100 x 256 16.9, 15.9.
+// Not taken, 512 x 192: 16 waves of 32 keys 52.7; dQ of the tile before between the products of a tile 49.7; waves 4 to 7 with
+// dQ at the end of a tile 52.7; S and dP of both blocks from the same fragments 54.2, and before, with P and dS in stretches
+// without MFMAs, 54.6; priorities +-1 %.
+// 512 x 192 slices, D = 64: 50.0 us, 640 TFLOP/s on the 192 CUs that have work; two passes that form S and dP twice: 61.  256 x
+// 256, D = 128: 34.6 us, 620 TFLOP/s; over dS in memory: 51.9.
 // At D = 128 without a mask 129 to 160 rows have four idle waves and one of up to 32 keys.  bwd_dkdv_block shares such keys
 // between its four pairs of waves, tile j to pair j mod 4, and adds the four sums up at the end; to have its bits the idle
 // waves do the same here.
@@ -3432,17 +3438,29 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
   const half_t* const c_base = copies_q ? Qb : Gb;
   const int c_stride = copies_q ? qs.n : gs.n;
   char* const c_dst = ring + (copies_q ? 0 : Geo::kTileBytes) + (wave & 3) * kC * 1024;
-  auto copy_tile = [&](int j, int slot) __attribute__((always_inline)) {
-    const int row0 = j * kResident;
-    const half_t* const base = c_base + (long)row0 * c_stride;
-    const int lane = thread_now() & 63;
+  // What depends on the lane is worked out once; a tile costs a few scalar additions.
+  int c_off[kC];
 #pragma unroll
-    for (int u = 0; u < kC; ++u) {
-      int row, off;
-      copy_src<D>((wave & 3) * kC + u, lane, c_stride, row, off);
-      const int back = max(row0 + row - (N - 1), 0);  // rows past the end re-read row N-1
-      copy16(base, off - back * c_stride * 2, c_dst + slot * 2 * Geo::kTileBytes + u * 1024);
+  for (int u = 0; u < kC; ++u) {
+    int row;
+    copy_src<D>((wave & 3) * kC + u, threadIdx.x & 63, c_stride, row, c_off[u]);
+  }
+  const half_t* c_next = c_base;  // the next tile to copy
+  auto copy_tile = [&](int j, int slot) __attribute__((always_inline)) {
+    char* const dst = c_dst + slot * 2 * Geo::kTileBytes;
+    if ((j + 1) * kResident <= N) {
+#pragma unroll
+      for (int u = 0; u < kC; ++u) copy16(c_next, c_off[u], dst + u * 1024);
+    } else {  // the last tile: rows past the end re-read row N-1
+      const int lane = thread_now() & 63;
+#pragma unroll
+      for (int u = 0; u < kC; ++u) {
+        int row, off;
+        copy_src<D>((wave & 3) * kC + u, lane, c_stride, row, off);
+        copy16(c_next, off - max(j * kResident + row - (N - 1), 0) * c_stride * 2, dst + u * 1024);
+      }
     }
+    c_next += kResident * (long)c_stride;
   };
   {  // K, all of it
     constexpr int kPer = T::kInstrs / kSliceWaves;
@@ -3476,20 +3494,26 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
   const bool makes_stats = wave < D / 16;
   char* const o_mine = smem + Geo::kOOff + (wave & (D / 16 - 1)) * 1024;
   char* const o_second = smem + Geo::kExOff + Geo::kExchange + (wave & (D / 16 - 1)) * 1024;  // free until dS of tile 1
+  const int st_row = (threadIdx.x / kLanes) & (kResident - 1), st_col = threadIdx.x % kLanes;
+  const int o_off = (st_row * rs + st_col * 8) * 2;
+  const half_t* o_next = O + head_off;  // the next tile to ask for
+  // of this lane's piece of O where it was copied to, and of dO (chunk st_col of row st_row of a tile, SwzTile) in slot 0
+  const unsigned o_at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)o_mine + (threadIdx.x & 63) * 16;
+  const unsigned g_at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)ring + Geo::kTileBytes +
+                        T::block_off(st_row >> 4, st_col >> 2) + (st_row & 15) * 64 +
+                        (((st_col & 3) ^ swz((st_row & 15) >> 2)) * 16);
   auto stats_load = [&](int j, char* to) __attribute__((always_inline)) {
     if (makes_stats) {
-      const int t = thread_now(), row0 = j * kResident;
-      copy16(O + head_off + (long)row0 * rs, (min(t / kLanes, N - 1 - row0) * rs + t % kLanes * 8) * 2, to);
+      const int past = max(j * kResident + st_row - (N - 1), 0);  // rows past the end re-read row N-1
+      copy16(o_next, o_off - past * rs * 2, to);
+      o_next += kResident * (long)rs;
     }
   };
-  auto stats_make = [&](int j, int slot, const char* from) __attribute__((always_inline)) {
+  auto stats_make = [&](int j, int slot, unsigned from) __attribute__((always_inline)) {
     if (makes_stats) {
-      const int t = thread_now(), st_row = t / kLanes, st_col = t % kLanes;
-      const h8 o8 = *reinterpret_cast<const h8*>(from + (t & 63) * 16);
-      // chunk st_col of row st_row of the tile of dO (SwzTile)
-      const h8 g8 = *reinterpret_cast<const h8*>(ring + slot * 2 * Geo::kTileBytes + Geo::kTileBytes +
-                                                 T::block_off(st_row >> 4, st_col >> 2) + (st_row & 15) * 64 +
-                                                 (((st_col & 3) ^ swz((st_row & 15) >> 2)) * 16));
+      typedef __attribute__((address_space(3))) h8 lds_h8;
+      const h8 o8 = *(const lds_h8*)(uintptr_t)from;
+      const h8 g8 = *(const lds_h8*)(uintptr_t)(g_at + slot * 2 * Geo::kTileBytes);
       float a = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) a = fmaf((float)o8[e], (float)g8[e], a);
@@ -3563,25 +3587,11 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
       asm volatile("" : "+v"(vf[kb][kk]));  // negated here, not in the loop
     }
 
-  // Fragments of LDS are read kLead units ahead of the MFMAs that take them, in an order that is written out and pinned.
-  auto in_order = [&](auto units_tag, auto lead_tag, auto read, auto use) __attribute__((always_inline)) {
-    constexpr int kUnits = decltype(units_tag)::value, kLead = decltype(lead_tag)::value;
-    decltype(read(0)) frag[kLead];
-#pragma unroll
-    for (int n = 0; n < kLead; ++n) frag[n] = read(n);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int n = 0; n < kUnits; ++n) {
-      use(n, frag[n % kLead]);
-      if (n + kLead < kUnits) frag[n % kLead] = read(n + kLead);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
   // dQ of tile j
   auto queries = [&](int j) __attribute__((always_inline)) {
     typedef __attribute__((address_space(3))) s4 lds_s4;
     struct Pair { h8 a, b[kQB]; };
-    const unsigned ex = ea + (j & 1) * Geo::kExchange;
+    unsigned ex = ea + (j & 1) * Geo::kExchange;
     const int n_blocks = CAUSAL ? j + 1 : nj;
     f4v dq[kQB];
 #pragma unroll
@@ -3592,7 +3602,7 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
       return __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
     // every address is one of these and a constant
-    const unsigned k_lo = ka, k_hi = ka ^ kUpper;
+    unsigned k_lo = ka, k_hi = ka ^ kUpper;
     auto read = [&](int kb) __attribute__((always_inline)) {
       Pair f;
       const unsigned kt = (kb >> 1) * T::kBytes + (kb & 1) * T::block_off(2, 0), et = kb * 2048;
@@ -3605,29 +3615,27 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
 #pragma unroll
       for (int n = 0; n < kQB; ++n) dq[n] = mfma16(f.a, f.b[n], dq[n]);
     };
-    constexpr int kLead = 4, kMost = kSliceWaves * KB;
-    Pair frag[kLead];
+    // Four blocks of keys at a time, the next four read while they are used; then the last one to four.  As a loop: unrolled, with
+    // an exit after each four, the compiler copies the fragments from registers to registers at every exit, 150 instructions.
+    constexpr int kGroup = CAUSAL ? 2 : 4;
+    Pair frag[kGroup];
 #pragma unroll
-    for (int u = 0; u < kLead; ++u) frag[u] = read(u);  // also past the last block: of no use then
+    for (int u = 0; u < kGroup; ++u) frag[u] = read(u);  // also past the last block: of no use then
     __builtin_amdgcn_sched_barrier(0);
-    bool more = true;
+    int left = n_blocks;
+#pragma unroll 1
+    for (; left > kGroup; left -= kGroup) {
+      k_lo += kGroup / 2 * T::kBytes, k_hi += kGroup / 2 * T::kBytes, ex += kGroup * 2048;
 #pragma unroll
-    for (int kb = 0; kb < kMost; kb += kLead) {
-      if (!more) continue;
-      more = kb + kLead <= n_blocks;
-      if (more) {
-#pragma unroll
-        for (int u = 0; u < kLead; ++u) {
-          use(frag[u]);
-          if (kb + kLead < kMost) frag[u] = read(kb + kLead + u);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < kLead - 1; ++u)
-          if (kb + u < n_blocks) use(frag[u]);
+      for (int u = 0; u < kGroup; ++u) {
+        use(frag[u]);
+        frag[u] = read(u);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u)
+      if (u < left) use(frag[u]);
     const int lane = thread_now() & 63;
 #pragma unroll
     for (int n = 0; n < kQB; ++n) {
@@ -3639,115 +3647,126 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  // tile j, NB of this wave's key blocks
+  // Tile j, NB of this wave's key blocks, in units of an A fragment and its MFMAs, and what is formed in their shadow:
+  //   NB x kKS  S of one block after the other          P of the block before
+  //   NB x kKS  dP - delta                              P of the last block
+  //   2 x kDB   dV += of queries 0..15, then 16..31     dS of queries 0..15, behind the products with their P
+  //   2 x kDB   dK                                      dS of queries 16..31
   auto work = [&](int j, int slot, auto nb_tag, auto masked_tag) __attribute__((always_inline)) {
     constexpr int NB = decltype(nb_tag)::value;
     constexpr bool MASKED = decltype(masked_tag)::value != 0;
-    struct Rows { h8 a, k[NB]; };
+    constexpr int kS = NB * kKS, kP = 2 * kS, kV = kP + 2 * kDB, kUnits = kV + 2 * kDB;  // the first unit past each kind
+    constexpr int kPairs = 8 / kKS;  // pairs of P formed in a unit
+    constexpr int kLead = NB == 2 ? 2 : 3;
+    struct Frag { h8 a, k; };
     const unsigned at = slot * 2 * Geo::kTileBytes;
     const int q0 = j * kResident, lane = thread_now() & 63, i = lane & 31, hh = lane >> 5;
     const char* const st = smem + Geo::kStOff + (q0 + 4 * hh) * 4;
-    f16v s[NB];
-    h8 y[NB][2];
-    {
-      const unsigned qa0 = ra + at, qa1 = qa0 ^ kOddRows;
-      in_order(IntTag<kKS>{}, IntTag<2>{}, [&](int kk) __attribute__((always_inline)) {
-        Rows f;
-        f.a = swz_rows_at<D>(qa0, qa1, 0, kk);
-#pragma unroll
-        for (int n = 0; n < NB; ++n) f.k[n] = swz_rows_at<D>(kr[n], kr[n] ^ kOddRows, 0, kk);
-        return f;
-      }, [&](int kk, const Rows& f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int n = 0; n < NB; ++n) s[n] = mfma(f.a, f.k[n], kk == 0 ? zero : s[n]);
-      });
-    }
-    auto p_quad = [&](int quad) __attribute__((always_inline)) {
-      const f4v l4 = *reinterpret_cast<const f4v*>(st + 32 * quad);
-#pragma unroll
-      for (int n = 0; n < NB; ++n)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float p = fast_exp2(fmaf(s[n][4 * quad + r], c, -l4[r]));
-          if (MASKED) {
-            const int q = q0 + 8 * quad + 4 * hh + r;
-            if ((CAUSAL && blk[n] * kResident + i > q) || q >= N) p = 0.f;
-          }
-          y[n][quad >> 1][(quad & 1) * 4 + r] = (half_t)p;
-        }
+    const unsigned qa0 = ra + at, qa1 = qa0 ^ kOddRows, qc0 = ca + at, qc1 = qc0 ^ kUpper;
+    f16v s[NB], x[NB];
+    u4v y[NB][2];  // [16 queries]: P, then dS, fp16 pairs in B-operand order
+    f4v l4[NB];
+    Frag frag[kLead];
+    auto read = [&](int m) __attribute__((always_inline)) {
+      Frag f;
+      if (m < kS) {
+        f.a = swz_rows_at<D>(qa0, qa1, 0, m % kKS);
+        f.k = swz_rows_at<D>(kr[m / kKS], kr[m / kKS] ^ kOddRows, 0, m % kKS);
+      } else if (m < kP) {
+        f.a = swz_rows_at<D>(qa0 + Geo::kTileBytes, qa1 + Geo::kTileBytes, 0, m % kKS);
+      } else if (m < kV) {
+        f.a = swz_cols_at<D>(qc0 + Geo::kTileBytes, qc1 + Geo::kTileBytes, (m - kP) / kDB, (m - kP) % kDB);
+      } else {
+        f.a = swz_cols_at<D>(qc0, qc1, (m - kV) / kDB, (m - kV) % kDB);
+      }
+      return f;
     };
-    p_quad(0);
-    p_quad(1);
-    __builtin_amdgcn_sched_barrier(0);
-    {  // the products with the first 16 queries while P of the others is formed
-      const unsigned a0 = ca + Geo::kTileBytes + at, a1 = a0 ^ kUpper;
-      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) {
-        return swz_cols_at<D>(a0, a1, n / kDB, n % kDB);
-      }, [&](int u, h8 f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int n = 0; n < NB; ++n) dv[n][u % kDB] = mfma(f, y[n][u / kDB], dv[n][u % kDB]);
-        if (u == 0) p_quad(2);
-        if (u == kDB / 2) p_quad(3);
-      });
-    }
-    f16v x[NB];
-    const char* const st2 = smem + Geo::kStOff + Geo::kRows * 4 + (q0 + 4 * ((thread_now() & 63) >> 5)) * 4;
-#pragma unroll
-    for (int quad = 0; quad < 4; ++quad) {
-      const f4v d4 = *reinterpret_cast<const f4v*>(st2 + 32 * quad);
-#pragma unroll
-      for (int n = 0; n < NB; ++n)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x[n][4 * quad + r] = d4[r];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      const unsigned a0 = ra + Geo::kTileBytes + at, a1 = a0 ^ kOddRows;
-      in_order(IntTag<kKS>{}, IntTag<3>{}, [&](int kk) __attribute__((always_inline)) { return swz_rows_at<D>(a0, a1, 0, kk); },
-               [&](int kk, h8 f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int n = 0; n < NB; ++n) x[n] = mfma(f, vf[n][kk], x[n]);
-      });
-    }
-    // neg_mul_to_f16x8 is inline asm: the compiler leaves no time in front of it for the last MFMA's results to arrive
-    if constexpr (NB == 1) asm volatile("s_nop 15\n\ts_nop 7" : "+v"(x[0]));
-    else asm volatile("s_nop 15\n\ts_nop 7" : "+v"(x[0]), "+v"(x[NB - 1]));
-    __builtin_amdgcn_sched_barrier(0);
-    const int lane2 = thread_now() & 63, i2 = lane2 & 31;
-    char* const ex = smem + Geo::kExOff + (j & 1) * Geo::kExchange + (2 * i2 + (lane2 >> 5)) * 16;
-    auto ds_half = [&](int cc) __attribute__((always_inline)) {
+    auto p_pair = [&](int n, int e) __attribute__((always_inline)) {  // of 8: two neighbouring queries
+      const int r = 2 * e;
+      if (e % 2 == 0) l4[n] = *reinterpret_cast<const f4v*>(st + 16 * e);
+      float p0 = fast_exp2(fmaf(s[n][r], c, -l4[n][r & 3])), p1 = fast_exp2(fmaf(s[n][r + 1], c, -l4[n][(r & 3) + 1]));
+      if (MASKED) {
+        const int q = q0 + 8 * (r >> 2) + 4 * hh + (r & 3), key = blk[n] * kResident + i;
+        if ((CAUSAL && key > q) || q >= N) p0 = 0.f;
+        if ((CAUSAL && key > q + 1) || q + 1 >= N) p1 = 0.f;
+      }
+      y[n][e >> 2][e & 3] = pack_f16(p0, p1);
+    };
+    auto ds_pair = [&](int n, int e) __attribute__((always_inline)) {
+      y[n][e >> 2][e & 3] = neg_mul_to_f16x2(y[n][e >> 2][e & 3], x[n][2 * e], x[n][2 * e + 1]);
+    };
+    auto ds_out = [&](int cc) __attribute__((always_inline)) {
+      const int lane2 = thread_now() & 63, i2 = lane2 & 31;
+      char* const ex = smem + Geo::kExOff + (j & 1) * Geo::kExchange + (2 * i2 + (lane2 >> 5)) * 16;
 #pragma unroll
       for (int n = 0; n < NB; ++n) {
-        float xr[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xr[e] = x[n][8 * cc + e];
-        y[n][cc] = neg_mul_to_f16x8(y[n][cc], xr);
-        if (blk[n] * kResident + kResident > N && blk[n] * kResident + i2 >= N) y[n][cc] = h8{};  // keys past the end: no dQ
-        *reinterpret_cast<h8*>(ex + blk[n] * 2048 + cc * 1024) = y[n][cc];
+        h8 v = __builtin_bit_cast(h8, y[n][cc]);
+        if (MASKED && blk[n] * kResident + i2 >= N) v = h8{};  // keys past the end: no dQ
+        *reinterpret_cast<h8*>(ex + blk[n] * 2048 + cc * 1024) = v;
       }
     };
-    ds_half(0);
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      const unsigned a0 = ca + at, a1 = a0 ^ kUpper;
-      in_order(IntTag<2 * kDB>{}, IntTag<3>{}, [&](int n) __attribute__((always_inline)) {
-        return swz_cols_at<D>(a0, a1, n / kDB, n % kDB);
-      }, [&](int u, h8 f) __attribute__((always_inline)) {
+    auto delta_in = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
-        for (int n = 0; n < NB; ++n) dk[n][u % kDB] = mfma(f, y[n][u / kDB], dk[n][u % kDB]);
-        if (u == 0) ds_half(1);
+      for (int quad = 0; quad < 4; ++quad) {
+        const f4v d4 = *reinterpret_cast<const f4v*>(st + Geo::kRows * 4 + 32 * quad);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[n][4 * quad + r] = d4[r];
+      }
+    };
+#pragma unroll
+    for (int m = 0; m < kLead; ++m) frag[m] = read(m);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<kUnits>([&](auto m_tag) __attribute__((always_inline)) {
+      constexpr int m = decltype(m_tag)::value;
+      const Frag f = frag[m % kLead];
+      if constexpr (m < kS) {
+        constexpr int n = m / kKS;
+        s[n] = mfma(f.a, f.k, m % kKS == 0 ? zero : s[n]);
+        if constexpr (m == kS - 1) delta_in(0);
+      } else if constexpr (m < kP) {
+        constexpr int n = (m - kS) / kKS;
+        x[n] = mfma(f.a, vf[n][m % kKS], x[n]);
+        if constexpr (NB == 2 && m == kS + kKS - 1) delta_in(NB - 1);
+      } else if constexpr (m < kV) {
+        constexpr int u = m - kP;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) dv[n][u % kDB] = mfma(f.a, __builtin_bit_cast(h8, y[n][u / kDB]), dv[n][u % kDB]);
+      } else {
+        constexpr int u = m - kV;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) dk[n][u % kDB] = mfma(f.a, __builtin_bit_cast(h8, y[n][u / kDB]), dk[n][u % kDB]);
+      }
+      if constexpr (m + kLead < kUnits) frag[m % kLead] = read(m + kLead);
+      static_for<NB>([&](auto n_tag) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_tag)::value, first = (n + 1) * kKS + 1;
+        if constexpr (m >= first && m < first + kKS) {
+#pragma unroll
+          for (int e = 0; e < kPairs; ++e) p_pair(n, kPairs * (m - first) + e);
+        }
       });
-    }
+      static_for<2>([&](auto cc_tag) __attribute__((always_inline)) {
+        constexpr int cc = decltype(cc_tag)::value, first = kP + (1 + cc) * kDB;
+        if constexpr (m >= first && m < first + kDB) {
+          constexpr int kOf = 4 / kDB;
+#pragma unroll
+          for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int e = 0; e < kOf; ++e) ds_pair(n, 4 * cc + kOf * (m - first) + e);
+          if constexpr (m == first + kDB - 1) ds_out(cc);
+        }
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
   };
 
   block_barrier();
-  stats_make(0, 0, o_mine);
-  if (nj > 1) stats_make(1, 1, o_second);
+  stats_make(0, 0, o_at);
+  if (nj > 1) stats_make(1, 1, o_at + (unsigned)(o_second - o_mine));
   int slot = 0, j = 0;
   auto top = [&]() __attribute__((always_inline)) {
     wait_vm<0>();  // tile j + 1 and its rows of O, asked for an iteration ago
     block_barrier();
-    if (j > 0 && j + 1 < nj) stats_make(j + 1, slot == 2 ? 0 : slot + 1, o_mine);
+    if (j > 0 && j + 1 < nj) stats_make(j + 1, slot == 2 ? 0 : slot + 1, o_at);
     if (j + 2 < nj) {
       stats_load(j + 2, o_mine);
       copy_tile(j + 2, slot == 0 ? 2 : slot - 1);
@@ -3761,14 +3780,15 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
   // Tiles in which none, one or both of this wave's key blocks count; those on the diagonal of one and at the end of the slice
   // with the mask, each in a loop of its own so that no accumulator crosses a branch.
   const int whole = N / kResident;
+  const bool past = nj > whole && (blk[0] == whole || blk[KB - 1] == whole);  // this wave has keys past the end
   auto span = [&](int end, int diag, auto nb_tag) __attribute__((always_inline)) {  // up to `end`, with a diagonal tile `diag`
     while (j < end) {
-      while (j < end && (j == diag || j >= whole)) {
+      while (j < end && (past || j == diag || j >= whole)) {
         top();
         work(j, slot, nb_tag, IntTag<1>{});
         next();
       }
-      while (j < end && j != diag && j < whole) {
+      while (j < end && !past && j != diag && j < whole) {
         top();
         work(j, slot, nb_tag, IntTag<0>{});
         next();
