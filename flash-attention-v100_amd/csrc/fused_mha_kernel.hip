@@ -103,6 +103,11 @@ __device__ __forceinline__ h8 neg_mul_to_f16x8(h8 p, const float* x) {
   return __builtin_bit_cast(h8, r);
 }
 
+struct Strides {
+  long b;
+  int n, h;
+};
+
 // Combine a value with the one held by the lane 32 positions away.
 __device__ __forceinline__ float other_half(float x) {
   int xi = __float_as_int(x);
@@ -487,6 +492,17 @@ __device__ __forceinline__ void store_resident16(half_t* __restrict__ base, int 
   store_staged<D, kPitch, h8>(base, row_stride, row0, n, lane, stage, upper_off);
 }
 
+// Arguments of a kernel, asked for here: left to the compiler they come in four or five groups, each where it is first needed and
+// each waited for by itself.  128-query forward, which also tests for a negative scale now instead of negating and
+// choosing, us before and after, N x slices: D = 64 77 x 8 causal 5.43, 5.22; 512 x 192 20.8, 20.2; 1024 x 64 causal 16.05, 15.7; D =
+// 128 200 x 48 causal 9.13, 8.87.  The kernels of the backward gain nothing from it.
+__device__ __forceinline__ void load_now(const Strides& s) { asm volatile("" ::"s"(s.b), "s"(s.n), "s"(s.h)); }
+__device__ __forceinline__ void load_now(const FmhaDivisor& v) { asm volatile("" ::"s"(v.d), "s"(v.mul), "s"(v.shift)); }
+template <typename T>
+__device__ __forceinline__ void load_now(T v) { asm volatile("" ::"s"(v)); }
+template <typename... T>
+__device__ __forceinline__ void load_all_now(const T&... v) { (load_now(v), ...); }
+
 // s_waitcnt vmcnt(N) with the other counters left alone.  Issued through the
 // builtin (not inline asm) so that the compiler's wait-count bookkeeping sees it.
 template <int N>
@@ -555,11 +571,6 @@ __device__ __forceinline__ void store_ds(half_t* p, h8 v, IntTag<kOffset>) {
 // Element strides of a (batch, n, head, d) tensor whose last dimension is
 // contiguous.  The dense layout of reference kernel/fused_mha_kernel.cu:57-59 is
 // {n*head*d, head*d, d}.
-struct Strides {
-  long b;
-  int n, h;
-};
-
 // Row statistics of 64-row tiles for a work group of 4 * D threads: D / 8 lanes to a row, two rows each, in the order of
 // fmha_bwd_delta_kernel.  load asks for the rows of a tile, one tile after the other; make sums up what was asked for.
 template <int D>
@@ -1219,6 +1230,7 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   __shared__ __attribute__((aligned(1024))) char smem[4 * T::kBytes];
   constexpr int kVOff = 2 * T::kBytes;
 
+  load_all_now(Q, K, V, H, N, order.run, order.last_level, order.slices, nb, qs, ks, vs, negate_q);
   if (ODD_FIRST) odd_slots_first();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // what depends on the lane is worked out again where it is needed, not kept in registers across the main loop
@@ -1288,7 +1300,6 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
 #pragma unroll
     for (int kk = 0; kk < G::kKSteps; ++kk) {
       qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
-      if (negate_q) qf[kk] = -qf[kk];
     }
   }
   int k_off[2], v_off[2];
@@ -1484,6 +1495,13 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   };
 
   wait_vm<0>();  // Q rows and the first tiles: no wait for a register load is left to be placed in the loop
+  if (negate_q) {
+#pragma unroll
+    for (int kk = 0; kk < G::kKSteps; ++kk) {
+      qf[kk] = -qf[kk];
+      asm volatile("" : "+v"(qf[kk]));
+    }
+  }
   block_barrier();
   if (ntw > 0) scores(0, sA);
   int j = 0;
