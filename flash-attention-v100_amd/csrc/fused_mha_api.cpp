@@ -18,9 +18,11 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
 #include <atomic>
@@ -65,18 +67,27 @@ at::Tensor dense(const at::Tensor& x) { return x.is_contiguous() ? x : x.contigu
 // (batch, heads, seqlen, head_size)-backed view), otherwise a dense copy.  The
 // reference copies (flash_attn_interface.py:14-15) or mis-reads such inputs.
 struct Operand {
-  at::Tensor t;
+  const void* ptr;
   fused_mha_strides st;
+  at::Tensor copy;  // undefined where the tensor itself is read
+  explicit Operand(const at::Tensor& x) : ptr(x.data_ptr()), st{x.stride(0), x.stride(1), x.stride(2)} {
+    const int64_t sb = st.batch, sn = st.seq, sh = st.head;
+    const bool ok = x.stride(3) == 1 && sb >= 0 && sn >= 0 && sh >= 0 && ((sb | sn | sh) & 7) == 0 &&
+                    sn < (int64_t(1) << 24) && sh < (int64_t(1) << 31) && (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0;
+    if (ok) return;
+    copy = x.contiguous();
+    ptr = copy.data_ptr();
+    st = {copy.stride(0), copy.stride(1), copy.stride(2)};
+  }
 };
-Operand operand(const at::Tensor& x) {
-  const int64_t sb = x.stride(0), sn = x.stride(1), sh = x.stride(2);
-  const bool ok = x.stride(3) == 1 && sb >= 0 && sn >= 0 && sh >= 0 && ((sb | sn | sh) & 7) == 0 &&
-                  sn < (int64_t(1) << 24) && sh < (int64_t(1) << 31) &&
-                  (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0;
-  if (ok) return {x, {sb, sn, sh}};
-  at::Tensor c = x.contiguous();
-  return {c, {c.stride(0), c.stride(1), c.stride(2)}};
-}
+
+// Makes the device of a tensor the current one, which it nearly always is: asking is cheaper than setting it and back.
+struct OnDeviceOf {
+  c10::OptionalDeviceGuard guard;
+  explicit OnDeviceOf(const at::Tensor& x) {
+    if (c10::hip::current_device() != x.get_device()) guard.reset_device(x.device());
+  }
+};
 
 // From this size on (where the backward takes about a millisecond) it is worth asking what memory there is.
 constexpr size_t kLargeWorkspace = (size_t)1 << 30;
@@ -148,17 +159,17 @@ at::Tensor forward(const at::Tensor& q,  // batch x seqlen x heads x head_size
     out = gpu_empty({batch_size, seqlen_q, num_heads, head_size}, at::kHalf, q);
   }
 
-  c10::DeviceGuard device_guard(q.device());
-  const Operand qo = operand(q), ko = operand(k), vo = operand(v);
+  const OnDeviceOf device_guard(q);
+  const Operand qo(q), ko(k), vo(v);
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
   if (lse) {
     *lse = gpu_empty({batch_size, num_heads, seqlen_q}, at::kFloat, q);
-    check_rc(fused_mha_forward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
+    check_rc(fused_mha_forward_strided(qo.ptr, &qo.st, ko.ptr, &ko.st, vo.ptr, &vo.st,
                                        out.data_ptr(), lse->data_ptr(), batch_size, num_heads, seqlen_q, head_size,
                                        softmax_scale, is_causal ? 1 : 0, stream),
              "fused_mha_forward");
   } else {
-    check_rc(fmha_forward_without_lse(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
+    check_rc(fmha_forward_without_lse(qo.ptr, &qo.st, ko.ptr, &ko.st, vo.ptr, &vo.st,
                                       out.data_ptr(), batch_size, num_heads, seqlen_q, head_size, softmax_scale,
                                       is_causal ? 1 : 0, stream),
              "fused_mha_forward");
@@ -216,7 +227,7 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
   CHECK_DEVICE(out); CHECK_DEVICE(dout); CHECK_DEVICE(lse);
   check_arch(q.get_device());
 
-  c10::DeviceGuard device_guard(q.device());
+  const OnDeviceOf device_guard(q);
   auto grad_like = [&](c10::optional<at::Tensor>& g, const char* name) {
     if (g.has_value()) {
       at::Tensor t = g.value();
@@ -230,7 +241,7 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
   };
   at::Tensor dq = grad_like(dq_, "dq"), dk = grad_like(dk_, "dk"), dv = grad_like(dv_, "dv");
 
-  const Operand qo = operand(q), ko = operand(k), vo = operand(v), go = operand(dout);
+  const Operand qo(q), ko(k), vo(v), go(dout);
   at::Tensor od = dense(out), ld = dense(lse);
   // Statistics, and at head size 128 room for dS; a large one only as far as it is there for the taking.
   const size_t min_bytes = fused_mha_backward_min_workspace_bytes(batch_size, num_heads, seqlen_q, head_size);
@@ -250,8 +261,8 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
     workspace = gpu_empty({(int64_t)ws_bytes}, at::kByte, q);
   }
   hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
-  check_rc(fused_mha_backward_strided(qo.t.data_ptr(), &qo.st, ko.t.data_ptr(), &ko.st, vo.t.data_ptr(), &vo.st,
-                                      od.data_ptr(), go.t.data_ptr(), &go.st, ld.data_ptr(), workspace.data_ptr(),
+  check_rc(fused_mha_backward_strided(qo.ptr, &qo.st, ko.ptr, &ko.st, vo.ptr, &vo.st,
+                                      od.data_ptr(), go.ptr, &go.st, ld.data_ptr(), workspace.data_ptr(),
                                       ws_bytes, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), batch_size, num_heads,
                                       seqlen_q, head_size, softmax_scale, is_causal ? 1 : 0, stream),
            "fused_mha_backward");
@@ -260,7 +271,9 @@ std::vector<at::Tensor> mha_bwd(const at::Tensor& dout,  // batch x seqlen x hea
 
 namespace {
 
-at::Tensor last_dim_contiguous(const at::Tensor& x) { return x.stride(-1) == 1 ? x : x.contiguous(); }
+c10::MaybeOwned<at::Tensor> last_dim_contiguous(const at::Tensor& x) {
+  return x.stride(-1) == 1 ? c10::MaybeOwned<at::Tensor>::borrowed(x) : c10::MaybeOwned<at::Tensor>::owned(x.contiguous());
+}
 
 // The autograd node of flash_attn_func.  Native on purpose: a torch.autograd.Function written in Python
 // costs about 60 us per forward and backward, most of it in handing the interpreter lock to the engine's
@@ -269,10 +282,10 @@ class AttentionNode : public torch::autograd::Function<AttentionNode> {
  public:
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q_in, const at::Tensor& k_in,
                             const at::Tensor& v_in, double softmax_scale, bool is_causal) {
-    const at::Tensor q = last_dim_contiguous(q_in), k = last_dim_contiguous(k_in), v = last_dim_contiguous(v_in);
+    const auto q = last_dim_contiguous(q_in), k = last_dim_contiguous(k_in), v = last_dim_contiguous(v_in);
     at::Tensor lse;
-    at::Tensor out = ::forward(q, k, v, c10::nullopt, &lse, (float)softmax_scale, is_causal);
-    ctx->save_for_backward(torch::autograd::variable_list{q, k, v, out, lse});
+    at::Tensor out = ::forward(*q, *k, *v, c10::nullopt, &lse, (float)softmax_scale, is_causal);
+    ctx->save_for_backward(torch::autograd::variable_list{*q, *k, *v, out, lse});
     ctx->saved_data["softmax_scale"] = softmax_scale;
     ctx->saved_data["causal"] = is_causal;
     return out;
@@ -282,7 +295,7 @@ class AttentionNode : public torch::autograd::Function<AttentionNode> {
                                                  torch::autograd::variable_list grad_out) {
     const auto saved = ctx->get_saved_variables();
     c10::optional<at::Tensor> none_q, none_k, none_v;
-    auto grads = mha_bwd(last_dim_contiguous(grad_out[0]), saved[0], saved[1], saved[2], saved[3], saved[4], none_q,
+    auto grads = mha_bwd(*last_dim_contiguous(grad_out[0]), saved[0], saved[1], saved[2], saved[3], saved[4], none_q,
                          none_k, none_v, (float)ctx->saved_data["softmax_scale"].toDouble(),
                          ctx->saved_data["causal"].toBool());
     return {grads[0], grads[1], grads[2], at::Tensor(), at::Tensor()};
@@ -300,13 +313,24 @@ at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
   if ((at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) ||
       has_tangent(q) || has_tangent(k) || has_tangent(v))
     return AttentionNode::apply(q, k, v, scale, is_causal);
-  return forward(last_dim_contiguous(q), last_dim_contiguous(k), last_dim_contiguous(v), c10::nullopt, nullptr,
+  return forward(*last_dim_contiguous(q), *last_dim_contiguous(k), *last_dim_contiguous(v), c10::nullopt, nullptr,
                  (float)scale, is_causal);
+}
+
+// What flash_attn_func calls.  torch.jit.trace records a Python autograd function as a node, and would keep what this module
+// returns as a constant: under it the call goes to the function in Python.
+py::object flash_attn(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c10::optional<double> softmax_scale,
+                      bool is_causal) {
+  if (torch::jit::tracer::isTracing())
+    return py::module_::import("flash_attn_v100.flash_attn_interface").attr("FlashAttnFunc").attr("apply")(q, k, v, softmax_scale,
+                                                                                                    is_causal);
+  return py::cast(attention(q, k, v, softmax_scale, is_causal));
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "FlashAttention forward/backward for gfx950";
   m.def("attention", &attention, "Attention, differentiable in q, k and v");
+  m.def("flash_attn", &flash_attn, "Attention, differentiable in q, k and v, also under torch.jit.trace");
   m.def("fwd", &mha_fwd, "Forward pass");
   m.def("bwd", &mha_bwd, "Backward pass");
 }

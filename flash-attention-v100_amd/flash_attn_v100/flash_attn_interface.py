@@ -27,6 +27,8 @@ except ImportError as exc:  # fail loudly: there is no fallback path
         "(run `python setup.py build_ext --inplace` in flash-attention-v100_amd/): %s" % exc
     ) from exc
 
+_flash_attn = flash_attn_cuda.flash_attn
+
 
 def _flash_attn_forward(q, k, v, softmax_scale, causal):
     maybe_contiguous = lambda x: x.contiguous() if x.stride(-1) != 1 else x
@@ -66,9 +68,5 @@ class FlashAttnFunc(torch.autograd.Function):
 
 
 def flash_attn_func(q, k, v, softmax_scale=None, causal=False):
-    if torch._C._get_tracing_state() is not None:
-        # torch.jit.trace records a Python autograd function as a node; it would keep what the extension returns as a
-        # constant
-        return FlashAttnFunc.apply(q, k, v, softmax_scale, causal)
-    # the same as FlashAttnFunc.apply, with the autograd node in the extension
-    return flash_attn_cuda.attention(q, k, v, softmax_scale, causal)
+    # FlashAttnFunc.apply with the autograd node in the extension, which under torch.jit.trace calls FlashAttnFunc itself
+    return _flash_attn(q, k, v, softmax_scale, causal)
