@@ -452,6 +452,59 @@ struct Cols16 {
     return __builtin_bit_cast(h8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   }
 };
+// s_waitcnt vmcnt(N) with the other counters left alone.  Issued through the
+// builtin (not inline asm) so that the compiler's wait-count bookkeeping sees it.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt immediate");  // bits 3:0 and 15:14 of the immediate
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// A wave's 32 resident rows on their way to registers: copied to D / 16 KiB of LDS that are the wave's own (rows row0 .. of a
+// slice, row N-1 in the place of those past the end) and, once they are there, read as MFMA B operands.  Loaded straight to
+// registers, neighbouring lanes ask for 16 bytes of different rows each, and the CU's path to memory takes 64 cycles for
+// what a copy takes 16 for, 64 bytes of a row from every four lanes: 2,000 to 4,000 cycles at the start of a block.
+// Kernels in graphs of 20 calls, us loaded straight and this way, forward and backward, N x slices: D = 64 128 x 4 4.74, 4.53 and 6.07,
+// 5.64; 300 x 80 causal 7.13, 7.01 and 12.7, 11.7; 1024 x 64 causal 16.6, 16.4 and 43.3, 42.4; D = 128 128 x 32 6.4, 5.9 and 9.5, 8.35;
+// 200 x 48 causal 8.87, 8.60 and 14.5, 13.1; 700 x 24 13.8, 13.4 and 34.3, 33.2; 2048 x 80 causal 94.5, 93.6 and 294.7, 293.8.
+template <int D>
+__device__ __forceinline__ void copy_rows(const half_t* slice, int stride, int row0, int n, int lane, char* lds) {
+  constexpr int kNC = SwzTile<D>::kNC, kBack = 960 * (kNC - 1);  // see copy16_blocks
+  row0 = min(row0, n - 1);
+  const half_t* const base = slice + (long)row0 * stride - kBack / 2;
+  const unsigned to = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int r16 = lane >> 2, col = ((lane & 3) ^ swz(lane >> 4)) * 16 + kBack;
+#pragma unroll
+  for (int R = 0; R < 2; ++R) {
+    const int row = min(16 * R + r16, n - 1 - row0);
+    copy16_blocks<kNC>(base, row * stride * 2 + col, to + SwzTile<D>::block_off(R, 0));
+  }
+}
+template <int D>
+struct StagedRows {
+  const char* at;
+  int lane;
+  __device__ __forceinline__ h8 wide(int kk) const {  // for 32 x 32 MFMAs: features 16 kk .. of row lane & 31
+    int off[2];
+    swz_rows_off<D>(lane, off);
+    return swz_rows<D>(at, 0, kk, off);
+  }
+  __device__ __forceinline__ h8 narrow(int kk, int cb) const {  // for 16 x 16 ones: features 32 kk .. of row 16 cb + (lane & 15)
+    const int i = lane & 15;
+    return *reinterpret_cast<const h8*>(at + SwzTile<D>::block_off(cb, kk) + i * 64 + (((lane >> 4) ^ swz(i >> 2)) * 16));
+  }
+};
+// The copies are there: read them.
+__device__ __forceinline__ void staged_rows_landed() {
+  wait_vm<0>();
+  asm volatile("" ::: "memory");
+}
+// They are read: others may take their place.
+__device__ __forceinline__ void staged_rows_read() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+}
+
 // Over the four lanes with the same l & 15: first the two that are 32 apart, then the others.
 __device__ __forceinline__ float max_over_groups(float x) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
@@ -503,13 +556,6 @@ __device__ __forceinline__ void load_now(T v) { asm volatile("" ::"s"(v)); }
 template <typename... T>
 __device__ __forceinline__ void load_all_now(const T&... v) { (load_now(v), ...); }
 
-// s_waitcnt vmcnt(N) with the other counters left alone.  Issued through the
-// builtin (not inline asm) so that the compiler's wait-count bookkeeping sees it.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt immediate");  // bits 3:0 and 15:14 of the immediate
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 // Wait until at most n (0 to 4) of this wave's LDS reads are on their way.
 __device__ __forceinline__ void wait_lds(int n) {
   if (n == 0) __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -1294,18 +1340,11 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     copy16_blocks<kIPW>(vp, v_goff, lds_w + kVOff + slot * T::kBytes);
     vp += (long)kTile * vs.n;
   };
+  char* const my_rows = smem + kVOff + wave * (T::kBytes / 2);  // the block's rows of Q fill the slots of V, which comes later
+  copy_rows<D>(Q + b * qs.b + (long)h * qs.h, qs.n, q0w, N, lane_now(), my_rows);
   copy_k(0, 0);
   if (nt > 1) copy_k(1, 1);
-
   h8 qf[G::kKSteps];
-  {
-    const half_t* qp = Q + b * qs.b + (long)h * qs.h + (long)min(q0w + (lane_now() & 31), N - 1) * qs.n +
-                       (lane_now() >> 5) * 8;
-#pragma unroll
-    for (int kk = 0; kk < G::kKSteps; ++kk) {
-      qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
-    }
-  }
   int k_off[2], v_off[2];
   swz_rows_off<D>(lane_now(), k_off);
   swz_cols_off<D>(lane_now(), v_off);
@@ -1498,7 +1537,15 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     return l0 + l1;
   };
 
-  wait_vm<0>();  // Q rows and the first tiles: no wait for a register load is left to be placed in the loop
+  if (nt > 1) wait_vm<kIPW>();  // the second tile of K may still be on its way
+  else wait_vm<0>();
+  asm volatile("" ::: "memory");
+  {
+    const StagedRows<D> rows{my_rows, lane_now()};
+#pragma unroll
+    for (int kk = 0; kk < G::kKSteps; ++kk) qf[kk] = rows.wide(kk);
+    staged_rows_read();
+  }
   if (negate_q) {
 #pragma unroll
     for (int kk = 0; kk < G::kKSteps; ++kk) {
@@ -1727,6 +1774,12 @@ bwd_dq_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const h
     }
   };
 
+  // rows of Q: slots 2 and 3 of K; of dO: slot 2 of V and the buffers of P
+  char* const my_rows = !role_b ? k_ring + 2 * T::kBytes + pair * (T::kBytes / 2)
+                        : pair < 2 ? v_ring + 2 * T::kBytes + pair * (T::kBytes / 2) : p_xchg + (pair - 2) * (T::kBytes / 2);
+  static_assert(2 * kPBytes >= T::kBytes, "the rows of dO of two pairs fit where P goes");
+  if (role_b) copy_rows<D>(dO + b * gs.b + (long)h * gs.h, gs.n, q0w, N, lane, my_rows);
+  else copy_rows<D>(Q + b * qs.b + (long)h * qs.h, qs.n, q0w, N, lane, my_rows);
   copy_tiles(0);
   if (nt > 1) copy_tiles(1);
 
@@ -1735,23 +1788,28 @@ bwd_dq_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const h
   const long stat_at = ((long)b * H + h) * N + qrow;
   float stat;
   {
-    const half_t* rp = (role_b ? dO + b * gs.b + (long)h * gs.h + (long)qrow * gs.n
-                               : Q + b * qs.b + (long)h * qs.h + (long)qrow * qs.n) + hh * 8;
+    h8 ov[STATS ? G::kKSteps : 1];
+    if (STATS && role_b) {
+      const half_t* op = O + head_off + (long)qrow * rs + hh * 8;
 #pragma unroll
-    for (int kk = 0; kk < G::kKSteps; ++kk) rf[kk] = *reinterpret_cast<const h8*>(rp + kk * 16);
+      for (int kk = 0; kk < (STATS ? G::kKSteps : 1); ++kk) ov[kk] = *reinterpret_cast<const h8*>(op + kk * 16);
+    }
+    staged_rows_landed();
+    const StagedRows<D> rows{my_rows, lane};
+#pragma unroll
+    for (int kk = 0; kk < G::kKSteps; ++kk) rf[kk] = rows.wide(kk);
+    staged_rows_read();
     if (STATS) {
       if (role_b) {
         // delta of this lane's query.  The lane has every other 8-feature chunk of
         // the row; the partial sums are combined in the order of
         // fmha_bwd_delta_kernel's shuffle tree, so both give the same bits.
-        const half_t* op = O + head_off + (long)qrow * rs + hh * 8;
         float part[G::kKSteps];
 #pragma unroll
         for (int kk = 0; kk < G::kKSteps; ++kk) {
-          const h8 ov = *reinterpret_cast<const h8*>(op + kk * 16);
           part[kk] = 0.f;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) part[kk] = fmaf((float)ov[e], (float)rf[kk][e], part[kk]);
+          for (int e = 0; e < 8; ++e) part[kk] = fmaf((float)ov[STATS ? kk : 0][e], (float)rf[kk][e], part[kk]);
         }
 #pragma unroll
         for (int stride = G::kKSteps / 2; stride > 0; stride >>= 1)
@@ -1922,7 +1980,7 @@ fmha_bwd_dq_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, c
 //
 // dQ pass.  The formulas are those of fmha_bwd_dq_kernel, and so are the results, bit for bit.
 // ---------------------------------------------------------------------------
-constexpr int kDqPipeLds = 2 * 3 * SwzTile<64>::kBytes;
+constexpr int kDqPipeLds = 2 * 3 * SwzTile<64>::kBytes + 2 * SwzTile<64>::kBytes;  // rings, rows of O
 template <bool CAUSAL, bool STATS>
 __device__ __forceinline__ void
 bwd_dq_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
@@ -1937,7 +1995,7 @@ bwd_dq_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, co
   static_assert(kIPW == T::kNC, "a wave copies the 16 rows of one block row of a tile");
   constexpr int kSlots = 3;  // K tiles, then V tiles: the current one, the one before it, the one being copied
   constexpr int kVOff = kSlots * T::kBytes;
-  static_assert(kDqPipeLds == 2 * kSlots * T::kBytes, "");
+  static_assert(kDqPipeLds == 2 * kSlots * T::kBytes + kPipeWaves * T::kBytes / 2, "");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1980,26 +2038,33 @@ bwd_dq_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, co
   };
   copy_tile(0, 0);
 
-  // Resident rows and the row statistics.  dO is negated: its product with V on top of delta gives delta - dP.
+  // Resident rows and the row statistics.  dO is negated: its product with V on top of delta gives delta - dP.  The rows come
+  // through slots 1 and 2 of the rings, those of O behind them.
   h8 qf[kKS], gf[kKS];
   float my_lse2, my_delta;
   {
-    const half_t* qp = Q + b * qs.b + (long)h * qs.h + (long)qrow * qs.n + hh * 8;
-    const half_t* gp = dO + b * gs.b + (long)h * gs.h + (long)qrow * gs.n + hh * 8;
+    char* const q_rows = smem + T::kBytes + wave * (T::kBytes / 2);
+    copy_rows<D>(Q + b * qs.b + (long)h * qs.h, qs.n, q0w, N, lane, q_rows);
+    copy_rows<D>(dO + b * gs.b + (long)h * gs.h, gs.n, q0w, N, lane, q_rows + kVOff);
+    char* const o_rows = smem + 2 * kVOff + wave * (T::kBytes / 2);
+    if (STATS) copy_rows<D>(O + head_off, rs, q0w, N, lane, o_rows);
     const long stat_at = ((long)b * H + h) * N + qrow;
+    my_lse2 = LSE[stat_at] * kLog2e;
+    if (!STATS) my_delta = delta[stat_at];
+    staged_rows_landed();
+    const StagedRows<D> q_at{q_rows, lane}, g_at{q_rows + kVOff, lane}, o_at{o_rows, lane};
 #pragma unroll
     for (int kk = 0; kk < kKS; ++kk) {
-      qf[kk] = *reinterpret_cast<const h8*>(qp + kk * 16);
-      gf[kk] = *reinterpret_cast<const h8*>(gp + kk * 16);
+      qf[kk] = q_at.wide(kk);
+      gf[kk] = g_at.wide(kk);
     }
-    my_lse2 = LSE[stat_at] * kLog2e;
+    staged_rows_read();
     if (STATS) {
       // partial sums combined in the order of fmha_bwd_delta_kernel's shuffle tree: the same bits
-      const half_t* op = O + head_off + (long)qrow * rs + hh * 8;
       float part[kKS];
 #pragma unroll
       for (int kk = 0; kk < kKS; ++kk) {
-        const h8 ov = *reinterpret_cast<const h8*>(op + kk * 16);
+        const h8 ov = o_at.wide(kk);
         part[kk] = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) part[kk] = fmaf((float)ov[e], (float)gf[kk][e], part[kk]);
@@ -2013,8 +2078,6 @@ bwd_dq_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, co
         delta[stat_at] = my_delta;
         lse2[stat_at] = my_lse2;
       }
-    } else {
-      my_delta = delta[stat_at];
     }
 #pragma unroll
     for (int kk = 0; kk < kKS; ++kk) {
@@ -2292,16 +2355,13 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
   // k0w + 16 cb + i.  They and the first tile are all that the loops need to start; the second tile is asked for when these
   // are there, not waited for with them.  What that gives, 0.2 to 0.8 % of B3 H20 N1031, B2 H40 N2048 causal and B2 H32 N4096
   // causal, is within what runs of one side differ by.
+  static_assert(2 * kKvPairs * 4096 >= T::kBytes, "the rows of V of two pairs fit where P goes");
   h8 rf[G::kKSteps];
-#pragma unroll
-  for (int cb = 0; cb < (WIDE ? 1 : 2); ++cb) {
-    const int krow = min(k0w + 16 * cb + i, N - 1);
-    const half_t* rp = (role_b ? V + b * vs.b + (long)h * vs.h + (long)krow * vs.n
-                               : K + b * ks.b + (long)h * ks.h + (long)krow * ks.n) + g * 8;
-#pragma unroll
-    for (int kk = 0; kk < (WIDE ? G::kKSteps : G16::kKS); ++kk)
-      rf[WIDE ? kk : 2 * kk + cb] = *reinterpret_cast<const h8*>(rp + kk * (WIDE ? 16 : 32));
-  }
+  // rows of K: slots 2 and 3 of Q; of V: slot 2 of dO and the buffers of P
+  char* const my_rows = !role_b ? q_ring + 2 * T::kBytes + pair * (T::kBytes / 2)
+                        : pair < 2 ? g_ring + 2 * T::kBytes + pair * (T::kBytes / 2) : p_xchg + (pair - 2) * (T::kBytes / 2);
+  if (role_b) copy_rows<D>(V + b * vs.b + (long)h * vs.h, vs.n, k0w, N, lane, my_rows);
+  else copy_rows<D>(K + b * ks.b + (long)h * ks.h, ks.n, k0w, N, lane, my_rows);
   copy_tiles(0);
 
   // statistics: the rows are asked for two tiles ahead, into registers, and summed up one tile ahead
@@ -2482,7 +2542,13 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
                                       ((k0w >> 5) & 1) * 4096 + lane * 8
                                 : nullptr;
   if (STATS) stats_ahead(-1);
-  wait_vm<0>();  // resident rows and the first tile: nothing is left for the compiler to wait on in the loops
+  staged_rows_landed();  // resident rows and the first tile: nothing is left for the compiler to wait on in the loops
+  {
+    const StagedRows<D> rows{my_rows, lane};
+#pragma unroll
+    for (int kk = 0; kk < G::kKSteps; ++kk) rf[kk] = WIDE ? rows.wide(kk) : rows.narrow(kk >> 1, kk & 1);
+    staged_rows_read();
+  }
   // Role B works with -V: its first GEMM then gives delta - dP on top of accumulators loaded with delta, with no
   // subtraction afterwards.
   const unsigned sign = role_b ? 0x80008000u : 0u;
@@ -2703,7 +2769,7 @@ bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, 
   const int rs = H * D;                                   // dK and dV are dense
   const long head_off = ((long)b * N * H + h) * D;
   const int n0 = nblk * kPipeBlockKeys;
-  const int k0w = n0 + wave * kResident, ki = k0w + i, krow = min(ki, N - 1);
+  const int k0w = n0 + wave * kResident, ki = k0w + i;
 
   const int nt = (N + kTile - 1) / kTile;
   const int t_begin = CAUSAL ? n0 / kTile : 0;
@@ -2734,6 +2800,9 @@ bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, 
     gp += (long)kTile * gs.n;
     if (!STATS && wave < 2) copy4(stat, min(t * kTile + lane, N - 1) * 4, smem + kStOff + slot * kStBytes + wave * 256);
   };
+  char* const k_rows = smem + T::kBytes + wave * (T::kBytes / 2);  // through slots 1 and 2 of the rings; of V: + kGOff
+  copy_rows<D>(K + b * ks.b + (long)h * ks.h, ks.n, k0w, N, lane, k_rows);
+  copy_rows<D>(V + b * vs.b + (long)h * vs.h, vs.n, k0w, N, lane, k_rows + kGOff);
   copy_tile(t_begin, 0);
 
   // statistics: the rows are asked for two tiles ahead, into registers, and summed up one tile ahead
@@ -2745,13 +2814,14 @@ bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, 
   // resident rows: K, and V negated, so that the dP product on top of delta gives delta - dP
   h8 kf[kKS], vf[kKS];
   {
-    const half_t* kp = K + b * ks.b + (long)h * ks.h + (long)krow * ks.n + hh * 8;
-    const half_t* vp = V + b * vs.b + (long)h * vs.h + (long)krow * vs.n + hh * 8;
+    staged_rows_landed();
+    const StagedRows<D> k_at{k_rows, lane}, v_at{k_rows + kGOff, lane};
 #pragma unroll
     for (int kk = 0; kk < kKS; ++kk) {
-      kf[kk] = *reinterpret_cast<const h8*>(kp + kk * 16);
-      vf[kk] = *reinterpret_cast<const h8*>(vp + kk * 16);
+      kf[kk] = k_at.wide(kk);
+      vf[kk] = v_at.wide(kk);
     }
+    staged_rows_read();
 #pragma unroll
     for (int kk = 0; kk < kKS; ++kk) {
       vf[kk] = -vf[kk];
@@ -3502,6 +3572,14 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
 
   // V rows, negated
   h8 vf[KB][kKS];
+  constexpr bool kStaged = D == 64;  // through where dS goes, which at D = 128 holds only half of them
+  if constexpr (kStaged) {
+    static_assert(D != 64 || 2 * Geo::kExchange >= kSliceWaves * KB * T::kBytes / 2, "");
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      copy_rows<D>(V + b * vs.b + (long)h * vs.h, vs.n, blk[kb] * kResident, N, thread_now() & 63,
+                   smem + Geo::kExOff + (wave * KB + kb) * (T::kBytes / 2));
+  } else {
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     const int lane = thread_now() & 63;
@@ -3510,12 +3588,13 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
 #pragma unroll
     for (int kk = 0; kk < kKS; ++kk) vf[kb][kk] = *reinterpret_cast<const h8*>(vp + kk * 16);
   }
+  }
   // Row statistics of 32 rows, in the order of fmha_bwd_delta_kernel, by the first D / 16 waves.  The rows of O that a wave
   // adds up it copies itself, 1 KiB of them, for its lanes to read back.
   constexpr int kLanes = D / 8;
   const bool makes_stats = wave < D / 16;
   char* const o_mine = smem + Geo::kOOff + (wave & (D / 16 - 1)) * 1024;
-  char* const o_second = smem + Geo::kExOff + Geo::kExchange + (wave & (D / 16 - 1)) * 1024;  // free until dS of tile 1
+  char* const o_second = ring + 2 * 2 * Geo::kTileBytes + (wave & (D / 16 - 1)) * 1024;  // free until tile 2 is copied
   const int st_row = (threadIdx.x / kLanes) & (kResident - 1), st_col = threadIdx.x % kLanes;
   const int o_off = (st_row * rs + st_col * 8) * 2;
   const half_t* o_next = O + head_off;  // the next tile to ask for
@@ -3600,7 +3679,16 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
   f16v zero;
 #pragma unroll
   for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-  wait_vm<0>();
+  staged_rows_landed();
+  if constexpr (kStaged) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const StagedRows<D> rows{smem + Geo::kExOff + (wave * KB + kb) * (T::kBytes / 2), (int)threadIdx.x & 63};
+#pragma unroll
+      for (int kk = 0; kk < kKS; ++kk) vf[kb][kk] = rows.wide(kk);
+    }
+    staged_rows_read();
+  }
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
