@@ -403,7 +403,7 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 // x 432 93.7, 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512
 // x 900 217, 198; 512 x 1030 247, 246; 300 x 1030 124, 141.
 // D = 64 without a mask, 385 to 512 rows, one round: the line is at the fewest slices that were timed, not where the passes are
-// as fast.  A round takes as long with fewer (512 rows: 52.7), and the passes 57.5 for 512 x 176.
+// as fast.  A round takes as long with fewer (512 rows: 50.0), and the passes 57.5 for 512 x 176.
 // Causal, D = 128, a second round of slices just past 96 rows (four tiles of 32 queries instead of three), us of forward and
 // backward, without it and with it: 97 x 257 37.1, 37.7; 97 x 266 37.8, 39.9; 97 x 296 39.2, 39.8; 97 x 320 39.8, 39.6; 105 x
 // 266 38.9, 40.3; 105 x 306 40.4, 40.2; 112 x 266 40.0, 40.6; 112 x 306 41.5, 40.5; 116 x 266 40.7, 40.7; 128 x 266 42.3, 41.4;
