@@ -1569,6 +1569,11 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     // done then is not held twice.  At D = 128 the kernel still uses all 256 registers and spills three (16 bytes of
     // scratch per lane): two across the whole loop, one in the path that raises the maximum, where the reload waits for
     // the tile copies in flight.  Nothing is spilled or reloaded inside a step.
+    // A wave alone on its SIMD is held up where instructions are fetched across a 32-byte line at the wrong place: the loop is put
+    // where it was fastest, with its first instruction 8 bytes past a line at D = 128 and on a multiple of 16 at D = 64, by nops that run
+    // once.  us as it falls and with the loop at + 24, + 8 (D = 128), + 16, + 0 (D = 64): D = 128 8415 x 3 causal 97.3, 96.9, 95.6;
+    // 4000 x 2 49.3, 48.4, 48.2; causal 47.4, 47.6, 47.3; D = 64 8143 x 6 causal 79.2, 78.6, 78.6; 1024 x 64 causal 15.0, 14.9 both.
+    asm volatile(".p2align 6\n\t.rept 4\n\ts_nop 0\n\t.endr");
     bool odd_done = false;
     for (;;) {
       int why;
