@@ -317,14 +317,36 @@ at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
                  (float)scale, is_causal);
 }
 
+// An argument and what the caller gave for it.  While torch.jit.trace records nothing is converted: a scale that is a tensor is an
+// input of the recorded node then, and its value at that time would be a constant of the graph.
+template <typename T>
+struct __attribute__((visibility("hidden"))) Given {  // as pybind11's handles are
+  py::handle object;
+  T value{};
+};
+namespace pybind11::detail {
+template <typename T>
+struct type_caster<Given<T>> {
+  PYBIND11_TYPE_CASTER(Given<T>, make_caster<T>::name);
+  bool load(handle src, bool convert) {
+    value.object = src;
+    if (torch::jit::tracer::isTracing()) return true;
+    make_caster<T> caster;
+    if (!caster.load(src, convert)) return false;
+    value.value = cast_op<T>(std::move(caster));
+    return true;
+  }
+};
+}  // namespace pybind11::detail
+
 // What flash_attn_func calls.  torch.jit.trace records a Python autograd function as a node, and would keep what this module
-// returns as a constant: under it the call goes to the function in Python.
-py::object flash_attn(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c10::optional<double> softmax_scale,
-                      bool is_causal) {
+// returns as a constant: under it the call goes to the function in Python, with the options as they were given.
+py::object flash_attn(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                      const Given<c10::optional<double>>& softmax_scale, const Given<bool>& is_causal) {
   if (torch::jit::tracer::isTracing())
-    return py::module_::import("flash_attn_v100.flash_attn_interface").attr("FlashAttnFunc").attr("apply")(q, k, v, softmax_scale,
-                                                                                                    is_causal);
-  return py::cast(attention(q, k, v, softmax_scale, is_causal));
+    return py::module_::import("flash_attn_v100.flash_attn_interface")
+        .attr("FlashAttnFunc").attr("apply")(q, k, v, softmax_scale.object, is_causal.object);
+  return py::cast(attention(q, k, v, softmax_scale.value, is_causal.value));
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

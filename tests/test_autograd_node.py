@@ -23,6 +23,29 @@ def test_trace_takes_the_recordable_node(monkeypatch):
     assert torch.equal(traced(-q, k, v), q * -2)
 
 
+@pytest.mark.parametrize("of", ["softmax_scale", "causal"])
+def test_trace_keeps_the_inputs_that_options_are(monkeypatch, of):
+    """On the CPU, with the extension's functions replaced: a scale or a mask that is an input of the traced function stays
+    one, so that a replay takes the new value."""
+    from flash_attn_v100 import flash_attn_interface as interface
+
+    class Stub:
+        @staticmethod
+        def fwd(q, k, v, out, scale, causal):
+            return torch.from_numpy(q.detach().numpy() * (float(scale) + 10 * bool(causal))), None
+
+    monkeypatch.setattr(interface, "flash_attn_cuda", Stub)
+    q, k, v, _ = ao.make_inputs(1, 8, 1, 64, seed=1)
+    q = q.clamp(-1, 1)
+    if of == "softmax_scale":
+        call, first, then = lambda a, b, c, s: interface.flash_attn_func(a, b, c, s), torch.tensor(2.0), torch.tensor(3.0)
+    else:
+        call, first, then = lambda a, b, c, s: interface.flash_attn_func(a, b, c, 2.0, s), torch.tensor(False), torch.tensor(True)
+    traced = torch.jit.trace(call, (q, k, v, first), check_trace=False)
+    assert torch.equal(traced(q, k, v, first), q * 2)
+    assert torch.equal(traced(q, k, v, then), q * (3 if of == "softmax_scale" else 12))
+
+
 @pytest.mark.gpu
 def test_trace_of_the_extension():
     from flash_attn_v100 import flash_attn_func
