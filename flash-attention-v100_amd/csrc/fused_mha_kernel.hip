@@ -1266,6 +1266,36 @@ __device__ __forceinline__ void fwd_tail_rows(const half_t* __restrict__ Q, cons
   if (LSE && lane < 32 && q0 + i < N) LSE[((long)b * H + h) * N + q0 + i] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
 }
 
+// The arguments of the kernel below as they lie in memory (checked behind it), and a second look at them.  A work group with the last
+// rows of slices takes them from there: from the loads at the kernel's start they stay in registers across the branch for both
+// ways, which spills six vector registers in the main body at D = 128, where without that way it spills three, and 22 to 25
+// scalar ones at both head sizes, where it spills none.  Forward, us that way and this way, N x slices: D = 128 129 x 400 16.4, 15.9;
+// causal 14.3, 13.9; 385 x 300 causal 33.0, 32.6; 1031 x 60 43.3, 43.2; D = 64 129 x 400 8.8, 8.5; 520 x 160 23.0, 22.7; 391 x 300
+// causal 20.7, 20.0.  With PipeArgs as the one parameter of the kernel, variants without that way got slower: D = 64, 300 x 80
+// causal 7.2, 7.4.
+struct PipeArgs {
+  const half_t *Q, *K, *V;
+  Strides qs, ks, vs;
+  half_t* O;
+  float* LSE;
+  FmhaDivisor H;
+  int N;
+  FmhaOrder order;
+  int nb, tails, tails_per_block;
+  float c;
+  int negate_q;
+};
+__device__ __forceinline__ PipeArgs pipe_args_again() {
+  typedef __attribute__((address_space(4))) const unsigned Word;
+  Word* from = (Word*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(from));
+  struct Words {
+    unsigned w[sizeof(PipeArgs) / 4];
+  } words;
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(PipeArgs) / 4; ++i) words.w[i] = from[i];
+  return __builtin_bit_cast(PipeArgs, words);
+}
 template <int D, bool CAUSAL, bool ODD_FIRST, bool TAIL>
 __global__ void __launch_bounds__(kPipeThreads, 2)
 fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K, const half_t* __restrict__ V,
@@ -1293,9 +1323,10 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   const int lin = CAUSAL ? fmha_paired_block(blockIdx.x, gridDim.x) : blockIdx.x;
   if constexpr (TAIL) {
     if (lin < tails) {
-      bh = fmha_tail_slice(lin, wave, tails, tails_per_block);
-      if (wave < tails_per_block && bh < order.slices)
-        fwd_tail_rows<D, CAUSAL>(Q, K, V, qs, ks, vs, O, LSE, H, N, bh, c, negate_q, smem + wave * T::kBytes);
+      const PipeArgs a = pipe_args_again();
+      bh = fmha_tail_slice(lin, wave, a.tails, a.tails_per_block);
+      if (wave < a.tails_per_block && bh < a.order.slices)
+        fwd_tail_rows<D, CAUSAL>(a.Q, a.K, a.V, a.qs, a.ks, a.vs, a.O, a.LSE, a.H, a.N, bh, a.c, a.negate_q, smem + wave * T::kBytes);
       return;
     }
   }
@@ -1623,6 +1654,24 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
   store_resident<D>(O + head_off, rs, q0w, N, o, inv, lane, smem + wave * StageGeom<D>::kBytes);
   if (LSE && lane < 32 && qi < N) LSE[((long)b * H + h) * N + qi] = (mc + __builtin_amdgcn_logf(l_tot)) * kLn2;
 }
+// A kernel's arguments lie one behind the other, each at the next multiple of its own alignment.
+template <typename... Params>
+constexpr bool lie_at(void (*)(Params...), const size_t (&at)[sizeof...(Params)]) {
+  constexpr size_t size[] = {sizeof(Params)...}, align[] = {alignof(Params)...};
+  size_t next = 0;
+  for (size_t i = 0; i < sizeof...(Params); ++i) {
+    next = (next + align[i] - 1) / align[i] * align[i];
+    if (next != at[i]) return false;
+    next += size[i];
+  }
+  return true;
+}
+#define AT(member) offsetof(PipeArgs, member)
+static_assert(lie_at(fmha_fwd_pipe_kernel<64, false, false, true>,
+                     {AT(Q), AT(K), AT(V), AT(qs), AT(ks), AT(vs), AT(O), AT(LSE), AT(H), AT(N), AT(order), AT(nb), AT(tails),
+                      AT(tails_per_block), AT(c), AT(negate_q)}),
+              "PipeArgs is not what the kernel takes");
+#undef AT
 
 // ---------------------------------------------------------------------------
 // delta[b][h][n] = sum_d dO * O in fp32.  One 16-byte chunk per thread.
