@@ -1600,11 +1600,15 @@ fmha_fwd_pipe_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K,
     // done then is not held twice.  At D = 128 the kernel still uses all 256 registers and spills three (16 bytes of
     // scratch per lane): two across the whole loop, one in the path that raises the maximum, where the reload waits for
     // the tile copies in flight.  Nothing is spilled or reloaded inside a step.
-    // A wave alone on its SIMD is held up where instructions are fetched across a 32-byte line at the wrong place: the loop is put
-    // where it was fastest, with its first instruction 8 bytes past a line at D = 128 and on a multiple of 16 at D = 64, by nops that run
-    // once.  us as it falls and with the loop at + 24, + 8 (D = 128), + 16, + 0 (D = 64): D = 128 8415 x 3 causal 97.3, 96.9, 95.6;
-    // 4000 x 2 49.3, 48.4, 48.2; causal 47.4, 47.6, 47.3; D = 64 8143 x 6 causal 79.2, 78.6, 78.6; 1024 x 64 causal 15.0, 14.9 both.
-    asm volatile(".p2align 6\n\t.rept 4\n\ts_nop 0\n\t.endr");
+    // A wave alone on its SIMD is held up where instructions are fetched across a 32-byte line at the wrong place.  The nops, which run
+    // once, put the loop where it was fastest in the variants without work groups for last rows, as ROCm 7.2.0's compiler lays them out:
+    // it begins on a line at D = 128 and 24 bytes past one at D = 64 (tests/test_code_object.py has it by the first barrier; where
+    // that moves, time 0 to 7 nops again).  us with the loop at + 8, 12, 16, 20, 24, 28, 0 and 4: D = 128 8415 x 3 causal 97.2, 96.3,
+    // 96.1, 97.5, 95.8, 97.3, 95.2, 98.1; 4000 x 2 49.0, 49.0, 48.9, 49.8, 48.7, 49.0, 48.4, 48.7; causal 48.2, 48.2, 48.2, 49.0, 47.9,
+    // 48.2, 47.6, 48.0; D = 64 8143 x 6 causal 79.1, 79.6, 79.9, 79.9, 79.1, 79.7, 79.2, 79.2; 8192 x 3 71.9, 72.4, 72.4, 72.6, 72.1, 72.6,
+    // 72.3, 72.1.  The variants with such work groups have the loop 8 bytes further on; they run two waves to a SIMD and are within
+    // 0.6 % wherever it is (1031 x 60 43.1 to 43.5, D = 64 520 x 60 12.65 to 12.77).
+    asm volatile(".p2align 6\n\t.rept %0\n\ts_nop 0\n\t.endr" ::"n"(D == 128 ? 6 : 4));
     bool odd_done = false;
     for (;;) {
       int why;
