@@ -3831,6 +3831,11 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
     constexpr int kS = NB * kKS, kP = 2 * kS, kV = kP + 2 * kDB, kUnits = kV + 2 * kDB;  // the first unit past each kind
     constexpr int kPairs = 8 / kKS;  // pairs of P formed in a unit
     constexpr int kLead = NB == 2 ? 2 : 3;
+    // The first unit that forms dS.  neg_mul_to_f16x2 is inline asm: the compiler leaves no time in front of it for the results of
+    // the last MFMA of dP - delta to arrive, 11 wait states after its issue.  The MFMAs of the units in between, of 8 passes
+    // each and issued one after the other, do: two of them are 16.
+    constexpr int kDs = kP + kDB;
+    static_assert(kDs - kP >= 2, "dS would be formed from a dP that is not there yet");
     struct Frag { h8 a, k; };
     const unsigned at = slot * 2 * Geo::kTileBytes;
     const int q0 = j * kResident, lane = thread_now() & 63, i = lane & 31, hh = lane >> 5;
@@ -3919,7 +3924,7 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
         }
       });
       static_for<2>([&](auto cc_tag) __attribute__((always_inline)) {
-        constexpr int cc = decltype(cc_tag)::value, first = kP + (1 + cc) * kDB;
+        constexpr int cc = decltype(cc_tag)::value, first = kDs + cc * kDB;
         if constexpr (m >= first && m < first + kDB) {
           constexpr int kOf = 4 / kDB;
 #pragma unroll
