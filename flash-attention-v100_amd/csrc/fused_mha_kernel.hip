@@ -103,6 +103,9 @@ __device__ __forceinline__ h8 neg_mul_to_f16x8(h8 p, const float* x) {
   return __builtin_bit_cast(h8, r);
 }
 
+// Element strides of a (batch, n, head, d) tensor whose last dimension is
+// contiguous.  The dense layout of reference kernel/fused_mha_kernel.cu:57-59 is
+// {n*head*d, head*d, d}.
 struct Strides {
   long b;
   int n, h;
@@ -122,16 +125,6 @@ __device__ __forceinline__ int acc_row(int rb, int r, int hh) {
   return rb * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
 }
 
-// Store a [D][32 resident] fp32 accumulator, scaled, as fp16 rows of a dense
-// (B, N, H, D) tensor, through a staging tile in LDS that belongs to the wave
-// (32 rows of kStagePitch bytes): each lane first writes the 4-feature pieces it
-// holds of its own row, then the wave reads the tile back row-wise, so that
-// every row leaves as whole 16-byte pieces written by neighbouring lanes (a
-// 256-byte row by 16 lanes, as the reference's epilogue does with its 128-bit
-// stores, kernel/fused_mha_kernel.cu:318-322, 714-734).  Lane (i, hh) owns row
-// row0 + i; per 32-feature block it holds features 8*g + 4*hh + 0..3 for g = 0..3.
-// The caller makes sure (with a block barrier) that nobody still reads what the
-// staging tile overwrites.
 // The rows of a staging tile as they leave.  All of them are asked for before the first is stored, and only a block with rows
 // past the end looks at each: one after the other, as read, wait, test and store, they take 200 cycles each.
 // Kernels in graphs of 20 calls, us one after the other and as it is, forward, then backward, N x slices: D = 64 77 x 8 causal
@@ -168,6 +161,16 @@ __device__ __forceinline__ void store_staged(half_t* __restrict__ base, int row_
   }
 }
 
+// Store a [D][32 resident] fp32 accumulator, scaled, as fp16 rows of a dense
+// (B, N, H, D) tensor, through a staging tile in LDS that belongs to the wave
+// (32 rows of kStagePitch bytes): each lane first writes the 4-feature pieces it
+// holds of its own row, then the wave reads the tile back row-wise, so that
+// every row leaves as whole 16-byte pieces written by neighbouring lanes (a
+// 256-byte row by 16 lanes, as the reference's epilogue does with its 128-bit
+// stores, kernel/fused_mha_kernel.cu:318-322, 714-734).  Lane (i, hh) owns row
+// row0 + i; per 32-feature block it holds features 8*g + 4*hh + 0..3 for g = 0..3.
+// The caller makes sure (with a block barrier) that nobody still reads what the
+// staging tile overwrites.
 template <int D>
 struct StageGeom {
   // bytes per row: a row plus 8, so that the lanes of a half wave, which write 8 bytes each to
@@ -614,9 +617,6 @@ __device__ __forceinline__ void store_ds(half_t* p, h8 v, IntTag<kOffset>) {
 #undef FMHA_STORE16
 }
 
-// Element strides of a (batch, n, head, d) tensor whose last dimension is
-// contiguous.  The dense layout of reference kernel/fused_mha_kernel.cu:57-59 is
-// {n*head*d, head*d, d}.
 // Row statistics of 64-row tiles for a work group of 4 * D threads: D / 8 lanes to a row, two rows each, in the order of
 // fmha_bwd_delta_kernel.  load asks for the rows of a tile, one tile after the other; make sums up what was asked for.
 template <int D>
@@ -3644,13 +3644,13 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
                    smem + Geo::kExOff + (wave * KB + kb) * (T::kBytes / 2));
   } else {
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-    const int lane = thread_now() & 63;
-    const half_t* const vp = V + b * vs.b + (long)h * vs.h + (long)min(blk[kb] * kResident + (lane & 31), N - 1) * vs.n +
-                             (lane >> 5) * 8;
+    for (int kb = 0; kb < KB; ++kb) {
+      const int lane = thread_now() & 63;
+      const half_t* const vp = V + b * vs.b + (long)h * vs.h + (long)min(blk[kb] * kResident + (lane & 31), N - 1) * vs.n +
+                               (lane >> 5) * 8;
 #pragma unroll
-    for (int kk = 0; kk < kKS; ++kk) vf[kb][kk] = *reinterpret_cast<const h8*>(vp + kk * 16);
-  }
+      for (int kk = 0; kk < kKS; ++kk) vf[kb][kk] = *reinterpret_cast<const h8*>(vp + kk * 16);
+    }
   }
   // Row statistics of 32 rows, in the order of fmha_bwd_delta_kernel, by the first D / 16 waves.  The rows of O that a wave
   // adds up it copies itself, 1 KiB of them, for its lanes to read back.
