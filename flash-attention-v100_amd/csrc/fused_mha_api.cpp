@@ -351,8 +351,7 @@ py::object flash_attn(const at::Tensor& q, const at::Tensor& k, const at::Tensor
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "FlashAttention forward/backward for gfx950";
-  m.def("attention", &attention, "Attention, differentiable in q, k and v");
-  m.def("flash_attn", &flash_attn, "Attention, differentiable in q, k and v, also under torch.jit.trace");
+  m.def("attention", &flash_attn, "Attention, differentiable in q, k and v, also under torch.jit.trace");
   m.def("fwd", &mha_fwd, "Forward pass");
   m.def("bwd", &mha_bwd, "Backward pass");
 }

@@ -27,7 +27,7 @@ except ImportError as exc:  # fail loudly: there is no fallback path
         "(run `python setup.py build_ext --inplace` in flash-attention-v100_amd/): %s" % exc
     ) from exc
 
-_flash_attn = flash_attn_cuda.flash_attn
+_attention = flash_attn_cuda.attention
 
 
 def _flash_attn_forward(q, k, v, softmax_scale, causal):
@@ -69,4 +69,4 @@ class FlashAttnFunc(torch.autograd.Function):
 
 def flash_attn_func(q, k, v, softmax_scale=None, causal=False):
     # FlashAttnFunc.apply with the autograd node in the extension, which under torch.jit.trace calls FlashAttnFunc itself
-    return _flash_attn(q, k, v, softmax_scale, causal)
+    return _attention(q, k, v, softmax_scale, causal)

@@ -46,6 +46,12 @@ def test_trace_keeps_the_inputs_that_options_are(monkeypatch, of):
     assert torch.equal(traced(q, k, v, then), q * (3 if of == "softmax_scale" else 12))
 
 
+def test_the_extension_has_no_function_without_a_caller():
+    import flash_attn_v100_cuda
+
+    assert {name for name in dir(flash_attn_v100_cuda) if not name.startswith("_")} == {"attention", "fwd", "bwd"}
+
+
 @pytest.mark.gpu
 def test_trace_of_the_extension():
     from flash_attn_v100 import flash_attn_func
