@@ -195,6 +195,8 @@ FMHA_HOST_DEVICE int fmha_last_level(int slices) {
 FMHA_HOST_DEVICE int fmha_blocks_in_order(int blocks_per_slice, bool heavy_first, bool short_last) {
   return !heavy_first && short_last && blocks_per_slice > 1 ? blocks_per_slice - 1 : blocks_per_slice;
 }
+// This and the two like it below, fmha_two_pass_block and fmha_ds_launch_block, are for checks on the host: the same order from
+// whole numbers, worked out anew for each block.  Kernels take an FmhaOrder.
 FMHA_HOST_DEVICE void fmha_scheduled_block(int lin, int slices, int blocks_per_slice, bool heavy_first, bool short_last,
                                            int& slice, int& blk) {
   const int run = fmha_blocks_in_order(blocks_per_slice, heavy_first, short_last);
@@ -315,7 +317,7 @@ FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool hea
 // us of forward and backward kernels with the divisions of ints, then with these, in graphs of 20 calls, N x slices: D = 64
 // 77 x 8 causal 5.61, 5.51 and 6.78, 6.63; 300 x 80 causal 7.52, 7.44 and 13.09, 12.95; 256 x 256 9.67, 9.62 and 21.8, 21.5; 3000
 // x 20 causal 33.9 both and 98.1, 97.1; D = 128 200 x 48 causal 9.41, 9.28 and 14.71, 14.51; 2048 x 80 causal 93.9 both and 290.6,
-// 287.7; 1031 x 60 42.0, 42.3 and 118.8, 117.8.
+// 287.7; 1031 x 60 equal and 118.8, 117.8.
 struct FmhaOrder {
   FmhaDivisor run, last_level;
   int slices;

@@ -381,6 +381,56 @@ int main() {
     assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
 
 
+def test_launches_with_last_rows_in_one_block_cover_every_block_once(tmp_path):
+    """csrc/block_map.h: the 128-query forward with work groups for the last rows of slices, as the kernel takes its order:
+    these first, then the blocks of one index fewer, each once and on the XCD of its slice."""
+    import subprocess
+
+    src = tmp_path / "check_tails.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <initializer_list>
+#include <vector>
+#include "block_map.h"
+int main() {
+  for (int slices : {1, 5, 8, 31, 60, 64, 71, 80, 129, 400, 1030})
+    for (int nb : {1, 2, 3, 4, 8, 9, 16})
+      for (int per : {2, 4})
+        for (bool causal : {false, true}) {
+          const FmhaOrder order(slices, nb, causal, false);
+          const int tails = fmha_tail_blocks(slices, per), grid = tails + slices * nb;
+          std::vector<int> seen(slices * (nb + 1), 0);
+          for (int w = 0; w < grid; ++w) {
+            const int lin = causal ? fmha_paired_block(w, grid) : w;
+            if (lin < 0 || lin >= grid || (lin & 7) != (w & 7)) { printf("%d of %d\n", lin, grid); return 1; }
+            if (lin < tails) {
+              for (int wave = 0; wave < per; ++wave) {
+                const int s = fmha_tail_slice(lin, wave, tails, per);
+                if (s < slices) ++seen[s * (nb + 1) + nb];
+              }
+            } else {
+              int s = -1, b = -1, t = -1, c = -1;
+              fmha_ordered_block(lin - tails, order.slices, order.run, order.last_level, causal, false, s, b);
+              fmha_ordered_block(lin - tails, slices, nb, fmha_last_level(slices), causal, false, t, c);
+              if (s != t || b != c || s < 0 || s >= slices || b < 0 || b >= nb) { printf("block %d of %d\n", lin, grid); return 1; }
+              const int q = slices >> 3;
+              if (s < 8 * q && s / q != (lin & 7)) { printf("slice %d of %d on XCD %d\n", s, slices, lin & 7); return 1; }
+              ++seen[s * (nb + 1) + b];
+            }
+          }
+          for (int n : seen)
+            if (n != 1) { printf("%d blocks of %d slices, %d to a block, %d: one %d times\n", nb, slices, per, causal, n); return 1; }
+        }
+  puts("ok");
+  return 0;
+}
+''')
+    inc = os.path.join(abi.ROOT, "flash-attention-v100_amd", "csrc")
+    exe = tmp_path / "check_tails"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", inc, str(src), "-o", str(exe)])
+    assert subprocess.check_output([str(exe)]).decode().strip() == "ok"
+
+
 def test_persistent_schedule_covers_every_block_once_and_balances(tmp_path):
     """csrc/block_map.h, compiled for the host: the rounds of the persistent work groups visit every block exactly
     once, a work group's blocks stay on its XCD (block number mod 8), and under causal masking the static
