@@ -317,8 +317,9 @@ at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
                  (float)scale, is_causal);
 }
 
-// An argument and what the caller gave for it.  While torch.jit.trace records nothing is converted: a scale that is a tensor is an
-// input of the recorded node then, and its value at that time would be a constant of the graph.
+// An argument and what the caller gave for it.  While torch.jit.trace records a tensor is not converted: a scale that is one is an
+// input of the recorded node then, and its value at that time would be a constant of the graph.  Plain values, which are the
+// rule, are converted without asking (small calls wait for the host: asking for each option costs 0.05 of their 4.6 us).
 template <typename T>
 struct __attribute__((visibility("hidden"))) Given {  // as pybind11's handles are
   py::handle object;
@@ -330,7 +331,8 @@ struct type_caster<Given<T>> {
   PYBIND11_TYPE_CASTER(Given<T>, make_caster<T>::name);
   bool load(handle src, bool convert) {
     value.object = src;
-    if (torch::jit::tracer::isTracing()) return true;
+    const bool plain = src.is_none() || PyBool_Check(src.ptr()) || PyFloat_CheckExact(src.ptr());
+    if (!plain && torch::jit::tracer::isTracing()) return true;
     make_caster<T> caster;
     if (!caster.load(src, convert)) return false;
     value.value = cast_op<T>(std::move(caster));
