@@ -315,9 +315,8 @@ FMHA_HOST_DEVICE bool fmha_ds_launch_block(int lin, int slices, int nb, bool hea
 
 // What the kernels take of a launch whose blocks are numbered in one of the orders above.
 // us of forward and backward kernels with the divisions of ints, then with these, in graphs of 20 calls, N x slices: D = 64
-// 77 x 8 causal 5.61, 5.51 and 6.78, 6.63; 300 x 80 causal 7.52, 7.44 and 13.09, 12.95; 256 x 256 9.67, 9.62 and 21.8, 21.5; 3000
-// x 20 causal 33.9 both and 98.1, 97.1; D = 128 200 x 48 causal 9.41, 9.28 and 14.71, 14.51; 2048 x 80 causal 93.9 both and 290.6,
-// 287.7; 1031 x 60 equal and 118.8, 117.8.
+// 77 x 8 causal 5.85, 5.76 and 7.02, 6.86; 300 x 80 causal 7.74, 7.65 and 13.5, 13.4; backward 256 x 256 23.1, 22.8; D = 128 200 x 48
+// causal 9.59, 9.45 and 15.1, 14.8; 2048 x 80 causal 95.5, 95.7 and 304, 297; 1031 x 60 43.2 both and 115.9, 114.6.
 struct FmhaOrder {
   FmhaDivisor run, last_level;
   int slices;
@@ -385,47 +384,50 @@ FMHA_HOST_DEVICE bool fmha_ds_in_one_launch(int slices, int n, int cus, bool cau
 // it reads Q, K, V and dO once.  It loses where slices leave CUs idle that blocks of 128 rows would fill: with few slices, and
 // with a last round that is far from full, the more so the longer a round is and under causal masking, where half of the blocks
 // of a slice are light, which the other launches pair with heavy ones.  At D = 64 up to 128 rows half of its waves have no
-// keys, and blocks of 128 rows, two to a CU, are ahead (64 x 256 equal, 128 x 256 and 128 x 1024 lose 4 and 18 %).
+// keys, and blocks of 128 rows, two to a CU, are ahead (64 x 256, 128 x 256 and 128 x 1024 lose 6, 2 and 15 %).
+// The lines are where the two were as fast when a work group per slice took 4 to 13 % longer than now, and were left there.  The
+// times are of the kernels as they are, in graphs of 20 calls, each side behind itself, mean of two cards, which differ by up to 5 %
+// in what one side takes of the other.  So some entries that the rule leaves to the passes are slower there, by up to 18 % (D = 64,
+// 512 x 1030).
 // us of the kernels of the backward, without it and with it, N x slices:
-// D = 128, without a mask.  One round: 40 x 128 7.5, 8.9; 40 x 160 12.9, 9.1; 200 x 128 25.5, 26.8; 256 x 136 43.0, 30.1; 256 x
-// 256 51.9, 37.4.  Two: 17 x 264 16.8, 11.9; 100 x 264 32.8, 28.6; 160 x 288 42.8, 46.0; 160 x 320 47.8, 45.8; 256 x 288 56.5,
-// 60.8; 256 x 320 61.2, 61.8; 256 x 512 100.3, 77.7.  More: 33 x 514 24.7, 23.9; 50 x 528 27.8, 27.6; 100 x 528 41.9, 44.2; 100
-// x 640 48.2, 45.0; 100 x 800 59.7, 61.0; 100 x 1030 73.0, 75.8; 100 x 1600 120.8, 114.0; 256 x 528 106.2, 99.8; 256 x 1024
-// 206, 163.
-// D = 128, causal.  160 x 128 22.1, 18.4 but 200 x 128 25.4, 24.3 and 100 x 128 slower; 256 x 160 35.8, 28.6; 256 x 256 43.5,
-// 32.5; 160 x 288 37.4, 35.5; 256 x 288 48.5, 55.3; 256 x 336 56.3, 57.5; 256 x 352 58.4, 58.0; 256 x 512 86.0, 64.9; 100 x 514
-// 40.1, 42.5; 100 x 640 48.8, 43.9; 256 x 528 90.9, 89.7.
-// D = 64, without a mask.  256 x 128 15.7, 18.8; 145 x 144 15.8, 12.9; 256 x 144 21.2, 19.1; 300 x 168 30.2, 32.1; 300 x 192
-// 34.3, 32.7; 512 x 192 60.9, 52.8; 512 x 256 78.5, 61.8; 300 x 352 60.1, 61.7; 300 x 384 61.2, 62.2; 300 x 400 62.9, 62.7; 512
-// x 384 115, 110; 512 x 448 131, 115; 300 x 560 85.2, 92.2; 300 x 600 92.6, 92.5; 512 x 560 173, 177; 512 x 620 191, 180; 300 x
-// 770 115, 123; 300 x 900 135, 129; 300 x 1030 157, 159; 512 x 1030 339, 299; 512 x 1300 427, 362.
-// D = 64, causal.  129 x 160 12.6, 13.1; 129 x 168 14.5, 13.1; 160 x 256 19.1, 15.1; 145 x 416 26.9, 26.6; 145 x 448 28.1,
-// 27.3; 145 x 600 35.9, 39.0; 180 x 208 16.8, 16.3; 200 x 230 20.1, 18.7; 256 x 240 22.0, 22.1; 300 x 208 27.3, 29.2; 300 x 230
-// 31.3, 29.3; 300 x 480 56.5, 57.6; 300 x 496 60.9, 58.2; 512 x 208 48.8, 47.3; 512 x 230 52.3, 48.1; 512 x 256 59.0, 49.5; 512
-// x 432 93.7, 94.6; 512 x 448 98.2, 95.8; 512 x 512 110, 98.4; 512 x 640 142, 149; 512 x 720 165, 154; 512 x 800 195, 199; 512
-// x 900 217, 198; 512 x 1030 247, 246; 300 x 1030 124, 141.
+// D = 128, without a mask.  One round: 40 x 128 7.1, 8.9; 40 x 160 12.2, 9.1; 200 x 128 25.3, 25.2; 256 x 136 41.0, 27.5; 256 x
+// 256 50.7, 35.8.  Two: 17 x 264 17.1, 12.3; 100 x 264 27.3, 26.3; 160 x 288 41.6, 43.6; 160 x 320 45.6, 43.4; 256 x 288 56.5,
+// 56.9; 256 x 320 62.4, 58.0; 256 x 512 97.1, 70.6.  More: 33 x 514 23.8, 23.5; 50 x 528 27.4, 27.0; 100 x 528 41.0, 41.6; 100 x
+// 640 47.0, 42.1; 100 x 800 58.2, 56.4; 100 x 1030 70.1, 70.5; 100 x 1600 116, 108; 256 x 528 107, 94.0; 256 x 1024 204, 158.
+// D = 128, causal.  160 x 128 19.4, 17.0 but 200 x 128 23.3, 22.1 and 100 x 128 slower; 256 x 160 33.8, 26.1; 256 x 256 42.0,
+// 30.9; 160 x 288 35.8, 32.7; 256 x 288 46.9, 50.2; 256 x 336 53.3, 51.4; 256 x 352 55.9, 52.4; 256 x 512 83.1, 60.3; 100 x 514
+// 39.4, 39.5; 100 x 640 46.8, 40.9; 256 x 528 87.3, 82.2.
+// D = 64, without a mask.  256 x 128 14.4, 17.5; 145 x 144 15.2, 12.8; 256 x 144 19.8, 17.9; 300 x 168 30.2, 31.8; 300 x 192
+// 34.2, 31.6; 512 x 192 61.1, 52.7; 512 x 256 80.5, 59.6; 300 x 352 61.1, 60.1; 300 x 384 62.3, 61.5; 300 x 400 64.3, 61.9; 512 x
+// 384 115, 105; 512 x 448 134, 111; 300 x 560 86.3, 89.4; 300 x 600 93.0, 89.7; 512 x 560 168, 161; 512 x 620 185, 166; 300 x 770
+// 116, 118; 300 x 900 131, 124; 300 x 1030 154, 155; 512 x 1030 328, 277; 512 x 1300 411, 340.
+// D = 64, causal.  129 x 160 12.3, 11.5; 129 x 168 12.5, 11.5; 160 x 256 17.4, 13.4; 145 x 416 25.4, 24.0; 145 x 448 26.8, 24.6;
+// 145 x 600 34.0, 34.8; 180 x 208 15.6, 14.4; 200 x 230 18.9, 16.8; 256 x 240 21.3, 20.1; 300 x 208 25.8, 25.3; 300 x 230 28.6,
+// 25.4; 300 x 480 53.8, 50.1; 300 x 496 59.7, 50.5; 512 x 208 46.9, 42.8; 512 x 230 50.8, 43.6; 512 x 256 58.4, 45.3; 512 x 432
+// 91.4, 84.9; 512 x 448 95.3, 85.7; 512 x 512 107, 89.2; 512 x 640 137, 134; 512 x 720 160, 143; 512 x 800 185, 179; 512 x 900
+// 212, 183; 512 x 1030 238, 220; 300 x 1030 118, 121.
 // D = 64 without a mask, 385 to 512 rows, one round: the line is at the fewest slices that were timed, not where the passes are
-// as fast.  A round takes as long with fewer (512 rows: 50.0), and the passes 57.5 for 512 x 176.
+// as fast.  A round takes as long with fewer: 512 x 176 57.9, 50.5.
 // Causal, D = 128, a second round of slices just past 96 rows (four tiles of 32 queries instead of three), us of forward and
-// backward, without it and with it: 97 x 257 37.1, 37.7; 97 x 266 37.8, 39.9; 97 x 296 39.2, 39.8; 97 x 320 39.8, 39.6; 105 x
-// 266 38.9, 40.3; 105 x 306 40.4, 40.2; 112 x 266 40.0, 40.6; 112 x 306 41.5, 40.5; 116 x 266 40.7, 40.7; 128 x 266 42.3, 41.4;
-// and 96 x 257 36.4, 33.4.
-// D = 64 without a mask, 161 to 176 rows, us of forward and backward, without it and with it: 161 x 598 63.0, 63.9; 161 x 612
-// 63.6, 65.1; 161 x 652 69.0, 66.9; 176 x 612 65.2, 65.2; 176 x 652 69.2, 67.3; 161 x 1812 166, 172; 161 x 1892 174, 174; 161 x
-// 1932 179, 177; 176 x 1812 173, 175; 176 x 1932 187, 182; 161 x 2068 190, 194; 176 x 2068 199, 200.
-// Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 27.0, 26.4; 161 x 256 27.3,
-// 27.4; 170 x 236 27.4, 26.5; 180 x 224 27.3, 27.2; 180 x 244 27.7, 27.4; 192 x 224 27.0, 27.5; 192 x 236 27.6, 27.1; 192 x 250
-// 27.7, 28.1; 193 x 224 29.3, 30.4; 193 x 250 30.5, 31.0; 200 x 230 29.9, 30.4; 200 x 240 30.3, 30.6; 200 x 256 32.0, 30.7.
+// backward, without it and with it: 97 x 257 34.4, 34.5; 97 x 266 34.7, 36.0; 97 x 296 35.9, 36.3; 97 x 320 36.6, 36.0; 105 x 266
+// 35.8, 36.3; 105 x 306 37.3, 36.3; 112 x 266 36.9, 36.5; 112 x 306 38.3, 36.6; 116 x 266 37.5, 36.8; 128 x 266 38.7, 37.4; and
+// 96 x 257 33.1, 31.4.
+// D = 64 without a mask, 161 to 176 rows, us of forward and backward, without it and with it: 161 x 598 64.3, 62.6; 161 x 612
+// 64.1, 62.3; 161 x 652 68.7, 65.5; 176 x 612 65.9, 64.5; 176 x 652 70.5, 66.5; 161 x 1812 166, 167; 161 x 1892 171, 169; 161 x
+// 1932 178, 174; 176 x 1812 171, 173; 176 x 1932 186, 180; 161 x 2068 192, 191; 176 x 2068 204, 198.
+// Causal, D = 64, 161 to 200 rows, us of forward and backward, without it and with it: 161 x 224 23.0, 23.9; 161 x 256 25.2,
+// 24.8; 170 x 236 24.4, 24.3; 180 x 224 23.5, 24.6; 180 x 244 25.4, 24.9; 192 x 224 23.6, 24.8; 192 x 236 24.7, 24.7; 192 x 250
+// 25.5, 25.1; 193 x 224 27.3, 27.8; 193 x 250 28.7, 28.8; 200 x 230 27.9, 27.8; 200 x 240 28.1, 28.1; 200 x 256 30.3, 28.1.
 // From 257 to 384 rows at D = 64 the line depends on the last tile of 64 rows too, of which the other launches do all even if
 // only half of it has rows (257 to 288 and 321 to 352 rows).  us of forward and backward, without it and with it, N x slices:
-// last tile whole, no mask: 290 x 448 99.7, 95.1; 384 x 448 119.6, 116.1; 290 x 704 144.3, 142.8; 304 x 960 195, 192; 384 x
-// 1216 317, 305; 290 x 1216 242, 245; 290 x 1440 294, 293; 320 x 1440 307, 300; 289 x 1576 329, 331; 304 x 1704 366, 351; but
-// 384 x 385 100, 103; 290 x 598 124, 127; 290 x 833 160, 167; 320 x 1076 218, 225; 290 x 1352 269, 281; 304 x 1544 330, 337.
-// Causal: 320 x 248 47.6, 45.2; 384 x 248 54.3, 53.2; 384 x 496 102, 100; 320 x 1264 216, 215; 289 x 1520 260, 251; but 320 x
-// 224 43.0, 43.7; 384 x 224 49.7, 51.2; 384 x 752 143, 150; 320 x 1014 160, 168.
-// Last tile half empty, no mask: 264 x 608 121, 116; 264 x 840 155, 153; 352 x 400 105, 102; 352 x 840 201, 201; 352 x 1080
-// 262, 263; 264 x 1336 244, 235; 352 x 1320 332, 321.  Causal: 264 x 232 44.1, 39.0; 352 x 224 48.7, 47.9; 264 x 752 116, 106;
-// 352 x 1008 191, 187.
+// last tile whole, no mask: 290 x 448 98.4, 91.1; 384 x 448 119, 105; 290 x 704 142, 136; 304 x 960 193, 184; 384 x 1216 313,
+// 279; 290 x 1216 237, 232; 290 x 1440 284, 281; 320 x 1440 299, 279; 289 x 1576 318, 316; 304 x 1704 346, 333; but 384 x 385
+// 101, 97.1; 290 x 598 123, 124; 290 x 833 163, 166; 320 x 1076 210, 212; 290 x 1352 260, 269; 304 x 1544 318, 318.
+// Causal: 320 x 248 44.5, 41.1; 384 x 248 52.1, 48.8; 384 x 496 97.2, 90.1; 320 x 1264 203, 190; 289 x 1520 242, 223; but 320 x
+// 224 40.3, 39.0; 384 x 224 47.5, 46.4; 384 x 752 139, 134; 320 x 1014 154, 148.
+// Last tile half empty, no mask: 264 x 608 117, 111; 264 x 840 152, 149; 352 x 400 103, 93.4; 352 x 840 198, 185; 352 x 1080 254,
+// 241; 264 x 1336 234, 227; 352 x 1320 324, 298.  Causal: 264 x 232 39.1, 35.0; 352 x 224 45.5, 42.6; 264 x 752 107, 94.4; 352 x
+// 1008 181, 166.
 FMHA_HOST_DEVICE bool fmha_backward_by_slice(int d, int n, int slices, int cus, bool causal) {
   if (n > 32768 / d) return false;  // LDS and registers hold no more keys
   const long rounds = ((long)slices + cus - 1) / cus, last = slices - (rounds - 1) * cus;

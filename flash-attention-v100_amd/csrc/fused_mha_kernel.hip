@@ -128,8 +128,8 @@ __device__ __forceinline__ int acc_row(int rb, int r, int hh) {
 // The rows of a staging tile as they leave.  All of them are asked for before the first is stored, and only a block with rows
 // past the end looks at each: one after the other, as read, wait, test and store, they take 200 cycles each.
 // Kernels in graphs of 20 calls, us one after the other and as it is, forward, then backward, N x slices: D = 64 77 x 8 causal
-// 5.51, 5.42 and 6.64, 6.40; 128 x 4 4.96, 4.88 and 6.25, 6.07; 1024 x 64 causal 15.7 both and 42.7, 42.1; D = 128 200 x 48
-// causal 9.27, 9.14 and 14.5 both; 2048 x 80 causal 93.9, 93.5 and 291, 289.
+// 5.76, 5.67 and 6.86, 6.61; 128 x 4 5.15, 5.06 and 6.48, 6.31; 1024 x 64 causal 17.3, 17.2 and 43.4, 43.1; D = 128 200 x 48
+// causal 9.45, 9.32 and 14.8 both; 2048 x 80 causal 95.7, 95.4 and 296, 295.
 template <int D, int kPitch, typename Piece>
 __device__ __forceinline__ void store_staged(half_t* __restrict__ base, int row_stride, int row0, int n, int lane,
                                              const char* __restrict__ stage, int upper_off) {
@@ -467,9 +467,9 @@ __device__ __forceinline__ void wait_vm() {
 // slice, row N-1 in the place of those past the end) and, once they are there, read as MFMA B operands.  Loaded straight to
 // registers, neighbouring lanes ask for 16 bytes of different rows each, and the CU's path to memory takes 64 cycles for
 // what a copy takes 16 for, 64 bytes of a row from every four lanes: 2,000 to 4,000 cycles at the start of a block.
-// Kernels in graphs of 20 calls, us loaded straight and this way, forward and backward, N x slices: D = 64 128 x 4 4.74, 4.53 and 6.07,
-// 5.64; 300 x 80 causal 7.13, 7.01 and 12.7, 11.7; 1024 x 64 causal 16.6, 16.4 and 43.3, 42.4; D = 128 128 x 32 6.4, 5.9 and 9.5, 8.35;
-// 200 x 48 causal 8.87, 8.60 and 14.5, 13.1; 700 x 24 13.8, 13.4 and 34.3, 33.2; 2048 x 80 causal 94.5, 93.6 and 294.7, 293.8.
+// Kernels in graphs of 20 calls, us loaded straight and this way, forward and backward, N x slices: D = 64 128 x 4 4.92, 4.70 and 6.31,
+// 5.87; 300 x 80 causal 7.38, 7.21 and 13.3, 12.4; 1024 x 64 causal 16.7, 16.6 and 43.1, 42.1; D = 128 128 x 32 6.69, 6.13 and 9.86,
+// 8.59; 200 x 48 causal 9.08, 8.79 and 14.9, 13.6; 700 x 24 13.9, 13.5 and 34.1, 33.2; 2048 x 80 causal 94.6, 93.3 and 296, 295.
 template <int D>
 __device__ __forceinline__ void copy_rows(const half_t* slice, int stride, int row0, int n, int lane, char* lds) {
   constexpr int kNC = SwzTile<D>::kNC, kBack = 960 * (kNC - 1);  // see copy16_blocks
@@ -550,8 +550,8 @@ __device__ __forceinline__ void store_resident16(half_t* __restrict__ base, int 
 
 // Arguments of a kernel, asked for here: left to the compiler they come in four or five groups, each where it is first needed and
 // each waited for by itself.  128-query forward, which also tests for a negative scale now instead of negating and
-// choosing, us before and after, N x slices: D = 64 77 x 8 causal 5.43, 5.22; 512 x 192 20.8, 20.2; 1024 x 64 causal 16.05, 15.7; D =
-// 128 200 x 48 causal 9.13, 8.87.  The kernels of the backward gain nothing from it.
+// choosing, us before and after, N x slices: D = 64 77 x 8 causal 5.66, 5.45; 512 x 192 21.8, 21.1; 1024 x 64 causal 17.2, 16.7; D =
+// 128 200 x 48 causal 9.33, 9.08.  The kernels of the backward gain nothing from it.
 __device__ __forceinline__ void load_now(const Strides& s) { asm volatile("" ::"s"(s.b), "s"(s.n), "s"(s.h)); }
 __device__ __forceinline__ void load_now(const FmhaDivisor& v) { asm volatile("" ::"s"(v.d), "s"(v.mul), "s"(v.shift)); }
 template <typename T>
@@ -2562,7 +2562,7 @@ bwd_dkdv_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, const
         for (int r = 0; r < 4; ++r) {
           const int f = WIDE ? quad >> 1 : 2 * (quad >> 1) + cb, e = (quad & 1) * 4 + r;
           float p = fast_exp2(fmaf(element(x, f, e), c, -l4[r]));
-          if (MASKED) {  // causal: queries key .. N - 1 count, one comparison: 200 x 48 12.9, 12.6 us; 2048 x 80 296, 295
+          if (MASKED) {  // causal: queries key .. N - 1 count, one comparison: 200 x 48 13.6, 13.1 us; 2048 x 80 295, 292
             const int row = stat_row(quad) + r;
             if (CAUSAL ? (unsigned)(row - (key + 16 * cb - at)) >= (unsigned)max(N - key - 16 * cb, 0) : row >= N - at) p = 0.f;
           }
@@ -2936,8 +2936,8 @@ bwd_dkdv_pipe_block(const half_t* __restrict__ Q, const half_t* __restrict__ K, 
     h8 frag[kLead];
     const int first_q = ki - t * kTile - 4 * hh, end_q = N - t * kTile - 4 * hh;  // queries that count, as acc_row(hq, r, 0)
     // Causal: how many count, from the first on, so a mask is one comparison and not two and a merge, in the shadow of the
-    // MFMAs, which masked tiles (the diagonal, the last) outgrow.  us before and with it: 77 x 8 6.39, 5.98; 300 x 80 11.7, 11.2;
-    // 777 x 36 21.7, 21.3; 1024 x 64 42.7 both
+    // MFMAs, which masked tiles (the diagonal, the last) outgrow.  us before and with it: 77 x 8 6.60, 6.19; 300 x 80 12.4, 11.9;
+    // 777 x 36 22.0, 21.6; 1024 x 64 42.1, 42.2
     const unsigned seen = max(N - ki, 0);
     f16v dl;
     f4v ls[4];
@@ -3530,13 +3530,13 @@ fmha_bwd_both_spill_kernel(const half_t* __restrict__ Q, const half_t* __restric
 // of which holds it for 15 cycles; the CU's LDS is busy half of the time.  What helps is fewer instructions between two
 // barriers, and MFMAs above all vector work: the products of a tile in an order in which P and dS are formed in the shadow of
 // others (work), no copies of fragments between registers (queries), what depends on the lane worked out once.  us without and
-// with these, backward, N x slices: D = 64 512 x 192 52.7, 50.0; 300 x 256 33.9, 32.4; 256 x 256 22.0, 20.9; causal 384 x 256 36.6,
-// 31.8; 160 x 256 14.7, 13.2; D = 128 256 x 256 36.0, 34.6; causal 31.9, 29.7; 100 x 256 16.9, 15.9.
+// with these, backward, N x slices: D = 64 512 x 192 52.9, 50.4; 300 x 256 33.9, 32.8; 256 x 256 22.9, 22.2; causal 384 x 256 36.5,
+// 33.1; 160 x 256 15.1, 13.8; D = 128 256 x 256 36.7, 35.4; causal 32.4, 30.5; 100 x 256 17.2, 16.2.
 // Not taken, 512 x 192: 16 waves of 32 keys 52.7; dQ of the tile before between the products of a tile 49.7; waves 4 to 7 with
 // dQ at the end of a tile 52.7; S and dP of both blocks from the same fragments 54.2, and before, with P and dS in stretches
 // without MFMAs, 54.6; priorities +-1 %.
-// 512 x 192 slices, D = 64: 50.0 us, 640 TFLOP/s on the 192 CUs that have work; two passes that form S and dP twice: 61.  256 x
-// 256, D = 128: 34.6 us, 620 TFLOP/s; over dS in memory: 51.9.
+// 512 x 192 slices, D = 64: 50.7 us, 635 TFLOP/s on the 192 CUs that have work; two passes that form S and dP twice: 61.  256 x
+// 256, D = 128: 35.3 us, 610 TFLOP/s; over dS in memory: 50.7.
 // At D = 128 without a mask 129 to 160 rows have four idle waves and one of up to 32 keys.  bwd_dkdv_block shares such keys
 // between its four pairs of waves, tile j to pair j mod 4, and adds the four sums up at the end; to have its bits the idle
 // waves do the same here.
@@ -3863,7 +3863,7 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
       const int r = 2 * e;
       if (e % 2 == 0) l4[n] = *reinterpret_cast<const f4v*>(st + 16 * e);
       float p0 = fast_exp2(fmaf(s[n][r], c, -l4[n][r & 3])), p1 = fast_exp2(fmaf(s[n][r + 1], c, -l4[n][(r & 3) + 1]));
-      if (MASKED) {  // causal: queries key .. N - 1 count, one comparison: 384 x 256, D = 64 32.7, 31.8 us
+      if (MASKED) {  // causal: queries key .. N - 1 count, one comparison: 384 x 256, D = 64 32.9, 32.2 us
         const int row = 8 * (r >> 2) + (r & 3), at = q0 + 4 * hh, q = q0 + row + 4 * hh, key = blk[n] * kResident + i;
         const unsigned seen = max(N - key, 0);
         if (CAUSAL ? (unsigned)(row - (key - at)) >= seen : q >= N) p0 = 0.f;
@@ -3959,7 +3959,9 @@ fmha_bwd_slice_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ K
   // Tiles in which none, one or both of this wave's key blocks count; those on the diagonal of one and at the end of the slice
   // with the mask, each in a loop of its own so that no accumulator crosses a branch.
   const int whole = N / kResident;
-  const bool past = nj > whole && (blk[0] == whole || blk[KB - 1] == whole);  // this wave has keys past the end
+  // This wave has keys past the end, which the mask keeps out of dQ.  (Under causal masking only tiles from `whole` on need it, which
+  // have a mask anyway; without it in the others, us: D = 64 300 x 256 26.4, 26.5; 500 x 256 45.0 both; 200 x 256 18.1, 17.9.)
+  const bool past = nj > whole && (blk[0] == whole || blk[KB - 1] == whole);
   auto span = [&](int end, int diag, auto nb_tag) __attribute__((always_inline)) {  // up to `end`, with a diagonal tile `diag`
     while (j < end) {
       while (j < end && (past || j == diag || j >= whole)) {
